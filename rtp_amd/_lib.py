@@ -6,12 +6,15 @@ The library is the only compute backend of this package: there is no PyTorch or 
 from __future__ import annotations
 
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 from typing import Optional
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # RTP_HIP_LIB in the environment names another build of the library (same ABI)
 LIB_PATH = os.environ.get("RTP_HIP_LIB") or os.path.join(_HERE, "lib", "librtp_hip.so")
+NATIVE_PATH = os.path.join(_HERE, "lib", "_rtp_native.so")
 
 RTP_F32 = 0
 RTP_BF16 = 1
@@ -201,6 +204,26 @@ def load() -> C.CDLL:
             raise RtpError("GemmDesc layout differs from the rtp_gemm_desc this library was built with")
         _lib = lib
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The extension module of csrc/host.cpp, bound to the library `load()` opens.  Touches no GPU."""
+    global _native
+    if _native is None:
+        if not os.path.exists(NATIVE_PATH):
+            raise RtpError(f"{NATIVE_PATH} is missing: build it with `make -C {os.path.join(_HERE, 'csrc')}` "
+                           "(or __graft_entry__.build())")
+        import torch  # noqa: F401  (the module's own dependencies are torch's libraries)
+        loader = importlib.machinery.ExtensionFileLoader("_rtp_native", NATIVE_PATH)
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_rtp_native", loader))
+        loader.exec_module(mod)
+        load()
+        mod.bind(LIB_PATH, RtpError)
+        _native = mod
+    return _native
 
 
 def last_error() -> str:

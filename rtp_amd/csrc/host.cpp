@@ -1,0 +1,510 @@
+// The Python side's way into librtp_hip.so for the calls of a training step: a CPython extension over the C ABI of
+// include/rtp_hip.h.  A layer's pass is a handful of 3 - 20 us launches, so what the host spends per launch decides the
+// time of every call that is not huge: through ctypes a product cost 9 us of argument handling (45 descriptor fields set
+// from Python, the stream object, the foreign call) around a 2.5 us launch; here it is under 1.5 us.
+//
+//   * every entry point that Python calls on the hot path, converted argument by argument from the C prototype itself
+//     (`invoke`), the current stream put in front, a negative status raised as RtpError;
+//   * `gemm` and the rotated linear products with their descriptors filled and their operands checked here;
+//   * GradBook: the parameters of a layer's shards and the slices of its gradient buffer, attached as .grad for a backward
+//     pass in one call (one Python attribute access per parameter otherwise).
+//
+// The library itself stays free of torch and Python: it is opened by path and resolved by name (`bind`).
+#include <Python.h>
+
+#include <ATen/core/Tensor.h>
+#include <c10/hip/HIPStream.h>
+#include <dlfcn.h>
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cstring>
+#include <string>
+#include <type_traits>
+#include <utility>
+#include <vector>
+
+#include "rtp_hip.h"
+
+namespace {
+
+PyObject* g_error = nullptr;  // rtp_amd._lib.RtpError
+decltype(&rtp_last_error) f_last_error = nullptr;
+
+void* current_stream() { return (void*)c10::hip::getCurrentHIPStream().stream(); }
+
+PyObject* raise_status(long rc) {
+  PyErr_Format(g_error, "librtp_hip status %ld: %s", rc, f_last_error());
+  return nullptr;
+}
+
+// ---- one argument ----
+template <class T>
+bool from_py(PyObject* o, T& out) {
+  if constexpr (std::is_pointer_v<T>) {
+    if (o == Py_None) {
+      out = nullptr;
+    } else if (THPVariable_Check(o)) {
+      out = (T)THPVariable_Unpack(o).data_ptr();
+    } else {
+      out = (T)PyLong_AsVoidPtr(o);
+    }
+  } else if constexpr (std::is_floating_point_v<T>) {
+    out = (T)PyFloat_AsDouble(o);
+  } else {
+    out = (T)PyLong_AsLongLong(o);
+  }
+  return !(out == (T)0 || out == (T)-1) || !PyErr_Occurred();
+}
+
+template <bool STREAM, class R, class... A, size_t... I>
+PyObject* invoke_at(R (*f)(A...), PyObject* const* args, std::index_sequence<I...>) {
+  std::tuple<A...> v;
+  if constexpr (STREAM) std::get<0>(v) = current_stream();
+  constexpr size_t S = STREAM ? 1 : 0;
+  bool ok = true;
+  (void)std::initializer_list<int>{(ok = ok && (I < S || from_py(args[I < S ? 0 : I - S], std::get<I>(v))), 0)...};
+  if (!ok) return nullptr;
+  R r;
+  Py_BEGIN_ALLOW_THREADS
+  r = std::apply(f, v);
+  Py_END_ALLOW_THREADS
+  if constexpr (std::is_same_v<R, int>) {
+    if (r < 0) return raise_status(r);
+  }
+  if constexpr (std::is_unsigned_v<R>) return PyLong_FromSize_t((size_t)r);
+  return PyLong_FromLongLong((long long)r);
+}
+template <bool STREAM, class R, class... A>
+PyObject* invoke(R (*f)(A...), const char* name, PyObject* const* args, Py_ssize_t n) {
+  constexpr Py_ssize_t want = (Py_ssize_t)sizeof...(A) - (STREAM ? 1 : 0);
+  if (n != want) return PyErr_Format(PyExc_TypeError, "%s takes %zd arguments, got %zd", name, want, n);
+  return invoke_at<STREAM>(f, args, std::index_sequence_for<A...>{});
+}
+
+// X(name): the stream of the C prototype is the current one and not passed;  P(name): passed as declared
+#define RTP_ENTRY_POINTS(X, P)                                                                                        \
+  P(rtp_gemm_warm_next) P(rtp_colsum_workspace_bytes) X(rtp_colsum) X(rtp_shard_copy_async) X(rtp_zero_async)        \
+  X(rtp_embedding_gather) X(rtp_embedding_gather_scale_pos) P(rtp_embedding_scatter_workspace_bytes)                  \
+  X(rtp_embedding_sort_ids) X(rtp_embedding_scatter_add_det) X(rtp_embedding_scatter_add_scaled)                      \
+  X(rtp_embedding_scatter_add_sgd) P(rtp_embedding_backward_supported) X(rtp_embedding_backward)                      \
+  X(rtp_softmax_fwd_masks) X(rtp_softmax_bwd) P(rtp_attn_supported) X(rtp_attn_fwd) X(rtp_attn_bwd)                   \
+  P(rtp_attn_flash_supported) X(rtp_attn_flash_fwd) X(rtp_attn_flash_bwd) P(rtp_layernorm_supported)                  \
+  X(rtp_add_layernorm_fwd) P(rtp_layernorm_bwd_workspace_bytes) X(rtp_layernorm_bwd) P(rtp_layernorm_bwd_blocks)      \
+  X(rtp_layernorm_bwd_finalize) X(rtp_softmax_xent_fwd) X(rtp_softmax_xent_reduce) X(rtp_softmax_xent_bwd)            \
+  P(rtp_top2_route_workspace_bytes) X(rtp_top2_route) X(rtp_top2_route_bwd) X(rtp_moe_dispatch) X(rtp_moe_combine)    \
+  X(rtp_moe_combine_dweight) P(rtp_gate_supported) X(rtp_gate_fwd) X(rtp_gate_dgrad)                                  \
+  P(rtp_gate_wgrad_workspace_bytes) X(rtp_gate_wgrad) X(rtp_conv2d_fwd) X(rtp_conv2d_wgrad)                           \
+  P(rtp_conv2d_wgrad_workspace_bytes) X(rtp_conv2d_dgrad) X(rtp_sgd_step) X(rtp_sgd_step_multi) X(rtp_adam_step)      \
+  X(rtp_adam_step_multi) X(rtp_cast)
+
+#define DECLARE(name) decltype(&name) f_##name = nullptr;
+RTP_ENTRY_POINTS(DECLARE, DECLARE)
+#undef DECLARE
+#define WRAP(name, stream)                                                     \
+  PyObject* py_##name(PyObject*, PyObject* const* args, Py_ssize_t n) {        \
+    return invoke<stream>(f_##name, #name, args, n);                           \
+  }
+#define WRAP_X(name) WRAP(name, true)
+#define WRAP_P(name) WRAP(name, false)
+RTP_ENTRY_POINTS(WRAP_X, WRAP_P)
+#undef WRAP_X
+#undef WRAP_P
+#undef WRAP
+
+decltype(&rtp_gemm) f_gemm = nullptr;
+decltype(&rtp_gemm_rowsum_fused) f_rowsum_fused = nullptr;
+decltype(&rtp_gemm_sgd_fused) f_sgd_fused = nullptr;
+decltype(&rtp_rotated_linear_fwd) f_linear_fwd = nullptr;
+decltype(&rtp_rotated_linear_bwd) f_linear_bwd = nullptr;
+
+PyObject* py_bind(PyObject*, PyObject* args) {
+  const char* path;
+  PyObject* error;
+  if (!PyArg_ParseTuple(args, "sO", &path, &error)) return nullptr;
+  void* lib = dlopen(path, RTLD_NOW | RTLD_LOCAL);
+  if (!lib) return PyErr_Format(PyExc_OSError, "%s", dlerror());
+  Py_INCREF(error);
+  g_error = error;
+  auto get = [lib](const char* name, auto& f) {
+    f = (std::remove_reference_t<decltype(f)>)dlsym(lib, name);
+    if (!f) PyErr_Format(PyExc_OSError, "librtp_hip.so has no %s", name);
+    return f != nullptr;
+  };
+  bool ok = get("rtp_last_error", f_last_error) && get("rtp_gemm", f_gemm) &&
+            get("rtp_gemm_rowsum_fused", f_rowsum_fused) && get("rtp_gemm_sgd_fused", f_sgd_fused) &&
+            get("rtp_rotated_linear_fwd", f_linear_fwd) && get("rtp_rotated_linear_bwd", f_linear_bwd);
+#define RESOLVE(name) ok = ok && get(#name, f_##name);
+  RTP_ENTRY_POINTS(RESOLVE, RESOLVE)
+#undef RESOLVE
+  if (!ok) return nullptr;
+  Py_RETURN_NONE;
+}
+
+int dtype_code(at::ScalarType t) {
+  return t == at::kFloat ? (int)RTP_F32 : t == at::kBFloat16 ? (int)RTP_BF16 : -1;
+}
+
+PyObject* bad(const char* what) {
+  PyErr_SetString(PyExc_ValueError, what);
+  return nullptr;
+}
+
+// ---- gemm(dtype, *, a=, b=, ...): the keyword arguments of ops.gemm_raw ----
+enum class K { ptr, i64, f32, flag, pair };
+struct Field {
+  const char* name;
+  K kind;
+  size_t at;  // offset in rtp_gemm_desc, or the flag's bit
+  PyObject* key;
+};
+#define AT(f) offsetof(rtp_gemm_desc, f)
+Field g_fields[] = {
+    {"a", K::ptr, AT(a)}, {"b", K::ptr, AT(b)}, {"c_out", K::ptr, AT(c_out)}, {"m", K::i64, AT(m)}, {"n", K::i64, AT(n)},
+    {"k", K::i64, AT(k)}, {"lda", K::i64, AT(lda)}, {"ldb", K::i64, AT(ldb)}, {"ldc", K::i64, AT(ldc)},
+    {"a_kcontig", K::flag, 1u << 16}, {"b_kcontig", K::flag, 1u << 17}, {"c_in", K::ptr, AT(c_in)},
+    {"ld_cin", K::i64, AT(ld_cin)}, {"bias", K::ptr, AT(bias)}, {"gate", K::ptr, AT(gate)},
+    {"ld_gate", K::i64, AT(ld_gate)}, {"alpha", K::f32, AT(alpha)}, {"relu", K::flag, RTP_GEMM_RELU},
+    {"out_f32", K::flag, RTP_GEMM_OUT_F32}, {"cin_f32", K::flag, RTP_GEMM_CIN_F32}, {"batch", K::i64, AT(batch)},
+    {"zdiv", K::i64, AT(zdiv)}, {"a_s", K::pair, AT(a_so)}, {"b_s", K::pair, AT(b_so)}, {"c_s", K::pair, AT(c_so)},
+    {"cin_s", K::pair, AT(cin_so)}, {"gate_s", K::pair, AT(gate_so)}, {"bias_s", K::pair, AT(bias_so)},
+    {"groups", K::i64, AT(groups)}, {"a_sg", K::i64, AT(a_sg)}, {"b_sg", K::i64, AT(b_sg)}, {"c_sg", K::i64, AT(c_sg)},
+    {"cin_sg", K::i64, AT(cin_sg)}, {"gate_sg", K::i64, AT(gate_sg)}, {"bias_sg", K::i64, AT(bias_sg)},
+    {"ksegs", K::i64, AT(ksegs)}, {"a_sk", K::i64, AT(a_sk)}, {"b_sk", K::i64, AT(b_sk)}, {"bias_sk", K::i64, AT(bias_sk)},
+    {"stream_out", K::flag, RTP_GEMM_STREAM_OUT}, {"rowsum", K::ptr, AT(a_rowsum)}, {"rowsum_sg", K::i64, AT(rowsum_sg)},
+    {"rowsum_accum", K::flag, RTP_GEMM_ROWSUM_ACCUM}, {"sgd_master", K::ptr, AT(sgd_master)},
+    {"sgd_weights", K::ptr, AT(sgd_weights)}, {"sgd_lr", K::f32, AT(sgd_lr)}, {"sgd_clip", K::f32, AT(sgd_clip)},
+    {"sgd_skip_out", K::flag, RTP_GEMM_SGD_SKIP_OUT},
+};
+#undef AT
+PyObject* g_field_index = nullptr;  // name -> index into g_fields
+
+// Runs the product; returns ROWSUM (1) if the row sums asked for were produced, SGD (2) if the update was applied: what the
+// operands do not allow is left out of the launch and reported by its missing bit.
+PyObject* py_gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObject* kwnames) {
+  if (nargs != 1 || !THPDtype_Check(args[0])) return PyErr_Format(PyExc_TypeError, "gemm(dtype, *, ...)");
+  const int dt = dtype_code(((THPDtype*)args[0])->scalar_type);
+  if (dt < 0) return PyErr_Format(PyExc_TypeError, "rtp_amd kernels support float32 and bfloat16, got %R", args[0]);
+  rtp_gemm_desc d;
+  memset(&d, 0, sizeof(d));
+  d.batch = d.zdiv = d.groups = d.ksegs = 1;
+  d.alpha = 1.0f;
+  uint32_t flags = 0;
+  const Py_ssize_t nk = kwnames ? PyTuple_GET_SIZE(kwnames) : 0;
+  for (Py_ssize_t i = 0; i < nk; ++i) {
+    PyObject *name = PyTuple_GET_ITEM(kwnames, i), *v = args[nargs + i];
+    PyObject* idx = PyDict_GetItemWithError(g_field_index, name);
+    if (!idx) return PyErr_Occurred() ? nullptr : PyErr_Format(PyExc_TypeError, "gemm: unknown argument %R", name);
+    const Field& f = g_fields[PyLong_AsLong(idx)];
+    char* at = (char*)&d + f.at;
+    bool ok = true;
+    switch (f.kind) {
+      case K::ptr: ok = from_py(v, *(void**)at); break;
+      case K::i64: ok = from_py(v, *(int64_t*)at); break;
+      case K::f32: ok = from_py(v, *(float*)at); break;
+      case K::pair:
+        ok = PyTuple_Check(v) && PyTuple_GET_SIZE(v) == 2 && from_py(PyTuple_GET_ITEM(v, 0), ((int64_t*)at)[0]) &&
+             from_py(PyTuple_GET_ITEM(v, 1), ((int64_t*)at)[1]);
+        if (!ok && !PyErr_Occurred()) PyErr_Format(PyExc_TypeError, "gemm: %s takes a pair", f.name);
+        break;
+      case K::flag: {
+        const int on = PyObject_IsTrue(v);
+        ok = on >= 0;
+        if (on) flags |= (uint32_t)f.at;
+        break;
+      }
+    }
+    if (!ok) return nullptr;
+  }
+  d.a_kcontig = (flags >> 16) & 1, d.b_kcontig = (flags >> 17) & 1;
+  int done = 0;
+  if (d.sgd_master) {
+    void *const master = d.sgd_master, *const weights = d.sgd_weights;
+    d.sgd_master = d.sgd_weights = nullptr;
+    d.flags = (int32_t)(flags & 0xffff & ~(uint32_t)RTP_GEMM_SGD_SKIP_OUT);
+    if (f_sgd_fused(dt, &d)) {
+      d.sgd_master = master, d.sgd_weights = weights;
+      done |= 2;
+    } else {
+      flags &= ~(uint32_t)RTP_GEMM_SGD_SKIP_OUT;
+    }
+  } else {
+    flags &= ~(uint32_t)RTP_GEMM_SGD_SKIP_OUT;
+  }
+  d.flags = (int32_t)(flags & 0xffff);
+  if (d.a_rowsum) {
+    if (f_rowsum_fused(dt, &d))
+      done |= 1;
+    else
+      d.a_rowsum = nullptr, d.rowsum_sg = 0;
+  }
+  int rc;
+  void* st = current_stream();
+  Py_BEGIN_ALLOW_THREADS
+  rc = f_gemm(st, dt, &d);
+  Py_END_ALLOW_THREADS
+  if (rc < 0) return raise_status(rc);
+  return PyLong_FromLong(done);
+}
+
+// ---- the rotated linear layer's products on tensors ----
+struct Mat {
+  char* p;
+  int64_t rows, cols, ld;
+};
+// [rows, cols] with unit column stride; leading dimension as the C ABI wants it
+bool as_mat(const at::Tensor& t, const char* what, Mat& m) {
+  if (t.dim() != 2 || (t.size(1) > 1 && t.stride(1) != 1)) {
+    PyErr_Format(PyExc_ValueError, "%s: need a 2-D tensor with unit column stride", what);
+    return false;
+  }
+  m.p = (char*)t.data_ptr();
+  m.rows = t.size(0), m.cols = t.size(1);
+  m.ld = m.rows > 1 ? t.stride(0) : std::max<int64_t>(m.cols, 1);
+  return true;
+}
+bool layer_of(const at::Tensor& home, int64_t w_off, PyObject* bias_off, int64_t n_s, int64_t k, rtp_rotated_linear& L,
+              int& dt) {
+  dt = dtype_code(home.scalar_type());
+  if (home.dim() != 2 || !home.is_contiguous() || dt < 0) {
+    PyErr_SetString(PyExc_ValueError,
+                    "rotated_linear: home must be the contiguous fp32 / bf16 [shards, numel] buffer of the layer");
+    return false;
+  }
+  if (!home.is_cuda()) {
+    PyErr_SetString(g_error, "rtp_amd kernels run on the GPU only; got a CPU tensor (there is no CPU path)");
+    return false;
+  }
+  L = rtp_rotated_linear{home.data_ptr(), home.size(1), home.size(0), w_off, -1, n_s, k};
+  return bias_off == Py_None || from_py(bias_off, L.bias_off);
+}
+const at::Tensor* opt_tensor(PyObject* o) { return o == Py_None ? nullptr : &THPVariable_Unpack(o); }
+
+// linear_fwd(x2, home, w_off, bias_off, n_s, k, y, col0, relu): y[:, col0 : col0 + shards*n_s] = x2 W_g^T + b_g
+PyObject* py_linear_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (n != 9 || !THPVariable_Check(a[0]) || !THPVariable_Check(a[1]) || !THPVariable_Check(a[6]))
+    return PyErr_Format(PyExc_TypeError, "linear_fwd(x2, home, w_off, bias_off, n_s, k, y, col0, relu)");
+  const at::Tensor &x2 = THPVariable_Unpack(a[0]), &home = THPVariable_Unpack(a[1]), &y = THPVariable_Unpack(a[6]);
+  int64_t w_off, n_s, k, col0;
+  if (!from_py(a[2], w_off) || !from_py(a[4], n_s) || !from_py(a[5], k) || !from_py(a[7], col0)) return nullptr;
+  rtp_rotated_linear L;
+  int dt;
+  Mat x, o;
+  if (!layer_of(home, w_off, a[3], n_s, k, L, dt) || !as_mat(x2, "x", x) || !as_mat(y, "y", o)) return nullptr;
+  const bool f32 = y.scalar_type() != home.scalar_type();
+  if (x.cols != k || o.rows != x.rows || col0 < 0 || o.cols - col0 < n_s * L.shards ||
+      x2.scalar_type() != home.scalar_type() || (f32 && y.scalar_type() != at::kFloat))
+    return bad("rotated_linear_fwd: x [rows, k] in the shards' dtype, y [rows, >= shards * n_s] (or fp32)");
+  const int flags = (PyObject_IsTrue(a[8]) ? RTP_GEMM_RELU : 0) | (f32 ? RTP_GEMM_OUT_F32 : 0);
+  int rc;
+  void* st = current_stream();
+  // one row: any leading dimension that holds it
+  const int64_t ldo = o.rows > 1 ? o.ld : std::max<int64_t>(o.cols, 1);
+  Py_BEGIN_ALLOW_THREADS
+  rc = f_linear_fwd(st, dt, &L, x.p, x.ld, x.rows, o.p + col0 * (int64_t)y.element_size(), ldo, flags);
+  Py_END_ALLOW_THREADS
+  if (rc < 0) return raise_status(rc);
+  Py_RETURN_NONE;
+}
+
+// linear_bwd(dy2, col0, x2, home, w_off, bias_off, n_s, k, dx, dx_init, relu_gate, grads, accumulate,
+//            sgd_master, sgd_weights, lr, clip, skip_store) -> done flags; see ops.rotated_linear_bwd
+PyObject* py_linear_bwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (n != 18 || !THPVariable_Check(a[0]) || !THPVariable_Check(a[3]))
+    return PyErr_Format(PyExc_TypeError, "linear_bwd: 18 arguments, got %zd", n);
+  for (int i : {2, 8, 9, 10, 11})
+    if (a[i] != Py_None && !THPVariable_Check(a[i])) return PyErr_Format(PyExc_TypeError, "linear_bwd: argument %d", i);
+  const at::Tensor &dy2 = THPVariable_Unpack(a[0]), &home = THPVariable_Unpack(a[3]);
+  int64_t col0, w_off, n_s, k;
+  if (!from_py(a[1], col0) || !from_py(a[4], w_off) || !from_py(a[6], n_s) || !from_py(a[7], k)) return nullptr;
+  rtp_rotated_linear L;
+  int dt;
+  Mat dy;
+  if (!layer_of(home, w_off, a[5], n_s, k, L, dt) || !as_mat(dy2, "dy", dy)) return nullptr;
+  if (col0 < 0 || dy.cols - col0 < n_s * L.shards || dy2.scalar_type() != home.scalar_type())
+    return bad("rotated_linear_bwd: dy must be [rows, >= shards * n_s] in the shards' dtype");
+  const at::Tensor *x2 = opt_tensor(a[2]), *dx = opt_tensor(a[8]), *init = opt_tensor(a[9]), *gate = opt_tensor(a[10]),
+                   *grads = opt_tensor(a[11]);
+  rtp_rotated_linear_bwd_args o;
+  memset(&o, 0, sizeof(o));
+  int32_t done = 0;
+  o.done = &done;
+  auto fits = [&](const at::Tensor& t, bool f32_ok) {
+    return t.scalar_type() == home.scalar_type() || (f32_ok && t.scalar_type() == at::kFloat);
+  };
+  Mat m, x{nullptr, dy.rows, k, k};
+  if (x2 && !as_mat(*x2, "x", x)) return nullptr;
+  if (dx) {
+    if (!as_mat(*dx, "dx", m)) return nullptr;
+    if (m.rows != dy.rows || m.cols != k) return bad("rotated_linear_bwd: dx must be [rows, k]");
+    if (!fits(*dx, true)) return PyErr_Format(PyExc_TypeError, "rotated_linear_bwd: dx must be in the shards' dtype or float32");
+    o.dx = m.p, o.ld_dx = m.ld;
+    o.dx_flags = dx->scalar_type() != home.scalar_type() ? RTP_GEMM_OUT_F32 : 0;
+    if (init) {
+      if (!as_mat(*init, "dx_init", m)) return nullptr;
+      if (m.rows != dy.rows || m.cols != k) return bad("rotated_linear_bwd: dx_init must match dx");
+      if (!fits(*init, true))
+        return PyErr_Format(PyExc_TypeError, "rotated_linear_bwd: dx_init must be in the shards' dtype or float32");
+      o.dx_init = m.p, o.ld_dx_init = m.ld;
+      if (init->scalar_type() != home.scalar_type()) o.dx_flags |= RTP_GEMM_CIN_F32;
+    }
+    if (gate) {
+      if (!as_mat(*gate, "relu_gate", m)) return nullptr;
+      if (m.rows != dy.rows || m.cols != k) return bad("rotated_linear_bwd: relu_gate must match dx");
+      if (!fits(*gate, false)) return PyErr_Format(PyExc_TypeError, "rotated_linear_bwd: relu_gate must be in the shards' dtype");
+      o.relu_gate = m.p, o.ld_relu_gate = m.ld;
+    }
+  }
+  if (grads) {
+    if (grads->sizes() != home.sizes() || grads->scalar_type() != home.scalar_type() || !grads->is_contiguous() || !x2)
+      return bad("rotated_linear_bwd: grads must be laid out like home, and the layer's input is needed");
+    o.grads = grads->data_ptr();
+    o.accumulate = PyObject_IsTrue(a[12]);
+    if (!from_py(a[13], o.sgd_master) || !from_py(a[14], o.sgd_weights) || !from_py(a[15], o.sgd_lr) ||
+        !from_py(a[16], o.sgd_clip))
+      return nullptr;
+    o.sgd_skip_grad_store = o.sgd_master ? PyObject_IsTrue(a[17]) : 0;
+  }
+  int rc;
+  void* st = current_stream();
+  const int64_t ldy = dy.rows > 1 ? dy.ld : std::max<int64_t>(dy.cols, 1);
+  Py_BEGIN_ALLOW_THREADS
+  rc = f_linear_bwd(st, dt, &L, dy.p + col0 * (int64_t)dy2.element_size(), ldy, x.p, x.ld, dy.rows, &o);
+  Py_END_ALLOW_THREADS
+  if (rc < 0) return raise_status(rc);
+  return PyLong_FromLong(done);
+}
+
+// ---- GradBook ----
+// The parameters of a layer, shard by shard, and their slices of the gradient buffer.  attach() is what a backward pass
+// does before it writes the buffer (allign_grad of the reference, rtp/module/collectives.py:75-79), for all shards at once:
+//   0  no parameter of some kind in every shard had a gradient: all slices attached, to be overwritten
+//   1  every parameter holds its own slice: to be accumulated into
+//  -1  anything else (shards that differ, a .grad somebody put there): nothing changed, the caller goes shard by shard
+struct GradBook {
+  PyObject_HEAD std::vector<std::vector<at::Tensor>>* params;
+  std::vector<std::vector<at::Tensor>>* views;
+};
+
+bool tensor_lists(PyObject* o, std::vector<std::vector<at::Tensor>>& out) {
+  PyObject* shards = PySequence_Fast(o, "GradBook: a list of lists of tensors");
+  if (!shards) return false;
+  bool ok = true;
+  for (Py_ssize_t s = 0; ok && s < PySequence_Fast_GET_SIZE(shards); ++s) {
+    PyObject* row = PySequence_Fast(PySequence_Fast_GET_ITEM(shards, s), "GradBook: a list of lists of tensors");
+    if (!row) {
+      ok = false;
+      break;
+    }
+    out.emplace_back();
+    for (Py_ssize_t i = 0; ok && i < PySequence_Fast_GET_SIZE(row); ++i) {
+      PyObject* t = PySequence_Fast_GET_ITEM(row, i);
+      if (!THPVariable_Check(t)) {
+        PyErr_SetString(PyExc_TypeError, "GradBook: a list of lists of tensors");
+        ok = false;
+      } else {
+        out.back().push_back(THPVariable_Unpack(t));
+      }
+    }
+    Py_DECREF(row);
+  }
+  Py_DECREF(shards);
+  return ok;
+}
+
+PyObject* book_new(PyTypeObject* type, PyObject* args, PyObject*) {
+  PyObject *p, *v;
+  if (!PyArg_ParseTuple(args, "OO", &p, &v)) return nullptr;
+  GradBook* b = (GradBook*)type->tp_alloc(type, 0);
+  if (!b) return nullptr;
+  b->params = new std::vector<std::vector<at::Tensor>>();
+  b->views = new std::vector<std::vector<at::Tensor>>();
+  bool ok = tensor_lists(p, *b->params) && tensor_lists(v, *b->views);
+  if (ok) {
+    ok = b->params->size() == b->views->size();
+    for (size_t s = 0; ok && s < b->params->size(); ++s) ok = (*b->params)[s].size() == (*b->views)[s].size();
+    if (!ok) PyErr_SetString(PyExc_ValueError, "GradBook: one slice per parameter");
+  }
+  if (!ok) {
+    Py_DECREF(b);
+    return nullptr;
+  }
+  return (PyObject*)b;
+}
+void book_dealloc(PyObject* o) {
+  GradBook* b = (GradBook*)o;
+  delete b->params;
+  delete b->views;
+  Py_TYPE(o)->tp_free(o);
+}
+PyObject* book_attach(PyObject* o, PyObject*) {
+  GradBook& b = *(GradBook*)o;
+  size_t fresh = 0, full = 0;
+  for (size_t s = 0; s < b.params->size(); ++s) {
+    bool none = false, own = true;
+    for (size_t i = 0; i < (*b.params)[s].size(); ++i) {
+      const at::Tensor& g = (*b.params)[s][i].grad();
+      none = none || !g.defined();
+      own = own && g.defined() && g.data_ptr() == (*b.views)[s][i].data_ptr();
+    }
+    fresh += none, full += own;
+  }
+  if (fresh == b.params->size()) {
+    for (size_t s = 0; s < b.params->size(); ++s)
+      for (size_t i = 0; i < (*b.params)[s].size(); ++i) (*b.params)[s][i].mutable_grad() = (*b.views)[s][i];
+    return PyLong_FromLong(0);
+  }
+  return PyLong_FromLong(full == b.params->size() ? 1 : -1);
+}
+// every parameter has some gradient
+PyObject* book_complete(PyObject* o, PyObject*) {
+  for (const auto& row : *((GradBook*)o)->params)
+    for (const at::Tensor& p : row)
+      if (!p.grad().defined()) Py_RETURN_FALSE;
+  Py_RETURN_TRUE;
+}
+// .grad = None for every parameter (zero_grad(set_to_none=True))
+PyObject* book_drop(PyObject* o, PyObject*) {
+  for (const auto& row : *((GradBook*)o)->params)
+    for (const at::Tensor& p : row)
+      if (p.grad().defined()) p.mutable_grad() = at::Tensor();
+  Py_RETURN_NONE;
+}
+
+PyMethodDef book_methods[] = {{"attach", book_attach, METH_NOARGS, nullptr},
+                              {"complete", book_complete, METH_NOARGS, nullptr},
+                              {"drop", book_drop, METH_NOARGS, nullptr},
+                              {nullptr, nullptr, 0, nullptr}};
+PyTypeObject g_book_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+#define METHOD(name) {#name, (PyCFunction)(void*)py_##name, METH_FASTCALL, nullptr},
+PyMethodDef g_methods[] = {{"bind", py_bind, METH_VARARGS, nullptr},
+                           {"gemm", (PyCFunction)(void*)py_gemm, METH_FASTCALL | METH_KEYWORDS, nullptr},
+                           METHOD(linear_fwd) METHOD(linear_bwd) RTP_ENTRY_POINTS(METHOD, METHOD){nullptr, nullptr, 0, nullptr}};
+#undef METHOD
+PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_rtp_native", "librtp_hip.so for the calls of a training step", -1, g_methods};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__rtp_native(void) {
+  g_field_index = PyDict_New();
+  for (size_t i = 0; i < sizeof(g_fields) / sizeof(g_fields[0]); ++i) {
+    g_fields[i].key = PyUnicode_InternFromString(g_fields[i].name);
+    PyObject* idx = PyLong_FromSize_t(i);
+    PyDict_SetItem(g_field_index, g_fields[i].key, idx);
+    Py_DECREF(idx);
+  }
+  g_book_type.tp_name = "_rtp_native.GradBook";
+  g_book_type.tp_basicsize = sizeof(GradBook);
+  g_book_type.tp_flags = Py_TPFLAGS_DEFAULT;
+  g_book_type.tp_new = book_new;
+  g_book_type.tp_dealloc = book_dealloc;
+  g_book_type.tp_methods = book_methods;
+  if (PyType_Ready(&g_book_type) < 0) return nullptr;
+  PyObject* m = PyModule_Create(&g_module);
+  if (m) {
+    Py_INCREF(&g_book_type);
+    PyModule_AddObject(m, "GradBook", (PyObject*)&g_book_type);
+  }
+  return m;
+}

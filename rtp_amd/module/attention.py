@@ -20,7 +20,7 @@ from torch.nn.modules.linear import NonDynamicallyQuantizableLinear
 from torch.nn.parameter import Parameter
 
 from .. import ops
-from ..ring import Rotation, ring_order, run_wgrad
+from ..ring import rotation, run_wgrad
 from . import shard_ops as S
 from .collectives import RotatedLayer
 from .utils import (affine_weight, affine_weight_attention, as_rows, attention_block_index,
@@ -166,8 +166,7 @@ class _AttentionFn(torch.autograd.Function):
         # drop: per-probability multiplier 0 or 1 / (1 - drop_p); pv: the probabilities that meet V
         drop = torch.empty(ws * Z, L, L, dtype=torch.float32, device=dev) if drop_p > 0.0 else None
         pv = torch.empty_like(p) if drop_p > 0.0 else p
-        order = ring_order(layer.rank, ws)
-        rot = Rotation(store.home, order, group=store.stage_group)
+        rot = rotation(store, layer.rank)
         acc = ops.ShardSum(out, sum(len(w) for w in rot.windows))
         i = 0
         for j in range(rot.steps):
@@ -213,7 +212,7 @@ class _AttentionFn(torch.autograd.Function):
             rot.release(j)
         weights = None
         if want_weights:
-            last = order[-1]
+            last = (layer.rank + ws - 1) % ws  # the shard of the last ring step
             weights = pv[last * Z:(last + 1) * Z].view(N, h_s, L, L)  # functional.py:789-792: after dropout
         ctx.layer = layer
         ctx.dims = (L, N, E)
@@ -246,8 +245,7 @@ class _AttentionFn(torch.autograd.Function):
         ldq = N * ws * 3 * e_s
         fused = ctx.fused
         delta = torch.empty_like(p) if ctx.flash is not None else None
-        order = ring_order(layer.rank, ws, reverse=True)
-        rot = Rotation(store.home, order, group=store.stage_group)
+        rot = rotation(store, layer.rank, reverse=True)
         # residual_grad: the caller's y = norm(x + attention(x)) sends x's whole gradient through this function,
         # which adds the output gradient to its own input gradient in the epilogue of the last product
         init = dout2 if ctx.residual_grad else None
@@ -305,7 +303,7 @@ class _AttentionFn(torch.autograd.Function):
                     S.col_dgrad(dqkv, flat, 0, 3 * e_s, E, c_out, q0, c_in=c_in)
                 i += 1
             rot.release(j)
-        runs = store.grad_runs(order)
+        runs = store.grad_runs()
 
         def param_grads():
             for first, cnt, accumulate in runs:
@@ -390,8 +388,7 @@ class _GeneralAttentionFn(torch.autograd.Function):
         drop = torch.empty(ws * Z, L, sk, dtype=torch.float32, device=dev) if drop_p > 0.0 else None
         pv = torch.empty_like(p) if drop_p > 0.0 else p
         ld = N * E  # one step along the sequence in q, k, v and o
-        order = ring_order(layer.rank, ws)
-        rot = Rotation(store.home, order, group=store.stage_group)
+        rot = rotation(store, layer.rank)
         acc = ops.ShardSum(out, sum(len(w) for w in rot.windows))
         i = 0
         for j in range(rot.steps):
@@ -425,7 +422,7 @@ class _GeneralAttentionFn(torch.autograd.Function):
             rot.release(j)
         weights = None
         if want_weights:
-            last = order[-1]
+            last = (layer.rank + ws - 1) % ws  # the shard of the last ring step
             weights = pv[last * Z:(last + 1) * Z].view(N, h_s, L, sk)
         ctx.layer = layer
         ctx.dims = (L, N, E, s_in, sk)
@@ -453,8 +450,7 @@ class _GeneralAttentionFn(torch.autograd.Function):
         dqb = torch.empty(L * N, E, dtype=dt, device=dev)
         dkb = torch.empty(sk * N, E, dtype=dt, device=dev)
         dvb = torch.empty(sk * N, E, dtype=dt, device=dev)
-        order = ring_order(layer.rank, ws, reverse=True)
-        rot = Rotation(store.home, order, group=store.stage_group)
+        rot = rotation(store, layer.rank, reverse=True)
         parts = sum(len(w) for w in rot.windows)
         # input gradients of the three projections, each summed over the shards; the rows of an appended zero key
         # belong to no input
@@ -502,7 +498,7 @@ class _GeneralAttentionFn(torch.autograd.Function):
                         S.col_dgrad(src, flat, w_off, e_s, width, c_out, c0, c_in=c_in)
                 i += 1
             rot.release(j)
-        runs = store.grad_runs(order)
+        runs = store.grad_runs()
         dk_in, dv_in = dkb[:s_in * N], dvb[:s_in * N]
 
         def param_grads():

@@ -75,6 +75,9 @@ class ShardStore:
                 raise ValueError("all shards of a layer must have identical parameter shapes")
         self.home: Optional[torch.Tensor] = None
         self.grads: Optional[torch.Tensor] = None
+        self.one_run = None                          # ring.OneRun over home
+        self._params: List[List[nn.Parameter]] = []  # of every shard, as packed
+        self._book = None                            # native.GradBook over _params and the slices of `grads`
         self._overwrite = set()
         self.stage_group = None  # set by ring.group_stores
         self.fused_sgd = None  # set by an optimiser that applies its update inside the weight-gradient products
@@ -99,11 +102,13 @@ class ShardStore:
             for s in range(self.world_size):
                 for p, off, n in zip(self.params(s), self.offsets, self.numels):
                     home[s, off:off + n].copy_(p.data.reshape(-1))
+        from .. import ring
         self.home = home
-        self.grads = None
+        self.one_run = ring.OneRun(home)
+        self._params = [list(m.parameters()) for m in self.modules]
+        self._drop_grad_storage()
         self._overwrite.clear()
         if home.is_cuda:
-            from .. import ring
             ring.fence(home.device)
         for s in range(self.world_size):
             self.modules[s]._full_param = home[s]
@@ -117,24 +122,37 @@ class ShardStore:
         return [flat[off:off + n].view(shape) for off, n, shape in zip(self.offsets, self.numels, self.shapes)]
 
     # -- gradients -------------------------------------------------------------------------------
+    def _drop_grad_storage(self) -> None:
+        self.grads = self._book = None
+        self._grad_rows: List[torch.Tensor] = []
+        self._grad_slices: List[List[torch.Tensor]] = []
+
+    def _grad_storage(self) -> None:
+        """The gradient buffer, its slices and the record the attaching works from: made on the first backward after
+        pack()."""
+        if self.grads is not None and self._book is not None:
+            return
+        from .. import _lib
+        self.grads = torch.empty_like(self.home)
+        self._grad_rows = list(self.grads.unbind(0))
+        self._grad_slices = [self.views(row) for row in self._grad_rows]
+        self._book = _lib.native().GradBook(self._params, self._grad_slices)
+        self._book.drop()
+
     def grad_views(self, s: int) -> Tuple[List[torch.Tensor], bool]:
         """Gradient slices of shard s and whether the caller must ACCUMULATE into them.
 
         If the shard's parameters carry no .grad (first backward, or after zero_grad(set_to_none=True))
         the slices are handed out for overwriting and attached as the parameters' .grad (allign_grad,
         collectives.py:75-79); otherwise they hold earlier gradients that must be added to."""
-        if self.grads is None or self.grads.device != self.home.device or self.grads.dtype != self.home.dtype:
-            self.grads = torch.empty_like(self.home)
-            for m in self.modules:
-                for p in m.parameters():
-                    p.grad = None
+        self._grad_storage()
         if s in self._overwrite:
             # zeroed by mark_overwrite(): the views are still attached, their contents are to be replaced
             self._overwrite.discard(s)
-            if all(p.grad is not None for p in self.params(s)):
-                return self.views(self.grads[s]), False
-        params = self.params(s)
-        views = self.views(self.grads[s])
+            if all(p.grad is not None for p in self._params[s]):
+                return self._grad_slices[s], False
+        params = self._params[s]
+        views = self._grad_slices[s]
         fresh = any(p.grad is None for p in params)
         if fresh:
             self.modules[s]._full_grad = self.grads[s]
@@ -163,16 +181,30 @@ class ShardStore:
                 self.grads[s].zero_()
         self._overwrite.clear()
 
-    def grad_runs(self, order: Sequence[int]):
+    def grad_runs(self, order: Optional[Sequence[int]] = None):
         if self.on_backward is not None:
             self.on_backward(self)
         return self._grad_runs(order)
 
-    def _grad_runs(self, order: Sequence[int]):
-        """Attach gradient storage to every shard in `order` and return maximal runs (first, count,
+    def _grad_runs(self, order: Optional[Sequence[int]] = None):
+        """Attach gradient storage to every shard (or those in `order`) and return maximal runs (first, count,
         accumulate) of consecutive shards that share the same accumulate flag, so that a grouped kernel can
         write a whole run of gradient rows in one launch."""
-        flags = {s: self.grad_views(s)[1] for s in order}
+        self._grad_storage()
+        ws = self.world_size
+        if order is None or len(order) == ws:
+            # all shards alike, as every pass of a training loop finds them: one call for the layer
+            if not self._overwrite:
+                state = self._book.attach()
+                if state >= 0:
+                    if state == 0:
+                        for s, m in enumerate(self.modules):
+                            m.__dict__["_full_grad"] = self._grad_rows[s]
+                    return [(0, ws, state == 1)]
+            elif len(self._overwrite) == ws and self._book.complete():
+                self._overwrite.clear()
+                return [(0, ws, False)]
+        flags = {s: self.grad_views(s)[1] for s in (range(ws) if order is None else order)}
         ids = sorted(flags)
         runs, start = [], ids[0]
         for a, b in zip(ids, ids[1:] + [None]):
@@ -230,6 +262,17 @@ class RotatedLayer(nn.Module):
         self._store.pack()
         self._anchor = torch.zeros((), dtype=torch.float32, device=self._store.home.device, requires_grad=True)
         return self
+
+    def zero_grad(self, set_to_none: bool = True) -> None:
+        """nn.Module.zero_grad; the usual case, gradients dropped, without a walk through the shards' modules."""
+        book = self._store._book
+        if not set_to_none or book is None or self._parameters:
+            super().zero_grad(set_to_none)
+            return
+        book.drop()
+        for m in self._modules.values():
+            if m is not self.shards and m not in self._store.modules:
+                m.zero_grad()
 
     def set_full_param(self, device=None, dtype=None):
         self.to(device=device, dtype=dtype)

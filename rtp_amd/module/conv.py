@@ -20,7 +20,7 @@ import torch
 import torch.nn as nn
 
 from .. import ops
-from ..ring import Rotation, ring_order, run_wgrad
+from ..ring import rotation, run_wgrad
 from .collectives import RotatedLayer, resolve_world
 from .utils import affine_weight, divide_and_check_no_remainder
 
@@ -65,7 +65,7 @@ class _ColumnConvFn(torch.autograd.Function):
         k = geom.c * geom.kh * geom.kw
         y = torch.empty(geom.n, co, geom.ho, geom.wo, dtype=x.dtype, device=x.device)
         b_off = n_s * k if layer.has_bias else None
-        rot = Rotation(store.home, ring_order(layer.rank, ws), group=store.stage_group)
+        rot = rotation(store, layer.rank)
         for j in range(rot.steps):
             for flat, first, cnt in rot.acquire(j):
                 ops.conv2d_fwd(x, geom, flat, 0, b_off, n_s, y, first * n_s)
@@ -81,11 +81,10 @@ class _ColumnConvFn(torch.autograd.Function):
         store = layer._store
         n_s, ws = layer.output_size_per_partition, layer.world_size
         k = geom.c * geom.kh * geom.kw
-        order = ring_order(layer.rank, ws, reverse=True)
         dx = None
         if ctx.needs_input_grad[0]:
             dx = torch.empty(geom.n, geom.c, geom.h, geom.w, dtype=dy.dtype, device=dy.device)
-            rot = Rotation(store.home, order, group=store.stage_group)
+            rot = rotation(store, layer.rank, reverse=True)
             acc = ops.ShardSum(dx, sum(len(w) for w in rot.windows))
             i = 0
             for j in range(rot.steps):
@@ -94,7 +93,7 @@ class _ColumnConvFn(torch.autograd.Function):
                     ops.conv2d_dgrad(dy, geom, flat, 0, n_s, first * n_s, c_out, addend=c_in)
                     i += 1
                 rot.release(j)
-        runs = store.grad_runs(order)
+        runs = store.grad_runs()
         b_off = n_s * k if layer.has_bias else None
 
         def param_grads():

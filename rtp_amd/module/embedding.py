@@ -15,7 +15,7 @@ import torch.nn as nn
 import torch.nn.init as init
 
 from .. import ops
-from ..ring import Rotation, ring_order
+from ..ring import rotation
 from .collectives import RotatedLayer
 from .shard_ops import _fused, _fused_done
 from .utils import affine_weight, divide_and_check_no_remainder
@@ -48,7 +48,7 @@ class _EmbeddingFn(torch.autograd.Function):
         d_s, ws = layer.embedding_dim_per_partition, layer.world_size
         flat_ids = ids.reshape(-1).contiguous()
         out = torch.empty(flat_ids.numel(), layer.embedding_dim, dtype=store.home.dtype, device=store.home.device)
-        rot = Rotation(store.home, ring_order(layer.rank, ws), group=store.stage_group)
+        rot = rotation(store, layer.rank)
         # tokens are [sequence, batch, ...]: every id of one position shares a positional row
         batch = flat_ids.numel() // ids.shape[0] if pos is not None else 1
         for j in range(rot.steps):
@@ -80,7 +80,7 @@ class _EmbeddingFn(torch.autograd.Function):
         if store.on_backward is not None:
             store.on_backward(store)
         # runs of consecutive shards with the same overwrite / accumulate state go out as one grouped launch
-        for first, cnt, accumulate in store._grad_runs(ring_order(layer.rank, ws, reverse=True)):
+        for first, cnt, accumulate in store._grad_runs():
             table = store.grads[first, :store.numels[0]].view(store.shapes[0])
             # an optimiser that applies its update where gradients are produced: the rows the step's tokens name are
             # updated by the scatter-add itself, the dense [V, D/ws] gradient is neither zero-filled nor written

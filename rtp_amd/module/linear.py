@@ -17,7 +17,7 @@ import torch.nn as nn
 import torch.nn.init as init
 
 from .. import ops
-from ..ring import Rotation, ring_order, run_wgrad
+from ..ring import rotation, run_wgrad
 from . import shard_ops as S
 from .collectives import RotatedLayer, resolve_world
 from .utils import affine_weight, as_rows, divide_and_check_no_remainder
@@ -72,7 +72,7 @@ class _ColumnLinearFn(torch.autograd.Function):
         x2 = as_rows(x, k)
         y = torch.empty(x2.shape[0], layer.out_features, dtype=x2.dtype, device=x2.device)
         b_off = n_s * k if layer.has_bias else None
-        rot = Rotation(store.home, ring_order(layer.rank, ws), group=store.stage_group)
+        rot = rotation(store, layer.rank)
         for j in range(rot.steps):
             for flat, first, cnt in rot.acquire(j):
                 S.col_fwd(x2, flat, 0, n_s, k, b_off, y, first * n_s)
@@ -80,7 +80,7 @@ class _ColumnLinearFn(torch.autograd.Function):
         ctx.layer = layer
         ctx.x_shape = x.shape
         ctx.save_for_backward(x2)
-        return y.view(*x.shape[:-1], layer.out_features)
+        return y if x.dim() == 2 else y.view(*x.shape[:-1], layer.out_features)
 
     @staticmethod
     def backward(ctx, dy):
@@ -90,11 +90,10 @@ class _ColumnLinearFn(torch.autograd.Function):
         n_s, k, ws = layer.output_size_per_partition, layer.in_features, layer.world_size
         dy2 = as_rows(dy, layer.out_features)
         need_dx = ctx.needs_input_grad[0]
-        order = ring_order(layer.rank, ws, reverse=True)
         dx = None
         if need_dx:
             dx = torch.empty_like(x2)
-            rot = Rotation(store.home, order, group=store.stage_group)
+            rot = rotation(store, layer.rank, reverse=True)
             acc = ops.ShardSum(dx, sum(len(w) for w in rot.windows))
             i = 0
             for j in range(rot.steps):
@@ -103,7 +102,7 @@ class _ColumnLinearFn(torch.autograd.Function):
                     S.col_dgrad(dy2, flat, 0, n_s, k, c_out, first * n_s, c_in=c_in)
                     i += 1
                 rot.release(j)
-        runs = store.grad_runs(order)
+        runs = store.grad_runs()
 
         def param_grads():
             for first, cnt, accumulate in runs:
@@ -112,7 +111,9 @@ class _ColumnLinearFn(torch.autograd.Function):
             store.grads_ready()
 
         run_wgrad(dy2.device, param_grads, (dy2, x2))
-        return (dx.view(ctx.x_shape) if need_dx else None), None, None
+        if need_dx and len(ctx.x_shape) != 2:
+            dx = dx.view(ctx.x_shape)
+        return dx, None, None
 
 
 class _ColumnReluMlpFn(torch.autograd.Function):
@@ -130,7 +131,7 @@ class _ColumnReluMlpFn(torch.autograd.Function):
         for lin, src, dst, relu in ((lin1, x2, h, True), (lin2, h, y, False)):
             n_s, k = lin.output_size_per_partition, lin.in_features
             b_off = n_s * k if lin.has_bias else None
-            rot = Rotation(lin._store.home, ring_order(lin.rank, lin.world_size), group=lin._store.stage_group)
+            rot = rotation(lin._store, lin.rank)
             for j in range(rot.steps):
                 for flat, first, cnt in rot.acquire(j):
                     S.col_fwd(src, flat, 0, n_s, k, b_off, dst, first * n_s, relu=relu)
@@ -156,9 +157,8 @@ class _ColumnReluMlpFn(torch.autograd.Function):
         for lin, g, inp, dinp, gate in ((lin2, dy2, h, dh, h), (lin1, dh, x2, dx, None)):
             store = lin._store
             n_s, k = lin.output_size_per_partition, lin.in_features
-            order = ring_order(lin.rank, lin.world_size, reverse=True)
             if dinp is not None:
-                rot = Rotation(store.home, order, group=store.stage_group)
+                rot = rotation(store, lin.rank, reverse=True)
                 steps = sum(len(w) for w in rot.windows)
                 # residual_grad: y = norm(x + mlp(x)) sends x's whole gradient through here (dy + mlp'(dy))
                 init = dy2 if (ctx.residual_grad and lin is lin1) else None
@@ -173,7 +173,7 @@ class _ColumnReluMlpFn(torch.autograd.Function):
                     rot.release(j)
                 if lin is lin2 and ctx.keep is not None:
                     dh.mul_(ctx.keep)  # h > 0 already implies a kept element; what is left is the 1 / (1 - p)
-            runs = store.grad_runs(order)
+            runs = store.grad_runs()
 
             def param_grads(lin=lin, store=store, g=g, inp=inp, runs=runs, n_s=n_s, k=k):
                 for first, cnt, accumulate in runs:
@@ -211,7 +211,7 @@ class _RowLinearFn(torch.autograd.Function):
         x2 = as_rows(x, layer.in_features)
         y = torch.empty(x2.shape[0], n, dtype=x2.dtype, device=x2.device)
         b_off = n * k_s if layer.has_bias else None
-        rot = Rotation(store.home, ring_order(layer.rank, ws), group=store.stage_group)
+        rot = rotation(store, layer.rank)
         acc = ops.ShardSum(y, sum(len(w) for w in rot.windows))
         i = 0
         for j in range(rot.steps):
@@ -223,7 +223,7 @@ class _RowLinearFn(torch.autograd.Function):
         ctx.layer = layer
         ctx.x_shape = x.shape
         ctx.save_for_backward(x2)
-        return y.view(*x.shape[:-1], n)
+        return y if x.dim() == 2 else y.view(*x.shape[:-1], n)
 
     @staticmethod
     def backward(ctx, dy):
@@ -233,16 +233,15 @@ class _RowLinearFn(torch.autograd.Function):
         k_s, n, ws = layer.input_size_per_partition, layer.out_features, layer.world_size
         dy2 = as_rows(dy, n)
         need_dx = ctx.needs_input_grad[0]
-        order = ring_order(layer.rank, ws, reverse=True)
         dx = None
         if need_dx:
             dx = torch.empty_like(x2)
-            rot = Rotation(store.home, order, group=store.stage_group)
+            rot = rotation(store, layer.rank, reverse=True)
             for j in range(rot.steps):
                 for flat, first, cnt in rot.acquire(j):
                     S.row_dgrad(dy2, flat, 0, n, k_s, dx, first * k_s)
                 rot.release(j)
-        runs = store.grad_runs(order)
+        runs = store.grad_runs()
 
         def param_grads():
             for first, cnt, accumulate in runs:
@@ -251,7 +250,9 @@ class _RowLinearFn(torch.autograd.Function):
             store.grads_ready()
 
         run_wgrad(dy2.device, param_grads, (dy2, x2))
-        return (dx.view(ctx.x_shape) if need_dx else None), None, None
+        if need_dx and len(ctx.x_shape) != 2:
+            dx = dx.view(ctx.x_shape)
+        return dx, None, None
 
 
 class _ParallelLinearBase(RotatedLayer):

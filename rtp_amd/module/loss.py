@@ -55,12 +55,12 @@ class _LinearCrossEntropyFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, anchor, layer, target, ignore_index, mean):
-        from ..ring import Rotation, ring_order
+        from ..ring import rotation
         from .utils import as_rows
         store = layer._store
         n_s, k = layer.output_size_per_partition, layer.in_features
         x2 = as_rows(x, k)
-        rot = Rotation(store.home, ring_order(layer.rank, layer.world_size), group=store.stage_group)
+        rot = rotation(store, layer.rank)
         runs = rot.acquire(0)
         if rot.steps != 1 or len(runs) != 1:
             raise RuntimeError("linear_cross_entropy needs all shards of the layer in one run (rotation window = all)")
@@ -74,15 +74,14 @@ class _LinearCrossEntropyFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dloss):
-        from ..ring import Rotation, ring_order, run_wgrad
+        from ..ring import rotation, run_wgrad
         from . import shard_ops as S
         layer = ctx.layer
         x2, target, stats, scale = ctx.saved_tensors
         store = layer._store
         n_s, k, ws = layer.output_size_per_partition, layer.in_features, layer.world_size
         b_off = n_s * k if layer.has_bias else None
-        order = ring_order(layer.rank, ws, reverse=True)
-        rot = Rotation(store.home, order, group=store.stage_group)
+        rot = rotation(store, layer.rank, reverse=True)
         flat = rot.acquire(0)[0][0]
         dlogits = ops.rotated_linear_xent_bwd(x2, flat, 0, b_off, n_s, k, target, ctx.ignore_index, stats,
                                               dloss.float().reshape(1), scale)
@@ -91,7 +90,7 @@ class _LinearCrossEntropyFn(torch.autograd.Function):
             dx = torch.empty_like(x2)
             S.col_dgrad(dlogits, flat, 0, n_s, k, dx, 0)
         rot.release(0)
-        runs = store.grad_runs(order)
+        runs = store.grad_runs()
 
         def param_grads():
             for first, cnt, accumulate in runs:

@@ -15,7 +15,7 @@ from torch import Tensor
 from torch.nn import Module, ModuleList
 
 from .. import ops
-from ..ring import Rotation, ring_order
+from ..ring import rotation
 from .collectives import RotatedLayer, resolve_world
 
 
@@ -105,7 +105,7 @@ class _ExpertsFn(torch.autograd.Function):
         es = x.element_size()
         h = torch.empty(x.shape[0], f_dim, dtype=x.dtype, device=x.device)
         y = torch.empty_like(x)
-        rot = Rotation(store.home, ring_order(layer.rank, layer.world_size), group=store.stage_group)
+        rot = rotation(store, layer.rank)
         for j in range(rot.steps):
             for flat, first, cnt in rot.acquire(j):
                 for le in range(n_local):
@@ -134,8 +134,7 @@ class _ExpertsFn(torch.autograd.Function):
         dy = dy.contiguous()
         dh = torch.empty_like(h)
         dx = torch.empty_like(x)
-        order = ring_order(layer.rank, layer.world_size, reverse=True)
-        rot = Rotation(store.home, order, group=store.stage_group)
+        rot = rotation(store, layer.rank, reverse=True)
         for j in range(rot.steps):
             for flat, first, cnt in rot.acquire(j):
                 for le in range(n_local):
@@ -153,7 +152,7 @@ class _ExpertsFn(torch.autograd.Function):
                                  ldb=m_dim, ldc=m_dim, a_sg=n_local * c_rows * f_dim, c_sg=n_local * c_rows * m_dim,
                                  **common)
             rot.release(j)
-        runs = store.grad_runs(order)  # attaches (and on first use allocates) the gradient storage
+        runs = store.grad_runs()  # attaches (and on first use allocates) the gradient storage
         g = store.grads
         for first, cnt, accumulate in runs:
             for le in range(n_local):

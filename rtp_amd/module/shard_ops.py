@@ -23,12 +23,13 @@ def _rows(t: torch.Tensor):
 def col_fwd(x2, flat, w_off, n_s, k, bias_off, out, col0, *, relu=False):
     """out[:, col0 + g*n_s : col0 + (g+1)*n_s] = x2 @ W_g^T (+ b_g), g over the run: the run is a rotated
     column-parallel layer of its own (rtp_rotated_linear_fwd) whose outputs start at column col0."""
-    ops.rotated_linear_fwd(x2, flat, w_off, bias_off, n_s, k, out[:, col0:], relu=relu)
+    ops.native().linear_fwd(x2, flat, w_off, bias_off, n_s, k, out, col0, relu)
 
 
 def col_dgrad(dy2, flat, w_off, n_s, k, out, col0, c_in: Optional[torch.Tensor] = None, gate=None):
     """out[M, k] = (c_in +) sum_g dy2[:, col0 + g*n_s : ...] @ W_g   (contraction segmented over shards)."""
-    ops.rotated_linear_bwd(dy2[:, col0:], None, flat, w_off, None, n_s, k, dx=out, dx_init=c_in, relu_gate=gate)
+    ops.native().linear_bwd(dy2, col0, None, flat, w_off, None, n_s, k, out, c_in, gate, None, False, None, None, 0.0, 0.0,
+                            False)
 
 
 def _fused(store, accumulate, first, cnt, w_off, length):
@@ -54,12 +55,12 @@ def col_wgrad(dy2, x2, grads, first, w_off, n_s, k, col0, cnt, accumulate, b_off
     """grads[first+g, w_off : w_off + n_s*k] (+)= dy2[:, col0 + g*n_s : ...]^T @ x2, g < cnt; with `b_off` also the
     bias gradients grads[first+g, b_off : b_off + n_s] (+)= column sums of the same block of dy2.  `store`: the
     layer's ShardStore, for an optimiser that applies its update inside this launch."""
-    numel = grads.shape[1]
     es = grads.element_size()
-    m, _, lda = _rows(dy2)
-    _, _, ldb = _rows(x2)
-    c = grads.data_ptr() + (first * numel + w_off) * es
     if n_s == 1 and cnt > 1:
+        numel = grads.shape[1]
+        m, _, lda = _rows(dy2)
+        _, _, ldb = _rows(x2)
+        c = grads.data_ptr() + (first * numel + w_off) * es
         # one output row per shard (a gate with one expert per shard): the run is a single product whose
         # output rows are the shards' gradient rows, `numel` apart -- vector loads instead of 1-row groups
         ops.gemm_raw(grads.dtype, a=dy2.data_ptr() + col0 * es, b=x2.data_ptr(), c_out=c, m=cnt, n=k, k=m, lda=lda,
@@ -71,11 +72,17 @@ def col_wgrad(dy2, x2, grads, first, w_off, n_s, k, col0, cnt, accumulate, b_off
     # one launch for the run (rtp_rotated_linear_bwd): the weight gradients, the bias gradients as the row sums of the
     # product's first operand dy^T, and the optimiser's update where one asked for it
     kw = _fused(store, accumulate, first, cnt, w_off, n_s * k)
+    # the weight-gradient half reads no weights: the gradient rows give the layout
+    run = grads if cnt == grads.shape[0] else grads[first:first + cnt]
     if kw:  # bound to the weight's own address; the entry point takes the run's base and adds w_off itself
-        kw = dict(sgd=kw["sgd"], sgd_master=kw["sgd_master"] - w_off * 4,
-                  sgd_weights=kw["sgd_weights"] - w_off * es if kw["sgd_weights"] else 0)
-    run = grads[first:first + cnt]  # the weight-gradient half reads no weights: the gradient rows give the layout
-    done = ops.rotated_linear_bwd(dy2[:, col0:], x2, run, w_off, b_off, n_s, k, grads=run, accumulate=accumulate, **kw)
+        sgd = kw["sgd"]
+        done = ops.native().linear_bwd(dy2, col0, x2, run, w_off, b_off, n_s, k, None, None, None, run, accumulate,
+                                       kw["sgd_master"] - w_off * 4,
+                                       kw["sgd_weights"] - w_off * es if kw["sgd_weights"] else None, sgd.lr, sgd.clip,
+                                       not sgd.keep_grads)
+    else:
+        done = ops.native().linear_bwd(dy2, col0, x2, run, w_off, b_off, n_s, k, None, None, None, run, accumulate, None,
+                                       None, 0.0, 0.0, False)
     if kw:
         if not done & _lib.ROTATED_SGD_DONE:
             kw["sgd"].missed = True

@@ -14,7 +14,7 @@ import torch.nn as nn
 from torch import Tensor
 
 from .. import ops
-from ..ring import Rotation, ring_order
+from ..ring import rotation
 from . import shard_ops as S
 from .collectives import RotatedLayer, resolve_world
 from .utils import affine_weight, as_rows, divide_and_check_no_remainder
@@ -102,7 +102,7 @@ class _GateProjectionFn(torch.autograd.Function):
         x2 = as_rows(x, layer.model_dim)
         ctx.box = box
         logits = torch.empty(x2.shape[0], layer.num_experts, dtype=torch.float32, device=x2.device)
-        rot = Rotation(store.home, ring_order(layer.rank, ws), group=store.stage_group)
+        rot = rotation(store, layer.rank)
         for j in range(rot.steps):
             for flat, first, cnt in rot.acquire(j):
                 rows = _run_rows(flat, e_s, layer.model_dim)
@@ -132,11 +132,10 @@ class _GateProjectionFn(torch.autograd.Function):
             return dl
 
         need_dx = ctx.needs_input_grad[0]
-        order = ring_order(layer.rank, ws, reverse=True)
         dx = None
         if need_dx:
             dx = torch.empty_like(x2)
-            rot = Rotation(store.home, order, group=store.stage_group)
+            rot = rotation(store, layer.rank, reverse=True)
             steps = sum(len(w) for w in rot.windows)
             acc = ops.ShardSum(dx, steps)
             i = 0
@@ -156,7 +155,7 @@ class _GateProjectionFn(torch.autograd.Function):
                         S.col_dgrad(low(), flat, 0, e_s, m, c_out, first * e_s, c_in=c_in)
                     i += 1
                 rot.release(j)
-        for first, cnt, accumulate in store.grad_runs(order):
+        for first, cnt, accumulate in store.grad_runs():
             rows = _run_rows(store.grads[first:first + cnt], e_s, m)
             if rows is not None and ops.gate_supported(x2, rows):
                 ops.gate_wgrad(dl32, first * e_s, x2, rows, accumulate)

@@ -60,7 +60,7 @@ def split_tensor_along_last_dim(tensor: torch.Tensor, num_partitions: int, conti
 
 def as_rows(x: torch.Tensor, width: int) -> torch.Tensor:
     """[..., width] -> [rows, width] with unit column stride (copies only if the layout forces it)."""
-    x2 = x.reshape(-1, width)
+    x2 = x if x.dim() == 2 and x.shape[1] == width else x.reshape(-1, width)
     if x2.shape[1] > 1 and x2.stride(1) != 1:
         x2 = x2.contiguous()
     if x2.shape[0] > 1 and x2.stride(0) < x2.shape[1]:

@@ -8,8 +8,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
-from ._lib import (GEMM_CIN_F32, GEMM_OUT_F32, GEMM_RELU, GEMM_ROWSUM_ACCUM, GEMM_STREAM_OUT, RTP_BF16, RTP_F32, GemmDesc,
-                   check)
+from ._lib import RTP_BF16, RTP_F32, check
 
 _DT = {torch.float32: RTP_F32, torch.bfloat16: RTP_BF16}
 
@@ -19,6 +18,20 @@ def dtype_code(dt: torch.dtype) -> int:
         return _DT[dt]
     except KeyError:
         raise TypeError(f"rtp_amd kernels support float32 and bfloat16, got {dt}") from None
+
+
+_native = None
+
+
+def native():
+    """The extension module behind every call here (csrc/host.cpp): entry points of the C ABI without their stream
+    argument -- the current stream is taken -- and gemm / linear_fwd / linear_bwd on keyword arguments and tensors.  Its
+    functions raise RtpError for a negative status.  The device is checked on first use."""
+    global _native
+    if _native is None:
+        _lib.require_device()
+        _native = _lib.native()
+    return _native
 
 
 def _stream() -> int:
@@ -43,16 +56,13 @@ def _mat(t: torch.Tensor, what: str):
     return t.shape[0], t.shape[1], max(ld, 1)
 
 
-def gemm_raw(dtype: torch.dtype, *, a: int, b: int, c_out: int, m: int, n: int, k: int, lda: int, ldb: int,
-             ldc: int, a_kcontig: bool, b_kcontig: bool, c_in: Optional[int] = None, ld_cin: int = 0,
-             bias: Optional[int] = None, gate: Optional[int] = None, ld_gate: int = 0, alpha: float = 1.0,
-             relu: bool = False, out_f32: bool = False, cin_f32: bool = False, batch: int = 1, zdiv: int = 1,
-             a_s=(0, 0), b_s=(0, 0), c_s=(0, 0), cin_s=(0, 0), gate_s=(0, 0), bias_s=(0, 0), groups: int = 1,
-             a_sg: int = 0, b_sg: int = 0, c_sg: int = 0, cin_sg: int = 0, gate_sg: int = 0, bias_sg: int = 0,
-             ksegs: int = 1, a_sk: int = 0, b_sk: int = 0, bias_sk: int = 0, stream_out: bool = False,
-             rowsum: Optional[int] = None, rowsum_sg: int = 0, rowsum_accum: bool = False,
-             sgd: Optional["FusedSgd"] = None, sgd_master: int = 0, sgd_weights: int = 0) -> bool:
-    """One rtp_gemm call on raw device addresses (see include/rtp_hip.h for the operand rules).
+def gemm_raw(dtype: torch.dtype, *, rowsum: Optional[int] = None, sgd: Optional["FusedSgd"] = None, sgd_master: int = 0,
+             sgd_weights: int = 0, **operands) -> bool:
+    """One rtp_gemm call on raw device addresses (see include/rtp_hip.h for the operand rules).  Operands: a, b, c_out,
+    m, n, k, lda, ldb, ldc, a_kcontig, b_kcontig, and optionally c_in, ld_cin, cin_f32, bias, gate, ld_gate, alpha, relu,
+    out_f32, stream_out, batch, zdiv, groups, ksegs, the (outer, inner) batch strides a_s, b_s, c_s, cin_s, gate_s, bias_s,
+    the group strides a_sg, b_sg, c_sg, cin_sg, gate_sg, bias_sg, the K-segment strides a_sk, b_sk, bias_sk, and rowsum_sg,
+    rowsum_accum.
 
     `sgd` (with the addresses of the fp32 parameters and of their compute-dtype copy that match c_out) asks for the
     clip + SGD update in the product's epilogue; if the library cannot fuse it for these operands the product runs
@@ -61,38 +71,13 @@ def gemm_raw(dtype: torch.dtype, *, a: int, b: int, c_out: int, m: int, n: int, 
     `rowsum` asks for the row sums of A (the bias gradient of a weight-gradient product) from the same launch.
     Returns whether they were produced: False means the library cannot fuse them for these operands, the
     product ran without them and the caller owes a separate column sum."""
-    _lib.require_device()
-    d = GemmDesc()
-    d.a, d.b, d.c_out, d.c_in, d.bias, d.gate = a, b, c_out, c_in, bias, gate
-    d.m, d.n, d.k = m, n, k
-    d.lda, d.ldb, d.ldc, d.ld_cin, d.ld_gate = lda, ldb, ldc, ld_cin, ld_gate
-    d.batch, d.zdiv = batch, zdiv
-    d.a_so, d.a_si = a_s
-    d.b_so, d.b_si = b_s
-    d.c_so, d.c_si = c_s
-    d.cin_so, d.cin_si = cin_s
-    d.gate_so, d.gate_si = gate_s
-    d.bias_so, d.bias_si = bias_s
-    d.groups, d.ksegs = groups, ksegs
-    d.a_sg, d.b_sg, d.c_sg, d.cin_sg, d.gate_sg, d.bias_sg = a_sg, b_sg, c_sg, cin_sg, gate_sg, bias_sg
-    d.a_sk, d.b_sk, d.bias_sk = a_sk, b_sk, bias_sk
-    d.alpha = alpha
-    d.flags = (GEMM_OUT_F32 if out_f32 else 0) | (GEMM_CIN_F32 if cin_f32 else 0) | (GEMM_RELU if relu else 0) | \
-        (GEMM_STREAM_OUT if stream_out else 0) | (GEMM_ROWSUM_ACCUM if rowsum_accum else 0)
-    d.a_kcontig, d.b_kcontig = int(a_kcontig), int(b_kcontig)
-    lib = _lib.load()
-    if sgd is not None:
-        if lib.rtp_gemm_sgd_fused(dtype_code(dtype), C.byref(d)):
-            d.sgd_master, d.sgd_weights = sgd_master, (sgd_weights or None)
-            d.sgd_lr, d.sgd_clip = sgd.lr, sgd.clip
-            if not sgd.keep_grads:
-                d.flags |= _lib.GEMM_SGD_SKIP_OUT
-        else:
-            sgd.missed = True
-    fused = rowsum is not None and bool(lib.rtp_gemm_rowsum_fused(dtype_code(dtype), C.byref(d)))
-    d.a_rowsum, d.rowsum_sg = (rowsum, rowsum_sg) if fused else (None, 0)
-    check(lib.rtp_gemm(_stream(), dtype_code(dtype), C.byref(d)))
-    return fused
+    if sgd is None:
+        return bool(native().gemm(dtype, rowsum=rowsum, **operands) & 1)
+    done = native().gemm(dtype, rowsum=rowsum, sgd_master=sgd_master, sgd_weights=sgd_weights or None, sgd_lr=sgd.lr,
+                         sgd_clip=sgd.clip, sgd_skip_out=not sgd.keep_grads, **operands)
+    if not done & 2:
+        sgd.missed = True
+    return bool(done & 1)
 
 
 def _rotated_layer(home: torch.Tensor, w_off: int, bias_off: Optional[int], n_s: int, k: int) -> "_lib.RotatedLinear":
@@ -107,16 +92,8 @@ def rotated_linear_fwd(x2: torch.Tensor, home: torch.Tensor, w_off: int, bias_of
                        y: torch.Tensor, relu: bool = False) -> None:
     """y[rows, shards * n_s] = x2 @ W_g^T + b_g for every shard g of `home` [shards, numel], one launch; y in the
     shards' dtype or fp32."""
-    layer = _rotated_layer(home, w_off, bias_off, n_s, k)
-    rows, kk, ldx = _mat(x2, "x")
-    ry, ny, ldy = _mat(y, "y")
-    if kk != k or ry != rows or ny < n_s * home.shape[0] or x2.dtype != home.dtype or \
-            y.dtype not in (home.dtype, torch.float32):
-        raise ValueError("rotated_linear_fwd: x [rows, k] in the shards' dtype, y [rows, >= shards * n_s] (or fp32)")
-    flags = (GEMM_RELU if relu else 0) | (GEMM_OUT_F32 if y.dtype != home.dtype else 0)
-    _lib.require_device()
-    check(_lib.load().rtp_rotated_linear_fwd(_stream(), dtype_code(home.dtype), C.byref(layer), x2.data_ptr(), ldx, rows,
-                                             y.data_ptr(), ldy, flags))
+    _dev(home)
+    native().linear_fwd(x2, home, w_off, bias_off, n_s, k, y, 0, relu)
 
 
 def rotated_linear_bwd(dy2: torch.Tensor, x2: Optional[torch.Tensor], home: torch.Tensor, w_off: int,
@@ -129,44 +106,12 @@ def rotated_linear_bwd(dy2: torch.Tensor, x2: Optional[torch.Tensor], home: torc
     has one), with the clip + SGD update `sgd` applied in the same launch to the fp32 parameters at address
     sgd_master and their compute-dtype copy at sgd_weights (both laid out like home).  Returns the library's
     done flags (ROTATED_BIAS_DONE, ROTATED_SGD_DONE): what is missing there is left to the caller."""
-    layer = _rotated_layer(home, w_off, bias_off, n_s, k)
-    rows, ny, ldy = _mat(dy2, "dy")
-    if ny < n_s * home.shape[0] or dy2.dtype != home.dtype:
-        raise ValueError("rotated_linear_bwd: dy must be [rows, >= shards * n_s] in the shards' dtype")
-    a = _lib.RotatedLinearBwdArgs()
-    done = C.c_int32(0)
-    a.done = C.pointer(done)
-    if dx is not None:
-        r, c, ld = _mat(dx, "dx")
-        if (r, c) != (rows, k):
-            raise ValueError("rotated_linear_bwd: dx must be [rows, k]")
-        a.dx, a.ld_dx = dx.data_ptr(), ld
-        for name, t in (("dx_init", dx_init), ("relu_gate", relu_gate)):
-            if t is not None:
-                r, c, ld = _mat(t, name)
-                if (r, c) != (rows, k):
-                    raise ValueError(f"rotated_linear_bwd: {name} must match dx")
-                setattr(a, name, t.data_ptr())
-                setattr(a, "ld_" + name, ld)
-        for t, what in ((dx, "dx"), (dx_init, "dx_init")):
-            if t is not None and t.dtype not in (home.dtype, torch.float32):
-                raise TypeError(f"rotated_linear_bwd: {what} must be {home.dtype} or float32")
-        if relu_gate is not None and relu_gate.dtype != home.dtype:
-            raise TypeError("rotated_linear_bwd: relu_gate must be in the shards' dtype")
-        a.dx_flags = (GEMM_OUT_F32 if dx.dtype != home.dtype else 0) | \
-            (GEMM_CIN_F32 if dx_init is not None and dx_init.dtype != home.dtype else 0)
-    if grads is not None:
-        if grads.shape != home.shape or grads.dtype != home.dtype or not grads.is_contiguous() or x2 is None:
-            raise ValueError("rotated_linear_bwd: grads must be laid out like home, and the layer's input is needed")
-        a.grads, a.accumulate = grads.data_ptr(), int(accumulate)
-        if sgd is not None:
-            a.sgd_master, a.sgd_weights = sgd_master, (sgd_weights or None)
-            a.sgd_lr, a.sgd_clip, a.sgd_skip_grad_store = sgd.lr, sgd.clip, int(not sgd.keep_grads)
-    xr = _mat(x2, "x") if x2 is not None else (rows, k, k)
-    _lib.require_device()
-    check(_lib.load().rtp_rotated_linear_bwd(_stream(), dtype_code(home.dtype), C.byref(layer), dy2.data_ptr(), ldy,
-                                             _ptr(x2), xr[2], rows, C.byref(a)))
-    return done.value
+    _dev(home)
+    if sgd is None:
+        return native().linear_bwd(dy2, 0, x2, home, w_off, bias_off, n_s, k, dx, dx_init, relu_gate, grads, accumulate, None,
+                                   None, 0.0, 0.0, False)
+    return native().linear_bwd(dy2, 0, x2, home, w_off, bias_off, n_s, k, dx, dx_init, relu_gate, grads, accumulate,
+                               sgd_master, sgd_weights or None, sgd.lr, sgd.clip, not sgd.keep_grads)
 
 
 def rotated_linear_xent_fwd(x2: torch.Tensor, home: torch.Tensor, w_off: int, bias_off: Optional[int], n_s: int, k: int,
@@ -180,11 +125,11 @@ def rotated_linear_xent_fwd(x2: torch.Tensor, home: torch.Tensor, w_off: int, bi
     if target.dtype != torch.int64 or target.numel() != rows or not target.is_contiguous() or target.device != x2.device:
         raise ValueError("rotated_linear_xent_fwd: target must be contiguous int64 [rows] on the device")
     lib = _lib.load()
+    _lib.require_device()
     nbytes = lib.rtp_rotated_linear_xent_workspace_bytes(C.byref(layer), rows)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=x2.device)
     loss = torch.empty(rows, dtype=torch.float32, device=x2.device)
     stats = torch.empty(rows, 2, dtype=torch.float32, device=x2.device)
-    _lib.require_device()
     check(lib.rtp_rotated_linear_xent_fwd(_stream(), dtype_code(home.dtype), C.byref(layer), x2.data_ptr(), ldx, rows,
                                           target.data_ptr(), int(ignore_index), loss.data_ptr(), stats.data_ptr(),
                                           ws.data_ptr(), nbytes))
@@ -202,7 +147,6 @@ def rotated_linear_xent_bwd(x2: torch.Tensor, home: torch.Tensor, w_off: int, bi
             not stats.is_contiguous() or dloss.dtype != torch.float32 or dloss.numel() != 1:
         raise ValueError("rotated_linear_xent_bwd: x [rows, k], stats fp32 [rows, 2], dloss one fp32 element")
     out = torch.empty(rows, n_s * home.shape[0], dtype=home.dtype, device=x2.device)
-    _lib.require_device()
     check(_lib.load().rtp_rotated_linear_xent_bwd(_stream(), dtype_code(home.dtype), C.byref(layer), x2.data_ptr(), ldx,
                                                   rows, target.data_ptr(), int(ignore_index), stats.data_ptr(),
                                                   dloss.data_ptr(), _ptr(scale), out.data_ptr(), out.stride(0)))
@@ -292,12 +236,10 @@ def colsum(x: torch.Tensor, out: torch.Tensor, accumulate: bool = False, seg: in
         raise ValueError("colsum: width must be a multiple of seg and seg_stride >= seg")
     if out.dtype not in (x.dtype, torch.float32):
         raise TypeError("colsum: out must be the input dtype or float32")
-    _lib.require_device()
-    lib = _lib.load()
-    nbytes = lib.rtp_colsum_workspace_bytes(m, n)
+    nbytes = native().rtp_colsum_workspace_bytes(m, n)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-    check(lib.rtp_colsum(_stream(), dtype_code(x.dtype), x.data_ptr(), m, n, ld, out.data_ptr(),
-                         int(out.dtype == torch.float32), int(accumulate), seg, seg_stride, ws.data_ptr(), nbytes))
+    native().rtp_colsum(dtype_code(x.dtype), x.data_ptr(), m, n, ld, out.data_ptr(), int(out.dtype == torch.float32),
+                        int(accumulate), seg, seg_stride, ws.data_ptr(), nbytes)
 
 
 def shard_copy(dst: torch.Tensor, src: torch.Tensor) -> None:
@@ -307,17 +249,14 @@ def shard_copy(dst: torch.Tensor, src: torch.Tensor) -> None:
     if not (dst.is_contiguous() and src.is_contiguous()) or dst.numel() * dst.element_size() != \
             src.numel() * src.element_size():
         raise ValueError("shard_copy: need contiguous tensors of equal byte size")
-    _lib.require_device()
-    check(_lib.load().rtp_shard_copy_async(_stream(), dst.data_ptr(), src.data_ptr(),
-                                           src.numel() * src.element_size()))
+    native().rtp_shard_copy_async(dst.data_ptr(), src.data_ptr(), src.numel() * src.element_size())
 
 
 def zero_(t: torch.Tensor) -> None:
     _dev(t)
     if not t.is_contiguous():
         raise ValueError("zero_: need a contiguous tensor")
-    _lib.require_device()
-    check(_lib.load().rtp_zero_async(_stream(), t.data_ptr(), t.numel() * t.element_size()))
+    native().rtp_zero_async(t.data_ptr(), t.numel() * t.element_size())
 
 
 def embedding_gather(table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor, row_begin: int = 0, groups: int = 1,
@@ -334,21 +273,19 @@ def embedding_gather(table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor, 
     if ids.dtype != torch.int64 or not ids.is_contiguous() or ids.numel() != n or cols_o != cols or \
             out.dtype != table.dtype:
         raise ValueError("embedding_gather: ids must be contiguous int64 with one id per output row")
-    _lib.require_device()
     if pos is not None:
         _dev(pos)
         p_rows, p_cols, ld_p = _mat(pos, "pos")
         if pos.dtype != table.dtype or p_cols != cols or batch < 1 or (n + batch - 1) // batch > p_rows:
             raise ValueError("embedding_gather: pos must hold one row of the table's dtype per position")
-        check(_lib.load().rtp_embedding_gather_scale_pos(
-            _stream(), dtype_code(table.dtype), table.data_ptr(), ld_t, row_begin, rows, cols, ids.data_ptr(), n,
-            out.data_ptr(), ld_o, groups, table_sg, out_sg, float(scale), pos.data_ptr(), ld_p, pos_sg, batch))
+        native().rtp_embedding_gather_scale_pos(dtype_code(table.dtype), table.data_ptr(), ld_t, row_begin, rows, cols,
+                                                ids.data_ptr(), n, out.data_ptr(), ld_o, groups, table_sg, out_sg,
+                                                float(scale), pos.data_ptr(), ld_p, pos_sg, batch)
         return
     if scale != 1.0:
         raise ValueError("embedding_gather: a scale needs the positional table")
-    check(_lib.load().rtp_embedding_gather(_stream(), dtype_code(table.dtype), table.data_ptr(), ld_t, row_begin,
-                                           rows, cols, ids.data_ptr(), n, out.data_ptr(), ld_o, groups, table_sg,
-                                           out_sg))
+    native().rtp_embedding_gather(dtype_code(table.dtype), table.data_ptr(), ld_t, row_begin, rows, cols,
+                                  ids.data_ptr(), n, out.data_ptr(), ld_o, groups, table_sg, out_sg)
 
 
 def embedding_sort_ids(ids: torch.Tensor) -> torch.Tensor:
@@ -356,17 +293,15 @@ def embedding_sort_ids(ids: torch.Tensor) -> torch.Tensor:
     _dev(ids)
     if ids.dtype != torch.int64 or not ids.is_contiguous():
         raise ValueError("embedding_sort_ids: ids must be contiguous int64")
-    _lib.require_device()
-    lib = _lib.load()
-    nbytes = lib.rtp_embedding_scatter_workspace_bytes(ids.numel())
+    nbytes = native().rtp_embedding_scatter_workspace_bytes(ids.numel())
     ws = torch.empty(nbytes, dtype=torch.uint8, device=ids.device)
-    check(lib.rtp_embedding_sort_ids(_stream(), ids.data_ptr(), ids.numel(), ws.data_ptr(), nbytes))
+    native().rtp_embedding_sort_ids(ids.data_ptr(), ids.numel(), ws.data_ptr(), nbytes)
     return ws
 
 
 def embedding_backward_supported(n_ids: int) -> bool:
     """Whether a step of n_ids tokens fits the one-launch embedding backward (its ids are staged in LDS)."""
-    return bool(_lib.load().rtp_embedding_backward_supported(int(n_ids)))
+    return bool(_lib.native().rtp_embedding_backward_supported(int(n_ids)))
 
 
 def embedding_backward(grad_out: torch.Tensor, ids: torch.Tensor, grad_table: torch.Tensor, *, row_begin: int = 0,
@@ -387,14 +322,14 @@ def embedding_backward(grad_out: torch.Tensor, ids: torch.Tensor, grad_table: to
     if sgd is not None and (not zero_fill or grad_table.dtype != grad_out.dtype):
         raise ValueError("embedding_backward: the fused update takes the whole gradient of the step, in the table's "
                          "own dtype")
-    _lib.require_device()
-    check(_lib.load().rtp_embedding_backward(
-        _stream(), dtype_code(grad_out.dtype), grad_out.data_ptr(), ld_go, n, ids.data_ptr(), grad_table.data_ptr(),
-        ld_gt, int(grad_table.dtype == torch.float32), row_begin, rows, cols,
-        -1 if padding_idx is None else padding_idx, int(scale_by_freq), int(zero_fill), groups, grad_out_sg,
-        grad_table_sg, float(grad_scale), (sgd_master or None) if sgd is not None else None,
-        (sgd_weights or None) if sgd is not None else None, sgd.lr if sgd is not None else 0.0,
-        sgd.clip if sgd is not None else 0.0, int(sgd.keep_grads) if sgd is not None else 1))
+    native().rtp_embedding_backward(dtype_code(grad_out.dtype), grad_out.data_ptr(), ld_go, n, ids.data_ptr(),
+                                    grad_table.data_ptr(), ld_gt, int(grad_table.dtype == torch.float32), row_begin,
+                                    rows, cols, -1 if padding_idx is None else padding_idx, int(scale_by_freq),
+                                    int(zero_fill), groups, grad_out_sg, grad_table_sg, float(grad_scale),
+                                    (sgd_master or None) if sgd is not None else None,
+                                    (sgd_weights or None) if sgd is not None else None,
+                                    sgd.lr if sgd is not None else 0.0, sgd.clip if sgd is not None else 0.0,
+                                    int(sgd.keep_grads) if sgd is not None else 1)
 
 
 def embedding_scatter_add(grad_out: torch.Tensor, n_ids: int, workspace: torch.Tensor, grad_table: torch.Tensor,
@@ -418,8 +353,7 @@ def embedding_scatter_add(grad_out: torch.Tensor, n_ids: int, workspace: torch.T
         raise ValueError("embedding_scatter_add: shape mismatch")
     if grad_table.dtype not in (grad_out.dtype, torch.float32):
         raise TypeError("embedding_scatter_add: grad_table must be the grad dtype or float32")
-    _lib.require_device()
-    args = (_stream(), dtype_code(grad_out.dtype), grad_out.data_ptr(), ld_go, n_ids, workspace.data_ptr(),
+    args = (dtype_code(grad_out.dtype), grad_out.data_ptr(), ld_go, n_ids, workspace.data_ptr(),
             grad_table.data_ptr(), ld_gt, int(grad_table.dtype == torch.float32), row_begin, rows, cols,
             -1 if padding_idx is None else padding_idx, int(scale_by_freq), int(zero_fill), groups, grad_out_sg,
             grad_table_sg)
@@ -427,16 +361,16 @@ def embedding_scatter_add(grad_out: torch.Tensor, n_ids: int, workspace: torch.T
         if not zero_fill or grad_table.dtype != grad_out.dtype:
             raise ValueError("embedding_scatter_add: the fused update takes the whole gradient of the step, in the "
                              "table's own dtype")
-        check(_lib.load().rtp_embedding_scatter_add_sgd(
-            _stream(), dtype_code(grad_out.dtype), grad_out.data_ptr(), ld_go, n_ids, workspace.data_ptr(),
-            grad_table.data_ptr(), ld_gt, row_begin, rows, cols, -1 if padding_idx is None else padding_idx,
-            int(scale_by_freq), groups, grad_out_sg, grad_table_sg, float(grad_scale), sgd_master, sgd_weights or None,
-            sgd.lr, sgd.clip, int(sgd.keep_grads)))
+        native().rtp_embedding_scatter_add_sgd(dtype_code(grad_out.dtype), grad_out.data_ptr(), ld_go, n_ids,
+                                               workspace.data_ptr(), grad_table.data_ptr(), ld_gt, row_begin, rows,
+                                               cols, -1 if padding_idx is None else padding_idx, int(scale_by_freq),
+                                               groups, grad_out_sg, grad_table_sg, float(grad_scale), sgd_master,
+                                               sgd_weights or None, sgd.lr, sgd.clip, int(sgd.keep_grads))
         return
     if grad_scale != 1.0:
-        check(_lib.load().rtp_embedding_scatter_add_scaled(*args, float(grad_scale)))
+        native().rtp_embedding_scatter_add_scaled(*args, float(grad_scale))
     else:
-        check(_lib.load().rtp_embedding_scatter_add_det(*args))
+        native().rtp_embedding_scatter_add_det(*args)
 
 
 def _key_bias_ptr(who: str, key_bias: Optional[torch.Tensor], n_batch: int, keys: int):
@@ -479,15 +413,14 @@ def softmax_fwd(scores: torch.Tensor, p: torch.Tensor, *, mask: Optional[torch.T
                 raise ValueError(f"softmax_fwd: {masks} masks do not divide {z} problems")
     n_batch = key_bias.shape[0] if key_bias is not None else 1
     kb = _key_bias_ptr("softmax_fwd", key_bias, n_batch, s)
-    _lib.require_device()
     if (keep is None) != (p_dropped is None):
         raise ValueError("softmax_fwd: keep and p_dropped go together")
     if p_dropped is not None and (p_dropped.shape != p.shape or p_dropped.dtype != p.dtype or
                                   not p_dropped.is_contiguous()):
         raise ValueError("softmax_fwd: p_dropped must match p")
-    check(_lib.load().rtp_softmax_fwd_masks(_stream(), dtype_code(p.dtype), scores.data_ptr(), _ptr(mask), masks, kb,
-                                            n_batch, heads, int(causal), scale, z, l, s, p.data_ptr(),
-                                            _keep_ptr("softmax_fwd", keep, p), _ptr(p_dropped)))
+    native().rtp_softmax_fwd_masks(dtype_code(p.dtype), scores.data_ptr(), _ptr(mask), masks, kb, n_batch, heads,
+                                   int(causal), scale, z, l, s, p.data_ptr(), _keep_ptr("softmax_fwd", keep, p),
+                                   _ptr(p_dropped))
 
 
 def softmax_bwd(p: torch.Tensor, dp: torch.Tensor, ds: torch.Tensor, scale: float,
@@ -498,16 +431,15 @@ def softmax_bwd(p: torch.Tensor, dp: torch.Tensor, ds: torch.Tensor, scale: floa
             ds.dtype != p.dtype or not (p.is_contiguous() and dp.is_contiguous() and ds.is_contiguous()):
         raise ValueError("softmax_bwd: need contiguous p/ds [Z,L,S] of one dtype and fp32 dp")
     z, l, s = p.shape
-    _lib.require_device()
-    check(_lib.load().rtp_softmax_bwd(_stream(), dtype_code(p.dtype), p.data_ptr(), dp.data_ptr(),
-                                      _keep_ptr("softmax_bwd", keep, p), scale, z, l, s, ds.data_ptr()))
+    native().rtp_softmax_bwd(dtype_code(p.dtype), p.data_ptr(), dp.data_ptr(), _keep_ptr("softmax_bwd", keep, p),
+                             scale, z, l, s, ds.data_ptr())
 
 
 def attn_supported(dtype: torch.dtype, L: int, d: int) -> bool:
     """Whether the fused short-sequence attention core handles this shape (bf16, L <= 32, d in {32, 64, 128})."""
     if dtype != torch.bfloat16:
         return False
-    return bool(_lib.load().rtp_attn_supported(dtype_code(dtype), L, d))
+    return bool(_lib.native().rtp_attn_supported(dtype_code(dtype), L, d))
 
 
 def attn_fwd(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, qkv_strides, o: torch.Tensor, o_off: int,
@@ -521,12 +453,11 @@ def attn_fwd(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, qkv_strides,
         raise ValueError("attn_fwd: p must be contiguous [G*N*H, L, L] of the operand dtype")
     if mask is not None and (mask.dtype != torch.float32 or tuple(mask.shape) != (L, L) or not mask.is_contiguous()):
         raise ValueError("attn_fwd: mask must be a contiguous fp32 [L, L] tensor")
-    _lib.require_device()
     base = qkv.data_ptr()
-    check(_lib.load().rtp_attn_fwd(_stream(), dtype_code(qkv.dtype), base + q_off * esz, base + k_off * esz,
-                                   base + v_off * esz, *qkv_strides, o.data_ptr() + o_off * esz, *o_strides,
-                                   p.data_ptr(), mask.data_ptr() if mask is not None else None,
-                                   _key_bias_ptr("attn_fwd", key_bias, N, L), int(causal), scale, L, N, H, d, G))
+    native().rtp_attn_fwd(dtype_code(qkv.dtype), base + q_off * esz, base + k_off * esz, base + v_off * esz,
+                          *qkv_strides, o.data_ptr() + o_off * esz, *o_strides, p.data_ptr(),
+                          mask.data_ptr() if mask is not None else None, _key_bias_ptr("attn_fwd", key_bias, N, L),
+                          int(causal), scale, L, N, H, d, G)
 
 
 def attn_bwd(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, qkv_strides, dout: torch.Tensor, o_off: int,
@@ -537,19 +468,17 @@ def attn_bwd(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, qkv_strides,
     esz = qkv.element_size()
     if dqkv.dtype != qkv.dtype or dqkv.shape != qkv.shape or dqkv.stride() != qkv.stride() or dout.dtype != qkv.dtype:
         raise ValueError("attn_bwd: dqkv must match qkv, dout must share its dtype")
-    _lib.require_device()
     base, dbase = qkv.data_ptr(), dqkv.data_ptr()
-    check(_lib.load().rtp_attn_bwd(_stream(), dtype_code(qkv.dtype), base + q_off * esz, base + k_off * esz,
-                                   base + v_off * esz, *qkv_strides, dout.data_ptr() + o_off * esz, *o_strides,
-                                   p.data_ptr(), dbase + q_off * esz, dbase + k_off * esz, dbase + v_off * esz, scale,
-                                   L, N, H, d, G))
+    native().rtp_attn_bwd(dtype_code(qkv.dtype), base + q_off * esz, base + k_off * esz, base + v_off * esz,
+                          *qkv_strides, dout.data_ptr() + o_off * esz, *o_strides, p.data_ptr(), dbase + q_off * esz,
+                          dbase + k_off * esz, dbase + v_off * esz, scale, L, N, H, d, G)
 
 
 def attn_flash_supported(dtype: torch.dtype, L: int, d: int) -> bool:
     """Whether the running-softmax attention core handles this shape (bf16, any L, d in {32, 64, 128})."""
     if dtype != torch.bfloat16:
         return False
-    return bool(_lib.load().rtp_attn_flash_supported(dtype_code(dtype), L, d))
+    return bool(_lib.native().rtp_attn_flash_supported(dtype_code(dtype), L, d))
 
 
 def _flash_rows(name: str, t: torch.Tensor, G: int, N: int, H: int, L: int) -> None:
@@ -576,12 +505,10 @@ def attn_flash_fwd(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, qkv_st
         raise ValueError("attn_flash_fwd: o must share the operand dtype")
     _flash_rows("attn_flash_fwd: lse", lse, G, N, H, L)
     mask_ptr = _flash_mask(mask, L)
-    _lib.require_device()
     base = qkv.data_ptr()
-    check(_lib.load().rtp_attn_flash_fwd(_stream(), dtype_code(qkv.dtype), base + q_off * esz, base + k_off * esz,
-                                         base + v_off * esz, *qkv_strides, o.data_ptr() + o_off * esz, *o_strides,
-                                         lse.data_ptr(), mask_ptr, _key_bias_ptr("attn_flash_fwd", key_bias, N, L),
-                                         int(causal), scale, L, N, H, d, G))
+    native().rtp_attn_flash_fwd(dtype_code(qkv.dtype), base + q_off * esz, base + k_off * esz, base + v_off * esz,
+                                *qkv_strides, o.data_ptr() + o_off * esz, *o_strides, lse.data_ptr(), mask_ptr,
+                                _key_bias_ptr("attn_flash_fwd", key_bias, N, L), int(causal), scale, L, N, H, d, G)
 
 
 def attn_flash_bwd(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, qkv_strides, o: torch.Tensor,
@@ -599,20 +526,18 @@ def attn_flash_bwd(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, qkv_st
     _flash_rows("attn_flash_bwd: lse", lse, G, N, H, L)
     _flash_rows("attn_flash_bwd: delta", delta, G, N, H, L)
     mask_ptr = _flash_mask(mask, L)
-    _lib.require_device()
     base, dbase = qkv.data_ptr(), dqkv.data_ptr()
-    check(_lib.load().rtp_attn_flash_bwd(_stream(), dtype_code(qkv.dtype), base + q_off * esz, base + k_off * esz,
-                                         base + v_off * esz, *qkv_strides, o.data_ptr() + o_off * esz,
-                                         dout.data_ptr() + o_off * esz, *o_strides, lse.data_ptr(), delta.data_ptr(),
-                                         dbase + q_off * esz, dbase + k_off * esz, dbase + v_off * esz, mask_ptr,
-                                         _key_bias_ptr("attn_flash_bwd", key_bias, N, L), int(causal), scale, L, N, H,
-                                         d, G))
+    native().rtp_attn_flash_bwd(dtype_code(qkv.dtype), base + q_off * esz, base + k_off * esz, base + v_off * esz,
+                                *qkv_strides, o.data_ptr() + o_off * esz, dout.data_ptr() + o_off * esz, *o_strides,
+                                lse.data_ptr(), delta.data_ptr(), dbase + q_off * esz, dbase + k_off * esz,
+                                dbase + v_off * esz, mask_ptr, _key_bias_ptr("attn_flash_bwd", key_bias, N, L),
+                                int(causal), scale, L, N, H, d, G)
 
 
 def layernorm_supported(dtype: torch.dtype, cols: int) -> bool:
     if dtype not in (torch.float32, torch.bfloat16):
         return False
-    return bool(_lib.load().rtp_layernorm_supported(dtype_code(dtype), cols))
+    return bool(_lib.native().rtp_layernorm_supported(dtype_code(dtype), cols))
 
 
 def add_layernorm_fwd(x: torch.Tensor, r: Optional[torch.Tensor], gamma: torch.Tensor, beta: Optional[torch.Tensor],
@@ -630,11 +555,10 @@ def add_layernorm_fwd(x: torch.Tensor, r: Optional[torch.Tensor], gamma: torch.T
         raise ValueError("add_layernorm_fwd: gamma / beta must be vectors of the row length in x's dtype")
     if mean.dtype != torch.float32 or rstd.dtype != torch.float32 or mean.numel() != rows or rstd.numel() != rows:
         raise ValueError("add_layernorm_fwd: mean / rstd must be fp32 [rows]")
-    _lib.require_device()
-    check(_lib.load().rtp_add_layernorm_fwd(
-        _stream(), dtype_code(x.dtype), x.data_ptr(), r.data_ptr() if r is not None else None, gamma.data_ptr(),
-        beta.data_ptr() if beta is not None else None, eps, rows, cols, z.data_ptr() if z is not None else None,
-        y.data_ptr(), mean.data_ptr(), rstd.data_ptr()))
+    native().rtp_add_layernorm_fwd(dtype_code(x.dtype), x.data_ptr(), r.data_ptr() if r is not None else None,
+                                   gamma.data_ptr(), beta.data_ptr() if beta is not None else None, eps, rows, cols,
+                                   z.data_ptr() if z is not None else None, y.data_ptr(), mean.data_ptr(),
+                                   rstd.data_ptr())
 
 
 def layernorm_bwd(dy: torch.Tensor, z: torch.Tensor, gamma: torch.Tensor, mean: torch.Tensor, rstd: torch.Tensor,
@@ -645,13 +569,11 @@ def layernorm_bwd(dy: torch.Tensor, z: torch.Tensor, gamma: torch.Tensor, mean: 
     if any(t.dtype != z.dtype or t.shape != z.shape or not t.is_contiguous() for t in (dy, dz)) or \
             not z.is_contiguous():
         raise ValueError("layernorm_bwd: dy, z, dz must be contiguous, of one shape and dtype")
-    _lib.require_device()
-    lib = _lib.load()
-    nbytes = lib.rtp_layernorm_bwd_workspace_bytes(rows, cols)
+    nbytes = native().rtp_layernorm_bwd_workspace_bytes(rows, cols)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=z.device)
-    check(lib.rtp_layernorm_bwd(_stream(), dtype_code(z.dtype), dy.data_ptr(), z.data_ptr(), gamma.data_ptr(),
-                                mean.data_ptr(), rstd.data_ptr(), rows, cols, dz.data_ptr(), dgamma.data_ptr(),
-                                dbeta.data_ptr() if dbeta is not None else None, ws.data_ptr(), nbytes))
+    native().rtp_layernorm_bwd(dtype_code(z.dtype), dy.data_ptr(), z.data_ptr(), gamma.data_ptr(), mean.data_ptr(),
+                               rstd.data_ptr(), rows, cols, dz.data_ptr(), dgamma.data_ptr(),
+                               dbeta.data_ptr() if dbeta is not None else None, ws.data_ptr(), nbytes)
 
 
 def layernorm_bwd_deferred(dy: torch.Tensor, z: torch.Tensor, gamma: torch.Tensor, mean: torch.Tensor,
@@ -664,14 +586,11 @@ def layernorm_bwd_deferred(dy: torch.Tensor, z: torch.Tensor, gamma: torch.Tenso
     if any(t.dtype != z.dtype or t.shape != z.shape or not t.is_contiguous() for t in (dy, dz)) or \
             not z.is_contiguous():
         raise ValueError("layernorm_bwd_deferred: dy, z, dz must be contiguous, of one shape and dtype")
-    _lib.require_device()
-    lib = _lib.load()
-    nbytes = lib.rtp_layernorm_bwd_workspace_bytes(rows, cols)
+    nbytes = native().rtp_layernorm_bwd_workspace_bytes(rows, cols)
     if part is None or part.numel() < nbytes or part.device != z.device:
         part = torch.empty(nbytes, dtype=torch.uint8, device=z.device)
-    check(lib.rtp_layernorm_bwd(_stream(), dtype_code(z.dtype), dy.data_ptr(), z.data_ptr(), gamma.data_ptr(),
-                                mean.data_ptr(), rstd.data_ptr(), rows, cols, dz.data_ptr(), None, None,
-                                part.data_ptr(), part.numel()))
+    native().rtp_layernorm_bwd(dtype_code(z.dtype), dy.data_ptr(), z.data_ptr(), gamma.data_ptr(), mean.data_ptr(),
+                               rstd.data_ptr(), rows, cols, dz.data_ptr(), None, None, part.data_ptr(), part.numel())
     return part
 
 
@@ -686,10 +605,9 @@ def _device_table(rows, device) -> torch.Tensor:
 
 def layernorm_final_table(items, device) -> torch.Tensor:
     """Device table for layernorm_finalize: items = [(part, rows, cols, dgamma, dbeta or None), ...]."""
-    lib = _lib.load()
     rows = []
     for part, n_rows, cols, dgamma, dbeta in items:
-        rows.append([part.data_ptr(), lib.rtp_layernorm_bwd_blocks(n_rows), cols, dgamma.data_ptr(),
+        rows.append([part.data_ptr(), native().rtp_layernorm_bwd_blocks(n_rows), cols, dgamma.data_ptr(),
                      dbeta.data_ptr() if dbeta is not None else 0])
     return _device_table(rows, device)
 
@@ -697,9 +615,7 @@ def layernorm_final_table(items, device) -> torch.Tensor:
 def layernorm_finalize(table: torch.Tensor, dtype: torch.dtype, max_cols: int) -> None:
     """dgamma / dbeta of every LayerNorm in `table` from its partial sums, one launch."""
     _dev(table)
-    _lib.require_device()
-    check(_lib.load().rtp_layernorm_bwd_finalize(_stream(), dtype_code(dtype), table.data_ptr(), table.shape[0],
-                                                 max_cols))
+    native().rtp_layernorm_bwd_finalize(dtype_code(dtype), table.data_ptr(), table.shape[0], max_cols)
 
 
 def _xent_check(who: str, logits: torch.Tensor, target: torch.Tensor) -> None:
@@ -721,10 +637,8 @@ def softmax_xent_fwd(logits: torch.Tensor, target: torch.Tensor,
     rows, cols = logits.shape
     loss = torch.empty(rows, dtype=torch.float32, device=logits.device)
     stats = torch.empty((rows, 2), dtype=torch.float32, device=logits.device)
-    _lib.require_device()
-    check(_lib.load().rtp_softmax_xent_fwd(_stream(), dtype_code(logits.dtype), logits.data_ptr(),
-                                           logits.stride(0) if rows > 1 else cols, rows, cols, target.data_ptr(),
-                                           int(ignore_index), loss.data_ptr(), stats.data_ptr()))
+    native().rtp_softmax_xent_fwd(dtype_code(logits.dtype), logits.data_ptr(), logits.stride(0) if rows > 1 else cols,
+                                  rows, cols, target.data_ptr(), int(ignore_index), loss.data_ptr(), stats.data_ptr())
     return loss, stats
 
 
@@ -737,9 +651,8 @@ def softmax_xent_reduce(loss_rows: torch.Tensor, target: torch.Tensor, ignore_in
         raise ValueError("softmax_xent_reduce: loss_rows must be contiguous fp32 [rows] and target int64 [rows]")
     out = torch.empty((), dtype=torch.float32, device=loss_rows.device)
     scale = torch.empty(1, dtype=torch.float32, device=loss_rows.device)
-    _lib.require_device()
-    check(_lib.load().rtp_softmax_xent_reduce(_stream(), loss_rows.data_ptr(), target.data_ptr(), int(ignore_index),
-                                              loss_rows.numel(), int(mean), out.data_ptr(), scale.data_ptr()))
+    native().rtp_softmax_xent_reduce(loss_rows.data_ptr(), target.data_ptr(), int(ignore_index), loss_rows.numel(),
+                                     int(mean), out.data_ptr(), scale.data_ptr())
     return out, scale
 
 
@@ -764,12 +677,10 @@ def softmax_xent_bwd(logits: torch.Tensor, target: torch.Tensor, stats: torch.Te
         out = torch.empty(rows, cols, dtype=logits.dtype, device=logits.device)
     elif out.shape != logits.shape or out.dtype != logits.dtype or (cols > 1 and out.stride(1) != 1):
         raise ValueError("softmax_xent_bwd: out must match the logits' shape and dtype")
-    _lib.require_device()
-    check(_lib.load().rtp_softmax_xent_bwd(_stream(), dtype_code(logits.dtype), logits.data_ptr(),
-                                           logits.stride(0) if rows > 1 else cols, rows, cols, target.data_ptr(),
-                                           int(ignore_index), stats.data_ptr(), dloss.data_ptr(),
-                                           0 if rows <= 1 else stride,
-                                           _ptr(scale), out.data_ptr(), out.stride(0) if rows > 1 else cols))
+    native().rtp_softmax_xent_bwd(dtype_code(logits.dtype), logits.data_ptr(), logits.stride(0) if rows > 1 else cols,
+                                  rows, cols, target.data_ptr(), int(ignore_index), stats.data_ptr(), dloss.data_ptr(),
+                                  0 if rows <= 1 else stride, _ptr(scale), out.data_ptr(),
+                                  out.stride(0) if rows > 1 else cols)
     return out
 
 
@@ -782,9 +693,8 @@ def sgd_step(master: torch.Tensor, grad: torch.Tensor, shadow: Optional[torch.Te
     if shadow is not None and (shadow.dtype != grad.dtype or shadow.numel() != master.numel() or
                                not shadow.is_contiguous()):
         raise ValueError("sgd_step: shadow must match grad dtype and master length")
-    _lib.require_device()
-    check(_lib.load().rtp_sgd_step(_stream(), dtype_code(grad.dtype), master.data_ptr(), grad.data_ptr(),
-                                   _ptr(shadow), master.numel(), lr, clip))
+    native().rtp_sgd_step(dtype_code(grad.dtype), master.data_ptr(), grad.data_ptr(), _ptr(shadow), master.numel(), lr,
+                          clip)
 
 
 def gate_supported(x2: torch.Tensor, w_rows: torch.Tensor) -> bool:
@@ -794,7 +704,7 @@ def gate_supported(x2: torch.Tensor, w_rows: torch.Tensor) -> bool:
         return False
     vec = 16 // x2.element_size()
     ok = all(t.stride(1) == 1 and t.stride(0) % vec == 0 and t.data_ptr() % 16 == 0 for t in (x2, w_rows))
-    return ok and bool(_lib.load().rtp_gate_supported(dtype_code(x2.dtype), w_rows.shape[0], x2.shape[1]))
+    return ok and bool(_lib.native().rtp_gate_supported(dtype_code(x2.dtype), w_rows.shape[0], x2.shape[1]))
 
 
 def gate_fwd(x2: torch.Tensor, w_rows: torch.Tensor, logits: torch.Tensor, col0: int) -> None:
@@ -803,10 +713,8 @@ def gate_fwd(x2: torch.Tensor, w_rows: torch.Tensor, logits: torch.Tensor, col0:
     if logits.dtype != torch.float32 or logits.stride(1) != 1 or logits.shape[0] != x2.shape[0] or \
             col0 + w_rows.shape[0] > logits.shape[1]:
         raise ValueError("gate_fwd: logits must be fp32 [S, >= col0 + E]")
-    _lib.require_device()
-    check(_lib.load().rtp_gate_fwd(_stream(), dtype_code(x2.dtype), x2.data_ptr(), x2.stride(0), w_rows.data_ptr(),
-                                   w_rows.stride(0), x2.shape[0], x2.shape[1], w_rows.shape[0],
-                                   logits.data_ptr() + 4 * col0, logits.stride(0)))
+    native().rtp_gate_fwd(dtype_code(x2.dtype), x2.data_ptr(), x2.stride(0), w_rows.data_ptr(), w_rows.stride(0),
+                          x2.shape[0], x2.shape[1], w_rows.shape[0], logits.data_ptr() + 4 * col0, logits.stride(0))
 
 
 def gate_dgrad(d_logits: torch.Tensor, col0: int, w_rows: torch.Tensor, dx: torch.Tensor,
@@ -820,11 +728,9 @@ def gate_dgrad(d_logits: torch.Tensor, col0: int, w_rows: torch.Tensor, dx: torc
     if d_logits.dtype != torch.float32 or d_logits.stride(1) != 1 or dx.dtype != w_rows.dtype or dx.stride(1) != 1 or \
             d_logits.shape[0] != dx.shape[0] or dx.shape[1] != w_rows.shape[1]:
         raise ValueError("gate_dgrad: need fp32 d_logits [S, E] and dx [S, M] of the weights' dtype")
-    _lib.require_device()
-    check(_lib.load().rtp_gate_dgrad(_stream(), dtype_code(dx.dtype), d_logits.data_ptr() + 4 * col0, d_logits.stride(0),
-                                     w_rows.data_ptr(), w_rows.stride(0), dx.shape[0], dx.shape[1], w_rows.shape[0],
-                                     dx.data_ptr(), dx.stride(0), _ptr(init),
-                                     init.stride(0) if init is not None else 0))
+    native().rtp_gate_dgrad(dtype_code(dx.dtype), d_logits.data_ptr() + 4 * col0, d_logits.stride(0),
+                            w_rows.data_ptr(), w_rows.stride(0), dx.shape[0], dx.shape[1], w_rows.shape[0],
+                            dx.data_ptr(), dx.stride(0), _ptr(init), init.stride(0) if init is not None else 0)
 
 
 def gate_wgrad(d_logits: torch.Tensor, col0: int, x2: torch.Tensor, dw_rows: torch.Tensor, accumulate: bool) -> None:
@@ -834,13 +740,11 @@ def gate_wgrad(d_logits: torch.Tensor, col0: int, x2: torch.Tensor, dw_rows: tor
     if d_logits.dtype != torch.float32 or d_logits.stride(1) != 1 or dw_rows.dtype != x2.dtype or \
             dw_rows.stride(1) != 1 or x2.shape[1] != m or d_logits.shape[0] != x2.shape[0]:
         raise ValueError("gate_wgrad: need fp32 d_logits [S, E], x2 [S, M] and dw_rows [E, M] of x2's dtype")
-    lib = _lib.load()
-    nbytes = lib.rtp_gate_wgrad_workspace_bytes(x2.shape[0], m, e)
+    nbytes = native().rtp_gate_wgrad_workspace_bytes(x2.shape[0], m, e)
     ws = torch.empty(nbytes // 4, dtype=torch.float32, device=x2.device)
-    _lib.require_device()
-    check(lib.rtp_gate_wgrad(_stream(), dtype_code(x2.dtype), d_logits.data_ptr() + 4 * col0, d_logits.stride(0),
-                             x2.data_ptr(), x2.stride(0), x2.shape[0], m, e, dw_rows.data_ptr(), dw_rows.stride(0),
-                             int(accumulate), ws.data_ptr(), nbytes))
+    native().rtp_gate_wgrad(dtype_code(x2.dtype), d_logits.data_ptr() + 4 * col0, d_logits.stride(0), x2.data_ptr(),
+                            x2.stride(0), x2.shape[0], m, e, dw_rows.data_ptr(), dw_rows.stride(0), int(accumulate),
+                            ws.data_ptr(), nbytes)
 
 
 def conv_geom(x_shape, kernel_size, stride, padding, dilation) -> "_lib.ConvGeom":
@@ -876,10 +780,9 @@ def conv2d_fwd(x: torch.Tensor, geom, flat: torch.Tensor, w_off: int, bias_off: 
             y.dtype != flat.dtype or not y.is_contiguous() or y.dim() != 4 or \
             (y.shape[0], y.shape[2], y.shape[3]) != (geom.n, geom.ho, geom.wo) or co_first + shards * n_s > y.shape[1]:
         raise ValueError("conv2d_fwd: x [N,C,H,W] and a contiguous y [N,Co,Ho,Wo] of the weights' dtype")
-    _lib.require_device()
-    check(_lib.load().rtp_conv2d_fwd(_stream(), dtype_code(x.dtype), x.data_ptr(), *x.stride(), geom, flat.data_ptr(),
-                                     numel, shards, w_off, -1 if bias_off is None else bias_off, n_s, y.data_ptr(),
-                                     co_first, y.shape[1]))
+    native().rtp_conv2d_fwd(dtype_code(x.dtype), x.data_ptr(), *x.stride(), C.addressof(geom), flat.data_ptr(), numel,
+                            shards, w_off, -1 if bias_off is None else bias_off, n_s, y.data_ptr(), co_first,
+                            y.shape[1])
 
 
 def conv2d_wgrad(dy: torch.Tensor, x: torch.Tensor, geom, grads: torch.Tensor, w_off: int, bias_off: Optional[int],
@@ -894,14 +797,12 @@ def conv2d_wgrad(dy: torch.Tensor, x: torch.Tensor, geom, grads: torch.Tensor, w
             (dy.shape[0], dy.shape[2], dy.shape[3]) != (geom.n, geom.ho, geom.wo) or \
             co_first + shards * n_s > dy.shape[1] or x.dtype != grads.dtype or dy.dtype != grads.dtype:
         raise ValueError("conv2d_wgrad: x [N,C,H,W] and dy [N,Co,Ho,Wo] of the gradients' dtype")
-    _lib.require_device()
-    lib = _lib.load()
-    nbytes = lib.rtp_conv2d_wgrad_workspace_bytes(geom, shards, n_s)
+    nbytes = native().rtp_conv2d_wgrad_workspace_bytes(C.addressof(geom), shards, n_s)
     ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=x.device)
-    check(lib.rtp_conv2d_wgrad(_stream(), dtype_code(x.dtype), dy.data_ptr(), *dy.stride(), x.data_ptr(),
-                               *x.stride(), geom, grads.data_ptr(), numel, shards, w_off,
-                               -1 if bias_off is None else bias_off, n_s, co_first, int(accumulate), ws.data_ptr(),
-                               nbytes))
+    native().rtp_conv2d_wgrad(dtype_code(x.dtype), dy.data_ptr(), *dy.stride(), x.data_ptr(), *x.stride(),
+                              C.addressof(geom), grads.data_ptr(), numel, shards, w_off,
+                              -1 if bias_off is None else bias_off, n_s, co_first, int(accumulate), ws.data_ptr(),
+                              nbytes)
 
 
 def conv2d_dgrad(dy: torch.Tensor, geom, flat: torch.Tensor, w_off: int, n_s: int, co_first: int, dx: torch.Tensor,
@@ -917,11 +818,10 @@ def conv2d_dgrad(dy: torch.Tensor, geom, flat: torch.Tensor, w_off: int, n_s: in
             tuple(dx.shape) != (geom.n, geom.c, geom.h, geom.w) or dx.dtype not in ok or \
             (addend is not None and (addend.shape != dx.shape or not addend.is_contiguous() or addend.dtype not in ok)):
         raise ValueError("conv2d_dgrad: dy [N,Co,Ho,Wo] of the weights' dtype, contiguous dx / addend [N,C,H,W]")
-    _lib.require_device()
-    check(_lib.load().rtp_conv2d_dgrad(_stream(), dtype_code(dy.dtype), dy.data_ptr(), *dy.stride(), geom,
-                                       flat.data_ptr(), numel, shards, w_off, n_s, co_first, dx.data_ptr(),
-                                       int(dx.dtype == torch.float32), None if addend is None else addend.data_ptr(),
-                                       int(addend is not None and addend.dtype == torch.float32)))
+    native().rtp_conv2d_dgrad(dtype_code(dy.dtype), dy.data_ptr(), *dy.stride(), C.addressof(geom), flat.data_ptr(),
+                              numel, shards, w_off, n_s, co_first, dx.data_ptr(), int(dx.dtype == torch.float32),
+                              None if addend is None else addend.data_ptr(),
+                              int(addend is not None and addend.dtype == torch.float32))
 
 
 def adam_step(master: torch.Tensor, grad: torch.Tensor, shadow: Optional[torch.Tensor], exp_avg: torch.Tensor,
@@ -944,10 +844,9 @@ def adam_step(master: torch.Tensor, grad: torch.Tensor, shadow: Optional[torch.T
         if step.dtype != torch.int64 or step.numel() != 1 or step.device != master.device:
             raise ValueError("adam_step: a device step count must be one int64 element on the master's device")
         step_dev, step = step.data_ptr(), 0
-    _lib.require_device()
-    check(_lib.load().rtp_adam_step(_stream(), dtype_code(grad.dtype), master.data_ptr(), grad.data_ptr(),
-                                    _ptr(shadow), exp_avg.data_ptr(), exp_avg_sq.data_ptr(), n, lr, betas[0],
-                                    betas[1], eps, weight_decay, int(step), step_dev, clip))
+    native().rtp_adam_step(dtype_code(grad.dtype), master.data_ptr(), grad.data_ptr(), _ptr(shadow),
+                           exp_avg.data_ptr(), exp_avg_sq.data_ptr(), n, lr, betas[0], betas[1], eps, weight_decay,
+                           int(step), step_dev, clip)
 
 
 SGD_CHUNK = 16384  # parameters per workgroup of the multi-buffer update
@@ -1003,16 +902,13 @@ def adam_step_multi(table: torch.Tensor, dtype: torch.dtype, step, lr: float, be
         if step.dtype != torch.int64 or step.numel() != 1 or step.device != table.device:
             raise ValueError("adam_step_multi: a device step count must be one int64 element on the table's device")
         step_dev, step = step.data_ptr(), 0
-    _lib.require_device()
-    check(_lib.load().rtp_adam_step_multi(_stream(), dtype_code(dtype), table.data_ptr(), table.shape[0], lr, betas[0],
-                                          betas[1], eps, weight_decay, int(step), step_dev, clip, float(total_params)))
+    native().rtp_adam_step_multi(dtype_code(dtype), table.data_ptr(), table.shape[0], lr, betas[0], betas[1], eps,
+                                 weight_decay, int(step), step_dev, clip, float(total_params))
 
 
 def sgd_step_multi(table: torch.Tensor, dtype: torch.dtype, lr: float, clip: float, total_params: int) -> None:
     _dev(table)
-    _lib.require_device()
-    check(_lib.load().rtp_sgd_step_multi(_stream(), dtype_code(dtype), table.data_ptr(), table.shape[0], lr, clip,
-                                         float(total_params)))
+    native().rtp_sgd_step_multi(dtype_code(dtype), table.data_ptr(), table.shape[0], lr, clip, float(total_params))
 
 
 def cast(src: torch.Tensor, dst: torch.Tensor) -> None:
@@ -1020,9 +916,7 @@ def cast(src: torch.Tensor, dst: torch.Tensor) -> None:
     _dev(dst)
     if not (src.is_contiguous() and dst.is_contiguous()) or src.numel() != dst.numel():
         raise ValueError("cast: need contiguous tensors of equal length")
-    _lib.require_device()
-    check(_lib.load().rtp_cast(_stream(), dtype_code(src.dtype), src.data_ptr(), dtype_code(dst.dtype),
-                               dst.data_ptr(), src.numel()))
+    native().rtp_cast(dtype_code(src.dtype), src.data_ptr(), dtype_code(dst.dtype), dst.data_ptr(), src.numel())
 
 
 class FusedSgd:
@@ -1098,14 +992,11 @@ def top2_route(logits: torch.Tensor, noise: torch.Tensor, l_aux_dtype: Optional[
     r.l_aux = torch.empty((), dtype=torch.float32, device=dev)
     r.counts = torch.empty(2 * e, dtype=torch.int32, device=dev)
     r.l_aux_typed = torch.empty((), dtype=torch.bfloat16, device=dev) if l_aux_dtype == torch.bfloat16 else None
-    _lib.require_device()
-    lib = _lib.load()
-    nbytes = lib.rtp_top2_route_workspace_bytes(s, e)
+    nbytes = native().rtp_top2_route_workspace_bytes(s, e)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-    check(lib.rtp_top2_route(_stream(), logits.data_ptr(), noise.data_ptr(), s, e, r.expert.data_ptr(),
-                             r.slot.data_ptr(), r.keep.data_ptr(), r.weight.data_ptr(), r.gates.data_ptr(),
-                             r.slot_token.data_ptr(), r.l_aux.data_ptr(), r.counts.data_ptr(), ws.data_ptr(), nbytes,
-                             _ptr(r.l_aux_typed)))
+    native().rtp_top2_route(logits.data_ptr(), noise.data_ptr(), s, e, r.expert.data_ptr(), r.slot.data_ptr(),
+                            r.keep.data_ptr(), r.weight.data_ptr(), r.gates.data_ptr(), r.slot_token.data_ptr(),
+                            r.l_aux.data_ptr(), r.counts.data_ptr(), ws.data_ptr(), nbytes, _ptr(r.l_aux_typed))
     return r
 
 
@@ -1116,9 +1007,8 @@ def top2_route_bwd(r: Routing, d_weight: Optional[torch.Tensor], d_l_aux: Option
     d_logits = torch.empty(r.s, r.e, dtype=torch.float32, device=r.gates.device)
     if d_l_aux is not None:
         d_l_aux = d_l_aux.contiguous().float()
-    check(_lib.load().rtp_top2_route_bwd(_stream(), r.gates.data_ptr(), r.expert.data_ptr(), r.keep.data_ptr(),
-                                         r.counts.data_ptr(), d_weight.data_ptr(), _ptr(d_l_aux), r.s, r.e,
-                                         d_logits.data_ptr()))
+    native().rtp_top2_route_bwd(r.gates.data_ptr(), r.expert.data_ptr(), r.keep.data_ptr(), r.counts.data_ptr(),
+                                d_weight.data_ptr(), _ptr(d_l_aux), r.s, r.e, d_logits.data_ptr())
     return d_logits
 
 
@@ -1129,9 +1019,8 @@ def moe_dispatch(x: torch.Tensor, r: Routing, out: torch.Tensor, weight: Optiona
     n_slots, cols_o, ld_o = _mat(out, "out")
     if rows != r.s or cols != cols_o or n_slots != r.e * r.capacity or out.dtype != x.dtype:
         raise ValueError("moe_dispatch: shape mismatch")
-    check(_lib.load().rtp_moe_dispatch(_stream(), dtype_code(x.dtype), x.data_ptr(), ld_x, r.slot_token.data_ptr(),
-                                       r.expert.data_ptr(), r.slot.data_ptr(), _ptr(weight), n_slots, r.capacity,
-                                       cols, out.data_ptr(), ld_o))
+    native().rtp_moe_dispatch(dtype_code(x.dtype), x.data_ptr(), ld_x, r.slot_token.data_ptr(), r.expert.data_ptr(),
+                              r.slot.data_ptr(), _ptr(weight), n_slots, r.capacity, cols, out.data_ptr(), ld_o)
 
 
 def moe_combine(y: torch.Tensor, r: Routing, out: torch.Tensor, weight: Optional[torch.Tensor]) -> None:
@@ -1141,9 +1030,8 @@ def moe_combine(y: torch.Tensor, r: Routing, out: torch.Tensor, weight: Optional
     rows, cols_o, ld_o = _mat(out, "out")
     if rows != r.s or cols != cols_o or n_slots != r.e * r.capacity or out.dtype != y.dtype:
         raise ValueError("moe_combine: shape mismatch")
-    check(_lib.load().rtp_moe_combine(_stream(), dtype_code(y.dtype), y.data_ptr(), ld_y, r.expert.data_ptr(),
-                                      r.slot.data_ptr(), r.keep.data_ptr(), _ptr(weight), r.s, r.capacity, cols,
-                                      out.data_ptr(), ld_o))
+    native().rtp_moe_combine(dtype_code(y.dtype), y.data_ptr(), ld_y, r.expert.data_ptr(), r.slot.data_ptr(),
+                             r.keep.data_ptr(), _ptr(weight), r.s, r.capacity, cols, out.data_ptr(), ld_o)
 
 
 def moe_combine_dweight(dout: torch.Tensor, y: torch.Tensor, r: Routing) -> torch.Tensor:
@@ -1153,7 +1041,7 @@ def moe_combine_dweight(dout: torch.Tensor, y: torch.Tensor, r: Routing) -> torc
     if rows != r.s or cols != cols_y or dout.dtype != y.dtype:
         raise ValueError("moe_combine_dweight: shape mismatch")
     dw = torch.empty(r.s, 2, dtype=torch.float32, device=dout.device)
-    check(_lib.load().rtp_moe_combine_dweight(_stream(), dtype_code(y.dtype), dout.data_ptr(), ld_d, y.data_ptr(),
-                                              ld_y, r.expert.data_ptr(), r.slot.data_ptr(), r.keep.data_ptr(), r.s,
-                                              r.capacity, cols, dw.data_ptr()))
+    native().rtp_moe_combine_dweight(dtype_code(y.dtype), dout.data_ptr(), ld_d, y.data_ptr(), ld_y,
+                                     r.expert.data_ptr(), r.slot.data_ptr(), r.keep.data_ptr(), r.s, r.capacity, cols,
+                                     dw.data_ptr())
     return dw

@@ -97,19 +97,20 @@ def _warm_step(home: torch.Tensor) -> None:
     here = home.data_ptr()
     if here == cur:
         return  # the same layer again (its backward pass right after its forward pass)
-    if len(_warm_next) > 4096:
-        _warm_next.clear()  # far more layers than any model rotates: stale entries of models long gone
-    _warm_next[(idx, prev, cur)] = weakref.ref(home)
+    seen = _warm_next.get((idx, prev, cur))
+    if seen is None or seen() is not home:
+        if len(_warm_next) > 4096:
+            _warm_next.clear()  # far more layers than any model rotates: stale entries of models long gone
+        _warm_next[(idx, prev, cur)] = weakref.ref(home)
     _warm_hist[idx] = (cur, here)
     ref = _warm_next.get((idx, cur, here))
     nxt = ref() if ref is not None else None
-    lib = _lib.load()
     if nxt is not None and nxt.is_cuda and nxt.data_ptr() != here:
         _warm_pending[idx] = nxt
-        check(lib.rtp_gemm_warm_next(nxt.data_ptr(), nxt.numel() * nxt.element_size()))
+        _lib.native().rtp_gemm_warm_next(nxt, nxt.numel() * nxt.element_size())
     elif _warm_pending.get(idx) is not None:
         _warm_pending[idx] = None
-        check(lib.rtp_gemm_warm_next(None, 0))
+        _lib.native().rtp_gemm_warm_next(None, 0)
 
 
 # ---- weight gradients on a second stream -----------------------------------------------------------
@@ -494,6 +495,33 @@ class Rotation:
                 g.slot = None
             return
         check(self.lib.rtp_ring_release(self.ring._handle, self.stream, self.slots[j]))
+
+
+class OneRun:
+    """The rotation of the direct mode when one window covers the layer: a single run, all shards read from home.  What
+    `rotation` returns then, one object per home tensor for good: nothing of it depends on the pass."""
+
+    steps = 1
+
+    def __init__(self, home: torch.Tensor):
+        self._runs = [(home, 0, home.shape[0])]
+        self.windows = [[(0, home.shape[0])]]
+
+    def acquire(self, j: int) -> List[Run]:
+        return self._runs
+
+    def release(self, j: int) -> None:
+        pass
+
+
+def rotation(store, rank: int, reverse: bool = False):
+    """One pass over the shards of a layer's store (ShardStore) in ring order."""
+    home = store.home
+    if _mode == "direct" and (_window is None or _window >= home.shape[0]):
+        if _warm_ahead:
+            _warm_step(home)
+        return store.one_run
+    return Rotation(home, ring_order(rank, home.shape[0], reverse), group=store.stage_group)
 
 
 def ring_order(rank: int, world_size: int, reverse: bool = False) -> List[int]:

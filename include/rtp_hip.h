@@ -373,13 +373,28 @@ int rtp_embedding_scatter_add_sgd(void* stream, int dtype, const void* grad_out,
  * zero_fill the rows that no token names are cleared by further workgroups of the same launch.  master == NULL: the
  * gradient is written (zero_fill != 0: overwriting, else added to what is there); master != NULL: the update of
  * rtp_embedding_scatter_add_sgd (weights may be NULL; store_grad as there).  At most 4096 ids
- * (rtp_embedding_backward_supported); longer steps take rtp_embedding_sort_ids + rtp_embedding_scatter_add_*. */
+ * (rtp_embedding_backward_supported); longer steps take rtp_embedding_backward_grouped. */
 int rtp_embedding_backward_supported(int64_t n_ids);
 int rtp_embedding_backward(void* stream, int dtype, const void* grad_out, int64_t ld_grad_out, int64_t n_ids,
                            const int64_t* ids, void* grad_table, int64_t ld_grad_table, int grad_table_f32,
                            int64_t row_begin, int64_t row_count, int64_t cols, int64_t padding_idx, int scale_by_freq,
                            int zero_fill, int64_t groups, int64_t grad_out_sg, int64_t grad_table_sg, float grad_scale,
                            float* master, void* weights, float lr, float clip, int store_grad);
+
+/* The same for longer steps, in two launches: the ids are first grouped by table row (counts, offsets and unordered
+ * position lists in the workspace: rtp_embedding_backward_grouped_workspace_bytes(n_ids, row_count) bytes, 256-byte
+ * aligned), then a wavefront per table row orders its positions, sums and writes or clears the row; a row that 64 or
+ * more positions name is dealt over workgroups by columns.  Arguments and results of rtp_embedding_backward, bit for
+ * bit.  1 .. 262144 ids and row_count below 2^26 (rtp_embedding_backward_grouped_supported); longer steps take
+ * rtp_embedding_sort_ids + rtp_embedding_scatter_add_*. */
+int rtp_embedding_backward_grouped_supported(int64_t n_ids, int64_t row_count);
+size_t rtp_embedding_backward_grouped_workspace_bytes(int64_t n_ids, int64_t row_count);
+int rtp_embedding_backward_grouped(void* stream, int dtype, const void* grad_out, int64_t ld_grad_out, int64_t n_ids,
+                                   const int64_t* ids, void* grad_table, int64_t ld_grad_table, int grad_table_f32,
+                                   int64_t row_begin, int64_t row_count, int64_t cols, int64_t padding_idx,
+                                   int scale_by_freq, int zero_fill, int64_t groups, int64_t grad_out_sg,
+                                   int64_t grad_table_sg, float grad_scale, float* master, void* weights, float lr,
+                                   float clip, int store_grad, void* workspace, size_t workspace_bytes);
 
 /* ---------------------------------------------------------------------------------------------
  * Attention softmax (reference: rtp/module/functional.py:779-792 baddbmm+softmax, :825

@@ -129,6 +129,10 @@ PROTOTYPES = {
     "rtp_embedding_backward_supported": (_i, [_i64]),
     "rtp_embedding_backward": (_i, [_vp, _i, _vp, _i64, _i64, _vp, _vp, _i64, _i, _i64, _i64, _i64, _i64, _i, _i, _i64,
                                     _i64, _i64, _f, _vp, _vp, _f, _f, _i]),
+    "rtp_embedding_backward_grouped_supported": (_i, [_i64, _i64]),
+    "rtp_embedding_backward_grouped_workspace_bytes": (_sz, [_i64, _i64]),
+    "rtp_embedding_backward_grouped": (_i, [_vp, _i, _vp, _i64, _i64, _vp, _vp, _i64, _i, _i64, _i64, _i64, _i64, _i, _i,
+                                            _i64, _i64, _i64, _f, _vp, _vp, _f, _f, _i, _vp, _sz]),
     "rtp_softmax_fwd": (_i, [_vp, _i, _vp, _vp, _vp, _i64, _i64, _i, _f, _i64, _i64, _i64, _vp]),
     "rtp_softmax_fwd_masks": (_i, [_vp, _i, _vp, _vp, _i64, _vp, _i64, _i64, _i, _f, _i64, _i64, _i64, _vp, _vp, _vp]),
     "rtp_softmax_bwd": (_i, [_vp, _i, _vp, _vp, _vp, _f, _i64, _i64, _i64, _vp]),

@@ -115,6 +115,28 @@ __device__ __forceinline__ void nt_store(uint4 a, uint4* p) {
 // rtp_gate_wgrad_static (gate.hip).  Part of rtp_device_check.
 int gate_static_setup();
 
+// Division of a 32-bit unsigned number by a launch constant with a multiply-high and two shifts (Granlund and
+// Montgomery's round-up method, exact for every 32-bit dividend): integer division by a run-time value costs a
+// few dozen dependent instructions on this hardware, and the wave-specialised kernel would otherwise do ten of
+// them before it can issue its first load.
+struct FastDiv {
+  unsigned d, mul, s1, s2;
+};
+inline FastDiv make_fastdiv(unsigned d) {
+  FastDiv f;
+  f.d = d;
+  unsigned s = 0;
+  while ((1ull << s) < d) ++s;  // ceil(log2 d)
+  f.mul = (unsigned)((((1ull << s) - d) << 32) / d + 1);
+  f.s1 = s < 1 ? s : 1;
+  f.s2 = s < 1 ? 0 : s - 1;
+  return f;
+}
+__device__ __forceinline__ unsigned fast_div(unsigned n, const FastDiv& f) {
+  const unsigned t = __umulhi(n, f.mul);
+  return (t + ((n - t) >> f.s1)) >> f.s2;
+}
+
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Reads one word of every 64-byte line of a kernel's BYTES bytes of arguments (and of the launch dimensions that

@@ -7,54 +7,62 @@
 
 namespace rtp {
 
-// One workgroup per (token, 4 KiB column chunk); 16-byte lanes when the shard rectangle allows it.
+// One wavefront per token, over the columns of all shards of the run: a token's output row is contiguous across the shards
+// (V elements per lane, kGatherDepth vectors requested before the first is stored), only the table they come from
+// differs.  Bound by memory: at 16368 tokens of 8 shards x 256 bf16 columns a workgroup per (token, shard) moved 512 bytes
+// with half of its lanes idle and took 55 us (2.4 TB/s); this form takes 21 us (6.4 TB/s; part of the reads hit the caches).
 // With `pos` the row is scaled and a positional row added on the way: out = T(T(table * scale) + pos[t / batch]),
 // each step rounded to T as the two separate element-wise operations would round it.
-template <typename T>
+constexpr int kGatherDepth = 4;
+template <typename T, int V, bool POS>
 __global__ __launch_bounds__(256) void gather_kernel(const T* table, long ld_table, long row_begin, long row_count,
-                                                     long cols, const int64_t* ids, T* out, long ld_out, int vec,
-                                                     long table_sg, long out_sg, float scale, const T* pos, long ld_pos,
-                                                     long pos_sg, long batch) {
-  const long t = blockIdx.x;
+                                                     int per_row, FastDiv d_row, int total, const int64_t* ids, long n, T* out,
+                                                     long ld_out, long table_sg, long out_sg, float scale, const T* pos,
+                                                     long ld_pos, long pos_sg, FastDiv d_batch) {
+  const long t = (long)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (t >= n) return;
   const long row = ids[t] - row_begin;
   if (row < 0 || row >= row_count) return;
-  const T* src = table + blockIdx.z * table_sg + row * ld_table;
-  T* dst = out + blockIdx.z * out_sg + t * ld_out;
-  constexpr int VEC = 16 / sizeof(T);
-  if (pos) {
-    const T* prow = pos + (long)((unsigned)t / (unsigned)batch) * ld_pos + blockIdx.z * pos_sg;
-    if (vec) {
-      const long nvec = cols / VEC;
-      union Pack {
-        uint4 u;
-        T e[VEC];
-      };
-      for (long i = (long)blockIdx.y * 256 + threadIdx.x; i < nvec; i += (long)gridDim.y * 256) {
-#pragma clang fp contract(off)
-        Pack a, b, r;
-        a.u = reinterpret_cast<const uint4*>(src)[i];
-        b.u = reinterpret_cast<const uint4*>(prow)[i];
+  const T* src = table + row * ld_table;
+  T* dst = out + t * ld_out;
+  const T* prow = POS ? pos + (long)fast_div((unsigned)t, d_batch) * ld_pos : nullptr;
+  union Pack {
+    uint4 q;
+    T e[V == 1 ? 1 : 16 / (int)sizeof(T)];
+  };
+  auto load = [](const T* p) {
+    Pack u;
+    if constexpr (V == 1)
+      u.e[0] = p[0];
+    else
+      u.q = *reinterpret_cast<const uint4*>(p);
+    return u;
+  };
+  for (int e0 = threadIdx.x & 63; e0 < total; e0 += kGatherDepth * 64) {
+    Pack a[kGatherDepth], b[kGatherDepth];
+    long at[kGatherDepth];
 #pragma unroll
-        for (int e = 0; e < VEC; ++e)
-          r.e[e] = from_f32<T>(to_f32(from_f32<T>(to_f32(a.e[e]) * scale)) + to_f32(b.e[e]));
-        reinterpret_cast<uint4*>(dst)[i] = r.u;
-      }
-      return;
+    for (int d = 0; d < kGatherDepth; ++d) {
+      const int e = e0 + d * 64 < total ? e0 + d * 64 : e0;  // past the row: the first vector again, not stored
+      const unsigned g = fast_div((unsigned)e, d_row);
+      const int c = (e - (int)g * per_row) * V;
+      at[d] = g * out_sg + c;
+      a[d] = load(src + g * table_sg + c);
+      if constexpr (POS) b[d] = load(prow + g * pos_sg + c);
     }
-    for (long i = (long)blockIdx.y * 256 + threadIdx.x; i < cols; i += (long)gridDim.y * 256) {
+#pragma unroll
+    for (int d = 0; d < kGatherDepth; ++d) {
+      if (e0 + d * 64 >= total) break;
+      if constexpr (POS) {
 #pragma clang fp contract(off)
-      const float a = to_f32(from_f32<T>(to_f32(src[i]) * scale));
-      dst[i] = from_f32<T>(a + to_f32(prow[i]));
+#pragma unroll
+        for (int v = 0; v < V; ++v) a[d].e[v] = from_f32<T>(to_f32(from_f32<T>(to_f32(a[d].e[v]) * scale)) + to_f32(b[d].e[v]));
+      }
+      if constexpr (V == 1)
+        dst[at[d]] = a[d].e[0];
+      else
+        *reinterpret_cast<uint4*>(dst + at[d]) = a[d].q;
     }
-    return;
-  }
-  if (vec) {
-    const long nvec = cols / VEC;
-    const uint4* s = reinterpret_cast<const uint4*>(src);
-    uint4* d = reinterpret_cast<uint4*>(dst);
-    for (long i = (long)blockIdx.y * 256 + threadIdx.x; i < nvec; i += (long)gridDim.y * 256) d[i] = s[i];
-  } else {
-    for (long i = (long)blockIdx.y * 256 + threadIdx.x; i < cols; i += (long)gridDim.y * 256) dst[i] = src[i];
   }
 }
 
@@ -328,6 +336,329 @@ __global__ __launch_bounds__(256) void embedding_bwd_kernel(const T* grad_out, l
   }
 }
 
+// ---- backward of long steps: ids grouped by table row, no sort ----
+// Two launches.  group_ids_kernel: workgroup w owns a slice of the table rows, counts the step's ids that fall into it (LDS
+// counters, every workgroup reads all ids), turns the counts into offsets and writes every position into its row's
+// segment of `pos` -- in any order -- and the rows with kLongRow positions or more into a list of its own.
+// grouped_bwd_kernel: a wavefront per table row orders the row's positions and sums their upstream rows front to back,
+// starting from +0.0f (the order of a sequential index_add_), or clears the row when no position names it; a long row
+// is dealt over workgroups by columns instead, which start first.
+//
+// Words of running text are what makes this worth its launches: with ids by word frequency one of 16368 positions in nine
+// is the same row, and the sum over that row's positions is a serial chain that only columns can share.  The sorted
+// path (radix sort, one workgroup per segment and shard, one row in flight) took 533 us there, this takes 83 (uniform ids: 122 against 37).
+constexpr int kLongRow = 64;             // positions from which a row is dealt over workgroups by columns
+constexpr int kGroupSlices = 32;         // workgroups of the grouping pass, at least
+constexpr int kGroupRowsMax = 8192;      // table rows per slice, at most (LDS counters)
+constexpr int kGroupMaxIds = 1 << 18;    // a long row's bitmap of positions in LDS: 32 KiB
+constexpr int kGroupThreads = 1024;
+
+struct GroupLayout {  // int32 arrays in the workspace
+  size_t offs, pos, nlong, longs, total;
+  int slices, rows_per, long_cap;
+};
+static GroupLayout group_layout(int64_t n, int64_t rows) {
+  GroupLayout L;
+  L.slices = (int)std::max<int64_t>(kGroupSlices, ceil_div(rows, kGroupRowsMax));
+  L.rows_per = (int)ceil_div(rows, L.slices);
+  L.long_cap = (int)(n / kLongRow);
+  L.offs = 0;
+  L.pos = ((size_t)(rows + 1) * 4 + 255) & ~(size_t)255;
+  L.nlong = L.pos + (((size_t)n * 4 + 255) & ~(size_t)255);
+  L.longs = L.nlong + (((size_t)L.slices * 4 + 255) & ~(size_t)255);
+  L.total = L.longs + (size_t)L.slices * L.long_cap * 4 + 256;
+  return L;
+}
+
+__global__ __launch_bounds__(kGroupThreads) void group_ids_kernel(const int64_t* ids, int n, long row_begin, int row_count,
+                                                                  long padding_idx, int rows_per, int* offs, int* pos,
+                                                                  int* nlong, int* longs, int long_cap) {
+  __shared__ int cnt[kGroupRowsMax];
+  __shared__ int wave_sum_[kGroupThreads / 64];
+  __shared__ int s_long;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r0 = blockIdx.x * rows_per, r1 = min(r0 + rows_per, row_count), mine = max(r1 - r0, 0);
+  for (int i = tid; i < mine; i += kGroupThreads) cnt[i] = 0;
+  if (tid == 0) s_long = 0;
+  __syncthreads();
+  // row of position i inside the table, or -1
+  constexpr int U = 8;
+  auto rows_of = [&](int i0, int (&r)[U]) {
+    int64_t v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = i0 + u * kGroupThreads;
+      v[u] = ids[i < n ? i : n - 1];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t q = (int64_t)(int)v[u] - row_begin;
+      r[u] = (i0 + u * kGroupThreads < n && v[u] != padding_idx && q >= 0 && q < row_count) ? (int)q : -1;
+    }
+  };
+  int below = 0;
+  for (int i0 = tid; i0 < n; i0 += U * kGroupThreads) {
+    int r[U];
+    rows_of(i0, r);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (r[u] >= r0 && r[u] < r1) atomicAdd(&cnt[r[u] - r0], 1);
+      below += (r[u] >= 0 && r[u] < r0) ? 1 : 0;
+    }
+  }
+  // base = positions of all earlier slices; then the exclusive scan of the slice's counts, in place
+  auto block_scan = [&](int v, int& all) {  // exclusive prefix of v over the workgroup, and the sum
+    int x = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    __syncthreads();
+    if (lane == 63) wave_sum_[wave] = x;
+    __syncthreads();
+    int before = 0;
+    all = 0;
+#pragma unroll
+    for (int w = 0; w < kGroupThreads / 64; ++w) {
+      before += w < wave ? wave_sum_[w] : 0;
+      all += wave_sum_[w];
+    }
+    return before + x - v;
+  };
+  int base = 0, all;
+  (void)block_scan(below, base);
+  const int per = (mine + kGroupThreads - 1) / kGroupThreads, c0 = min(tid * per, mine), c1 = min(c0 + per, mine);
+  int sum = 0;
+  for (int c = c0; c < c1; ++c) sum += cnt[c];
+  int run = base + block_scan(sum, all);
+  for (int c = c0; c < c1; ++c) {
+    const int k = cnt[c];
+    if (k >= kLongRow) longs[(long)blockIdx.x * long_cap + atomicAdd(&s_long, 1)] = r0 + c;
+    cnt[c] = run;
+    offs[r0 + c] = run;
+    run += k;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    nlong[blockIdx.x] = s_long;
+    if (r1 == row_count && mine > 0) offs[row_count] = base + all;
+  }
+  for (int i0 = tid; i0 < n; i0 += U * kGroupThreads) {
+    int r[U];
+    rows_of(i0, r);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (r[u] >= r0 && r[u] < r1) pos[atomicAdd(&cnt[r[u] - r0], 1)] = i0 + u * kGroupThreads;
+  }
+}
+
+template <typename T, typename G>
+struct GroupedBwd {
+  const T* grad_out;
+  long ld_go, go_sg;
+  G* grad_table;
+  long ld_gt, gt_sg;
+  float* master;
+  T* weights;
+  float grad_scale, lr, clip;
+  int scale_by_freq, overwrite, store_grad, zero_fill;
+  int n, row_count, groups, cols;
+  const int *offs, *pos, *nlong, *longs;
+  int slices, long_cap;
+
+  // one upstream value as it joins the sum
+  __device__ __forceinline__ float take(T g) const {
+#pragma clang fp contract(off)
+    return grad_scale == 1.0f ? to_f32(g) : to_f32(from_f32<T>(to_f32(g) * grad_scale));
+  }
+  // the finished sums of V columns of a row that `cnt` positions name
+  template <int V>
+  __device__ __forceinline__ void finish(float (&acc)[V], long off, int cnt) const {
+#pragma clang fp contract(off)
+    if (scale_by_freq) {
+      const float inv = 1.0f / (float)cnt;
+#pragma unroll
+      for (int v = 0; v < V; ++v) acc[v] *= inv;
+    }
+    if (master != nullptr) {
+      float w[V];
+      vec_load<float, V>(master + off, w);
+#pragma unroll
+      for (int v = 0; v < V; ++v) w[v] = sgd_update<G>(w[v], acc[v], lr, clip);
+      vec_store<float, V>(master + off, w);
+      if (weights != nullptr) vec_store<T, V>(weights + off, w);
+      if (store_grad) vec_store<G, V>(grad_table + off, acc);
+      return;
+    }
+    if (!overwrite) {
+      float old[V];
+      vec_load<G, V>(grad_table + off, old);
+#pragma unroll
+      for (int v = 0; v < V; ++v) acc[v] = old[v] + acc[v];
+    }
+    vec_store<G, V>(grad_table + off, acc);
+  }
+};
+
+// Sums the upstream rows of list[0 .. cnt) (ascending positions: list[k] + at) for the columns at `src` of this lane.  W
+// columns per lane, one 4-byte (or smaller) load each row: with 64 rows in flight per wave the chain advances 64 rows
+// per trip to memory.
+template <int U, int W, typename T, typename G>
+__device__ __forceinline__ void sum_rows(const GroupedBwd<T, G>& a, const T* src, const unsigned short* list, int at, int k,
+                                         float (&acc)[W]) {
+  typedef T vec_t __attribute__((ext_vector_type(W)));
+  const int lane = threadIdx.x & 63;
+  const int mine = list[k + (lane < U ? lane : 0)] + at;
+  vec_t g[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    g[u] = *reinterpret_cast<const vec_t*>(src + (long)__builtin_amdgcn_readlane(mine, u) * a.ld_go);
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int w = 0; w < W; ++w) acc[w] += a.take(g[u][w]);
+}
+
+// long_wgs workgroups for the long rows (long row j, column chunk y: j * chunks + y), then one wavefront per table row.
+// V: columns per lane of a short row (16-byte vectors, or 1), W: columns per lane of a long row.
+template <typename T, typename G, int V, int W>
+__global__ __launch_bounds__(256) void grouped_bwd_kernel(GroupedBwd<T, G> a, int long_wgs, int chunks) {
+  extern __shared__ unsigned bits[];  // a long row's positions as a bitmap, then the window's list
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if ((int)blockIdx.x < long_wgs) {
+    __shared__ int s_row, s_part[4];
+    const int want = blockIdx.x / chunks, chunk = blockIdx.x - want * chunks;
+    if (tid == 0) {
+      int left = want, row = -1;
+      for (int s = 0; s < a.slices; ++s) {
+        const int c = a.nlong[s];
+        if (left < c) {
+          row = a.longs[(long)s * a.long_cap + left];
+          break;
+        }
+        left -= c;
+      }
+      s_row = row;
+    }
+    __syncthreads();
+    const int row = s_row;
+    if (row < 0) return;
+    const int p0 = a.offs[row], cnt = a.offs[row + 1] - p0;
+    const int words = (a.n + 31) / 32, windows = (words + 255) / 256;
+    unsigned short* list = reinterpret_cast<unsigned short*>(bits + windows * 256);
+    for (int i = tid; i < windows * 256; i += 256) bits[i] = 0u;
+    __syncthreads();
+    for (int i = tid; i < cnt; i += 256) {
+      const int q = a.pos[p0 + i];
+      atomicOr(&bits[q >> 5], 1u << (q & 31));
+    }
+    const int per_row = a.cols / W, e = chunk * 256 + tid;  // W-column pieces of the row over all shards
+    const bool live = e < per_row * a.groups;
+    const int g = live ? e / per_row : 0, c = live ? (e - g * per_row) * W : 0;
+    const T* src = a.grad_out + g * a.go_sg + c;
+    float acc[W];
+#pragma unroll
+    for (int w = 0; w < W; ++w) acc[w] = 0.0f;
+    for (int win = 0; win < windows; ++win) {
+      __syncthreads();  // the bitmap is complete; the previous window's list has been read
+      // the window's 8192 positions: a word per thread, listed in ascending order
+      unsigned b = bits[win * 256 + tid];
+      int x = __popc(b);
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+      }
+      if (lane == 63) s_part[wave] = x;
+      __syncthreads();
+      int at = x - __popc(b);
+#pragma unroll
+      for (int w = 0; w < 4; ++w) at += w < wave ? s_part[w] : 0;
+      const int m = (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
+      while (b) {
+        list[at++] = (unsigned short)(tid * 32 + __builtin_ctz(b));
+        b &= b - 1;
+      }
+      __syncthreads();
+      int k = 0;
+      for (; k + 64 <= m; k += 64) sum_rows<64, W>(a, src, list, win * 8192, k, acc);
+      for (; k + 8 <= m; k += 8) sum_rows<8, W>(a, src, list, win * 8192, k, acc);
+      for (; k < m; ++k) sum_rows<1, W>(a, src, list, win * 8192, k, acc);
+    }
+    if (!live) return;
+    const long off = g * a.gt_sg + (long)row * a.ld_gt + c;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      float one[1] = {acc[w]};
+      a.template finish<1>(one, off + w, cnt);
+    }
+    return;
+  }
+  const int row = (int)(blockIdx.x - long_wgs) * 4 + wave;
+  if (row >= a.row_count) return;
+  const int p0 = a.offs[row], cnt = a.offs[row + 1] - p0;
+  if (cnt >= kLongRow || (cnt == 0 && !a.zero_fill)) return;
+  const int per_row = a.cols / V, total = per_row * a.groups;
+  // the row's positions in ascending order, one per lane: each lane counts the smaller ones, then they change places
+  int sorted = 0;
+  if (cnt > 0) {
+    const int mine = lane < cnt ? a.pos[p0 + lane] : 0x7fffffff;
+    int rank = 0;
+    for (int k = 0; k < cnt; ++k) rank += __builtin_amdgcn_readlane(mine, k) < mine ? 1 : 0;
+    // lanes beyond the row's positions keep out of the way: each its own slot behind them
+    sorted = __builtin_amdgcn_ds_permute((lane < cnt ? rank : lane) * 4, mine);
+  }
+  constexpr int CB = 4;  // vectors per lane worked on at once
+  for (int e0 = lane; e0 < total; e0 += CB * 64) {
+    float acc[CB][V];
+    long at[CB], to[CB];
+#pragma unroll
+    for (int d = 0; d < CB; ++d) {
+      const int e = e0 + d * 64 < total ? e0 + d * 64 : e0;
+      const int g = e / per_row, c = (e - g * per_row) * V;
+      at[d] = g * a.go_sg + c, to[d] = g * a.gt_sg + (long)row * a.ld_gt + c;
+#pragma unroll
+      for (int v = 0; v < V; ++v) acc[d][v] = 0.0f;
+    }
+    auto add = [&](int k, auto rows_tag) {
+      constexpr int R = decltype(rows_tag)::value;
+      union {
+        uint4 q;
+        T e[16 / sizeof(T)];
+      } u[R][CB];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const T* src = a.grad_out + (long)__builtin_amdgcn_readlane(sorted, k + r) * a.ld_go;
+#pragma unroll
+        for (int d = 0; d < CB; ++d) {
+          if constexpr (V == 1)
+            u[r][d].e[0] = src[at[d]];
+          else
+            u[r][d].q = *reinterpret_cast<const uint4*>(src + at[d]);
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int d = 0; d < CB; ++d)
+#pragma unroll
+          for (int v = 0; v < V; ++v) acc[d][v] += a.take(u[r][d].e[v]);
+    };
+    int k = 0;
+    for (; k + 2 <= cnt; k += 2) add(k, std::integral_constant<int, 2>{});
+    if (k < cnt) add(k, std::integral_constant<int, 1>{});
+#pragma unroll
+    for (int d = 0; d < CB; ++d) {
+      if (e0 + d * 64 >= total) break;
+      if (cnt == 0)
+        vec_store<G, V>(a.grad_table + to[d], acc[d]);
+      else
+        a.template finish<V>(acc[d], to[d], cnt);
+    }
+  }
+}
+
 struct SortLayout {
   size_t keys_in, vals_in, keys_out, vals_out, temp, total, temp_bytes;
 };
@@ -369,20 +700,24 @@ static int gather_impl(void* stream, int dtype, const void* table, int64_t ld_ta
                   (ld_out * esz) % 16 == 0 && (cols * esz) % 16 == 0 && (table_sg * esz) % 16 == 0 &&
                   (out_sg * esz) % 16 == 0 &&
                   (!pos || ((uintptr_t)pos % 16 == 0 && (ld_pos * esz) % 16 == 0 && (pos_sg * esz) % 16 == 0));
-  const unsigned chunks = (unsigned)std::min<int64_t>(16, std::max<int64_t>(1, ceil_div(cols * (int64_t)esz, 4096)));
-  dim3 grid((unsigned)n_ids, chunks, (unsigned)groups);
+  const int64_t per_row = vec ? cols * (int64_t)esz / 16 : cols;
+  RTP_REQUIRE(per_row * groups < (1ll << 30), "rtp_embedding_gather: rows too long");
+  const dim3 grid((unsigned)ceil_div(n_ids, 4));
   hipStream_t s = (hipStream_t)stream;
   ProfileScope prof(s, "embedding_gather", 0.0, (2.0 * (double)n_ids * cols * esz + 8.0 * n_ids) * groups);
-  if (dtype == RTP_F32)
-    hipLaunchKernelGGL(gather_kernel<float>, grid, dim3(256), 0, s, (const float*)table, (long)ld_table,
-                       (long)row_begin, (long)row_count, (long)cols, ids, (float*)out, (long)ld_out, vec,
-                       (long)table_sg, (long)out_sg, scale, (const float*)pos, (long)ld_pos, (long)pos_sg,
-                       (long)batch);
-  else
-    hipLaunchKernelGGL(gather_kernel<bf16_t>, grid, dim3(256), 0, s, (const bf16_t*)table, (long)ld_table,
-                       (long)row_begin, (long)row_count, (long)cols, ids, (bf16_t*)out, (long)ld_out, vec,
-                       (long)table_sg, (long)out_sg, scale, (const bf16_t*)pos, (long)ld_pos, (long)pos_sg,
-                       (long)batch);
+#define RTP_GATHER(T, V, POS)                                                                                          \
+  hipLaunchKernelGGL((gather_kernel<T, V, POS>), grid, dim3(256), 0, s, (const T*)table, (long)ld_table, (long)row_begin, \
+                     (long)row_count, (int)per_row, make_fastdiv((unsigned)per_row), (int)(per_row * groups), ids, (long)n_ids, \
+                     (T*)out, (long)ld_out, (long)table_sg, (long)out_sg, scale, (const T*)pos, (long)ld_pos, (long)pos_sg, \
+                     make_fastdiv((unsigned)batch))
+#define RTP_GATHER_V(T, V) do { if (pos) RTP_GATHER(T, V, true); else RTP_GATHER(T, V, false); } while (0)
+  if (dtype == RTP_F32) {
+    if (vec) RTP_GATHER_V(float, 4); else RTP_GATHER_V(float, 1);
+  } else {
+    if (vec) RTP_GATHER_V(bf16_t, 8); else RTP_GATHER_V(bf16_t, 1);
+  }
+#undef RTP_GATHER_V
+#undef RTP_GATHER
   RTP_LAUNCH_CHECK();
   return RTP_OK;
 }
@@ -603,6 +938,86 @@ extern "C" int rtp_embedding_backward(void* stream, int dtype, const void* grad_
     if (aligned) RTP_EMB_BWD(bf16_t, bf16_t, 8); else RTP_EMB_BWD(bf16_t, bf16_t, 1);
   }
 #undef RTP_EMB_BWD
+  RTP_LAUNCH_CHECK();
+  return RTP_OK;
+}
+
+extern "C" int rtp_embedding_backward_grouped_supported(int64_t n_ids, int64_t row_count) {
+  return n_ids > 0 && n_ids <= kGroupMaxIds && row_count > 0 && row_count < (1ll << 26) ? 1 : 0;
+}
+
+extern "C" size_t rtp_embedding_backward_grouped_workspace_bytes(int64_t n_ids, int64_t row_count) {
+  if (!rtp_embedding_backward_grouped_supported(n_ids, row_count)) return 256;
+  return group_layout(n_ids, row_count).total;
+}
+
+extern "C" int rtp_embedding_backward_grouped(void* stream, int dtype, const void* grad_out, int64_t ld_grad_out,
+                                              int64_t n_ids, const int64_t* ids, void* grad_table, int64_t ld_grad_table,
+                                              int grad_table_f32, int64_t row_begin, int64_t row_count, int64_t cols,
+                                              int64_t padding_idx, int scale_by_freq, int zero_fill, int64_t groups,
+                                              int64_t grad_out_sg, int64_t grad_table_sg, float grad_scale, float* master,
+                                              void* weights, float lr, float clip, int store_grad, void* workspace,
+                                              size_t workspace_bytes) {
+  const char* who = "rtp_embedding_backward_grouped";
+  RTP_REQUIRE(grad_out && grad_table && ids && workspace, "%s: null pointer", who);
+  RTP_REQUIRE(rtp_embedding_backward_grouped_supported(n_ids, row_count), "%s: %lld ids, %lld rows out of range", who,
+              (long long)n_ids, (long long)row_count);
+  RTP_REQUIRE(dtype == RTP_F32 || dtype == RTP_BF16, "%s: unknown dtype %d", who, dtype);
+  RTP_REQUIRE(groups >= 1 && groups < 65536 && cols >= 0 && cols * groups < (1ll << 30) && ld_grad_out >= cols &&
+                  ld_grad_table >= cols,
+              "%s: bad shape", who);
+  if (master != nullptr) {
+    RTP_REQUIRE(!grad_table_f32 || dtype == RTP_F32, "%s: with an update the gradient table has the table's dtype", who);
+    RTP_REQUIRE(dtype != RTP_F32 || weights == nullptr || weights == (void*)master, "%s: fp32 tables are their own master", who);
+    RTP_REQUIRE(zero_fill || !store_grad, "%s: a stored gradient beside the update starts from a zero fill", who);
+    if (!store_grad) zero_fill = 0;  // the update replaces the dense gradient: nothing to fill
+    if (dtype == RTP_F32) weights = nullptr;
+  } else {
+    store_grad = 1;
+  }
+  if (cols == 0) return RTP_OK;
+  RTP_REQUIRE((uintptr_t)workspace % 256 == 0, "%s: workspace must be 256-byte aligned", who);
+  const GroupLayout L = group_layout(n_ids, row_count);
+  if (workspace_bytes < L.total) return fail(RTP_ERR_WORKSPACE, "%s: workspace %zu < required %zu", who, workspace_bytes, L.total);
+  char* w = (char*)workspace;
+  int *offs = (int*)(w + L.offs), *pos = (int*)(w + L.pos), *nlong = (int*)(w + L.nlong), *longs = (int*)(w + L.longs);
+  hipStream_t s = (hipStream_t)stream;
+  const size_t esz = dtype == RTP_F32 ? 4 : 2, gsz = (dtype == RTP_F32 || grad_table_f32) ? 4 : 2;
+  {
+    ProfileScope prof(s, "embedding_group_ids", 0.0, 8.0 * (double)n_ids);
+    hipLaunchKernelGGL(group_ids_kernel, dim3((unsigned)L.slices), dim3(kGroupThreads), 0, s, ids, (int)n_ids, (long)row_begin,
+                       (int)row_count, (long)padding_idx, L.rows_per, offs, pos, nlong, longs, L.long_cap);
+    RTP_LAUNCH_CHECK();
+  }
+  const int64_t vec = 16 / (int64_t)esz;
+  const bool aligned = cols % vec == 0 && (uintptr_t)grad_out % 16 == 0 && (ld_grad_out * esz) % 16 == 0 &&
+                       (grad_out_sg * esz) % 16 == 0 && (uintptr_t)grad_table % 16 == 0 &&
+                       (ld_grad_table * gsz) % 16 == 0 && (grad_table_sg * gsz) % 16 == 0 &&
+                       (master == nullptr || (uintptr_t)master % 16 == 0) &&
+                       (weights == nullptr || (uintptr_t)weights % 16 == 0);
+  const int W = aligned && dtype == RTP_BF16 ? 2 : 1;
+  const int64_t chunks = ceil_div(cols / W * groups, 256), long_wgs = n_ids / kLongRow * chunks;
+  RTP_REQUIRE(long_wgs + ceil_div(row_count, 4) < (1ll << 31), "%s: grid too large", who);
+  const dim3 grid((unsigned)(long_wgs + ceil_div(row_count, 4)));
+  const size_t lds = (size_t)ceil_div(ceil_div(n_ids, 32), 256) * 1024 + 8192 * 2;
+  ProfileScope prof(s, "embedding_backward_grouped", (double)groups * n_ids * cols,
+                    (double)groups * cols * ((double)n_ids * esz + (zero_fill ? (double)row_count : 2.0 * n_ids) * gsz));
+#define RTP_EMB_GROUPED(T, G, V, W_)                                                                                    \
+  do {                                                                                                                \
+    GroupedBwd<T, G> a{(const T*)grad_out, (long)ld_grad_out, (long)grad_out_sg, (G*)grad_table, (long)ld_grad_table,   \
+                       (long)grad_table_sg, master, (T*)weights, grad_scale, lr, clip, scale_by_freq, zero_fill ? 1 : 0, \
+                       store_grad, zero_fill, (int)n_ids, (int)row_count, (int)groups, (int)cols, offs, pos, nlong,      \
+                       longs, L.slices, L.long_cap};                                                                  \
+    hipLaunchKernelGGL((grouped_bwd_kernel<T, G, V, W_>), grid, dim3(256), lds, s, a, (int)long_wgs, (int)chunks);      \
+  } while (0)
+  if (dtype == RTP_F32) {
+    if (aligned) RTP_EMB_GROUPED(float, float, 4, 1); else RTP_EMB_GROUPED(float, float, 1, 1);
+  } else if (grad_table_f32) {
+    if (aligned) RTP_EMB_GROUPED(bf16_t, float, 8, 2); else RTP_EMB_GROUPED(bf16_t, float, 1, 1);
+  } else {
+    if (aligned) RTP_EMB_GROUPED(bf16_t, bf16_t, 8, 2); else RTP_EMB_GROUPED(bf16_t, bf16_t, 1, 1);
+  }
+#undef RTP_EMB_GROUPED
   RTP_LAUNCH_CHECK();
   return RTP_OK;
 }

@@ -23,28 +23,6 @@ namespace rtp {
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
-// Division of a 32-bit unsigned number by a launch constant with a multiply-high and two shifts (Granlund and
-// Montgomery's round-up method, exact for every 32-bit dividend): integer division by a run-time value costs a
-// few dozen dependent instructions on this hardware, and the wave-specialised kernel would otherwise do ten of
-// them before it can issue its first load.
-struct FastDiv {
-  unsigned d, mul, s1, s2;
-};
-inline FastDiv make_fastdiv(unsigned d) {
-  FastDiv f;
-  f.d = d;
-  unsigned s = 0;
-  while ((1ull << s) < d) ++s;  // ceil(log2 d)
-  f.mul = (unsigned)((((1ull << s) - d) << 32) / d + 1);
-  f.s1 = s < 1 ? s : 1;
-  f.s2 = s < 1 ? 0 : s - 1;
-  return f;
-}
-__device__ __forceinline__ unsigned fast_div(unsigned n, const FastDiv& f) {
-  const unsigned t = __umulhi(n, f.mul);
-  return (t + ((n - t) >> f.s1)) >> f.s2;
-}
-
 struct GemmArgs {
   const char* a;
   const char* b;

@@ -88,6 +88,8 @@ PyObject* invoke(R (*f)(A...), const char* name, PyObject* const* args, Py_ssize
   X(rtp_embedding_gather) X(rtp_embedding_gather_scale_pos) P(rtp_embedding_scatter_workspace_bytes)                  \
   X(rtp_embedding_sort_ids) X(rtp_embedding_scatter_add_det) X(rtp_embedding_scatter_add_scaled)                      \
   X(rtp_embedding_scatter_add_sgd) P(rtp_embedding_backward_supported) X(rtp_embedding_backward)                      \
+  P(rtp_embedding_backward_grouped_supported) P(rtp_embedding_backward_grouped_workspace_bytes)                       \
+  X(rtp_embedding_backward_grouped)                                                                                   \
   X(rtp_softmax_fwd_masks) X(rtp_softmax_bwd) P(rtp_attn_supported) X(rtp_attn_fwd) X(rtp_attn_bwd)                   \
   P(rtp_attn_flash_supported) X(rtp_attn_flash_fwd) X(rtp_attn_flash_bwd) P(rtp_layernorm_supported)                  \
   X(rtp_add_layernorm_fwd) P(rtp_layernorm_bwd_workspace_bytes) X(rtp_layernorm_bwd) P(rtp_layernorm_bwd_blocks)      \

@@ -72,10 +72,10 @@ class _EmbeddingFn(torch.autograd.Function):
         g2 = dout.reshape(-1, layer.embedding_dim)
         if g2.stride(1) != 1:
             g2 = g2.contiguous()
-        # up to a few thousand tokens: one launch per run of shards, from the raw ids; longer steps sort the ids once
-        # and scatter-add per run
-        onepass = ops.embedding_backward_supported(flat_ids.numel())
-        workspace = None if onepass else ops.embedding_sort_ids(flat_ids)
+        # one or two launches per run of shards straight from the ids; steps beyond that (more than 2^18 tokens) sort the
+        # ids once and scatter-add per run
+        form = ops.embedding_backward_form(flat_ids.numel(), layer.num_embeddings)
+        workspace = None if form else ops.embedding_sort_ids(flat_ids)
         pad = -1 if layer.padding_idx is None else layer.padding_idx
         if store.on_backward is not None:
             store.on_backward(store)
@@ -87,8 +87,9 @@ class _EmbeddingFn(torch.autograd.Function):
             kw = _fused(store, accumulate, first, cnt, store.offsets[0], store.numels[0])
             common = dict(padding_idx=pad, scale_by_freq=layer.scale_grad_by_freq, zero_fill=not accumulate, groups=cnt,
                           grad_out_sg=d_s, grad_table_sg=store.grads.shape[1], grad_scale=ctx.grad_scale, **kw)
-            if onepass:
-                ops.embedding_backward(g2[:, first * d_s:(first + 1) * d_s], flat_ids, table, **common)
+            if form:
+                ops.embedding_backward(g2[:, first * d_s:(first + 1) * d_s], flat_ids, table, grouped=form == "grouped",
+                                       **common)
             else:
                 ops.embedding_scatter_add(g2[:, first * d_s:(first + 1) * d_s], flat_ids.numel(), workspace, table,
                                           **common)

@@ -304,13 +304,28 @@ def embedding_backward_supported(n_ids: int) -> bool:
     return bool(_lib.native().rtp_embedding_backward_supported(int(n_ids)))
 
 
+# The one-launch form stages all ids in every token's workgroup, n^2 words of LDS traffic, and sums a frequent id's rows one at
+# a time; the grouped form costs a second launch.  bf16, 10240 x 2048 table, one / grouped, us: 256 ids 10 / 17; 1024 ids
+# 14 / 25 uniform, 41 / 33 by word frequency; 2048 ids 21 / 25 and 79 / 37; 4096 ids 38 / 26 and 143 / 46.
+EMBEDDING_ONE_LAUNCH_IDS = 1024
+
+
+def embedding_backward_form(n_ids: int, rows: int) -> Optional[str]:
+    """Which backward takes a step of n_ids tokens over a table of `rows` rows straight from its ids: "one" launch,
+    "grouped" by row in two, or None -- the sort and scatter-add -- beyond the grouped form's sizes."""
+    if n_ids <= EMBEDDING_ONE_LAUNCH_IDS:
+        return "one"
+    return "grouped" if native().rtp_embedding_backward_grouped_supported(n_ids, rows) else None
+
+
 def embedding_backward(grad_out: torch.Tensor, ids: torch.Tensor, grad_table: torch.Tensor, *, row_begin: int = 0,
                        padding_idx: int = -1, scale_by_freq: bool = False, zero_fill: bool = True, groups: int = 1,
                        grad_out_sg: int = 0, grad_table_sg: int = 0, grad_scale: float = 1.0,
-                       sgd: Optional["FusedSgd"] = None, sgd_master: int = 0, sgd_weights: int = 0) -> None:
-    """embedding_sort_ids + embedding_scatter_add in one launch, from the raw ids (contiguous int64, one per row of
-    grad_out): same arguments, same results bit for bit; rows no token names are cleared by the same launch when
-    zero_fill.  Only for steps embedding_backward_supported() accepts."""
+                       sgd: Optional["FusedSgd"] = None, sgd_master: int = 0, sgd_weights: int = 0,
+                       grouped: bool = False) -> None:
+    """embedding_sort_ids + embedding_scatter_add in one launch (or, `grouped`, in two), from the raw ids (contiguous
+    int64, one per row of grad_out): same arguments, same results bit for bit; rows no token names are cleared by the
+    same launch when zero_fill.  For the steps embedding_backward_form() names."""
     for t in (grad_out, ids, grad_table):
         _dev(t)
     n, cols, ld_go = _mat(grad_out, "grad_out")
@@ -322,14 +337,18 @@ def embedding_backward(grad_out: torch.Tensor, ids: torch.Tensor, grad_table: to
     if sgd is not None and (not zero_fill or grad_table.dtype != grad_out.dtype):
         raise ValueError("embedding_backward: the fused update takes the whole gradient of the step, in the table's "
                          "own dtype")
-    native().rtp_embedding_backward(dtype_code(grad_out.dtype), grad_out.data_ptr(), ld_go, n, ids.data_ptr(),
-                                    grad_table.data_ptr(), ld_gt, int(grad_table.dtype == torch.float32), row_begin,
-                                    rows, cols, -1 if padding_idx is None else padding_idx, int(scale_by_freq),
-                                    int(zero_fill), groups, grad_out_sg, grad_table_sg, float(grad_scale),
-                                    (sgd_master or None) if sgd is not None else None,
-                                    (sgd_weights or None) if sgd is not None else None,
-                                    sgd.lr if sgd is not None else 0.0, sgd.clip if sgd is not None else 0.0,
-                                    int(sgd.keep_grads) if sgd is not None else 1)
+    args = (dtype_code(grad_out.dtype), grad_out.data_ptr(), ld_go, n, ids.data_ptr(), grad_table.data_ptr(), ld_gt,
+            int(grad_table.dtype == torch.float32), row_begin, rows, cols, -1 if padding_idx is None else padding_idx,
+            int(scale_by_freq), int(zero_fill), groups, grad_out_sg, grad_table_sg, float(grad_scale),
+            (sgd_master or None) if sgd is not None else None, (sgd_weights or None) if sgd is not None else None,
+            sgd.lr if sgd is not None else 0.0, sgd.clip if sgd is not None else 0.0,
+            int(sgd.keep_grads) if sgd is not None else 1)
+    if not grouped:
+        native().rtp_embedding_backward(*args)
+        return
+    nbytes = native().rtp_embedding_backward_grouped_workspace_bytes(n, rows)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=ids.device)
+    native().rtp_embedding_backward_grouped(*args, ws, nbytes)
 
 
 def embedding_scatter_add(grad_out: torch.Tensor, n_ids: int, workspace: torch.Tensor, grad_table: torch.Tensor,

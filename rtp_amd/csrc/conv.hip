@@ -1,14 +1,19 @@
 // Out-channel-sharded 2-D convolution as an implicit GEMM on the MFMA: the patch matrix
 //   patches[(n*Ho + ho)*Wo + wo][(ci*kh + i)*kw + j] = x[n][ci][ho*sh - ph + i*dh][wo*sw - pw + j*dw]   (0 outside)
-// is never written to memory.  One tile kernel computes  C[m][n] = sum_k A(m, k) * B(n, k)  for operands given as index
-// functions; the three products of the layer are three pairs of such functions:
-//   forward          y[img][co][ho][wo] = sum_k W_s[co][k] * patches[pix][k] + b_s[co]         (m = co, n = pix)
-//   weight gradient  dW_s[co][k']       = sum_pix dy[img][co][ho][wo] * patches[pix][k']       (m = co, n = k')
-//   input gradient   dx[img][ci][h][w]  = sum_(s,co,i,j) W_s[co][ci][i][j] * dy[img][co][ho][wo]   (m = ci, n = (img,h,w))
-// A shard's weight [Co_s, Ci, kh, kw] is, as stored in its flat buffer, the row-major [Co_s, Ci*kh*kw] operand.  The
-// lanes of the MFMA result run along n, which is the contiguous direction of every output (NCHW pixels, or the
-// weight's k'), so stores are coalesced and the forward needs no layout copy.  Correctness first: operands are
-// gathered element by element (index arithmetic per element); the reference's use of the layer is the MNIST demo.
+// is never written to memory.  Three products, one tile kernel  C[m][n] = sum_k A(m, k) * B(n, k):
+//   forward          y[img][co][ho][wo] = sum_k W[co][k] * patches[pix][k] + b[co]           (m = co, n = pix)
+//   weight gradient  dW[co][k']         = sum_pix dy[img][co][ho][wo] * patches[pix][k']     (m = co, n = k')
+//   input gradient   dx[img][ci][h][w]  = sum_(co,i,j) W[co][ci][i][j] * dy[img][co][ho][wo] (m = ci, n = (img,h,w))
+// co runs over the channels of all shards of the run: shard s holds channels s*n_s .. of it at s*numel, so a layer whose
+// shards own 16 channels each still fills a 64-row tile.  The lanes of the MFMA result run along n, which is the
+// contiguous direction of every output (NCHW pixels, or the weight's k'), so stores are coalesced and the forward needs
+// no layout copy.
+//
+// What bounds it is the gather, so an operand element costs an add, a bounds test and a load: a thread keeps its pixel (or
+// its rows) for the whole contraction, and everything that depends on k alone -- offset inside an image, kernel position --
+// is worked out once per slab by one thread per k and handed round through LDS.  The first version called an index function
+// with five integer divisions per element and gave every shard tiles of its own: MNIST's second convolution (64 x 32 x 26 x
+// 26 -> 64, four shards, fp32) took 127 + 162 + 196 us forward / input / weight gradient; this one takes 29 + 43 + 34.
 #include <algorithm>
 
 #include "common.h"
@@ -20,185 +25,17 @@ namespace rtp {
 typedef __attribute__((ext_vector_type(8))) __bf16 conv_bf16x8;
 typedef __attribute__((ext_vector_type(16))) float conv_f32x16;
 
-// Sizes and indices are 32-bit on the device (integer division per gathered element; the host checks the ranges);
-// only the final address arithmetic is 64-bit.
+// Sizes and indices are 32-bit on the device (the host checks the ranges); addresses are 64-bit.
 struct ConvGeom {
   int n, c, h, w, kh, kw, sh, sw, ph, pw, dh, dw, ho, wo;
 };
 
-// A 4-D activation addressed by element strides (any memory format).
-template <typename T>
-struct Act4 {
-  const T* p;
-  long sn, sc, sh, sw;
-  __device__ __forceinline__ T at(int n, int c, int h, int w) const { return p[n * sn + c * sc + h * sh + w * sw]; }
+// Element strides of a 4-D activation (any memory format).
+struct Strides {
+  long n, c, h, w;
 };
 
-// ---- operand functions: value(group, row, k); the kernel never asks beyond rows() x depth() ----
-
-// Rows of the weights of the shards of a run: W_g[row][k], g = group.
-template <typename T>
-struct WeightRows {
-  const T* w;  // first shard of the run, weight at element w_off of every shard row
-  long numel, kp;
-  __device__ __forceinline__ T operator()(int g, int row, int k) const { return w[g * numel + (long)row * kp + k]; }
-};
-
-// patches[pix][k] (TRANSPOSED: asked as (row = k, k = pix)).
-template <typename T, bool TRANSPOSED>
-struct Patches {
-  Act4<T> x;
-  ConvGeom g;
-  __device__ __forceinline__ T operator()(int, int row, int k) const {
-    const int pix = TRANSPOSED ? k : row, kk = TRANSPOSED ? row : k;
-    const int j = kk % g.kw, i = (kk / g.kw) % g.kh, ci = kk / (g.kw * g.kh);
-    const int wo = pix % g.wo, ho = (pix / g.wo) % g.ho, n = pix / (g.wo * g.ho);
-    const int h = ho * g.sh - g.ph + i * g.dh, w = wo * g.sw - g.pw + j * g.dw;
-    if (h < 0 || h >= g.h || w < 0 || w >= g.w) return from_f32<T>(0.0f);
-    return x.at(n, ci, h, w);
-  }
-};
-
-// dy[img][co0 + g*n_s + row][ho][wo] asked as (row = co, k = pix).
-template <typename T>
-struct GradRowsT {
-  Act4<T> dy;
-  int co0, n_s, wo, howo;
-  __device__ __forceinline__ T operator()(int g, int row, int k) const {
-    const int img = k / howo, r = k - img * howo;
-    return dy.at(img, co0 + g * n_s + row, r / wo, r % wo);
-  }
-};
-
-// Input gradient, first operand: W_s[co][ci][i][j] asked as (row = ci, k = ((s*n_s + co)*kh + i)*kw + j).
-template <typename T>
-struct WeightByInput {
-  const T* w;
-  long numel;
-  int n_s, c, khkw;
-  __device__ __forceinline__ T operator()(int, int row, int k) const {
-    const int ij = k % khkw, sco = k / khkw, s = sco / n_s, co = sco - s * n_s;
-    return w[s * numel + ((long)co * c + row) * khkw + ij];
-  }
-};
-
-// Input gradient, second operand: the entry of dy that patch position (i, j) of output channel co reads at input
-// pixel (img, h, w), asked as (row = (img*H + h)*W + w, k as above); 0 where no output pixel reads it.
-template <typename T>
-struct GradByInput {
-  Act4<T> dy;
-  ConvGeom g;
-  int co0;
-  __device__ __forceinline__ T operator()(int, int row, int k) const {
-    const int j = k % g.kw, i = (k / g.kw) % g.kh, sco = k / (g.kw * g.kh);
-    const int w = row % g.w, h = (row / g.w) % g.h, img = row / (g.w * g.h);
-    const int hn = h + g.ph - i * g.dh, wn = w + g.pw - j * g.dw;
-    if (hn < 0 || wn < 0 || hn % g.sh != 0 || wn % g.sw != 0) return from_f32<T>(0.0f);
-    const int ho = hn / g.sh, wo = wn / g.sw;
-    if (ho >= g.ho || wo >= g.wo) return from_f32<T>(0.0f);
-    return dy.at(img, co0 + sco, ho, wo);
-  }
-};
-
-// ---- where a result element goes ----
-
-// forward: y[img][co0 + g*n_s + m][ho][wo] (contiguous NCHW with `co_total` channels) = acc + bias_g[m]
-template <typename T>
-struct StoreNCHW {
-  T* y;
-  const T* bias;  // of the run's first shard (element bias_off of its row), or nullptr
-  long numel;
-  int co0, n_s, co_total, howo;
-  __device__ __forceinline__ void operator()(int g, int, int m, int n, float v) const {
-    if (bias != nullptr) v += to_f32(bias[g * numel + m]);
-    const int img = n / howo, r = n - img * howo;
-    y[((long)img * co_total + co0 + g * n_s + m) * howo + r] = from_f32<T>(v);
-  }
-  __device__ __forceinline__ void rowsum(int, int, int, float) const {}
-  static constexpr bool kRowSum = false;
-};
-
-// weight gradient: grads_g[w_off + m*kp + n] (+)= acc; the row sums of the first operand are the bias gradient.
-// With the contraction (the pixels) split over several workgroups, each writes its fp32 partial sums
-// part[split][g][m][0 .. kp] (entry kp of a row: the partial row sum) and wgrad_reduce_kernel adds them in order.
-template <typename T>
-struct StoreWeightGrad {
-  T* grads;  // gradient row of the run's first shard
-  long numel, w_off, b_off, kp;
-  int accumulate;
-  float* part;  // nullptr: one workgroup per output tile, results go straight to grads
-  int groups, n_s;
-  __device__ __forceinline__ float* partial(int g, int split, int m) const {
-    return part + (((long)split * groups + g) * n_s + m) * (kp + 1);
-  }
-  __device__ __forceinline__ void operator()(int g, int split, int m, int n, float v) const {
-    if (part != nullptr) {
-      partial(g, split, m)[n] = v;
-      return;
-    }
-    T* dst = grads + g * numel + w_off + (long)m * kp + n;
-    if (accumulate) v += to_f32(*dst);
-    *dst = from_f32<T>(v);
-  }
-  __device__ __forceinline__ void rowsum(int g, int split, int m, float v) const {
-    if (part != nullptr) {
-      partial(g, split, m)[kp] = v;
-      return;
-    }
-    if (b_off < 0) return;
-    T* dst = grads + g * numel + b_off + m;
-    if (accumulate) v += to_f32(*dst);
-    *dst = from_f32<T>(v);
-  }
-  static constexpr bool kRowSum = true;
-};
-
-// grads (+)= sum over the splits, ascending, of the partial sums: one thread per entry of a shard's [n_s, kp + 1] block
-template <typename T>
-__global__ __launch_bounds__(256) void wgrad_reduce_kernel(StoreWeightGrad<T> o, int splits) {
-  const long per = (long)o.n_s * (o.kp + 1), total = per * o.groups;
-  for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (long)gridDim.x * blockDim.x) {
-    const int g = (int)(idx / per);
-    const long r = idx - g * per;
-    const int m = (int)(r / (o.kp + 1)), n = (int)(r - m * (o.kp + 1));
-    float v = 0.0f;
-    for (int sp = 0; sp < splits; ++sp) v += o.partial(g, sp, m)[n];
-    T* dst;
-    if (n < o.kp) {
-      dst = o.grads + g * o.numel + o.w_off + (long)m * o.kp + n;
-    } else {
-      if (o.b_off < 0) continue;
-      dst = o.grads + g * o.numel + o.b_off + m;
-    }
-    if (o.accumulate) v += to_f32(*dst);
-    *dst = from_f32<T>(v);
-  }
-}
-
-// input gradient: out[img][m][h][w] = acc + addend, out / addend in T or fp32 (the sum over rotation windows is kept
-// in fp32 and rounded once)
-template <typename T>
-struct StoreInputGrad {
-  void* out;
-  const void* addend;
-  int out_f32, addend_f32;
-  int c, hw;
-  __device__ __forceinline__ void operator()(int, int, int m, int n, float v) const {
-    const int img = n / hw, r = n - img * hw;
-    const long idx = ((long)img * c + m) * hw + r;
-    if (addend != nullptr)
-      v += addend_f32 ? reinterpret_cast<const float*>(addend)[idx] : to_f32(reinterpret_cast<const T*>(addend)[idx]);
-    if (out_f32)
-      reinterpret_cast<float*>(out)[idx] = v;
-    else
-      reinterpret_cast<T*>(out)[idx] = from_f32<T>(v);
-  }
-  __device__ __forceinline__ void rowsum(int, int, int, float) const {}
-  static constexpr bool kRowSum = false;
-};
-
-// ---- the tile kernel: 64 x 64 outputs per workgroup, K in slabs of 32, four waves of one 32 x 32 MFMA block ----
-constexpr int kConvTile = 64, kConvSlab = 32;
+constexpr int kConvSlab = 32;  // contraction per slab
 
 template <typename T>
 struct ConvFrag;
@@ -221,42 +58,255 @@ __device__ __forceinline__ void conv_mma(const ConvFrag<float>& a, const ConvFra
   for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a.f[e], b.f[e], c, 0, 0, 0);
 }
 
-template <typename T, class OpA, class OpB, class Out>
-__global__ __launch_bounds__(256) void conv_igemm_kernel(OpA opa, OpB opb, Out out, int M, int N, int K, int splits,
-                                                         int kchunk) {
+enum ConvPass { kConvFwd, kConvDgrad, kConvWgrad };
+
+template <typename T>
+struct ConvArgs {
+  ConvGeom g;
+  FastDiv d_pix_img, d_pix_row;  // pixels per image and per row of the pixel grid (output, or input for the input gradient)
+  FastDiv d_khkw, d_kw, d_ns, d_sh, d_sw;
+  int M, N, K, splits, kchunk;
+  int n_s, kp, khkw;             // channels per shard, weights per channel, kernel positions
+  long numel;                    // elements per shard row
+  const T* act;                  // x (forward, weight gradient) or dy (input gradient), at the run's first channel
+  Strides s;
+  const T* w;                    // weights of the run's first shard
+  const T* dy;                   // weight gradient: dy at the run's first channel
+  Strides sd;
+  // outputs
+  T* y;                          // forward: NCHW with co_total channels, at the run's first channel
+  const T* bias;
+  int co_total;
+  void* dx;                      // input gradient, contiguous NCHW
+  const void* addend;
+  int dx_f32, addend_f32;
+  T* grads;                      // weight gradient rows
+  long w_off, b_off;
+  int accumulate;
+  float* part;                   // fp32 partial sums [split][M][kp + 1] (entry kp: the row sum), or null: one split
+};
+
+// An operand read element by element at byte offsets from its base: buffer loads with a 32-bit offset, which return zero
+// for an offset beyond the buffer -- how an element outside the image or the contraction becomes zero without a branch, a
+// mask or a select --, or plain 64-bit addresses for an operand of 4 GiB or more (WIDE).
+constexpr unsigned kBeyond = 0xffffff00u;
+template <typename T, bool WIDE>
+struct Gather {
+  typedef unsigned off_t;
+  __amdgpu_buffer_rsrc_t r;
+  __device__ __forceinline__ explicit Gather(const T* base)
+      : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), 0, kBeyond, 0x00020000)) {}
+  __device__ __forceinline__ T get(unsigned off, bool ok) const {
+    off = ok ? off : kBeyond;
+    if constexpr (sizeof(T) == 4)
+      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0));
+    else
+      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b16(r, (int)off, 0, 0));
+  }
+};
+template <typename T>
+struct Gather<T, true> {
+  typedef long off_t;
+  const char* base;
+  __device__ __forceinline__ explicit Gather(const T* b) : base(reinterpret_cast<const char*>(b)) {}
+  __device__ __forceinline__ T get(long off, bool ok) const {
+    return ok ? *reinterpret_cast<const T*>(base + off) : from_f32<T>(0.0f);
+  }
+};
+// What depends on a k of the slab alone.
+template <class Off>
+struct alignas(16) KEntry {
+  Off b;       // byte offset of the gathered activation relative to the pixel
+  int di, dj;  // kernel position in input pixels; di = kOutside: beyond the contraction
+};
+constexpr int kOutside = 1 << 30;
+
+// BM x BN outputs per workgroup (BM * BN = 4096), four waves, each one row of MFMA blocks wide: 64 x 64 as 2 x 2 waves, or
+// 32 x 128 as 1 x 4 for products of at most 32 rows.  LDS is double buffered and elements are requested two slabs ahead of
+// their MFMAs: the grids are small (MNIST's second convolution: two waves per SIMD), so the trip to memory has to
+// be covered by the wave itself.  SIMPLE: forward and weight gradient without padding (every gathered element exists),
+// input gradient with unit strides.
+template <typename T, ConvPass PASS, int BM, int BN, bool SIMPLE, bool WIDE>
+__global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
+  typedef typename Gather<T, WIDE>::off_t Off;
   constexpr int PITCH = kConvSlab + 16 / (int)sizeof(T);  // elements; rows stay 16-byte aligned
-  __shared__ __attribute__((aligned(16))) T As[kConvTile * PITCH];
-  __shared__ __attribute__((aligned(16))) T Bs[kConvTile * PITCH];
+  constexpr int NA = BM * kConvSlab / 256, NB = BN * kConvSlab / 256;
+  constexpr int ES = (int)sizeof(T);
+  __shared__ __attribute__((aligned(16))) T As[2][BM * PITCH];
+  __shared__ __attribute__((aligned(16))) T Bs[2][BN * PITCH];
+  __shared__ KEntry<Off> tab[PASS == kConvWgrad ? 1 : 4][PASS == kConvWgrad ? BN : kConvSlab];
+  __shared__ Off tab_a[4][kConvSlab];  // input gradient: offset of the weight
+  const ConvGeom& g = p.g;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1, li = lane & 31, g = lane >> 5;
-  const int m0 = blockIdx.y * kConvTile, n0 = blockIdx.x * kConvTile;
-  // blockIdx.z = (group, part of the contraction): this workgroup sums k in [kb, ke)
-  const int grp = blockIdx.z / splits, split = blockIdx.z - grp * splits;
-  const int kb = split * kchunk, ke = kb + kchunk < K ? kb + kchunk : K;
-  const int lr = tid >> 2, lk = (tid & 3) * 8;  // the thread fills 8 consecutive k of one row of either operand
+  const int wm = BM == 64 ? wave >> 1 : 0, wn = BM == 64 ? wave & 1 : wave, li = lane & 31, lg = lane >> 5;
+  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+  const int split = blockIdx.z, kb = split * p.kchunk, ke = min(kb + p.kchunk, p.K);
+  const Gather<T, WIDE> act(p.act), wts(PASS == kConvWgrad ? p.dy : p.w);  // wts: operand A
+
+  // kernel position and activation offset of contraction index (or weight column) k
+  auto entry_of = [&](int k, bool live, Off* a) {
+    KEntry<Off> e;
+    const unsigned ci = fast_div((unsigned)k, p.d_khkw), ij = k - ci * p.khkw;  // ci: the channel of the gathered operand
+    const unsigned i = fast_div(ij, p.d_kw), j = ij - i * g.kw;
+    const int di = (int)i * g.dh, dj = (int)j * g.dw;
+    e.di = live ? di : kOutside;
+    e.dj = dj;
+    if (PASS == kConvDgrad) {
+      const unsigned sft = fast_div(ci, p.d_ns), co = ci - sft * p.n_s;
+      *a = live ? (Off)((sft * p.numel + (long)co * p.kp + ij) * ES) : (Off)0;
+      e.b = (Off)((ci * p.s.c - (SIMPLE ? di * p.s.h + dj * p.s.w : 0)) * ES);
+    } else {
+      e.b = live ? (Off)((ci * p.s.c + di * p.s.h + dj * p.s.w) * ES) : (Off)0;
+    }
+    return e;
+  };
+  auto build_table = [&](int slab) {  // of the slab `slab` steps behind kb
+    if (PASS != kConvWgrad && tid < kConvSlab) {
+      const int k = kb + slab * kConvSlab + tid;
+      Off a = 0;
+      tab[PASS == kConvWgrad ? 0 : slab & 3][tid] = entry_of(min(k, p.K - 1), k < ke, &a);
+      if (PASS == kConvDgrad) tab_a[slab & 3][tid] = a;
+    }
+  };
+
+  // ---- operand A: k = tid % 32, rows tid / 32 + 8 q ----
+  const int ak = tid & 31, ar = tid >> 5;
+  Off aoff[NA];
+#pragma unroll
+  for (int q = 0; q < NA; ++q) {
+    const int m = min(m0 + ar + 8 * q, p.M - 1);
+    if (PASS == kConvFwd) {
+      const unsigned sft = fast_div((unsigned)m, p.d_ns);
+      aoff[q] = (Off)((sft * p.numel + (long)(m - sft * p.n_s) * p.kp) * ES);
+    } else if (PASS == kConvDgrad) {
+      aoff[q] = (Off)((long)m * p.khkw * ES);
+    } else {
+      aoff[q] = (Off)(m * p.sd.c * ES);
+    }
+  }
+  // ---- operand B ----
+  // forward / input gradient: the thread's pixel n, k = kq*NB + e;  weight gradient: k = tid % 32, rows tid / 32 + 8 q
+  const int bn = tid & (BN - 1), kq = tid / BN;
+  Off bpix = 0;
+  int bh = 0, bw = 0;
+  KEntry<Off> brow[PASS == kConvWgrad ? NB : 1];
+  // pixel -> offset, row and column of the gathered activation before the kernel position
+  auto locate = [&](int pix, int& h, int& w) {
+    const unsigned img = fast_div((unsigned)pix, p.d_pix_img);
+    const int r = pix - img * p.d_pix_img.d;
+    const unsigned y = fast_div((unsigned)r, p.d_pix_row);
+    const int x = r - y * p.d_pix_row.d;
+    if (PASS == kConvDgrad) {
+      h = (int)y + g.ph, w = x + g.pw;
+      return (Off)(((long)img * p.s.n + (SIMPLE ? h * p.s.h + w * p.s.w : 0)) * ES);
+    }
+    h = (int)y * g.sh - g.ph, w = x * g.sw - g.pw;
+    return (Off)(((long)img * p.s.n + h * p.s.h + w * p.s.w) * ES);
+  };
+  if (PASS != kConvWgrad) {
+    bpix = locate(min(n0 + bn, p.N - 1), bh, bw);
+    build_table(0), build_table(1), build_table(2);
+    __syncthreads();
+  } else {
+    Off unused;
+    if (tid < BN) tab[0][tid] = entry_of(min(n0 + tid, p.N - 1), n0 + tid < p.N, &unused);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NB; ++q) brow[PASS == kConvWgrad ? q : 0] = tab[0][(ar + 8 * q) & (BN - 1)];
+  }
+
+  struct Regs {
+    T a[NA], b[NB];
+  } reg[2];
+  // requests a slab (one behind the contraction: nothing but zeros)
+  auto fetch = [&](int slab, Regs& v) {
+    const int k0 = kb + slab * kConvSlab;
+    if (PASS == kConvWgrad) {
+      const bool live = k0 + ak < ke;
+      const int pix = live ? k0 + ak : p.K - 1;
+      int h, w;
+      const Off base = locate(pix, h, w);
+      const unsigned img = fast_div((unsigned)pix, p.d_pix_img);
+      const int r = pix - img * p.d_pix_img.d;
+      const unsigned yo = fast_div((unsigned)r, p.d_pix_row);
+      const Off d = (Off)(((long)img * p.sd.n + (long)yo * p.sd.h + (long)(r - yo * p.d_pix_row.d) * p.sd.w) * ES);
+#pragma unroll
+      for (int q = 0; q < NA; ++q) v.a[q] = wts.get(d + aoff[q], live);
+#pragma unroll
+      for (int q = 0; q < NB; ++q) {
+        const KEntry<Off>& e = brow[PASS == kConvWgrad ? q : 0];
+        const bool in = SIMPLE ? e.di != kOutside
+                               : ((unsigned)(h + e.di) < (unsigned)g.h) & ((unsigned)(w + e.dj) < (unsigned)g.w);
+        v.b[q] = act.get(base + e.b, live & in);
+      }
+      return;
+    }
+    const int slot = PASS == kConvWgrad ? 0 : slab & 3;
+    {
+      const bool live = k0 + ak < ke;
+      const Off off = PASS == kConvDgrad ? tab_a[slot][ak] : (Off)(k0 + ak) * ES;
+#pragma unroll
+      for (int q = 0; q < NA; ++q) v.a[q] = wts.get(aoff[q] + off, live);
+    }
+    KEntry<Off> e[NB];
+#pragma unroll
+    for (int q = 0; q < NB; ++q) e[q] = tab[slot][(kq * NB + q) & (kConvSlab - 1)];
+#pragma unroll
+    for (int q = 0; q < NB; ++q) {
+      if (PASS == kConvFwd) {
+        const bool in = SIMPLE ? e[q].di != kOutside
+                               : ((unsigned)(bh + e[q].di) < (unsigned)g.h) & ((unsigned)(bw + e[q].dj) < (unsigned)g.w);
+        v.b[q] = act.get(bpix + e[q].b, in);
+      } else if (SIMPLE) {
+        v.b[q] = act.get(bpix + e[q].b, ((unsigned)(bh - e[q].di) < (unsigned)g.ho) & ((unsigned)(bw - e[q].dj) < (unsigned)g.wo));
+      } else {
+        const int hn = bh - e[q].di, wn_ = bw - e[q].dj;
+        const int ho = (int)fast_div((unsigned)max(hn, 0), p.d_sh), wo = (int)fast_div((unsigned)max(wn_, 0), p.d_sw);
+        const bool in = (hn >= 0) & (wn_ >= 0) & (ho * g.sh == hn) & (wo * g.sw == wn_) & (ho < g.ho) & (wo < g.wo);
+        v.b[q] = act.get(bpix + e[q].b + (Off)((ho * p.s.h + wo * p.s.w) * ES), in);
+      }
+    }
+  };
+  float rsum[NA];
+#pragma unroll
+  for (int q = 0; q < NA; ++q) rsum[q] = 0.0f;
+  const bool want_rows = PASS == kConvWgrad && blockIdx.x == 0;
+  auto stash = [&](int buf, const Regs& v) {
+#pragma unroll
+    for (int q = 0; q < NA; ++q) {
+      As[buf][(ar + 8 * q) * PITCH + ak] = v.a[q];
+      if (PASS == kConvWgrad) rsum[q] += to_f32(v.a[q]);
+    }
+    if (PASS == kConvWgrad) {
+#pragma unroll
+      for (int q = 0; q < NB; ++q) Bs[buf][(ar + 8 * q) * PITCH + ak] = v.b[q];
+    } else {
+      constexpr int VEC = 16 / (int)sizeof(T);
+#pragma unroll
+      for (int u8 = 0; u8 < NB / VEC; ++u8) {
+        union {
+          uint4 q;
+          T e[VEC];
+        } u;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) u.e[e] = v.b[u8 * VEC + e];
+        *reinterpret_cast<uint4*>(&Bs[buf][bn * PITCH + kq * NB + u8 * VEC]) = u.q;
+      }
+    }
+  };
+
   conv_f32x16 acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-  float rsum = 0.0f;
-  for (int k0 = kb; k0 < ke; k0 += kConvSlab) {
-    T va[8], vb[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int k = k0 + lk + e;
-      va[e] = (m0 + lr < M && k < ke) ? opa(grp, m0 + lr, k) : from_f32<T>(0.0f);
-      vb[e] = (n0 + lr < N && k < ke) ? opb(grp, n0 + lr, k) : from_f32<T>(0.0f);
-    }
-    __syncthreads();  // the previous slab has been consumed
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      As[lr * PITCH + lk + e] = va[e];
-      Bs[lr * PITCH + lk + e] = vb[e];
-    }
-    __syncthreads();
-    if (Out::kRowSum && blockIdx.x == 0 && tid < kConvTile) {
-      // row sums of the first operand (a bias gradient): row tid, ascending k
-      for (int k = 0; k < kConvSlab; ++k) rsum += to_f32(As[tid * PITCH + k]);
-    }
+  const int slabs = (ke - kb + kConvSlab - 1) / kConvSlab;
+  fetch(0, reg[0]);
+  fetch(1, reg[1]);
+  stash(0, reg[0]);
+  __syncthreads();
+  // step s: requests slab s + 2 into the registers that slab s left, multiplies slab s, stores slab s + 1.  The table of slab
+  // s + 3 is built meanwhile: it is read behind the next barrier, and its slot (s + 3) % 4 by nobody now.
+  auto step = [&](int sl, Regs& mine, Regs& next, int buf) {
+    fetch(sl + 2, mine);  // unconditionally: the wait for slab s + 1 below counts the loads in flight
     constexpr int STEP = ConvFrag<T>::kStep, VEC = 16 / (int)sizeof(T);
 #pragma unroll
     for (int ks = 0; ks < kConvSlab / STEP; ++ks) {
@@ -264,19 +314,109 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(OpA opa, OpB opb, Out o
         uint4 q;
         ConvFrag<T> f;
       } a, b;
-      a.q = *reinterpret_cast<const uint4*>(&As[(wm * 32 + li) * PITCH + ks * STEP + g * VEC]);
-      b.q = *reinterpret_cast<const uint4*>(&Bs[(wn * 32 + li) * PITCH + ks * STEP + g * VEC]);
+      a.q = *reinterpret_cast<const uint4*>(&As[buf][(wm * 32 + li) * PITCH + ks * STEP + lg * VEC]);
+      b.q = *reinterpret_cast<const uint4*>(&Bs[buf][(wn * 32 + li) * PITCH + ks * STEP + lg * VEC]);
       conv_mma(a.f, b.f, acc);
     }
+    build_table(sl + 3);
+    stash(buf ^ 1, next);
+    __syncthreads();
+  };
+  for (int sl = 0; sl < slabs; sl += 2) {
+    step(sl, reg[0], reg[1], 0);
+    step(sl + 1, reg[1], reg[0], 1);  // past the last slab: zeros
   }
-  // accumulator register r of lane (li, g): row 8*(r/4) + 4*g + r%4 of the wave's block, column li
+
+  // ---- results: accumulator register r of lane (li, lg) is row 8*(r/4) + 4*lg + r%4 of the wave's block, column li ----
   const int col = n0 + wn * 32 + li;
+  if (col < p.N) {
+    long at = 0;
+    if (PASS != kConvWgrad) {
+      const unsigned img = fast_div((unsigned)col, p.d_pix_img);
+      const long plane = p.d_pix_img.d;
+      at = (long)img * (PASS == kConvFwd ? p.co_total : p.M) * plane + (col - (long)img * plane);
+    }
+    float bias[16];  // requested together: one trip to memory for the 16 rows
+    if (PASS == kConvFwd && p.bias != nullptr) {
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int row = m0 + wm * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
-    if (row < M && col < N) out(grp, split, row, col, acc[r]);
+      for (int r = 0; r < 16; ++r) {
+        const int m = min(m0 + wm * 32 + 8 * (r >> 2) + 4 * lg + (r & 3), p.M - 1);
+        const unsigned sft = fast_div((unsigned)m, p.d_ns);
+        bias[r] = to_f32(p.bias[sft * p.numel + (m - sft * p.n_s)]);
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bias[r] = 0.0f;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int m = m0 + wm * 32 + 8 * (r >> 2) + 4 * lg + (r & 3);
+      if (m >= p.M) continue;
+      float v = acc[r];
+      if (PASS == kConvFwd) {
+        v += bias[r];
+        p.y[at + (long)m * p.d_pix_img.d] = from_f32<T>(v);
+      } else if (PASS == kConvDgrad) {
+        // dx = acc + addend, either in T or fp32 (the sum over rotation windows is kept in fp32 and rounded once)
+        const long o = at + (long)m * p.d_pix_img.d;
+        if (p.addend != nullptr)
+          v += p.addend_f32 ? reinterpret_cast<const float*>(p.addend)[o] : to_f32(reinterpret_cast<const T*>(p.addend)[o]);
+        if (p.dx_f32)
+          reinterpret_cast<float*>(p.dx)[o] = v;
+        else
+          reinterpret_cast<T*>(p.dx)[o] = from_f32<T>(v);
+      } else if (p.part != nullptr) {
+        p.part[((long)split * p.M + m) * (p.kp + 1) + col] = v;
+      } else {
+        const unsigned sft = fast_div((unsigned)m, p.d_ns);
+        T* dst = p.grads + sft * p.numel + p.w_off + (long)(m - sft * p.n_s) * p.kp + col;
+        if (p.accumulate) v += to_f32(*dst);
+        *dst = from_f32<T>(v);
+      }
+    }
   }
-  if (Out::kRowSum && blockIdx.x == 0 && tid < kConvTile && m0 + tid < M) out.rowsum(grp, split, m0 + tid, rsum);
+  if (want_rows) {  // bias gradient: the rows' sums over this workgroup's pixels, 32 lanes each in a fixed order
+#pragma unroll
+    for (int q = 0; q < NA; ++q) {
+      float v = rsum[q];
+#pragma unroll
+      for (int o = 16; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+      const int m = m0 + ar + 8 * q;
+      if (ak != 0 || m >= p.M) continue;
+      if (p.part != nullptr) {
+        p.part[((long)split * p.M + m) * (p.kp + 1) + p.kp] = v;
+      } else if (p.b_off >= 0) {
+        const unsigned sft = fast_div((unsigned)m, p.d_ns);
+        T* dst = p.grads + sft * p.numel + p.b_off + (m - sft * p.n_s);
+        if (p.accumulate) v += to_f32(*dst);
+        *dst = from_f32<T>(v);
+      }
+    }
+  }
+}
+
+// grads (+)= sum over the splits, ascending, of the partial sums: one thread per entry of the [M, kp + 1] block
+template <typename T>
+__global__ __launch_bounds__(256) void wgrad_reduce_kernel(ConvArgs<T> o) {
+  const int total = o.M * (o.kp + 1), idx = blockIdx.x * 256 + threadIdx.x;
+  if (idx >= total) return;
+  const int m = idx / (o.kp + 1), n = idx - m * (o.kp + 1);
+  const unsigned sft = fast_div((unsigned)m, o.d_ns);
+  const int co = m - (int)sft * o.n_s;
+  if (n == o.kp && o.b_off < 0) return;
+  float v = 0.0f;
+  int sp = 0;
+  for (; sp + 8 <= o.splits; sp += 8) {
+    float t[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) t[u] = o.part[(long)(sp + u) * total + idx];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v += t[u];
+  }
+  for (; sp < o.splits; ++sp) v += o.part[(long)sp * total + idx];
+  T* dst = o.grads + sft * o.numel + (n < o.kp ? o.w_off + (long)co * o.kp + n : o.b_off + co);
+  if (o.accumulate) v += to_f32(*dst);
+  *dst = from_f32<T>(v);
 }
 
 static int check_geom(const char* who, const rtp_conv_geom* geom, ConvGeom& g) {
@@ -313,51 +453,93 @@ static int check_run(const char* who, int dtype, int64_t numel, int64_t shards, 
   return RTP_OK;
 }
 
-template <typename T, class OpA, class OpB, class Out>
-static int launch_igemm(hipStream_t st, const char* name, OpA a, OpB b, Out o, long M, long N, long K, long groups,
-                        double bytes, long splits = 1, long kchunk = 0) {
-  const long tm = ceil_div(M, kConvTile), tn = ceil_div(N, kConvTile);
-  RTP_REQUIRE(tn < (1l << 31) && tm < 65536 && groups * splits < 65536, "%s: grid %ld x %ld x %ld too large", name, tn,
-              tm, groups * splits);
-  if (splits == 1) kchunk = ceil_div(K, kConvSlab) * kConvSlab;
-  ProfileScope prof(st, name, 2.0 * (double)M * (double)N * (double)K * (double)groups, bytes);
-  RTP_REQUIRE(M < (1l << 30) && N < (1l << 30) && K < (1l << 30), "%s: product %ld x %ld x %ld beyond 32-bit indices", name,
-              M, N, K);
-  hipLaunchKernelGGL((conv_igemm_kernel<T, OpA, OpB, Out>), dim3((unsigned)tn, (unsigned)tm, (unsigned)(groups * splits)),
-                     dim3(256), 0, st, a, b, o, (int)M, (int)N, (int)K, (int)splits, (int)kchunk);
+template <typename T, ConvPass PASS, int BM, int BN>
+static void launch_tile(hipStream_t st, const ConvArgs<T>& a, dim3 grid) {
+  const ConvGeom& g = a.g;
+  const bool simple = PASS == kConvDgrad ? g.sh == 1 && g.sw == 1 : g.ph == 0 && g.pw == 0;
+  // the furthest element of each operand, in bytes from its base
+  auto reach = [](const Strides& s, long n, long c, long h, long w) {
+    return (double)(n - 1) * s.n + (double)(c - 1) * s.c + (double)(h - 1) * s.h + (double)(w - 1) * s.w;
+  };
+  const long co = PASS == kConvDgrad ? a.K / a.khkw : a.M;
+  double far = (double)ceil_div(co, a.n_s) * a.numel;
+  far = std::max(far, PASS == kConvDgrad ? reach(a.s, g.n, co, g.ho, g.wo) : reach(a.s, g.n, g.c, g.h, g.w));
+  if (PASS == kConvWgrad) far = std::max(far, reach(a.sd, g.n, co, g.ho, g.wo));
+  const bool wide = (far + 1.0) * sizeof(T) >= (double)kBeyond;
+#define RTP_CONV(SIMPLE, WIDE) hipLaunchKernelGGL((conv_igemm_kernel<T, PASS, BM, BN, SIMPLE, WIDE>), grid, dim3(256), 0, st, a)
+  if (wide)
+    RTP_CONV(false, true);
+  else if (simple)
+    RTP_CONV(true, false);
+  else
+    RTP_CONV(false, false);
+#undef RTP_CONV
+}
+
+// Products of at most 32 rows (few channels) take the 32-row tile.
+static int tile_rows(long M) { return M <= 32 ? 32 : 64; }
+
+template <typename T, ConvPass PASS>
+static int launch_igemm(hipStream_t st, const char* name, ConvArgs<T>& a, double bytes) {
+  const int bm = tile_rows(a.M), bn = 4096 / bm;
+  const long tm = ceil_div(a.M, bm), tn = ceil_div(a.N, bn);
+  RTP_REQUIRE(tn < (1l << 31) && tm < 65536 && a.splits < 65536, "%s: grid %ld x %ld x %d too large", name, tn, tm, a.splits);
+  if (a.splits == 1) a.kchunk = (int)(ceil_div(a.K, kConvSlab) * kConvSlab);
+  ProfileScope prof(st, name, 2.0 * (double)a.M * (double)a.N * (double)a.K, bytes);
+  const dim3 grid((unsigned)tn, (unsigned)tm, (unsigned)a.splits);
+  if (bm == 32)
+    launch_tile<T, PASS, 32, 128>(st, a, grid);
+  else
+    launch_tile<T, PASS, 64, 64>(st, a, grid);
   RTP_LAUNCH_CHECK();
   return RTP_OK;
 }
+
+// What the three passes share.  pix_h x pix_w: the pixel grid (output pixels, or input pixels for the input gradient).
+template <typename T>
+static ConvArgs<T> common_args(const ConvGeom& g, int64_t numel, int64_t n_s, int pix_h, int pix_w) {
+  ConvArgs<T> a{};
+  a.g = g;
+  a.khkw = g.kh * g.kw, a.kp = g.c * a.khkw, a.n_s = (int)n_s, a.numel = numel;
+  a.d_pix_img = make_fastdiv((unsigned)(pix_h * pix_w)), a.d_pix_row = make_fastdiv((unsigned)pix_w);
+  a.d_khkw = make_fastdiv((unsigned)a.khkw), a.d_kw = make_fastdiv((unsigned)g.kw), a.d_ns = make_fastdiv((unsigned)n_s);
+  a.d_sh = make_fastdiv((unsigned)g.sh), a.d_sw = make_fastdiv((unsigned)g.sw);
+  a.splits = 1;
+  return a;
+}
+static Strides strides_of(const int64_t* s) { return Strides{(long)s[0], (long)s[1], (long)s[2], (long)s[3]}; }
 
 template <typename T>
 static int conv_fwd(hipStream_t st, const void* x, const int64_t* sx, const ConvGeom& g, const void* w, int64_t numel,
                     int64_t shards, int64_t w_off, int64_t bias_off, int64_t n_s, void* y, int64_t co_first,
                     int64_t co_total) {
-  const long kp = (long)g.c * g.kh * g.kw, pix = (long)g.n * g.ho * g.wo;
+  ConvArgs<T> a = common_args<T>(g, numel, n_s, g.ho, g.wo);
+  const long pix = (long)g.n * g.ho * g.wo;
   const T* wt = reinterpret_cast<const T*>(w);
-  WeightRows<T> a{wt + w_off, numel, kp};
-  Patches<T, false> b{Act4<T>{reinterpret_cast<const T*>(x), sx[0], sx[1], sx[2], sx[3]}, g};
-  StoreNCHW<T> o{reinterpret_cast<T*>(y), bias_off >= 0 ? wt + bias_off : nullptr, numel, (int)co_first, (int)n_s,
-                 (int)co_total, g.ho * g.wo};
-  const double bytes = sizeof(T) * ((double)g.n * g.c * g.h * g.w + (double)shards * n_s * (kp + pix));
-  return launch_igemm<T>(st, "conv2d_fwd", a, b, o, n_s, pix, kp, shards, bytes);
+  a.M = (int)(shards * n_s), a.N = (int)pix, a.K = a.kp;
+  a.act = reinterpret_cast<const T*>(x), a.s = strides_of(sx);
+  a.w = wt + w_off, a.bias = bias_off >= 0 ? wt + bias_off : nullptr;
+  a.y = reinterpret_cast<T*>(y) + co_first * g.ho * g.wo, a.co_total = (int)co_total;
+  const double bytes = sizeof(T) * ((double)g.n * g.c * g.h * g.w + (double)shards * n_s * ((double)a.kp + pix));
+  return launch_igemm<T, kConvFwd>(st, "conv2d_fwd", a, bytes);
 }
 
 // The weight gradient contracts over all pixels of the batch and has few outputs: the contraction is dealt over
-// `splits` workgroups per output tile (about four workgroups per CU in all, at least 8 slabs each).
+// `splits` workgroups per output tile (about three workgroups per CU in all, at least 4 slabs each).
 struct WgradSplit {
   long splits, kchunk;
   size_t workspace;
 };
 static WgradSplit wgrad_split(const ConvGeom& g, int64_t shards, int64_t n_s) {
-  const long kp = (long)g.c * g.kh * g.kw, pix = (long)g.n * g.ho * g.wo;
-  const long tiles = ceil_div(n_s, kConvTile) * ceil_div(kp, kConvTile) * shards, slabs = ceil_div(pix, kConvSlab);
-  long want = std::min<long>(ceil_div(1024, tiles), std::max<long>(1, slabs / 8));
-  want = std::max<long>(1, std::min<long>(want, 65535 / shards));
+  const long kp = (long)g.c * g.kh * g.kw, pix = (long)g.n * g.ho * g.wo, M = shards * n_s;
+  const int bm = tile_rows(M), bn = 4096 / bm;
+  const long tiles = ceil_div(M, bm) * ceil_div(kp, bn), slabs = ceil_div(pix, kConvSlab);
+  long want = std::min<long>(ceil_div(768, tiles), std::max<long>(1, slabs / 4));
+  want = std::max<long>(1, std::min<long>(want, 65535));
   WgradSplit r;
   r.kchunk = ceil_div(slabs, want) * kConvSlab;
   r.splits = ceil_div(pix, r.kchunk);
-  r.workspace = r.splits > 1 ? (size_t)r.splits * shards * n_s * (kp + 1) * sizeof(float) : 0;
+  r.workspace = r.splits > 1 ? (size_t)r.splits * M * (kp + 1) * sizeof(float) : 0;
   return r;
 }
 
@@ -365,22 +547,24 @@ template <typename T>
 static int conv_wgrad(hipStream_t st, const void* dy, const int64_t* sdy, const void* x, const int64_t* sx,
                       const ConvGeom& g, void* grads, int64_t numel, int64_t shards, int64_t w_off, int64_t bias_off,
                       int64_t n_s, int64_t co_first, int accumulate, void* workspace, size_t workspace_bytes) {
-  const long kp = (long)g.c * g.kh * g.kw, pix = (long)g.n * g.ho * g.wo;
+  ConvArgs<T> a = common_args<T>(g, numel, n_s, g.ho, g.wo);
+  const long pix = (long)g.n * g.ho * g.wo;
   const WgradSplit sp = wgrad_split(g, shards, n_s);
   if (workspace_bytes < sp.workspace || (sp.workspace && workspace == nullptr))
     return fail(RTP_ERR_WORKSPACE, "rtp_conv2d_wgrad: workspace %zu < required %zu", workspace_bytes, sp.workspace);
-  GradRowsT<T> a{Act4<T>{reinterpret_cast<const T*>(dy), sdy[0], sdy[1], sdy[2], sdy[3]}, (int)co_first, (int)n_s,
-                 g.wo, g.ho * g.wo};
-  Patches<T, true> b{Act4<T>{reinterpret_cast<const T*>(x), sx[0], sx[1], sx[2], sx[3]}, g};
-  StoreWeightGrad<T> o{reinterpret_cast<T*>(grads), numel, w_off, bias_off, kp, accumulate,
-                       sp.splits > 1 ? reinterpret_cast<float*>(workspace) : nullptr, (int)shards, (int)n_s};
-  const double bytes = sizeof(T) * ((double)g.n * g.c * g.h * g.w + (double)shards * n_s * (kp + pix));
-  if (int rc = launch_igemm<T>(st, "conv2d_wgrad", a, b, o, n_s, kp, pix, shards, bytes, sp.splits, sp.kchunk)) return rc;
+  a.M = (int)(shards * n_s), a.N = a.kp, a.K = (int)pix;
+  RTP_REQUIRE((long)a.M * (a.kp + 1) < (1l << 31), "rtp_conv2d_wgrad: weight gradient of %d x %d entries too large", a.M, a.kp);
+  a.splits = (int)sp.splits, a.kchunk = (int)sp.kchunk;
+  a.act = reinterpret_cast<const T*>(x), a.s = strides_of(sx);
+  a.sd = strides_of(sdy), a.dy = reinterpret_cast<const T*>(dy) + co_first * a.sd.c;
+  a.grads = reinterpret_cast<T*>(grads), a.w_off = w_off, a.b_off = bias_off, a.accumulate = accumulate;
+  a.part = sp.splits > 1 ? reinterpret_cast<float*>(workspace) : nullptr;
+  const double bytes = sizeof(T) * ((double)g.n * g.c * g.h * g.w + (double)shards * n_s * ((double)a.kp + pix));
+  if (int rc = launch_igemm<T, kConvWgrad>(st, "conv2d_wgrad", a, bytes)) return rc;
   if (sp.splits > 1) {
-    const long total = (long)shards * n_s * (kp + 1);
+    const long total = (long)a.M * (a.kp + 1);
     ProfileScope prof(st, "conv2d_wgrad_reduce", 0.0, (double)sp.workspace + (double)total * sizeof(T));
-    hipLaunchKernelGGL(wgrad_reduce_kernel<T>, dim3((unsigned)std::min<long>(4096, ceil_div(total, 256))), dim3(256), 0, st,
-                       o, (int)sp.splits);
+    hipLaunchKernelGGL(wgrad_reduce_kernel<T>, dim3((unsigned)ceil_div(total, 256)), dim3(256), 0, st, a);
     RTP_LAUNCH_CHECK();
   }
   return RTP_OK;
@@ -390,14 +574,14 @@ template <typename T>
 static int conv_dgrad(hipStream_t st, const void* dy, const int64_t* sdy, const ConvGeom& g, const void* w,
                       int64_t numel, int64_t shards, int64_t w_off, int64_t n_s, int64_t co_first, void* dx, int dx_f32,
                       const void* addend, int addend_f32) {
-  const int khkw = g.kh * g.kw;
-  const long inpix = (long)g.n * g.h * g.w;
-  WeightByInput<T> a{reinterpret_cast<const T*>(w) + w_off, numel, (int)n_s, g.c, khkw};
-  GradByInput<T> b{Act4<T>{reinterpret_cast<const T*>(dy), sdy[0], sdy[1], sdy[2], sdy[3]}, g, (int)co_first};
-  StoreInputGrad<T> o{dx, addend, dx_f32, addend_f32, g.c, g.h * g.w};
+  ConvArgs<T> a = common_args<T>(g, numel, n_s, g.h, g.w);
+  a.M = g.c, a.N = g.n * g.h * g.w, a.K = (int)(shards * n_s * a.khkw);
+  a.s = strides_of(sdy), a.act = reinterpret_cast<const T*>(dy) + co_first * a.s.c;
+  a.w = reinterpret_cast<const T*>(w) + w_off;
+  a.dx = dx, a.addend = addend, a.dx_f32 = dx_f32, a.addend_f32 = addend_f32;
   const double bytes = sizeof(T) * ((double)g.n * g.c * g.h * g.w +
-                                    (double)shards * n_s * ((double)g.c * khkw + (double)g.n * g.ho * g.wo));
-  return launch_igemm<T>(st, "conv2d_dgrad", a, b, o, g.c, inpix, shards * n_s * khkw, 1, bytes);
+                                    (double)shards * n_s * ((double)g.c * a.khkw + (double)g.n * g.ho * g.wo));
+  return launch_igemm<T, kConvDgrad>(st, "conv2d_dgrad", a, bytes);
 }
 
 }  // namespace rtp

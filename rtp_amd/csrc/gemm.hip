@@ -407,8 +407,8 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs p) {
 
 // Epilogue of the direct-to-LDS kernel.  `ct` is the BM x BN tile of raw accumulators in LDS (row pitch BN+4
 // floats).  Thread `tid` of NTHR finishes chunks of 8 consecutive columns: alpha * acc (+ c_in) (+ bias) -> ReLU ->
-// gate mask -> store, the same order of operations as store_tile.  With p.vec_c (16-byte aligned operands and
-// n % 8 == 0, checked by the host) every global access of a chunk is a 16-byte vector.
+// gate mask -> store, the same order of operations as store_tile.  p.vec_c holds (16-byte aligned operands and
+// n % 8 == 0, checked by the host): every global access of a chunk is a 16-byte vector.
 template <typename T>
 __device__ __forceinline__ void load8(const T* src, float (&v)[8]) {
   if (sizeof(T) == 2) {
@@ -492,10 +492,6 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& p, const float* ct, 
   const T* gate =
       p.gate ? reinterpret_cast<const T*>(p.gate) + grp * p.gate_sg + zo * p.gate_so + zi * p.gate_si : nullptr;
   const int nb_seg = p.bias_sk ? p.ksegs : 1;  // a bias per K segment is summed in segment order
-  const long zoff = grp * p.c_sg + zo * p.c_so + zi * p.c_si;
-  float* master = p.sgd_master ? p.sgd_master + zoff : nullptr;
-  T* wcopy = p.sgd_w ? reinterpret_cast<T*>(p.sgd_w) + zoff : nullptr;
-  const bool skip_out = p.flags & RTP_GEMM_SGD_SKIP_OUT;
 
   if constexpr (CHUNKS % NTHR == 0) {
     // The common form (vector-aligned operands, one bias vector): a thread requests the bias, the addend and the mask
@@ -503,7 +499,7 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& p, const float* ct, 
     // chunk (a store to c_out may alias a later chunk's c_in as far as the compiler knows, so left alone the loads of
     // chunk i + 1 wait behind the store of chunk i).  When the thread count is a multiple of the chunks per row all of
     // a thread's chunks lie in the same 8 columns and share one bias vector.
-    if (p.vec_c && nb_seg == 1 && p.xent_mode == 0 && master == nullptr) {
+    if (nb_seg == 1 && p.xent_mode == 0) {
       constexpr int NCH = CHUNKS / NTHR;
       constexpr bool SAMECOL = NTHR % CPR == 0;
       constexpr int NB = SAMECOL ? 1 : NCH;
@@ -581,101 +577,136 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& p, const float* ct, 
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] *= p.alpha;
-    if (p.vec_c) {
+    if (cin) {
+      const long off = (long)row * p.ld_cin + col;
+      if (cin_f32)
+        load8(reinterpret_cast<const float*>(cin) + off, t);
+      else
+        load8(reinterpret_cast<const T*>(cin) + off, t);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] += t[e];
+    }
+    if (bias) {
+      // The per-segment biases of a row-parallel layer sit in eight different home rows, far from any cache: the
+      // loads of eight segments are issued together (segments past the last re-read segment 0 and count as zero)
+      // and then added in segment order -- one trip to memory instead of one per segment.
+      float bv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      for (int s0 = 0; s0 < nb_seg; s0 += 8) {
+        float bt[8][8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) load8(bias + (s0 + j < nb_seg ? s0 + j : 0) * p.bias_sk + col, bt[j]);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float on = s0 + j < nb_seg ? 1.0f : 0.0f;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) bv[e] += on * bt[j][e];
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] += bv[e];
+    }
+    if (relu) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = fmaxf(v[e], 0.0f);
+    }
+    if (gate) {
+      load8(gate + (long)row * p.ld_gate + col, t);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = t[e] > 0.0f ? v[e] : 0.0f;
+    }
+    if (p.xent_mode == 2) {
+      // logits -> their cross-entropy gradient: (softmax - onehot(target)) * dloss (* scale); rows whose target
+      // is the ignore index or outside the classes get zeros
+      const long tg = p.xent_target[row];
+      const bool live = tg != p.xent_ignore && tg >= 0 && tg < (long)p.xent_blocks * 64;
+      const float2 st = p.xent_stats[row];
+      const float inv = 1.0f / st.y;
+      const float sc = live ? p.xent_dloss[0] * (p.xent_scale ? p.xent_scale[0] : 1.0f) : 0.0f;
+      const long gcol = (long)grp * p.n + col;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float gq = expf(to_f32(from_f32<T>(v[e])) - st.x) * inv;
+        if (gcol + e == tg) gq -= 1.0f;
+        v[e] = gq * sc;
+      }
+    }
+    const long off = (long)row * p.ldc + col;
+    if (out_f32)
+      store8(reinterpret_cast<float*>(cbase) + off, v, stream_out);
+    else
+      store8(reinterpret_cast<T*>(cbase) + off, v, stream_out);
+  }
+}
+
+// The epilogue where an operand of it is not vector-aligned (an odd width, a shard of odd size): the same operations
+// element by element, the lanes of a wave on consecutive columns of a row (with 8 columns per lane each store would touch every
+// line of the row), the addends and masks of EB elements requested together.
+template <typename T, int BM, int BN, int NTHR>
+__device__ __forceinline__ void finish_tile_ragged(const GemmArgs& p, const float* ct, int m0, int n0, int tid, int grp,
+                                                   long zo, long zi) {
+  constexpr int CP = BN + 4, TOTAL = BM * BN, EB = 4;
+  static_assert(TOTAL % (NTHR * EB) == 0, "whole batches");
+  const bool out_f32 = p.flags & RTP_GEMM_OUT_F32;
+  const bool cin_f32 = p.flags & RTP_GEMM_CIN_F32;
+  const bool relu = p.flags & RTP_GEMM_RELU;
+  const long zoff = grp * p.c_sg + zo * p.c_so + zi * p.c_si;
+  char* cbase = p.c_out + zoff * (out_f32 ? 4 : (long)sizeof(T));
+  const char* cin =
+      p.c_in ? p.c_in + (grp * p.cin_sg + zo * p.cin_so + zi * p.cin_si) * (cin_f32 ? 4 : (long)sizeof(T)) : nullptr;
+  const T* bias =
+      p.bias ? reinterpret_cast<const T*>(p.bias) + grp * p.bias_sg + zo * p.bias_so + zi * p.bias_si : nullptr;
+  const T* gate =
+      p.gate ? reinterpret_cast<const T*>(p.gate) + grp * p.gate_sg + zo * p.gate_so + zi * p.gate_si : nullptr;
+  const int nb_seg = p.bias_sk ? p.ksegs : 1;
+  float* master = p.sgd_master ? p.sgd_master + zoff : nullptr;
+  T* wcopy = p.sgd_w ? reinterpret_cast<T*>(p.sgd_w) + zoff : nullptr;
+  const bool skip_out = p.flags & RTP_GEMM_SGD_SKIP_OUT;
+  // a thread's elements all lie in one column where the thread count is a multiple of the tile's width
+  constexpr bool SAMECOL = NTHR % BN == 0;
+  auto bias_of = [&](int col) {
+    float bv = 0.0f;
+    if (bias)
+      for (int sgm = 0; sgm < nb_seg; ++sgm) bv += to_f32(bias[sgm * p.bias_sk + col]);
+    return bv;
+  };
+  float bcol = SAMECOL ? bias_of(min(n0 + tid % BN, p.n - 1)) : 0.0f;
+  for (int e0 = tid; e0 < TOTAL; e0 += NTHR * EB) {
+    float v[EB], add[EB], msk[EB];
+    long row[EB];
+    int col[EB];
+#pragma unroll
+    for (int i = 0; i < EB; ++i) {
+      const int e = e0 + i * NTHR;
+      row[i] = m0 + e / BN, col[i] = n0 + e % BN;
+      const long rc = row[i] < p.m ? row[i] : p.m - 1;
+      const int cc = col[i] < p.n ? col[i] : p.n - 1;
+      add[i] = 0.0f, msk[i] = 1.0f;
       if (cin) {
-        const long off = (long)row * p.ld_cin + col;
-        if (cin_f32)
-          load8(reinterpret_cast<const float*>(cin) + off, t);
-        else
-          load8(reinterpret_cast<const T*>(cin) + off, t);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] += t[e];
+        const long off = rc * p.ld_cin + cc;
+        add[i] = cin_f32 ? reinterpret_cast<const float*>(cin)[off] : to_f32(reinterpret_cast<const T*>(cin)[off]);
       }
-      if (bias) {
-        // The per-segment biases of a row-parallel layer sit in eight different home rows, far from any cache: the
-        // loads of eight segments are issued together (segments past the last re-read segment 0 and count as zero)
-        // and then added in segment order -- one trip to memory instead of one per segment.
-        float bv[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        for (int s0 = 0; s0 < nb_seg; s0 += 8) {
-          float bt[8][8];
+      if (gate) msk[i] = to_f32(gate[rc * p.ld_gate + cc]);
+      v[i] = p.alpha * ct[(e / BN) * CP + e % BN];
+    }
 #pragma unroll
-          for (int j = 0; j < 8; ++j) load8(bias + (s0 + j < nb_seg ? s0 + j : 0) * p.bias_sk + col, bt[j]);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const float on = s0 + j < nb_seg ? 1.0f : 0.0f;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) bv[e] += on * bt[j][e];
-          }
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] += bv[e];
-      }
-      if (relu) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = fmaxf(v[e], 0.0f);
-      }
-      if (gate) {
-        load8(gate + (long)row * p.ld_gate + col, t);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = t[e] > 0.0f ? v[e] : 0.0f;
-      }
-      if (p.xent_mode == 2) {
-        // logits -> their cross-entropy gradient: (softmax - onehot(target)) * dloss (* scale); rows whose target
-        // is the ignore index or outside the classes get zeros
-        const long tg = p.xent_target[row];
-        const bool live = tg != p.xent_ignore && tg >= 0 && tg < (long)p.xent_blocks * 64;
-        const float2 st = p.xent_stats[row];
-        const float inv = 1.0f / st.y;
-        const float sc = live ? p.xent_dloss[0] * (p.xent_scale ? p.xent_scale[0] : 1.0f) : 0.0f;
-        const long gcol = (long)grp * p.n + col;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          float gq = expf(to_f32(from_f32<T>(v[e])) - st.x) * inv;
-          if (gcol + e == tg) gq -= 1.0f;
-          v[e] = gq * sc;
-        }
-      }
-      const long off = (long)row * p.ldc + col;
+    for (int i = 0; i < EB; ++i) {
+      if (row[i] >= p.m || col[i] >= p.n) continue;
+      float x = v[i];
+      if (cin) x += add[i];
+      if (bias) x += SAMECOL ? bcol : bias_of(col[i]);
+      if (relu) x = fmaxf(x, 0.0f);
+      if (gate) x = msk[i] > 0.0f ? x : 0.0f;
+      const long off = row[i] * p.ldc + col[i];
       if (master) {
-        float w[8];
-        load8(master + off, w);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) w[e] = sgd_update<T>(w[e], v[e], p.sgd_lr, p.sgd_clip);
-        store8(master + off, w, true);
-        if (wcopy) store8(wcopy + off, w, true);
+        const float w = sgd_update<T>(master[off], x, p.sgd_lr, p.sgd_clip);
+        master[off] = w;
+        if (wcopy) wcopy[off] = from_f32<T>(w);
       }
-      if (!skip_out) {
-        if (out_f32)
-          store8(reinterpret_cast<float*>(cbase) + off, v, stream_out);
-        else
-          store8(reinterpret_cast<T*>(cbase) + off, v, stream_out);
-      }
-    } else {
-      for (int e = 0; e < 8 && col + e < p.n; ++e) {
-        float x = v[e];
-        if (cin) {
-          const long off = (long)row * p.ld_cin + col + e;
-          x += cin_f32 ? reinterpret_cast<const float*>(cin)[off] : to_f32(reinterpret_cast<const T*>(cin)[off]);
-        }
-        if (bias) {
-          float bv = 0.0f;
-          for (int sgm = 0; sgm < nb_seg; ++sgm) bv += to_f32(bias[sgm * p.bias_sk + col + e]);
-          x += bv;
-        }
-        if (relu) x = fmaxf(x, 0.0f);
-        if (gate) x = to_f32(gate[(long)row * p.ld_gate + col + e]) > 0.0f ? x : 0.0f;
-        const long off = (long)row * p.ldc + col + e;
-        if (master) {
-          const float w = sgd_update<T>(master[off], x, p.sgd_lr, p.sgd_clip);
-          master[off] = w;
-          if (wcopy) wcopy[off] = from_f32<T>(w);
-        }
-        if (skip_out) continue;
-        if (out_f32)
-          reinterpret_cast<float*>(cbase)[off] = x;
-        else
-          reinterpret_cast<T*>(cbase)[off] = from_f32<T>(x);
-      }
+      if (skip_out) continue;
+      if (out_f32)
+        reinterpret_cast<float*>(cbase)[off] = x;
+      else
+        reinterpret_cast<T*>(cbase)[off] = from_f32<T>(x);
     }
   }
 }
@@ -827,6 +858,7 @@ struct DmaOperand {
   static_assert((R * SB / 1024) % NL == 0, "every loader wave issues the same number of loads");
   static constexpr int NI = R * SB / 1024 / NL;   // load instructions (1 KiB each) per loader wave and slab
   static constexpr int BYTES = R * SB;            // one stage of this operand
+  static constexpr int BK_ = SB / (int)sizeof(T);  // k per slab
   static constexpr int LINE = R * (int)sizeof(T); // bytes of one k line when rows are contiguous
   static_assert(KC || 1024 % LINE == 0 || LINE % 1024 == 0, "a 1 KiB load covers whole k lines or a whole fraction of one");
   // The lane's vector sits at `ofs` bytes from the slab's base pointer, which is the same for every lane and lives
@@ -886,6 +918,104 @@ struct DmaOperand {
                      : "s"(lds_stage + (unsigned)((lw * NI + i) * 1024)), "v"(ofs[i]), "s"(base)
                      : "memory");
       }
+    }
+  }
+};
+
+// A 16-byte vector shifted down by `n` elements, zeros moving in from the top: what a vector that was read `n` elements
+// before its place (to stay inside the operand) has to undergo.
+template <typename T>
+__device__ __forceinline__ uint4 shift_down(uint4 q, int n) {
+  constexpr int PER = 4 / (int)sizeof(T);  // elements per word
+  const int w = n / PER;
+  const unsigned d[4] = {q.x, q.y, q.z, q.w};
+  unsigned r[5];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    r[i] = 0u;
+#pragma unroll
+    for (int j = i; j < 4; ++j) r[i] = w == j - i ? d[j] : r[i];
+  }
+  r[4] = 0u;
+  if (PER == 2) {
+    const unsigned odd = (n & 1) * 16u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = odd ? (r[i] >> 16) | (r[i + 1] << 16) : r[i];
+  }
+  return make_uint4(r[0], r[1], r[2], r[3]);
+}
+
+// The loader for operands the direct-to-LDS loads cannot take: rows, extents or base addresses that are no multiples of 16
+// bytes (a 1001-class head, shards of odd size).  Vectors are read with unaligned 16-byte loads into registers, kRegDepth
+// slabs ahead, and written to the stage in the layout DmaOperand leaves there.  A vector that would reach beyond its row (or k
+// line) is read further down, inside it, and shifted into place; this is decided per vector without a branch, and
+// the shift only runs in slabs and tiles that have such vectors.  Needs rows (k lines) of at least one vector.
+// Bound by the rate of unaligned vector loads: 25 - 28 bytes a clock and CU from the L1 against 56 for aligned ones.  A layer of
+// 992 x 1001 x 2048 (bf16, 8 shards, forward + both gradients): 54 us, 185 us with the guarded scalar loads; 4096^3 with
+// one extent odd 180 - 290 us.
+constexpr int kRegDepth = 3;
+template <typename T, int R, bool KC, int NL, int SB>
+struct RegOperand {
+  using D = DmaOperand<T, R, KC, NL, SB>;
+  static constexpr int VEC = D::VEC, NI = D::NI, BYTES = D::BYTES;
+  typedef unsigned vec_t __attribute__((ext_vector_type(4), aligned(2)));  // global loads take any alignment
+  const char* base;  // the operand's element 0 (K-contiguous: of row row0)
+  long ldb;          // leading dimension in bytes
+  unsigned ofs[NI];  // K-contiguous: of the lane's row;  else of the lane's rows inside a k line
+  int koff[NI];      // k of the vector inside its slab
+  int shift[NI];     // !KC: elements the vector was read early
+  bool edge;         // !KC: the tile has such vectors
+  uint4 val[kRegDepth][NI];
+
+  __device__ __forceinline__ void init(const T* x, long ld, int row0, int rows, int lw, int lane) {
+    ldb = ld * (long)sizeof(T);
+    base = reinterpret_cast<const char*>(KC ? x + (long)row0 * ld : x);
+    edge = !KC && row0 + R > rows;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int j = lw * NI + i;
+      if (KC) {
+        constexpr int LPR = SB / 16;
+        const int row = j * (64 / LPR) + lane / LPR;
+        const int rr = row0 + row < rows ? row : rows - 1 - row0;
+        ofs[i] = (unsigned)(rr * ldb);
+        koff[i] = ((lane % LPR) ^ kc_swizzle<SB>(row)) * VEC;
+        shift[i] = 0;
+      } else {
+        const int byte = lane * 16;
+        koff[i] = j * (1024 / D::LINE) + byte / D::LINE;
+        const int r = row0 + (((byte % D::LINE) >> 4) ^ rc_swizzle<T, R>(koff[i])) * VEC;
+        const int start = min(r, rows - VEC);
+        ofs[i] = (unsigned)(start * (int)sizeof(T));
+        shift[i] = r - start;
+      }
+    }
+  }
+  // request the slab whose first k is k0 (in a segment that starts seg bytes from the operand's base)
+  template <int S>
+  __device__ __forceinline__ void fetch(long seg, int k0, int kdim) {
+    const char* b = base + seg + (KC ? 0 : (long)k0 * ldb);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const unsigned o = KC ? ofs[i] + (unsigned)(min(k0 + koff[i], kdim - VEC) * (int)sizeof(T))
+                            : ofs[i] + (unsigned)(min(koff[i], kdim - 1 - k0) * ldb);
+      const vec_t v = *reinterpret_cast<const vec_t*>(b + o);
+      val[S][i] = make_uint4(v.x, v.y, v.z, v.w);
+    }
+  }
+  template <int S>
+  __device__ __forceinline__ void store(char* stage, int lw, int lane, int k0, int kdim) {
+    const bool tail = k0 + D::BK_ > kdim;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      uint4 q = val[S][i];
+      if (KC) {
+        if (tail) q = shift_down<T>(q, min(max(k0 + koff[i] - (kdim - VEC), 0), VEC));
+      } else {
+        if (edge) q = shift_down<T>(q, min(shift[i], VEC));
+        if (tail && k0 + koff[i] >= kdim) q = make_uint4(0u, 0u, 0u, 0u);
+      }
+      *reinterpret_cast<uint4*>(stage + (lw * NI + i) * 1024 + lane * 16) = q;
     }
   }
 };
@@ -951,7 +1081,10 @@ __device__ __forceinline__ Frag<T> read_frag_dma(const char* st, int rowbase, in
 
 // The body of the product kernel: workgroup `id` of the `nwg` that work on the problem `p` (`bx`, `by`: its
 // coordinates in a launch that does not use XCD bricks).  `p` lives in the kernel-argument segment.
-template <typename T, int BM, int BN, bool AKC, bool BKC, int NSTAGE, int SB, int PD>
+// REG: the loader waves go through registers (RegOperand) instead of loading straight into LDS.  RAG: the epilogue's operands
+// may be unaligned; kernels of their own, since the element-wise epilogue inside every kernel cost the others registers
+// and code (1 % of the LM attention's time).
+template <typename T, int BM, int BN, bool AKC, bool BKC, int NSTAGE, int SB, int PD, bool REG, bool RAG>
 __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned id, const unsigned bx, const unsigned by,
                                               const unsigned nwg) {
   constexpr int NL = 4;  // loader waves (waves 4..7); waves 0..3 compute
@@ -1036,6 +1169,56 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
     const int lw = wave - 4;
     const T* A = reinterpret_cast<const T*>(p.a) + grp * p.a_sg + zo * p.a_so + zi * p.a_si;
     const T* B = reinterpret_cast<const T*>(p.b) + grp * p.b_sg + zo * p.b_so + zi * p.b_si;
+    if constexpr (REG) {
+      // slab k+1 is written before barrier k+1 -- the stage it takes held slab k+1-NSTAGE, whose last reader passed barrier
+      // k+3-NSTAGE -- and slab k+1+kRegDepth requested into its registers.  Slabs behind the last one re-read it, so
+      // that the number of loads in flight is known at every wait.
+      RegOperand<T, BM, AKC, NL, SB> ra;
+      RegOperand<T, BN, BKC, NL, SB> rb;
+      ra.init(A, p.lda, m0, p.m, lw, lane);
+      rb.init(B, p.ldb, n0, p.n, lw, lane);
+      int fs = 0, fk = 0, ws = 0, wk = 0;  // segment and k of the next slab to request and to write
+      auto next = [&](int& seg, int& k0) {
+        k0 += BK;
+        if (k0 < p.k) return;
+        if (seg + 1 < p.ksegs) {
+          ++seg;
+          k0 = 0;
+        } else {
+          k0 -= BK;
+        }
+      };
+      auto fetch = [&](auto S) {
+        ra.template fetch<decltype(S)::value>(fs * p.a_sk * (long)sizeof(T), fk, p.k);
+        rb.template fetch<decltype(S)::value>(fs * p.b_sk * (long)sizeof(T), fk, p.k);
+        next(fs, fk);
+        asm volatile("" ::: "memory");  // requests stay in this order: the waits count them
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      int stage = 0;
+      auto write = [&](auto S) {
+        ra.template store<decltype(S)::value>(lds + stage * STAGE, lw, lane, wk, p.k);
+        rb.template store<decltype(S)::value>(lds + stage * STAGE + DA::BYTES, lw, lane, wk, p.k);
+        next(ws, wk);
+        stage = stage + 1 == NSTAGE ? 0 : stage + 1;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      };
+      [&]<int... S>(std::integer_sequence<int, S...>) { (fetch(std::integral_constant<int, S>{}), ...); }
+      (std::make_integer_sequence<int, kRegDepth>{});
+      auto slab = [&](auto S) {
+        write(S);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        fetch(S);
+      };
+      int k = 0;
+      for (; k + kRegDepth <= nk; k += kRegDepth)  // no exit inside a round: the waits of the next one stay exact
+        [&]<int... S>(std::integer_sequence<int, S...>) { (slab(std::integral_constant<int, S>{}), ...); }
+        (std::make_integer_sequence<int, kRegDepth>{});
+      [&]<int... S>(std::integer_sequence<int, S...>) {
+        ((k + S < nk ? slab(std::integral_constant<int, S>{}) : (void)0), ...);
+      }(std::make_integer_sequence<int, kRegDepth>{});
+    } else {
     DA da;
     DB db;
     da.init(p.lda, m0, p.m, lw, lane);
@@ -1088,6 +1271,7 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
     for (; k + 1 < nk; ++k) {
       RTP_WAIT_VM(0);
       __builtin_amdgcn_s_barrier();
+    }
     }
   } else {
     // ---- compute waves ----
@@ -1167,7 +1351,7 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
       }(std::make_integer_sequence<int, NSTAGE>{});
     };
     warm_ahead(p, (unsigned)(uintptr_t)(lptr_t)lds + NSTAGE * STAGE, id, nwg, wave, lane);
-    if (p.bias != nullptr && wave == 0) {
+    if (p.bias != nullptr && wave == 0 && (!RAG || p.vec_c)) {
       // the epilogue's bias values (one vector per K segment of a row-parallel layer, each in another home row) are
       // requested now and sit in the L2 when the epilogue asks for them
       const int nb = p.bias_sk ? p.ksegs : 1;
@@ -1182,7 +1366,7 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
                      : "memory");
       }
     }
-    if (p.gate != nullptr && p.vec_c) {
+    if (p.gate != nullptr && (!RAG || p.vec_c)) {
       // the ReLU mask of the epilogue is an activation saved by the forward pass, long gone from the caches: the
       // tile's part of it is requested now, 16 bytes per lane
       constexpr int CPR = BN * (int)sizeof(T) / 16, NCH = BM * CPR;  // 16-byte chunks per tile row, per tile
@@ -1240,7 +1424,13 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
           ct[(wm * WM + i * 32 + 8 * (r >> 2) + 4 * g + (r & 3)) * CP + wn * WN + j * 32 + li] = acc[i][j][r];
   }
   __syncthreads();
-  if (p.sgd_master != nullptr && p.vec_c)
+  if constexpr (RAG) {
+    // (the statistics and the vectorised update are only fused into products that are aligned throughout)
+    if (REG && p.vec_c)
+      finish_tile<T, BM, BN, 512>(p, ct, m0, n0, tid, grp, zo, zi);
+    else
+      finish_tile_ragged<T, BM, BN, 512>(p, ct, m0, n0, tid, grp, zo, zi);
+  } else if (p.sgd_master != nullptr)
     finish_tile_sgd<T, BM, BN, 512>(p, ct, m0, n0, tid, grp, zo, zi);
   else if (p.xent_mode == 1) {
     // (tiles whose width is no multiple of the 64-column statistics blocks are never chosen for this epilogue)
@@ -1263,8 +1453,16 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
 template <typename T, int BM, int BN, bool AKC, bool BKC, int NSTAGE, int SB, int PD>
 __global__ __launch_bounds__(512) void gemm_dma_kernel(GemmArgs p) {
   touch_kernel_arguments<sizeof(GemmArgs)>();
-  gemm_dma_body<T, BM, BN, AKC, BKC, NSTAGE, SB, PD>(p, blockIdx.x + blockIdx.y * gridDim.x, blockIdx.x, blockIdx.y,
-                                                     gridDim.x * gridDim.y);
+  gemm_dma_body<T, BM, BN, AKC, BKC, NSTAGE, SB, PD, false, false>(p, blockIdx.x + blockIdx.y * gridDim.x, blockIdx.x,
+                                                            blockIdx.y, gridDim.x * gridDim.y);
+}
+
+// Operands of any alignment; REG where that includes A or B.
+template <typename T, int BM, int BN, bool AKC, bool BKC, int NSTAGE, int SB, int PD, bool REG>
+__global__ __launch_bounds__(512) void gemm_unaligned_kernel(GemmArgs p) {
+  touch_kernel_arguments<sizeof(GemmArgs)>();
+  gemm_dma_body<T, BM, BN, AKC, BKC, NSTAGE, SB, PD, REG, true>(p, blockIdx.x + blockIdx.y * gridDim.x, blockIdx.x, blockIdx.y,
+                                                          gridDim.x * gridDim.y);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1541,6 +1739,21 @@ static int launch_dma(hipStream_t s, const GemmArgs& a, bool akc, bool bkc, dim3
   return RTP_OK;
 }
 
+template <typename T, int BM, int BN, int NSTAGE, int SB, int PD, bool REG>
+static int launch_unaligned(hipStream_t s, const GemmArgs& a, bool akc, bool bkc, dim3 grid) {
+  const dim3 block(512);
+  if (akc && bkc)
+    hipLaunchKernelGGL((gemm_unaligned_kernel<T, BM, BN, true, true, NSTAGE, SB, PD, REG>), grid, block, 0, s, a);
+  else if (akc && !bkc)
+    hipLaunchKernelGGL((gemm_unaligned_kernel<T, BM, BN, true, false, NSTAGE, SB, PD, REG>), grid, block, 0, s, a);
+  else if (!akc && bkc)
+    hipLaunchKernelGGL((gemm_unaligned_kernel<T, BM, BN, false, true, NSTAGE, SB, PD, REG>), grid, block, 0, s, a);
+  else
+    hipLaunchKernelGGL((gemm_unaligned_kernel<T, BM, BN, false, false, NSTAGE, SB, PD, REG>), grid, block, 0, s, a);
+  RTP_LAUNCH_CHECK();
+  return RTP_OK;
+}
+
 // ---------------------------------------------------------------------------------------------
 // Tiny batched problems (one attention head at sequence length <= 64: 32 x 32 x 64 per (batch, head)):
 // one wavefront per 32 x 32 output block, operands read straight from global memory into MFMA
@@ -1645,6 +1858,16 @@ static bool takes_dma_kernel(const rtp_gemm_desc* d) {
          (bkc || mult(d->n, VEC)) && d->k > 0 && d->lda <= ld_max && d->ldb <= ld_max;
 }
 
+// Whether the same kernel with register loaders can: any alignment, as long as every row (or k line) holds one vector.
+template <typename T>
+static bool takes_reg_kernel(const rtp_gemm_desc* d) {
+  constexpr int VEC = 16 / sizeof(T);
+  const bool akc = d->a_kcontig, bkc = d->b_kcontig;
+  const int64_t ld_max = ((int64_t)1 << 24) / (int64_t)sizeof(T) - 64;
+  return ((akc || bkc) ? d->k >= VEC : d->k > 0) && (akc || d->m >= VEC) && (bkc || d->n >= VEC) && d->lda <= ld_max &&
+         d->ldb <= ld_max;
+}
+
 // The fused clip + SGD lives in the epilogue of the wave-specialised kernel; the gradient keeps the compute dtype.
 template <typename T>
 static bool sgd_fused(const rtp_gemm_desc* d) {
@@ -1654,7 +1877,7 @@ static bool sgd_fused(const rtp_gemm_desc* d) {
 
 template <typename T>
 static bool rowsum_fused(const rtp_gemm_desc* d) {
-  return !d->a_kcontig && d->batch == 1 && !is_tiny(d) && takes_dma_kernel<T>(d);
+  return !d->a_kcontig && d->batch == 1 && !is_tiny(d) && (takes_dma_kernel<T>(d) || takes_reg_kernel<T>(d));
 }
 
 // rtp_gemm_warm_next: bytes the next product launched by this host thread requests at its start
@@ -1709,7 +1932,7 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   }
 
   const bool akc = d->a_kcontig, bkc = d->b_kcontig;
-  const bool fast = takes_dma_kernel<T>(d);
+  const bool direct = takes_dma_kernel<T>(d), fast = direct || takes_reg_kernel<T>(d);
   const int64_t nz = d->batch * d->groups;
   a.a_rowsum = (char*)d->a_rowsum;
   a.rowsum_sg = d->rowsum_sg;
@@ -1780,6 +2003,7 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   }();
   static const double slab_ns[kNumShapes] = {966.0, 470.0, 283.0, 167.0, 800.0, 1680.0, 545.0};
   static const int slab_bytes[kNumShapes] = {128, 128, 128, 128, 128, 128, 128};
+  const bool vec = direct && a.vec_c;  // else the kernels for operands of any alignment
   int shape = 3;  // 64 x 64 unless the model finds something cheaper
   double best = 0.0;
   for (int i = 0; fast && i < kNumShapes; ++i) {
@@ -1790,6 +2014,7 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
     // (its epilogue is the plain one: the update and the statistics epilogue are never routed to it, forced or not)
     if (i == 5 && (sizeof(T) != 2 || d->sgd_master || d->xent_mode == 1)) continue;
     if (i == 6 && d->xent_mode == 1) continue;  // 160 columns are no whole number of 64-column statistics blocks
+    if (!vec && i != 1 && i != 3) continue;  // the kernels for unaligned operands: 128 x 128 and 64 x 64
     // 128 x 160 is priced at the rate measured where it is meant for -- products of at most two rounds of tiles, such
     // as the LM's logits layer (shards of 1280 columns); larger products keep the shapes measured on large products
     if (i == 6 && ceil_div(d->m, 128) * ceil_div(d->n, 160) * nz > 512 && i != forced) continue;
@@ -1873,11 +2098,11 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
 
   // variant name = the kernel template instance, e.g. gemm_bf16_128x64_kc_kc
   static const char* const layout_tag[2][2] = {{"rc_rc", "rc_kc"}, {"kc_rc", "kc_kc"}};
-  static thread_local char names[2][kNumShapes + 1][2][2][40];
-  char* name = names[sizeof(T) == 2][fast ? shape : kNumShapes][akc][bkc];
+  static thread_local char names[2][2][kNumShapes + 1][2][2][40];
+  char* name = names[sizeof(T) == 2][vec][fast ? shape : kNumShapes][akc][bkc];
   if (!name[0])
-    snprintf(name, 40, "gemm_%s_%s_%s", sizeof(T) == 2 ? "bf16" : "f32", fast ? ts.tag : "64x64_guarded",
-             layout_tag[akc][bkc]);
+    snprintf(name, 40, "gemm_%s_%s%s_%s", sizeof(T) == 2 ? "bf16" : "f32", fast ? ts.tag : "64x64_guarded",
+             fast && !vec ? "_unaligned" : "", layout_tag[akc][bkc]);
   const double mn = (double)d->m * (double)d->n * (double)nz;
   const double kk = (double)d->k * (double)d->ksegs;
   const double out_sz = (d->flags & RTP_GEMM_OUT_F32) ? 4.0 : (double)sizeof(T);
@@ -1902,6 +2127,14 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   a.warm = nullptr;
   a.warm_bytes = 0;
   if (!fast) return launch_layout<T, 64, 64, 1, false>(s, a, akc, bkc, grid);
+  if (!vec) {
+    if (warm_src != nullptr) a.warm = (const char*)warm_src, a.warm_bytes = (long)t_warm_bytes;
+    if (direct)
+      return shape == 1 ? launch_unaligned<T, 128, 128, 4, 128, 1, false>(s, a, akc, bkc, grid)
+                        : launch_unaligned<T, 64, 64, 4, 128, 3, false>(s, a, akc, bkc, grid);
+    return shape == 1 ? launch_unaligned<T, 128, 128, 4, 128, 1, true>(s, a, akc, bkc, grid)
+                      : launch_unaligned<T, 64, 64, 4, 128, 3, true>(s, a, akc, bkc, grid);
+  }
   if (shape != 5 && warm_src != nullptr) {
     a.warm = (const char*)warm_src;
     a.warm_bytes = (long)t_warm_bytes;

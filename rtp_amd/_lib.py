@@ -146,6 +146,11 @@ PROTOTYPES = {
                                 _i, _f, _i64, _i64, _i64, _i64, _i64]),
     "rtp_attn_flash_bwd": (_i, [_vp, _i, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _vp,
                                 _vp, _vp, _vp, _vp, _vp, _vp, _i, _f, _i64, _i64, _i64, _i64, _i64]),
+    "rtp_attn_flash_kv_supported": (_i, [_i, _i64, _i64, _i64]),
+    "rtp_attn_flash_kv_fwd": (_i, [_vp, _i, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _vp,
+                                   _i64, _i64, _i64, _i64, _vp, _vp, _vp, _i, _f, _i64, _i64, _i64, _i64, _i64, _i64]),
+    "rtp_attn_flash_kv_bwd": (_i, [_vp, _i, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp,
+                                   _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _f, _i64, _i64, _i64, _i64, _i64, _i64]),
     "rtp_layernorm_supported": (_i, [_i, _i64]),
     "rtp_add_layernorm_fwd": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _f, _i64, _i64, _vp, _vp, _vp, _vp]),
     "rtp_layernorm_bwd_workspace_bytes": (_sz, [_i64, _i64]),

@@ -91,7 +91,8 @@ PyObject* invoke(R (*f)(A...), const char* name, PyObject* const* args, Py_ssize
   P(rtp_embedding_backward_grouped_supported) P(rtp_embedding_backward_grouped_workspace_bytes)                       \
   X(rtp_embedding_backward_grouped)                                                                                   \
   X(rtp_softmax_fwd_masks) X(rtp_softmax_bwd) P(rtp_attn_supported) X(rtp_attn_fwd) X(rtp_attn_bwd)                   \
-  P(rtp_attn_flash_supported) X(rtp_attn_flash_fwd) X(rtp_attn_flash_bwd) P(rtp_layernorm_supported)                  \
+  P(rtp_attn_flash_supported) X(rtp_attn_flash_fwd) X(rtp_attn_flash_bwd) P(rtp_attn_flash_kv_supported)              \
+  X(rtp_attn_flash_kv_fwd) X(rtp_attn_flash_kv_bwd) P(rtp_layernorm_supported)                                        \
   X(rtp_add_layernorm_fwd) P(rtp_layernorm_bwd_workspace_bytes) X(rtp_layernorm_bwd) P(rtp_layernorm_bwd_blocks)      \
   X(rtp_layernorm_bwd_finalize) X(rtp_softmax_xent_fwd) X(rtp_softmax_xent_reduce) X(rtp_softmax_xent_bwd)            \
   P(rtp_top2_route_workspace_bytes) X(rtp_top2_route) X(rtp_top2_route_bwd) X(rtp_moe_dispatch) X(rtp_moe_combine)    \

@@ -136,7 +136,7 @@ class _AttentionFn(torch.autograd.Function):
     batch, head) triple is addressed by strides inside the batched GEMM, so nothing is re-laid out.
 
     The core runs in one of three forms: bf16 with L <= 32 in one launch that keeps the scores in registers and
-    stores p; bf16 with longer sequences in a running-softmax launch that stores only the log-sum-exp per
+    stores p; longer sequences and fp32 in a running-softmax launch that stores only the log-sum-exp per
     query (not when the caller wants the attention weights back); otherwise as batched products and a softmax
     kernel with p in memory."""
 
@@ -158,7 +158,7 @@ class _AttentionFn(torch.autograd.Function):
         # attention dropout and per-head masks work on the probabilities in memory: the product + softmax form
         plain = drop_p == 0.0 and (mask is None or mask.dim() == 2)
         fused = plain and ops.attn_supported(dt, L, d)
-        flash = plain and not fused and not want_weights and ops.attn_flash_supported(dt, L, d)
+        flash = plain and not fused and not want_weights and ops.attn_flash_kv_supported(dt, L, L, d)
         if flash:
             p = torch.empty(ws * Z, L, dtype=torch.float32, device=dev)  # log-sum-exp in place of probabilities
         else:
@@ -352,13 +352,23 @@ def _bias_kv_layout(layer):
     return off[nxt], off[nxt + 1]
 
 
+def _shard_inputs_grad(sums, flat, e_s, c0, i) -> None:
+    """The run's part of the three projections' input gradients; an entry of `sums` is None where nobody asks for it."""
+    for item in sums:
+        if item is not None:
+            _, acc, src, width, w_off = item
+            c_out, c_in = acc.target(i)
+            S.col_dgrad(src, flat, w_off, e_s, width, c_out, c0, c_in=c_in)
+
+
 class _GeneralAttentionFn(torch.autograd.Function):
     """Attention whose keys and values come from their own tensors (query [L, N, E], key [S, N, kdim], value
     [S, N, vdim]; functional.py:575-609 projects them with three row blocks of the shard), optionally with the
     learned key / value bias_k / bias_v (add_bias_kv, functional.py:711-716) and then one all-zero key / value
     (add_zero_attn, functional.py:746-753) appended per batch entry.  Three projections per shard run into
-    q [L*N, E], k and v [(S+z)*N, E] (group g at column block g; z appended positions); the core is batched products
-    and the softmax kernel with p [ws*N*h_s, L, S+z] in memory."""
+    q [L*N, E], k and v [(S+z)*N, E] (group g at column block g; z appended positions); the core is the running-softmax
+    launch, or, with dropout, per-head masks or the weights wanted back, batched products and the softmax kernel with
+    p [ws*N*h_s, L, S+z] in memory."""
 
     @staticmethod
     def forward(ctx, query, key, value, anchor, layer, mask, key_bias, want_weights, drop_p=0.0):
@@ -384,7 +394,12 @@ class _GeneralAttentionFn(torch.autograd.Function):
         bk_off, bv_off = _bias_kv_layout(layer) if bkv else (None, None)
         o = torch.empty(L * N, E, dtype=dt, device=dev)
         out = torch.empty(L * N, E, dtype=dt, device=dev)
-        p = torch.empty(ws * Z, L, sk, dtype=dt, device=dev)
+        flash = drop_p == 0.0 and not want_weights and (mask is None or mask.dim() == 2) and \
+            ops.attn_flash_kv_supported(dt, L, sk, d)
+        if flash:
+            p = torch.empty(ws * Z, L, dtype=torch.float32, device=dev)  # log-sum-exp in place of probabilities
+        else:
+            p = torch.empty(ws * Z, L, sk, dtype=dt, device=dev)
         drop = torch.empty(ws * Z, L, sk, dtype=torch.float32, device=dev) if drop_p > 0.0 else None
         pv = torch.empty_like(p) if drop_p > 0.0 else p
         ld = N * E  # one step along the sequence in q, k, v and o
@@ -400,6 +415,13 @@ class _GeneralAttentionFn(torch.autograd.Function):
                 if bkv:  # position s_in of every batch entry: the head groups' slices of bias_k / bias_v
                     kb[s_in * N:(s_in + 1) * N, c0:c0 + cnt * e_s] = flat[:, bk_off:bk_off + e_s].reshape(1, cnt * e_s)
                     vb[s_in * N:(s_in + 1) * N, c0:c0 + cnt * e_s] = flat[:, bv_off:bv_off + e_s].reshape(1, cnt * e_s)
+                if flash:
+                    ops.attn_flash_kv_fwd(qb, kb, vb, o, c0, (ld, E, d, e_s), (ld, E, d, e_s), p[first * Z:(first + cnt) * Z],
+                                          mask, scale, L, sk, N, h_s, d, cnt, key_bias=key_bias)
+                    c_out, c_in = acc.target(i)
+                    S.row_fwd(o, flat, w_o, E, e_s, b_o, c_out, c0, c_in=c_in)
+                    i += 1
+                    continue
                 scores = torch.empty(cnt * Z, L, sk, dtype=torch.float32, device=dev)
                 _bmm(dt, a=qb, a_off=c0, lda=ld, a_kc=True, a_s=(E, d), a_sg=e_s, b=kb, b_off=c0, ldb=ld, b_kc=True,
                      b_s=(E, d), b_sg=e_s, c=scores, c_off=0, ldc=sk, c_s=(h_s * L * sk, L * sk), c_sg=Z * L * sk,
@@ -426,6 +448,7 @@ class _GeneralAttentionFn(torch.autograd.Function):
             weights = pv[last * Z:(last + 1) * Z].view(N, h_s, L, sk)
         ctx.layer = layer
         ctx.dims = (L, N, E, s_in, sk)
+        ctx.flash = (mask, key_bias) if flash else None
         ctx.dropped = drop is not None
         ctx.save_for_backward(q2, k2, v2, qb, kb, vb, p, o, *((drop, pv) if drop is not None else ()))
         ctx.mark_non_differentiable(*([weights] if weights is not None else []))
@@ -450,6 +473,7 @@ class _GeneralAttentionFn(torch.autograd.Function):
         dqb = torch.empty(L * N, E, dtype=dt, device=dev)
         dkb = torch.empty(sk * N, E, dtype=dt, device=dev)
         dvb = torch.empty(sk * N, E, dtype=dt, device=dev)
+        delta = torch.empty_like(p) if ctx.flash is not None else None
         rot = rotation(store, layer.rank, reverse=True)
         parts = sum(len(w) for w in rot.windows)
         # input gradients of the three projections, each summed over the shards; the rows of an appended zero key
@@ -470,6 +494,13 @@ class _GeneralAttentionFn(torch.autograd.Function):
                 p_off = first * Z * L * sk
                 p_s, p_sg = (h_s * L * sk, L * sk), Z * L * sk
                 S.row_dgrad(dout2, flat, w_o, E, e_s, do, c0)
+                if ctx.flash is not None:
+                    ops.attn_flash_kv_bwd(qb, kb, vb, o, do, c0, (ld, E, d, e_s), (ld, E, d, e_s),
+                                          p[first * Z:(first + cnt) * Z], delta[first * Z:(first + cnt) * Z], dqb, dkb, dvb,
+                                          ctx.flash[0], scale, L, sk, N, h_s, d, cnt, key_bias=ctx.flash[1])
+                    _shard_inputs_grad(sums, flat, e_s, c0, i)
+                    i += 1
+                    continue
                 # dP = dO V^T
                 dp = torch.empty(cnt * Z, L, sk, dtype=torch.float32, device=dev)
                 _bmm(dt, a=do, a_off=c0, lda=ld, a_kc=True, a_s=(E, d), a_sg=e_s, b=vb, b_off=c0, ldb=ld, b_kc=True,
@@ -491,11 +522,7 @@ class _GeneralAttentionFn(torch.autograd.Function):
                 _bmm(dt, a=ds, a_off=0, lda=sk, a_kc=False, a_s=p_s, a_sg=p_sg, b=qb, b_off=c0, ldb=ld, b_kc=False,
                      b_s=(E, d), b_sg=e_s, c=dkb, c_off=c0, ldc=ld, c_s=(E, d), c_sg=e_s, m=sk, n=d, k=L, batch=Z,
                      zdiv=h_s, groups=cnt)
-                for item in sums:
-                    if item is not None:
-                        _, acc, src, width, w_off = item
-                        c_out, c_in = acc.target(i)
-                        S.col_dgrad(src, flat, w_off, e_s, width, c_out, c0, c_in=c_in)
+                _shard_inputs_grad(sums, flat, e_s, c0, i)
                 i += 1
             rot.release(j)
         runs = store.grad_runs()

@@ -494,7 +494,8 @@ def attn_bwd(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, qkv_strides,
 
 
 def attn_flash_supported(dtype: torch.dtype, L: int, d: int) -> bool:
-    """Whether the running-softmax attention core handles this shape (bf16, any L, d in {32, 64, 128})."""
+    """Whether the running-softmax core is the one for self-attention over packed projections (bf16, any L, d in
+    {32, 64, 128})."""
     if dtype != torch.bfloat16:
         return False
     return bool(_lib.native().rtp_attn_flash_supported(dtype_code(dtype), L, d))
@@ -505,11 +506,11 @@ def _flash_rows(name: str, t: torch.Tensor, G: int, N: int, H: int, L: int) -> N
         raise ValueError(f"{name} must be a contiguous fp32 [G*N*H, L] tensor")
 
 
-def _flash_mask(mask: Optional[torch.Tensor], L: int):
+def _flash_mask(mask: Optional[torch.Tensor], L: int, S: int):
     if mask is None:
         return None
-    if mask.dtype != torch.float32 or tuple(mask.shape) != (L, L) or not mask.is_contiguous():
-        raise ValueError("attention mask must be a contiguous fp32 [L, L] tensor")
+    if mask.dtype != torch.float32 or tuple(mask.shape) != (L, S) or not mask.is_contiguous():
+        raise ValueError("attention mask must be a contiguous fp32 [queries, keys] tensor")
     return mask.data_ptr()
 
 
@@ -523,7 +524,7 @@ def attn_flash_fwd(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, qkv_st
     if o.dtype != qkv.dtype:
         raise ValueError("attn_flash_fwd: o must share the operand dtype")
     _flash_rows("attn_flash_fwd: lse", lse, G, N, H, L)
-    mask_ptr = _flash_mask(mask, L)
+    mask_ptr = _flash_mask(mask, L, L)
     base = qkv.data_ptr()
     native().rtp_attn_flash_fwd(dtype_code(qkv.dtype), base + q_off * esz, base + k_off * esz, base + v_off * esz,
                                 *qkv_strides, o.data_ptr() + o_off * esz, *o_strides, lse.data_ptr(), mask_ptr,
@@ -544,13 +545,54 @@ def attn_flash_bwd(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, qkv_st
         raise ValueError("attn_flash_bwd: o and dout must share dtype and layout")
     _flash_rows("attn_flash_bwd: lse", lse, G, N, H, L)
     _flash_rows("attn_flash_bwd: delta", delta, G, N, H, L)
-    mask_ptr = _flash_mask(mask, L)
+    mask_ptr = _flash_mask(mask, L, L)
     base, dbase = qkv.data_ptr(), dqkv.data_ptr()
     native().rtp_attn_flash_bwd(dtype_code(qkv.dtype), base + q_off * esz, base + k_off * esz, base + v_off * esz,
                                 *qkv_strides, o.data_ptr() + o_off * esz, dout.data_ptr() + o_off * esz, *o_strides,
                                 lse.data_ptr(), delta.data_ptr(), dbase + q_off * esz, dbase + k_off * esz,
                                 dbase + v_off * esz, mask_ptr, _key_bias_ptr("attn_flash_bwd", key_bias, N, L),
                                 int(causal), scale, L, N, H, d, G)
+
+
+def attn_flash_kv_supported(dtype: torch.dtype, L: int, S: int, d: int) -> bool:
+    """Whether the running-softmax core handles L queries and S keys: bf16 or fp32, d in {32, 64, 128}."""
+    if dtype not in (torch.float32, torch.bfloat16):
+        return False
+    return bool(_lib.native().rtp_attn_flash_kv_supported(dtype_code(dtype), L, S, d))
+
+
+def attn_flash_kv_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor, off: int, q_strides, kv_strides,
+                      lse: torch.Tensor, mask: Optional[torch.Tensor], scale: float, L: int, S: int, N: int, H: int,
+                      d: int, G: int, key_bias: Optional[torch.Tensor] = None) -> None:
+    """attn_flash_fwd for queries and keys of two sequences: q and o [L, N, ...] share `q_strides`, k and v [S, N, ...]
+    `kv_strides` ((l, b, h, g) in elements), all four start `off` elements into their buffers; mask [L, S]."""
+    _dev(q)
+    if not (k.dtype == v.dtype == o.dtype == q.dtype):
+        raise ValueError("attn_flash_kv_fwd: q, k, v and o must share a dtype")
+    _flash_rows("attn_flash_kv_fwd: lse", lse, G, N, H, L)
+    by = off * q.element_size()
+    native().rtp_attn_flash_kv_fwd(dtype_code(q.dtype), q.data_ptr() + by, *q_strides, k.data_ptr() + by, v.data_ptr() + by,
+                                   *kv_strides, o.data_ptr() + by, *q_strides, lse.data_ptr(), _flash_mask(mask, L, S),
+                                   _key_bias_ptr("attn_flash_kv_fwd", key_bias, N, S), 0, scale, L, S, N, H, d, G)
+
+
+def attn_flash_kv_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor, dout: torch.Tensor, off: int,
+                      q_strides, kv_strides, lse: torch.Tensor, delta: torch.Tensor, dq: torch.Tensor, dk: torch.Tensor,
+                      dv: torch.Tensor, mask: Optional[torch.Tensor], scale: float, L: int, S: int, N: int, H: int, d: int,
+                      G: int, key_bias: Optional[torch.Tensor] = None) -> None:
+    """Backward of attn_flash_kv_fwd; dout and dq are laid out like q, dk and dv like k; `delta` is scratch like lse."""
+    _dev(q)
+    for t, like in ((dout, q), (dq, q), (dk, k), (dv, k)):
+        if t.dtype != q.dtype or t.shape != like.shape or t.stride() != like.stride():
+            raise ValueError("attn_flash_kv_bwd: gradients must match their operands")
+    _flash_rows("attn_flash_kv_bwd: lse", lse, G, N, H, L)
+    _flash_rows("attn_flash_kv_bwd: delta", delta, G, N, H, L)
+    by = off * q.element_size()
+    native().rtp_attn_flash_kv_bwd(dtype_code(q.dtype), q.data_ptr() + by, *q_strides, k.data_ptr() + by, v.data_ptr() + by,
+                                   *kv_strides, o.data_ptr() + by, dout.data_ptr() + by, *q_strides, lse.data_ptr(),
+                                   delta.data_ptr(), dq.data_ptr() + by, dk.data_ptr() + by, dv.data_ptr() + by,
+                                   _flash_mask(mask, L, S), _key_bias_ptr("attn_flash_kv_bwd", key_bias, N, S), 0, scale, L,
+                                   S, N, H, d, G)
 
 
 def layernorm_supported(dtype: torch.dtype, cols: int) -> bool:

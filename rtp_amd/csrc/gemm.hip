@@ -476,6 +476,24 @@ struct Raw8 {
   }
 };
 
+// Eight logits -> their cross-entropy gradient: (softmax - onehot(target)) * dloss (* scale); rows whose target is the
+// ignore index or outside the classes get zeros.
+template <typename T>
+__device__ __forceinline__ void xent_gradient8(const GemmArgs& p, float (&v)[8], long row, int col, int grp) {
+  const long tg = p.xent_target[row];
+  const bool live = tg != p.xent_ignore && tg >= 0 && tg < (long)p.xent_blocks * 64;
+  const float2 st = p.xent_stats[row];
+  const float inv = 1.0f / st.y;
+  const float sc = live ? p.xent_dloss[0] * (p.xent_scale ? p.xent_scale[0] : 1.0f) : 0.0f;
+  const long gcol = (long)grp * p.n + col;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    float gq = expf(to_f32(from_f32<T>(v[e])) - st.x) * inv;
+    if (gcol + e == tg) gq -= 1.0f;
+    v[e] = gq * sc;
+  }
+}
+
 template <typename T, int BM, int BN, int NTHR>
 __device__ __forceinline__ void finish_tile(const GemmArgs& p, const float* ct, int m0, int n0, int tid, int grp,
                                             long zo, long zi) {
@@ -615,20 +633,7 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& p, const float* ct, 
       for (int e = 0; e < 8; ++e) v[e] = t[e] > 0.0f ? v[e] : 0.0f;
     }
     if (p.xent_mode == 2) {
-      // logits -> their cross-entropy gradient: (softmax - onehot(target)) * dloss (* scale); rows whose target
-      // is the ignore index or outside the classes get zeros
-      const long tg = p.xent_target[row];
-      const bool live = tg != p.xent_ignore && tg >= 0 && tg < (long)p.xent_blocks * 64;
-      const float2 st = p.xent_stats[row];
-      const float inv = 1.0f / st.y;
-      const float sc = live ? p.xent_dloss[0] * (p.xent_scale ? p.xent_scale[0] : 1.0f) : 0.0f;
-      const long gcol = (long)grp * p.n + col;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        float gq = expf(to_f32(from_f32<T>(v[e])) - st.x) * inv;
-        if (gcol + e == tg) gq -= 1.0f;
-        v[e] = gq * sc;
-      }
+      xent_gradient8<T>(p, v, row, col, grp);
     }
     const long off = (long)row * p.ldc + col;
     if (out_f32)
@@ -873,8 +878,13 @@ struct DmaOperand {
     return reinterpret_cast<const char*>(KC ? x + (long)row0 * ld : x + row0);
   }
 
-  // lw: index of the loader wave (0..NL-1).  The host guarantees that a tile's offsets fit 32 bits.
-  __device__ __forceinline__ void init(long ld, int row0, int rows, int lw, int lane) {
+  struct Same {
+    __device__ __forceinline__ int operator()(int r) const { return r; }
+  };
+  // lw: index of the loader wave (0..NL-1).  The host guarantees that a tile's offsets fit 32 bits.  row_of: which row behind
+  // row0 the operand's row r is (runs of a vector's rows or more stay together).
+  template <typename RowOf = Same>
+  __device__ __forceinline__ void init(long ld, int row0, int rows, int lw, int lane, RowOf row_of = RowOf()) {
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const int j = lw * NI + i;  // which KiB of the stage
@@ -882,15 +892,17 @@ struct DmaOperand {
         constexpr int LPR = SB / 16;  // lanes (16-byte chunks) per row
         const int row = j * (64 / LPR) + lane / LPR;
         const int c = (lane % LPR) ^ kc_swizzle<SB>(row);
-        const int rr = row0 + row < rows ? row : rows - 1 - row0;  // rows past the end re-read the last one
+        const int src = row_of(row);
+        const int rr = row0 + src < rows ? src : rows - 1 - row0;  // rows past the end re-read the last one
         ofs[i] = (unsigned)((long)rr * ld * (long)sizeof(T)) + (unsigned)(c * 16);
         koff[i] = c * VEC;
       } else {
         const int byte = lane * 16;
         const int kl = j * (1024 / LINE) + byte / LINE;
-        int chunk = ((byte % LINE) >> 4) ^ rc_swizzle<T, R>(kl);  // which 16 bytes of the k line land here
-        if (row0 + chunk * VEC + VEC > rows) chunk = 0;           // past the end: re-read the tile's first rows
-        ofs[i] = (unsigned)((long)kl * ld * (long)sizeof(T)) + (unsigned)(chunk * 16);
+        const int chunk = ((byte % LINE) >> 4) ^ rc_swizzle<T, R>(kl);  // which 16 bytes of the k line land here
+        int src = row_of(chunk * VEC);
+        if (row0 + src + VEC > rows) src = 0;  // past the end: re-read the tile's first rows
+        ofs[i] = (unsigned)((long)kl * ld * (long)sizeof(T)) + (unsigned)(src * (int)sizeof(T));
         koff[i] = kl;
       }
     }
@@ -1467,33 +1479,56 @@ __global__ __launch_bounds__(512) void gemm_unaligned_kernel(GemmArgs p) {
 
 // ---------------------------------------------------------------------------------------------
 // 256 x 256 tiles for large products.  What bounds the kernel above on a large product is the stream of operand
-// bytes from the L2 into the LDS (a product of 4096^3 takes as long with its MFMAs removed), and that stream is
-// (1/BM + 1/BN) bytes per flop: a 256 x 256 tile moves two thirds of what 256 x 128 moves.  Its 256 KiB of fp32
-// accumulators need all eight waves of the workgroup as MFMA waves (2 x 4 wave tiles of 128 x 64, 128 accumulator
-// registers each), so here the waves issue the direct-to-LDS loads themselves, each an eighth of a slab, right
-// after the barrier that frees a stage.  Both roles in one wave allow a tighter stage protocol than above: every
-// read of slab k's fragments is issued before the first read of slab k+1, and the barrier of slab k+1 sits in front
-// of that read -- so once a wave has seen its own LDS reads return (lgkmcnt 0) and has passed barrier k+1, nobody
-// reads the stage of slab k any more and slab k + NSTAGE may go there.  NSTAGE slabs are in LDS or on their way;
-// the k-step being multiplied lives in registers.  With NSTAGE = 2 this is the plain double buffer, and the two
-// stages can hold slabs of 128 bytes of k per row (2 x 64 KiB): a load instruction then fetches whole cache lines
-// of a K-contiguous operand (with 64-byte rows its operand stream alone took 1.5 x as long as that of a
-// row-contiguous operand), and a barrier comes every 4 k-steps.  The epilogue goes through LDS in four passes of
-// 64 rows.
-template <typename T, bool AKC, bool BKC, int NSTAGE, int SB, int PD>
+// bytes from the L2 into the LDS, and that stream is (1/BM + 1/BN) bytes per flop: a 256 x 256 tile moves two thirds of
+// what 256 x 128 moves.  Its 256 KiB of fp32 accumulators need all eight waves of the workgroup as MFMA waves (2 x 4 wave
+// tiles of 128 x 64, 128 accumulator registers each), so here the waves issue the direct-to-LDS loads themselves.
+//
+// A SIMD holds two of the waves, and their work alternates: a K slab (128 bytes of k per row) is four phases, a phase is a
+// read half -- fragments of half an operand into registers, two load instructions -- and an MFMA half of eight MFMAs,
+// each closed by a workgroup barrier.  The waves of the lower tile half (wm = 1, the second wave of every SIMD) pass one
+// barrier more at the start, so they read while the others multiply and the other way round: LDS reads, loads and scalar
+// work of one wave lie under the MFMAs of the other, and neither waits for its own.
+//
+// An operand's slab is two half tiles of 128 rows (16 KiB each, stored like a 128-row operand), and a wave tile takes half of
+// its rows (columns) from each, so a phase multiplies one quadrant of the wave tile by all of the slab's k:
+//   phase    reads               multiplies        loads (into the half tile freed two phases before)
+//   1        A half 0            A0 x B0           A half 1 of slab k + 1
+//   2        B half 1            A0 x B1           B half 0 of slab k + 2
+//   3        A half 1            A1 x B1           A half 0 of slab k + 2
+//   4        B half 0 of k + 1   A1 x B0           B half 1 of slab k + 2
+// Two barrier-separated halves make phase p's reads complete in every wave before the read half of phase p + 2 begins (the
+// reads have returned when the MFMA half ends), which is where that half tile may be overwritten; and a load has six
+// phases from its issue to its read.  Before a read half ends, a wave waits until its loads of five phases ago have
+// landed (the ten youngest may be on their way); the next phase's reads lie two barriers behind, so that holds for every
+// wave's share.  The epilogue goes through LDS in four passes of 64 rows.
+//
+// Bound by LDS and the matrix pipes together: a slab is 2048 clocks of MFMA per SIMD, 1536 of fragment reads at 128
+// bytes a clock and 64 KiB of arriving loads.  us, forward / input gradient / weight gradient layout (before: all eight
+// waves in step, one barrier a slab, a whole slab requested at once and waited for whole): 4096 x 8192 x 1024 77 / 77 / 80
+// -> 70 / 72 / 73, 6000 x 2048 x 2048 59 / 59 / 60 -> 53 / 54 / 55, 4096^3 128 / 136 / 124 -> 121 / 131 / 124, 8192^3
+// 866 / 848 / 851 -> 840 / 837 / 842.  Closing the MFMA half before its last two MFMAs instead of behind them, so that the
+// waves' MFMAs overlap, costs 10 - 20 %: the two waves of a SIMD then drift into the same half.
+//
+// The half tile of the rows r' = 0 .. 127 holds tile rows half_row<BLK>(r', h): blocks of BLK rows, every other one.
+template <int BLK>
+__device__ __forceinline__ constexpr int half_row(int r, int h) {
+  return ((r & ~(BLK - 1)) << 1) | (h * BLK) | (r & (BLK - 1));
+}
+
+template <typename T, bool AKC, bool BKC>
 __global__ __launch_bounds__(512) void gemm_dma8_kernel(GemmArgs p) {
-  constexpr int BM = 256, BN = 256, NL = 8;
-  using DA = DmaOperand<T, BM, AKC, NL, SB>;
-  using DB = DmaOperand<T, BN, BKC, NL, SB>;
+  constexpr int BM = 256, BN = 256, NL = 8, SB = 128;
+  constexpr int WM = 128, WN = 64, MT = 4, NT = 2;
+  constexpr int BLKA = WM / 2, BLKB = WN / 2;
+  using DA = DmaOperand<T, BM / 2, AKC, NL, SB>;
+  using DB = DmaOperand<T, BN / 2, BKC, NL, SB>;
   constexpr int BK = SB / sizeof(T);
   constexpr int KS = SB / 32;
-  constexpr int WM = 128, WN = 64, MT = 4, NT = 2;
-  constexpr int STAGE = DA::BYTES + DB::BYTES;
-  constexpr int NI = DA::NI + DB::NI;
-  static_assert((NSTAGE - 1) * NI < 64, "vmcnt is a 6-bit counter");
-  static_assert(NSTAGE >= 2 && NSTAGE * STAGE <= 160 * 1024, "2 or more stages within 160 KiB of LDS");
-  static_assert(64 * (BN + 4) * 4 <= NSTAGE * STAGE, "an epilogue pass stages 64 rows of the fp32 tile");
-  __shared__ __attribute__((aligned(1024))) char lds[NSTAGE * STAGE];
+  constexpr int HALF = DA::BYTES;
+  constexpr int NI = DA::NI;  // load instructions per wave and half tile
+  static_assert(DB::BYTES == HALF && DB::NI == NI && 5 * NI < 64, "half tiles of one size; vmcnt is a 6-bit counter");
+  static_assert(64 * (BN + 4) * 4 <= 8 * HALF, "an epilogue pass stages 64 rows of the fp32 tile");
+  __shared__ __attribute__((aligned(1024))) char lds[8 * HALF];  // [slab & 1][A0, A1, B0, B1]
 
   touch_kernel_arguments<sizeof(GemmArgs)>();
   const int tid = threadIdx.x;
@@ -1540,10 +1575,13 @@ __global__ __launch_bounds__(512) void gemm_dma8_kernel(GemmArgs p) {
   // ---- this wave's share of the loads ----
   const T* A = reinterpret_cast<const T*>(p.a) + grp * p.a_sg + zo * p.a_so + zi * p.a_si;
   const T* B = reinterpret_cast<const T*>(p.b) + grp * p.b_sg + zo * p.b_so + zi * p.b_si;
-  DA da;
-  DB db;
-  da.init(p.lda, m0, p.m, wave, lane);
-  db.init(p.ldb, n0, p.n, wave, lane);
+  DA da[2];
+  DB db[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    da[h].init(p.lda, m0, p.m, wave, lane, [=](int r) { return half_row<BLKA>(r, h); });
+    db[h].init(p.ldb, n0, p.n, wave, lane, [=](int r) { return half_row<BLKB>(r, h); });
+  }
   const char* ca = DA::slab_base(A, p.lda, m0);
   const char* cb = DB::slab_base(B, p.ldb, n0);
   constexpr long SZ = (long)sizeof(T);
@@ -1552,116 +1590,128 @@ __global__ __launch_bounds__(512) void gemm_dma8_kernel(GemmArgs p) {
   const int k0_last = (nk_seg - 1) * BK;
   const bool tail = p.k % BK != 0;
   const unsigned lds0 = (unsigned)(uintptr_t)(lptr_t)lds;
-  unsigned fill = lds0;
-  int left = nk_seg;
-  auto issue = [&]() {
-    if (left != 1 || !tail) {
-      da.template issue<false>(fill, wave, ca, 0, 0);
-      db.template issue<false>(fill + DA::BYTES, wave, cb, 0, 0);
-    } else {
-      da.template issue<true>(fill, wave, ca, k0_last, p.k);
-      db.template issue<true>(fill + DA::BYTES, wave, cb, k0_last, p.k);
+  int left_a = nk_seg, left_b = nk_seg;
+  // the next half tile of an operand, half 0 of a slab and then half 1, into the slab at byte `slot` of the LDS
+  auto issue_a = [&](unsigned slot, auto H) {
+    constexpr int h = decltype(H)::value;
+    if (left_a != 1 || !tail)
+      da[h].template issue<false>(lds0 + slot + h * HALF, wave, ca, 0, 0);
+    else
+      da[h].template issue<true>(lds0 + slot + h * HALF, wave, ca, k0_last, p.k);
+    if (h == 1) {
+      ca += left_a != 1 ? step_a : last_a;
+      left_a = left_a != 1 ? left_a - 1 : nk_seg;
     }
-    if (left != 1) {
-      ca += step_a;
-      cb += step_b;
-      --left;
-    } else {
-      ca += last_a;
-      cb += last_b;
-      left = nk_seg;
+  };
+  auto issue_b = [&](unsigned slot, auto H) {
+    constexpr int h = decltype(H)::value;
+    if (left_b != 1 || !tail)
+      db[h].template issue<false>(lds0 + slot + (2 + h) * HALF, wave, cb, 0, 0);
+    else
+      db[h].template issue<true>(lds0 + slot + (2 + h) * HALF, wave, cb, k0_last, p.k);
+    if (h == 1) {
+      cb += left_b != 1 ? step_b : last_b;
+      left_b = left_b != 1 ? left_b - 1 : nk_seg;
     }
-    fill += STAGE;
-    if (fill == lds0 + NSTAGE * STAGE) fill = lds0;
   };
 
-  constexpr int NSET = PD + 1;
-  static_assert(PD >= 1 && PD <= KS, "prefetch distance of 1..KS k-steps");
-  static_assert((NSTAGE * KS) % NSET == 0, "register set of a k-step must not depend on the round");
-  Frag<T> fa[NSET][MT], fb[NSET][NT];
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  Frag<T> fa[2][KS], fb0[KS], fb0n[KS], fb1[KS];  // B half 0 of the next slab is read while this slab's is multiplied
   const bool rowsum = p.a_rowsum != nullptr && tile_n == 0 && wn == 0;
-  auto read_step = [&](auto S, auto Q, auto SET) {
-    const char* sa = lds + (decltype(S)::value % NSTAGE) * STAGE;
-    const char* sb = sa + DA::BYTES;
-    constexpr int q = decltype(Q)::value, set = decltype(SET)::value;
+  auto read_a = [&](unsigned slot, auto H) {
+    const char* st = lds + slot + decltype(H)::value * HALF;
 #pragma unroll
-    for (int i = 0; i < MT; ++i) fa[set][i] = read_frag_dma<T, BM, AKC, SB>(sa, wm * WM + i * 32, lane, q);
+    for (int q = 0; q < KS; ++q)
 #pragma unroll
-    for (int j = 0; j < NT; ++j) fb[set][j] = read_frag_dma<T, BN, BKC, SB>(sb, wn * WN + j * 32, lane, q);
+      for (int i = 0; i < 2; ++i) fa[i][q] = read_frag_dma<T, BM / 2, AKC, SB>(st, wm * BLKA + i * 32, lane, q);
   };
-  auto mma_step = [&](auto SET) {
-    constexpr int set = decltype(SET)::value;
+  auto read_b = [&](unsigned slot, auto H, Frag<T>(&fb)[KS]) {
+    const char* st = lds + slot + (2 + decltype(H)::value) * HALF;
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int j = 0; j < NT; ++j) mma(fa[set][i], fb[set][j], acc[i][j]);
-    if (rowsum) {
-#pragma unroll
-      for (int i = 0; i < MT; ++i) rsum[i] = frag_sum(fa[set][i], rsum[i]);
-    }
+    for (int q = 0; q < KS; ++q) fb[q] = read_frag_dma<T, BN / 2, BKC, SB>(st, wn * BLKB, lane, q);
   };
-  auto step = [&](auto S, auto Q, int k, auto STEADY) {
-    constexpr bool steady = decltype(STEADY)::value;
-    constexpr int s = decltype(S)::value, q = decltype(Q)::value;
-    constexpr int t = s * KS + q;
-    constexpr int tq = (q + PD) % KS, ds = (q + PD) / KS;
-    if (steady || k + ds < nk) {
-      if (ds == 1 && tq == 0) {
-        // barrier k+1: my loads of slab k+1 have landed (those of the slabs up to k+NSTAGE-1 may be on their way)
-        // and my reads of slab k have returned; behind it that holds for everybody, and the stage of slab k takes
-        // slab k+NSTAGE
-        if (k + NSTAGE - 1 < nk) {
-          RTP_WAIT_VM_LGKM0((NSTAGE - 2) * NI);
-        } else {
-          RTP_WAIT_VM_LGKM0(0);
-        }
-        __builtin_amdgcn_s_barrier();
-        if (k + NSTAGE < nk) issue();
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      read_step(std::integral_constant<int, (s + ds) % NSTAGE>{}, std::integral_constant<int, tq>{},
-                std::integral_constant<int, (t + PD) % NSET>{});
+  // the barrier that ends a read half, the MFMA half and its end, where this wave's reads have returned (the first MFMAs
+  // wait only for their own fragments)
+  auto multiply = [&](auto H, auto J, const Frag<T>(&fb)[KS], bool sums) {
+    constexpr int h = decltype(H)::value, j = decltype(J)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int q = 0; q < KS; ++q)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) mma(fa[i][q], fb[q], acc[h * 2 + i][j]);
+    __builtin_amdgcn_s_setprio(0);
+    if (sums && rowsum) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int q = 0; q < KS; ++q) rsum[h * 2 + i] = frag_sum(fa[i][q], rsum[h * 2 + i]);
     }
-    mma_step(std::integral_constant<int, t % NSET>{});
-    constexpr int RPF_A = AKC ? 1 : (sizeof(T) == 2 ? 2 : 4), RPF_B = BKC ? 1 : (sizeof(T) == 2 ? 2 : 4);
-    constexpr int NR = MT * RPF_A + NT * RPF_B, NM = MT * NT * (sizeof(T) == 2 ? 1 : 4);
-    constexpr int PER = (NR + NM - 1) / NM;
-    [&]<int... I>(std::integer_sequence<int, I...>) {
-      ((__builtin_amdgcn_sched_group_barrier(0x008, 1, 0),
-        (I * PER < NR ? __builtin_amdgcn_sched_group_barrier(0x100, (I + 1) * PER <= NR ? PER : NR - I * PER, 0)
-                      : (void)0)),
-       ...);
-    }(std::make_integer_sequence<int, NM>{});
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto phase = [&](auto S, int k, auto STEADY) {
-    if (!decltype(STEADY)::value && k >= nk) return;
-    [&]<int... Q>(std::integer_sequence<int, Q...>) {
-      (step(S, std::integral_constant<int, Q>{}, k, STEADY), ...);
-    }(std::make_integer_sequence<int, KS>{});
-  };
-  auto round = [&](int kt, auto STEADY) {
-    [&]<int... S>(std::integer_sequence<int, S...>) {
-      (phase(std::integral_constant<int, S>{}, kt + S, STEADY), ...);
-    }(std::make_integer_sequence<int, NSTAGE>{});
+  // the slab at byte `cur` of the LDS; REST: slabs behind it (2: two or more)
+  unsigned cur = 0;
+  auto slab = [&](auto REST) {
+    constexpr int rest = decltype(REST)::value;
+    const unsigned other = cur ^ (4 * HALF);
+    read_a(cur, I0{});
+    if constexpr (rest >= 1) issue_a(other, I1{});
+    if constexpr (rest >= 1) RTP_WAIT_VM(5 * NI);
+    else RTP_WAIT_VM(NI);
+    multiply(I0{}, I0{}, fb0, true);
+
+    read_b(cur, I1{}, fb1);
+    if constexpr (rest >= 2) issue_b(cur, I0{});
+    if constexpr (rest >= 2) RTP_WAIT_VM(5 * NI);
+    else if constexpr (rest == 1) RTP_WAIT_VM(4 * NI);
+    else RTP_WAIT_VM(0);
+    multiply(I0{}, I1{}, fb1, false);
+
+    read_a(cur, I1{});
+    if constexpr (rest >= 2) issue_a(cur, I0{});
+    if constexpr (rest >= 2) RTP_WAIT_VM(5 * NI);
+    else if constexpr (rest == 1) RTP_WAIT_VM(3 * NI);
+    multiply(I1{}, I1{}, fb1, true);
+
+    if constexpr (rest >= 1) read_b(other, I0{}, fb0n);
+    if constexpr (rest >= 2) issue_b(cur, I1{});
+    if constexpr (rest >= 2) RTP_WAIT_VM(5 * NI);
+    else if constexpr (rest == 1) RTP_WAIT_VM(2 * NI);
+    multiply(I1{}, I0{}, fb0, false);
+    if constexpr (rest >= 1) {
+#pragma unroll
+      for (int q = 0; q < KS; ++q) fb0[q] = fb0n[q];
+    }
+    cur = other;
   };
 
-  // prologue: NSTAGE slabs on their way, slab 0 landed
-  const int ahead = nk < NSTAGE ? nk : NSTAGE;
-  for (int s_ = 0; s_ < ahead; ++s_) issue();
-  if (nk >= NSTAGE) {
-    RTP_WAIT_VM((NSTAGE - 1) * NI);
-  } else {
-    RTP_WAIT_VM(0);
-  }
-  __builtin_amdgcn_s_barrier();  // barrier 0
-  [&]<int... Q>(std::integer_sequence<int, Q...>) {
-    (read_step(std::integral_constant<int, 0>{}, std::integral_constant<int, Q>{}, std::integral_constant<int, Q>{}), ...);
-  }(std::make_integer_sequence<int, PD>{});
+  // what phases before the first would have issued, in their order; the host sends no problem of a single slab here
+  issue_b(0, I0{});
+  issue_a(0, I0{});
+  issue_b(0, I1{});
+  issue_a(0, I1{});
+  issue_b(4 * HALF, I0{});
+  issue_a(4 * HALF, I0{});
+  issue_b(4 * HALF, I1{});
+  RTP_WAIT_VM(5 * NI);  // halves 0 of slab 0 have landed
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
-  int kt = 0;
-  for (; kt + NSTAGE < nk; kt += NSTAGE) round(kt, std::true_type{});
-  for (; kt < nk; kt += NSTAGE) round(kt, std::false_type{});
+  read_b(0, I0{}, fb0);
+  __builtin_amdgcn_sched_barrier(0);
+  if (wm == 1) __builtin_amdgcn_s_barrier();
+  for (int k = 0; k + 2 < nk; ++k) slab(std::integral_constant<int, 2>{});
+  slab(I1{});
+  slab(I0{});
+  if (wm == 0) __builtin_amdgcn_s_barrier();
 
   if (p.a_rowsum != nullptr && tile_n == 0 && wn == 0) {
     T* dst = reinterpret_cast<T*>(p.a_rowsum) + grp * p.rowsum_sg;
@@ -1674,39 +1724,128 @@ __global__ __launch_bounds__(512) void gemm_dma8_kernel(GemmArgs p) {
   }
 
   // Epilogue in MT passes: pass i stages rows i*32 .. i*32+31 of both tile halves (64 rows of 256 columns, fp32)
-  // in the slab memory; every thread then finishes chunks of 8 columns as in the other kernel.
-  constexpr int CP = BN + 4;
+  // in the slab memory; every thread then finishes four chunks of 8 columns, all in the same columns, whose bias it reads
+  // once per tile.  The barriers wait for LDS alone: __syncthreads would also wait until the previous pass's stores have
+  // reached memory.  The passes are a loop and not unrolled: unrolled, with the shared epilogue function inlined for every
+  // pass, the kernel was 70 - 90 KB of code for an instruction cache of 64 KB; it is 18 KB (-1 to -2 % per launch).
+  auto lds_barrier = [] {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  constexpr int CP = BN + 4, NCH = 4, NB = 2;
   float* ct = reinterpret_cast<float*>(lds);
+  const bool stream_out = p.flags & RTP_GEMM_STREAM_OUT, relu = p.flags & RTP_GEMM_RELU;
+  const bool out_f32 = p.flags & RTP_GEMM_OUT_F32, cin_f32 = p.flags & RTP_GEMM_CIN_F32;
+  char* cbase = p.c_out + (grp * p.c_sg + zo * p.c_so + zi * p.c_si) * (out_f32 ? 4 : SZ);
+  const char* cin = p.c_in ? p.c_in + (grp * p.cin_sg + zo * p.cin_so + zi * p.cin_si) * (cin_f32 ? 4 : SZ) : nullptr;
+  const T* gate =
+      p.gate ? reinterpret_cast<const T*>(p.gate) + grp * p.gate_sg + zo * p.gate_so + zi * p.gate_si : nullptr;
+  const int lc = (tid & 31) * 8, col = n0 + lc, colc = col < p.n ? col : 0;
+  float bcol[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (p.bias) {
+    const T* bias = reinterpret_cast<const T*>(p.bias) + grp * p.bias_sg + zo * p.bias_so + zi * p.bias_si + colc;
+    const int nb_seg = p.bias_sk ? p.ksegs : 1;  // a bias per K segment is summed in segment order
+    for (int sgm = 0; sgm < nb_seg; ++sgm) {
+      float t[8];
+      load8(bias + sgm * p.bias_sk, t);
 #pragma unroll
-  for (int i = 0; i < MT; ++i) {
-    __syncthreads();  // the fragments (first pass) or the previous pass's rows have been read
+      for (int e = 0; e < 8; ++e) bcol[e] += t[e];
+    }
+  }
+  auto stage = [&](const f32x16(&part)[NT]) {
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r)
-        ct[(wm * 32 + 8 * (r >> 2) + 4 * g + (r & 3)) * CP + wn * WN + j * 32 + li] = acc[i][j][r];
-    __syncthreads();
+        ct[(wm * 32 + 8 * (r >> 2) + 4 * g + (r & 3)) * CP + wn * WN + j * 32 + li] = part[j][r];
+  };
+#pragma unroll 1
+  for (int i = 0; i < MT; ++i) {
+    lds_barrier();  // the fragments (first pass) or the previous pass's rows have been read
+    if (i == 0)
+      stage(acc[0]);
+    else if (i == 1)
+      stage(acc[1]);
+    else if (i == 2)
+      stage(acc[2]);
+    else
+      stage(acc[3]);
+    lds_barrier();
+#pragma unroll 1
+    for (int c0 = 0; c0 < NCH; c0 += NB) {
+      auto row_of = [&](int c) {
+        const int lr = (tid >> 5) + 16 * (c0 + c);
+        return m0 + (lr >> 5) * WM + i * 32 + (lr & 31);
+      };
+      Raw8<T> rg[NB], rc16[NB];
+      Raw8<float> rc32[NB];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int mrow = m0 + h * WM + i * 32;
-      if (mrow >= p.m) continue;
-      finish_tile<T, 32, BN, 512>(p, ct + h * 32 * CP, mrow, n0, tid, grp, zo, zi);
+      for (int c = 0; c < NB; ++c) {
+        const int row = row_of(c);
+        const long rowc = row < p.m ? row : p.m - 1;
+        if (cin) {
+          if (cin_f32)
+            rc32[c].load(reinterpret_cast<const float*>(cin) + rowc * p.ld_cin + colc);
+          else
+            rc16[c].load(reinterpret_cast<const T*>(cin) + rowc * p.ld_cin + colc);
+        }
+        if (gate) rg[c].load(gate + rowc * p.ld_gate + colc);
+      }
+#pragma unroll
+      for (int c = 0; c < NB; ++c) {
+        const int lr = (tid >> 5) + 16 * (c0 + c), row = row_of(c);
+        float v[8], t[8];
+        const float4 lo = *reinterpret_cast<const float4*>(ct + lr * CP + lc);
+        const float4 hi = *reinterpret_cast<const float4*>(ct + lr * CP + lc + 4);
+        v[0] = lo.x, v[1] = lo.y, v[2] = lo.z, v[3] = lo.w, v[4] = hi.x, v[5] = hi.y, v[6] = hi.z, v[7] = hi.w;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] *= p.alpha;
+        if (cin) {
+          if (cin_f32)
+            rc32[c].get(t);
+          else
+            rc16[c].get(t);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] += t[e];
+        }
+        if (p.bias) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] += bcol[e];
+        }
+        if (relu) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = fmaxf(v[e], 0.0f);
+        }
+        if (gate) {
+          rg[c].get(t);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = t[e] > 0.0f ? v[e] : 0.0f;
+        }
+        if (row >= p.m || col >= p.n) continue;
+        if (p.xent_mode == 2) xent_gradient8<T>(p, v, row, col, grp);
+        const long off = (long)row * p.ldc + col;
+        if (out_f32)
+          store8(reinterpret_cast<float*>(cbase) + off, v, stream_out);
+        else
+          store8(reinterpret_cast<T*>(cbase) + off, v, stream_out);
+      }
     }
   }
   if (p.trace != nullptr && tid == 0) atomicMax(p.trace + 1, (unsigned long long)wall_clock64());
 }
 
-template <typename T, int NSTAGE, int SB, int PD>
+template <typename T>
 static int launch_dma8(hipStream_t s, const GemmArgs& a, bool akc, bool bkc, dim3 grid) {
   const dim3 block(512);
   if (akc && bkc)
-    hipLaunchKernelGGL((gemm_dma8_kernel<T, true, true, NSTAGE, SB, PD>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((gemm_dma8_kernel<T, true, true>), grid, block, 0, s, a);
   else if (akc && !bkc)
-    hipLaunchKernelGGL((gemm_dma8_kernel<T, true, false, NSTAGE, SB, PD>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((gemm_dma8_kernel<T, true, false>), grid, block, 0, s, a);
   else if (!akc && bkc)
-    hipLaunchKernelGGL((gemm_dma8_kernel<T, false, true, NSTAGE, SB, PD>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((gemm_dma8_kernel<T, false, true>), grid, block, 0, s, a);
   else
-    hipLaunchKernelGGL((gemm_dma8_kernel<T, false, false, NSTAGE, SB, PD>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((gemm_dma8_kernel<T, false, false>), grid, block, 0, s, a);
   RTP_LAUNCH_CHECK();
   return RTP_OK;
 }
@@ -2001,32 +2140,34 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
     const char* e = getenv("RTP_GEMM_TILE");  // debugging aid: index into kShapes
     return e ? atoi(e) : -1;
   }();
-  static const double slab_ns[kNumShapes] = {966.0, 470.0, 283.0, 167.0, 800.0, 1680.0, 545.0};
+  static const double slab_ns[kNumShapes] = {966.0, 470.0, 283.0, 167.0, 800.0, 1400.0, 545.0};
+  // per tile outside the K loop; 256 x 256: 128 KiB of output per CU are 6 us at the memory's rate
+  static const double fixed_ns[kNumShapes] = {3000.0, 3000.0, 3000.0, 3000.0, 3000.0, 9000.0, 3000.0};
   static const int slab_bytes[kNumShapes] = {128, 128, 128, 128, 128, 128, 128};
   const bool vec = direct && a.vec_c;  // else the kernels for operands of any alignment
   int shape = 3;  // 64 x 64 unless the model finds something cheaper
   double best = 0.0;
   for (int i = 0; fast && i < kNumShapes; ++i) {
-    // the 256 x 256 kernel is built for 16-bit operands and the plain epilogue, and pays on products that give
-    // every CU at least one such tile and contract over 1024 or more (measured against the next best shape:
-    // +10 - 25 % at 8192^3, +10 % at 4096^3, +5 - 10 % at K = 1024 .. 1536 when the tiles fill the CUs evenly,
-    // -10 % on the MoE layer's time; a loss where it leaves CUs without a tile or K is shorter)
-    // (its epilogue is the plain one: the update and the statistics epilogue are never routed to it, forced or not)
+    // the 256 x 256 kernel is built for 16-bit operands and the plain epilogue (the update and the statistics epilogue
+    // are never routed to it, forced or not)
     if (i == 5 && (sizeof(T) != 2 || d->sgd_master || d->xent_mode == 1)) continue;
     if (i == 6 && d->xent_mode == 1) continue;  // 160 columns are no whole number of 64-column statistics blocks
     if (!vec && i != 1 && i != 3) continue;  // the kernels for unaligned operands: 128 x 128 and 64 x 64
     // 128 x 160 is priced at the rate measured where it is meant for -- products of at most two rounds of tiles, such
     // as the LM's logits layer (shards of 1280 columns); larger products keep the shapes measured on large products
     if (i == 6 && ceil_div(d->m, 128) * ceil_div(d->n, 160) * nz > 512 && i != forced) continue;
-    if (i == 5 && (ceil_div(d->m, 256) * ceil_div(d->n, 256) * nz < 256 || d->k * d->ksegs < 1024) && i != forced)
-      continue;
+    // Its price holds for contractions of 1024 or more; it needs no full round: on 192 - 255 tiles it is one round where
+    // the others take two or more (6000 x 2048 x 2048, 192 tiles: 53 us against 57 with 128 x 128 and 65 with 256 x 128;
+    // 3000 x 3000 x 1096, 144 tiles: 35 against 48 and 50).
+    if (i == 5 && d->k * d->ksegs < 1024 && i != forced) continue;
+    if (i == 5 && ceil_div(d->k, 64) * d->ksegs < 2) continue;  // its pipeline is primed with two slabs
     // never a tile that is mostly padding: a 32 x 32 problem (one attention head at seq 32) stays at 64 x 64
     if ((!akc && (kShapes[i].bm & (kShapes[i].bm - 1))) || (!bkc && (kShapes[i].bn & (kShapes[i].bn - 1)))) continue;
     if (kShapes[i].bm > 64 && kShapes[i].bm > ceil_div(d->m, 64) * 64) continue;
     if (kShapes[i].bn > 64 && kShapes[i].bn > ceil_div(d->n, 64) * 64) continue;
     const int64_t tiles = ceil_div(d->m, kShapes[i].bm) * ceil_div(d->n, kShapes[i].bn) * nz;
     const double nslabs = (double)ceil_div(d->k * (int64_t)sizeof(T), slab_bytes[i]) * (double)d->ksegs;
-    const double cost = (double)ceil_div(tiles, 256) * (nslabs * slab_ns[i] + 3000.0);
+    const double cost = (double)ceil_div(tiles, 256) * (nslabs * slab_ns[i] + fixed_ns[i]);
     if (best == 0.0 || cost < best || i == forced) {
       best = i == forced ? -1.0 : cost;
       shape = i;
@@ -2156,7 +2297,7 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
       // shard and fills the CUs in two even rounds where 128 x 128 tiles need two and a half
       return launch_dma<T, 128, 160, 4, 128, 1>(s, a, akc, bkc, grid);
     case 5:
-      if constexpr (sizeof(T) == 2) return launch_dma8<T, 2, 128, 1>(s, a, akc, bkc, grid);
+      if constexpr (sizeof(T) == 2) return launch_dma8<T>(s, a, akc, bkc, grid);
       return fail(RTP_ERR_ARG, "gemm: no 256 x 256 kernel for this dtype");
     default:
       return launch_dma<T, 64, 64, 4, 128, 3>(s, a, akc, bkc, grid);

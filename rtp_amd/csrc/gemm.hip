@@ -2156,10 +2156,9 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
     // 128 x 160 is priced at the rate measured where it is meant for -- products of at most two rounds of tiles, such
     // as the LM's logits layer (shards of 1280 columns); larger products keep the shapes measured on large products
     if (i == 6 && ceil_div(d->m, 128) * ceil_div(d->n, 160) * nz > 512 && i != forced) continue;
-    // Its price holds for contractions of 1024 or more; it needs no full round: on 192 - 255 tiles it is one round where
-    // the others take two or more (6000 x 2048 x 2048, 192 tiles: 53 us against 57 with 128 x 128 and 65 with 256 x 128;
-    // 3000 x 3000 x 1096, 144 tiles: 35 against 48 and 50).
-    if (i == 5 && d->k * d->ksegs < 1024 && i != forced) continue;
+    // It needs neither a full round nor a long contraction to pay: on 144 - 255 tiles it is one round where the others take
+    // two or more (6000 x 2048 x 2048, 192 tiles: 53 us against 57 with 128 x 128 and 65 with 256 x 128; 3000 x 3000 x
+    // 1096, 144 tiles: 35 against 48 and 50), and at K = 512 it is 27 us against 34 (8192 x 2048) and 99 against 123 (8192^2).
     if (i == 5 && ceil_div(d->k, 64) * d->ksegs < 2) continue;  // its pipeline is primed with two slabs
     // never a tile that is mostly padding: a 32 x 32 problem (one attention head at seq 32) stays at 64 x 64
     if ((!akc && (kShapes[i].bm & (kShapes[i].bm - 1))) || (!bkc && (kShapes[i].bn & (kShapes[i].bn - 1)))) continue;

@@ -28,9 +28,9 @@ def _pair(gen, m, n, k, akc, bkc):
     return a, b, (a if akc else a.t()).float() @ (b.t() if bkc else b).float()
 
 
-@pytest.mark.parametrize("akc,bkc,k", [(True, True, 1024), (True, False, 1088), (False, False, 1048)])
+@pytest.mark.parametrize("akc,bkc,k", [(True, True, 1024), (True, False, 1088), (False, False, 1048), (True, True, 520), (False, False, 512)])
 def test_mask_and_row_sums(akc, bkc, k):
-    """16, 17 and 17 slabs (the last with 24 k): ReLU mask in the epilogue, and the row sums of A beside the product."""
+    """8 to 17 slabs, whole and ragged last ones: ReLU mask in the epilogue, and the row sums of A beside the product."""
     gen = torch.Generator().manual_seed(k)
     m = n = 3848
     a, b, ref = _pair(gen, m, n, k, akc, bkc)

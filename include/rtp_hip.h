@@ -447,7 +447,7 @@ int rtp_attn_bwd(void* stream, int dtype, const void* q, const void* k, const vo
 /* ---------------------------------------------------------------------------------------------
  * Fused attention core for any number of queries and keys (reference: the same per-head-group core,
  * rtp/module/functional.py:779-800 and :815-830, there bmm -> softmax -> bmm with the [L, S] probabilities
- * in memory).  fp32 or bf16, D in {32, 64, 128}; L queries, S keys; addressing, mask [L][S], key_bias [N][S], causal and
+ * in memory).  bf16, D in {32, 64, 128}; L queries, S keys; addressing, mask [L][S], key_bias [N][S], causal and
  * scale as for rtp_attn_fwd, with element strides of their own for q (and dq) and for k, v (and dk, dv).  One workgroup
  * per (group, batch, head, block of queries) walks the keys in blocks with a running softmax; the probabilities are
  * never stored.  lse and delta are fp32 [G][N][H][L].

@@ -1,4 +1,6 @@
-// Attention core for any number of queries and keys, bf16 and fp32, without the probabilities in memory.
+// Attention core for any number of queries and keys, bf16, without the probabilities in memory.  (In fp32 the backward
+// pass's probabilities, recomputed from a rounded log-sum-exp, were further from fp64 than stored ones -- input gradients 3 - 7 %,
+// the key bias's up to 20 % --, for 4 - 7 % of a layer's time: fp32 keeps the products and the softmax kernel.)
 //
 //   forward : S^T = K Q^T (MFMA) -> running softmax over keys (fp32, in registers) -> O^T += V^T P^T (MFMA);
 //             keeps O and the log-sum-exp per query
@@ -60,16 +62,6 @@ struct Op<bf16_t> {
   static constexpr int ROWS = 64, MR = 8;
   static __device__ __forceinline__ f32x16 mma(Frag a, Frag b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-  }
-};
-template <>
-struct Op<float> {
-  typedef f32x4 Frag;
-  static constexpr int ROWS = 32, MR = 4;
-  static __device__ __forceinline__ f32x16 mma(Frag a, Frag b, f32x16 c) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], c, 0, 0, 0);
-    return c;
   }
 };
 
@@ -271,15 +263,15 @@ __device__ __forceinline__ void lds_values(const float* src, int g, float (&v)[1
 // Waves per SIMD the register allocation aims at.
 template <typename T, int D, bool ADD>
 constexpr int fwd_waves() {
-  return D == 128 ? 2 : D == 64 && (ADD || sizeof(T) == 4) ? 3 : 4;
+  return D == 128 ? 2 : D == 64 && ADD ? 3 : 4;
 }
 template <typename T, int D>
 constexpr int dq_waves() {
-  return sizeof(T) == 4 ? (D == 128 ? 1 : 2) : (D == 128 ? 2 : D == 64 ? 3 : 4);
+  return D == 128 ? 2 : D == 64 ? 3 : 4;
 }
 template <typename T, int D>
 constexpr int dkv_waves() {
-  return D == 128 ? 1 : D == 64 ? 2 : sizeof(T) == 4 ? 2 : 3;
+  return D == 128 ? 1 : D == 64 ? 2 : 3;
 }
 
 // ADD: something joins the scaled scores (a mask, a key bias), or the scale is not positive and their order turns round.
@@ -689,14 +681,13 @@ static void flash_pass(hipStream_t st, FlashArgs a, int64_t own) {
 }
 // `own`: rows of the axis whose blocks the workgroups own
 template <template <typename, int> class Pass>
-static int flash_launch(hipStream_t st, int dtype, int64_t D, const FlashArgs& a, int64_t own) {
-  const bool half = dtype == RTP_BF16;
+static int flash_launch(hipStream_t st, int64_t D, const FlashArgs& a, int64_t own) {
   if (D == 32)
-    half ? flash_pass<Pass<bf16_t, 32>>(st, a, own) : flash_pass<Pass<float, 32>>(st, a, own);
+    flash_pass<Pass<bf16_t, 32>>(st, a, own);
   else if (D == 64)
-    half ? flash_pass<Pass<bf16_t, 64>>(st, a, own) : flash_pass<Pass<float, 64>>(st, a, own);
+    flash_pass<Pass<bf16_t, 64>>(st, a, own);
   else
-    half ? flash_pass<Pass<bf16_t, 128>>(st, a, own) : flash_pass<Pass<float, 128>>(st, a, own);
+    flash_pass<Pass<bf16_t, 128>>(st, a, own);
   RTP_LAUNCH_CHECK();
   return RTP_OK;
 }
@@ -707,7 +698,7 @@ static int flash_args(const char* who, FlashArgs& a, int dtype, const int64_t (&
   RTP_REQUIRE(rtp_attn_flash_kv_supported(dtype, L, S, D), "%s: dtype %d with L = %lld, S = %lld, head dimension %lld", who,
               dtype, (long long)L, (long long)S, (long long)D);
   RTP_REQUIRE(N >= 1 && H >= 1 && G >= 1, "%s: batch, heads and groups must be >= 1", who);
-  const int64_t esz = dtype == RTP_BF16 ? 2 : 4;
+  const int64_t esz = 2;
   for (const auto& s : {&qs, &ks, &os}) {
     for (int i = 0; i < 4; ++i)
       RTP_REQUIRE((*s)[i] * esz % 16 == 0, "%s: strides must be multiples of 16 bytes", who);
@@ -728,7 +719,7 @@ static int flash_args(const char* who, FlashArgs& a, int dtype, const int64_t (&
 using namespace rtp;
 
 extern "C" int rtp_attn_flash_kv_supported(int dtype, int64_t L, int64_t S, int64_t D) {
-  return (dtype == RTP_BF16 || dtype == RTP_F32) && L >= 1 && L <= kFlashMaxLen && S >= 1 && S <= kFlashMaxLen &&
+  return dtype == RTP_BF16 && L >= 1 && L <= kFlashMaxLen && S >= 1 && S <= kFlashMaxLen &&
          (D == 32 || D == 64 || D == 128);
 }
 
@@ -746,9 +737,9 @@ extern "C" int rtp_attn_flash_kv_fwd(void* stream, int dtype, const void* q, int
     return rc;
   a.q = (const char*)q, a.k = (const char*)k, a.v = (const char*)v, a.out = (char*)o, a.lse = lse;
   hipStream_t st = (hipStream_t)stream;
-  const double np = (double)a.nprob, vis = causal ? 0.5 : 1.0, esz = dtype == RTP_BF16 ? 2.0 : 4.0;
+  const double np = (double)a.nprob, vis = causal ? 0.5 : 1.0, esz = 2.0;
   ProfileScope prof(st, "attn_flash_fwd", 4.0 * np * L * S * D * vis, np * (2.0 * (L + S) * D * esz + 4.0 * L));
-  return flash_launch<FlashFwd>(st, dtype, D, a, L);
+  return flash_launch<FlashFwd>(st, D, a, L);
 }
 
 extern "C" int rtp_attn_flash_kv_bwd(void* stream, int dtype, const void* q, int64_t q_l, int64_t q_b, int64_t q_h,
@@ -770,19 +761,19 @@ extern "C" int rtp_attn_flash_kv_bwd(void* stream, int dtype, const void* q, int
   a.o = (const char*)o, a.dout = (const char*)dout;
   a.lse = const_cast<float*>(lse), a.delta = delta;
   hipStream_t st = (hipStream_t)stream;
-  const double np = (double)a.nprob, vis = causal ? 0.5 : 1.0, esz = dtype == RTP_BF16 ? 2.0 : 4.0;
+  const double np = (double)a.nprob, vis = causal ? 0.5 : 1.0, esz = 2.0;
   {
     // the query pass writes delta, the key pass reads it: same stream, in this order
     ProfileScope prof(st, "attn_flash_dq", 6.0 * np * L * S * D * vis, np * ((4.0 * L + 2.0 * S) * D * esz + 8.0 * L));
-    if (int rc = flash_launch<FlashDq>(st, dtype, D, a, L)) return rc;
+    if (int rc = flash_launch<FlashDq>(st, D, a, L)) return rc;
   }
   ProfileScope prof(st, "attn_flash_dkv", 8.0 * np * L * S * D * vis, np * ((2.0 * L + 4.0 * S) * D * esz + 8.0 * L));
-  return flash_launch<FlashDkv>(st, dtype, D, a, S);
+  return flash_launch<FlashDkv>(st, D, a, S);
 }
 
-// q, k and v packed side by side with common strides, as many keys as queries, bf16
+// q, k and v packed side by side with common strides, as many keys as queries
 extern "C" int rtp_attn_flash_supported(int dtype, int64_t L, int64_t D) {
-  return dtype == RTP_BF16 && rtp_attn_flash_kv_supported(dtype, L, L, D);
+  return rtp_attn_flash_kv_supported(dtype, L, L, D);
 }
 
 extern "C" int rtp_attn_flash_fwd(void* stream, int dtype, const void* q, const void* k, const void* v, int64_t s_l,

@@ -136,7 +136,7 @@ class _AttentionFn(torch.autograd.Function):
     batch, head) triple is addressed by strides inside the batched GEMM, so nothing is re-laid out.
 
     The core runs in one of three forms: bf16 with L <= 32 in one launch that keeps the scores in registers and
-    stores p; longer sequences and fp32 in a running-softmax launch that stores only the log-sum-exp per
+    stores p; bf16 with longer sequences in a running-softmax launch that stores only the log-sum-exp per
     query (not when the caller wants the attention weights back); otherwise as batched products and a softmax
     kernel with p in memory."""
 
@@ -367,7 +367,7 @@ class _GeneralAttentionFn(torch.autograd.Function):
     learned key / value bias_k / bias_v (add_bias_kv, functional.py:711-716) and then one all-zero key / value
     (add_zero_attn, functional.py:746-753) appended per batch entry.  Three projections per shard run into
     q [L*N, E], k and v [(S+z)*N, E] (group g at column block g; z appended positions); the core is the running-softmax
-    launch, or, with dropout, per-head masks or the weights wanted back, batched products and the softmax kernel with
+    launch, or, in fp32, with dropout, per-head masks or the weights wanted back, batched products and the softmax kernel with
     p [ws*N*h_s, L, S+z] in memory."""
 
     @staticmethod
@@ -395,7 +395,7 @@ class _GeneralAttentionFn(torch.autograd.Function):
         o = torch.empty(L * N, E, dtype=dt, device=dev)
         out = torch.empty(L * N, E, dtype=dt, device=dev)
         flash = drop_p == 0.0 and not want_weights and (mask is None or mask.dim() == 2) and \
-            ops.attn_flash_kv_supported(dt, L, sk, d)
+            N * E < 1 << 24 and ops.attn_flash_kv_supported(dt, L, sk, d)  # its sequence strides are below 32 MiB
         if flash:
             p = torch.empty(ws * Z, L, dtype=torch.float32, device=dev)  # log-sum-exp in place of probabilities
         else:

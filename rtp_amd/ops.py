@@ -555,7 +555,7 @@ def attn_flash_bwd(qkv: torch.Tensor, q_off: int, k_off: int, v_off: int, qkv_st
 
 
 def attn_flash_kv_supported(dtype: torch.dtype, L: int, S: int, d: int) -> bool:
-    """Whether the running-softmax core handles L queries and S keys: bf16 or fp32, d in {32, 64, 128}."""
+    """Whether the running-softmax core handles L queries and S keys: bf16, d in {32, 64, 128}."""
     if dtype not in (torch.float32, torch.bfloat16):
         return False
     return bool(_lib.native().rtp_attn_flash_kv_supported(dtype_code(dtype), L, S, d))

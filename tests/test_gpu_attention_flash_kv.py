@@ -1,4 +1,4 @@
-"""rtp_attn_flash_kv_fwd / _bwd: queries and keys of two sequences, both dtypes, at the edges of the 32-row groups, the
+"""rtp_attn_flash_kv_fwd / _bwd: queries and keys of two sequences at the edges of the 32-row groups, the
 64- and 128-row workgroups and the key blocks, against float64 on the CPU."""
 import pytest
 import torch
@@ -8,13 +8,13 @@ from gpu_util import DEV, TOL, rel_err
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("L,S,d,N,H,G,mask,pad,scale", [
     (1, 1, 32, 1, 1, 1, False, False, 1.0), (31, 33, 64, 2, 2, 1, True, False, 1.0), (33, 31, 128, 1, 2, 2, False, True, 1.0),
     (64, 65, 32, 2, 1, 2, True, True, 1.0), (65, 64, 64, 1, 3, 1, False, False, 1.0), (129, 97, 128, 1, 2, 1, True, True, 1.0),
     (100, 180, 64, 16, 4, 2, False, True, 1.0), (16, 300, 64, 2, 2, 1, False, False, -1.0), (130, 32, 64, 64, 4, 1, True, False, 1.0)])
-def test_two_sequences(dtype, L, S, d, N, H, G, mask, pad, scale):
+def test_two_sequences(L, S, d, N, H, G, mask, pad, scale):
     from rtp_amd import ops
+    dtype = torch.bfloat16
     gen = torch.Generator().manual_seed(L * 1000 + S)
     e_s, E = H * d, G * H * d
     scale = scale * d ** -0.5

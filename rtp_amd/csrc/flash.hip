@@ -309,8 +309,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_wav
   landed(qf);
   int lrow = B::lane_rows(lane), lcol = B::lane_cols(lane);
   const float c = ADD ? kLog2e : a.scale * kLog2e;
-  // The running maximum (log2 domain) lags behind the true one by up to 2^8: the output is rescaled only when
-  // some query's maximum has moved further than that, and P keeps its relative precision.
+  // The running maximum (log2 domain) follows the true one: the largest P of a query is then 1, which bf16 holds exactly (with
+  // a maximum that may lag behind by 2^8 and fewer rescales, peaked rows lost up to 1 % of the result's accuracy).
   float m_run = -INFINITY, l_run = 0.0f;
   f32x16 acc[DB];
 #pragma unroll
@@ -367,7 +367,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_wav
     float lo, hi;
     halves(bm, lo, hi);
     bm = fmaxf(lo, hi) * c;
-    if (__any(bm > m_run + 8.0f)) {
+    if (__any(bm > m_run)) {
       const float m_new = fmaxf(m_run, bm);
       const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.0f : m_new));
       m_run = m_new;

@@ -1951,6 +1951,92 @@ __global__ __launch_bounds__(kThreads) void gemm_tiny_kernel(GemmArgs p, long nb
   store_tile<T, 1, 1, 32, 32>(p, acc, m0, n0, 0, 0, li, g, grp, zo, zi);
 }
 
+// ---------------------------------------------------------------------------------------------
+// fp32 weight gradients with few output tiles and a long contraction (512 x 512 over thousands of tokens): 64 x 64 tiles
+// leave most CUs idle, one serial chain each.  Here a workgroup owns 32 x 32 outputs and its eight waves an eighth of the
+// contraction each; the partial sums meet in LDS and are added in wave order.  Both operands are row-contiguous, so a lane's
+// MFMA operand is one float of a k line: fragments come straight from global memory (two 128-byte lines per load, any
+// alignment), 16 k ahead of the MFMAs that use them, and there is no staging and no barrier in the loop.
+// Loads and MFMAs of a CU balance (a CU's four SIMDs take eight 256-byte loads per 64-clock MFMA round).
+// us, 64 x 64 tiles -> this: 512 x 512 x 1600 31 -> 21, 512 x 512 x 2880 51 -> 34, 256 x 256 x 1024 21 -> 13, 128 x 128 x 8192
+// 128 -> 74; error against fp64 7.2e-7 -> 2.6e-7 (eight short sums instead of one long one).
+constexpr int kSplitWaves = 8, kSplitBatch = 8;  // waves, MFMAs (two k each) per batch of loads
+__global__ __launch_bounds__(64 * kSplitWaves) void gemm_ksplit_kernel(GemmArgs p) {
+  __shared__ float part[kSplitWaves][32][33];
+  __shared__ float sums[kSplitWaves][32];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int li = lane & 31, g = lane >> 5;
+  int bid = blockIdx.x;
+  const int nb = p.tiles_m * p.tiles_n;
+  if ((nb & 7) == 0) bid = (bid & 7) * (nb >> 3) + (bid >> 3);  // neighbouring tiles on one XCD
+  const int m0 = bid / p.tiles_n * 32, n0 = bid % p.tiles_n * 32;
+  const int grp = blockIdx.y / p.batch, zb = blockIdx.y % p.batch;
+  const long zo = zb / p.zdiv, zi = zb % p.zdiv;
+  // rows past the end re-read the last one: they feed accumulators that are never stored
+  const float* A = reinterpret_cast<const float*>(p.a) + grp * p.a_sg + zo * p.a_so + zi * p.a_si + min(m0 + li, p.m - 1);
+  const float* B = reinterpret_cast<const float*>(p.b) + grp * p.b_sg + zo * p.b_so + zi * p.b_si + min(n0 + li, p.n - 1);
+
+  f32x16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+  float rs = 0.0f;
+  constexpr int STEP = 2 * kSplitBatch;
+  const int chunk = ((p.k + kSplitWaves * STEP - 1) / (kSplitWaves * STEP)) * STEP;
+  const int kb = min(wave * chunk, p.k), ke = min(kb + chunk, p.k);
+  float a[2][kSplitBatch], b[2][kSplitBatch];
+  auto fetch = [&](const float* As, const float* Bs, int k0, float (&fa)[kSplitBatch], float (&fb)[kSplitBatch]) {
+#pragma unroll
+    for (int e = 0; e < kSplitBatch; ++e) {
+      const long k = min(k0 + 2 * e + g, p.k - 1);
+      fa[e] = As[k * p.lda];
+      fb[e] = Bs[k * p.ldb];
+    }
+  };
+  auto multiply = [&](int k0, float (&fa)[kSplitBatch], float (&fb)[kSplitBatch]) {
+#pragma unroll
+    for (int e = 0; e < kSplitBatch; ++e) {
+      const bool live = k0 + 2 * e + g < ke;
+      const float x = live ? fa[e] : 0.0f, y = live ? fb[e] : 0.0f;
+      rs += x;
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc, 0, 0, 0);
+    }
+  };
+  for (int seg = 0; seg < p.ksegs; ++seg) {
+    const float* As = A + seg * p.a_sk;
+    const float* Bs = B + seg * p.b_sk;
+    if (kb < ke) fetch(As, Bs, kb, a[0], b[0]);
+    for (int k0 = kb; k0 < ke; k0 += 2 * STEP) {
+      if (k0 + STEP < ke) fetch(As, Bs, k0 + STEP, a[1], b[1]);
+      multiply(k0, a[0], b[0]);
+      if (k0 + 2 * STEP < ke) fetch(As, Bs, k0 + 2 * STEP, a[0], b[0]);
+      if (k0 + STEP < ke) multiply(k0 + STEP, a[1], b[1]);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 16; ++r) part[wave][8 * (r >> 2) + 4 * g + (r & 3)][li] = acc[r];
+  const float both = rs + __shfl_xor(rs, 32, kWave);
+  if (g == 0) sums[wave][li] = both;
+  __syncthreads();
+
+  if (p.a_rowsum != nullptr && n0 == 0 && threadIdx.x < 32 && m0 + (int)threadIdx.x < p.m) {
+    float v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kSplitWaves; ++w) v += sums[w][threadIdx.x];
+    float* dst = reinterpret_cast<float*>(p.a_rowsum) + grp * p.rowsum_sg + m0 + threadIdx.x;
+    *dst = (p.flags & RTP_GEMM_ROWSUM_ACCUM) ? *dst + v : v;
+  }
+  f32x16 whole[1][1];
+  if (wave != 0) return;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    float v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kSplitWaves; ++w) v += part[w][8 * (r >> 2) + 4 * g + (r & 3)][li];
+    whole[0][0][r] = v;
+  }
+  store_tile<float, 1, 1, 32, 32>(p, whole, m0, n0, 0, 0, li, g, grp, zo, zi);
+}
+
 template <typename T, int BM, int BN, int DEPTH, bool FAST>
 static int launch_layout(hipStream_t s, const GemmArgs& a, bool akc, bool bkc, dim3 grid) {
   if (akc && bkc)
@@ -2130,6 +2216,19 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
       hipLaunchKernelGGL((gemm_tiny_kernel<T, false, true>), tgrid, dim3(kThreads), 0, s, a, (long)nblocks);
     else
       hipLaunchKernelGGL((gemm_tiny_kernel<T, false, false>), tgrid, dim3(kThreads), 0, s, a, (long)nblocks);
+    RTP_LAUNCH_CHECK();
+    return RTP_OK;
+  }
+  // few fp32 weight-gradient tiles, long contraction: see gemm_ksplit_kernel.  At 64 tiles of 64 x 64 it is ahead (512 x 512 x 512
+  // 13 -> 9 us), at 128 behind (512 x 1024 x 2048 38 -> 46 us: every CU has work in both, and this one reads more).
+  if (sizeof(T) == 4 && fast && !akc && !bkc && !d->sgd_master && !d->xent_mode && d->k >= 512 && nz < 65536 &&
+      ceil_div(d->m, 64) * ceil_div(d->n, 64) * nz <= 64) {
+    a.tiles_m = (int)ceil_div(d->m, 32);
+    a.tiles_n = (int)ceil_div(d->n, 32);
+    const double mn_ = (double)d->m * (double)d->n * (double)nz, kk_ = (double)d->k * (double)d->ksegs;
+    ProfileScope prof(s, "gemm_f32_32x32_ksplit_rc_rc", 2.0 * mn_ * kk_,
+                      ((double)d->m + (double)d->n) * kk_ * nz * sizeof(T) + mn_ * sizeof(T));
+    hipLaunchKernelGGL(gemm_ksplit_kernel, dim3((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nz), dim3(64 * kSplitWaves), 0, s, a);
     RTP_LAUNCH_CHECK();
     return RTP_OK;
   }

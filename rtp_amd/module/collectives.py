@@ -113,9 +113,31 @@ class ShardStore:
         for s in range(self.world_size):
             self.modules[s]._full_param = home[s]
             self.modules[s]._full_grad = None
-            for p, off, n, shape in zip(self.params(s), self.offsets, self.numels, self.shapes):
-                p.data = home[s, off:off + n].view(shape)
+            for p, v in zip(self._params[s], self.views(home[s])):
+                p.data = v
                 p.grad = None
+
+    # what follows from `home`, `grads` and the shard modules: not part of a copied or saved store (the book is an object
+    # of the extension module, which neither copies nor pickles), made again when the copy is
+    _DERIVED = ("one_run", "_params", "_book", "_grad_rows", "_grad_slices")
+
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k not in self._DERIVED}
+
+    def __setstate__(self, state) -> None:
+        """A deep copy clones every parameter, and so does a plain pickle: the parameters are pointed at the copy's own
+        home rows again, as pack() left them (torch.save / torch.load kept that by itself)."""
+        from .. import ring
+        self.__dict__.update(state)
+        self.one_run = ring.OneRun(self.home)
+        self._params = [list(m.parameters()) for m in self.modules]
+        self._book, self._grad_rows, self._grad_slices = None, [], []
+        for s, m in enumerate(self.modules):
+            m._full_param = self.home[s]
+            if self.grads is not None and m._full_grad is not None:
+                m._full_grad = self.grads[s]
+            for p, v in zip(self._params[s], self.views(self.home[s])):
+                p.data = v
 
     def views(self, flat: torch.Tensor) -> List[torch.Tensor]:
         """Parameter-shaped views of one flat shard (home row or staged copy)."""
@@ -129,15 +151,18 @@ class ShardStore:
 
     def _grad_storage(self) -> None:
         """The gradient buffer, its slices and the record the attaching works from: made on the first backward after
-        pack()."""
-        if self.grads is not None and self._book is not None:
+        pack(), the last two also on the first one of a copied store, which holds a buffer already."""
+        if self._book is not None:
             return
         from .. import _lib
-        self.grads = torch.empty_like(self.home)
+        first = self.grads is None
+        if first:
+            self.grads = torch.empty_like(self.home)
         self._grad_rows = list(self.grads.unbind(0))
         self._grad_slices = [self.views(row) for row in self._grad_rows]
         self._book = _lib.native().GradBook(self._params, self._grad_slices)
-        self._book.drop()
+        if first:
+            self._book.drop()
 
     def grad_views(self, s: int) -> Tuple[List[torch.Tensor], bool]:
         """Gradient slices of shard s and whether the caller must ACCUMULATE into them.

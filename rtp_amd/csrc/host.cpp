@@ -16,9 +16,12 @@
 #include <c10/hip/HIPStream.h>
 #include <dlfcn.h>
 #include <torch/csrc/Dtype.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <cstring>
+#include <exception>
 #include <string>
 #include <type_traits>
 #include <utility>
@@ -37,6 +40,28 @@ PyObject* raise_status(long rc) {
   PyErr_Format(g_error, "librtp_hip status %ld: %s", rc, f_last_error());
   return nullptr;
 }
+
+// A C++ exception may not cross into the interpreter, it would end the process: a tensor's data_ptr() throws for a sparse or
+// a functorch tensor, its sizes for a nested one.  Every function Python can call is entered through here and such an
+// exception raised as the Python one torch's own bindings make of it.
+template <auto F>
+struct Entry;
+template <class... A, PyObject* (*F)(A...)>
+struct Entry<F> {
+  static PyObject* call(A... a) {
+    try {
+      return F(a...);
+    } catch (const std::exception&) {
+      torch::translate_exception_to_python(std::current_exception());
+    }
+    return nullptr;
+  }
+};
+
+struct WithoutGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~WithoutGil() { PyEval_RestoreThread(state); }
+};
 
 // ---- one argument ----
 template <class T>
@@ -65,10 +90,7 @@ PyObject* invoke_at(R (*f)(A...), PyObject* const* args, std::index_sequence<I..
   bool ok = true;
   (void)std::initializer_list<int>{(ok = ok && (I < S || from_py(args[I < S ? 0 : I - S], std::get<I>(v))), 0)...};
   if (!ok) return nullptr;
-  R r;
-  Py_BEGIN_ALLOW_THREADS
-  r = std::apply(f, v);
-  Py_END_ALLOW_THREADS
+  const R r = (WithoutGil(), std::apply(f, v));
   if constexpr (std::is_same_v<R, int>) {
     if (r < 0) return raise_status(r);
   }
@@ -241,11 +263,8 @@ PyObject* py_gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObject* 
     else
       d.a_rowsum = nullptr, d.rowsum_sg = 0;
   }
-  int rc;
   void* st = current_stream();
-  Py_BEGIN_ALLOW_THREADS
-  rc = f_gemm(st, dt, &d);
-  Py_END_ALLOW_THREADS
+  const int rc = (WithoutGil(), f_gemm(st, dt, &d));
   if (rc < 0) return raise_status(rc);
   return PyLong_FromLong(done);
 }
@@ -299,13 +318,11 @@ PyObject* py_linear_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
       x2.scalar_type() != home.scalar_type() || (f32 && y.scalar_type() != at::kFloat))
     return bad("rotated_linear_fwd: x [rows, k] in the shards' dtype, y [rows, >= shards * n_s] (or fp32)");
   const int flags = (PyObject_IsTrue(a[8]) ? RTP_GEMM_RELU : 0) | (f32 ? RTP_GEMM_OUT_F32 : 0);
-  int rc;
   void* st = current_stream();
   // one row: any leading dimension that holds it
   const int64_t ldo = o.rows > 1 ? o.ld : std::max<int64_t>(o.cols, 1);
-  Py_BEGIN_ALLOW_THREADS
-  rc = f_linear_fwd(st, dt, &L, x.p, x.ld, x.rows, o.p + col0 * (int64_t)y.element_size(), ldo, flags);
-  Py_END_ALLOW_THREADS
+  char* out = o.p + col0 * (int64_t)y.element_size();
+  const int rc = (WithoutGil(), f_linear_fwd(st, dt, &L, x.p, x.ld, x.rows, out, ldo, flags));
   if (rc < 0) return raise_status(rc);
   Py_RETURN_NONE;
 }
@@ -368,12 +385,10 @@ PyObject* py_linear_bwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
       return nullptr;
     o.sgd_skip_grad_store = o.sgd_master ? PyObject_IsTrue(a[17]) : 0;
   }
-  int rc;
   void* st = current_stream();
   const int64_t ldy = dy.rows > 1 ? dy.ld : std::max<int64_t>(dy.cols, 1);
-  Py_BEGIN_ALLOW_THREADS
-  rc = f_linear_bwd(st, dt, &L, dy.p + col0 * (int64_t)dy2.element_size(), ldy, x.p, x.ld, dy.rows, &o);
-  Py_END_ALLOW_THREADS
+  const char* in = dy.p + col0 * (int64_t)dy2.element_size();
+  const int rc = (WithoutGil(), f_linear_bwd(st, dt, &L, in, ldy, x.p, x.ld, dy.rows, &o));
   if (rc < 0) return raise_status(rc);
   return PyLong_FromLong(done);
 }
@@ -444,12 +459,10 @@ PyObject* book_attach(PyObject* o, PyObject*) {
   GradBook& b = *(GradBook*)o;
   size_t fresh = 0, full = 0;
   for (size_t s = 0; s < b.params->size(); ++s) {
-    bool none = false, own = true;
-    for (size_t i = 0; i < (*b.params)[s].size(); ++i) {
-      const at::Tensor& g = (*b.params)[s][i].grad();
-      none = none || !g.defined();
-      own = own && g.defined() && g.data_ptr() == (*b.views)[s][i].data_ptr();
-    }
+    const auto& row = (*b.params)[s];
+    const bool none = std::any_of(row.begin(), row.end(), [](const at::Tensor& p) { return !p.grad().defined(); });
+    bool own = !none;
+    for (size_t i = 0; own && i < row.size(); ++i) own = row[i].grad().data_ptr() == (*b.views)[s][i].data_ptr();
     fresh += none, full += own;
   }
   if (fresh == b.params->size()) {
@@ -474,15 +487,15 @@ PyObject* book_drop(PyObject* o, PyObject*) {
   Py_RETURN_NONE;
 }
 
-PyMethodDef book_methods[] = {{"attach", book_attach, METH_NOARGS, nullptr},
-                              {"complete", book_complete, METH_NOARGS, nullptr},
-                              {"drop", book_drop, METH_NOARGS, nullptr},
+PyMethodDef book_methods[] = {{"attach", Entry<book_attach>::call, METH_NOARGS, nullptr},
+                              {"complete", Entry<book_complete>::call, METH_NOARGS, nullptr},
+                              {"drop", Entry<book_drop>::call, METH_NOARGS, nullptr},
                               {nullptr, nullptr, 0, nullptr}};
 PyTypeObject g_book_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
-#define METHOD(name) {#name, (PyCFunction)(void*)py_##name, METH_FASTCALL, nullptr},
-PyMethodDef g_methods[] = {{"bind", py_bind, METH_VARARGS, nullptr},
-                           {"gemm", (PyCFunction)(void*)py_gemm, METH_FASTCALL | METH_KEYWORDS, nullptr},
+#define METHOD(name) {#name, (PyCFunction)(void*)Entry<py_##name>::call, METH_FASTCALL, nullptr},
+PyMethodDef g_methods[] = {{"bind", Entry<py_bind>::call, METH_VARARGS, nullptr},
+                           {"gemm", (PyCFunction)(void*)Entry<py_gemm>::call, METH_FASTCALL | METH_KEYWORDS, nullptr},
                            METHOD(linear_fwd) METHOD(linear_bwd) RTP_ENTRY_POINTS(METHOD, METHOD){nullptr, nullptr, 0, nullptr}};
 #undef METHOD
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_rtp_native", "librtp_hip.so for the calls of a training step", -1, g_methods};
@@ -500,7 +513,7 @@ PyMODINIT_FUNC PyInit__rtp_native(void) {
   g_book_type.tp_name = "_rtp_native.GradBook";
   g_book_type.tp_basicsize = sizeof(GradBook);
   g_book_type.tp_flags = Py_TPFLAGS_DEFAULT;
-  g_book_type.tp_new = book_new;
+  g_book_type.tp_new = Entry<book_new>::call;
   g_book_type.tp_dealloc = book_dealloc;
   g_book_type.tp_methods = book_methods;
   if (PyType_Ready(&g_book_type) < 0) return nullptr;

@@ -49,3 +49,43 @@ def test_argument_errors():
     with pytest.raises(_lib.RtpError):
         n.linear_fwd(torch.zeros(2, 4), torch.zeros(1, 8), 0, None, 2, 4, torch.zeros(2, 2), 0, False)
     assert n.rtp_attn_supported(_lib.RTP_BF16, 32, 64) == 1 and n.rtp_attn_supported(_lib.RTP_F32, 32, 64) == 0
+
+
+def test_a_tensor_without_plain_storage_raises():
+    """data_ptr(), strides and sizes throw in C++ for such tensors; every function turns that into a Python error."""
+    n = _lib.native()
+    sparse = torch.eye(4).to_sparse()
+    with pytest.raises(RuntimeError):
+        n.gemm(torch.float32, a=sparse, m=1)
+    with pytest.raises(RuntimeError):
+        n.rtp_gemm_warm_next(sparse, 0)
+    with pytest.raises((RuntimeError, ValueError)):
+        n.linear_fwd(torch.zeros(2, 4), sparse, 0, None, 2, 4, torch.zeros(2, 2), 0, False)
+    with pytest.raises((RuntimeError, ValueError)):
+        n.linear_bwd(sparse, 0, None, sparse, 0, None, 1, 4, None, None, None, None, False, None, None, 0.0, 0.0, False)
+    seen = []
+
+    def probe(x):  # a functorch tensor has no storage of its own
+        with pytest.raises(RuntimeError):
+            n.rtp_gemm_warm_next(x, 0)
+        seen.append(x)
+        return x.sum()
+
+    torch.func.grad(probe)(torch.ones(3))
+    assert len(seen) == 1
+
+
+def test_grad_book_with_a_gradient_of_another_layout():
+    params, grads, views, book = _layer()
+    book.attach()
+    w, b = params[0]
+    w.grad = torch.ones(2, 3).to_sparse()
+    with pytest.raises(RuntimeError):
+        book.attach()
+    assert w.grad.is_sparse and book.complete()                                 # nothing was attached
+    b.grad = None                                                               # a fresh shard is attached as a whole
+    params[1][0].grad = None
+    assert book.attach() == 0 and w.grad.data_ptr() == views[0][0].data_ptr()
+    w.grad = torch.ones(2, 3).to_sparse()
+    book.drop()
+    assert w.grad is None

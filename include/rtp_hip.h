@@ -454,8 +454,9 @@ int rtp_attn_bwd(void* stream, int dtype, const void* q, const void* k, const vo
  *   fwd: o = softmax(scale * q k^T + mask) v,  lse = log sum_j exp(scale * q k_j + mask_j)
  *   bwd: p recomputed from lse; delta = rowsum(dout o o) (written here, scratch for the caller);
  *        dv = p^T dout, ds = scale * p o (dout v^T - delta), dq = ds k, dk = ds^T q
- * A query whose keys are all masked with -inf gets o = 0 and lse = 0 (torch gives NaN there).
  * rtp_attn_flash_fwd / _bwd: the form with common strides for q, k and v and S == L.
+ * A query whose keys are all masked with -inf gets NaN in o and lse from the kv form, and NaN gradients through it, as
+ * rtp_softmax_fwd and torch give; from the common-stride form it gets o = 0, lse = 0 and no gradients.
  * --------------------------------------------------------------------------------------------- */
 int rtp_attn_flash_kv_supported(int dtype, int64_t L, int64_t S, int64_t D);
 int rtp_attn_flash_kv_fwd(void* stream, int dtype, const void* q, int64_t q_l, int64_t q_b, int64_t q_h, int64_t q_g,

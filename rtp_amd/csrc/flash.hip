@@ -45,6 +45,7 @@ struct FlashArgs {
   float scale;
   int L, S, N, H, nblk;  // nblk: workgroups along the owned axis
   int nprob;             // G * N * H; nprob * nblk < 2^31
+  float empty;           // forward: what a query without a visible key gets, in o and in lse
 };
 
 constexpr float kLog2e = 1.44269504088896340736f;
@@ -415,11 +416,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_wav
   halves(l_run, lo, hi);
   const float l = lo + hi;
   if (query < a.L) {
-    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    const float inv = l > 0.0f ? 1.0f / l : a.empty;
     char* row = a.out + it.o + (long)query * a.o_l;
 #pragma unroll
     for (int db = 0; db < DB; ++db) store_acc<T>(row, db, g, acc[db], inv);
-    if (g == 0) a.lse[(long)it.z * a.L + query] = l > 0.0f ? (m_run + __builtin_amdgcn_logf(l)) * kLn2 : 0.0f;
+    if (g == 0) a.lse[(long)it.z * a.L + query] = l > 0.0f ? (m_run + __builtin_amdgcn_logf(l)) * kLn2 : a.empty;
   }
 }
 
@@ -723,23 +724,29 @@ extern "C" int rtp_attn_flash_kv_supported(int dtype, int64_t L, int64_t S, int6
          (D == 32 || D == 64 || D == 128);
 }
 
+static int flash_forward(void* stream, int dtype, const void* q, const int64_t (&qs)[4], const void* k, const void* v,
+                         const int64_t (&ks)[4], void* o, const int64_t (&os)[4], float* lse, const float* mask,
+                         const float* key_bias, int causal, float scale, int64_t L, int64_t S, int64_t N, int64_t H,
+                         int64_t D, int64_t G, float empty) {
+  RTP_REQUIRE(q && k && v && o && lse, "rtp_attn_flash_fwd: null pointer");
+  RTP_REQUIRE(((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)o) % 16 == 0,
+              "rtp_attn_flash_fwd: q, k, v, o must be 16-byte aligned");
+  FlashArgs a{};
+  if (int rc = flash_args("rtp_attn_flash_fwd", a, dtype, qs, ks, os, mask, key_bias, causal, scale, L, S, N, H, D, G)) return rc;
+  a.q = (const char*)q, a.k = (const char*)k, a.v = (const char*)v, a.out = (char*)o, a.lse = lse, a.empty = empty;
+  hipStream_t st = (hipStream_t)stream;
+  const double np = (double)a.nprob, vis = causal ? 0.5 : 1.0, esz = 2.0;
+  ProfileScope prof(st, "attn_flash_fwd", 4.0 * np * L * S * D * vis, np * (2.0 * (L + S) * D * esz + 4.0 * L));
+  return flash_launch<FlashFwd>(st, D, a, L);
+}
+
 extern "C" int rtp_attn_flash_kv_fwd(void* stream, int dtype, const void* q, int64_t q_l, int64_t q_b, int64_t q_h,
                                      int64_t q_g, const void* k, const void* v, int64_t k_l, int64_t k_b, int64_t k_h,
                                      int64_t k_g, void* o, int64_t o_l, int64_t o_b, int64_t o_h, int64_t o_g, float* lse,
                                      const float* mask, const float* key_bias, int causal, float scale, int64_t L,
                                      int64_t S, int64_t N, int64_t H, int64_t D, int64_t G) {
-  RTP_REQUIRE(q && k && v && o && lse, "rtp_attn_flash_fwd: null pointer");
-  RTP_REQUIRE(((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)o) % 16 == 0,
-              "rtp_attn_flash_fwd: q, k, v, o must be 16-byte aligned");
-  FlashArgs a{};
-  if (int rc = flash_args("rtp_attn_flash_fwd", a, dtype, {q_l, q_b, q_h, q_g}, {k_l, k_b, k_h, k_g}, {o_l, o_b, o_h, o_g},
-                          mask, key_bias, causal, scale, L, S, N, H, D, G))
-    return rc;
-  a.q = (const char*)q, a.k = (const char*)k, a.v = (const char*)v, a.out = (char*)o, a.lse = lse;
-  hipStream_t st = (hipStream_t)stream;
-  const double np = (double)a.nprob, vis = causal ? 0.5 : 1.0, esz = 2.0;
-  ProfileScope prof(st, "attn_flash_fwd", 4.0 * np * L * S * D * vis, np * (2.0 * (L + S) * D * esz + 4.0 * L));
-  return flash_launch<FlashFwd>(st, D, a, L);
+  return flash_forward(stream, dtype, q, {q_l, q_b, q_h, q_g}, k, v, {k_l, k_b, k_h, k_g}, o, {o_l, o_b, o_h, o_g}, lse, mask,
+                       key_bias, causal, scale, L, S, N, H, D, G, __builtin_nanf(""));
 }
 
 extern "C" int rtp_attn_flash_kv_bwd(void* stream, int dtype, const void* q, int64_t q_l, int64_t q_b, int64_t q_h,
@@ -780,8 +787,8 @@ extern "C" int rtp_attn_flash_fwd(void* stream, int dtype, const void* q, const 
                                   int64_t s_b, int64_t s_h, int64_t s_g, void* o, int64_t o_l, int64_t o_b,
                                   int64_t o_h, int64_t o_g, float* lse, const float* mask, const float* key_bias,
                                   int causal, float scale, int64_t L, int64_t N, int64_t H, int64_t D, int64_t G) {
-  return rtp_attn_flash_kv_fwd(stream, dtype, q, s_l, s_b, s_h, s_g, k, v, s_l, s_b, s_h, s_g, o, o_l, o_b, o_h, o_g, lse,
-                               mask, key_bias, causal, scale, L, L, N, H, D, G);
+  return flash_forward(stream, dtype, q, {s_l, s_b, s_h, s_g}, k, v, {s_l, s_b, s_h, s_g}, o, {o_l, o_b, o_h, o_g}, lse, mask,
+                       key_bias, causal, scale, L, L, N, H, D, G, 0.0f);
 }
 
 extern "C" int rtp_attn_flash_bwd(void* stream, int dtype, const void* q, const void* k, const void* v, int64_t s_l,

@@ -1,0 +1,47 @@
+"""bf16 attention for queries that see no key, keys and values of another sequence: NaN, as nn.MultiheadAttention gives."""
+import pytest
+import torch
+import torch.nn as nn
+
+from gpu_util import DEV, TOL, rel_err
+
+pytestmark = pytest.mark.gpu
+
+DT = torch.bfloat16
+
+
+def _pair(E, H, ws):
+    from rtp_amd.module.attention import ParallelMultiheadAttention
+    ref = nn.MultiheadAttention(E, H).to(DT)
+    layer = ParallelMultiheadAttention(E, H, ws, 0, MultiheadAttention_layer=ref, device=DEV, dtype=DT)
+    return layer, ref.float()
+
+
+def _run(layer, ref, L, S, N, E, **masks):
+    gen = torch.Generator().manual_seed(L + S)
+    q, k, g = (torch.randn(n, N, E, generator=gen).to(DT) for n in (L, S, L))
+    qd, kd = (t.to(DEV).requires_grad_() for t in (q, k))
+    qf, kf = (t.float().requires_grad_() for t in (q, k))
+    out, _ = layer(qd, kd, kd, need_weights=False, **{n: m.to(DEV) for n, m in masks.items()})
+    out.backward(g.to(DEV))
+    want, _ = ref(qf, kf, kf, need_weights=True, **masks)   # the explicit form: scores + mask, softmax
+    want.backward(g.float())
+    return [t.detach().float().cpu() for t in (out, qd.grad, kd.grad)], [t.detach() for t in (want, qf.grad, kf.grad)]
+
+
+@pytest.mark.parametrize("L,S", [(5, 40), (70, 33)])
+def test_boolean_masks_that_hide_every_key_give_nan(L, S):
+    layer, ref = _pair(128, 4, 2)
+    kpm = torch.zeros(3, S, dtype=torch.bool)
+    kpm[1] = True
+    kpm[2, S // 2:] = True
+    got, want = _run(layer, ref, L, S, 3, 128, key_padding_mask=kpm)
+    for a, b in zip(got, want):
+        assert torch.equal(a[:, 1].isnan(), b[:, 1].isnan()) and b[:, 1].isnan().all()
+        assert rel_err(a[:, ::2], b[:, ::2]) <= TOL[DT]
+    hidden = torch.zeros(L, S, dtype=torch.bool)
+    hidden[L - 1] = True
+    got, want = _run(layer, ref, L, S, 3, 128, attn_mask=hidden)
+    assert got[0][L - 1].isnan().all() and got[1][L - 1].isnan().all() and got[2].isnan().all() and want[2].isnan().all()
+    for a, b in zip(got[:2], want[:2]):
+        assert rel_err(a[:L - 1], b[:L - 1]) <= TOL[DT]

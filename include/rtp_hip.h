@@ -457,6 +457,8 @@ int rtp_attn_bwd(void* stream, int dtype, const void* q, const void* k, const vo
  * rtp_attn_flash_fwd / _bwd: the form with common strides for q, k and v and S == L.
  * A query whose keys are all masked with -inf gets NaN in o and lse from the kv form, and NaN gradients through it, as
  * rtp_softmax_fwd and torch give; from the common-stride form it gets o = 0, lse = 0 and no gradients.
+ * The backward pass knows a query's scores only relative to an fp32 lse: masks that add a large finite value to ALL keys of
+ * a query (-1e9 instead of -inf) leave it p with an error of |lse| * 2^-24; rtp_softmax_fwd with stored p has no such bound.
  * --------------------------------------------------------------------------------------------- */
 int rtp_attn_flash_kv_supported(int dtype, int64_t L, int64_t S, int64_t D);
 int rtp_attn_flash_kv_fwd(void* stream, int dtype, const void* q, int64_t q_l, int64_t q_b, int64_t q_h, int64_t q_g,

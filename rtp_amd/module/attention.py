@@ -367,11 +367,15 @@ class _GeneralAttentionFn(torch.autograd.Function):
     learned key / value bias_k / bias_v (add_bias_kv, functional.py:711-716) and then one all-zero key / value
     (add_zero_attn, functional.py:746-753) appended per batch entry.  Three projections per shard run into
     q [L*N, E], k and v [(S+z)*N, E] (group g at column block g; z appended positions); the core is the running-softmax
-    launch, or, in fp32, with dropout, per-head masks or the weights wanted back, batched products and the softmax kernel with
-    p [ws*N*h_s, L, S+z] in memory."""
+    launch, or, in fp32, with dropout, per-head masks, masks given as floats or the weights wanted back, batched products and
+    the softmax kernel with p [ws*N*h_s, L, S+z] in memory.
+
+    `hides_only`: mask and key_bias hold 0 and -inf alone.  The running-softmax backward recomputes p from the queries' fp32
+    log-sum-exp; a float mask may add any value to all keys of a query (-1e9, the type's lowest), and p recomputed next to
+    a log-sum-exp of that size would be lost in its rounding.  A query without a visible key gives NaN in both forms."""
 
     @staticmethod
-    def forward(ctx, query, key, value, anchor, layer, mask, key_bias, want_weights, drop_p=0.0):
+    def forward(ctx, query, key, value, anchor, layer, mask, key_bias, want_weights, drop_p=0.0, hides_only=True):
         store = layer._store
         L, N, E = query.shape
         s_in = key.shape[0]
@@ -394,7 +398,7 @@ class _GeneralAttentionFn(torch.autograd.Function):
         bk_off, bv_off = _bias_kv_layout(layer) if bkv else (None, None)
         o = torch.empty(L * N, E, dtype=dt, device=dev)
         out = torch.empty(L * N, E, dtype=dt, device=dev)
-        flash = drop_p == 0.0 and not want_weights and (mask is None or mask.dim() == 2) and \
+        flash = drop_p == 0.0 and not want_weights and hides_only and (mask is None or mask.dim() == 2) and \
             N * E < 1 << 24 and ops.attn_flash_kv_supported(dt, L, sk, d)  # its sequence strides are below 32 MiB
         if flash:
             p = torch.empty(ws * Z, L, dtype=torch.float32, device=dev)  # log-sum-exp in place of probabilities
@@ -547,7 +551,7 @@ class _GeneralAttentionFn(torch.autograd.Function):
         dq = None if grads[0] is None else grads[0].view(L, N, E)
         dk = None if grads[1] is None else grads[1].view(s_in, N, layer.kdim)
         dv = None if grads[2] is None else grads[2].view(s_in, N, layer.vdim)
-        return dq, dk, dv, None, None, None, None, None, None
+        return dq, dk, dv, None, None, None, None, None, None, None
 
 
 class ParallelMultiheadAttention(RotatedLayer):
@@ -647,8 +651,9 @@ class ParallelMultiheadAttention(RotatedLayer):
                     mask = F.pad(mask, (0, extra))
                 if key_bias is not None:
                     key_bias = F.pad(key_bias, (0, extra))
+            hides_only = all(m is None or m.dtype == torch.bool for m in (attn_mask, key_padding_mask))
             out, weights = _GeneralAttentionFn.apply(x, k_in, v_in, self._anchor, self, mask, key_bias,
-                                                     bool(need_weights), drop_p)
+                                                     bool(need_weights), drop_p, hides_only)
         else:
             out, weights = _AttentionFn.apply(x, self._anchor, self, mask, causal, bool(need_weights),
                                               bool(residual_grad), key_bias, drop_p)

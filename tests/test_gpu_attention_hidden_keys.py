@@ -1,4 +1,5 @@
-"""bf16 attention for queries that see no key, keys and values of another sequence: NaN, as nn.MultiheadAttention gives."""
+"""bf16 attention for queries that see no key: hidden by boolean masks (NaN, as nn.MultiheadAttention gives) or pushed down by
+large finite ones (which cancel in the softmax), keys and values of another sequence, against nn.MultiheadAttention in fp32."""
 import pytest
 import torch
 import torch.nn as nn
@@ -45,3 +46,20 @@ def test_boolean_masks_that_hide_every_key_give_nan(L, S):
     assert got[0][L - 1].isnan().all() and got[1][L - 1].isnan().all() and got[2].isnan().all() and want[2].isnan().all()
     for a, b in zip(got[:2], want[:2]):
         assert rel_err(a[:L - 1], b[:L - 1]) <= TOL[DT]
+
+
+@pytest.mark.parametrize("low", [-1e4, -1e9, -1e12, torch.finfo(torch.float32).min])
+def test_large_finite_masks_cancel(low):
+    layer, ref = _pair(128, 4, 2)
+    L, S, N = 40, 70, 3
+    bias = torch.zeros(N, S)
+    bias[1] = low
+    bias[2, S // 2:] = low
+    got, want = _run(layer, ref, L, S, N, 128, key_padding_mask=bias)
+    for a, b in zip(got, want):
+        assert rel_err(a, b) <= TOL[DT]
+    mask = torch.randn(L, S, generator=torch.Generator().manual_seed(1))
+    mask[7] = low
+    got, want = _run(layer, ref, L, S, N, 128, attn_mask=mask)
+    for a, b in zip(got, want):
+        assert rel_err(a, b) <= TOL[DT]

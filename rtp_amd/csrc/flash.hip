@@ -310,8 +310,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_wav
   landed(qf);
   int lrow = B::lane_rows(lane), lcol = B::lane_cols(lane);
   const float c = ADD ? kLog2e : a.scale * kLog2e;
-  // The running maximum (log2 domain) follows the true one: the largest P of a query is then 1, which bf16 holds exactly (with
-  // a maximum that may lag behind by 2^8 and fewer rescales, peaked rows lost up to 1 % of the result's accuracy).
+  // The running maximum follows the true one: the largest P of a query is then 1, which bf16 holds exactly (with a maximum
+  // that may lag behind by 2^8 and fewer rescales, peaked rows lost up to 1 % of the result's accuracy).  It is kept in the
+  // log2 domain, or with ADD in the scores' own and subtracted before the factor: a mask may lower all keys by 1e9 or more,
+  // where the rounding of maximum * log2(e) alone is 2^64.  A score below -FLT_MAX / log2(e) is a hidden key's.
+  const float c_max = ADD ? 1.0f : c;
   float m_run = -INFINITY, l_run = 0.0f;
   f32x16 acc[DB];
 #pragma unroll
@@ -367,10 +370,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_wav
       for (int r = 0; r < 16; ++r) bm = fmaxf(bm, val[h][r]);
     float lo, hi;
     halves(bm, lo, hi);
-    bm = fmaxf(lo, hi) * c;
+    bm = fmaxf(lo, hi) * c_max;
     if (__any(bm > m_run)) {
       const float m_new = fmaxf(m_run, bm);
-      const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.0f : m_new));
+      const float alpha = __builtin_amdgcn_exp2f((m_run - (m_new == -INFINITY ? 0.0f : m_new)) * (ADD ? c : 1.0f));
       m_run = m_new;
       l_run *= alpha;
 #pragma unroll
@@ -378,14 +381,15 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_wav
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
     }
-    const float m_ref = m_run == -INFINITY ? 0.0f : m_run;  // everything hidden so far: 2^(-inf - 0) = 0 all round
+    // everything hidden so far: 2^(-inf - 0) = 0 all round
+    const float m_ref = (ADD ? m_run * c : m_run) == -INFINITY ? 0.0f : m_run;
     float rs[2] = {0.0f, 0.0f};
     Frag pf[H][NM];
 #pragma unroll
     for (int h = 0; h < H; ++h) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        val[h][r] = __builtin_amdgcn_exp2f(fmaf(val[h][r], c, -m_ref));
+        val[h][r] = __builtin_amdgcn_exp2f(ADD ? (val[h][r] - m_ref) * c : fmaf(val[h][r], c, -m_ref));
         rs[r & 1] += val[h][r];
       }
       pack<T>(val[h], pf[h]);
@@ -420,7 +424,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_wav
     char* row = a.out + it.o + (long)query * a.o_l;
 #pragma unroll
     for (int db = 0; db < DB; ++db) store_acc<T>(row, db, g, acc[db], inv);
-    if (g == 0) a.lse[(long)it.z * a.L + query] = l > 0.0f ? (m_run + __builtin_amdgcn_logf(l)) * kLn2 : a.empty;
+    const float log2l = __builtin_amdgcn_logf(l);
+    if (g == 0) a.lse[(long)it.z * a.L + query] = !(l > 0.0f) ? a.empty : ADD ? fmaf(log2l, kLn2, m_run) : (m_run + log2l) * kLn2;
   }
 }
 
@@ -732,7 +737,8 @@ static int flash_forward(void* stream, int dtype, const void* q, const int64_t (
   RTP_REQUIRE(((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)o) % 16 == 0,
               "rtp_attn_flash_fwd: q, k, v, o must be 16-byte aligned");
   FlashArgs a{};
-  if (int rc = flash_args("rtp_attn_flash_fwd", a, dtype, qs, ks, os, mask, key_bias, causal, scale, L, S, N, H, D, G)) return rc;
+  if (int rc = flash_args("rtp_attn_flash_fwd", a, dtype, qs, ks, os, mask, key_bias, causal, scale, L, S, N, H, D, G))
+    return rc;
   a.q = (const char*)q, a.k = (const char*)k, a.v = (const char*)v, a.out = (char*)o, a.lse = lse, a.empty = empty;
   hipStream_t st = (hipStream_t)stream;
   const double np = (double)a.nprob, vis = causal ? 0.5 : 1.0, esz = 2.0;

@@ -1,5 +1,6 @@
 """bf16 attention for queries that see no key: hidden by boolean masks (NaN, as nn.MultiheadAttention gives) or pushed down by
-large finite ones (which cancel in the softmax), keys and values of another sequence, against nn.MultiheadAttention in fp32."""
+large finite ones (which cancel in the softmax), over keys of another sequence and, in the forward pass, its own, against
+nn.MultiheadAttention in fp32."""
 import pytest
 import torch
 import torch.nn as nn
@@ -63,3 +64,22 @@ def test_large_finite_masks_cancel(low):
     got, want = _run(layer, ref, L, S, N, 128, attn_mask=mask)
     for a, b in zip(got, want):
         assert rel_err(a, b) <= TOL[DT]
+
+
+@pytest.mark.parametrize("low", [-1e4, -1e9, -1e10, -1e12])
+def test_large_finite_masks_cancel_in_the_packed_forward(low):
+    """Self-attention, running softmax: the maximum is subtracted before the change of base."""
+    layer, ref = _pair(128, 4, 2)
+    L, N = 70, 3
+    x = torch.randn(L, N, 128, generator=torch.Generator().manual_seed(3)).to(DT)
+    bias = torch.zeros(N, L)
+    bias[1] = low
+    bias[2, L // 2:] = low
+    mask = torch.randn(L, L, generator=torch.Generator().manual_seed(1))
+    mask[7] = low
+    for masks in ({"key_padding_mask": bias}, {"attn_mask": mask}):
+        with torch.no_grad():
+            xd = x.to(DEV)
+            out, _ = layer(xd, xd, xd, need_weights=False, **{n: m.to(DEV) for n, m in masks.items()})
+            want, _ = ref(x.float(), x.float(), x.float(), need_weights=True, **masks)
+        assert rel_err(out, want) <= TOL[DT], list(masks)

@@ -2234,14 +2234,18 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   }
   // Tile choice by a cost model: the launch runs in ceil(tiles / 256 CUs) rounds, a round costs the tile's
   // measured time per K slab (ns, 4096^3 bf16 on MI355X: bigger tiles do ~30 % more outputs per ns, so what
-  // decides is mostly how evenly the tile count fills the CUs) plus a fixed prologue / epilogue.
+  // decides is mostly how evenly the tile count fills the CUs) plus a fixed prologue / epilogue.  Only the ratios of
+  // the prices matter: with every CU busy on operands from memory all shapes take 1.2 - 1.4 times theirs.
   static const int forced = [] {
     const char* e = getenv("RTP_GEMM_TILE");  // debugging aid: index into kShapes
     return e ? atoi(e) : -1;
   }();
-  static const double slab_ns[kNumShapes] = {966.0, 470.0, 283.0, 167.0, 800.0, 1400.0, 545.0};
-  // per tile outside the K loop; 256 x 256: 128 KiB of output per CU are 6 us at the memory's rate
-  static const double fixed_ns[kNumShapes] = {3000.0, 3000.0, 3000.0, 3000.0, 3000.0, 9000.0, 3000.0};
+  static const double slab_ns[kNumShapes] = {966.0, 470.0, 283.0, 167.0, 800.0, 1350.0, 545.0};
+  // Per tile outside the K loop.  256 x 256 is priced by its ratio to the others with every CU busy: measured there over 117
+  // products x 3 layouts at 1510 ns a slab and 13 us a tile, against 1040 ns and 8.5 us for 256 x 128, 540 ns and 5.4 us for 128 x 128.
+  // With these two numbers it is taken on none of them where another shape is more than 1 % faster, and on 25 more than with
+  // 1400 and 9000 ns: 4096 x 6144 x 2048 121 -> 113 us, 8192 x 8192 x 256 98 -> 80, 8 of 3072 x 1024 x 768 72 -> 59.
+  static const double fixed_ns[kNumShapes] = {3000.0, 3000.0, 3000.0, 3000.0, 3000.0, 5000.0, 3000.0};
   static const int slab_bytes[kNumShapes] = {128, 128, 128, 128, 128, 128, 128};
   const bool vec = direct && a.vec_c;  // else the kernels for operands of any alignment
   int shape = 3;  // 64 x 64 unless the model finds something cheaper

@@ -155,8 +155,9 @@ int rtp_rotated_linear_xent_bwd(void* stream, int dtype, const rtp_rotated_linea
  * whole contraction of A(m, k), in fp32 with a fixed order, stored as `dtype` (added to the existing value
  * with RTP_GEMM_ROWSUM_ACCUM).  In the weight-gradient product dW = dY^T X the operand A is dY^T, so this
  * is nn.Linear's bias gradient (reference: autograd of rtp/module/linear.py:216) without a second pass
- * over dY.  Only for descriptors rtp_gemm_rowsum_fused() accepts (A stored K x M, batch == 1, and the
- * alignment the wave-specialised kernel needs); rtp_gemm rejects others, callers use rtp_colsum there.
+ * over dY.  Only for descriptors rtp_gemm_rowsum_fused() accepts (A stored K x M, batch == 1, 16 bytes or more along
+ * either operand's contiguous axis at any alignment, a product beyond 64 x 64 x 256); rtp_gemm rejects others, callers
+ * use rtp_colsum there.
  * --------------------------------------------------------------------------------------------- */
 enum {
   RTP_GEMM_OUT_F32 = 1,

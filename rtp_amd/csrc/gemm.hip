@@ -2194,7 +2194,8 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
     a.vec_c = a.vec_c && mult((int64_t)(uintptr_t)d->sgd_master, 16) &&
               (!d->sgd_weights || mult((int64_t)(uintptr_t)d->sgd_weights, 16));
   RTP_REQUIRE(!d->a_rowsum || rowsum_fused<T>(d),
-              "rtp_gemm: a_rowsum needs A stored K x M, batch == 1 and vector-aligned operands (rtp_gemm_rowsum_fused)");
+              "rtp_gemm: a_rowsum needs A stored K x M, batch == 1, 16 bytes or more along either operand's contiguous axis and a product "
+              "beyond 64 x 64 x 256 (rtp_gemm_rowsum_fused)");
   if (is_tiny(d)) {
     // one wavefront per 32 x 32 block
     a.tiles_m = (int)ceil_div(d->m, 32);
@@ -2219,8 +2220,9 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
     RTP_LAUNCH_CHECK();
     return RTP_OK;
   }
-  // few fp32 weight-gradient tiles, long contraction: see gemm_ksplit_kernel.  At 64 tiles of 64 x 64 it is ahead (512 x 512 x 512
-  // 13 -> 9 us), at 128 behind (512 x 1024 x 2048 38 -> 46 us: every CU has work in both, and this one reads more).
+  // few fp32 weight-gradient tiles, long contraction: see gemm_ksplit_kernel.  64 tiles of 64 x 64 are 256 of its workgroups, one
+  // a CU, and it is ahead (512 x 512: K = 512 12.8 -> 9.2 us, K = 2880 49 -> 33); from 65 on some CU has two and it is behind, with
+  // 72 as with 128 tiles (512 x 576: 12.7 against 14.6 and 49 against 56; 512 x 1024: 13.0 against 15.1 and 49 against 58).
   if (sizeof(T) == 4 && fast && !akc && !bkc && !d->sgd_master && !d->xent_mode && d->k >= 512 && nz < 65536 &&
       ceil_div(d->m, 64) * ceil_div(d->n, 64) * nz <= 64) {
     a.tiles_m = (int)ceil_div(d->m, 32);

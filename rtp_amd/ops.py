@@ -305,8 +305,15 @@ def embedding_backward_supported(n_ids: int) -> bool:
 
 
 # The one-launch form stages all ids in every token's workgroup, n^2 words of LDS traffic, and sums a frequent id's rows one at
-# a time; the grouped form costs a second launch.  bf16, 10240 x 2048 table, one / grouped, us: 256 ids 10 / 17; 1024 ids
-# 14 / 25 uniform, 41 / 33 by word frequency; 2048 ids 21 / 25 and 79 / 37; 4096 ids 38 / 26 and 143 / 46.
+# a time; the grouped form costs a second launch.  One / grouped, us, uniform ids and ids by word frequency:
+#            10240 x 2048 bf16          10240 x 2048 fp32          1000 x 2048 bf16
+#   256 ids  12 / 23 and 13 / 24        16 / 20 and 16 / 26        8.5 / 13 and 11 / 19
+#   512      12 / 23 and 24 / 35        16 / 20 and 20 / 38        8.9 / 13 and 17 / 27
+#   768      13 / 24 and 23 / 36        17 / 21 and 21 / 40        9.0 / 13 and 28 / 27
+#   1024     14 / 25 and 35 / 37        20 / 22 and 25 / 48        9.1 / 13 and 38 / 25
+#   1536     18 / 25 and 60 / 33        23 / 22 and 41 / 39        9.8 / 13 and 48 / 28
+#   2048     21 / 25 and 68 / 39        26 / 22 and 48 / 46        11 / 13 and 65 / 33
+# Uniform ids cross beyond 1500 (fp32) or 2048 (bf16), frequent words between 700 and 1500: 1024 lies between.
 EMBEDDING_ONE_LAUNCH_IDS = 1024
 
 

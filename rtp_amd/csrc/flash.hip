@@ -68,20 +68,18 @@ struct Op<bf16_t> {
 
 // A block of ROWS x D elements in LDS, row after row, the 16-byte chunks of a row permuted by XOR with swz(row) so that
 // both ways of reading it spread over all banks: 16 lanes on the same chunk of 16 consecutive rows (row-major fragments),
-// and rows r .. r+3 (bf16, transposing read of 4 x 16 blocks) or r and r+4 (fp32) side by side.  swz is linear over
-// XOR of disjoint row bits, which lets the constant part of an address be folded in with one XOR.
+// and rows r .. r+3 (transposing read of 4 x 16 blocks) side by side.  swz is linear over XOR of disjoint row bits, which
+// lets the constant part of an address be folded in with one XOR.
 template <typename T, int D, int NW>
 struct Block {
   static constexpr int ROWS = Op<T>::ROWS, PITCH = D * (int)sizeof(T), CPR = PITCH / 16, BYTES = ROWS * PITCH;
   static constexpr int NI = BYTES / 1024 / NW;  // 1 KiB loads per wave
   static_assert(NI * NW * 1024 == BYTES, "whole loads");
+  static_assert(sizeof(T) == 2, "the transposing read is for 16-bit elements");
   typedef typename Op<T>::Frag Frag;
 
   static __host__ __device__ constexpr int swz(int row) {
-    return sizeof(T) == 2 ? (CPR == 16  ? ((row & 3) << 2) | ((row >> 2) & 3)
-                             : CPR == 8 ? (((row >> 1) & 1) << 2) | ((row >> 2) & 3)
-                                        : (row >> 2) & 3)
-                          : (CPR >= 16 ? (row & 3) | (((row >> 2) & 1) << 3) | (((row >> 3) & 1) << 2) : (row >> 1) & 7);
+    return CPR == 16 ? ((row & 3) << 2) | ((row >> 2) & 3) : CPR == 8 ? (((row >> 1) & 1) << 2) | ((row >> 2) & 3) : (row >> 2) & 3;
   }
 
   unsigned ofs[NI];  // of the lane's chunk inside a block, per load
@@ -116,12 +114,9 @@ struct Block {
     return li * PITCH + ((g ^ swz(li)) << 4);
   }
   static __device__ __forceinline__ int lane_cols(int lane) {
-    const int li = lane & 31, g = lane >> 5, t = lane & 15;
-    if (sizeof(T) == 2) {
-      const int row = 4 * g + (t >> 2), chunk = 2 * ((lane >> 4) & 1) + ((t & 3) >> 1);
-      return row * PITCH + ((chunk ^ swz(row)) << 4) + (t & 1) * 8;
-    }
-    return 4 * g * PITCH + (((li >> 2) ^ swz(4 * g)) << 4) + (li & 3) * 4;
+    const int g = lane >> 5, t = lane & 15;
+    const int row = 4 * g + (t >> 2), chunk = 2 * ((lane >> 4) & 1) + ((t & 3) >> 1);
+    return row * PITCH + ((chunk ^ swz(row)) << 4) + (t & 1) * 8;
   }
   static __device__ __forceinline__ int at(int lane_part, int row, int chunk) {
     return (lane_part ^ ((chunk ^ swz(row)) << 4)) + row * PITCH;
@@ -132,23 +127,15 @@ struct Block {
   }
   // accumulator-order fragment m of row group h, columns 32*db ...
   static __device__ __forceinline__ Frag cols(const char* blk, int lane_part, int h, int m, int db) {
-    if constexpr (sizeof(T) == 2) {
-      typedef __attribute__((address_space(3))) s16x4* lds_ptr;
-      union {
-        s16x4 h2[2];
-        Frag f;
-      } u;
-#pragma unroll
-      for (int x = 0; x < 2; ++x)
-        u.h2[x] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(blk + at(lane_part, 32 * h + 16 * m + 8 * x, 4 * db)));
-      return u.f;
-    } else {
+    typedef __attribute__((address_space(3))) s16x4* lds_ptr;
+    union {
+      s16x4 h2[2];
       Frag f;
+    } u;
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        f[e] = *reinterpret_cast<const float*>(blk + at(lane_part, 32 * h + 8 * m + e, 8 * db));
-      return f;
-    }
+    for (int x = 0; x < 2; ++x)
+      u.h2[x] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(blk + at(lane_part, 32 * h + 16 * m + 8 * x, 4 * db)));
+    return u.f;
   }
 };
 
@@ -190,10 +177,7 @@ __device__ __forceinline__ void store_acc(char* row, int db, int g, const f32x16
 #pragma unroll
     for (int i = 0; i < 4; ++i) e[i] = from_f32<T>(acc[4 * a4 + i] * scale);
     char* dst = row + (32 * db + 8 * a4 + 4 * g) * (int)sizeof(T);
-    if constexpr (sizeof(T) == 2)
-      *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<const uint2*>(e);
-    else
-      *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(e);
+    *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<const uint2*>(e);
   }
 }
 

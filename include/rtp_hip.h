@@ -224,8 +224,12 @@ int rtp_gemm(void* stream, int dtype, const rtp_gemm_desc* d);
  * (weights are read once per pass and would otherwise come from HBM at their turn).  Up to 192 KiB per workgroup
  * of the carrying launch.  A hint: no result depends on it; it ends with that next product launch whether or not
  * the launch could carry it (other kernels than the wave-specialised one cannot).  The carrying kernel reads `src` when
- * it RUNS, not when it is launched: `src` has to stay mapped until that launch has completed on its stream.  bytes == 0 withdraws a pending hint. */
+ * it RUNS, not when it is launched: `src` has to stay mapped until that launch has completed on its stream.  bytes == 0
+ * withdraws a pending hint.  One hint is pending in a process: a call ends the hint of any other thread too, so the
+ * caller need only keep the last `src`.
+ *   rtp_gemm_warm_pending: 1 if the calling thread's next product would carry a hint, else 0. */
 int rtp_gemm_warm_next(const void* src, size_t bytes);
+int rtp_gemm_warm_pending(void);
 
 /* Measurement aid (no counterpart in the reference; bench.py reports it beside the published peak): TFLOP/s of a
  * register-only loop of v_mfma_f32_32x32x16_bf16 on every SIMD of the device, `iters` iterations of 32 MFMAs per

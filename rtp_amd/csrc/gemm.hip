@@ -15,6 +15,7 @@
 // ring of register buffers, which is what hides HBM/L2 latency when only one workgroup fits a CU.
 #include "common.h"
 
+#include <atomic>
 #include <cstdlib>
 #include <type_traits>
 
@@ -2105,14 +2106,21 @@ static bool rowsum_fused(const rtp_gemm_desc* d) {
   return !d->a_kcontig && d->batch == 1 && !is_tiny(d) && (takes_dma_kernel<T>(d) || takes_reg_kernel<T>(d));
 }
 
-// rtp_gemm_warm_next: bytes the next product launched by this host thread requests at its start
+// rtp_gemm_warm_next: bytes the next product launched by this host thread requests at its start.  A later call, from any
+// thread, ends an earlier hint: a caller holds the memory of the last one only, and a forward pass and its backward pass
+// run on two threads.
+static std::atomic<unsigned long long> g_warm_call{0};
 static thread_local const void* t_warm_src = nullptr;
 static thread_local size_t t_warm_bytes = 0;
+static thread_local unsigned long long t_warm_call = 0;
+static const void* warm_source() {
+  return t_warm_src && t_warm_call == g_warm_call.load(std::memory_order_relaxed) ? t_warm_src : nullptr;
+}
 
 template <typename T>
 static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   // the hint of rtp_gemm_warm_next rides in this launch or ends with it
-  const void* warm_src = t_warm_src;
+  const void* warm_src = warm_source();
   t_warm_src = nullptr;
   constexpr int VEC = 16 / sizeof(T);
   GemmArgs a;
@@ -2555,8 +2563,11 @@ extern "C" int rtp_gemm_warm_next(const void* src, size_t bytes) {
   RTP_REQUIRE(((uintptr_t)src & 15) == 0, "rtp_gemm_warm_next: source must be 16-byte aligned");
   rtp::t_warm_src = bytes ? src : nullptr;
   rtp::t_warm_bytes = bytes;
+  rtp::t_warm_call = ++rtp::g_warm_call;
   return RTP_OK;
 }
+
+extern "C" int rtp_gemm_warm_pending(void) { return rtp::warm_source() != nullptr; }
 
 extern "C" int rtp_gemm_sgd_fused(int dtype, const rtp_gemm_desc* d) {
   using namespace rtp;

@@ -91,7 +91,8 @@ def warm_ahead() -> bool:
 def _warm_step(home: torch.Tensor) -> None:
     """A rotation over `home` starts (direct mode).  The table holds weak references, so it keeps no model alive; the
     one tensor a pending hint points into is held until the next rotation replaces or withdraws the hint (the
-    library drops a hint with the first product launched after it, carried or not)."""
+    library drops a hint with the first product launched after it, carried or not, and with any later call of
+    rtp_gemm_warm_next, also one of another thread: a backward pass rotates on the autograd engine's)."""
     idx = home.device.index if home.device.index is not None else torch.cuda.current_device()
     prev, cur = _warm_hist.get(idx, (0, 0))
     here = home.data_ptr()

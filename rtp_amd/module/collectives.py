@@ -296,7 +296,7 @@ class RotatedLayer(nn.Module):
             return
         book.drop()
         for m in self._modules.values():
-            if m is not self.shards and m not in self._store.modules:
+            if m is not None and m is not self.shards and m not in self._store.modules:
                 m.zero_grad()
 
     def set_full_param(self, device=None, dtype=None):

@@ -73,3 +73,11 @@ def test_gradients_put_on_a_copy_are_accumulated_into():
         p.grad = torch.full_like(p, 2.0)
     assert other._store.grad_runs() == [(0, 4, True)]
     assert all(v.eq(2.0).all() for s in range(4) for v in other._store.views(other._store.grads[s]))
+
+
+def test_zero_grad_with_an_empty_child_slot():
+    layer = _column()
+    layer._store.grad_runs()
+    layer.register_module("extra", None)  # as torch modules may have
+    layer.zero_grad()
+    assert all(p.grad is None for p in layer.parameters())

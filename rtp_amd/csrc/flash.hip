@@ -18,8 +18,9 @@
 // wait for.  Shared blocks need a quarter of that and their latency is hidden; the loop is then bound by LDS
 // reads, MFMA and the softmax's vector instructions in equal parts (about 1000 clocks each for a wave's 32 x 64 scores at
 // D = 128, bf16), which two or more waves per SIMD overlap.
-// Measured (one wave per tile -> this; forward, backward): 64 heads of 1500 x 128 in bf16 261 -> 107 us (690 TFLOP/s), 636 ->
-// 316 us; 256 causal heads of 512 x 64 28 -> 20 us, 78 -> 68 us; with a [512, 512] mask, D = 32, 44 -> 41 us, 116 -> 92 us.
+// Measured (one wave per tile -> this; forward, backward): 64 heads of 1500 x 128 in bf16 261 -> 113 us (650 TFLOP/s), with a key
+// bias 117, 636 -> 340 us; 256 causal heads of 512 x 64 28 -> 21 us, 78 -> 70 us; with a [512, 512] mask, D = 32, 44 us both
+// ways, 116 -> 93 us.
 #include "common.h"
 
 #include <type_traits>
@@ -214,9 +215,9 @@ __device__ __forceinline__ void issue_floats(unsigned dst, const float* src, int
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" : : "s"(dst), "v"(o), "s"(src) : "memory");
 }
 
-// mask[mine][base + 8*(r/4) + 4*g + r%4] (ROWS_IN_REGS false: the transposed entry), clamped into the matrix
+// factor * mask[mine][base + 8*(r/4) + 4*g + r%4] (KEYS_IN_REGS false: the transposed entry), clamped into the matrix
 template <bool KEYS_IN_REGS>
-__device__ __forceinline__ void add_mask(const FlashArgs& a, int mine, int base, int g, float (&v)[16]) {
+__device__ __forceinline__ void add_mask(const FlashArgs& a, int mine, int base, int g, float factor, float (&v)[16]) {
   if (!a.mask) return;
   const int own = min(mine, (KEYS_IN_REGS ? a.L : a.S) - 1), last = (KEYS_IN_REGS ? a.S : a.L) - 1;
   if (KEYS_IN_REGS && a.S % 4 == 0 && reinterpret_cast<uintptr_t>(a.mask) % 16 == 0) {
@@ -224,13 +225,13 @@ __device__ __forceinline__ void add_mask(const FlashArgs& a, int mine, int base,
     for (int a4 = 0; a4 < 4; ++a4) {
       const f32x4 m = *reinterpret_cast<const f32x4*>(a.mask + (long)own * a.S + min(base + 8 * a4 + 4 * g, last - 3));
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[4 * a4 + e] += m[e];
+      for (int e = 0; e < 4; ++e) v[4 * a4 + e] = fmaf(m[e], factor, v[4 * a4 + e]);
     }
   } else {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int other = min(base + 8 * (r >> 2) + 4 * g + (r & 3), last);
-      v[r] += a.mask[KEYS_IN_REGS ? (long)own * a.S + other : (long)other * a.S + own];
+      v[r] = fmaf(a.mask[KEYS_IN_REGS ? (long)own * a.S + other : (long)other * a.S + own], factor, v[r]);
     }
   }
 }
@@ -259,7 +260,10 @@ constexpr int dkv_waves() {
   return D == 128 ? 1 : D == 64 ? 2 : 3;
 }
 
-// ADD: something joins the scaled scores (a mask, a key bias), or the scale is not positive and their order turns round.
+// ADD: something joins the scaled scores (a mask, a key bias), or the scale is not positive and their order turns round: scores
+// are brought to the log2 domain first and their maximum is subtracted there, exactly: a mask may lower all keys of a query by
+// 1e9 or more, where a maximum rounded after the change of base is off by 2^6 and the exponential by 2^(2^6).  The key bias
+// arrives in LDS already in that domain.  A score of less than -FLT_MAX / log2(e) is a hidden key's.
 // Otherwise scores stay raw and scale * log2(e) is applied inside the exponential's FMA.
 template <typename T, int D, int NW, bool ADD>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_waves<T, D, ADD>()))) void flash_fwd_kernel(
@@ -284,21 +288,24 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_wav
     const unsigned dst = lds0 + (kb & 1) * 2 * B::BYTES;
     blk.issue(dst, kp + kb * step, a.k_l, a.S - kb * ROWS, wave, lane);
     blk.issue(dst + B::BYTES, vp + kb * step, a.k_l, a.S - kb * ROWS, wave, lane);
-    if (kbias && wave == 0) issue_floats(lds0 + 4 * B::BYTES + (kb & 1) * 256, kbias, kb * ROWS, a.S, lane);
   };
   int nkb = (a.S + ROWS - 1) / ROWS;
   if (a.causal) nkb = min(nkb, (min(wg_q0 + 32 * NW, a.L) - 1) / ROWS + 1);
+  // wave 0 writes the key bias of a block into LDS a block ahead of its use and holds the one after that in a register
+  float* const bias_lds = reinterpret_cast<float*>(lds + 4 * B::BYTES);
+  const bool writes_bias = ADD && kbias && wave == 0;
+  auto bias_of = [&](int kb) { return kbias[min(kb * ROWS + lane, a.S - 1)]; };
+  const float bias_first = writes_bias ? bias_of(0) : 0.0f;
+  float bias_next = writes_bias ? bias_of(1) : 0.0f;
   issue(0);
   Frag qf[NK];
   load_rows<T>(a.q + it.q + min(query, a.L - 1) * a.q_l, g, qf);
   landed(qf);
+  if (writes_bias) bias_lds[lane] = bias_first * kLog2e;
   int lrow = B::lane_rows(lane), lcol = B::lane_cols(lane);
-  const float c = ADD ? kLog2e : a.scale * kLog2e;
-  // The running maximum follows the true one: the largest P of a query is then 1, which bf16 holds exactly (with a maximum
-  // that may lag behind by 2^8 and fewer rescales, peaked rows lost up to 1 % of the result's accuracy).  It is kept in the
-  // log2 domain, or with ADD in the scores' own and subtracted before the factor: a mask may lower all keys by 1e9 or more,
-  // where the rounding of maximum * log2(e) alone is 2^64.  A score below -FLT_MAX / log2(e) is a hidden key's.
-  const float c_max = ADD ? 1.0f : c;
+  const float c = a.scale * kLog2e;
+  // The running maximum (log2 domain) follows the true one: the largest P of a query is then 1, which bf16 holds exactly (with
+  // a maximum that may lag behind by 2^8 and fewer rescales, peaked rows lost up to 1 % of the result's accuracy).
   float m_run = -INFINITY, l_run = 0.0f;
   f32x16 acc[DB];
 #pragma unroll
@@ -316,11 +323,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_wav
 #pragma unroll
       for (int h = 0; h < H; ++h) {
         if (kbias)
-          lds_values(reinterpret_cast<const float*>(lds + 4 * B::BYTES) + (kb & 1) * 64 + 32 * h, g, add[h]);
+          lds_values(bias_lds + (kb & 1) * 64 + 32 * h, g, add[h]);
         else
 #pragma unroll
           for (int r = 0; r < 16; ++r) add[h][r] = 0.0f;
-        add_mask<true>(a, query, k0 + 32 * h, g, add[h]);
+        add_mask<true>(a, query, k0 + 32 * h, g, kLog2e, add[h]);
       }
     }
     f32x16 s[H];
@@ -336,7 +343,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_wav
 #pragma unroll
     for (int h = 0; h < H; ++h)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) val[h][r] = ADD ? fmaf(s[h][r], a.scale, add[ADD ? h : 0][r]) : s[h][r];
+      for (int r = 0; r < 16; ++r) val[h][r] = ADD ? fmaf(s[h][r], c, add[ADD ? h : 0][r]) : s[h][r];
     if (k0 + 32 * H > a.S || (a.causal && k0 + 32 * H - 1 > q0)) {  // wave-uniform: only these blocks hold hidden keys
 #pragma unroll
       for (int h = 0; h < H; ++h)
@@ -354,10 +361,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_wav
       for (int r = 0; r < 16; ++r) bm = fmaxf(bm, val[h][r]);
     float lo, hi;
     halves(bm, lo, hi);
-    bm = fmaxf(lo, hi) * c_max;
+    bm = ADD ? fmaxf(lo, hi) : fmaxf(lo, hi) * c;
     if (__any(bm > m_run)) {
       const float m_new = fmaxf(m_run, bm);
-      const float alpha = __builtin_amdgcn_exp2f((m_run - (m_new == -INFINITY ? 0.0f : m_new)) * (ADD ? c : 1.0f));
+      const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.0f : m_new));
       m_run = m_new;
       l_run *= alpha;
 #pragma unroll
@@ -365,15 +372,14 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_wav
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
     }
-    // everything hidden so far: 2^(-inf - 0) = 0 all round
-    const float m_ref = (ADD ? m_run * c : m_run) == -INFINITY ? 0.0f : m_run;
+    const float m_ref = m_run == -INFINITY ? 0.0f : m_run;  // everything hidden so far: 2^(-inf - 0) = 0 all round
     float rs[2] = {0.0f, 0.0f};
     Frag pf[H][NM];
 #pragma unroll
     for (int h = 0; h < H; ++h) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        val[h][r] = __builtin_amdgcn_exp2f(ADD ? (val[h][r] - m_ref) * c : fmaf(val[h][r], c, -m_ref));
+        val[h][r] = __builtin_amdgcn_exp2f(ADD ? val[h][r] - m_ref : fmaf(val[h][r], c, -m_ref));
         rs[r & 1] += val[h][r];
       }
       pack<T>(val[h], pf[h]);
@@ -390,6 +396,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_wav
   for (int kb = 0; kb < nkb; ++kb) {
     block_barrier();  // block kb is there, and every wave has left block kb - 1
     keep_in_loop(lrow, lcol);
+    if (writes_bias && kb + 1 < nkb) {
+      asm volatile("" : "+v"(bias_next));  // it landed with the barrier: waited for here, before the next block's loads
+      bias_lds[((kb + 1) & 1) * 64 + lane] = bias_next * kLog2e;
+      bias_next = bias_of(kb + 2);
+    }
     if (kb + 1 < nkb) issue(kb + 1);
     const int k0 = kb * ROWS;
     int keys = a.S - k0;
@@ -408,8 +419,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_wav
     char* row = a.out + it.o + (long)query * a.o_l;
 #pragma unroll
     for (int db = 0; db < DB; ++db) store_acc<T>(row, db, g, acc[db], inv);
-    const float log2l = __builtin_amdgcn_logf(l);
-    if (g == 0) a.lse[(long)it.z * a.L + query] = !(l > 0.0f) ? a.empty : ADD ? fmaf(log2l, kLn2, m_run) : (m_run + log2l) * kLn2;
+    if (g == 0) a.lse[(long)it.z * a.L + query] = l > 0.0f ? (m_run + __builtin_amdgcn_logf(l)) * kLn2 : a.empty;
   }
 }
 
@@ -507,7 +517,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dq_wave
 #pragma unroll
         for (int r = 0; r < 16; ++r) off[r] += kb16[r];
       }
-      add_mask<true>(a, query, k0, g, off);
+      add_mask<true>(a, query, k0, g, 1.0f, off);
       f32x16 s, dp;
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.0f;
@@ -605,7 +615,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dkv_wav
       lds_values(stat + 64 + 32 * h, g, delta);
 #pragma unroll
       for (int r = 0; r < 16; ++r) off[r] = kb - off[r];
-      add_mask<false>(a, key, q0, g, off);
+      add_mask<false>(a, key, q0, g, 1.0f, off);
       const bool edge = q0 + 32 > a.L || (a.causal && k0 + 31 > q0);
       p_and_ds<false>(a, s, dp, off, delta, key, q0, g, edge, p, ds);
       Frag pf[NM], df[NM];

@@ -378,7 +378,8 @@ int rtp_embedding_scatter_add_sgd(void* stream, int dtype, const void* grad_out,
  * zero_fill the rows that no token names are cleared by further workgroups of the same launch.  master == NULL: the
  * gradient is written (zero_fill != 0: overwriting, else added to what is there); master != NULL: the update of
  * rtp_embedding_scatter_add_sgd (weights may be NULL; store_grad as there).  At most 4096 ids
- * (rtp_embedding_backward_supported); longer steps take rtp_embedding_backward_grouped. */
+ * (rtp_embedding_backward_supported); longer steps take rtp_embedding_backward_grouped, which is faster from about 1024
+ * ids of running text on (where the Python layer changes over) and from 2048 uniform ones. */
 int rtp_embedding_backward_supported(int64_t n_ids);
 int rtp_embedding_backward(void* stream, int dtype, const void* grad_out, int64_t ld_grad_out, int64_t n_ids,
                            const int64_t* ids, void* grad_table, int64_t ld_grad_table, int grad_table_f32,

@@ -76,6 +76,7 @@ class ShardStore:
         self.home: Optional[torch.Tensor] = None
         self.grads: Optional[torch.Tensor] = None
         self.one_run = None                          # ring.OneRun over home
+        self.captured_hints = {}                     # address -> rows of other layers that captured launches read (ring.rotation)
         self._params: List[List[nn.Parameter]] = []  # of every shard, as packed
         self._book = None                            # native.GradBook over _params and the slices of `grads`
         self._overwrite = set()
@@ -119,7 +120,7 @@ class ShardStore:
 
     # what follows from `home`, `grads` and the shard modules: not part of a copied or saved store (the book is an object
     # of the extension module, which neither copies nor pickles), made again when the copy is
-    _DERIVED = ("one_run", "_params", "_book", "_grad_rows", "_grad_slices")
+    _DERIVED = ("one_run", "captured_hints", "_params", "_book", "_grad_rows", "_grad_slices")
 
     def __getstate__(self):
         return {k: v for k, v in self.__dict__.items() if k not in self._DERIVED}
@@ -129,7 +130,7 @@ class ShardStore:
         home rows again, as pack() left them (torch.save / torch.load kept that by itself)."""
         from .. import ring
         self.__dict__.update(state)
-        self.one_run = ring.OneRun(self.home)
+        self.one_run, self.captured_hints = ring.OneRun(self.home), {}
         self._params = [list(m.parameters()) for m in self.modules]
         self._book, self._grad_rows, self._grad_slices = None, [], []
         for s, m in enumerate(self.modules):

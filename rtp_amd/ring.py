@@ -88,16 +88,17 @@ def warm_ahead() -> bool:
     return _warm_ahead
 
 
-def _warm_step(home: torch.Tensor) -> None:
+def _warm_step(home: torch.Tensor) -> Optional[torch.Tensor]:
     """A rotation over `home` starts (direct mode).  The table holds weak references, so it keeps no model alive; the
     one tensor a pending hint points into is held until the next rotation replaces or withdraws the hint (the
     library drops a hint with the first product launched after it, carried or not, and with any later call of
-    rtp_gemm_warm_next, also one of another thread: a backward pass rotates on the autograd engine's)."""
+    rtp_gemm_warm_next, also one of another thread: a backward pass rotates on the autograd engine's).  Returns the
+    tensor the hint points into, if it sets one."""
     idx = home.device.index if home.device.index is not None else torch.cuda.current_device()
     prev, cur = _warm_hist.get(idx, (0, 0))
     here = home.data_ptr()
     if here == cur:
-        return  # the same layer again (its backward pass right after its forward pass)
+        return None  # the same layer again (its backward pass right after its forward pass)
     seen = _warm_next.get((idx, prev, cur))
     if seen is None or seen() is not home:
         if len(_warm_next) > 4096:
@@ -109,9 +110,11 @@ def _warm_step(home: torch.Tensor) -> None:
     if nxt is not None and nxt.is_cuda and nxt.data_ptr() != here:
         _warm_pending[idx] = nxt
         _lib.native().rtp_gemm_warm_next(nxt, nxt.numel() * nxt.element_size())
-    elif _warm_pending.get(idx) is not None:
+        return nxt
+    if _warm_pending.get(idx) is not None:
         _warm_pending[idx] = None
         _lib.native().rtp_gemm_warm_next(None, 0)
+    return None
 
 
 # ---- weight gradients on a second stream -----------------------------------------------------------
@@ -435,9 +438,10 @@ class Rotation:
             self.windows.append(runs)
         self.steps = len(self.windows)
         self.direct = _mode == "direct"
+        self.hinted = None  # the tensor this rotation's warm-ahead hint points into
         if self.direct:
             if _warm_ahead:
-                _warm_step(home)
+                self.hinted = _warm_step(home)
             return
         self.ring = device_ring(home.device)
         self.lib = _lib.load()
@@ -519,10 +523,15 @@ def rotation(store, rank: int, reverse: bool = False):
     """One pass over the shards of a layer's store (ShardStore) in ring order."""
     home = store.home
     if _mode == "direct" and (_window is None or _window >= home.shape[0]):
-        if _warm_ahead:
-            _warm_step(home)
-        return store.one_run
-    return Rotation(home, ring_order(rank, home.shape[0], reverse), group=store.stage_group)
+        rot, hinted = store.one_run, _warm_step(home) if _warm_ahead else None
+    else:
+        rot = Rotation(home, ring_order(rank, home.shape[0], reverse), group=store.stage_group)
+        hinted = rot.hinted
+    if hinted is not None and torch.cuda.is_current_stream_capturing():
+        # The recorded launch reads these rows at every replay, and they may be another model's (one that ran between this
+        # one's passes): the layer whose graph it is holds them.
+        store.captured_hints[hinted.data_ptr()] = hinted
+    return rot
 
 
 def ring_order(rank: int, world_size: int, reverse: bool = False) -> List[int]:

@@ -346,8 +346,13 @@ __global__ __launch_bounds__(256) void embedding_bwd_kernel(const T* grad_out, l
 //
 // Words of running text are what makes this worth its launches: with ids by word frequency one of 16368 positions in nine
 // is the same row, and the sum over that row's positions is a serial chain that only columns can share.  The sorted
-// path (radix sort, one workgroup per segment and shard, one row in flight) took 533 us there, this takes 83 (uniform ids: 122 against 37).
-constexpr int kLongRow = 64;             // positions from which a row is dealt over workgroups by columns
+// path (radix sort, one workgroup per segment and shard, one row in flight) took 533 us there, this takes 48 (uniform ids: 122
+// against 34): 12 us the grouping, 35 the chain of the most frequent row, 36 clocks a position.
+//
+// kLongRow: with 64 (two rows of a short row's wavefront in flight) 2000 ids by word frequency over 5000 x 1024 took 29 us, with 32
+// (four) 20.  kRankRow: 65536 uniform ids over 1000 x 512, rows of 65, 136 us by windows and 53 by counting.
+constexpr int kLongRow = 32;             // positions from which a row is dealt over workgroups by columns
+constexpr int kRankRow = 512;            // positions up to which such a row's are ordered by counting
 constexpr int kGroupSlices = 32;         // workgroups of the grouping pass, at least
 constexpr int kGroupRowsMax = 8192;      // table rows per slice, at most (LDS counters)
 constexpr int kGroupMaxIds = 1 << 18;    // a long row's bitmap of positions in LDS: 32 KiB
@@ -466,6 +471,7 @@ struct GroupedBwd {
   int n, row_count, groups, cols;
   const int *offs, *pos, *nlong, *longs;
   int slices, long_cap;
+  int plain;  // the upstream gradient lies within 2 GiB of its start and is not scaled
 
   // one upstream value as it joins the sum
   __device__ __forceinline__ float take(T g) const {
@@ -501,98 +507,149 @@ struct GroupedBwd {
   }
 };
 
-// Sums the upstream rows of list[0 .. cnt) (ascending positions: list[k] + at) for the columns at `src` of this lane.  W
-// columns per lane, one 4-byte (or smaller) load each row: with 64 rows in flight per wave the chain advances 64 rows
-// per trip to memory.
-template <int U, int W, typename T, typename G>
-__device__ __forceinline__ void sum_rows(const GroupedBwd<T, G>& a, const T* src, const unsigned short* list, int at, int k,
-                                         float (&acc)[W]) {
-  typedef T vec_t __attribute__((ext_vector_type(W)));
+// Adds column `src` of the upstream rows at list[0 .. m) + at (ascending positions).  The sum is a serial chain of one wave: kBlocks
+// blocks of kBlockRows rows are on their way to registers while the oldest is added, and a row costs the wave five
+// instructions: its offset, worked out by 64 lanes at once, becomes the scalar offset of a buffer load, and what is loaded is
+// widened and added.  (With the row's 64-bit address from scalar multiplications, and two columns a lane, a row
+// took 80 clocks: a wave of 1670 rows 68 us.)  PLAIN: the upstream gradient lies within 2 GiB, so that offsets are 32 bits, and
+// joins the sum unscaled.
+constexpr int kBlockRows = 16, kBlocks = 4;
+template <bool PLAIN, typename T, typename G, typename L>
+__device__ __forceinline__ void sum_rows(const GroupedBwd<T, G>& a, long src, const L* list, int at, int m, float& acc) {
   const int lane = threadIdx.x & 63;
-  const int mine = list[k + (lane < U ? lane : 0)] + at;
-  vec_t g[U];
+  const __amdgpu_buffer_rsrc_t all = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.grad_out), 0, 0x7fffffff, 0x00020000);
+  const int mine_col = (int)(src * (long)sizeof(T));
+  T g[kBlocks][kBlockRows];
+  auto load = [&](int b, auto S) __attribute__((always_inline)) {
+    const int mine = (int)list[min(b * kBlockRows + (lane & (kBlockRows - 1)), m - 1)] + at;
+    const int ofs = (int)((unsigned)mine * (unsigned)(a.ld_go * (long)sizeof(T)));
 #pragma unroll
-  for (int u = 0; u < U; ++u)
-    g[u] = *reinterpret_cast<const vec_t*>(src + (long)__builtin_amdgcn_readlane(mine, u) * a.ld_go);
+    for (int u = 0; u < kBlockRows; ++u) {
+      T& v = g[decltype(S)::value][u];
+      if constexpr (!PLAIN)
+        v = a.grad_out[(long)__builtin_amdgcn_readlane(mine, u) * a.ld_go + src];
+      else if constexpr (sizeof(T) == 4)
+        v = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(all, mine_col, __builtin_amdgcn_readlane(ofs, u), 0));
+      else
+        v = __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b16(all, mine_col, __builtin_amdgcn_readlane(ofs, u), 0));
+    }
+  };
+  auto add = [&](int b, auto S) __attribute__((always_inline)) {
+    const int left = m - b * kBlockRows;
+    if (left >= kBlockRows) {
 #pragma unroll
-  for (int u = 0; u < U; ++u)
+      for (int u = 0; u < kBlockRows; ++u) acc += PLAIN ? to_f32(g[decltype(S)::value][u]) : a.take(g[decltype(S)::value][u]);
+    } else if (left > 0) {
 #pragma unroll
-    for (int w = 0; w < W; ++w) acc[w] += a.take(g[u][w]);
+      for (int u = 0; u < kBlockRows; ++u) acc = u < left ? acc + (PLAIN ? to_f32(g[decltype(S)::value][u]) : a.take(g[decltype(S)::value][u])) : acc;
+    }
+  };
+  // blocks behind the last one re-read its last row: with loads under a condition every block would wait for all of them
+  [&]<int... S>(std::integer_sequence<int, S...>) __attribute__((always_inline)) {
+    (load(S, std::integral_constant<int, S>{}), ...);
+  }(std::make_integer_sequence<int, kBlocks - 1>{});
+  for (int b = 0; b * kBlockRows < m; b += kBlocks)
+    [&]<int... S>(std::integer_sequence<int, S...>) __attribute__((always_inline)) {
+      ((load(b + S + kBlocks - 1, std::integral_constant<int, (S + kBlocks - 1) % kBlocks>{}),
+        add(b + S, std::integral_constant<int, S>{})),
+       ...);
+    }(std::make_integer_sequence<int, kBlocks>{});
 }
 
 // long_wgs workgroups for the long rows (long row j, column chunk y: j * chunks + y), then one wavefront per table row.
-// V: columns per lane of a short row (16-byte vectors, or 1), W: columns per lane of a long row.
-template <typename T, typename G, int V, int W>
+// V: columns per lane of a short row (16-byte vectors, or 1); a lane of a long row has one.
+template <typename T, typename G, int V>
 __global__ __launch_bounds__(256) void grouped_bwd_kernel(GroupedBwd<T, G> a, int long_wgs, int chunks) {
-  extern __shared__ unsigned bits[];  // a long row's positions as a bitmap, then the window's list
+  extern __shared__ __attribute__((aligned(16))) unsigned bits[];  // a long row's positions as a bitmap, then the window's list
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   if ((int)blockIdx.x < long_wgs) {
     __shared__ int s_row, s_part[4];
     const int want = blockIdx.x / chunks, chunk = blockIdx.x - want * chunks;
-    if (tid == 0) {
+    if (wave == 0) {  // long row `want` of all slices: 64 slices' counts at a time
       int left = want, row = -1;
-      for (int s = 0; s < a.slices; ++s) {
-        const int c = a.nlong[s];
-        if (left < c) {
-          row = a.longs[(long)s * a.long_cap + left];
-          break;
+      for (int s0 = 0; s0 < a.slices && row < 0; s0 += 64) {
+        const int c = s0 + lane < a.slices ? a.nlong[s0 + lane] : 0;
+        int x = c;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+          const int y = __shfl_up(x, o, 64);
+          if (lane >= o) x += y;
         }
-        left -= c;
+        const bool here = left < x && left >= x - c;
+        if (here) row = a.longs[(long)(s0 + lane) * a.long_cap + left - (x - c)];
+        const unsigned long long at = __ballot(here);
+        row = at ? __shfl(row, __builtin_ctzll(at), 64) : -1;
+        left -= __shfl(x, 63, 64);
       }
-      s_row = row;
+      if (lane == 0) s_row = row;
     }
     __syncthreads();
     const int row = s_row;
     if (row < 0) return;
     const int p0 = a.offs[row], cnt = a.offs[row + 1] - p0;
-    const int words = (a.n + 31) / 32, windows = (words + 255) / 256;
-    unsigned short* list = reinterpret_cast<unsigned short*>(bits + windows * 256);
-    for (int i = tid; i < windows * 256; i += 256) bits[i] = 0u;
-    __syncthreads();
-    for (int i = tid; i < cnt; i += 256) {
-      const int q = a.pos[p0 + i];
-      atomicOr(&bits[q >> 5], 1u << (q & 31));
-    }
-    const int per_row = a.cols / W, e = chunk * 256 + tid;  // W-column pieces of the row over all shards
-    const bool live = e < per_row * a.groups;
-    const int g = live ? e / per_row : 0, c = live ? (e - g * per_row) * W : 0;
-    const T* src = a.grad_out + g * a.go_sg + c;
-    float acc[W];
-#pragma unroll
-    for (int w = 0; w < W; ++w) acc[w] = 0.0f;
-    for (int win = 0; win < windows; ++win) {
-      __syncthreads();  // the bitmap is complete; the previous window's list has been read
-      // the window's 8192 positions: a word per thread, listed in ascending order
-      unsigned b = bits[win * 256 + tid];
-      int x = __popc(b);
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-      }
-      if (lane == 63) s_part[wave] = x;
+    const int e = chunk * 256 + tid;  // column of the row over all shards
+    const bool live = e < a.cols * a.groups;
+    const int g = live ? e / a.cols : 0, c = live ? e - g * a.cols : 0;
+    const long src = g * a.go_sg + c;
+    float acc = 0.0f;
+    if (cnt <= kRankRow) {
+      // every thread counts the positions below its own; (a window at a time, as below, a row of 65 positions in 65536
+      // had a trip to memory for every eight of them)
+      int* raw = reinterpret_cast<int*>(bits);
+      int* sorted = raw + kRankRow;
+      for (int i = tid; i < kRankRow; i += 256) raw[i] = i < cnt ? a.pos[p0 + i] : 0x7fffffff;
       __syncthreads();
-      int at = x - __popc(b);
-#pragma unroll
-      for (int w = 0; w < 4; ++w) at += w < wave ? s_part[w] : 0;
-      const int m = (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
-      while (b) {
-        list[at++] = (unsigned short)(tid * 32 + __builtin_ctz(b));
-        b &= b - 1;
+      for (int i = tid; i < cnt; i += 256) {
+        const int mine = raw[i];
+        int rank = 0;
+        for (int k = 0; k < cnt; k += 4) {
+          const int4 q = *reinterpret_cast<const int4*>(raw + k);
+          rank += (q.x < mine) + (q.y < mine) + (q.z < mine) + (q.w < mine);
+        }
+        sorted[rank] = mine;
       }
       __syncthreads();
-      int k = 0;
-      for (; k + 64 <= m; k += 64) sum_rows<64, W>(a, src, list, win * 8192, k, acc);
-      for (; k + 8 <= m; k += 8) sum_rows<8, W>(a, src, list, win * 8192, k, acc);
-      for (; k < m; ++k) sum_rows<1, W>(a, src, list, win * 8192, k, acc);
+      if (a.plain)
+        sum_rows<true>(a, src, sorted, 0, cnt, acc);
+      else
+        sum_rows<false>(a, src, sorted, 0, cnt, acc);
+    } else {
+      const int words = (a.n + 31) / 32, windows = (words + 255) / 256;
+      unsigned short* list = reinterpret_cast<unsigned short*>(bits + windows * 256);
+      for (int i = tid; i < windows * 256; i += 256) bits[i] = 0u;
+      __syncthreads();
+      for (int i = tid; i < cnt; i += 256) {
+        const int q = a.pos[p0 + i];
+        atomicOr(&bits[q >> 5], 1u << (q & 31));
+      }
+      for (int win = 0; win < windows; ++win) {
+        __syncthreads();  // the bitmap is complete; the previous window's list has been read
+        // the window's 8192 positions: a word per thread, listed in ascending order
+        unsigned b = bits[win * 256 + tid];
+        int x = __popc(b);
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+          const int y = __shfl_up(x, o, 64);
+          if (lane >= o) x += y;
+        }
+        if (lane == 63) s_part[wave] = x;
+        __syncthreads();
+        int at = x - __popc(b);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) at += w < wave ? s_part[w] : 0;
+        const int m = (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);
+        while (b) {
+          list[at++] = (unsigned short)(tid * 32 + __builtin_ctz(b));
+          b &= b - 1;
+        }
+        __syncthreads();
+        if (m > 0 && a.plain) sum_rows<true>(a, src, list, win * 8192, m, acc);
+        else if (m > 0) sum_rows<false>(a, src, list, win * 8192, m, acc);
+      }
     }
     if (!live) return;
-    const long off = g * a.gt_sg + (long)row * a.ld_gt + c;
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-      float one[1] = {acc[w]};
-      a.template finish<1>(one, off + w, cnt);
-    }
+    float one[1] = {acc};
+    a.template finish<1>(one, g * a.gt_sg + (long)row * a.ld_gt + c, cnt);
     return;
   }
   const int row = (int)(blockIdx.x - long_wgs) * 4 + wave;
@@ -646,7 +703,8 @@ __global__ __launch_bounds__(256) void grouped_bwd_kernel(GroupedBwd<T, G> a, in
           for (int v = 0; v < V; ++v) acc[d][v] += a.take(u[r][d].e[v]);
     };
     int k = 0;
-    for (; k + 2 <= cnt; k += 2) add(k, std::integral_constant<int, 2>{});
+    for (; k + 4 <= cnt; k += 4) add(k, std::integral_constant<int, 4>{});
+    if (k + 2 <= cnt) add(k, std::integral_constant<int, 2>{}), k += 2;
     if (k < cnt) add(k, std::integral_constant<int, 1>{});
 #pragma unroll
     for (int d = 0; d < CB; ++d) {
@@ -995,27 +1053,28 @@ extern "C" int rtp_embedding_backward_grouped(void* stream, int dtype, const voi
                        (ld_grad_table * gsz) % 16 == 0 && (grad_table_sg * gsz) % 16 == 0 &&
                        (master == nullptr || (uintptr_t)master % 16 == 0) &&
                        (weights == nullptr || (uintptr_t)weights % 16 == 0);
-  const int W = aligned && dtype == RTP_BF16 ? 2 : 1;
-  const int64_t chunks = ceil_div(cols / W * groups, 256), long_wgs = n_ids / kLongRow * chunks;
+  const int64_t reach = ((n_ids - 1) * ld_grad_out + (groups - 1) * grad_out_sg + cols) * (int64_t)esz;
+  const int plain = grad_scale == 1.0f && grad_out_sg >= 0 && reach < (1ll << 31) - 4;
+  const int64_t chunks = ceil_div(cols * groups, 256), long_wgs = n_ids / kLongRow * chunks;
   RTP_REQUIRE(long_wgs + ceil_div(row_count, 4) < (1ll << 31), "%s: grid too large", who);
   const dim3 grid((unsigned)(long_wgs + ceil_div(row_count, 4)));
   const size_t lds = (size_t)ceil_div(ceil_div(n_ids, 32), 256) * 1024 + 8192 * 2;
   ProfileScope prof(s, "embedding_backward_grouped", (double)groups * n_ids * cols,
                     (double)groups * cols * ((double)n_ids * esz + (zero_fill ? (double)row_count : 2.0 * n_ids) * gsz));
-#define RTP_EMB_GROUPED(T, G, V, W_)                                                                                    \
+#define RTP_EMB_GROUPED(T, G, V)                                                                                    \
   do {                                                                                                                \
     GroupedBwd<T, G> a{(const T*)grad_out, (long)ld_grad_out, (long)grad_out_sg, (G*)grad_table, (long)ld_grad_table,   \
                        (long)grad_table_sg, master, (T*)weights, grad_scale, lr, clip, scale_by_freq, zero_fill ? 1 : 0, \
                        store_grad, zero_fill, (int)n_ids, (int)row_count, (int)groups, (int)cols, offs, pos, nlong,      \
-                       longs, L.slices, L.long_cap};                                                                  \
-    hipLaunchKernelGGL((grouped_bwd_kernel<T, G, V, W_>), grid, dim3(256), lds, s, a, (int)long_wgs, (int)chunks);      \
+                       longs, L.slices, L.long_cap, plain};                                                                \
+    hipLaunchKernelGGL((grouped_bwd_kernel<T, G, V>), grid, dim3(256), lds, s, a, (int)long_wgs, (int)chunks);      \
   } while (0)
   if (dtype == RTP_F32) {
-    if (aligned) RTP_EMB_GROUPED(float, float, 4, 1); else RTP_EMB_GROUPED(float, float, 1, 1);
+    if (aligned) RTP_EMB_GROUPED(float, float, 4); else RTP_EMB_GROUPED(float, float, 1);
   } else if (grad_table_f32) {
-    if (aligned) RTP_EMB_GROUPED(bf16_t, float, 8, 2); else RTP_EMB_GROUPED(bf16_t, float, 1, 1);
+    if (aligned) RTP_EMB_GROUPED(bf16_t, float, 8); else RTP_EMB_GROUPED(bf16_t, float, 1);
   } else {
-    if (aligned) RTP_EMB_GROUPED(bf16_t, bf16_t, 8, 2); else RTP_EMB_GROUPED(bf16_t, bf16_t, 1, 1);
+    if (aligned) RTP_EMB_GROUPED(bf16_t, bf16_t, 8); else RTP_EMB_GROUPED(bf16_t, bf16_t, 1);
   }
 #undef RTP_EMB_GROUPED
   RTP_LAUNCH_CHECK();

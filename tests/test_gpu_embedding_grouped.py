@@ -67,3 +67,24 @@ def test_gather_over_shards(dtype, n, cols, groups):
     assert torch.equal(out, want)
     ops.embedding_gather(table[0], ids, out[:, :cols], scale=3.0, pos=pos[:, :cols], pos_sg=cols, batch=2, **kw)
     assert torch.equal(out, want * 3.0 + pos[torch.arange(n, device=DEV) // 2])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("scale", [1.0, 0.5])
+@pytest.mark.parametrize("n,cols,groups", [(2300, 300, 1), (9000, 40, 3)])
+def test_long_rows(dtype, scale, n, cols, groups):
+    """Rows of every length around the blocks of 16 and rounds of 64 that a long row is summed in, the 32 positions from which
+    a row is dealt over columns and the 512 from which its positions are listed by windows; columns that end inside a workgroup."""
+    from rtp_amd import ops
+    gen = torch.Generator().manual_seed(n)
+    counts = [1, 3, 4, 5, 15, 16, 31, 32, 33, 47, 48, 49, 63, 64, 65, 127, 511, 512, 513]
+    ids = torch.cat([torch.full((c,), r) for r, c in enumerate(counts)])
+    ids = torch.cat([ids, torch.full((n - ids.numel(),), len(counts))])[torch.randperm(n, generator=gen)].to(DEV)
+    rows = len(counts) + 2
+    g = torch.randn(n, groups * cols, generator=gen).to(dtype).to(DEV)
+    ws = ops.embedding_sort_ids(ids)
+    a, b = (torch.full((groups, rows, cols), 7.0, dtype=dtype, device=DEV) for _ in range(2))
+    kw = dict(row_begin=0, zero_fill=True, groups=groups, grad_out_sg=cols, grad_table_sg=rows * cols, grad_scale=scale)
+    ops.embedding_scatter_add(g[:, :cols], n, ws, a[0], **kw)
+    ops.embedding_backward(g[:, :cols], ids, b[0], grouped=True, **kw)
+    assert torch.equal(a, b)

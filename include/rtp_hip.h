@@ -701,8 +701,9 @@ int rtp_adam_step(void* stream, int dtype, float* master, const void* grad, void
                   double weight_decay, int64_t step, const int64_t* step_dev, double clip);
 
 /* The same update for many buffers in one launch.  `chunks` is a table in DEVICE memory, one entry per
- * workgroup: 16-byte aligned pointers into the buffers and a parameter count that is a multiple of 4 (the
- * caller cuts its buffers into chunks of, say, 16384 parameters).  total_params only feeds the profiler. */
+ * workgroup: pointers into the buffers and a parameter count (the caller cuts its buffers into chunks of, say, 16384
+ * parameters; arrays that stand alike between two boundaries of four elements are read and written four at a time).
+ * total_params only feeds the profiler. */
 typedef struct {
   float* master;
   const void* grad;
@@ -713,8 +714,7 @@ int rtp_sgd_step_multi(void* stream, int dtype, const rtp_sgd_chunk* chunks, int
                        float clip, double total_params);
 
 /* Adam for many buffers in one launch, like rtp_sgd_step_multi: `chunks` is a table in DEVICE memory, one entry per
- * workgroup (16-byte aligned pointers, a parameter count that is a multiple of 4); the other arguments as for
- * rtp_adam_step.  total_params only feeds the profiler. */
+ * workgroup; the other arguments as for rtp_adam_step.  total_params only feeds the profiler. */
 typedef struct {
   float* master;
   const void* grad;

@@ -5,20 +5,20 @@
 
 namespace rtp {
 
+// Two roundings (product, then difference): the plain closed form w - lr*g, not a fused multiply-add.
+__device__ __forceinline__ float sgd_update(float w, float g, float lr, float clip) {
+#pragma clang fp contract(off)
+  if (clip > 0.0f) g = fminf(fmaxf(g, -clip), clip);
+  const float step = lr * g;
+  return w - step;
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void sgd_kernel(float* master, const T* grad, T* shadow, long n, float lr,
                                                   float clip) {
   const long stride = (long)gridDim.x * blockDim.x;
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    float g = to_f32(grad[i]);
-    if (clip > 0.0f) g = fminf(fmaxf(g, -clip), clip);
-    // two roundings (product, then difference): the plain closed form w - lr*g, not a fused multiply-add
-    float w;
-    {
-#pragma clang fp contract(off)
-      const float step = lr * g;
-      w = master[i] - step;
-    }
+    const float w = sgd_update(master[i], to_f32(grad[i]), lr, clip);
     master[i] = w;
     if (shadow) shadow[i] = from_f32<T>(w);
   }
@@ -51,13 +51,7 @@ struct Sgd4 {
     float* wf = reinterpret_cast<float*>(&w);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      float gv = to_f32(g.e[e]);
-      if (clip > 0.0f) gv = fminf(fmaxf(gv, -clip), clip);
-      {
-#pragma clang fp contract(off)
-        const float step = lr * gv;
-        wf[e] = wf[e] - step;
-      }
+      wf[e] = sgd_update(wf[e], to_f32(g.e[e]), lr, clip);
       sh.e[e] = from_f32<T>(wf[e]);
     }
   }
@@ -92,23 +86,45 @@ __global__ __launch_bounds__(256) void sgd_vec4_kernel(float4* master, const T* 
   }
 }
 
-// Many tensors in one launch: workgroup b updates chunk b of a device-resident table, four parameters per lane
-// and access, two accesses in flight.
+// Many tensors in one launch: workgroup b updates chunk b of a device-resident table.  The arrays of a chunk may start
+// anywhere: if they stand at the same place between two boundaries of four elements (slices of equally laid out
+// buffers do), the elements before the first boundary and after the last are taken one by one and those between four
+// per lane and access, two accesses in flight; otherwise all of them one by one.
 struct SgdChunk {
   float* master;
   const void* grad;
   void* shadow;  // may be null
-  long n;        // parameters in the chunk, a multiple of 4; the three pointers are 16-byte aligned
+  long n;        // parameters in the chunk
 };
 
+// Elements of a chunk before its arrays' first common boundary of four, n when they have none.
+template <typename T>
+__device__ __forceinline__ long chunk_head(const float* master, const T* grad, const T* shadow, long n) {
+  const unsigned at = (unsigned)((uintptr_t)master / sizeof(float)) & 3;
+  const bool same = at == ((unsigned)((uintptr_t)grad / sizeof(T)) & 3) &&
+                    (!shadow || at == ((unsigned)((uintptr_t)shadow / sizeof(T)) & 3));
+  return same ? min((long)(-at & 3), n) : n;
+}
+
+// Bound by memory where chunks are full.  Layers of odd widths leave some hundred short slices per step (the biases of
+// each shard); a launch for each, and the views for it, took 12 us of the host: 97 slices of a two-block language model
+// in fp32 1220 us per update, in one launch 65 us; those of ten blocks of width 1024 and 1000 in bf16 6630 us, now 560.
 template <typename T>
 __global__ __launch_bounds__(256) void sgd_multi_kernel(const SgdChunk* chunks, float lr, float clip) {
   using P = typename Sgd4<T>::Pack;
   const SgdChunk c = chunks[blockIdx.x];
-  float4* master = reinterpret_cast<float4*>(c.master);
   const T* grad = reinterpret_cast<const T*>(c.grad);
   T* shadow = reinterpret_cast<T*>(c.shadow);
-  const long n4 = c.n >> 2;
+  const long head = chunk_head(c.master, grad, shadow, c.n), n4 = (c.n - head) >> 2;
+  for (long i = threadIdx.x; i < c.n - 4 * n4; i += 256) {
+    const long k = i < head ? i : i + 4 * n4;
+    const float w = sgd_update(c.master[k], to_f32(grad[k]), lr, clip);
+    c.master[k] = w;
+    if (shadow) shadow[k] = from_f32<T>(w);
+  }
+  float4* master = reinterpret_cast<float4*>(c.master + head);
+  grad += head;
+  if (shadow) shadow += head;
   long i = threadIdx.x;
   for (; i + 256 < n4; i += 512) {
     const P g0 = Sgd4<T>::load(grad, i), g1 = Sgd4<T>::load(grad, i + 256);
@@ -216,25 +232,39 @@ __global__ __launch_bounds__(256) void adam_vec4_kernel(float4* master, const T*
   }
 }
 
-// Adam for many buffers in one launch: workgroup b updates chunk b of a device-resident table.
+// Adam for many buffers in one launch: workgroup b updates chunk b of a device-resident table, whose arrays may start
+// anywhere as in sgd_multi_kernel (where one buffer's length is odd, each took a launch of its own, most of them element
+// by element: 612 us for ten blocks of width 1024 and 1003 in bf16, 83 M parameters, now 466).
 struct AdamChunk {
   float* master;
   const void* grad;
   void* shadow;  // may be null
   float *exp_avg, *exp_avg_sq;
-  long n;  // parameters in the chunk, a multiple of 4; the pointers are 16-byte aligned
+  long n;  // parameters in the chunk
 };
 template <typename T>
 __global__ __launch_bounds__(256) void adam_multi_kernel(const AdamChunk* chunks, AdamScalars c) {
   using P = typename Sgd4<T>::Pack;
   adam_bias_corrections(c);
   const AdamChunk ch = chunks[blockIdx.x];
-  float4* master = reinterpret_cast<float4*>(ch.master);
-  float4* m4 = reinterpret_cast<float4*>(ch.exp_avg);
-  float4* v4 = reinterpret_cast<float4*>(ch.exp_avg_sq);
   const T* grad = reinterpret_cast<const T*>(ch.grad);
   T* shadow = reinterpret_cast<T*>(ch.shadow);
-  const long n4 = ch.n >> 2;
+  // the moments are checked as two more arrays of the master's type
+  const long head = max(chunk_head(ch.master, grad, shadow, ch.n),
+                        chunk_head<float>(ch.master, ch.exp_avg, ch.exp_avg_sq, ch.n));
+  const long n4 = (ch.n - head) >> 2;
+  for (long i = threadIdx.x; i < ch.n - 4 * n4; i += 256) {
+    const long k = i < head ? i : i + 4 * n4;
+    float w = ch.master[k], m = ch.exp_avg[k], v = ch.exp_avg_sq[k];
+    adam_update(w, m, v, to_f32(grad[k]), c);
+    ch.master[k] = w, ch.exp_avg[k] = m, ch.exp_avg_sq[k] = v;
+    if (shadow) shadow[k] = from_f32<T>(w);
+  }
+  float4* master = reinterpret_cast<float4*>(ch.master + head);
+  float4* m4 = reinterpret_cast<float4*>(ch.exp_avg + head);
+  float4* v4 = reinterpret_cast<float4*>(ch.exp_avg_sq + head);
+  grad += head;
+  if (shadow) shadow += head;
   auto one = [&](long i, const P& g, float4 w, float4 m, float4 v) {
     float *wf = reinterpret_cast<float*>(&w), *mf = reinterpret_cast<float*>(&m), *vf = reinterpret_cast<float*>(&v);
     P sh;

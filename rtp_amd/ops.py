@@ -921,42 +921,41 @@ SGD_CHUNK = 16384  # parameters per workgroup of the multi-buffer update
 
 
 def sgd_chunk_table(items, device) -> Optional[torch.Tensor]:
-    """Device table for sgd_step_multi from (master, grad, shadow-or-None) triples of flat tensors, or None when
-    some buffer does not allow 16-byte accesses (then update the buffers one by one)."""
-    rows = []
+    """Device table for sgd_step_multi from (master, grad, shadow-or-None) triples of flat tensors of any length and
+    alignment, or None when there is nothing in them, their lengths differ, or they need 4-byte accesses and a graph is
+    being captured, into which the table's upload cannot go (then update the buffers one by one)."""
+    rows, odd = [], False
     for master, grad, shadow in items:
         n = master.numel()
-        ptrs = [master.data_ptr(), grad.data_ptr()] + ([shadow.data_ptr()] if shadow is not None else [])
-        if n % 4 or any(p % 16 for p in ptrs) or grad.numel() != n or (shadow is not None and shadow.numel() != n):
+        if grad.numel() != n or (shadow is not None and shadow.numel() != n):
             return None
+        odd = odd or n % 4 != 0 or any(t.data_ptr() % 16 for t in (master, grad, shadow) if t is not None)
         gs = grad.element_size()
         for off in range(0, n, SGD_CHUNK):
             cnt = min(SGD_CHUNK, n - off)
             rows.append((master.data_ptr() + off * 4, grad.data_ptr() + off * gs,
                          shadow.data_ptr() + off * gs if shadow is not None else 0, cnt))
-    if not rows:
+    if not rows or (odd and torch.cuda.is_current_stream_capturing()):
         return None
     return _device_table(rows, device)
 
 
 def adam_chunk_table(items, device) -> Optional[torch.Tensor]:
-    """Device table for adam_step_multi from (master, grad, shadow-or-None, exp_avg, exp_avg_sq) tuples of flat
-    tensors, or None when some buffer does not allow 16-byte accesses (then update the buffers one by one)."""
-    rows = []
+    """Device table for adam_step_multi from (master, grad, shadow-or-None, exp_avg, exp_avg_sq) tuples of flat tensors
+    of any length and alignment, or None as in sgd_chunk_table."""
+    rows, odd = [], False
     for master, grad, shadow, m, v in items:
         n = master.numel()
-        ptrs = [master.data_ptr(), grad.data_ptr(), m.data_ptr(), v.data_ptr()] + \
-               ([shadow.data_ptr()] if shadow is not None else [])
-        if n % 4 or any(p % 16 for p in ptrs) or any(t.numel() != n for t in (grad, m, v)) or \
-                (shadow is not None and shadow.numel() != n):
+        if any(t.numel() != n for t in (grad, m, v)) or (shadow is not None and shadow.numel() != n):
             return None
+        odd = odd or n % 4 != 0 or any(t.data_ptr() % 16 for t in (master, grad, shadow, m, v) if t is not None)
         gs = grad.element_size()
         for off in range(0, n, SGD_CHUNK):
             cnt = min(SGD_CHUNK, n - off)
             rows.append((master.data_ptr() + off * 4, grad.data_ptr() + off * gs,
                          shadow.data_ptr() + off * gs if shadow is not None else 0, m.data_ptr() + off * 4,
                          v.data_ptr() + off * 4, cnt))
-    if not rows:
+    if not rows or (odd and torch.cuda.is_current_stream_capturing()):
         return None
     return _device_table(rows, device)
 

@@ -95,7 +95,7 @@ class RotatedSGD:
         self._table_params, self._table_dtype = 0, None
         self._aux = None
         self._rest_table = self._rest_key = None
-        self._rest_params = 0
+        self._rest_params, self._rest_dtype = 0, None
         if self.fused_backward:
             ctx = ops.FusedSgd(self.lr, self.clip_value, keep_grads, source=self)
             for st, master in zip(self.stores, self.masters):
@@ -213,43 +213,58 @@ class RotatedSGD:
                          else (self.flat_master, self.flat_grad, self.flat))
         key = tuple(t.data_ptr() for it in items for t in it if t is not None)
         if key != self._table_key:
-            self._table_key = key
             self._table = ops.sgd_chunk_table(items, items[0][0].device) if items else None
+            self._table_key = key if self._table is not None else None
             self._table_params = sum(it[0].numel() for it in items)
             self._table_dtype = dtype
         return self._table
 
     def _step_rest(self) -> None:
-        """fused_backward: update every parameter range the weight-gradient products of this pass did not."""
-        items = []
+        """fused_backward: update every parameter range the weight-gradient products of this pass did not.  The slices
+        and their table are made again only when a buffer moved or other ranges are left."""
+        key = []
         for st, master in zip(self.stores, self.masters):
             if st.grads is None:
                 continue
             done = st.fused_sgd.applied
-            for off, n in zip(st.offsets, st.numels):
-                for s in range(st.world_size):
-                    if s in done.get((off, n), ()):
-                        continue
-                    g, h = st.grads[s, off:off + n], st.home[s, off:off + n]
-                    items.append((h, g, None) if master is None else (master[s, off:off + n], g, h))
+            key.append((st.home.data_ptr(), st.grads.data_ptr(), 0 if master is None else master.data_ptr(), st.numels,
+                        [sorted(done.get((off, n), ())) for off, n in zip(st.offsets, st.numels)]))
             done.clear()
         if self.flat is not None:
             self._fold_other_grads()
+            key.append((self.flat.data_ptr(), self.flat_grad.data_ptr()))
+        if not key:
+            return
+        if key != self._rest_key:
+            items = self._rest_items([k[4] for k in key if len(k) > 2])
+            same = len({it[1].dtype for it in items}) == 1
+            self._rest_table = ops.sgd_chunk_table(items, items[0][0].device) if same else None
+            self._rest_key = key if self._rest_table is not None or not items else None
+            self._rest_params = sum(it[0].numel() for it in items)
+            if self._rest_table is None:
+                for m, g, sh in items:
+                    ops.sgd_step(m, g, sh, self.lr, self.clip_value)
+                return
+            self._rest_dtype = items[0][1].dtype
+        if self._rest_table is not None:
+            ops.sgd_step_multi(self._rest_table, self._rest_dtype, self.lr, self.clip_value, self._rest_params)
+
+    def _rest_items(self, updated) -> list:
+        """(update target, gradients, weights to refresh or None) of the parameter ranges that are not among `updated`:
+        per store with gradients and parameter, the shards that its products have updated."""
+        items = []
+        stores = [(st, master) for st, master in zip(self.stores, self.masters) if st.grads is not None]
+        for (st, master), per_param in zip(stores, updated):
+            for off, n, done in zip(st.offsets, st.numels, per_param):
+                for s in range(st.world_size):
+                    if s in done:
+                        continue
+                    g, h = st.grads[s, off:off + n], st.home[s, off:off + n]
+                    items.append((h, g, None) if master is None else (master[s, off:off + n], g, h))
+        if self.flat is not None:
             items.append((self.flat, self.flat_grad, None) if self.flat_master is None
                          else (self.flat_master, self.flat_grad, self.flat))
-        if not items:
-            return
-        key = tuple(t.data_ptr() for it in items for t in it if t is not None)
-        if key != self._rest_key:
-            same = len({it[1].dtype for it in items}) == 1
-            self._rest_key = key
-            self._rest_table = ops.sgd_chunk_table(items, items[0][0].device) if same else None
-            self._rest_params = sum(it[0].numel() for it in items)
-        if self._rest_table is not None:
-            ops.sgd_step_multi(self._rest_table, items[0][1].dtype, self.lr, self.clip_value, self._rest_params)
-        else:
-            for m, g, sh in items:
-                ops.sgd_step(m, g, sh, self.lr, self.clip_value)
+        return items
 
     @torch.no_grad()
     def step(self) -> None:
@@ -289,8 +304,7 @@ class RotatedSGD:
 class RotatedAdam(RotatedSGD):
     """The reference harness's optimiser (benchmarks/rtp_benchmark.py:41-42: torch.optim.Adam(lr 1e-3) after
     clip_grad_value_(0.05)) over the same flat buffers as RotatedSGD, fp32 moments beside the fp32 master: one launch
-    over a device chunk table for all of them (or one per buffer where a buffer is not 16-byte aligned or the buffers
-    differ in dtype).  The step count lives in device
+    over a device chunk table for all of them (or one per buffer where the buffers differ in dtype).  The step count lives in device
     memory and the kernels form the bias corrections 1 - beta^step themselves, so step() may be recorded into a HIP
     graph and replayed (`steps` then only counts the eager calls)."""
 
@@ -335,8 +349,8 @@ class RotatedAdam(RotatedSGD):
             items.append((target, grads, shadow, m, v))
         ptr_key = tuple(t.data_ptr() for it in items for t in it if t is not None)
         if ptr_key != self._adam_key:
-            self._adam_key = ptr_key
             self._adam_table = ops.adam_chunk_table(items, items[0][0].device)
+            self._adam_key = ptr_key if self._adam_table is not None else None
             self._adam_params = sum(it[0].numel() for it in items)
             self._adam_dtype = items[0][1].dtype
         return self._adam_table

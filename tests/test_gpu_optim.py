@@ -139,3 +139,42 @@ def test_adam_device_step_counter_follows_graph_replays():
         assert int(step_dev) == step
         torch.testing.assert_close(master.cpu(), ref.detach(), rtol=RTOL, atol=ATOL)
         _ = (master * 2).sum().item()           # unrelated eager work between replays
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("adam", [False, True])
+def test_multi_step_at_any_alignment(dtype, adam):
+    """One launch over slices of any length and start, alike or not between two boundaries of four, against one launch
+    per slice: the same single operations on each element, so bit for bit the same, and nothing beside the slices."""
+    from rtp_amd import ops
+    gen = torch.Generator().manual_seed(11)
+    # (length, start of the fp32 arrays, start of the gradient, start of the weights)
+    forms = [(n, at, at, at) for n in (1, 2, 3, 4, 5, 7, 1027, 2048, ops.SGD_CHUNK + 5) for at in (0, 1, 2, 3, 6)]
+    forms += [(n, a, b, c) for n in (3, 4, 1030) for a, b, c in ((0, 1, 0), (1, 1, 0), (2, 0, 1), (3, 7, 3), (0, 0, 2))]
+
+    def place(values, at):
+        buf = torch.full((at + values.numel() + 9,), 7.0, dtype=values.dtype, device=DEV)
+        buf[at:at + values.numel()] = values.to(DEV)
+        return buf, buf[at:at + values.numel()]
+
+    sides = ([], [])
+    for n, at, at_g, at_w in forms:
+        w, g = torch.randn(n, generator=gen), (torch.randn(n, generator=gen) * 0.1).to(dtype)
+        for side in sides:
+            arrays = [place(w, at), place(g, at_g), place(w.to(dtype), at_w) if dtype != torch.float32 else (None, None)]
+            if adam:
+                arrays += [place(w * 0.01, at), place(w.abs() * 0.001, at_w)]
+            side.append(arrays)
+    items = [[tuple(v for _, v in arrays) for arrays in side] for side in sides]
+    total = sum(f[0] for f in forms)
+    if adam:
+        ops.adam_step_multi(ops.adam_chunk_table(items[0], DEV), dtype, 3, 1e-3, (0.9, 0.999), 1e-8, 0.01, 0.05, total)
+        for m, g, sh, a, b in items[1]:
+            ops.adam_step(m, g, sh, a, b, 3, 1e-3, (0.9, 0.999), 1e-8, 0.01, 0.05)
+    else:
+        ops.sgd_step_multi(ops.sgd_chunk_table(items[0], DEV), dtype, 0.1, 0.05, total)
+        for m, g, sh in items[1]:
+            ops.sgd_step(m, g, sh, 0.1, 0.05)
+    for form, got, want in zip(forms, *sides):
+        for (a, _), (b, _) in zip(got, want):
+            assert a is None or torch.equal(a, b), form

@@ -5,7 +5,8 @@
 //
 //   * every entry point that Python calls on the hot path, converted argument by argument from the C prototype itself
 //     (`invoke`), the current stream put in front, a negative status raised as RtpError;
-//   * `gemm` and the rotated linear products with their descriptors filled and their operands checked here;
+//   * `gemm`, and the products of the rotated linear layers, attention cores and experts on tensors, with their descriptors
+//     filled and their operands checked here;
 //   * GradBook: the parameters of a layer's shards and the slices of its gradient buffer, attached as .grad for a backward
 //     pass in one call (one Python attribute access per parameter otherwise).
 //
@@ -204,16 +205,53 @@ Field g_fields[] = {
 #undef AT
 PyObject* g_field_index = nullptr;  // name -> index into g_fields
 
-// Runs the product; returns ROWSUM (1) if the row sums asked for were produced, SGD (2) if the update was applied: what the
-// operands do not allow is left out of the launch and reported by its missing bit.
-PyObject* py_gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObject* kwnames) {
-  if (nargs != 1 || !THPDtype_Check(args[0])) return PyErr_Format(PyExc_TypeError, "gemm(dtype, *, ...)");
-  const int dt = dtype_code(((THPDtype*)args[0])->scalar_type);
-  if (dt < 0) return PyErr_Format(PyExc_TypeError, "rtp_amd kernels support float32 and bfloat16, got %R", args[0]);
+// Runs the product on the current stream and adds to `done` ROWSUM (1) if the row sums asked for were produced, SGD (2) if the
+// update was applied: what the operands do not allow is left out of the launch and reported by its missing bit.
+bool launch_product(int dt, rtp_gemm_desc& d, uint32_t flags, int& done) {
+  if (d.sgd_master) {
+    void *const master = d.sgd_master, *const weights = d.sgd_weights;
+    d.sgd_master = d.sgd_weights = nullptr;
+    d.flags = (int32_t)(flags & 0xffff & ~(uint32_t)RTP_GEMM_SGD_SKIP_OUT);
+    if (f_sgd_fused(dt, &d)) {
+      d.sgd_master = master, d.sgd_weights = weights;
+      done |= 2;
+    } else {
+      flags &= ~(uint32_t)RTP_GEMM_SGD_SKIP_OUT;
+    }
+  } else {
+    flags &= ~(uint32_t)RTP_GEMM_SGD_SKIP_OUT;
+  }
+  d.flags = (int32_t)(flags & 0xffff);
+  if (d.a_rowsum) {
+    if (f_rowsum_fused(dt, &d))
+      done |= 1;
+    else
+      d.a_rowsum = nullptr, d.rowsum_sg = 0;
+  }
+  void* st = current_stream();
+  const int rc = (WithoutGil(), f_gemm(st, dt, &d));
+  if (rc < 0) raise_status(rc);
+  return rc >= 0;
+}
+PyObject* run_product(int dt, rtp_gemm_desc& d, uint32_t flags) {
+  int done = 0;
+  return launch_product(dt, d, flags, done) ? PyLong_FromLong(done) : nullptr;
+}
+rtp_gemm_desc product(int64_t m, int64_t n, int64_t k, bool a_kcontig, bool b_kcontig) {
   rtp_gemm_desc d;
   memset(&d, 0, sizeof(d));
   d.batch = d.zdiv = d.groups = d.ksegs = 1;
   d.alpha = 1.0f;
+  d.m = m, d.n = n, d.k = k;
+  d.a_kcontig = a_kcontig, d.b_kcontig = b_kcontig;
+  return d;
+}
+
+PyObject* py_gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObject* kwnames) {
+  if (nargs != 1 || !THPDtype_Check(args[0])) return PyErr_Format(PyExc_TypeError, "gemm(dtype, *, ...)");
+  const int dt = dtype_code(((THPDtype*)args[0])->scalar_type);
+  if (dt < 0) return PyErr_Format(PyExc_TypeError, "rtp_amd kernels support float32 and bfloat16, got %R", args[0]);
+  rtp_gemm_desc d = product(0, 0, 0, false, false);
   uint32_t flags = 0;
   const Py_ssize_t nk = kwnames ? PyTuple_GET_SIZE(kwnames) : 0;
   for (Py_ssize_t i = 0; i < nk; ++i) {
@@ -242,33 +280,8 @@ PyObject* py_gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObject* 
     if (!ok) return nullptr;
   }
   d.a_kcontig = (flags >> 16) & 1, d.b_kcontig = (flags >> 17) & 1;
-  int done = 0;
-  if (d.sgd_master) {
-    void *const master = d.sgd_master, *const weights = d.sgd_weights;
-    d.sgd_master = d.sgd_weights = nullptr;
-    d.flags = (int32_t)(flags & 0xffff & ~(uint32_t)RTP_GEMM_SGD_SKIP_OUT);
-    if (f_sgd_fused(dt, &d)) {
-      d.sgd_master = master, d.sgd_weights = weights;
-      done |= 2;
-    } else {
-      flags &= ~(uint32_t)RTP_GEMM_SGD_SKIP_OUT;
-    }
-  } else {
-    flags &= ~(uint32_t)RTP_GEMM_SGD_SKIP_OUT;
-  }
-  d.flags = (int32_t)(flags & 0xffff);
-  if (d.a_rowsum) {
-    if (f_rowsum_fused(dt, &d))
-      done |= 1;
-    else
-      d.a_rowsum = nullptr, d.rowsum_sg = 0;
-  }
-  void* st = current_stream();
-  const int rc = (WithoutGil(), f_gemm(st, dt, &d));
-  if (rc < 0) return raise_status(rc);
-  return PyLong_FromLong(done);
+  return run_product(dt, d, flags);
 }
-
 // ---- the rotated linear layer's products on tensors ----
 struct Mat {
   char* p;
@@ -393,6 +406,241 @@ PyObject* py_linear_bwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return PyLong_FromLong(done);
 }
 
+// ---- the products of a row-parallel layer, of an attention core and of a run of experts, on tensors ----
+// The same launches as gemm() with the descriptor filled here instead of by some twenty keyword arguments and their lookup.
+// Forward + backward of layers that the host bounds, in processes of the slower / faster kind (a backward pass wakes a thread):
+// row-parallel Linear 254x176x2368 122 / 61 -> 95 / 48 us, attention over 80 x 3 positions 200 / 122 -> 177 / 107, 16 experts of
+// 192x256 473 / 335 -> 424 / 299.
+
+// every argument at one of `at` is a tensor
+template <size_t N>
+bool tensors_at(const char* who, PyObject* const* a, const int (&at)[N]) {
+  for (int i : at)
+    if (!THPVariable_Check(a[i])) {
+      PyErr_Format(PyExc_TypeError, "%s: argument %d has to be a tensor", who, i);
+      return false;
+    }
+  return true;
+}
+char* at_element(const at::Tensor& t, int64_t i) { return (char*)t.data_ptr() + i * (int64_t)t.element_size(); }
+
+// row_fwd(x2, flat, w_off, bias_off, n, k_s, out, col0, c_in):
+// out = (c_in +) sum_g x2[:, col0 + g*k_s : ...] W_g^T + sum_g b_g
+PyObject* py_row_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  if (nargs != 9) return PyErr_Format(PyExc_TypeError, "row_fwd(x2, flat, w_off, bias_off, n, k_s, out, col0, c_in)");
+  if (!tensors_at("row_fwd", a, {0, 1, 6})) return nullptr;
+  if (a[8] != Py_None && !THPVariable_Check(a[8])) return PyErr_Format(PyExc_TypeError, "row_fwd: c_in");
+  const at::Tensor &x2 = THPVariable_Unpack(a[0]), &flat = THPVariable_Unpack(a[1]), &out = THPVariable_Unpack(a[6]);
+  const at::Tensor* c_in = opt_tensor(a[8]);
+  int64_t w_off, n, k_s, col0;
+  if (!from_py(a[2], w_off) || !from_py(a[4], n) || !from_py(a[5], k_s) || !from_py(a[7], col0)) return nullptr;
+  rtp_rotated_linear L;
+  int dt;
+  Mat x, o, ci;
+  if (!layer_of(flat, w_off, a[3], n, k_s, L, dt) || !as_mat(x2, "operand", x) || !as_mat(out, "operand", o)) return nullptr;
+  uint32_t flags = 0;
+  auto f32 = [&](const at::Tensor& t, const char* what, uint32_t flag) {
+    if (t.scalar_type() == flat.scalar_type()) return true;
+    flags |= flag;
+    if (t.scalar_type() == at::kFloat) return true;
+    PyErr_Format(PyExc_TypeError, "row_fwd: %s must be in the shards' dtype or float32", what);
+    return false;
+  };
+  rtp_gemm_desc d = product(x.rows, n, k_s, true, true);
+  if (!f32(out, "out", RTP_GEMM_OUT_F32)) return nullptr;
+  if (c_in) {
+    if (!as_mat(*c_in, "c_in", ci) || !f32(*c_in, "c_in", RTP_GEMM_CIN_F32)) return nullptr;
+    if (ci.rows != o.rows || ci.cols != o.cols) return bad("row_fwd: c_in must have the output's shape");
+    d.c_in = ci.p, d.ld_cin = ci.ld;
+  }
+  d.a = at_element(x2, col0), d.lda = x.ld;
+  d.b = at_element(flat, w_off), d.ldb = k_s;
+  d.c_out = o.p, d.ldc = o.ld;
+  if (L.bias_off >= 0) d.bias = at_element(flat, L.bias_off);
+  d.bias_sk = d.b_sk = L.numel, d.a_sk = k_s, d.ksegs = L.shards;
+  return run_product(dt, d, flags);
+}
+
+// row_dgrad(dy2, flat, w_off, n, k_s, out, col0): out[:, col0 + g*k_s : ...] = dy2 W_g
+PyObject* py_row_dgrad(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  if (nargs != 7) return PyErr_Format(PyExc_TypeError, "row_dgrad(dy2, flat, w_off, n, k_s, out, col0)");
+  if (!tensors_at("row_dgrad", a, {0, 1, 5})) return nullptr;
+  const at::Tensor &dy2 = THPVariable_Unpack(a[0]), &flat = THPVariable_Unpack(a[1]), &out = THPVariable_Unpack(a[5]);
+  int64_t w_off, n, k_s, col0;
+  if (!from_py(a[2], w_off) || !from_py(a[3], n) || !from_py(a[4], k_s) || !from_py(a[6], col0)) return nullptr;
+  rtp_rotated_linear L;
+  int dt;
+  Mat dy, o;
+  if (!layer_of(flat, w_off, Py_None, n, k_s, L, dt) || !as_mat(dy2, "operand", dy) || !as_mat(out, "operand", o)) return nullptr;
+  rtp_gemm_desc d = product(dy.rows, k_s, n, true, false);
+  d.a = dy.p, d.lda = dy.ld;
+  d.b = at_element(flat, w_off), d.ldb = k_s, d.b_sg = L.numel;
+  d.c_out = at_element(out, col0), d.ldc = o.ld, d.c_sg = k_s;
+  d.groups = L.shards;
+  return run_product(dt, d, 0);
+}
+
+// row_wgrad(dy2, x2, grads, first, w_off, bias_off, n, k_s, col0, cnt, accumulate, sgd_master, sgd_weights, lr, clip,
+//           skip_store) -> done flags: grads[first+g, w_off : ...] (+)= dy2^T x2[:, col0 + g*k_s : ...], and the bias rows
+PyObject* py_row_wgrad(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  if (nargs != 16) return PyErr_Format(PyExc_TypeError, "row_wgrad: 16 arguments, got %zd", nargs);
+  if (!tensors_at("row_wgrad", a, {0, 1, 2})) return nullptr;
+  const at::Tensor &dy2 = THPVariable_Unpack(a[0]), &x2 = THPVariable_Unpack(a[1]), &grads = THPVariable_Unpack(a[2]);
+  int64_t first, w_off, n, k_s, col0, cnt;
+  if (!from_py(a[3], first) || !from_py(a[4], w_off) || !from_py(a[6], n) || !from_py(a[7], k_s) || !from_py(a[8], col0) ||
+      !from_py(a[9], cnt))
+    return nullptr;
+  rtp_rotated_linear L;
+  int dt;
+  Mat dy, x;
+  if (!layer_of(grads, w_off, a[5], n, k_s, L, dt) || !as_mat(dy2, "operand", dy) || !as_mat(x2, "operand", x)) return nullptr;
+  const bool accumulate = PyObject_IsTrue(a[10]);
+  uint32_t flags = RTP_GEMM_STREAM_OUT;
+  rtp_gemm_desc d = product(n, k_s, dy.rows, false, false);
+  d.a = dy.p, d.lda = dy.ld;
+  d.b = at_element(x2, col0), d.ldb = x.ld, d.b_sg = k_s;
+  d.c_out = at_element(grads, first * L.numel + w_off), d.ldc = k_s, d.c_sg = L.numel;
+  d.c_in = accumulate ? d.c_out : nullptr, d.ld_cin = k_s, d.cin_sg = L.numel;
+  if (L.bias_off >= 0) d.a_rowsum = at_element(grads, first * L.numel + L.bias_off);
+  d.rowsum_sg = L.numel;
+  if (accumulate) flags |= RTP_GEMM_ROWSUM_ACCUM;
+  d.groups = cnt;
+  if (!from_py(a[11], d.sgd_master) || !from_py(a[12], d.sgd_weights) || !from_py(a[13], d.sgd_lr) ||
+      !from_py(a[14], d.sgd_clip))
+    return nullptr;
+  if (PyObject_IsTrue(a[15])) flags |= RTP_GEMM_SGD_SKIP_OUT;
+  return run_product(dt, d, flags);
+}
+
+// bmm(a, a_off, lda, a_kcontig, a_s, a_sg,  b, ... (as a),  c, c_off, ldc, c_s, c_sg,  m, n, k, batch, zdiv, groups):
+// C = A B for every (group, outer, inner) problem, offsets and strides in elements, (outer, inner) strides as pairs; C in the
+// operands' dtype or fp32
+PyObject* py_bmm(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  if (nargs != 23) return PyErr_Format(PyExc_TypeError, "bmm: 23 arguments, got %zd", nargs);
+  if (!tensors_at("bmm", a, {0, 6, 12})) return nullptr;
+  const at::Tensor &A = THPVariable_Unpack(a[0]), &B = THPVariable_Unpack(a[6]), &C = THPVariable_Unpack(a[12]);
+  const int dt = dtype_code(B.scalar_type());
+  if (dt < 0 || A.scalar_type() != B.scalar_type() || (C.scalar_type() != B.scalar_type() && C.scalar_type() != at::kFloat))
+    return bad("bmm: a and b fp32 or bf16, c in their dtype or fp32");
+  if (!B.is_cuda()) {
+    PyErr_SetString(g_error, "rtp_amd kernels run on the GPU only; got a CPU tensor (there is no CPU path)");
+    return nullptr;
+  }
+  rtp_gemm_desc d = product(0, 0, 0, PyObject_IsTrue(a[3]), PyObject_IsTrue(a[9]));
+  auto pair = [](PyObject* v, int64_t& so, int64_t& si) {
+    if (!PyTuple_Check(v) || PyTuple_GET_SIZE(v) != 2) return PyErr_SetString(PyExc_TypeError, "bmm: a pair of strides"), false;
+    return from_py(PyTuple_GET_ITEM(v, 0), so) && from_py(PyTuple_GET_ITEM(v, 1), si);
+  };
+  int64_t a_off, b_off, c_off;
+  if (!from_py(a[1], a_off) || !from_py(a[2], d.lda) || !pair(a[4], d.a_so, d.a_si) || !from_py(a[5], d.a_sg) ||
+      !from_py(a[7], b_off) || !from_py(a[8], d.ldb) || !pair(a[10], d.b_so, d.b_si) || !from_py(a[11], d.b_sg) ||
+      !from_py(a[13], c_off) || !from_py(a[14], d.ldc) || !pair(a[15], d.c_so, d.c_si) || !from_py(a[16], d.c_sg) ||
+      !from_py(a[17], d.m) || !from_py(a[18], d.n) || !from_py(a[19], d.k) || !from_py(a[20], d.batch) ||
+      !from_py(a[21], d.zdiv) || !from_py(a[22], d.groups))
+    return nullptr;
+  d.a = at_element(A, a_off), d.b = at_element(B, b_off), d.c_out = at_element(C, c_off);
+  return run_product(dt, d, C.scalar_type() != B.scalar_type() ? RTP_GEMM_OUT_F32 : 0);
+}
+
+// One local expert of every shard of a run: x, y [slots, m_dim] and h [slots, f_dim] contiguous, the expert's slab of
+// `rows` slots starts at row r0 in the run's first shard and `row_step` rows further in each next one; w1, b1, w2, b2 are
+// offsets inside a flat shard.
+struct Experts {
+  int dt;
+  int64_t numel, shards, r0, row_step, rows, m_dim, f_dim, w1, b1, w2, b2;
+  bool read(const char* who, const at::Tensor& flat, PyObject* const* a, const at::Tensor& narrow, const at::Tensor& wide) {
+    dt = dtype_code(flat.scalar_type());
+    if (flat.dim() != 2 || !flat.is_contiguous() || dt < 0) return bad("experts: flat must be a contiguous fp32 / bf16 matrix"), false;
+    for (const at::Tensor* t : {&narrow, &wide})
+      if (t->dim() != 2 || !t->is_contiguous() || t->scalar_type() != flat.scalar_type() || !t->is_cuda())
+        return PyErr_Format(PyExc_ValueError, "%s: activations must be contiguous matrices in the shards' dtype on the GPU", who), false;
+    numel = flat.size(1), shards = flat.size(0), m_dim = narrow.size(1), f_dim = wide.size(1);
+    return from_py(a[0], r0) && from_py(a[1], row_step) && from_py(a[2], rows) && from_py(a[3], w1) && from_py(a[4], b1) &&
+           from_py(a[5], w2) && from_py(a[6], b2);
+  }
+};
+bool same_layout(const at::Tensor& t, const at::Tensor& like) {
+  return t.sizes() == like.sizes() && t.is_contiguous() && t.scalar_type() == like.scalar_type();
+}
+
+// experts_fwd(flat, x, h, y, r0, row_step, rows, w1, b1, w2, b2): h = relu(x W1^T + b1), y = h W2^T + b2
+PyObject* py_experts_fwd(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  if (nargs != 11) return PyErr_Format(PyExc_TypeError, "experts_fwd: 11 arguments, got %zd", nargs);
+  if (!tensors_at("experts_fwd", a, {0, 1, 2, 3})) return nullptr;
+  const at::Tensor &flat = THPVariable_Unpack(a[0]), &x = THPVariable_Unpack(a[1]), &h = THPVariable_Unpack(a[2]),
+                   &y = THPVariable_Unpack(a[3]);
+  Experts e;
+  if (!e.read("experts_fwd", flat, a + 4, x, h)) return nullptr;
+  if (!same_layout(y, x)) return bad("experts_fwd: y must be laid out like x");
+  auto half = [&](const at::Tensor& in, const at::Tensor& out, int64_t w, int64_t b, int64_t n, int64_t k, uint32_t flags) {
+    rtp_gemm_desc d = product(e.rows, n, k, true, true);
+    d.a = at_element(in, e.r0 * k), d.lda = k, d.a_sg = e.row_step * k;
+    d.b = at_element(flat, w), d.ldb = k, d.b_sg = e.numel;
+    d.bias = at_element(flat, b), d.bias_sg = e.numel;
+    d.c_out = at_element(out, e.r0 * n), d.ldc = n, d.c_sg = e.row_step * n;
+    d.groups = e.shards;
+    int done = 0;
+    return launch_product(e.dt, d, flags, done);
+  };
+  if (!half(x, h, e.w1, e.b1, e.f_dim, e.m_dim, RTP_GEMM_RELU) || !half(h, y, e.w2, e.b2, e.m_dim, e.f_dim, 0)) return nullptr;
+  Py_RETURN_NONE;
+}
+
+// experts_dgrad(flat, dy, h, dh, dx, r0, row_step, rows, w1, b1, w2, b2): dh = (dy W2) where h > 0, dx = dh W1
+PyObject* py_experts_dgrad(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  if (nargs != 12) return PyErr_Format(PyExc_TypeError, "experts_dgrad: 12 arguments, got %zd", nargs);
+  if (!tensors_at("experts_dgrad", a, {0, 1, 2, 3, 4})) return nullptr;
+  const at::Tensor &flat = THPVariable_Unpack(a[0]), &dy = THPVariable_Unpack(a[1]), &h = THPVariable_Unpack(a[2]),
+                   &dh = THPVariable_Unpack(a[3]), &dx = THPVariable_Unpack(a[4]);
+  Experts e;
+  if (!e.read("experts_dgrad", flat, a + 5, dy, h)) return nullptr;
+  if (!same_layout(dh, h) || !same_layout(dx, dy)) return bad("experts_dgrad: dh and dx must be laid out like h and dy");
+  auto half = [&](const at::Tensor& in, const at::Tensor& out, const at::Tensor* gate, int64_t w, int64_t n, int64_t k) {
+    rtp_gemm_desc d = product(e.rows, n, k, true, false);
+    d.a = at_element(in, e.r0 * k), d.lda = k, d.a_sg = e.row_step * k;
+    d.b = at_element(flat, w), d.ldb = n, d.b_sg = e.numel;
+    d.c_out = at_element(out, e.r0 * n), d.ldc = n, d.c_sg = e.row_step * n;
+    if (gate) d.gate = at_element(*gate, e.r0 * n), d.ld_gate = n, d.gate_sg = e.row_step * n;
+    d.groups = e.shards;
+    int done = 0;
+    return launch_product(e.dt, d, 0, done);
+  };
+  if (!half(dy, dh, &h, e.w2, e.f_dim, e.m_dim) || !half(dh, dx, nullptr, e.w1, e.m_dim, e.f_dim)) return nullptr;
+  Py_RETURN_NONE;
+}
+
+// experts_wgrad(grads, dy, h, dh, x, r0, row_step, rows, w1, b1, w2, b2, first, cnt, accumulate) -> bit 0: the second layer's
+// bias rows were produced, bit 1: the first layer's.  grads[first+g]: W2 (+)= dy^T h, W1 (+)= dh^T x over the slabs' rows, the
+// bias gradients as the row sums of the first operands
+PyObject* py_experts_wgrad(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  if (nargs != 15) return PyErr_Format(PyExc_TypeError, "experts_wgrad: 15 arguments, got %zd", nargs);
+  if (!tensors_at("experts_wgrad", a, {0, 1, 2, 3, 4})) return nullptr;
+  const at::Tensor &grads = THPVariable_Unpack(a[0]), &dy = THPVariable_Unpack(a[1]), &h = THPVariable_Unpack(a[2]),
+                   &dh = THPVariable_Unpack(a[3]), &x = THPVariable_Unpack(a[4]);
+  Experts e;
+  if (!e.read("experts_wgrad", grads, a + 5, dy, h)) return nullptr;
+  if (!same_layout(dh, h) || !same_layout(x, dy)) return bad("experts_wgrad: dh and x must be laid out like h and dy");
+  int64_t first, cnt;
+  if (!from_py(a[12], first) || !from_py(a[13], cnt)) return nullptr;
+  const bool accumulate = PyObject_IsTrue(a[14]);
+  // streamed stores: an expert's gradient (tens of MB per launch) is not read again before the optimiser, and written with
+  // ordinary ones it evicts the launch's own operands from the caches (468 -> 338 us)
+  const uint32_t flags = RTP_GEMM_STREAM_OUT | (accumulate ? (uint32_t)RTP_GEMM_ROWSUM_ACCUM : 0u);
+  auto half = [&](const at::Tensor& g, const at::Tensor& in, int64_t w, int64_t b, int64_t m, int64_t n, int& done) {
+    rtp_gemm_desc d = product(m, n, e.rows, false, false);
+    d.a = at_element(g, e.r0 * m), d.lda = m, d.a_sg = e.row_step * m;
+    d.b = at_element(in, e.r0 * n), d.ldb = n, d.b_sg = e.row_step * n;
+    d.c_out = at_element(grads, first * e.numel + w), d.ldc = n, d.c_sg = e.numel;
+    d.c_in = accumulate ? d.c_out : nullptr, d.ld_cin = n, d.cin_sg = e.numel;
+    d.a_rowsum = at_element(grads, first * e.numel + b), d.rowsum_sg = e.numel;
+    d.groups = cnt;
+    return launch_product(e.dt, d, flags, done);
+  };
+  int done2 = 0, done1 = 0;
+  if (!half(dy, h, e.w2, e.b2, e.m_dim, e.f_dim, done2) || !half(dh, x, e.w1, e.b1, e.f_dim, e.m_dim, done1)) return nullptr;
+  return PyLong_FromLong((done2 & 1) | (done1 & 1) << 1);
+}
+
 // ---- GradBook ----
 // The parameters of a layer, shard by shard, and their slices of the gradient buffer.  attach() is what a backward pass
 // does before it writes the buffer (allign_grad of the reference, rtp/module/collectives.py:75-79), for all shards at once:
@@ -496,7 +744,9 @@ PyTypeObject g_book_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 #define METHOD(name) {#name, (PyCFunction)(void*)Entry<py_##name>::call, METH_FASTCALL, nullptr},
 PyMethodDef g_methods[] = {{"bind", Entry<py_bind>::call, METH_VARARGS, nullptr},
                            {"gemm", (PyCFunction)(void*)Entry<py_gemm>::call, METH_FASTCALL | METH_KEYWORDS, nullptr},
-                           METHOD(linear_fwd) METHOD(linear_bwd) RTP_ENTRY_POINTS(METHOD, METHOD){nullptr, nullptr, 0, nullptr}};
+                           METHOD(linear_fwd) METHOD(linear_bwd) METHOD(row_fwd) METHOD(row_dgrad)
+                           METHOD(row_wgrad) METHOD(bmm) METHOD(experts_fwd) METHOD(experts_dgrad) METHOD(experts_wgrad)
+                           RTP_ENTRY_POINTS(METHOD, METHOD){nullptr, nullptr, 0, nullptr}};
 #undef METHOD
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_rtp_native", "librtp_hip.so for the calls of a training step", -1, g_methods};
 

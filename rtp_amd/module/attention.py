@@ -121,15 +121,6 @@ class SubParallelMultiheadAttention(nn.Module):
                 self.out_proj.bias.data.div_(self.world_size)
 
 
-def _bmm(dtype, *, a, a_off, lda, a_kc, a_s, a_sg, b, b_off, ldb, b_kc, b_s, b_sg, c, c_off, ldc, c_s, c_sg, m, n, k,
-         batch, zdiv, groups, out_f32=False):
-    esz = a.element_size()
-    csz = 4 if out_f32 else esz
-    ops.gemm_raw(dtype, a=a.data_ptr() + a_off * esz, b=b.data_ptr() + b_off * esz, c_out=c.data_ptr() + c_off * csz,
-                 m=m, n=n, k=k, lda=lda, ldb=ldb, ldc=ldc, a_kcontig=a_kc, b_kcontig=b_kc, batch=batch, zdiv=zdiv,
-                 a_s=a_s, b_s=b_s, c_s=c_s, out_f32=out_f32, groups=groups, a_sg=a_sg, b_sg=b_sg, c_sg=c_sg)
-
-
 class _AttentionFn(torch.autograd.Function):
     """Buffers hold all head groups side by side: qkv [L*N, ws*3E_s] (group g at column block g, inside it
     Q | K | V of that group), p [ws*N*h_s, L, L], o [L*N, E] (= the unsharded head order).  A (group,
@@ -138,7 +129,8 @@ class _AttentionFn(torch.autograd.Function):
     The core runs in one of three forms: bf16 with L <= 32 in one launch that keeps the scores in registers and
     stores p; bf16 with longer sequences in a running-softmax launch that stores only the log-sum-exp per
     query (not when the caller wants the attention weights back); otherwise as batched products and a softmax
-    kernel with p in memory."""
+    kernel with p in memory.  `bmm` takes (tensor, offset, leading dimension, contraction index contiguous, (batch, head)
+    strides, group stride) for each operand, the same without the flag for the result, and m, n, k, batch, heads, groups."""
 
     @staticmethod
     def forward(ctx, x, anchor, layer, mask, causal, want_weights, residual_grad=False, key_bias=None, drop_p=0.0):
@@ -166,6 +158,7 @@ class _AttentionFn(torch.autograd.Function):
         # drop: per-probability multiplier 0 or 1 / (1 - drop_p); pv: the probabilities that meet V
         drop = torch.empty(ws * Z, L, L, dtype=torch.float32, device=dev) if drop_p > 0.0 else None
         pv = torch.empty_like(p) if drop_p > 0.0 else p
+        bmm = ops.native().bmm
         rot = rotation(store, layer.rank)
         acc = ops.ShardSum(out, sum(len(w) for w in rot.windows))
         i = 0
@@ -191,10 +184,9 @@ class _AttentionFn(torch.autograd.Function):
                     i += 1
                     continue
                 scores = torch.empty(cnt * Z, L, L, dtype=torch.float32, device=dev)
-                _bmm(dt, a=qkv, a_off=q0, lda=ldq, a_kc=True, a_s=(ws * 3 * e_s, d), a_sg=3 * e_s, b=qkv,
-                     b_off=q0 + e_s, ldb=ldq, b_kc=True, b_s=(ws * 3 * e_s, d), b_sg=3 * e_s, c=scores, c_off=0, ldc=L,
-                     c_s=(h_s * L * L, L * L), c_sg=Z * L * L, m=L, n=L, k=d, batch=Z, zdiv=h_s, groups=cnt,
-                     out_f32=True)
+                bmm(qkv, q0, ldq, True, (ws * 3 * e_s, d), 3 * e_s,
+                    qkv, q0 + e_s, ldq, True, (ws * 3 * e_s, d), 3 * e_s,
+                    scores, 0, L, (h_s * L * L, L * L), Z * L * L, L, L, d, Z, h_s, cnt)
                 p_run = p[first * Z:(first + cnt) * Z]
                 if drop is not None:
                     ops.softmax_fwd(scores, p_run, mask=mask, causal=causal, scale=scale, key_bias=key_bias, heads=h_s,
@@ -203,9 +195,9 @@ class _AttentionFn(torch.autograd.Function):
                 else:
                     ops.softmax_fwd(scores, p_run, mask=mask, causal=causal, scale=scale, key_bias=key_bias, heads=h_s)
                 del scores
-                _bmm(dt, a=pv, a_off=first * Z * L * L, lda=L, a_kc=True, a_s=(h_s * L * L, L * L), a_sg=Z * L * L,
-                     b=qkv, b_off=q0 + 2 * e_s, ldb=ldq, b_kc=False, b_s=(ws * 3 * e_s, d), b_sg=3 * e_s, c=o,
-                     c_off=first * e_s, ldc=N * E, c_s=(E, d), c_sg=e_s, m=L, n=d, k=L, batch=Z, zdiv=h_s, groups=cnt)
+                bmm(pv, first * Z * L * L, L, True, (h_s * L * L, L * L), Z * L * L,
+                    qkv, q0 + 2 * e_s, ldq, False, (ws * 3 * e_s, d), 3 * e_s, o, first * e_s, N * E, (E, d), e_s,
+                    L, d, L, Z, h_s, cnt)
                 c_out, c_in = acc.target(i)
                 S.row_fwd(o, flat, w_o_off, E, e_s, b_o_off, c_out, first * e_s, c_in=c_in)
                 i += 1
@@ -245,6 +237,7 @@ class _AttentionFn(torch.autograd.Function):
         ldq = N * ws * 3 * e_s
         fused = ctx.fused
         delta = torch.empty_like(p) if ctx.flash is not None else None
+        bmm = ops.native().bmm
         rot = rotation(store, layer.rank, reverse=True)
         # residual_grad: the caller's y = norm(x + attention(x)) sends x's whole gradient through this function,
         # which adds the output gradient to its own input gradient in the epilogue of the last product
@@ -277,26 +270,24 @@ class _AttentionFn(torch.autograd.Function):
                     continue
                 # attention core, all (group, batch, head) triples of the run in one launch each
                 dp = torch.empty(cnt * Z, L, L, dtype=torch.float32, device=dev)
-                _bmm(dt, a=do, a_off=first * e_s, lda=N * E, a_kc=True, a_s=(E, d), a_sg=e_s, b=qkv, b_off=q0 + 2 * e_s,
-                     ldb=ldq, b_kc=True, b_s=(ws * 3 * e_s, d), b_sg=3 * e_s, c=dp, c_off=0, ldc=L,
-                     c_s=(h_s * L * L, L * L), c_sg=Z * L * L, m=L, n=L, k=d, batch=Z, zdiv=h_s, groups=cnt, out_f32=True)
+                bmm(do, first * e_s, N * E, True, (E, d), e_s,
+                    qkv, q0 + 2 * e_s, ldq, True, (ws * 3 * e_s, d), 3 * e_s,
+                    dp, 0, L, (h_s * L * L, L * L), Z * L * L, L, L, d, Z, h_s, cnt)
                 p_off = first * Z * L * L
                 # dV = P^T dO
-                _bmm(dt, a=pv, a_off=p_off, lda=L, a_kc=False, a_s=(h_s * L * L, L * L), a_sg=Z * L * L, b=do,
-                     b_off=first * e_s, ldb=N * E, b_kc=False, b_s=(E, d), b_sg=e_s, c=dqkv, c_off=q0 + 2 * e_s, ldc=ldq,
-                     c_s=(ws * 3 * e_s, d), c_sg=3 * e_s, m=L, n=d, k=L, batch=Z, zdiv=h_s, groups=cnt)
+                bmm(pv, p_off, L, False, (h_s * L * L, L * L), Z * L * L, do, first * e_s, N * E, False, (E, d), e_s,
+                    dqkv, q0 + 2 * e_s, ldq, (ws * 3 * e_s, d), 3 * e_s, L, d, L, Z, h_s, cnt)
                 ds = torch.empty(cnt * Z, L, L, dtype=dt, device=dev)
                 ops.softmax_bwd(p[first * Z:(first + cnt) * Z], dp, ds, scale,
                                 keep=None if drop is None else drop[first * Z:(first + cnt) * Z])
                 del dp
                 # dQ = dS K
-                _bmm(dt, a=ds, a_off=0, lda=L, a_kc=True, a_s=(h_s * L * L, L * L), a_sg=Z * L * L, b=qkv,
-                     b_off=q0 + e_s, ldb=ldq, b_kc=False, b_s=(ws * 3 * e_s, d), b_sg=3 * e_s, c=dqkv, c_off=q0, ldc=ldq,
-                     c_s=(ws * 3 * e_s, d), c_sg=3 * e_s, m=L, n=d, k=L, batch=Z, zdiv=h_s, groups=cnt)
+                bmm(ds, 0, L, True, (h_s * L * L, L * L), Z * L * L,
+                    qkv, q0 + e_s, ldq, False, (ws * 3 * e_s, d), 3 * e_s, dqkv, q0, ldq, (ws * 3 * e_s, d), 3 * e_s,
+                    L, d, L, Z, h_s, cnt)
                 # dK = dS^T Q
-                _bmm(dt, a=ds, a_off=0, lda=L, a_kc=False, a_s=(h_s * L * L, L * L), a_sg=Z * L * L, b=qkv, b_off=q0,
-                     ldb=ldq, b_kc=False, b_s=(ws * 3 * e_s, d), b_sg=3 * e_s, c=dqkv, c_off=q0 + e_s, ldc=ldq,
-                     c_s=(ws * 3 * e_s, d), c_sg=3 * e_s, m=L, n=d, k=L, batch=Z, zdiv=h_s, groups=cnt)
+                bmm(ds, 0, L, False, (h_s * L * L, L * L), Z * L * L, qkv, q0, ldq, False, (ws * 3 * e_s, d), 3 * e_s,
+                    dqkv, q0 + e_s, ldq, (ws * 3 * e_s, d), 3 * e_s, L, d, L, Z, h_s, cnt)
                 # in-projection input gradient: dX += sum_g dQKV_g W_in,g
                 if need_dx:
                     c_out, c_in = acc.target(i)
@@ -407,6 +398,7 @@ class _GeneralAttentionFn(torch.autograd.Function):
         drop = torch.empty(ws * Z, L, sk, dtype=torch.float32, device=dev) if drop_p > 0.0 else None
         pv = torch.empty_like(p) if drop_p > 0.0 else p
         ld = N * E  # one step along the sequence in q, k, v and o
+        bmm = ops.native().bmm
         rot = rotation(store, layer.rank)
         acc = ops.ShardSum(out, sum(len(w) for w in rot.windows))
         i = 0
@@ -427,9 +419,8 @@ class _GeneralAttentionFn(torch.autograd.Function):
                     i += 1
                     continue
                 scores = torch.empty(cnt * Z, L, sk, dtype=torch.float32, device=dev)
-                _bmm(dt, a=qb, a_off=c0, lda=ld, a_kc=True, a_s=(E, d), a_sg=e_s, b=kb, b_off=c0, ldb=ld, b_kc=True,
-                     b_s=(E, d), b_sg=e_s, c=scores, c_off=0, ldc=sk, c_s=(h_s * L * sk, L * sk), c_sg=Z * L * sk,
-                     m=L, n=sk, k=d, batch=Z, zdiv=h_s, groups=cnt, out_f32=True)
+                bmm(qb, c0, ld, True, (E, d), e_s, kb, c0, ld, True, (E, d), e_s,
+                    scores, 0, sk, (h_s * L * sk, L * sk), Z * L * sk, L, sk, d, Z, h_s, cnt)
                 if drop is not None:
                     ops.softmax_fwd(scores, p[first * Z:(first + cnt) * Z], mask=mask, causal=False, scale=scale,
                                     key_bias=key_bias, heads=h_s,
@@ -439,9 +430,8 @@ class _GeneralAttentionFn(torch.autograd.Function):
                     ops.softmax_fwd(scores, p[first * Z:(first + cnt) * Z], mask=mask, causal=False, scale=scale,
                                     key_bias=key_bias, heads=h_s)
                 del scores
-                _bmm(dt, a=pv, a_off=first * Z * L * sk, lda=sk, a_kc=True, a_s=(h_s * L * sk, L * sk),
-                     a_sg=Z * L * sk, b=vb, b_off=c0, ldb=ld, b_kc=False, b_s=(E, d), b_sg=e_s, c=o, c_off=c0, ldc=ld,
-                     c_s=(E, d), c_sg=e_s, m=L, n=d, k=sk, batch=Z, zdiv=h_s, groups=cnt)
+                bmm(pv, first * Z * L * sk, sk, True, (h_s * L * sk, L * sk), Z * L * sk,
+                    vb, c0, ld, False, (E, d), e_s, o, c0, ld, (E, d), e_s, L, d, sk, Z, h_s, cnt)
                 c_out, c_in = acc.target(i)
                 S.row_fwd(o, flat, w_o, E, e_s, b_o, c_out, c0, c_in=c_in)
                 i += 1
@@ -478,6 +468,7 @@ class _GeneralAttentionFn(torch.autograd.Function):
         dkb = torch.empty(sk * N, E, dtype=dt, device=dev)
         dvb = torch.empty(sk * N, E, dtype=dt, device=dev)
         delta = torch.empty_like(p) if ctx.flash is not None else None
+        bmm = ops.native().bmm
         rot = rotation(store, layer.rank, reverse=True)
         parts = sum(len(w) for w in rot.windows)
         # input gradients of the three projections, each summed over the shards; the rows of an appended zero key
@@ -507,25 +498,21 @@ class _GeneralAttentionFn(torch.autograd.Function):
                     continue
                 # dP = dO V^T
                 dp = torch.empty(cnt * Z, L, sk, dtype=torch.float32, device=dev)
-                _bmm(dt, a=do, a_off=c0, lda=ld, a_kc=True, a_s=(E, d), a_sg=e_s, b=vb, b_off=c0, ldb=ld, b_kc=True,
-                     b_s=(E, d), b_sg=e_s, c=dp, c_off=0, ldc=sk, c_s=p_s, c_sg=p_sg, m=L, n=sk, k=d, batch=Z,
-                     zdiv=h_s, groups=cnt, out_f32=True)
+                bmm(do, c0, ld, True, (E, d), e_s, vb, c0, ld, True, (E, d), e_s, dp, 0, sk, p_s, p_sg,
+                    L, sk, d, Z, h_s, cnt)
                 # dV = P^T dO
-                _bmm(dt, a=pv, a_off=p_off, lda=sk, a_kc=False, a_s=p_s, a_sg=p_sg, b=do, b_off=c0, ldb=ld, b_kc=False,
-                     b_s=(E, d), b_sg=e_s, c=dvb, c_off=c0, ldc=ld, c_s=(E, d), c_sg=e_s, m=sk, n=d, k=L, batch=Z,
-                     zdiv=h_s, groups=cnt)
+                bmm(pv, p_off, sk, False, p_s, p_sg, do, c0, ld, False, (E, d), e_s, dvb, c0, ld, (E, d), e_s,
+                    sk, d, L, Z, h_s, cnt)
                 ds = torch.empty(cnt * Z, L, sk, dtype=dt, device=dev)
                 ops.softmax_bwd(p[first * Z:(first + cnt) * Z], dp, ds, scale,
                                 keep=None if drop is None else drop[first * Z:(first + cnt) * Z])
                 del dp
                 # dQ = dS K
-                _bmm(dt, a=ds, a_off=0, lda=sk, a_kc=True, a_s=p_s, a_sg=p_sg, b=kb, b_off=c0, ldb=ld, b_kc=False,
-                     b_s=(E, d), b_sg=e_s, c=dqb, c_off=c0, ldc=ld, c_s=(E, d), c_sg=e_s, m=L, n=d, k=sk, batch=Z,
-                     zdiv=h_s, groups=cnt)
+                bmm(ds, 0, sk, True, p_s, p_sg, kb, c0, ld, False, (E, d), e_s, dqb, c0, ld, (E, d), e_s,
+                    L, d, sk, Z, h_s, cnt)
                 # dK = dS^T Q
-                _bmm(dt, a=ds, a_off=0, lda=sk, a_kc=False, a_s=p_s, a_sg=p_sg, b=qb, b_off=c0, ldb=ld, b_kc=False,
-                     b_s=(E, d), b_sg=e_s, c=dkb, c_off=c0, ldc=ld, c_s=(E, d), c_sg=e_s, m=sk, n=d, k=L, batch=Z,
-                     zdiv=h_s, groups=cnt)
+                bmm(ds, 0, sk, False, p_s, p_sg, qb, c0, ld, False, (E, d), e_s, dkb, c0, ld, (E, d), e_s,
+                    sk, d, L, Z, h_s, cnt)
                 _shard_inputs_grad(sums, flat, e_s, c0, i)
                 i += 1
             rot.release(j)

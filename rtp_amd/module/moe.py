@@ -102,7 +102,6 @@ class _ExpertsFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, anchor, layer):
         store, n_local, c_rows, m_dim, f_dim = _ExpertsFn._geom(layer, x)
-        es = x.element_size()
         h = torch.empty(x.shape[0], f_dim, dtype=x.dtype, device=x.device)
         y = torch.empty_like(x)
         rot = rotation(store, layer.rank)
@@ -111,15 +110,7 @@ class _ExpertsFn(torch.autograd.Function):
                 for le in range(n_local):
                     w1, b1, w2, b2 = store.offsets[4 * le:4 * le + 4]
                     r0 = (first * n_local + le) * c_rows
-                    common = dict(groups=cnt, b_sg=store.numel, bias_sg=store.numel, a_kcontig=True, b_kcontig=True)
-                    ops.gemm_raw(x.dtype, a=x.data_ptr() + r0 * m_dim * es, b=flat.data_ptr() + w1 * es,
-                                 bias=flat.data_ptr() + b1 * es, c_out=h.data_ptr() + r0 * f_dim * es, m=c_rows,
-                                 n=f_dim, k=m_dim, lda=m_dim, ldb=m_dim, ldc=f_dim, relu=True,
-                                 a_sg=n_local * c_rows * m_dim, c_sg=n_local * c_rows * f_dim, **common)
-                    ops.gemm_raw(x.dtype, a=h.data_ptr() + r0 * f_dim * es, b=flat.data_ptr() + w2 * es,
-                                 bias=flat.data_ptr() + b2 * es, c_out=y.data_ptr() + r0 * m_dim * es, m=c_rows,
-                                 n=m_dim, k=f_dim, lda=f_dim, ldb=f_dim, ldc=m_dim,
-                                 a_sg=n_local * c_rows * f_dim, c_sg=n_local * c_rows * m_dim, **common)
+                    ops.native().experts_fwd(flat, x, h, y, r0, n_local * c_rows, c_rows, w1, b1, w2, b2)
             rot.release(j)
         ctx.layer = layer
         ctx.save_for_backward(x, h)
@@ -130,7 +121,6 @@ class _ExpertsFn(torch.autograd.Function):
         layer = ctx.layer
         x, h = ctx.saved_tensors
         store, n_local, c_rows, m_dim, f_dim = _ExpertsFn._geom(layer, x)
-        es = x.element_size()
         dy = dy.contiguous()
         dh = torch.empty_like(h)
         dx = torch.empty_like(x)
@@ -138,19 +128,9 @@ class _ExpertsFn(torch.autograd.Function):
         for j in range(rot.steps):
             for flat, first, cnt in rot.acquire(j):
                 for le in range(n_local):
-                    w1, _, w2, _ = store.offsets[4 * le:4 * le + 4]
+                    w1, b1, w2, b2 = store.offsets[4 * le:4 * le + 4]
                     r0 = (first * n_local + le) * c_rows
-                    common = dict(groups=cnt, b_sg=store.numel, a_kcontig=True, b_kcontig=False)
-                    # dH = (dY W2) masked by H > 0 ; dX = dH W1
-                    ops.gemm_raw(x.dtype, a=dy.data_ptr() + r0 * m_dim * es, b=flat.data_ptr() + w2 * es,
-                                 c_out=dh.data_ptr() + r0 * f_dim * es, gate=h.data_ptr() + r0 * f_dim * es,
-                                 ld_gate=f_dim, gate_sg=n_local * c_rows * f_dim, m=c_rows, n=f_dim, k=m_dim, lda=m_dim,
-                                 ldb=f_dim, ldc=f_dim, a_sg=n_local * c_rows * m_dim, c_sg=n_local * c_rows * f_dim,
-                                 **common)
-                    ops.gemm_raw(x.dtype, a=dh.data_ptr() + r0 * f_dim * es, b=flat.data_ptr() + w1 * es,
-                                 c_out=dx.data_ptr() + r0 * m_dim * es, m=c_rows, n=m_dim, k=f_dim, lda=f_dim,
-                                 ldb=m_dim, ldc=m_dim, a_sg=n_local * c_rows * f_dim, c_sg=n_local * c_rows * m_dim,
-                                 **common)
+                    ops.native().experts_dgrad(flat, dy, h, dh, dx, r0, n_local * c_rows, c_rows, w1, b1, w2, b2)
             rot.release(j)
         runs = store.grad_runs()  # attaches (and on first use allocates) the gradient storage
         g = store.grads
@@ -158,30 +138,16 @@ class _ExpertsFn(torch.autograd.Function):
             for le in range(n_local):
                 w1, b1, w2, b2 = store.offsets[4 * le:4 * le + 4]
                 r0 = (first * n_local + le) * c_rows
-                base = g.data_ptr() + first * store.numel * es
-                # stream_out: an expert's gradient (tens of MB per launch) is not read again before the optimiser, and
-                # written with ordinary stores it evicts the launch's own operands from the caches (468 -> 338 us)
-                common = dict(groups=cnt, c_sg=store.numel, cin_sg=store.numel, a_kcontig=False, b_kcontig=False,
-                              stream_out=True)
-                # dW2 = dY^T H ; dW1 = dH^T X  (contraction over the expert's capacity rows); the bias gradients are
-                # the row sums of the first operands and come out of the same launches where the library can fuse them
-                c2 = base + w2 * es
-                fused2 = ops.gemm_raw(
-                    x.dtype, a=dy.data_ptr() + r0 * m_dim * es, b=h.data_ptr() + r0 * f_dim * es, c_out=c2,
-                    c_in=c2 if accumulate else None, ld_cin=f_dim, m=m_dim, n=f_dim, k=c_rows, lda=m_dim, ldb=f_dim,
-                    ldc=f_dim, a_sg=n_local * c_rows * m_dim, b_sg=n_local * c_rows * f_dim, rowsum=base + b2 * es,
-                    rowsum_sg=store.numel, rowsum_accum=accumulate, **common)
-                c1 = base + w1 * es
-                fused1 = ops.gemm_raw(
-                    x.dtype, a=dh.data_ptr() + r0 * f_dim * es, b=x.data_ptr() + r0 * m_dim * es, c_out=c1,
-                    c_in=c1 if accumulate else None, ld_cin=m_dim, m=f_dim, n=m_dim, k=c_rows, lda=f_dim, ldb=m_dim,
-                    ldc=m_dim, a_sg=n_local * c_rows * f_dim, b_sg=n_local * c_rows * m_dim, rowsum=base + b1 * es,
-                    rowsum_sg=store.numel, rowsum_accum=accumulate, **common)
+                # the bias gradients come out of the same launches where the library can fuse them
+                fused = ops.native().experts_wgrad(g, dy, h, dh, x, r0, n_local * c_rows, c_rows, w1, b1, w2, b2, first, cnt,
+                                                   accumulate)
+                if fused == 3:
+                    continue
                 for s in range(first, first + cnt):  # otherwise: column sums over each expert's own rows
                     r = (s * n_local + le) * c_rows
-                    if not fused2:
+                    if not fused & 1:
                         ops.colsum(dy[r:r + c_rows], g[s, b2:b2 + m_dim], accumulate=accumulate)
-                    if not fused1:
+                    if not fused & 2:
                         ops.colsum(dh[r:r + c_rows], g[s, b1:b1 + f_dim], accumulate=accumulate)
         store.grads_ready()
         return dx, None, None

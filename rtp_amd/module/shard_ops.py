@@ -100,45 +100,30 @@ def col_bgrad(dy2, grads, first, b_off, n_s, col0, cnt, accumulate):
 
 def row_fwd(x2, flat, w_off, n, k_s, bias_off, out, col0, c_in: Optional[torch.Tensor] = None):
     """out[M, n] = (c_in +) sum_g x2[:, col0 + g*k_s : ...] @ W_g^T + sum_g b_g."""
-    cnt, numel = flat.shape
-    es = flat.element_size()
-    m, _, lda = _rows(x2)
-    _, _, ldc = _rows(out)
-    kw = ops._epilogue_args(flat.dtype, out, c_in, None, None)
-    ops.gemm_raw(flat.dtype, a=x2.data_ptr() + col0 * es, b=flat.data_ptr() + w_off * es, c_out=out.data_ptr(), m=m,
-                 n=n, k=k_s, lda=lda, ldb=k_s, ldc=ldc, a_kcontig=True, b_kcontig=True,
-                 bias=None if bias_off is None else flat.data_ptr() + bias_off * es, bias_sk=numel, ksegs=cnt,
-                 a_sk=k_s, b_sk=numel, **kw)
+    ops.native().row_fwd(x2, flat, w_off, bias_off, n, k_s, out, col0, c_in)
 
 
 def row_dgrad(dy2, flat, w_off, n, k_s, out, col0):
     """out[:, col0 + g*k_s : ...] = dy2 @ W_g, g over the run."""
-    cnt, numel = flat.shape
-    es = flat.element_size()
-    m, _, lda = _rows(dy2)
-    _, _, ldc = _rows(out)
-    ops.gemm_raw(flat.dtype, a=dy2.data_ptr(), b=flat.data_ptr() + w_off * es, c_out=out.data_ptr() + col0 * es, m=m,
-                 n=k_s, k=n, lda=lda, ldb=k_s, ldc=ldc, a_kcontig=True, b_kcontig=False, groups=cnt, b_sg=numel,
-                 c_sg=k_s)
+    ops.native().row_dgrad(dy2, flat, w_off, n, k_s, out, col0)
 
 
 def row_wgrad(dy2, x2, grads, first, w_off, n, k_s, col0, cnt, accumulate, b_off: Optional[int] = None, store=None):
     """grads[first+g, w_off : w_off + n*k_s] (+)= dy2^T @ x2[:, col0 + g*k_s : ...]; with `b_off` also the bias
     gradients grads[first+g, b_off : b_off + n] (+)= column sums of dy2 (every shard of a row-style layer stores
     bias/ws and receives the full sum, tests/test_linear.py:181-186)."""
-    numel = grads.shape[1]
-    es = grads.element_size()
-    m, _, lda = _rows(dy2)
-    _, _, ldb = _rows(x2)
-    c = grads.data_ptr() + (first * numel + w_off) * es
-    rs = None if b_off is None else grads.data_ptr() + (first * numel + b_off) * es
     kw = _fused(store, accumulate, first, cnt, w_off, n * k_s)
-    fused = ops.gemm_raw(grads.dtype, a=dy2.data_ptr(), b=x2.data_ptr() + col0 * es, c_out=c, m=n, n=k_s, k=m, lda=lda,
-                         ldb=ldb, ldc=k_s, a_kcontig=False, b_kcontig=False, groups=cnt, b_sg=k_s, c_sg=numel,
-                         c_in=c if accumulate else None, ld_cin=k_s, cin_sg=numel, stream_out=True,
-                         rowsum=rs, rowsum_sg=numel, rowsum_accum=accumulate, **kw)
-    _fused_done(store, kw)
-    if b_off is not None and not fused:
+    if kw:
+        sgd = kw["sgd"]
+        done = ops.native().row_wgrad(dy2, x2, grads, first, w_off, b_off, n, k_s, col0, cnt, accumulate, kw["sgd_master"],
+                                      kw["sgd_weights"] or None, sgd.lr, sgd.clip, not sgd.keep_grads)
+        if not done & _lib.ROTATED_SGD_DONE:
+            sgd.missed = True
+        _fused_done(store, kw)
+    else:
+        done = ops.native().row_wgrad(dy2, x2, grads, first, w_off, b_off, n, k_s, col0, cnt, accumulate, None, None, 0.0, 0.0,
+                                      False)
+    if b_off is not None and not done & _lib.ROTATED_BIAS_DONE:
         row_bgrad(dy2, grads, first, b_off, n, cnt, accumulate)
 
 

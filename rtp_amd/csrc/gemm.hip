@@ -1202,11 +1202,15 @@ __global__ __launch_bounds__(kThreads) void gemm_tiny_kernel(GemmArgs p, long nb
 // leave most CUs idle, one serial chain each.  Here a workgroup owns 32 x 32 outputs and its eight waves an eighth of the
 // contraction each; the partial sums meet in LDS and are added in wave order.  Both operands are row-contiguous, so a lane's
 // MFMA operand is one float of a k line: fragments come straight from global memory (two 128-byte lines per load, any
-// alignment), 16 k ahead of the MFMAs that use them, and there is no staging and no barrier in the loop.
-// Loads and MFMAs of a CU balance (a CU's four SIMDs take eight 256-byte loads per 64-clock MFMA round).
-// us, 64 x 64 tiles -> this: 512 x 512 x 1600 31 -> 21, 512 x 512 x 2880 51 -> 34, 256 x 256 x 1024 21 -> 13, 128 x 128 x 8192
-// 128 -> 74; error against fp64 7.2e-7 -> 2.6e-7 (eight short sums instead of one long one).
-constexpr int kSplitWaves = 8, kSplitBatch = 8;  // waves, MFMAs (two k each) per batch of loads
+// alignment) and there is no staging and no barrier in the loop.  Bound by the fp32 MFMAs (3.4 ns per k at 2.35 GHz) where
+// the loads' latency is hidden: four batches of 16 loads are in flight per wave, as many as the counter of outstanding loads
+// (63) can tell apart, with the lines' addresses on the scalar unit (a buffer resource per batch) and the order held by scheduling
+// barriers, or the compiler gathers all the loads behind all the products.
+// us, 64 x 64 tiles of fp32 MFMAs -> one batch ahead -> this: 512 x 512 x 1600 31 -> 19.8 -> 12.9, 512 x 512 x 2880 51 -> 30.2 -> 17.4,
+// 256 x 256 x 1024 21 -> 12.9 -> 9.6, 128 x 128 x 8192 128 -> 74.8 -> 36.0; error against fp64 7.2e-7 -> 2.6e-7 (eight short sums
+// instead of one long one).
+// waves, MFMAs (two k each) per batch of loads, batches of loads ahead of the MFMAs
+constexpr int kSplitWaves = 8, kSplitBatch = 8, kSplitAhead = 4;
 __global__ __launch_bounds__(64 * kSplitWaves) void gemm_ksplit_kernel(GemmArgs p) {
   __shared__ float part[kSplitWaves][32][33];
   __shared__ float sums[kSplitWaves][32];
@@ -1218,9 +1222,11 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemm_ksplit_kernel(GemmArgs 
   const int m0 = bid / p.tiles_n * 32, n0 = bid % p.tiles_n * 32;
   const int grp = blockIdx.y / p.batch, zb = blockIdx.y % p.batch;
   const long zo = zb / p.zdiv, zi = zb % p.zdiv;
-  // rows past the end re-read the last one: they feed accumulators that are never stored
-  const float* A = reinterpret_cast<const float*>(p.a) + grp * p.a_sg + zo * p.a_so + zi * p.a_si + min(m0 + li, p.m - 1);
-  const float* B = reinterpret_cast<const float*>(p.b) + grp * p.b_sg + zo * p.b_so + zi * p.b_si + min(n0 + li, p.n - 1);
+  const float* A = reinterpret_cast<const float*>(p.a) + grp * p.a_sg + zo * p.a_so + zi * p.a_si;
+  const float* B = reinterpret_cast<const float*>(p.b) + grp * p.b_sg + zo * p.b_so + zi * p.b_si;
+  // a lane's place from the start of a pair of k lines; rows past the end re-read the last one: they feed accumulators that
+  // are never stored
+  const unsigned at_a = (unsigned)(min(m0 + li, p.m - 1) + g * (int)p.lda), at_b = (unsigned)(min(n0 + li, p.n - 1) + g * (int)p.ldb);
 
   f32x16 acc;
 #pragma unroll
@@ -1229,33 +1235,53 @@ __global__ __launch_bounds__(64 * kSplitWaves) void gemm_ksplit_kernel(GemmArgs 
   constexpr int STEP = 2 * kSplitBatch;
   const int chunk = ((p.k + kSplitWaves * STEP - 1) / (kSplitWaves * STEP)) * STEP;
   const int kb = min(wave * chunk, p.k), ke = min(kb + chunk, p.k);
-  float a[2][kSplitBatch], b[2][kSplitBatch];
-  auto fetch = [&](const float* As, const float* Bs, int k0, float (&fa)[kSplitBatch], float (&fb)[kSplitBatch]) {
-#pragma unroll
-    for (int e = 0; e < kSplitBatch; ++e) {
-      const long k = min(k0 + 2 * e + g, p.k - 1);
-      fa[e] = As[k * p.lda];
-      fb[e] = Bs[k * p.ldb];
-    }
-  };
-  auto multiply = [&](int k0, float (&fa)[kSplitBatch], float (&fb)[kSplitBatch]) {
-#pragma unroll
-    for (int e = 0; e < kSplitBatch; ++e) {
-      const bool live = k0 + 2 * e + g < ke;
-      const float x = live ? fa[e] : 0.0f, y = live ? fb[e] : 0.0f;
-      rs += x;
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc, 0, 0, 0);
-    }
+  const int full = (ke - kb) / STEP;
+  struct Batch {
+    float a[kSplitBatch], b[kSplitBatch];
   };
   for (int seg = 0; seg < p.ksegs; ++seg) {
     const float* As = A + seg * p.a_sk;
     const float* Bs = B + seg * p.b_sk;
-    if (kb < ke) fetch(As, Bs, kb, a[0], b[0]);
-    for (int k0 = kb; k0 < ke; k0 += 2 * STEP) {
-      if (k0 + STEP < ke) fetch(As, Bs, k0 + STEP, a[1], b[1]);
-      multiply(k0, a[0], b[0]);
-      if (k0 + 2 * STEP < ke) fetch(As, Bs, k0 + 2 * STEP, a[0], b[0]);
-      if (k0 + STEP < ke) multiply(k0 + STEP, a[1], b[1]);
+    Batch ring[kSplitAhead];
+    auto fetch = [&](int i, Batch& f) {  // batch i, or the last whole one again
+      const long k0 = kb + min(i, full - 1) * STEP;
+      const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(As + k0 * p.lda), 0, 0x7fffffff, 0x00020000);
+      const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(Bs + k0 * p.ldb), 0, 0x7fffffff, 0x00020000);
+#pragma unroll
+      for (int e = 0; e < kSplitBatch; ++e) {
+        f.a[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ra, (int)(4 * at_a), 8 * e * (int)p.lda, 0));
+        f.b[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, (int)(4 * at_b), 8 * e * (int)p.ldb, 0));
+      }
+      __builtin_amdgcn_sched_barrier(0);  // in the order written: the loads of a batch right behind the products of the one before
+    };
+    auto multiply = [&](const Batch& f) {
+#pragma unroll
+      for (int e = 0; e < kSplitBatch; ++e) {
+        rs += f.a[e];
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(f.a[e], f.b[e], acc, 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    if (full > 0) {
+#pragma unroll
+      for (int u = 0; u < kSplitAhead; ++u) fetch(u, ring[u]);
+      int i = 0;
+      for (; i + kSplitAhead <= full; i += kSplitAhead)
+#pragma unroll
+        for (int u = 0; u < kSplitAhead; ++u) {
+          multiply(ring[u]);
+          fetch(i + u + kSplitAhead, ring[u]);
+        }
+#pragma unroll
+      for (int u = 0; u < kSplitAhead; ++u)
+        if (i + u < full) multiply(ring[u]);
+    }
+    for (int k0 = kb + full * STEP; k0 < ke; k0 += 2) {  // what is no whole batch
+      const long k = min(k0 + g, p.k - 1) - g;
+      const bool live = k0 + g < ke;
+      const float x = live ? As[k * p.lda + at_a] : 0.0f, y = live ? Bs[k * p.ldb + at_b] : 0.0f;
+      rs += x;
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc, 0, 0, 0);
     }
   }
 #pragma unroll
@@ -1473,11 +1499,13 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
     RTP_LAUNCH_CHECK();
     return RTP_OK;
   }
-  // few fp32 weight-gradient tiles, long contraction: see gemm_ksplit_kernel.  64 tiles of 64 x 64 are 256 of its workgroups, one
-  // a CU, and it is ahead (512 x 512: K = 512 12.8 -> 9.2 us, K = 2880 49 -> 33); from 65 on some CU has two and it is behind, with
-  // 72 as with 128 tiles (512 x 576: 12.7 against 14.6 and 49 against 56; 512 x 1024: 13.0 against 15.1 and 49 against 58).
+  // few fp32 weight-gradient tiles, long contraction: see gemm_ksplit_kernel.  128 tiles of 64 x 64 are 512 of its workgroups, two a
+  // CU, and it is ahead of the tiles of gemm_split_kernel, which take the same time for 65 tiles as for 256; with three it is
+  // behind.  us, gemm_split_kernel -> this, K = 512 / 2048 / 4096: 512 x 576 13.7 / 36 / 65 -> 13.3 / 25 / 40, 512 x 1024
+  // 14.1 / 36 / 65 -> 13.3 / 32 / 53, 256 x 2048 13.9 / 36 / 65 -> 13.6 / 37 / 61; 768 x 768 (144 tiles) 14.3 / 36 / 65 against
+  // 18.9 / 37 / 60.
   if (sizeof(T) == 4 && fast && !akc && !bkc && !d->sgd_master && !d->xent_mode && d->k >= 512 && nz < 65536 &&
-      ceil_div(d->m, 64) * ceil_div(d->n, 64) * nz <= 64) {
+      ceil_div(d->m, 64) * ceil_div(d->n, 64) * nz <= 128) {
     a.tiles_m = (int)ceil_div(d->m, 32);
     a.tiles_n = (int)ceil_div(d->n, 32);
     const double mn_ = (double)d->m * (double)d->n * (double)nz, kk_ = (double)d->k * (double)d->ksegs;

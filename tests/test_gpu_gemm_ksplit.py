@@ -42,3 +42,27 @@ def test_split_contraction(m, n, k, groups, segs, accum):
     assert rel_err(out, ref) <= TOL[torch.float32]
     if fused:
         assert rel_err(sums, rows) <= TOL[torch.float32]
+
+
+@pytest.mark.parametrize("k", [512, 640, 767, 898, 1024, 1025, 1283])  # 4 - 11 batches a wave, whole and ragged
+@pytest.mark.parametrize("m,n,taken", [(40, 72, True), (512, 1024, True), (513, 1024, False)])
+def test_split_contraction_batches(m, n, taken, k):
+    """Every remainder of the loop over batches in flight, and both sides of the last tile count that goes here.  Rows and
+    columns behind the operands' last hold NaN: nothing of them may reach a result."""
+    from rtp_amd import _lib
+    gen = torch.Generator().manual_seed(k)
+    a, b = _rand((k, m + 4), torch.float32, gen), _rand((k, n + 4), torch.float32, gen)
+    a[:, m:], b[:, n:] = float("nan"), float("nan")
+    ref = a[:, :m].double().t() @ b[:, :n].double()
+    ad, bd = a.to(DEV), b.to(DEV)
+    out = torch.full((m, n), float("nan"), device=DEV)
+    _lib.profile_enable(1)
+    try:
+        _ops().gemm_raw(torch.float32, a=ad.data_ptr(), b=bd.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=m + 4,
+                        ldb=n + 4, ldc=n, a_kcontig=False, b_kcontig=False)
+        torch.cuda.synchronize()
+        names = list(_lib.profile_collect())
+    finally:
+        _lib.profile_enable(0)
+    assert any("ksplit" in nm for nm in names) == taken, names
+    assert rel_err(out, ref) <= TOL[torch.float32]

@@ -1499,6 +1499,24 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
     RTP_LAUNCH_CHECK();
     return RTP_OK;
   }
+  // Few tiles, whatever the layout: see gemm_kwaves.hip.  256 tiles of 32 x 32 are one workgroup a CU, and up to there it is ahead at
+  // every contraction from 256 on (measured in a replayed graph on 70 shapes x 3 layouts x 2 types; bf16 1.1 - 2.5 times, fp32 1.5 - 2.3).
+  // From 257 on some CU has two and only fp32 with K of 768 and more gains, up to 512.  us, before -> this:
+  // 256 tiles bf16 64 x 4096, K = 512 5.7 -> 4.6, 4096 19.2 -> 10.3; 288 tiles 384 x 768, K = 256 5.2 -> 6.7, 1024 7.6 -> 8.7, 2048
+  // 12.1 -> 11.7; 512 tiles fp32 512 x 1024, K = 384 10.8 -> 12.6, 1024 19.6 -> 18.1; 768 tiles 512 x 1536, K = 2048 36 -> 44.
+  const int64_t tiles32 = ceil_div(d->m, 32) * ceil_div(d->n, 32) * nz, k_all = d->k * d->ksegs;
+  if (direct && a.vec_c && !d->xent_mode && nz < 65536 && k_all >= 256 &&
+      tiles32 <= (sizeof(T) == 4 && k_all >= 768 ? 512 : 256)) {
+    a.tiles_m = (int)ceil_div(d->m, 32);
+    a.tiles_n = (int)ceil_div(d->n, 32);
+    static const char* const names[2][2][2] = {
+        {{"gemm_f32_32x32_kwaves_rc_rc", "gemm_f32_32x32_kwaves_rc_kc"}, {"gemm_f32_32x32_kwaves_kc_rc", "gemm_f32_32x32_kwaves_kc_kc"}},
+        {{"gemm_bf16_32x32_kwaves_rc_rc", "gemm_bf16_32x32_kwaves_rc_kc"}, {"gemm_bf16_32x32_kwaves_kc_rc", "gemm_bf16_32x32_kwaves_kc_kc"}}};
+    const double mn_ = (double)d->m * (double)d->n * (double)nz, kk_ = (double)d->k * (double)d->ksegs;
+    ProfileScope prof(s, names[sizeof(T) == 2][akc][bkc], 2.0 * mn_ * kk_,
+                      ((double)d->m + (double)d->n) * kk_ * nz * sizeof(T) + mn_ * sizeof(T));
+    return launch_kwaves(s, a, sizeof(T) == 2, akc, bkc, dim3((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nz));
+  }
   // few fp32 weight-gradient tiles, long contraction: see gemm_ksplit_kernel.  128 tiles of 64 x 64 are 512 of its workgroups, two a
   // CU, and it is ahead of the tiles of gemm_split_kernel, which take the same time for 65 tiles as for 256; with three it is
   // behind.  us, gemm_split_kernel -> this, K = 512 / 2048 / 4096: 512 x 576 13.7 / 36 / 65 -> 13.3 / 25 / 40, 512 x 1024

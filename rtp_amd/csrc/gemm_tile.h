@@ -584,7 +584,7 @@ typedef __attribute__((address_space(3))) void* lptr_t;
 //    chunk index inside k line kl is XORed with rc_swizzle(kl) so that the 4 lines fall on different slots.
 template <typename T, int R>
 __device__ __forceinline__ constexpr int rc_swizzle(int kl) {
-  if (sizeof(T) != 2) return 0;
+  if (sizeof(T) != 2 || R < 64) return 0;  // (the 64-byte lines of 32 rows fall on different slots as they stand)
   return R >= 128 ? (kl & 3) << 2 : ((kl >> 1) & 1) << 2;
 }
 
@@ -774,5 +774,8 @@ __device__ __forceinline__ Frag<T> read_frag_dma(const char* st, int rowbase, in
 
 // The fp32 products of gemm_split.hip, in tiles of bm (128 or 64) x 64; ragged: an operand is not vector-aligned.
 int launch_split(hipStream_t s, const GemmArgs& a, bool akc, bool bkc, int bm, bool ragged, dim3 grid);
+
+// Few tiles of 32 x 32, the contraction over the waves (gemm_kwaves.hip).
+int launch_kwaves(hipStream_t s, const GemmArgs& a, bool bf16, bool akc, bool bkc, dim3 grid);
 
 }  // namespace rtp

@@ -51,15 +51,15 @@ def test_split_contraction_batches(m, n, taken, k):
     columns behind the operands' last hold NaN: nothing of them may reach a result."""
     from rtp_amd import _lib
     gen = torch.Generator().manual_seed(k)
-    a, b = _rand((k, m + 4), torch.float32, gen), _rand((k, n + 4), torch.float32, gen)
+    a, b = _rand((k, m + 3), torch.float32, gen), _rand((k, n + 1), torch.float32, gen)
     a[:, m:], b[:, n:] = float("nan"), float("nan")
     ref = a[:, :m].double().t() @ b[:, :n].double()
     ad, bd = a.to(DEV), b.to(DEV)
     out = torch.full((m, n), float("nan"), device=DEV)
     _lib.profile_enable(1)
     try:
-        _ops().gemm_raw(torch.float32, a=ad.data_ptr(), b=bd.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=m + 4,
-                        ldb=n + 4, ldc=n, a_kcontig=False, b_kcontig=False)
+        _ops().gemm_raw(torch.float32, a=ad.data_ptr(), b=bd.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=m + 3,
+                        ldb=n + 1, ldc=n, a_kcontig=False, b_kcontig=False)
         torch.cuda.synchronize()
         names = list(_lib.profile_collect())
     finally:

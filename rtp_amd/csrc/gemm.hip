@@ -1504,8 +1504,11 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   // From 257 on some CU has two and only fp32 with K of 768 and more gains, up to 512.  us, before -> this:
   // 256 tiles bf16 64 x 4096, K = 512 5.7 -> 4.6, 4096 19.2 -> 10.3; 288 tiles 384 x 768, K = 256 5.2 -> 6.7, 1024 7.6 -> 8.7, 2048
   // 12.1 -> 11.7; 512 tiles fp32 512 x 1024, K = 384 10.8 -> 12.6, 1024 19.6 -> 18.1; 768 tiles 512 x 1536, K = 2048 36 -> 44.
+  // A product under a ReLU stays in the order of its sums, here and below: a sum within its rounding of zero decides whether the
+  // backward pass sees the unit at all, and of 16 M such sums (1000 tokens, 8 experts of 768 x 8064) some ten are that near.
+  const bool relu = d->flags & RTP_GEMM_RELU;
   const int64_t tiles32 = ceil_div(d->m, 32) * ceil_div(d->n, 32) * nz, k_all = d->k * d->ksegs;
-  if (direct && a.vec_c && !d->xent_mode && nz < 65536 && k_all >= 256 &&
+  if (direct && a.vec_c && !relu && !d->xent_mode && nz < 65536 && k_all >= 256 &&
       tiles32 <= (sizeof(T) == 4 && k_all >= 768 ? 512 : 256)) {
     a.tiles_m = (int)ceil_div(d->m, 32);
     a.tiles_n = (int)ceil_div(d->n, 32);
@@ -1582,7 +1585,7 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   // 1024 x 2048 x 2048 74 -> 56; 8 of 122 x 1088 x 1536 51 -> 32.
   // Its two tiles cost 700 and 430 ns a slab and 4 us a round with every CU busy.  (The launches that take 128 x 160 tiles, two even
   // rounds of an fp32 logits layer, stay with them.)
-  const bool split = sizeof(T) == 4 && fast && d->k * d->ksegs >= 384 && shape != 6;
+  const bool split = sizeof(T) == 4 && fast && !relu && k_all >= 384 && shape != 6;
   if (split) {
     const double nslabs = (double)ceil_div(d->k, 32) * (double)d->ksegs;
     const auto cost = [&](int bm, double slab) {

@@ -72,11 +72,13 @@ def test_epilogue(dtype, akc, bkc):
     size = (a.double().abs() @ b.double().abs().t()).cpu() + 16
     common = dict(lda=k, ldb=k if bkc else n, ldc=n)
     for f32 in (True, False):
-        out = torch.empty(m, n, dtype=torch.float32 if f32 else dtype, device=DEV)
-        _run(dtype, a, bt, m, n, k, akc, bkc, c_out=out.data_ptr(), bias=bias.data_ptr(), c_in=cin.data_ptr(), ld_cin=n,
-             cin_f32=True, out_f32=f32, relu=True, **common)
-        ref = (prod + bias.double().cpu() + cin.double().cpu()).clamp(min=0)
-        assert ((out.cpu().double() - ref).abs() <= _bound(out.dtype, k // 2, size, ref)).all()
+        for relu in (False, True):  # (a ReLU's sums keep their order)
+            out = torch.empty(m, n, dtype=torch.float32 if f32 else dtype, device=DEV)
+            _run(dtype, a, bt, m, n, k, akc, bkc, taken=not relu, c_out=out.data_ptr(), bias=bias.data_ptr(),
+                 c_in=cin.data_ptr(), ld_cin=n, cin_f32=True, out_f32=f32, relu=relu, **common)
+            ref = prod + bias.double().cpu() + cin.double().cpu()
+            ref = ref.clamp(min=0) if relu else ref
+            assert ((out.cpu().double() - ref).abs() <= _bound(out.dtype, k // 2, size, ref)).all()
     out = torch.empty(m, n, dtype=dtype, device=DEV)
     _run(dtype, a, bt, m, n, k, akc, bkc, c_out=out.data_ptr(), gate=gate.data_ptr(), ld_gate=n, alpha=0.5, **common)
     ref = 0.5 * prod * (gate.cpu() > 0)

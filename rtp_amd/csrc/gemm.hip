@@ -1520,6 +1520,23 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
                       ((double)d->m + (double)d->n) * kk_ * nz * sizeof(T) + mn_ * sizeof(T));
     return launch_kwaves(s, a, sizeof(T) == 2, akc, bkc, dim3((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nz));
   }
+  // Many outputs, at most two K slabs: see gemm_shortk.hip.  From 384 of its tiles on it is ahead, in every layout; with 256, one
+  // workgroup a CU, it is behind (us, before -> this, bf16: 2048 x 2048 x 64 7.0 -> 7.0, 1024 x 4096 x 96 7.6 -> 8.1, 4096 x 1536 x 32
+  // 9.0 -> 8.0, 2048 x 8192 x 96 16.7 -> 13.3; three slabs: 8192 x 1536 x 256 18.8 -> 17.0 in bf16, but 66 -> 70 in fp32).
+  if (direct && a.vec_c && !d->xent_mode && nz < 65536 && k_all * (int64_t)sizeof(T) <= 256 &&
+      ceil_div(d->m, 128) * ceil_div(d->n, 128) * nz >= 384) {
+    a.tiles_m = (int)ceil_div(d->m, 128);
+    a.tiles_n = (int)ceil_div(d->n, 128);
+    a.d_tiles_n = make_fastdiv((unsigned)a.tiles_n);
+    static const char* const names[2][2][2] = {
+        {{"gemm_f32_128x128_shortk_rc_rc", "gemm_f32_128x128_shortk_rc_kc"}, {"gemm_f32_128x128_shortk_kc_rc", "gemm_f32_128x128_shortk_kc_kc"}},
+        {{"gemm_bf16_128x128_shortk_rc_rc", "gemm_bf16_128x128_shortk_rc_kc"},
+         {"gemm_bf16_128x128_shortk_kc_rc", "gemm_bf16_128x128_shortk_kc_kc"}}};
+    const double mn_ = (double)d->m * (double)d->n * (double)nz, kk_ = (double)d->k * (double)d->ksegs;
+    ProfileScope prof(s, names[sizeof(T) == 2][akc][bkc], 2.0 * mn_ * kk_,
+                      ((double)d->m + (double)d->n) * kk_ * nz * sizeof(T) + mn_ * sizeof(T));
+    return launch_shortk(s, a, sizeof(T) == 2, akc, bkc, dim3((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nz));
+  }
   // few fp32 weight-gradient tiles, long contraction: see gemm_ksplit_kernel.  128 tiles of 64 x 64 are 512 of its workgroups, two a
   // CU, and it is ahead of the tiles of gemm_split_kernel, which take the same time for 65 tiles as for 256; with three it is
   // behind.  us, gemm_split_kernel -> this, K = 512 / 2048 / 4096: 512 x 576 13.7 / 36 / 65 -> 13.3 / 25 / 40, 512 x 1024

@@ -775,6 +775,8 @@ __device__ __forceinline__ Frag<T> read_frag_dma(const char* st, int rowbase, in
 // The fp32 products of gemm_split.hip, in tiles of bm (128 or 64) x 64; ragged: an operand is not vector-aligned.
 int launch_split(hipStream_t s, const GemmArgs& a, bool akc, bool bkc, int bm, bool ragged, dim3 grid);
 
+// Many tiles of 128 x 128 over a K slab or two (gemm_shortk.hip).
+int launch_shortk(hipStream_t s, const GemmArgs& a, bool bf16, bool akc, bool bkc, dim3 grid);
 // Few tiles of 32 x 32, the contraction over the waves (gemm_kwaves.hip).
 int launch_kwaves(hipStream_t s, const GemmArgs& a, bool bf16, bool akc, bool bkc, dim3 grid);
 

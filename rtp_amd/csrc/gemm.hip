@@ -270,104 +270,6 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs p) {
   store_tile<T, MT, NT, WM, WN>(p, acc, t.m0, t.n0, wm, wn, li, g, grp, zo, zi);
 }
 
-// A 16-byte vector shifted down by `n` elements, zeros moving in from the top: what a vector that was read `n` elements
-// before its place (to stay inside the operand) has to undergo.
-template <typename T>
-__device__ __forceinline__ uint4 shift_down(uint4 q, int n) {
-  constexpr int PER = 4 / (int)sizeof(T);  // elements per word
-  const int w = n / PER;
-  const unsigned d[4] = {q.x, q.y, q.z, q.w};
-  unsigned r[5];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    r[i] = 0u;
-#pragma unroll
-    for (int j = i; j < 4; ++j) r[i] = w == j - i ? d[j] : r[i];
-  }
-  r[4] = 0u;
-  if (PER == 2) {
-    const unsigned odd = (n & 1) * 16u;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) r[i] = odd ? (r[i] >> 16) | (r[i + 1] << 16) : r[i];
-  }
-  return make_uint4(r[0], r[1], r[2], r[3]);
-}
-
-// The loader for operands the direct-to-LDS loads cannot take: rows, extents or base addresses that are no multiples of 16
-// bytes (a 1001-class head, shards of odd size).  Vectors are read with unaligned 16-byte loads into registers, kRegDepth
-// slabs ahead, and written to the stage in the layout DmaOperand leaves there.  A vector that would reach beyond its row (or k
-// line) is read further down, inside it, and shifted into place; this is decided per vector without a branch, and
-// the shift only runs in slabs and tiles that have such vectors.  Needs rows (k lines) of at least one vector.
-// Bound by the rate of unaligned vector loads: 25 - 28 bytes a clock and CU from the L1 against 56 for aligned ones.  A layer of
-// 992 x 1001 x 2048 (bf16, 8 shards, forward + both gradients): 54 us, 185 us with the guarded scalar loads; 4096^3 with
-// one extent odd 180 - 290 us.
-constexpr int kRegDepth = 3;
-template <typename T, int R, bool KC, int NL, int SB>
-struct RegOperand {
-  using D = DmaOperand<T, R, KC, NL, SB>;
-  static constexpr int VEC = D::VEC, NI = D::NI, BYTES = D::BYTES;
-  typedef unsigned vec_t __attribute__((ext_vector_type(4), aligned(2)));  // global loads take any alignment
-  const char* base;  // the operand's element 0 (K-contiguous: of row row0)
-  long ldb;          // leading dimension in bytes
-  unsigned ofs[NI];  // K-contiguous: of the lane's row;  else of the lane's rows inside a k line
-  int koff[NI];      // k of the vector inside its slab
-  int shift[NI];     // !KC: elements the vector was read early
-  bool edge;         // !KC: the tile has such vectors
-  uint4 val[kRegDepth][NI];
-
-  __device__ __forceinline__ void init(const T* x, long ld, int row0, int rows, int lw, int lane) {
-    ldb = ld * (long)sizeof(T);
-    base = reinterpret_cast<const char*>(KC ? x + (long)row0 * ld : x);
-    edge = !KC && row0 + R > rows;
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int j = lw * NI + i;
-      if (KC) {
-        constexpr int LPR = SB / 16;
-        const int row = j * (64 / LPR) + lane / LPR;
-        const int rr = row0 + row < rows ? row : rows - 1 - row0;
-        ofs[i] = (unsigned)(rr * ldb);
-        koff[i] = ((lane % LPR) ^ kc_swizzle<SB>(row)) * VEC;
-        shift[i] = 0;
-      } else {
-        const int byte = lane * 16;
-        koff[i] = j * (1024 / D::LINE) + byte / D::LINE;
-        const int r = row0 + (((byte % D::LINE) >> 4) ^ rc_swizzle<T, R>(koff[i])) * VEC;
-        const int start = min(r, rows - VEC);
-        ofs[i] = (unsigned)(start * (int)sizeof(T));
-        shift[i] = r - start;
-      }
-    }
-  }
-  // request the slab whose first k is k0 (in a segment that starts seg bytes from the operand's base)
-  template <int S>
-  __device__ __forceinline__ void fetch(long seg, int k0, int kdim) {
-    const char* b = base + seg + (KC ? 0 : (long)k0 * ldb);
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const unsigned o = KC ? ofs[i] + (unsigned)(min(k0 + koff[i], kdim - VEC) * (int)sizeof(T))
-                            : ofs[i] + (unsigned)(min(koff[i], kdim - 1 - k0) * ldb);
-      const vec_t v = *reinterpret_cast<const vec_t*>(b + o);
-      val[S][i] = make_uint4(v.x, v.y, v.z, v.w);
-    }
-  }
-  template <int S>
-  __device__ __forceinline__ void store(char* stage, int lw, int lane, int k0, int kdim) {
-    const bool tail = k0 + D::BK_ > kdim;
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      uint4 q = val[S][i];
-      if (KC) {
-        if (tail) q = shift_down<T>(q, min(max(k0 + koff[i] - (kdim - VEC), 0), VEC));
-      } else {
-        if (edge) q = shift_down<T>(q, min(shift[i], VEC));
-        if (tail && k0 + koff[i] >= kdim) q = make_uint4(0u, 0u, 0u, 0u);
-      }
-      *reinterpret_cast<uint4*>(stage + (lw * NI + i) * 1024 + lane * 16) = q;
-    }
-  }
-};
-
 // The body of the product kernel: workgroup `id` of the `nwg` that work on the problem `p` (`bx`, `by`: its
 // coordinates in a launch that does not use XCD bricks).  `p` lives in the kernel-argument segment.
 // REG: the loader waves go through registers (RegOperand) instead of loading straight into LDS.  RAG: the epilogue's operands
@@ -1504,12 +1406,14 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   // From 257 on some CU has two and only fp32 with K of 768 and more gains, up to 512.  us, before -> this:
   // 256 tiles bf16 64 x 4096, K = 512 5.7 -> 4.6, 4096 19.2 -> 10.3; 288 tiles 384 x 768, K = 256 5.2 -> 6.7, 1024 7.6 -> 8.7, 2048
   // 12.1 -> 11.7; 512 tiles fp32 512 x 1024, K = 384 10.8 -> 12.6, 1024 19.6 -> 18.1; 768 tiles 512 x 1536, K = 2048 36 -> 44.
+  // Operands that are not vector-aligned, 12 shapes: bf16 255 x 1023 x 3333 24.0 -> 17.6, 31 x 2049 x 515 8.6 -> 8.2, one of 25 behind
+  // (7 x 8101 x 1027, input gradient, 13.4 -> 14.2); fp32 65.6 -> 28.5 and 15.8 -> 11.1.  (Row-contiguous fp32 has gemm_ksplit_kernel.)
   // A product under a ReLU stays in the order of its sums, here and below: a sum within its rounding of zero decides whether the
   // backward pass sees the unit at all, and of 16 M such sums (1000 tokens, 8 experts of 768 x 8064) some ten are that near.
   const bool relu = d->flags & RTP_GEMM_RELU;
   const int64_t tiles32 = ceil_div(d->m, 32) * ceil_div(d->n, 32) * nz, k_all = d->k * d->ksegs;
-  if (direct && a.vec_c && !relu && !d->xent_mode && nz < 65536 && k_all >= 256 &&
-      tiles32 <= (sizeof(T) == 4 && k_all >= 768 ? 512 : 256)) {
+  if (fast && !relu && !d->xent_mode && nz < 65536 && k_all >= 256 &&
+      !(sizeof(T) == 4 && !direct && !akc && !bkc) && tiles32 <= (sizeof(T) == 4 && k_all >= 768 ? 512 : 256)) {
     a.tiles_m = (int)ceil_div(d->m, 32);
     a.tiles_n = (int)ceil_div(d->n, 32);
     static const char* const names[2][2][2] = {
@@ -1518,7 +1422,7 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
     const double mn_ = (double)d->m * (double)d->n * (double)nz, kk_ = (double)d->k * (double)d->ksegs;
     ProfileScope prof(s, names[sizeof(T) == 2][akc][bkc], 2.0 * mn_ * kk_,
                       ((double)d->m + (double)d->n) * kk_ * nz * sizeof(T) + mn_ * sizeof(T));
-    return launch_kwaves(s, a, sizeof(T) == 2, akc, bkc, dim3((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nz));
+    return launch_kwaves(s, a, sizeof(T) == 2, akc, bkc, direct, dim3((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nz));
   }
   // Many outputs, at most two K slabs: see gemm_shortk.hip.  From 384 of its tiles on it is ahead, in every layout; with 256, one
   // workgroup a CU, it is behind (us, before -> this, bf16: 2048 x 2048 x 64 7.0 -> 7.0, 1024 x 4096 x 96 7.6 -> 8.1, 4096 x 1536 x 32

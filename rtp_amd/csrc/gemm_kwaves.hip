@@ -13,7 +13,11 @@ namespace rtp {
 // us in a replayed graph on operands that are not in the caches, 64 x 64 tiles -> this: bf16 64 x 1024 x 1024 7.0 -> 4.9, 32 x 4096 x 4096
 // 18.9 -> 9.9, 32 x 1024 x 8192 31.1 -> 13.9, input gradient 64 x 4096 x 4096 19.5 -> 14.7; fp32 (split tiles before) 64 x 1024 x 1024
 // 18.4 -> 8.7, 64 x 4096 x 4096 57.7 -> 26.7.  Eight short sums: error against fp64 below that of one long one.
-template <typename T, bool AKC, bool BKC>
+//
+// REG: operands of any alignment, through registers into the wave's LDS, three slabs ahead (bf16 255 x 1023 x 3333 24.0 -> 17.6 us,
+// 64 x 1001 x 2048 10.7 -> 7.8, its weight gradient 22.5 -> 14.4; fp32 255 x 1023 x 3333 65.6 -> 28.5, 1 x 1303 x 1364 29.4 -> 11.7); RAG: the element-wise epilogue (an output,
+// addend or mask that is not vector-aligned).
+template <typename T, bool AKC, bool BKC, bool REG, bool RAG>
 __global__ __launch_bounds__(512) void gemm_kwaves_kernel(GemmArgs p) {
   constexpr int SB = 128, NST = 2;  // bytes of a slab's row, stages per wave
   using DA = DmaOperand<T, 32, AKC, 1, SB>;
@@ -42,34 +46,11 @@ __global__ __launch_bounds__(512) void gemm_kwaves_kernel(GemmArgs p) {
   const int per = (nk + WAVES - 1) / WAVES;
   const int first = min(wave * per, nk), n = min(per, nk - first);
 
-  DA da;
-  DB db;
-  da.init(p.lda, m0, p.m, 0, lane);
-  db.init(p.ldb, n0, p.n, 0, lane);
   constexpr long SZ = (long)sizeof(T);
   const long step_a = (AKC ? (long)BK : (long)BK * p.lda) * SZ, step_b = (BKC ? (long)BK : (long)BK * p.ldb) * SZ;
   const long last_a = step_a + p.a_sk * SZ - nk_seg * step_a, last_b = step_b + p.b_sk * SZ - nk_seg * step_b;
   const int seg = first / nk_seg, in_seg = first - seg * nk_seg;
-  const char* ca = DA::slab_base(A, p.lda, m0) + seg * p.a_sk * SZ + in_seg * step_a;
-  const char* cb = DB::slab_base(B, p.ldb, n0) + seg * p.b_sk * SZ + in_seg * step_b;
-  int left = nk_seg - in_seg;  // slabs left in the K segment, the next one included
-  const bool tail = p.k % BK != 0;
   char* const mine = lds + wave * (NST * STAGE);
-  const unsigned lds_mine = (unsigned)(uintptr_t)(lptr_t)lds + (unsigned)(wave * (NST * STAGE));
-  auto issue = [&](int stage) __attribute__((always_inline)) {
-    const unsigned at = lds_mine + (unsigned)(stage * STAGE);
-    if (left != 1 || !tail) {
-      da.template issue<false>(at, 0, ca, 0, 0);
-      db.template issue<false>(at + DA::BYTES, 0, cb, 0, 0);
-    } else {
-      da.template issue<true>(at, 0, ca, (nk_seg - 1) * BK, p.k);
-      db.template issue<true>(at + DA::BYTES, 0, cb, (nk_seg - 1) * BK, p.k);
-    }
-    const bool more = left != 1;
-    ca += more ? step_a : last_a;
-    cb += more ? step_b : last_b;
-    left = more ? left - 1 : nk_seg;
-  };
 
   f32x16 acc;
 #pragma unroll
@@ -95,27 +76,93 @@ __global__ __launch_bounds__(512) void gemm_kwaves_kernel(GemmArgs p) {
     }
   };
 
-#pragma unroll
-  for (int s = 0; s < NST; ++s)
-    if (s < n) issue(s);
-  int i = 0;
-  for (; i + 2 * NST <= n; i += NST)
-#pragma unroll
-    for (int s = 0; s < NST; ++s) {
-      asm volatile("s_waitcnt vmcnt(%0)" : : "n"((NST - 1) * NI) : "memory");
-      read(s);
-      issue(s);
+  if constexpr (REG) {
+    // slabs behind the wave's last one re-read it, so that the loop has no branch around a request
+    RegOperand<T, 32, AKC, 1, SB> ra;
+    RegOperand<T, 32, BKC, 1, SB> rb;
+    ra.init(A, p.lda, m0, p.m, 0, lane);
+    rb.init(B, p.ldb, n0, p.n, 0, lane);
+    struct Place {
+      int seg, k0, i;
+    };
+    Place f{seg, in_seg * BK, 0}, w = f;  // the next slab to request and to write
+    auto next = [&](Place& at) __attribute__((always_inline)) {
+      if (++at.i >= n) return;
+      at.k0 += BK;
+      if (at.k0 >= p.k) at.k0 = 0, ++at.seg;
+    };
+    auto fetch = [&](auto S) __attribute__((always_inline)) {
+      ra.template fetch<decltype(S)::value>(f.seg * p.a_sk * SZ, f.k0, p.k);
+      rb.template fetch<decltype(S)::value>(f.seg * p.b_sk * SZ, f.k0, p.k);
+      next(f);
+      asm volatile("" ::: "memory");  // requests stay in this order
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto slab = [&](auto S) __attribute__((always_inline)) {
+      ra.template store<decltype(S)::value>(mine, 0, lane, w.k0, p.k);
+      rb.template store<decltype(S)::value>(mine + DA::BYTES, 0, lane, w.k0, p.k);
+      next(w);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      read(0);
+      fetch(S);
       multiply();
+    };
+    constexpr auto ring = std::make_integer_sequence<int, kRegDepth>{};
+    if (n > 0) {
+      [&]<int... S>(std::integer_sequence<int, S...>) { (fetch(std::integral_constant<int, S>{}), ...); }(ring);
+      int i = 0;
+      for (; i + kRegDepth <= n; i += kRegDepth)
+        [&]<int... S>(std::integer_sequence<int, S...>) { (slab(std::integral_constant<int, S>{}), ...); }(ring);
+      [&]<int... S>(std::integer_sequence<int, S...>) {
+        ((i + S < n ? slab(std::integral_constant<int, S>{}) : (void)0), ...);
+      }(ring);
     }
-  for (int s = 0; i < n; ++i) {
-    if (i + NST <= n)
-      asm volatile("s_waitcnt vmcnt(%0)" : : "n"((NST - 1) * NI) : "memory");
-    else
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    read(s);
-    if (i + NST < n) issue(s);
-    multiply();
-    s = s + 1 == NST ? 0 : s + 1;
+  } else {
+    DA da;
+    DB db;
+    da.init(p.lda, m0, p.m, 0, lane);
+    db.init(p.ldb, n0, p.n, 0, lane);
+    const char* ca = DA::slab_base(A, p.lda, m0) + seg * p.a_sk * SZ + in_seg * step_a;
+    const char* cb = DB::slab_base(B, p.ldb, n0) + seg * p.b_sk * SZ + in_seg * step_b;
+    int left = nk_seg - in_seg;  // slabs left in the K segment, the next one included
+    const bool tail = p.k % BK != 0;
+    const unsigned lds_mine = (unsigned)(uintptr_t)(lptr_t)lds + (unsigned)(wave * (NST * STAGE));
+    auto issue = [&](int stage) __attribute__((always_inline)) {
+      const unsigned at = lds_mine + (unsigned)(stage * STAGE);
+      if (left != 1 || !tail) {
+        da.template issue<false>(at, 0, ca, 0, 0);
+        db.template issue<false>(at + DA::BYTES, 0, cb, 0, 0);
+      } else {
+        da.template issue<true>(at, 0, ca, (nk_seg - 1) * BK, p.k);
+        db.template issue<true>(at + DA::BYTES, 0, cb, (nk_seg - 1) * BK, p.k);
+      }
+      const bool more = left != 1;
+      ca += more ? step_a : last_a;
+      cb += more ? step_b : last_b;
+      left = more ? left - 1 : nk_seg;
+    };
+#pragma unroll
+    for (int s = 0; s < NST; ++s)
+      if (s < n) issue(s);
+    int i = 0;
+    for (; i + 2 * NST <= n; i += NST)
+#pragma unroll
+      for (int s = 0; s < NST; ++s) {
+        asm volatile("s_waitcnt vmcnt(%0)" : : "n"((NST - 1) * NI) : "memory");
+        read(s);
+        issue(s);
+        multiply();
+      }
+    for (int s = 0; i < n; ++i) {
+      if (i + NST <= n)
+        asm volatile("s_waitcnt vmcnt(%0)" : : "n"((NST - 1) * NI) : "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      read(s);
+      if (i + NST < n) issue(s);
+      multiply();
+      s = s + 1 == NST ? 0 : s + 1;
+    }
   }
 
   __syncthreads();  // nobody reads slabs any more, and no load is on its way
@@ -143,30 +190,41 @@ __global__ __launch_bounds__(512) void gemm_kwaves_kernel(GemmArgs p) {
     *dst = from_f32<T>((p.flags & RTP_GEMM_ROWSUM_ACCUM) ? to_f32(*dst) + v : v);
   }
   __syncthreads();
-  if (tid >= 128) return;  // a thread finishes eight columns of a row
-  if (p.sgd_master != nullptr)
+  if (tid >= 128) return;  // a thread finishes eight outputs
+  if (RAG && !(REG && p.vec_c))
+    finish_tile_ragged<T, 32, 32, 128>(p, ct, m0, n0, tid, grp, zo, zi);
+  else if (p.sgd_master != nullptr)
     finish_tile_sgd<T, 32, 32, 128>(p, ct, m0, n0, tid, grp, zo, zi);
   else
     finish_tile<T, 32, 32, 128>(p, ct, m0, n0, tid, grp, zo, zi);
 }
 
-template <typename T>
+template <typename T, bool REG, bool RAG>
 static void launch_layouts(hipStream_t s, const GemmArgs& a, bool akc, bool bkc, dim3 grid) {
   if (akc && bkc)
-    hipLaunchKernelGGL((gemm_kwaves_kernel<T, true, true>), grid, dim3(512), 0, s, a);
+    hipLaunchKernelGGL((gemm_kwaves_kernel<T, true, true, REG, RAG>), grid, dim3(512), 0, s, a);
   else if (akc)
-    hipLaunchKernelGGL((gemm_kwaves_kernel<T, true, false>), grid, dim3(512), 0, s, a);
+    hipLaunchKernelGGL((gemm_kwaves_kernel<T, true, false, REG, RAG>), grid, dim3(512), 0, s, a);
   else if (bkc)
-    hipLaunchKernelGGL((gemm_kwaves_kernel<T, false, true>), grid, dim3(512), 0, s, a);
+    hipLaunchKernelGGL((gemm_kwaves_kernel<T, false, true, REG, RAG>), grid, dim3(512), 0, s, a);
   else
-    hipLaunchKernelGGL((gemm_kwaves_kernel<T, false, false>), grid, dim3(512), 0, s, a);
+    hipLaunchKernelGGL((gemm_kwaves_kernel<T, false, false, REG, RAG>), grid, dim3(512), 0, s, a);
+}
+template <typename T>
+static void launch_kind(hipStream_t s, const GemmArgs& a, bool akc, bool bkc, bool direct, dim3 grid) {
+  if (!direct)
+    launch_layouts<T, true, true>(s, a, akc, bkc, grid);
+  else if (!a.vec_c)
+    launch_layouts<T, false, true>(s, a, akc, bkc, grid);
+  else
+    launch_layouts<T, false, false>(s, a, akc, bkc, grid);
 }
 
-int launch_kwaves(hipStream_t s, const GemmArgs& a, bool bf16, bool akc, bool bkc, dim3 grid) {
+int launch_kwaves(hipStream_t s, const GemmArgs& a, bool bf16, bool akc, bool bkc, bool direct, dim3 grid) {
   if (bf16)
-    launch_layouts<bf16_t>(s, a, akc, bkc, grid);
+    launch_kind<bf16_t>(s, a, akc, bkc, direct, grid);
   else
-    launch_layouts<float>(s, a, akc, bkc, grid);
+    launch_kind<float>(s, a, akc, bkc, direct, grid);
   RTP_LAUNCH_CHECK();
   return RTP_OK;
 }

@@ -772,12 +772,110 @@ __device__ __forceinline__ Frag<T> read_frag_dma(const char* st, int rowbase, in
   return u.f;
 }
 
+// A 16-byte vector shifted down by `n` elements, zeros moving in from the top: what a vector that was read `n` elements
+// before its place (to stay inside the operand) has to undergo.
+template <typename T>
+__device__ __forceinline__ uint4 shift_down(uint4 q, int n) {
+  constexpr int PER = 4 / (int)sizeof(T);  // elements per word
+  const int w = n / PER;
+  const unsigned d[4] = {q.x, q.y, q.z, q.w};
+  unsigned r[5];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    r[i] = 0u;
+#pragma unroll
+    for (int j = i; j < 4; ++j) r[i] = w == j - i ? d[j] : r[i];
+  }
+  r[4] = 0u;
+  if (PER == 2) {
+    const unsigned odd = (n & 1) * 16u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = odd ? (r[i] >> 16) | (r[i + 1] << 16) : r[i];
+  }
+  return make_uint4(r[0], r[1], r[2], r[3]);
+}
+
+// The loader for operands the direct-to-LDS loads cannot take: rows, extents or base addresses that are no multiples of 16
+// bytes (a 1001-class head, shards of odd size).  Vectors are read with unaligned 16-byte loads into registers, kRegDepth
+// slabs ahead, and written to the stage in the layout DmaOperand leaves there.  A vector that would reach beyond its row (or k
+// line) is read further down, inside it, and shifted into place; this is decided per vector without a branch, and
+// the shift only runs in slabs and tiles that have such vectors.  Needs rows (k lines) of at least one vector.
+// Bound by the rate of unaligned vector loads: 25 - 28 bytes a clock and CU from the L1 against 56 for aligned ones.  A layer of
+// 992 x 1001 x 2048 (bf16, 8 shards, forward + both gradients): 54 us, 185 us with the guarded scalar loads; 4096^3 with
+// one extent odd 180 - 290 us.
+constexpr int kRegDepth = 3;
+template <typename T, int R, bool KC, int NL, int SB>
+struct RegOperand {
+  using D = DmaOperand<T, R, KC, NL, SB>;
+  static constexpr int VEC = D::VEC, NI = D::NI, BYTES = D::BYTES;
+  typedef unsigned vec_t __attribute__((ext_vector_type(4), aligned(2)));  // global loads take any alignment
+  const char* base;  // the operand's element 0 (K-contiguous: of row row0)
+  long ldb;          // leading dimension in bytes
+  unsigned ofs[NI];  // K-contiguous: of the lane's row;  else of the lane's rows inside a k line
+  int koff[NI];      // k of the vector inside its slab
+  int shift[NI];     // !KC: elements the vector was read early
+  bool edge;         // !KC: the tile has such vectors
+  uint4 val[kRegDepth][NI];
+
+  __device__ __forceinline__ void init(const T* x, long ld, int row0, int rows, int lw, int lane) {
+    ldb = ld * (long)sizeof(T);
+    base = reinterpret_cast<const char*>(KC ? x + (long)row0 * ld : x);
+    edge = !KC && row0 + R > rows;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int j = lw * NI + i;
+      if (KC) {
+        constexpr int LPR = SB / 16;
+        const int row = j * (64 / LPR) + lane / LPR;
+        const int rr = row0 + row < rows ? row : rows - 1 - row0;
+        ofs[i] = (unsigned)(rr * ldb);
+        koff[i] = ((lane % LPR) ^ kc_swizzle<SB>(row)) * VEC;
+        shift[i] = 0;
+      } else {
+        const int byte = lane * 16;
+        koff[i] = j * (1024 / D::LINE) + byte / D::LINE;
+        const int r = row0 + (((byte % D::LINE) >> 4) ^ rc_swizzle<T, R>(koff[i])) * VEC;
+        const int start = min(r, rows - VEC);
+        ofs[i] = (unsigned)(start * (int)sizeof(T));
+        shift[i] = r - start;
+      }
+    }
+  }
+  // request the slab whose first k is k0 (in a segment that starts seg bytes from the operand's base)
+  template <int S>
+  __device__ __forceinline__ void fetch(long seg, int k0, int kdim) {
+    const char* b = base + seg + (KC ? 0 : (long)k0 * ldb);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const unsigned o = KC ? ofs[i] + (unsigned)(min(k0 + koff[i], kdim - VEC) * (int)sizeof(T))
+                            : ofs[i] + (unsigned)(min(koff[i], kdim - 1 - k0) * ldb);
+      const vec_t v = *reinterpret_cast<const vec_t*>(b + o);
+      val[S][i] = make_uint4(v.x, v.y, v.z, v.w);
+    }
+  }
+  template <int S>
+  __device__ __forceinline__ void store(char* stage, int lw, int lane, int k0, int kdim) {
+    const bool tail = k0 + D::BK_ > kdim;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      uint4 q = val[S][i];
+      if (KC) {
+        if (tail) q = shift_down<T>(q, min(max(k0 + koff[i] - (kdim - VEC), 0), VEC));
+      } else {
+        if (edge) q = shift_down<T>(q, min(shift[i], VEC));
+        if (tail && k0 + koff[i] >= kdim) q = make_uint4(0u, 0u, 0u, 0u);
+      }
+      *reinterpret_cast<uint4*>(stage + (lw * NI + i) * 1024 + lane * 16) = q;
+    }
+  }
+};
+
 // The fp32 products of gemm_split.hip, in tiles of bm (128 or 64) x 64; ragged: an operand is not vector-aligned.
 int launch_split(hipStream_t s, const GemmArgs& a, bool akc, bool bkc, int bm, bool ragged, dim3 grid);
 
 // Many tiles of 128 x 128 over a K slab or two (gemm_shortk.hip).
 int launch_shortk(hipStream_t s, const GemmArgs& a, bool bf16, bool akc, bool bkc, dim3 grid);
-// Few tiles of 32 x 32, the contraction over the waves (gemm_kwaves.hip).
-int launch_kwaves(hipStream_t s, const GemmArgs& a, bool bf16, bool akc, bool bkc, dim3 grid);
+// Few tiles of 32 x 32, the contraction over the waves (gemm_kwaves.hip); direct: vector-aligned operands.
+int launch_kwaves(hipStream_t s, const GemmArgs& a, bool bf16, bool akc, bool bkc, bool direct, dim3 grid);
 
 }  // namespace rtp

@@ -31,15 +31,19 @@ def _bound(dtype, steps, size, ref):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("akc,bkc", LAYOUTS)
+# aligned; aligned but for the output; odd (with slabs and rounds of slabs that end anywhere)
 @pytest.mark.parametrize("m,n,k", [(8, 64, 512), (32, 32, 520), (40, 24, 1024), (64, 256, 1032), (136, 72, 2056), (8, 8, 4104),
-                                   (24, 1000, 776)])
+                                   (24, 1000, 776), (36, 68, 520), (40, 12, 2048), (33, 65, 513), (9, 31, 1027), (70, 101, 2055),
+                                   (31, 8, 4099)])
 @pytest.mark.parametrize("ksegs,groups", [(1, 1), (3, 2)])
 def test_edges(dtype, akc, bkc, m, n, k, ksegs, groups):
+    pad = 8 if k % 8 == 0 else 7
+    if dtype == torch.float32 and not akc and not bkc and pad == 7:
+        pytest.skip("unaligned row-contiguous fp32 operands have a kernel of their own")
     gen = torch.Generator().manual_seed(m + n + k)
     a = torch.randn(ksegs, groups, m, k, generator=gen).to(dtype)
     b = torch.randn(ksegs, groups, n, k, generator=gen).to(dtype)
-    # NaN behind the last row of each matrix: nothing of it may reach a result
-    pad = 8
+    # NaN behind the last row and column of each matrix: nothing of it may reach a result
     A = torch.full((ksegs, groups, m, k + pad) if akc else (ksegs, groups, k, m + pad), float("nan"), dtype=dtype)
     B = torch.full((ksegs, groups, n, k + pad) if bkc else (ksegs, groups, k, n + pad), float("nan"), dtype=dtype)
     A[..., :k if akc else m] = a if akc else a.transpose(2, 3)

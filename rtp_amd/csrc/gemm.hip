@@ -1471,6 +1471,12 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   // With these two numbers it is taken on none of them where another shape is more than 1 % faster, and on 25 more than with
   // 1400 and 9000 ns: 4096 x 6144 x 2048 121 -> 113 us, 8192 x 8192 x 256 98 -> 80, 8 of 3072 x 1024 x 768 72 -> 59.
   static const double fixed_ns[kNumShapes] = {3000.0, 3000.0, 3000.0, 3000.0, 3000.0, 5000.0, 3000.0};
+  // The two tiles for operands or outputs of any alignment, 64 x 64 and 128 x 128: the element-wise epilogue makes the larger one's
+  // share outside the loop 14.5 us, the register loaders make a slab take twice as long.  Measured on 16 odd shapes x 3 layouts
+  // with either tile forced; with the prices above, 128 x 128 was taken where 64 x 64 is ahead: us, bf16 3864 x 321 x 201 17.4 -> 11.9,
+  // 500 x 3001 x 1000 23.2 -> 19.8, 4001 x 1025 x 33 29.4 -> 20.2, 8 of 1001 x 256 x 992 (weight gradient) 24.5 -> 21.3; fp32 3222 x
+  // 4321 x 137 94 -> 80.  Where it is behind, 2001 x 2003 x 2005 39 against 54, it is not taken.
+  static const double odd_slab_ns[2][2] = {{330.0, 750.0}, {480.0, 2100.0}}, odd_fixed_ns[2] = {3600.0, 14500.0};
   static const int slab_bytes[kNumShapes] = {128, 128, 128, 128, 128, 128, 128};
   const bool vec = direct && a.vec_c;  // else the kernels for operands of any alignment
   int shape = 3;  // 64 x 64 unless the model finds something cheaper
@@ -1494,7 +1500,8 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
     if (kShapes[i].bn > 64 && kShapes[i].bn > ceil_div(d->n, 64) * 64) continue;
     const int64_t tiles = ceil_div(d->m, kShapes[i].bm) * ceil_div(d->n, kShapes[i].bn) * nz;
     const double nslabs = (double)ceil_div(d->k * (int64_t)sizeof(T), slab_bytes[i]) * (double)d->ksegs;
-    const double cost = (double)ceil_div(tiles, 256) * (nslabs * slab_ns[i] + fixed_ns[i]);
+    const double cost = (double)ceil_div(tiles, 256) *
+                        (vec ? nslabs * slab_ns[i] + fixed_ns[i] : nslabs * odd_slab_ns[sizeof(T) == 4][i == 1] + odd_fixed_ns[i == 1]);
     if (best == 0.0 || cost < best || i == forced) {
       best = i == forced ? -1.0 : cost;
       shape = i;

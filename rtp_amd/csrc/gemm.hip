@@ -1403,7 +1403,7 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   }
   // Few tiles, whatever the layout: see gemm_kwaves.hip.  256 tiles of 32 x 32 are one workgroup a CU, and up to there it is ahead at
   // every contraction from 256 on (measured in a replayed graph on 70 shapes x 3 layouts x 2 types; bf16 1.1 - 2.5 times, fp32 1.5 - 2.3).
-  // From 257 on some CU has two and only fp32 with K of 768 and more gains, up to 512.  us, before -> this:
+  // From 257 on some CU has two and only fp32 with K of 768 and more gains, up to 512 (where 64 x 32, below, does not fit).  us, before -> this:
   // 256 tiles bf16 64 x 4096, K = 512 5.7 -> 4.6, 4096 19.2 -> 10.3; 288 tiles 384 x 768, K = 256 5.2 -> 6.7, 1024 7.6 -> 8.7, 2048
   // 12.1 -> 11.7; 512 tiles fp32 512 x 1024, K = 384 10.8 -> 12.6, 1024 19.6 -> 18.1; 768 tiles 512 x 1536, K = 2048 36 -> 44.
   // Operands that are not vector-aligned, 12 shapes: bf16 255 x 1023 x 3333 24.0 -> 17.6, 31 x 2049 x 515 8.6 -> 8.2, one of 25 behind
@@ -1412,17 +1412,23 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   // backward pass sees the unit at all, and of 16 M such sums (1000 tokens, 8 experts of 768 x 8064) some ten are that near.
   const bool relu = d->flags & RTP_GEMM_RELU;
   const int64_t tiles32 = ceil_div(d->m, 32) * ceil_div(d->n, 32) * nz, k_all = d->k * d->ksegs;
-  if (fast && !relu && !d->xent_mode && nz < 65536 && k_all >= 256 &&
-      !(sizeof(T) == 4 && !direct && !akc && !bkc) && tiles32 <= (sizeof(T) == 4 && k_all >= 768 ? 512 : 256)) {
-    a.tiles_m = (int)ceil_div(d->m, 32);
+  // With tiles of 64 x 32 twice as many outputs are one workgroup a CU: in fp32 ahead at any contraction (1.05 - 1.46 times on 24 shapes,
+  // two of 72 behind by 1 and 3 %), in bf16 only at long ones, with operands that lie alike (K >= 2048: 1.0 - 1.2, unaligned weight gradients
+  // 1.4 - 1.8; K = 512 0.83 - 0.98; the input gradient's layout 0.95 - 1.09).
+  const int64_t tiles64 = ceil_div(d->m, 64) * ceil_div(d->n, 32) * nz;
+  const int kw_bm = tiles32 <= 256                                                                 ? 32
+                    : tiles64 <= 256 && (sizeof(T) == 4 || (k_all >= 2048 && akc == bkc))          ? 64
+                    : sizeof(T) == 4 && k_all >= 768 && tiles32 <= 512                             ? 32
+                                                                                                   : 0;
+  if (fast && !relu && !d->xent_mode && nz < 65536 && k_all >= 256 && !(sizeof(T) == 4 && !direct && !akc && !bkc) && kw_bm != 0) {
+    a.tiles_m = (int)ceil_div(d->m, kw_bm);
     a.tiles_n = (int)ceil_div(d->n, 32);
-    static const char* const names[2][2][2] = {
-        {{"gemm_f32_32x32_kwaves_rc_rc", "gemm_f32_32x32_kwaves_rc_kc"}, {"gemm_f32_32x32_kwaves_kc_rc", "gemm_f32_32x32_kwaves_kc_kc"}},
-        {{"gemm_bf16_32x32_kwaves_rc_rc", "gemm_bf16_32x32_kwaves_rc_kc"}, {"gemm_bf16_32x32_kwaves_kc_rc", "gemm_bf16_32x32_kwaves_kc_kc"}}};
+    static const char* const names[2][2][2] = {{{"gemm_f32_kwaves_rc_rc", "gemm_f32_kwaves_rc_kc"}, {"gemm_f32_kwaves_kc_rc", "gemm_f32_kwaves_kc_kc"}},
+                                               {{"gemm_bf16_kwaves_rc_rc", "gemm_bf16_kwaves_rc_kc"}, {"gemm_bf16_kwaves_kc_rc", "gemm_bf16_kwaves_kc_kc"}}};
     const double mn_ = (double)d->m * (double)d->n * (double)nz, kk_ = (double)d->k * (double)d->ksegs;
     ProfileScope prof(s, names[sizeof(T) == 2][akc][bkc], 2.0 * mn_ * kk_,
                       ((double)d->m + (double)d->n) * kk_ * nz * sizeof(T) + mn_ * sizeof(T));
-    return launch_kwaves(s, a, sizeof(T) == 2, akc, bkc, direct, dim3((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nz));
+    return launch_kwaves(s, a, kw_bm, sizeof(T) == 2, akc, bkc, direct, dim3((unsigned)(a.tiles_m * a.tiles_n), (unsigned)nz));
   }
   // Many outputs, at most two K slabs: see gemm_shortk.hip.  From 384 of its tiles on it is ahead, in every layout; with 256, one
   // workgroup a CU, it is behind (us, before -> this, bf16: 2048 x 2048 x 64 7.0 -> 7.0, 1024 x 4096 x 96 7.6 -> 8.1, 4096 x 1536 x 32

@@ -14,19 +14,21 @@ namespace rtp {
 // 18.9 -> 9.9, 32 x 1024 x 8192 31.1 -> 13.9, input gradient 64 x 4096 x 4096 19.5 -> 14.7; fp32 (split tiles before) 64 x 1024 x 1024
 // 18.4 -> 8.7, 64 x 4096 x 4096 57.7 -> 26.7.  Eight short sums: error against fp64 below that of one long one.
 //
+// MT = 2: tiles of 64 x 32, slabs of 64 bytes a row and three stages, where 32 x 32 would be two workgroups a CU (fp32 256 x 2048 x 512
+// 13.1 -> 11.0 us, 100 x 3072 x 384 10.5 -> 8.2; bf16 100 x 3072 x 8192 32.6 -> 27.3, weight gradient 250 x 2048 x 4096 37.6 -> 24.5).
 // REG: operands of any alignment, through registers into the wave's LDS, three slabs ahead (bf16 255 x 1023 x 3333 24.0 -> 17.6 us,
 // 64 x 1001 x 2048 10.7 -> 7.8, its weight gradient 22.5 -> 14.4; fp32 255 x 1023 x 3333 65.6 -> 28.5, 1 x 1303 x 1364 29.4 -> 11.7); RAG: the element-wise epilogue (an output,
 // addend or mask that is not vector-aligned).
-template <typename T, bool AKC, bool BKC, bool REG, bool RAG>
+template <typename T, int MT, bool AKC, bool BKC, bool REG, bool RAG>
 __global__ __launch_bounds__(512) void gemm_kwaves_kernel(GemmArgs p) {
-  constexpr int SB = 128, NST = 2;  // bytes of a slab's row, stages per wave
-  using DA = DmaOperand<T, 32, AKC, 1, SB>;
+  constexpr int BM = 32 * MT, SB = MT == 1 ? 128 : 64, NST = MT == 1 ? 2 : 3;  // bytes of a slab's row, stages per wave
+  using DA = DmaOperand<T, BM, AKC, 1, SB>;
   using DB = DmaOperand<T, 32, BKC, 1, SB>;
   constexpr int WAVES = 8, BK = SB / (int)sizeof(T), KS = BK / (2 * DA::VEC);
   constexpr int STAGE = DA::BYTES + DB::BYTES, NI = DA::NI + DB::NI;
-  constexpr int PITCH = 33, PART = WAVES * 32 * PITCH * 4;
+  constexpr int PITCH = 33, PART = WAVES * BM * PITCH * 4;
   static_assert((NST - 1) * NI < 64, "vmcnt is a 6-bit counter");
-  static_assert(WAVES * NST * STAGE <= 160 * 1024 && PART + 32 * 36 * 4 + WAVES * 32 * 4 <= WAVES * NST * STAGE,
+  static_assert(WAVES * NST * STAGE <= 160 * 1024 && PART + BM * 36 * 4 + WAVES * BM * 4 <= WAVES * NST * STAGE,
                 "160 KiB of LDS; the sums reuse the slabs' memory");
   __shared__ __attribute__((aligned(1024))) char lds[WAVES * NST * STAGE];
 
@@ -36,7 +38,7 @@ __global__ __launch_bounds__(512) void gemm_kwaves_kernel(GemmArgs p) {
   unsigned bid = blockIdx.x;
   const unsigned nb = gridDim.x;
   if ((nb & 7) == 0) bid = (bid & 7) * (nb >> 3) + (bid >> 3);
-  const int n0 = (int)(bid / (unsigned)p.tiles_m) * 32, m0 = (int)(bid % (unsigned)p.tiles_m) * 32;
+  const int n0 = (int)(bid / (unsigned)p.tiles_m) * 32, m0 = (int)(bid % (unsigned)p.tiles_m) * BM;
   const int grp = blockIdx.y / p.batch, zb = blockIdx.y % p.batch;
   const long zo = zb / p.zdiv, zi = zb % p.zdiv;
 
@@ -52,16 +54,21 @@ __global__ __launch_bounds__(512) void gemm_kwaves_kernel(GemmArgs p) {
   const int seg = first / nk_seg, in_seg = first - seg * nk_seg;
   char* const mine = lds + wave * (NST * STAGE);
 
-  f32x16 acc;
+  f32x16 acc[MT];
+  float rs[MT];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-  float rs = 0.0f;
+  for (int t = 0; t < MT; ++t) {
+    rs[t] = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[t][r] = 0.0f;
+  }
   const bool rowsum = p.a_rowsum != nullptr && n0 == 0;
-  Frag<T> fa[KS], fb[KS];
+  Frag<T> fa[MT][KS], fb[KS];
   auto read = [&](int stage) __attribute__((always_inline)) {
 #pragma unroll
     for (int q = 0; q < KS; ++q) {
-      fa[q] = read_frag_dma<T, 32, AKC, SB>(mine + stage * STAGE, 0, lane, q);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) fa[t][q] = read_frag_dma<T, BM, AKC, SB>(mine + stage * STAGE, 32 * t, lane, q);
       fb[q] = read_frag_dma<T, 32, BKC, SB>(mine + stage * STAGE + DA::BYTES, 0, lane, q);
     }
     // the stage is free when its reads have returned
@@ -71,14 +78,17 @@ __global__ __launch_bounds__(512) void gemm_kwaves_kernel(GemmArgs p) {
   auto multiply = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int q = 0; q < KS; ++q) {
-      mma(fa[q], fb[q], acc);
-      if (rowsum) rs = frag_sum(fa[q], rs);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        mma(fa[t][q], fb[q], acc[t]);
+        if (rowsum) rs[t] = frag_sum(fa[t][q], rs[t]);
+      }
     }
   };
 
   if constexpr (REG) {
     // slabs behind the wave's last one re-read it, so that the loop has no branch around a request
-    RegOperand<T, 32, AKC, 1, SB> ra;
+    RegOperand<T, BM, AKC, 1, SB> ra;
     RegOperand<T, 32, BKC, 1, SB> rb;
     ra.init(A, p.lda, m0, p.m, 0, lane);
     rb.init(B, p.ldb, n0, p.n, 0, lane);
@@ -166,65 +176,72 @@ __global__ __launch_bounds__(512) void gemm_kwaves_kernel(GemmArgs p) {
   }
 
   __syncthreads();  // nobody reads slabs any more, and no load is on its way
-  float(*part)[32][PITCH] = reinterpret_cast<float(*)[32][PITCH]>(lds);
+  float(*part)[BM][PITCH] = reinterpret_cast<float(*)[BM][PITCH]>(lds);
   float* ct = reinterpret_cast<float*>(lds + PART);
-  float* sums = ct + 32 * 36;
+  float* sums = ct + BM * 36;
 #pragma unroll
-  for (int r = 0; r < 16; ++r) part[wave][8 * (r >> 2) + 4 * g + (r & 3)][li] = acc[r];
-  const float both = rs + __shfl_xor(rs, 32, kWave);
-  if (g == 0) sums[wave * 32 + li] = both;
+  for (int t = 0; t < MT; ++t) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) part[wave][32 * t + 8 * (r >> 2) + 4 * g + (r & 3)][li] = acc[t][r];
+    const float both = rs[t] + __shfl_xor(rs[t], 32, kWave);
+    if (g == 0) sums[wave * BM + 32 * t + li] = both;
+  }
   __syncthreads();
 #pragma unroll
-  for (int e = 0; e < 2; ++e) {
+  for (int e = 0; e < 2 * MT; ++e) {
     const int row = (tid >> 5) + 16 * e;
     float v = 0.0f;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) v += part[w][row][li];
     ct[row * 36 + li] = v;
   }
-  if (rowsum && tid < 32 && m0 + tid < p.m) {
+  if (rowsum && tid < BM && m0 + tid < p.m) {
     float v = 0.0f;
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) v += sums[w * 32 + tid];
+    for (int w = 0; w < WAVES; ++w) v += sums[w * BM + tid];
     T* dst = reinterpret_cast<T*>(p.a_rowsum) + grp * p.rowsum_sg + m0 + tid;
     *dst = from_f32<T>((p.flags & RTP_GEMM_ROWSUM_ACCUM) ? to_f32(*dst) + v : v);
   }
   __syncthreads();
-  if (tid >= 128) return;  // a thread finishes eight outputs
+  if (tid >= 128 * MT) return;  // a thread finishes eight outputs
   if (RAG && !(REG && p.vec_c))
-    finish_tile_ragged<T, 32, 32, 128>(p, ct, m0, n0, tid, grp, zo, zi);
+    finish_tile_ragged<T, BM, 32, 128 * MT>(p, ct, m0, n0, tid, grp, zo, zi);
   else if (p.sgd_master != nullptr)
-    finish_tile_sgd<T, 32, 32, 128>(p, ct, m0, n0, tid, grp, zo, zi);
+    finish_tile_sgd<T, BM, 32, 128 * MT>(p, ct, m0, n0, tid, grp, zo, zi);
   else
-    finish_tile<T, 32, 32, 128>(p, ct, m0, n0, tid, grp, zo, zi);
+    finish_tile<T, BM, 32, 128 * MT>(p, ct, m0, n0, tid, grp, zo, zi);
 }
 
-template <typename T, bool REG, bool RAG>
+template <typename T, int MT, bool REG, bool RAG>
 static void launch_layouts(hipStream_t s, const GemmArgs& a, bool akc, bool bkc, dim3 grid) {
   if (akc && bkc)
-    hipLaunchKernelGGL((gemm_kwaves_kernel<T, true, true, REG, RAG>), grid, dim3(512), 0, s, a);
+    hipLaunchKernelGGL((gemm_kwaves_kernel<T, MT, true, true, REG, RAG>), grid, dim3(512), 0, s, a);
   else if (akc)
-    hipLaunchKernelGGL((gemm_kwaves_kernel<T, true, false, REG, RAG>), grid, dim3(512), 0, s, a);
+    hipLaunchKernelGGL((gemm_kwaves_kernel<T, MT, true, false, REG, RAG>), grid, dim3(512), 0, s, a);
   else if (bkc)
-    hipLaunchKernelGGL((gemm_kwaves_kernel<T, false, true, REG, RAG>), grid, dim3(512), 0, s, a);
+    hipLaunchKernelGGL((gemm_kwaves_kernel<T, MT, false, true, REG, RAG>), grid, dim3(512), 0, s, a);
   else
-    hipLaunchKernelGGL((gemm_kwaves_kernel<T, false, false, REG, RAG>), grid, dim3(512), 0, s, a);
+    hipLaunchKernelGGL((gemm_kwaves_kernel<T, MT, false, false, REG, RAG>), grid, dim3(512), 0, s, a);
 }
-template <typename T>
+template <typename T, int MT>
 static void launch_kind(hipStream_t s, const GemmArgs& a, bool akc, bool bkc, bool direct, dim3 grid) {
   if (!direct)
-    launch_layouts<T, true, true>(s, a, akc, bkc, grid);
+    launch_layouts<T, MT, true, true>(s, a, akc, bkc, grid);
   else if (!a.vec_c)
-    launch_layouts<T, false, true>(s, a, akc, bkc, grid);
+    launch_layouts<T, MT, false, true>(s, a, akc, bkc, grid);
   else
-    launch_layouts<T, false, false>(s, a, akc, bkc, grid);
+    launch_layouts<T, MT, false, false>(s, a, akc, bkc, grid);
 }
 
-int launch_kwaves(hipStream_t s, const GemmArgs& a, bool bf16, bool akc, bool bkc, bool direct, dim3 grid) {
-  if (bf16)
-    launch_kind<bf16_t>(s, a, akc, bkc, direct, grid);
+int launch_kwaves(hipStream_t s, const GemmArgs& a, int bm, bool bf16, bool akc, bool bkc, bool direct, dim3 grid) {
+  if (bf16 && bm == 32)
+    launch_kind<bf16_t, 1>(s, a, akc, bkc, direct, grid);
+  else if (bf16)
+    launch_kind<bf16_t, 2>(s, a, akc, bkc, direct, grid);
+  else if (bm == 32)
+    launch_kind<float, 1>(s, a, akc, bkc, direct, grid);
   else
-    launch_kind<float>(s, a, akc, bkc, direct, grid);
+    launch_kind<float, 2>(s, a, akc, bkc, direct, grid);
   RTP_LAUNCH_CHECK();
   return RTP_OK;
 }

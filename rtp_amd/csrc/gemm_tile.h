@@ -875,7 +875,7 @@ int launch_split(hipStream_t s, const GemmArgs& a, bool akc, bool bkc, int bm, b
 
 // Many tiles of 128 x 128 over a K slab or two (gemm_shortk.hip).
 int launch_shortk(hipStream_t s, const GemmArgs& a, bool bf16, bool akc, bool bkc, dim3 grid);
-// Few tiles of 32 x 32, the contraction over the waves (gemm_kwaves.hip); direct: vector-aligned operands.
-int launch_kwaves(hipStream_t s, const GemmArgs& a, bool bf16, bool akc, bool bkc, bool direct, dim3 grid);
+// Few tiles of bm (32 or 64) x 32, the contraction over the waves (gemm_kwaves.hip); direct: vector-aligned operands.
+int launch_kwaves(hipStream_t s, const GemmArgs& a, int bm, bool bf16, bool akc, bool bkc, bool direct, dim3 grid);
 
 }  // namespace rtp

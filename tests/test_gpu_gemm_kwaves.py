@@ -36,7 +36,7 @@ def _bound(dtype, steps, size, ref):
                                    (24, 1000, 776), (36, 68, 520), (40, 12, 2048), (33, 65, 513), (9, 31, 1027), (70, 101, 2055),
                                    (31, 8, 4099)])
 @pytest.mark.parametrize("ksegs,groups", [(1, 1), (3, 2)])
-def test_edges(dtype, akc, bkc, m, n, k, ksegs, groups):
+def test_edges(dtype, akc, bkc, m, n, k, ksegs, groups, taken=True):
     pad = 8 if k % 8 == 0 else 7
     if dtype == torch.float32 and not akc and not bkc and pad == 7:
         pytest.skip("unaligned row-contiguous fp32 operands have a kernel of their own")
@@ -51,7 +51,7 @@ def test_edges(dtype, akc, bkc, m, n, k, ksegs, groups):
     A, B = A.to(DEV), B.to(DEV)
     out = torch.full((groups, m, n), float("nan"), dtype=dtype, device=DEV)
     sums = torch.full((groups, m), float("nan"), dtype=dtype, device=DEV)
-    done = _run(dtype, A, B, m, n, k, akc, bkc, c_out=out.data_ptr(), lda=A.stride(2), ldb=B.stride(2), ldc=n, groups=groups,
+    done = _run(dtype, A, B, m, n, k, akc, bkc, taken=taken, c_out=out.data_ptr(), lda=A.stride(2), ldb=B.stride(2), ldc=n, groups=groups,
                 a_sg=A.stride(1), b_sg=B.stride(1), c_sg=m * n, ksegs=ksegs, a_sk=A.stride(0), b_sk=B.stride(0),
                 rowsum=None if akc else sums.data_ptr(), rowsum_sg=m)
     ref = (a.double() @ b.double().transpose(2, 3)).sum(0)
@@ -61,6 +61,14 @@ def test_edges(dtype, akc, bkc, m, n, k, ksegs, groups):
     if done:
         rows, size = a.double().sum((0, 3)), a.double().abs().sum((0, 3))
         assert ((sums.cpu().double() - rows).abs() <= _bound(dtype, ksegs * k, size, rows)).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("akc,bkc", LAYOUTS)
+# more than 256 tiles of 32 x 32 and at most 256 of 64 x 32: whole and ragged, the last 64 rows all there, half or a sliver
+@pytest.mark.parametrize("m,n,k", [(192, 1408, 2048), (264, 1032, 2056), (72, 2728, 2112), (100, 2101, 2051), (65, 2753, 2049)])
+def test_taller_tiles(dtype, akc, bkc, m, n, k):
+    test_edges(dtype, akc, bkc, m, n, k, 1, 1, taken=dtype == torch.float32 or akc == bkc)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

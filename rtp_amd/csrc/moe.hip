@@ -181,6 +181,102 @@ __global__ __launch_bounds__(kTok) void route_bwd_kernel(const float* gates, con
 
 // out[row,:] = x[token(row),:] (* weight of the choice that put the token there), zero if the slot is
 // empty.  One workgroup per (slot row, column chunk).
+// The row moves and the weights' gradient, 16 bytes per lane and access: VEC consecutive columns of a row.  A thread of the
+// moves is one vector of the flattened (row, vector) space, so narrow rows share a workgroup.  Bound by memory.  us, a column per lane
+// and access -> this, 4096 tokens, 8 experts, 2048 columns: bf16 dispatch 18.0 -> 11.6, with weights 21.5 -> 13.5, combine 17.2 -> 10.4,
+// the weights' gradient 13.9 -> 9.5; fp32 21.9 -> 20.4, 25.3 -> 22.5, 20.8 -> 17.5, 16.9 -> 17.8.  The kernels further down serve rows
+// that are not vector-aligned.
+template <typename T>
+struct alignas(16) RowVec {
+  static constexpr int N = 16 / (int)sizeof(T);
+  T e[N];
+};
+
+template <typename T>
+__global__ __launch_bounds__(256) void dispatch_vec_kernel(const T* x, long ld_x, const int* slot_token, const int* expert,
+                                                           const int* slot, const float* weight, int capacity, FastDiv nvec,
+                                                           unsigned total, T* out, long ld_out) {
+  typedef RowVec<T> V;
+  const unsigned id = blockIdx.x * 256 + threadIdx.x;
+  if (id >= total) return;
+  const unsigned row = fast_div(id, nvec), v = id - row * nvec.d;
+  const int tok = slot_token[row];
+  V q;
+  if (tok < 0) {
+#pragma unroll
+    for (int i = 0; i < V::N; ++i) q.e[i] = (T)0.0f;
+  } else {
+    q = reinterpret_cast<const V*>(x + (long)tok * ld_x)[v];
+    if (weight) {
+      const int e = (int)row / capacity, c0 = (int)row % capacity;
+      const int j = (expert[2 * tok] == e && slot[2 * tok] == c0 && weight[2 * tok] != 0.0f) ? 0 : 1;
+      const float w = weight[2 * tok + j];
+#pragma unroll
+      for (int i = 0; i < V::N; ++i) q.e[i] = from_f32<T>(w * to_f32(q.e[i]));
+    }
+  }
+  reinterpret_cast<V*>(out + (long)row * ld_out)[v] = q;
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void combine_vec_kernel(const T* y, long ld_y, const int* expert, const int* slot,
+                                                          const int* keep, const float* weight, long capacity, FastDiv nvec,
+                                                          unsigned total, T* out, long ld_out) {
+  typedef RowVec<T> V;
+  const unsigned id = blockIdx.x * 256 + threadIdx.x;
+  if (id >= total) return;
+  const unsigned s = fast_div(id, nvec), v = id - s * nvec.d;
+  const bool k1 = keep[2 * s], k2 = keep[2 * s + 1];
+  const float w1 = weight ? weight[2 * s] : 1.0f, w2 = weight ? weight[2 * s + 1] : 1.0f;
+  V a, b, q;
+  if (k1) a = reinterpret_cast<const V*>(y + ((long)expert[2 * s] * capacity + slot[2 * s]) * ld_y)[v];
+  if (k2) b = reinterpret_cast<const V*>(y + ((long)expert[2 * s + 1] * capacity + slot[2 * s + 1]) * ld_y)[v];
+#pragma unroll
+  for (int i = 0; i < V::N; ++i) {
+    float t = 0.0f;
+    if (k1) t += w1 * to_f32(a.e[i]);
+    if (k2) t += w2 * to_f32(b.e[i]);
+    q.e[i] = from_f32<T>(t);
+  }
+  reinterpret_cast<V*>(out + (long)s * ld_out)[v] = q;
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void combine_dweight_vec_kernel(const T* dout, long ld_dout, const T* y, long ld_y,
+                                                                  const int* expert, const int* slot, const int* keep, long S,
+                                                                  long capacity, int nvec, float* dweight) {
+  typedef RowVec<T> V;
+  const int lane = threadIdx.x & 63;
+  const long idx = (long)blockIdx.x * 4 + (threadIdx.x >> 6);  // = 2*s + j
+  if (idx >= 2 * S) return;
+  float acc = 0.0f;
+  if (keep[idx]) {
+    const V* a = reinterpret_cast<const V*>(dout + (idx >> 1) * ld_dout);
+    const V* b = reinterpret_cast<const V*>(y + ((long)expert[idx] * capacity + slot[idx]) * ld_y);
+    int v = lane;
+    for (; v + kWave < nvec; v += 2 * kWave) {
+      const V a0 = a[v], b0 = b[v], a1 = a[v + kWave], b1 = b[v + kWave];
+#pragma unroll
+      for (int i = 0; i < V::N; ++i) acc += to_f32(a0.e[i]) * to_f32(b0.e[i]);
+#pragma unroll
+      for (int i = 0; i < V::N; ++i) acc += to_f32(a1.e[i]) * to_f32(b1.e[i]);
+    }
+    if (v < nvec) {
+      const V a0 = a[v], b0 = b[v];
+#pragma unroll
+      for (int i = 0; i < V::N; ++i) acc += to_f32(a0.e[i]) * to_f32(b0.e[i]);
+    }
+  }
+  acc = wave_sum(acc);
+  if (lane == 0) dweight[idx] = acc;
+}
+
+// whether rows of `cols` elements of `esz` bytes at these addresses and leading dimensions are whole 16-byte vectors
+static bool row_vectors(size_t esz, int64_t cols, const void* a, int64_t ld_a, const void* b, int64_t ld_b) {
+  return ((uintptr_t)a | (uintptr_t)b | (uintptr_t)(cols * (int64_t)esz) | (uintptr_t)(ld_a * (int64_t)esz) |
+          (uintptr_t)(ld_b * (int64_t)esz)) % 16 == 0;
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void dispatch_kernel(const T* x, long ld_x, const int* slot_token,
                                                        const int* expert, const int* slot, const float* weight,
@@ -323,6 +419,21 @@ extern "C" int rtp_moe_dispatch(void* stream, int dtype, const void* x, int64_t 
   if (n_slots == 0 || cols == 0) return RTP_OK;
   dim3 grid((unsigned)n_slots, col_chunks(cols));
   ProfileScope prof((hipStream_t)stream, "moe_dispatch", 0.0, 2.0 * (double)n_slots * cols * (dtype == RTP_F32 ? 4 : 2));
+  const size_t esz = dtype == RTP_F32 ? 4 : 2;
+  const int64_t nvec = cols * (int64_t)esz / 16, total = n_slots * nvec;
+  if ((dtype == RTP_F32 || dtype == RTP_BF16) && row_vectors(esz, cols, x, ld_x, out, ld_out) && total < (1ll << 31) &&
+      capacity < (1ll << 31)) {
+    const dim3 vgrid((unsigned)ceil_div(total, 256));
+    const FastDiv d = make_fastdiv((unsigned)nvec);
+    if (dtype == RTP_F32)
+      hipLaunchKernelGGL(dispatch_vec_kernel<float>, vgrid, dim3(256), 0, (hipStream_t)stream, (const float*)x, (long)ld_x,
+                         slot_token, expert, slot, weight, (int)capacity, d, (unsigned)total, (float*)out, (long)ld_out);
+    else
+      hipLaunchKernelGGL(dispatch_vec_kernel<bf16_t>, vgrid, dim3(256), 0, (hipStream_t)stream, (const bf16_t*)x, (long)ld_x,
+                         slot_token, expert, slot, weight, (int)capacity, d, (unsigned)total, (bf16_t*)out, (long)ld_out);
+    RTP_LAUNCH_CHECK();
+    return RTP_OK;
+  }
 #define A_(T) (const T*)x, (long)ld_x, slot_token, expert, slot, weight, (long)capacity, (long)cols, (T*)out, (long)ld_out
   if (dtype == RTP_F32)
     hipLaunchKernelGGL(dispatch_kernel<float>, grid, dim3(256), 0, (hipStream_t)stream, A_(float));
@@ -344,6 +455,20 @@ extern "C" int rtp_moe_combine(void* stream, int dtype, const void* y, int64_t l
   if (s == 0 || cols == 0) return RTP_OK;
   dim3 grid((unsigned)s, col_chunks(cols));
   ProfileScope prof((hipStream_t)stream, "moe_combine", 4.0 * (double)s * cols, 3.0 * (double)s * cols * (dtype == RTP_F32 ? 4 : 2));
+  const size_t esz = dtype == RTP_F32 ? 4 : 2;
+  const int64_t nvec = cols * (int64_t)esz / 16, total = s * nvec;
+  if ((dtype == RTP_F32 || dtype == RTP_BF16) && row_vectors(esz, cols, y, ld_y, out, ld_out) && total < (1ll << 31)) {
+    const dim3 vgrid((unsigned)ceil_div(total, 256));
+    const FastDiv d = make_fastdiv((unsigned)nvec);
+    if (dtype == RTP_F32)
+      hipLaunchKernelGGL(combine_vec_kernel<float>, vgrid, dim3(256), 0, (hipStream_t)stream, (const float*)y, (long)ld_y,
+                         expert, slot, keep, weight, (long)capacity, d, (unsigned)total, (float*)out, (long)ld_out);
+    else
+      hipLaunchKernelGGL(combine_vec_kernel<bf16_t>, vgrid, dim3(256), 0, (hipStream_t)stream, (const bf16_t*)y, (long)ld_y,
+                         expert, slot, keep, weight, (long)capacity, d, (unsigned)total, (bf16_t*)out, (long)ld_out);
+    RTP_LAUNCH_CHECK();
+    return RTP_OK;
+  }
 #define A_(T) (const T*)y, (long)ld_y, expert, slot, keep, weight, (long)capacity, (long)cols, (T*)out, (long)ld_out
   if (dtype == RTP_F32)
     hipLaunchKernelGGL(combine_kernel<float>, grid, dim3(256), 0, (hipStream_t)stream, A_(float));
@@ -364,6 +489,18 @@ extern "C" int rtp_moe_combine_dweight(void* stream, int dtype, const void* dout
               "rtp_moe_combine_dweight: bad shape");
   if (s == 0) return RTP_OK;
   dim3 grid((unsigned)ceil_div(2 * s, 4));
+  const size_t esz = dtype == RTP_F32 ? 4 : 2;
+  const int64_t nvec = cols * (int64_t)esz / 16;
+  if ((dtype == RTP_F32 || dtype == RTP_BF16) && row_vectors(esz, cols, dout, ld_dout, y, ld_y) && nvec < (1ll << 30)) {
+    if (dtype == RTP_F32)
+      hipLaunchKernelGGL(combine_dweight_vec_kernel<float>, grid, dim3(256), 0, (hipStream_t)stream, (const float*)dout,
+                         (long)ld_dout, (const float*)y, (long)ld_y, expert, slot, keep, (long)s, (long)capacity, (int)nvec, dweight);
+    else
+      hipLaunchKernelGGL(combine_dweight_vec_kernel<bf16_t>, grid, dim3(256), 0, (hipStream_t)stream, (const bf16_t*)dout,
+                         (long)ld_dout, (const bf16_t*)y, (long)ld_y, expert, slot, keep, (long)s, (long)capacity, (int)nvec, dweight);
+    RTP_LAUNCH_CHECK();
+    return RTP_OK;
+  }
 #define A_(T) (const T*)dout, (long)ld_dout, (const T*)y, (long)ld_y, expert, slot, keep, (long)s, (long)capacity, (long)cols, dweight
   if (dtype == RTP_F32)
     hipLaunchKernelGGL(combine_dweight_kernel<float>, grid, dim3(256), 0, (hipStream_t)stream, A_(float));

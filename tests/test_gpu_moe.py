@@ -307,3 +307,51 @@ def test_moe_input_gradient_paths_meet_in_the_gate_kernel(dtype):
     layer(xc, noise=noise)
     layer.l_aux.backward()                                        # only the auxiliary loss: the outputs' grads are None
     assert xc.grad is not None and torch.isfinite(xc.grad).all() and float(xc.grad.abs().sum()) > 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tokens,cols,pad,offset", [(8, 8, 0, 0), (16, 520, 8, 8), (64, 2048, 0, 0), (64, 264, 0, 1), (24, 257, 3, 0)])
+def test_row_moves_at_any_alignment(dtype, tokens, cols, pad, offset):
+    """Dispatch, combine and the weights' gradient over rows that are whole vectors, padded, shifted by one element or of odd width,
+    against the same moves in torch: bit for bit, but for the order of a dot product's sum."""
+    from rtp_amd import ops
+    E = 8
+    gen = torch.Generator().manual_seed(tokens + cols)
+    r = ops.top2_route(torch.randn(tokens, E, generator=gen).to(DEV), torch.randn(tokens, E, generator=gen).to(DEV))
+    n_slots = E * r.capacity
+
+    def rows(n):
+        buf = torch.full((n * (cols + pad) + offset + 16,), 7.0, dtype=dtype, device=DEV)
+        view = buf[offset:offset + n * (cols + pad)].view(n, cols + pad)[:, :cols]
+        view.copy_(torch.randn(n, cols, generator=gen))
+        return buf, view
+
+    (_, x), (_, y), (_, dout) = rows(tokens), rows(n_slots), rows(tokens)
+    w = torch.rand(tokens, 2, generator=gen).to(DEV)
+    expert, slot, keep = r.expert.cpu().long(), r.slot.cpu().long(), r.keep.cpu().bool()
+    at = expert * r.capacity + slot
+    for weight in (None, w):
+        buf, out = rows(n_slots)
+        ops.moe_dispatch(x, r, out, weight)
+        want = torch.zeros(n_slots, cols, dtype=dtype)
+        for s in range(tokens):
+            for j in range(2):
+                if keep[s, j]:
+                    want[at[s, j]] = x[s].cpu() if weight is None else (weight[s, j].cpu() * x[s].cpu().float()).to(dtype)
+        assert torch.equal(out.cpu(), want)
+        assert pad == 0 or bool((buf[offset:offset + n_slots * (cols + pad)].view(n_slots, -1)[:, cols:] == 7.0).all())
+        _, out = rows(tokens)
+        ops.moe_combine(y, r, out, weight)
+        v = torch.zeros(tokens, cols, dtype=torch.float64)
+        for j in range(2):
+            k = keep[:, j].nonzero().flatten()
+            v[k] += (1.0 if weight is None else weight[k.to(DEV), j].cpu().double()[:, None]) * y[at[k, j].to(DEV)].cpu().double()
+        # two products and their sum, rounded once each, and the result's own rounding
+        tol = 3 * 2.0 ** -24 * 8 + (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24) * v.abs()
+        assert ((out.cpu().double() - v).abs() <= tol).all()
+    dw = ops.moe_combine_dweight(dout, y, r).cpu().double()
+    for j in range(2):
+        k = keep[:, j].nonzero().flatten()
+        a, b = dout[k.to(DEV)].cpu().double(), y[at[k, j].to(DEV)].cpu().double()
+        assert ((dw[k, j] - (a * b).sum(1)).abs() <= cols * 2.0 ** -24 * (a * b).abs().sum(1)).all()
+        assert (dw[~keep[:, j], j] == 0).all()

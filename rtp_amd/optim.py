@@ -96,6 +96,7 @@ class RotatedSGD:
         self._aux = None
         self._rest_table = self._rest_key = None
         self._rest_params, self._rest_dtype = 0, None
+        self._captured_tables = {}  # address -> chunk table that a captured step() reads at every replay
         if self.fused_backward:
             ctx = ops.FusedSgd(self.lr, self.clip_value, keep_grads, source=self)
             for st, master in zip(self.stores, self.masters):
@@ -193,6 +194,13 @@ class RotatedSGD:
         with torch.cuda.stream(self._aux):
             self._update_store(st, self.masters[self.stores.index(st)])
 
+    def _launching(self, table: torch.Tensor) -> torch.Tensor:
+        """`table`, about to be launched: a launch recorded into a graph reads it by address at every replay, so it lives as
+        long as the optimiser, like the buffers it points into, also when other ranges are left to a later step."""
+        if torch.cuda.is_current_stream_capturing():
+            self._captured_tables[table.data_ptr()] = table
+        return table
+
     def _multi_table(self):
         """Chunk table covering every buffer (rotated stores + the flat non-rotated parameters), rebuilt only when
         a buffer moved; None when a buffer cannot be updated this way."""
@@ -247,7 +255,7 @@ class RotatedSGD:
                 return
             self._rest_dtype = items[0][1].dtype
         if self._rest_table is not None:
-            ops.sgd_step_multi(self._rest_table, self._rest_dtype, self.lr, self.clip_value, self._rest_params)
+            ops.sgd_step_multi(self._launching(self._rest_table), self._rest_dtype, self.lr, self.clip_value, self._rest_params)
 
     def _rest_items(self, updated) -> list:
         """(update target, gradients, weights to refresh or None) of the parameter ranges that are not among `updated`:
@@ -280,7 +288,7 @@ class RotatedSGD:
         table = None if (self._early or self.overlap_backward) else self._multi_table()
         if table is not None:
             self._fold_other_grads()
-            ops.sgd_step_multi(table, self._table_dtype, self.lr, self.clip_value, self._table_params)
+            ops.sgd_step_multi(self._launching(table), self._table_dtype, self.lr, self.clip_value, self._table_params)
             if self.stores:
                 ring.fence(self.stores[0].home.device)
             return
@@ -373,7 +381,7 @@ class RotatedAdam(RotatedSGD):
         buffers = self._buffers()
         table = self._multi_adam_table(buffers) if buffers else None
         if table is not None:
-            ops.adam_step_multi(table, self._adam_dtype, self._step_dev, self.lr, self.betas, self.eps,
+            ops.adam_step_multi(self._launching(table), self._adam_dtype, self._step_dev, self.lr, self.betas, self.eps,
                                 self.weight_decay, self.clip_value, self._adam_params)
         else:
             for key, target, grads, shadow in buffers:

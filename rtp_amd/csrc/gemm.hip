@@ -1515,8 +1515,8 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   }
   // fp32 contractions of 384 and more go to gemm_split.hip, whose K loop is 1.2 - 1.9 times as fast and whose prologue and epilogue
   // are 1 - 2 us longer (a workgroup fills a CU there): us, fp32 MFMA -> this, forward layout: 64 matrices of 420 x 420 with
-  // K = 128 76 -> 78, 160 84 -> 81, 320 119 -> 104; 2048 x 512 with K = 224 9.1 -> 9.5, 320 10.5 -> 10.8; 1600 x 512 x 512 12.9 -> 12.7;
-  // 1024 x 2048 x 2048 74 -> 56; 8 of 122 x 1088 x 1536 51 -> 32.
+  // K = 128 76 -> 78, 160 84 -> 81, 320 119 -> 104; 2048 x 512 with K = 224 9.1 -> 9.5, 320 10.5 -> 10.8; 1600 x 512 x 512 12.9 -> 13.0;
+  // 1024 x 2048 x 2048 74 -> 60; 8 of 122 x 1088 x 1536 51 -> 35.
   // Its two tiles cost 700 and 430 ns a slab and 4 us a round with every CU busy.  (The launches that take 128 x 160 tiles, two even
   // rounds of an fp32 logits layer, stay with them.)
   const bool split = sizeof(T) == 4 && fast && !relu && k_all >= 384 && shape != 6;

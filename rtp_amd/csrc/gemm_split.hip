@@ -1,23 +1,25 @@
 // fp32 products on the bf16 matrix pipes.
 //
-// An fp32 number is the sum of three bf16 numbers, each the rounding of what the ones before leave (8 + 8 + 8 bits; exact above
-// 2^-110).  Of the nine products of two such sums the six whose parts i + j <= 2 reach an fp32 product's last bits;
+// An fp32 number is the sum of three bf16 numbers, each the rounding of what the ones before leave (8 + 8 + 8 bits).  It is taken
+// apart 2^24 times as large, so that the last bit of the smallest number, 2^-149, is a normal bf16 number and no part is ever rounded
+// or flushed, and the sums are scaled back by 2^-48; numbers of 2^103 and sums of 2^80 and more do not fit and are worked out by
+// the fp32 MFMA, see the epilogue.  Of the nine products of two such sums the six whose parts i + j <= 2 reach an fp32 product's last bits;
 // v_mfma_f32_32x32x16_bf16 does each at 16 times the rate of the fp32 MFMA, so the six cost 6 / 16 of it.  The leading product has
 // an accumulator of its own and the five others, 2^-8 of it and less, share another one or two: 16 k of a contraction round the
 // large sum once, where the fp32 MFMA rounds it for every k.
 //
 // The workgroup: four MFMA waves, each with 32 rows and 64 columns of the tile, and four loader waves.  Taking an element apart
-// costs 5.5 vector instructions (v_dot2_f32_bf16 would do a remainder in one, but occupies the matrix pipe), and its parts are
+// costs 6.5 vector instructions (v_dot2_f32_bf16 would do a remainder in one, but occupies the matrix pipe), and its parts are
 // six bytes instead of four, so as little as possible is taken apart twice or staged as parts: an MFMA wave loads its own rows of A
 // straight into LDS of its own, needs no barrier for them, and takes them apart between the MFMAs of the step before; B, which the
 // waves share, is taken apart once, by the loaders, and staged as three planes laid out like bf16 operands.  In a tile of
 // 64 rows two waves share a block of 32 x 64, a step of 16 k each of every slab, and their sums meet in the epilogue.
 //
-// What bounds it: power.  A slab of 32 k of a 128 x 64 tile takes 685 ns with every CU busy; its MFMAs alone, on random numbers, take
+// What bounds it: power.  A slab of 32 k of a 128 x 64 tile takes 700 ns with every CU busy; its MFMAs alone, on random numbers, take
 // 522, because the clock goes down to 1.5 GHz for them; without the loads, the LDS reads of B, or the taking apart it is 140 -
-// 180 less each.  us, fp32 MFMA -> this, forward / input gradient / weight gradient layout: 1024 x 2048 x 2048 74 / 68 / 65 -> 58 /
-// 56 / 58, 4096 x 4096 x 1024 256 / 254 / 262 -> 223 / 227 / 240, 8 of 122 x 1088 x 1536 51 / 50 / 70 -> 34 / 35 / 42; error against
-// fp64 of 1024 x 2048 x 2048 8.1e-7 -> 2.7e-7, of K = 384 and 4096 as much smaller.
+// 180 less each, without the scaling 15 - 20.  us, fp32 MFMA -> this, forward / input gradient / weight gradient layout: 1024 x 2048 x
+// 2048 74 / 68 / 65 -> 60 / 58 / 60, 4096 x 4096 x 1024 256 / 254 / 262 -> 230 / 234 / 245, 8 of 122 x 1088 x 1536 51 / 50 / 70 -> 35 /
+// 36 / 43; error against fp64 of 1024 x 2048 x 2048 8.1e-7 -> 2.7e-7, of K = 384 and 4096 as much smaller.
 #include "gemm_tile.h"
 
 namespace rtp {
@@ -30,19 +32,22 @@ typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // global
 // operation never waits for the one before.  The remainders replace the numbers.
 struct Split8 {
   unsigned h[3][4];  // part, pair of elements
-  static constexpr int OPS = 28;
+  static constexpr int OPS = 36;
+  static constexpr float SCALE = 0x1p24f;
   template <int O>
   __device__ __forceinline__ void op(float (&x)[8]) {
-    if constexpr (O < 4) {
-      pair<0, O>(x);
+    if constexpr (O < 8) {
+      x[O] *= SCALE;
     } else if constexpr (O < 12) {
-      rest<0, O - 4>(x);
-    } else if constexpr (O < 16) {
-      pair<1, O - 12>(x);
+      pair<0, O - 8>(x);
+    } else if constexpr (O < 20) {
+      rest<0, O - 12>(x);
     } else if constexpr (O < 24) {
-      rest<1, O - 16>(x);
+      pair<1, O - 20>(x);
+    } else if constexpr (O < 32) {
+      rest<1, O - 24>(x);
     } else {
-      pair<2, O - 24>(x);
+      pair<2, O - 32>(x);
     }
   }
   template <int L, int I>
@@ -505,7 +510,7 @@ __global__ __launch_bounds__(512) void gemm_split_kernel(GemmArgs p) {
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[j][r] += cor[0][j][r] + cor[1][j][r];
+      for (int r = 0; r < 16; ++r) acc[j][r] = (acc[j][r] + (cor[0][j][r] + cor[1][j][r])) * (1.0f / (Split8::SCALE * Split8::SCALE));
   }
 
   // Epilogue through LDS, as in gemm_dma_kernel
@@ -530,27 +535,16 @@ __global__ __launch_bounds__(512) void gemm_split_kernel(GemmArgs p) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[j][r] += at_tile(j, r);
     }
-    // What the parts cannot stand for: an infinite number has no remainder, one next to the type's largest rounds to infinity,
-    // and below 2^-110 the last part loses bits.  The first two leave an infinity or a NaN in every output they reach, and
-    // with the third the outputs are small, unless the other operand is beyond 2^20: a wave that finds such an output does its
-    // part of the tile again with the fp32 MFMA.
-    constexpr float kLow = 0x1p-90f;
-    float low = 1.0f, bad = 0.0f;
+    // What the parts cannot stand for: a number that is infinite, or is when scaled, has no remainder, and a scaled sum may overflow
+    // where the sum itself does not.  Either leaves an infinity or a NaN in every output it reaches: a wave that finds one does
+    // its part of the tile again with the fp32 MFMA.  (Not pipelined: with such an output in every wave 1024 x 2048 x 2048 takes 370 -
+    // 635 us instead of 58 - 66.)
+    float bad = 0.0f;
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        low = fminf(low, fabsf(acc[j][r]));
-        bad = fmaf(acc[j][r], 0.0f, bad);
-      }
-    bool again = bad != 0.0f;  // NaN
-    if (low < kLow) {          // zeros are ordinary results
-#pragma unroll
-      for (int j = 0; j < NT; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) again |= acc[j][r] != 0.0f && fabsf(acc[j][r]) < kLow;
-    }
-    if (__any(again)) {
+      for (int r = 0; r < 16; ++r) bad = fmaf(acc[j][r], 0.0f, bad);
+    if (__any(bad != 0.0f)) {  // NaN
 #pragma unroll
       for (int j = 0; j < NT; ++j)
 #pragma unroll

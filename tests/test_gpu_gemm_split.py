@@ -90,3 +90,25 @@ def test_small_numbers(akc, bkc):
     out, _ = _product(a[None, None], b[None, None], m, n, k, akc, bkc)
     ref, size = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
     assert ((out[0].double() - ref).abs() <= (k + 4) * 2.0 ** -24 * size + 2.0 ** -149).all()
+
+
+@pytest.mark.parametrize("akc,bkc", LAYOUTS)
+@pytest.mark.parametrize("swap", [False, True])
+@pytest.mark.parametrize("small,large", [(-116, 40), (-119, 40), (-125, 60), (-134, 60), (-140, 80), (-100, -40), (-60, -70),
+                                         (100, -30), (110, -60), (60, 30), (-140, 110)])
+def test_small_by_large_numbers(akc, bkc, swap, small, large):
+    """Operands at 2**small, whose parts would lie below bf16's smallest numbers, by operands at 2**large; and numbers and
+    results beyond the range that the parts are scaled to.  As precise as ordinary numbers, subnormal ones included."""
+    m, n, k = 130, 72, 448
+    gen = torch.Generator().manual_seed(2)
+    a, b = torch.randn(m, k, generator=gen) * 2.0 ** small, torch.randn(n, k, generator=gen) * 2.0 ** large
+    a[5], b[7] = 0, 0
+    if swap:
+        a, b, m, n = b, a, n, m
+    out, _ = _product(a[None, None], b[None, None], m, n, k, akc, bkc)
+    ref, size = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
+    steps = -(-k // 16)  # as in test_edges, and half a unit of the smallest subnormal number for the result's rounding
+    bound = (3 * 2.0 ** -26 + (2 * steps + 4) * 2.0 ** -24) * size + 2.0 ** -150
+    # outputs below fp32's smallest normal number: a sum of products that are subnormal themselves rounds each of them
+    bound = torch.where(size < 2.0 ** -126, bound + k * 2.0 ** -150, bound)
+    assert ((out[0].double() - ref).abs() <= bound).all()

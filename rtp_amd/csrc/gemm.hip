@@ -1622,7 +1622,12 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   a.warm = nullptr;
   a.warm_bytes = 0;
   if (!fast) return launch_layout<T, 64, 64, 1, false>(s, a, akc, bkc, grid);
-  if (shape != 5 && warm_src != nullptr) {
+  // Carried by the kernels whose MFMA waves wait for loader waves at their start.  In the others every wave's own loads would queue
+  // behind the hint's.  fp32 products lose nothing by it, their slabs take longer than HBM does: us, weights in the memory-side
+  // cache / in HBM, 1024 x 2048 x 2048 split 56 - 61 / 58 - 60, with fp32 MFMAs 77 / 71, 1024 x 6144 x 2048 164 / 164 and 196 / 184.
+  // Few rows do (bf16 64 x 2048 x 2048 6.3 / 8.5, input gradient 7.0 / 11.9; fp32 13.5 / 15.3), and are ahead of the tiles that
+  // carry hints all the same (gemm_kwaves.hip).
+  if (shape != 5 && !split && warm_src != nullptr) {
     a.warm = (const char*)warm_src;
     a.warm_bytes = (long)t_warm_bytes;
   }

@@ -60,8 +60,9 @@ def rotation_mode() -> str:
 
 # ---- the next layer's shards arrive while the current layer computes (direct mode) ------------------------
 # Read from their home rows, a layer's weights are touched once per pass, so at their turn they come from HBM, and the
-# products' load pipeline (a few K slabs in flight) does not cover that latency: measured on the LM's shapes, a
-# product takes 15 - 30 % longer on weights from HBM than on weights that sit in the 256 MiB memory-side cache.  With
+# products' load pipeline (a few K slabs in flight) does not cover that latency: measured on the LM's shapes, a bf16
+# product takes 15 - 30 % longer on weights from HBM than on weights that sit in the 256 MiB memory-side cache (an fp32
+# one does not, and neither it nor the kernel for few rows carries the hint that is set here).  With
 # the switch on, a rotation that starts hands the home rows of the layer that followed this one the last time round
 # to its own first product (rtp_gemm_warm_next), whose workgroups request them at their start: the one-GPU form of
 # the reference's irecv of the next shard during the current step (rtp/module/linear.py:211-220).  Which layer

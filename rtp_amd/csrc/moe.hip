@@ -179,13 +179,14 @@ __global__ __launch_bounds__(kTok) void route_bwd_kernel(const float* gates, con
   }
 }
 
-// out[row,:] = x[token(row),:] (* weight of the choice that put the token there), zero if the slot is
-// empty.  One workgroup per (slot row, column chunk).
 // The row moves and the weights' gradient, 16 bytes per lane and access: VEC consecutive columns of a row.  A thread of the
 // moves is one vector of the flattened (row, vector) space, so narrow rows share a workgroup.  Bound by memory.  us, a column per lane
 // and access -> this, 4096 tokens, 8 experts, 2048 columns: bf16 dispatch 18.0 -> 11.6, with weights 21.5 -> 13.5, combine 17.2 -> 10.4,
-// the weights' gradient 13.9 -> 9.5; fp32 21.9 -> 20.4, 25.3 -> 22.5, 20.8 -> 17.5, 16.9 -> 17.8.  The kernels further down serve rows
-// that are not vector-aligned.
+// the weights' gradient 13.9 -> 9.5; fp32 21.9 -> 20.4, 25.3 -> 22.5, 20.8 -> 17.5.  The weights' gradient in fp32, one set of operands in
+// turn / six: 4096 x 2048, 8 experts 16.7 -> 17.1 / 23.5 -> 21.7, 16 experts 17.0 -> 20.1 / 25.8 -> 26.5, 4096 x 1024 9.9 -> 9.5 / 14.4 ->
+// 10.8, 4096 x 512 5.5 -> 4.2 / 6.5 -> 6.2, 1024 x 2048 11.3 -> 3.7 / 12.4 -> 6.0, 512 x 1024 3.8 -> 2.6 / 7.1 -> 3.4, 64 x 2048 5.3 ->
+// 2.8, 128 x 128 2.4 -> 2.4: behind only on rows of 8 KB and more of so many tokens that hardly stay in the caches from one launch to
+// the next.  The kernels further down serve rows that are not vector-aligned.
 template <typename T>
 struct alignas(16) RowVec {
   static constexpr int N = 16 / (int)sizeof(T);
@@ -277,6 +278,8 @@ static bool row_vectors(size_t esz, int64_t cols, const void* a, int64_t ld_a, c
           (uintptr_t)(ld_b * (int64_t)esz)) % 16 == 0;
 }
 
+// out[row,:] = x[token(row),:] (* weight of the choice that put the token there), zero if the slot is
+// empty.  One workgroup per (slot row, column chunk).
 template <typename T>
 __global__ __launch_bounds__(256) void dispatch_kernel(const T* x, long ld_x, const int* slot_token,
                                                        const int* expert, const int* slot, const float* weight,

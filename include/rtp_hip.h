@@ -223,8 +223,8 @@ int rtp_gemm(void* stream, int dtype, const rtp_gemm_desc* d);
  * That launch requests them at its start, so they sit in the GPU's memory-side cache when their own products run
  * (weights are read once per pass and would otherwise come from HBM at their turn).  Up to 192 KiB per workgroup
  * of the carrying launch.  A hint: no result depends on it; it ends with that next product launch whether or not
- * the launch could carry it: the wave-specialised kernels of up to 256 x 192 outputs can, those for few tiles, short
- * contractions, 256 x 256 outputs and fp32 contractions of 384 and more cannot.  The carrying kernel reads `src` when
+ * the launch could carry it: the wave-specialised kernels of tiles below 256 x 256 can, those for few tiles, for
+ * short contractions, of 256 x 256 and for fp32 contractions of 384 and more cannot.  The carrying kernel reads `src` when
  * it RUNS, not when it is launched: `src` has to stay mapped until that launch has completed on its stream.  bytes == 0
  * withdraws a pending hint.  One hint is pending in a process: a call ends the hint of any other thread too, so the
  * caller need only keep the last `src`.

@@ -625,379 +625,6 @@ __global__ __launch_bounds__(512) void gemm_unaligned_kernel(GemmArgs p) {
                                                           gridDim.x * gridDim.y);
 }
 
-// ---------------------------------------------------------------------------------------------
-// 256 x 256 tiles for large products.  What bounds the kernel above on a large product is the stream of operand
-// bytes from the L2 into the LDS, and that stream is (1/BM + 1/BN) bytes per flop: a 256 x 256 tile moves two thirds of
-// what 256 x 128 moves.  Its 256 KiB of fp32 accumulators need all eight waves of the workgroup as MFMA waves (2 x 4 wave
-// tiles of 128 x 64, 128 accumulator registers each), so here the waves issue the direct-to-LDS loads themselves.
-//
-// A SIMD holds two of the waves, and their work alternates: a K slab (128 bytes of k per row) is four phases, a phase is a
-// read half -- fragments of half an operand into registers, two load instructions -- and an MFMA half of eight MFMAs,
-// each closed by a workgroup barrier.  The waves of the lower tile half (wm = 1, the second wave of every SIMD) pass one
-// barrier more at the start, so they read while the others multiply and the other way round: LDS reads, loads and scalar
-// work of one wave lie under the MFMAs of the other, and neither waits for its own.
-//
-// An operand's slab is two half tiles of 128 rows (16 KiB each, stored like a 128-row operand), and a wave tile takes half of
-// its rows (columns) from each, so a phase multiplies one quadrant of the wave tile by all of the slab's k:
-//   phase    reads               multiplies        loads (into the half tile freed two phases before)
-//   1        A half 0            A0 x B0           A half 1 of slab k + 1
-//   2        B half 1            A0 x B1           B half 0 of slab k + 2
-//   3        A half 1            A1 x B1           A half 0 of slab k + 2
-//   4        B half 0 of k + 1   A1 x B0           B half 1 of slab k + 2
-// Two barrier-separated halves make phase p's reads complete in every wave before the read half of phase p + 2 begins (the
-// reads have returned when the MFMA half ends), which is where that half tile may be overwritten; and a load has six
-// phases from its issue to its read.  Before a read half ends, a wave waits until its loads of five phases ago have
-// landed (the ten youngest may be on their way); the next phase's reads lie two barriers behind, so that holds for every
-// wave's share.  The epilogue goes through LDS in four passes of 64 rows.
-//
-// Bound by LDS and the matrix pipes together: a slab is 2048 clocks of MFMA per SIMD, 1536 of fragment reads at 128
-// bytes a clock and 64 KiB of arriving loads.  us, forward / input gradient / weight gradient layout (before: all eight
-// waves in step, one barrier a slab, a whole slab requested at once and waited for whole): 4096 x 8192 x 1024 77 / 77 / 80
-// -> 70 / 72 / 73, 6000 x 2048 x 2048 59 / 59 / 60 -> 53 / 54 / 55, 4096^3 128 / 136 / 124 -> 121 / 131 / 124, 8192^3
-// 866 / 848 / 851 -> 840 / 837 / 842.  Closing the MFMA half before its last two MFMAs instead of behind them, so that the
-// waves' MFMAs overlap, costs 10 - 20 %: the two waves of a SIMD then drift into the same half.
-//
-// The half tile of the rows r' = 0 .. 127 holds tile rows half_row<BLK>(r', h): blocks of BLK rows, every other one.
-template <int BLK>
-__device__ __forceinline__ constexpr int half_row(int r, int h) {
-  return ((r & ~(BLK - 1)) << 1) | (h * BLK) | (r & (BLK - 1));
-}
-
-template <typename T, bool AKC, bool BKC>
-__global__ __launch_bounds__(512) void gemm_dma8_kernel(GemmArgs p) {
-  constexpr int BM = 256, BN = 256, NL = 8, SB = 128;
-  constexpr int WM = 128, WN = 64, MT = 4, NT = 2;
-  constexpr int BLKA = WM / 2, BLKB = WN / 2;
-  using DA = DmaOperand<T, BM / 2, AKC, NL, SB>;
-  using DB = DmaOperand<T, BN / 2, BKC, NL, SB>;
-  constexpr int BK = SB / sizeof(T);
-  constexpr int KS = SB / 32;
-  constexpr int HALF = DA::BYTES;
-  constexpr int NI = DA::NI;  // load instructions per wave and half tile
-  static_assert(DB::BYTES == HALF && DB::NI == NI && 5 * NI < 64, "half tiles of one size; vmcnt is a 6-bit counter");
-  static_assert(64 * (BN + 4) * 4 <= 8 * HALF, "an epilogue pass stages 64 rows of the fp32 tile");
-  __shared__ __attribute__((aligned(1024))) char lds[8 * HALF];  // [slab & 1][A0, A1, B0, B1]
-
-  touch_kernel_arguments<sizeof(GemmArgs)>();
-  const int tid = threadIdx.x;
-  if (p.trace != nullptr && tid == 0) atomicMin(p.trace, (unsigned long long)wall_clock64());
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 2, wn = wave & 3;
-  const int li = lane & 31, g = lane >> 5;
-
-  // tile mapping: as in gemm_dma_kernel
-  const unsigned id = blockIdx.x + blockIdx.y * gridDim.x;
-  const unsigned xcd = id & 7, slot = id >> 3;
-  const unsigned zl = fast_div(slot, p.d_brick);
-  const unsigned t_ = slot - zl * p.d_brick.d;
-  const unsigned q_ = fast_div(t_, p.d_panel), r_ = t_ - q_ * p.d_panel.d;
-  const unsigned cn = fast_div(r_, p.d_prow), cm = r_ - cn * p.d_prow.d;
-  const unsigned qn = fast_div(q_, p.d_pm), qm = q_ - qn * p.d_pm.d;
-  const int tile_n_x = (int)((xcd & ((1u << p.xn_shift) - 1)) * p.nbk + qn * p.pcol + cn);
-  const int tile_m_x = (int)(((xcd >> p.xn_shift) & ((1u << p.xm_shift) - 1)) * p.mbk + qm * p.prow + cm);
-  const int z_x = (int)((xcd >> (p.xn_shift + p.xm_shift)) * p.zbk + zl);
-  const int tile_m_p = (int)fast_div(blockIdx.x, p.d_tiles_n);
-  const int tile_n_p = (int)(blockIdx.x - tile_m_p * p.d_tiles_n.d);
-  const bool bricks = p.xg != 0;
-  const int tile_m = bricks ? tile_m_x : tile_m_p, tile_n = bricks ? tile_n_x : tile_n_p;
-  const int z = bricks ? z_x : (int)blockIdx.y;
-  const int m0 = tile_m * BM;
-  const int n0 = tile_n * BN;
-  const int grp = (int)fast_div(z, p.d_batch), zb = z - grp * (int)p.d_batch.d;
-  const long zo = fast_div(zb, p.d_zdiv), zi = zb - (int)zo * (int)p.d_zdiv.d;
-  const int nk_seg = (p.k + BK - 1) / BK;
-  const int nk = nk_seg * p.ksegs;
-
-  f32x16 acc[MT][NT];
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < NT; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-  float rsum[MT];
-#pragma unroll
-  for (int i = 0; i < MT; ++i) rsum[i] = 0.0f;
-
-  // ---- this wave's share of the loads ----
-  const T* A = reinterpret_cast<const T*>(p.a) + grp * p.a_sg + zo * p.a_so + zi * p.a_si;
-  const T* B = reinterpret_cast<const T*>(p.b) + grp * p.b_sg + zo * p.b_so + zi * p.b_si;
-  DA da[2];
-  DB db[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    da[h].init(p.lda, m0, p.m, wave, lane, [=](int r) { return half_row<BLKA>(r, h); });
-    db[h].init(p.ldb, n0, p.n, wave, lane, [=](int r) { return half_row<BLKB>(r, h); });
-  }
-  const char* ca = DA::slab_base(A, p.lda, m0);
-  const char* cb = DB::slab_base(B, p.ldb, n0);
-  constexpr long SZ = (long)sizeof(T);
-  const long step_a = (AKC ? (long)BK : (long)BK * p.lda) * SZ, step_b = (BKC ? (long)BK : (long)BK * p.ldb) * SZ;
-  const long last_a = step_a + p.a_sk * SZ - nk_seg * step_a, last_b = step_b + p.b_sk * SZ - nk_seg * step_b;
-  const int k0_last = (nk_seg - 1) * BK;
-  const bool tail = p.k % BK != 0;
-  const unsigned lds0 = (unsigned)(uintptr_t)(lptr_t)lds;
-  int left_a = nk_seg, left_b = nk_seg;
-  // the next half tile of an operand, half 0 of a slab and then half 1, into the slab at byte `slot` of the LDS
-  auto issue_a = [&](unsigned slot, auto H) {
-    constexpr int h = decltype(H)::value;
-    if (left_a != 1 || !tail)
-      da[h].template issue<false>(lds0 + slot + h * HALF, wave, ca, 0, 0);
-    else
-      da[h].template issue<true>(lds0 + slot + h * HALF, wave, ca, k0_last, p.k);
-    if (h == 1) {
-      ca += left_a != 1 ? step_a : last_a;
-      left_a = left_a != 1 ? left_a - 1 : nk_seg;
-    }
-  };
-  auto issue_b = [&](unsigned slot, auto H) {
-    constexpr int h = decltype(H)::value;
-    if (left_b != 1 || !tail)
-      db[h].template issue<false>(lds0 + slot + (2 + h) * HALF, wave, cb, 0, 0);
-    else
-      db[h].template issue<true>(lds0 + slot + (2 + h) * HALF, wave, cb, k0_last, p.k);
-    if (h == 1) {
-      cb += left_b != 1 ? step_b : last_b;
-      left_b = left_b != 1 ? left_b - 1 : nk_seg;
-    }
-  };
-
-  using I0 = std::integral_constant<int, 0>;
-  using I1 = std::integral_constant<int, 1>;
-  Frag<T> fa[2][KS], fb0[KS], fb0n[KS], fb1[KS];  // B half 0 of the next slab is read while this slab's is multiplied
-  const bool rowsum = p.a_rowsum != nullptr && tile_n == 0 && wn == 0;
-  auto read_a = [&](unsigned slot, auto H) {
-    const char* st = lds + slot + decltype(H)::value * HALF;
-#pragma unroll
-    for (int q = 0; q < KS; ++q)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) fa[i][q] = read_frag_dma<T, BM / 2, AKC, SB>(st, wm * BLKA + i * 32, lane, q);
-  };
-  auto read_b = [&](unsigned slot, auto H, Frag<T>(&fb)[KS]) {
-    const char* st = lds + slot + (2 + decltype(H)::value) * HALF;
-#pragma unroll
-    for (int q = 0; q < KS; ++q) fb[q] = read_frag_dma<T, BN / 2, BKC, SB>(st, wn * BLKB, lane, q);
-  };
-  // the barrier that ends a read half, the MFMA half and its end, where this wave's reads have returned (the first MFMAs
-  // wait only for their own fragments)
-  auto multiply = [&](auto H, auto J, const Frag<T>(&fb)[KS], bool sums) {
-    constexpr int h = decltype(H)::value, j = decltype(J)::value;
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int q = 0; q < KS; ++q)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) mma(fa[i][q], fb[q], acc[h * 2 + i][j]);
-    __builtin_amdgcn_s_setprio(0);
-    if (sums && rowsum) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int q = 0; q < KS; ++q) rsum[h * 2 + i] = frag_sum(fa[i][q], rsum[h * 2 + i]);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  // the slab at byte `cur` of the LDS; REST: slabs behind it (2: two or more)
-  unsigned cur = 0;
-  auto slab = [&](auto REST) {
-    constexpr int rest = decltype(REST)::value;
-    const unsigned other = cur ^ (4 * HALF);
-    read_a(cur, I0{});
-    if constexpr (rest >= 1) issue_a(other, I1{});
-    if constexpr (rest >= 1) RTP_WAIT_VM(5 * NI);
-    else RTP_WAIT_VM(NI);
-    multiply(I0{}, I0{}, fb0, true);
-
-    read_b(cur, I1{}, fb1);
-    if constexpr (rest >= 2) issue_b(cur, I0{});
-    if constexpr (rest >= 2) RTP_WAIT_VM(5 * NI);
-    else if constexpr (rest == 1) RTP_WAIT_VM(4 * NI);
-    else RTP_WAIT_VM(0);
-    multiply(I0{}, I1{}, fb1, false);
-
-    read_a(cur, I1{});
-    if constexpr (rest >= 2) issue_a(cur, I0{});
-    if constexpr (rest >= 2) RTP_WAIT_VM(5 * NI);
-    else if constexpr (rest == 1) RTP_WAIT_VM(3 * NI);
-    multiply(I1{}, I1{}, fb1, true);
-
-    if constexpr (rest >= 1) read_b(other, I0{}, fb0n);
-    if constexpr (rest >= 2) issue_b(cur, I1{});
-    if constexpr (rest >= 2) RTP_WAIT_VM(5 * NI);
-    else if constexpr (rest == 1) RTP_WAIT_VM(2 * NI);
-    multiply(I1{}, I0{}, fb0, false);
-    if constexpr (rest >= 1) {
-#pragma unroll
-      for (int q = 0; q < KS; ++q) fb0[q] = fb0n[q];
-    }
-    cur = other;
-  };
-
-  // what phases before the first would have issued, in their order; the host sends no problem of a single slab here
-  issue_b(0, I0{});
-  issue_a(0, I0{});
-  issue_b(0, I1{});
-  issue_a(0, I1{});
-  issue_b(4 * HALF, I0{});
-  issue_a(4 * HALF, I0{});
-  issue_b(4 * HALF, I1{});
-  RTP_WAIT_VM(5 * NI);  // halves 0 of slab 0 have landed
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-  read_b(0, I0{}, fb0);
-  __builtin_amdgcn_sched_barrier(0);
-  if (wm == 1) __builtin_amdgcn_s_barrier();
-  for (int k = 0; k + 2 < nk; ++k) slab(std::integral_constant<int, 2>{});
-  slab(I1{});
-  slab(I0{});
-  if (wm == 0) __builtin_amdgcn_s_barrier();
-
-  if (p.a_rowsum != nullptr && tile_n == 0 && wn == 0) {
-    T* dst = reinterpret_cast<T*>(p.a_rowsum) + grp * p.rowsum_sg;
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      const float v = rsum[i] + __shfl_xor(rsum[i], 32, 64);
-      const int row = m0 + wm * WM + i * 32 + li;
-      if (g == 0 && row < p.m) dst[row] = from_f32<T>((p.flags & RTP_GEMM_ROWSUM_ACCUM) ? to_f32(dst[row]) + v : v);
-    }
-  }
-
-  // Epilogue in MT passes: pass i stages rows i*32 .. i*32+31 of both tile halves (64 rows of 256 columns, fp32)
-  // in the slab memory; every thread then finishes four chunks of 8 columns, all in the same columns, whose bias it reads
-  // once per tile.  The barriers wait for LDS alone: __syncthreads would also wait until the previous pass's stores have
-  // reached memory.  The passes are a loop and not unrolled: unrolled, with the shared epilogue function inlined for every
-  // pass, the kernel was 70 - 90 KB of code for an instruction cache of 64 KB; it is 18 KB (-1 to -2 % per launch).
-  auto lds_barrier = [] {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-  };
-  constexpr int CP = BN + 4, NCH = 4, NB = 2;
-  float* ct = reinterpret_cast<float*>(lds);
-  const bool stream_out = p.flags & RTP_GEMM_STREAM_OUT, relu = p.flags & RTP_GEMM_RELU;
-  const bool out_f32 = p.flags & RTP_GEMM_OUT_F32, cin_f32 = p.flags & RTP_GEMM_CIN_F32;
-  char* cbase = p.c_out + (grp * p.c_sg + zo * p.c_so + zi * p.c_si) * (out_f32 ? 4 : SZ);
-  const char* cin = p.c_in ? p.c_in + (grp * p.cin_sg + zo * p.cin_so + zi * p.cin_si) * (cin_f32 ? 4 : SZ) : nullptr;
-  const T* gate =
-      p.gate ? reinterpret_cast<const T*>(p.gate) + grp * p.gate_sg + zo * p.gate_so + zi * p.gate_si : nullptr;
-  const int lc = (tid & 31) * 8, col = n0 + lc, colc = col < p.n ? col : 0;
-  float bcol[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  if (p.bias) {
-    const T* bias = reinterpret_cast<const T*>(p.bias) + grp * p.bias_sg + zo * p.bias_so + zi * p.bias_si + colc;
-    const int nb_seg = p.bias_sk ? p.ksegs : 1;  // a bias per K segment is summed in segment order
-    for (int sgm = 0; sgm < nb_seg; ++sgm) {
-      float t[8];
-      load8(bias + sgm * p.bias_sk, t);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) bcol[e] += t[e];
-    }
-  }
-  auto stage = [&](const f32x16(&part)[NT]) {
-#pragma unroll
-    for (int j = 0; j < NT; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        ct[(wm * 32 + 8 * (r >> 2) + 4 * g + (r & 3)) * CP + wn * WN + j * 32 + li] = part[j][r];
-  };
-#pragma unroll 1
-  for (int i = 0; i < MT; ++i) {
-    lds_barrier();  // the fragments (first pass) or the previous pass's rows have been read
-    if (i == 0)
-      stage(acc[0]);
-    else if (i == 1)
-      stage(acc[1]);
-    else if (i == 2)
-      stage(acc[2]);
-    else
-      stage(acc[3]);
-    lds_barrier();
-#pragma unroll 1
-    for (int c0 = 0; c0 < NCH; c0 += NB) {
-      auto row_of = [&](int c) {
-        const int lr = (tid >> 5) + 16 * (c0 + c);
-        return m0 + (lr >> 5) * WM + i * 32 + (lr & 31);
-      };
-      Raw8<T> rg[NB], rc16[NB];
-      Raw8<float> rc32[NB];
-#pragma unroll
-      for (int c = 0; c < NB; ++c) {
-        const int row = row_of(c);
-        const long rowc = row < p.m ? row : p.m - 1;
-        if (cin) {
-          if (cin_f32)
-            rc32[c].load(reinterpret_cast<const float*>(cin) + rowc * p.ld_cin + colc);
-          else
-            rc16[c].load(reinterpret_cast<const T*>(cin) + rowc * p.ld_cin + colc);
-        }
-        if (gate) rg[c].load(gate + rowc * p.ld_gate + colc);
-      }
-#pragma unroll
-      for (int c = 0; c < NB; ++c) {
-        const int lr = (tid >> 5) + 16 * (c0 + c), row = row_of(c);
-        float v[8], t[8];
-        const float4 lo = *reinterpret_cast<const float4*>(ct + lr * CP + lc);
-        const float4 hi = *reinterpret_cast<const float4*>(ct + lr * CP + lc + 4);
-        v[0] = lo.x, v[1] = lo.y, v[2] = lo.z, v[3] = lo.w, v[4] = hi.x, v[5] = hi.y, v[6] = hi.z, v[7] = hi.w;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] *= p.alpha;
-        if (cin) {
-          if (cin_f32)
-            rc32[c].get(t);
-          else
-            rc16[c].get(t);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] += t[e];
-        }
-        if (p.bias) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] += bcol[e];
-        }
-        if (relu) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] = fmaxf(v[e], 0.0f);
-        }
-        if (gate) {
-          rg[c].get(t);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] = t[e] > 0.0f ? v[e] : 0.0f;
-        }
-        if (row >= p.m || col >= p.n) continue;
-        if (p.xent_mode == 2) xent_gradient8<T>(p, v, row, col, grp);
-        const long off = (long)row * p.ldc + col;
-        if (out_f32)
-          store8(reinterpret_cast<float*>(cbase) + off, v, stream_out);
-        else
-          store8(reinterpret_cast<T*>(cbase) + off, v, stream_out);
-      }
-    }
-  }
-  if (p.trace != nullptr && tid == 0) atomicMax(p.trace + 1, (unsigned long long)wall_clock64());
-}
-
-template <typename T>
-static int launch_dma8(hipStream_t s, const GemmArgs& a, bool akc, bool bkc, dim3 grid) {
-  const dim3 block(512);
-  if (akc && bkc)
-    hipLaunchKernelGGL((gemm_dma8_kernel<T, true, true>), grid, block, 0, s, a);
-  else if (akc && !bkc)
-    hipLaunchKernelGGL((gemm_dma8_kernel<T, true, false>), grid, block, 0, s, a);
-  else if (!akc && bkc)
-    hipLaunchKernelGGL((gemm_dma8_kernel<T, false, true>), grid, block, 0, s, a);
-  else
-    hipLaunchKernelGGL((gemm_dma8_kernel<T, false, false>), grid, block, 0, s, a);
-  RTP_LAUNCH_CHECK();
-  return RTP_OK;
-}
-
 template <typename T, int BM, int BN, int NSTAGE, int SB, int PD>
 static int launch_dma(hipStream_t s, const GemmArgs& a, bool akc, bool bkc, dim3 grid) {
   const dim3 block(512);
@@ -1471,12 +1098,12 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
     const char* e = getenv("RTP_GEMM_TILE");  // debugging aid: index into kShapes
     return e ? atoi(e) : -1;
   }();
-  static const double slab_ns[kNumShapes] = {966.0, 470.0, 283.0, 167.0, 800.0, 1350.0, 545.0};
-  // Per tile outside the K loop.  256 x 256 is priced by its ratio to the others with every CU busy: measured there over 117
-  // products x 3 layouts at 1510 ns a slab and 13 us a tile, against 1040 ns and 8.5 us for 256 x 128, 540 ns and 5.4 us for 128 x 128.
-  // With these two numbers it is taken on none of them where another shape is more than 1 % faster, and on 25 more than with
-  // 1400 and 9000 ns: 4096 x 6144 x 2048 121 -> 113 us, 8192 x 8192 x 256 98 -> 80, 8 of 3072 x 1024 x 768 72 -> 59.
-  static const double fixed_ns[kNumShapes] = {3000.0, 3000.0, 3000.0, 3000.0, 3000.0, 5000.0, 3000.0};
+  static const double slab_ns[kNumShapes] = {966.0, 470.0, 283.0, 167.0, 800.0, 1050.0, 545.0};
+  // Per tile outside the K loop.  256 x 256 is priced by its ratio to the others with every CU busy.  Every tile forced on 59 products
+  // x 3 layouts, operands from memory: with these two numbers the shape taken costs 0.1 % over the best one in the mean (with 1350 and
+  // 5000 ns, the price of the kernel before this one, 0.8 %), the most 12 % (4096 x 2048 x 6144, 128 tiles: 119 us with 256 x 128 against 111); it is
+  // the same for 975 - 1100 and 4000 - 5000 ns.  Where 256 x 256 is close and not taken: 4096 x 2048 x 2048, 128 tiles, 39 - 43 us against 37 - 38.
+  static const double fixed_ns[kNumShapes] = {3000.0, 3000.0, 3000.0, 3000.0, 3000.0, 4500.0, 3000.0};
   // The two tiles for operands or outputs of any alignment, 64 x 64 and 128 x 128: the element-wise epilogue makes the larger one's
   // share outside the loop 14.5 us, the register loaders make a slab take twice as long.  Measured on 16 odd shapes x 3 layouts
   // with either tile forced; with the prices above, 128 x 128 was taken where 64 x 64 is ahead: us, bf16 3864 x 321 x 201 17.4 -> 11.9,
@@ -1497,8 +1124,8 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
     // as the LM's logits layer (shards of 1280 columns); larger products keep the shapes measured on large products
     if (i == 6 && ceil_div(d->m, 128) * ceil_div(d->n, 160) * nz > 512 && i != forced) continue;
     // It needs neither a full round nor a long contraction to pay: on 144 - 255 tiles it is one round where the others take
-    // two or more (6000 x 2048 x 2048, 192 tiles: 53 us against 57 with 128 x 128 and 65 with 256 x 128; 3000 x 3000 x
-    // 1096, 144 tiles: 35 against 48 and 50), and at K = 512 it is 27 us against 34 (8192 x 2048) and 99 against 123 (8192^2).
+    // two or more (6000 x 2048 x 2048, 192 tiles: 51 us against 57 with 128 x 128 and 65 with 256 x 128), and at K = 512 it is
+    // 89 us against 123 (8192^2).
     if (i == 5 && ceil_div(d->k, 64) * d->ksegs < 2) continue;  // its pipeline is primed with two slabs
     // never a tile that is mostly padding: a 32 x 32 problem (one attention head at seq 32) stays at 64 x 64
     if ((!akc && (kShapes[i].bm & (kShapes[i].bm - 1))) || (!bkc && (kShapes[i].bn & (kShapes[i].bn - 1)))) continue;
@@ -1562,7 +1189,7 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   a.d_zdiv = make_fastdiv((unsigned)d->zdiv);
   a.d_tiles_n = make_fastdiv((unsigned)a.tiles_n);
   {
-    const int nbk = a.xg ? a.tiles_n / a.xn : 1, mbk = a.xg ? a.tiles_m / a.xm : 1;
+    const int nbk = a.xg ? a.tiles_n / a.xn : a.tiles_n, mbk = a.xg ? a.tiles_m / a.xm : a.tiles_m;
     // Panel = prow x pcol tiles, about one round of an XCD's 32 CUs.  pcol: the widest divisor of nbk (at most 32)
     // whose strip of B tiles (pcol * BN rows x all of K) stays within ~3 MB of the XCD's 4 MB L2 -- the A rows stream
     // past the strip once, so the L2 fills are about A * nbk / pcol + B per brick.  prow: the tallest divisor of mbk
@@ -1590,6 +1217,8 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   a.xn_shift = a.xn == 8 ? 3 : a.xn == 4 ? 2 : a.xn == 2 ? 1 : 0;
   a.xm_shift = a.xm == 8 ? 3 : a.xm == 4 ? 2 : a.xm == 2 ? 1 : 0;
   a.zbk = a.xg ? (int)(nz / a.xg) : 0;
+  a.tiles = (unsigned)(nb * nz);
+  a.per_xcd = (unsigned)ceil_div(nb * nz, 8);
 
   // variant name = the kernel template instance, e.g. gemm_bf16_128x64_kc_kc
   static const char* const layout_tag[2][2] = {{"rc_rc", "rc_kc"}, {"kc_rc", "kc_kc"}};
@@ -1656,7 +1285,7 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
       // shard and fills the CUs in two even rounds where 128 x 128 tiles need two and a half
       return launch_dma<T, 128, 160, 4, 128, 1>(s, a, akc, bkc, grid);
     case 5:
-      if constexpr (sizeof(T) == 2) return launch_dma8<T>(s, a, akc, bkc, grid);
+      if constexpr (sizeof(T) == 2) return launch_large(s, a, akc, bkc);
       return fail(RTP_ERR_ARG, "gemm: no 256 x 256 kernel for this dtype");
     default:
       return launch_dma<T, 64, 64, 4, 128, 3>(s, a, akc, bkc, grid);

@@ -1,0 +1,709 @@
+// bf16 products in tiles of 256 x 256.
+#include "gemm_tile.h"
+
+namespace rtp {
+
+// What bounds the kernels of gemm.hip on a large product is the stream of operand bytes from the L2 into the LDS, and that stream is
+// (1/BM + 1/BN) bytes per flop: a 256 x 256 tile moves two thirds of what 256 x 128 moves.  Its 256 KiB of fp32 accumulators need all
+// eight waves of the workgroup as MFMA waves (2 x 4 wave tiles of 128 x 64, 128 accumulator registers each), so here the waves issue
+// the direct-to-LDS loads themselves.
+//
+// A SIMD holds two of the waves, and their work alternates: a K slab (128 bytes of k per row) is four phases, a phase is a
+// read half -- fragments of half an operand into registers, two load instructions -- and an MFMA half of eight MFMAs,
+// each closed by a workgroup barrier.  The waves of the lower tile half (wm = 1, the second wave of every SIMD) pass one
+// barrier more at the start of a tile, so they read while the others multiply and the other way round: LDS reads, loads and scalar
+// work of one wave lie under the MFMAs of the other, and neither waits for its own.  That holds as long as a read half takes no
+// longer than eight MFMAs (256 clocks): it is some 25 instructions, addresses in registers and offsets in the instructions, and its
+// rare events are branches that are not taken.
+//
+// An operand's slab is two half tiles of 128 rows (16 KiB each, stored like a 128-row operand), and a wave tile takes half of
+// its rows (columns) from each, so a phase multiplies one quadrant of the wave tile by all of the slab's k:
+//   phase    reads               multiplies        loads (into the half tile freed two phases before)
+//   1        A half 0            A0 x B0           A half 1 of slab k + 1
+//   2        B half 1            A0 x B1           B half 0 of slab k + 2
+//   3        A half 1            A1 x B1           A half 0 of slab k + 2
+//   4        B half 0 of k + 1   A1 x B0           B half 1 of slab k + 2
+// Two barrier-separated halves make phase p's reads complete in every wave before the read half of phase p + 2 begins (the
+// reads have returned when the MFMA half ends), which is where that half tile may be overwritten; and a load has six
+// phases from its issue to its read.  Before a read half ends, a wave waits until its loads of five phases ago have
+// landed (the ten youngest may be on their way); the next phase's reads lie two barriers behind, so that holds for every
+// wave's share.
+//
+// A workgroup stays on its CU and goes through its tiles (the tile number advances by the number of workgroups), and the loads run on
+// into the next tile: when a tile's last MFMAs are done, the first slab and a half of the next are in the LDS or on their way, and the
+// epilogue touches neither.  It brings 32 rows of a wave tile at a time through 4 KiB of the wave's own, without a barrier.  The
+// operands of the MFMA are exchanged, so that a lane holds four neighbouring columns of a row, and the results are bf16 before they
+// are written there: 8 bytes a lane in, 16 bytes out, whole 128-byte lines to memory.  (Stores straight from the registers, 32 bytes
+// of a line each, take 9 - 20 us a tile: the L2 takes a request, not a byte, per clock.)  vmcnt counts loads and stores in the
+// order of their issue, so the first phases behind an epilogue let its 16 stores be on their way too.
+//
+// Time stamps in the kernel, 8192 x 8192 x 1024 on zeros (at the full clock), us a tile: before (a workgroup a tile, the epilogue
+// through 64 KiB of slab memory in four passes between barriers) prologue 2.8, 16 slabs 21 - 22, epilogue 7.9, gap 1.2; now 0.8, 21 -
+// 24 (the stores of the tile before drain beside its loads), 1.7 - 2.5.  On one tile a CU (4096 x 4096 x 2048) 49.9 -> 40.7.  Random
+// operands cost power, and the clock follows (1.5 - 1.9 us a slab instead of 1.1), so they gain less.  us, forward / input gradient /
+// weight gradient layout, before -> now: 8 of 1024 x 8192 x 2048 256 / 261 -> 232 / 238, 8 of 8192 x 2048 x 1024 - / - / 318 -> 286,
+// 4096 x 6144 x 2048 114 -> 99, 6000 x 6144 x 2048 169 -> 148, 6000 x 2048 x 2048 55 -> 51, 6144 x 2048 x 6000 - / - / 148 -> 141,
+// 8192^3 846 -> 798.
+// Closing the MFMA half before its last two MFMAs, so that the waves' MFMAs overlap, costs 10 - 20 %: the two waves of a SIMD then
+// drift into the same half.
+
+// The half tile of the rows r' = 0 .. 127 holds tile rows half_row<BLK>(r', h): blocks of BLK rows, every other one.
+template <int BLK>
+__device__ __forceinline__ constexpr int half_row(int r, int h) {
+  return ((r & ~(BLK - 1)) << 1) | (h * BLK) | (r & (BLK - 1));
+}
+
+// The kernel's arguments where they stand, in the kernel-argument segment, through a pointer that the compiler knows nothing
+// about: what is fetched through it is not kept in scalar registers over the K loops (all of them together do not fit).
+typedef const __attribute__((address_space(4))) GemmArgs* KernArgs;
+__device__ __forceinline__ KernArgs kernel_args() {
+  KernArgs q = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(q));
+  return q;
+}
+__device__ __forceinline__ unsigned fast_div(unsigned n, const __attribute__((address_space(4))) FastDiv& f) {
+  const unsigned t = __umulhi(n, f.mul);
+  return (t + ((n - t) >> f.s1)) >> f.s2;
+}
+
+// The lane's number, worked out anew: what is derived from it stands in registers only where it is used.  (Addresses of an epilogue
+// held over the K loop spill, and a spilled register's way back waits for all loads on their way to the LDS.)
+__device__ __forceinline__ int lane_now() {
+  int l;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+  return l;
+}
+
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+// LDS by byte address: base registers and constant offsets, which an LDS instruction adds by itself.
+typedef __attribute__((address_space(3))) char* lds_t;
+template <typename V>
+__device__ __forceinline__ V lds_load(unsigned at) {
+  return *(const __attribute__((address_space(3))) V*)(uintptr_t)at;
+}
+template <typename V>
+__device__ __forceinline__ void lds_store(unsigned at, V v) {
+  *(__attribute__((address_space(3))) V*)(uintptr_t)at = v;
+}
+
+// Where a lane's fragments of a half tile (128 rows, as DmaOperand leaves them) are: of BLOCKS blocks of 32 rows from `row0` on, in
+// the slab at `at`.  k-contiguous: an address for every k-step, the blocks at constant distances; row-contiguous the other way round.
+template <bool KC, int BLOCKS>
+struct FragPlace {
+  unsigned v[KC ? 4 : BLOCKS];
+  __device__ __forceinline__ void init(unsigned at, int row0, int lane) {
+    const int li = lane & 31, g = lane >> 5;
+    if (KC) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] = at + (row0 + li) * 128 + (((2 * q + g) ^ kc_swizzle<128>(li)) << 4);
+    } else {
+      const int s16 = lane & 15, kl = g * 8 + (s16 >> 2);
+#pragma unroll
+      for (int i = 0; i < BLOCKS; ++i) {
+        const int rb = (row0 + i * 32 + 16 * ((lane >> 4) & 1) + 4 * (s16 & 3)) * 2;
+        v[i] = at + kl * 256 + (((rb >> 4) ^ rc_swizzle<bf16_t, 128>(kl)) << 4) + (rb & 15);
+      }
+    }
+  }
+  __device__ __forceinline__ void other_slab(unsigned bytes) {
+#pragma unroll
+    for (int i = 0; i < (KC ? 4 : BLOCKS); ++i) v[i] ^= bytes;
+  }
+  // block i, k-step q of the half tile `half` bytes into the slab
+  __device__ __forceinline__ Frag<bf16_t> read(int half, int i, int q) const {
+    Frag<bf16_t> f;
+    if (KC) {
+      f.v = __builtin_bit_cast(bf16x8, lds_load<u32x4>(v[q] + half + i * 4096));
+    } else {
+      typedef short short8_t __attribute__((ext_vector_type(8)));
+      typedef __attribute__((address_space(3))) short4_t* tr_t;
+      const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_t)(uintptr_t)(v[i] + half + q * 4096));
+      const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_t)(uintptr_t)(v[i] + half + q * 4096 + 1024));
+      f.v = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    }
+    return f;
+  }
+};
+
+template <bool AKC, bool BKC>
+__global__ __launch_bounds__(512) void gemm_large_kernel(GemmArgs) {
+  using T = bf16_t;
+  constexpr int BM = 256, BN = 256, NL = 8, SB = 128;
+  constexpr int WM = 128, WN = 64, MT = 4, NT = 2;
+  constexpr int BLKA = WM / 2, BLKB = WN / 2;
+  using DA = DmaOperand<T, BM / 2, AKC, NL, SB>;
+  using DB = DmaOperand<T, BN / 2, BKC, NL, SB>;
+  constexpr int BK = SB / sizeof(T);
+  constexpr int KS = SB / 32;
+  constexpr int HALF = DA::BYTES, SLAB = 4 * HALF;
+  constexpr int NI = DA::NI;           // load instructions per wave and half tile
+  constexpr int NSTORE = MT * NT * 2;  // stores of a wave in a whole tile's epilogue, at least
+  constexpr int PAGE = 4096;           // a wave's own LDS: 32 rows of its 64 columns in bf16, or the bias of its columns
+  constexpr int kBiasSegs = 16;        // K segments whose biases are brought there
+  static_assert(DB::BYTES == HALF && DB::NI == NI && 5 * NI + NSTORE < 64, "half tiles of one size; vmcnt is a 6-bit counter");
+  static_assert(2 * SLAB + NL * PAGE <= 160 * 1024 && kBiasSegs * WN * 2 <= PAGE, "160 KiB of LDS");
+  __shared__ __attribute__((aligned(1024))) char lds[2 * SLAB + NL * PAGE];  // [slab & 1][A0, A1, B0, B1], pages
+
+  touch_kernel_arguments<sizeof(GemmArgs)>();
+  const KernArgs args = kernel_args();
+  const int tid = threadIdx.x;
+  if (args->trace != nullptr && tid == 0) atomicMin(args->trace, (unsigned long long)wall_clock64());
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 2, wn = wave & 3;
+
+  // ---- the tiles of this workgroup ----
+  const unsigned xcd = blockIdx.x & 7, stride = gridDim.x >> 3;
+  const unsigned chunk = args->xg != 0 ? 0 : xcd * args->per_xcd;  // where no split into bricks fits: an eighth of the tiles
+  const unsigned mine = args->xg != 0 ? args->per_xcd : chunk >= args->tiles ? 0 : min(args->per_xcd, args->tiles - chunk);
+  unsigned slot = blockIdx.x >> 3;
+  if (slot >= mine) return;
+  struct Tile {
+    int m0, n0, grp, zo, zi;
+    const char *a, *b;
+  };
+  auto tile_at = [&](unsigned s) {
+    const KernArgs p = kernel_args();
+    const unsigned in_brick = p->xg != 0 ? ~0u : 0u;
+    s += chunk;
+    const unsigned zl = fast_div(s, p->d_brick), t = s - zl * p->d_brick.d;
+    const unsigned q = fast_div(t, p->d_panel), r = t - q * p->d_panel.d;
+    const unsigned cn = fast_div(r, p->d_prow), cm = r - cn * p->d_prow.d;
+    const unsigned qn = fast_div(q, p->d_pm), qm = q - qn * p->d_pm.d;
+    const unsigned bn = xcd & ((1u << p->xn_shift) - 1), bm = (xcd >> p->xn_shift) & ((1u << p->xm_shift) - 1);
+    const unsigned bz = xcd >> (p->xn_shift + p->xm_shift);
+    const int tn = (int)((in_brick & (bn * p->nbk)) + qn * p->pcol + cn);
+    const int tm = (int)((in_brick & (bm * p->mbk)) + qm * p->prow + cm);
+    const int z = (int)((in_brick & (bz * p->zbk)) + zl);
+    Tile w;
+    w.m0 = tm * BM, w.n0 = tn * BN;
+    w.grp = (int)fast_div(z, p->d_batch);
+    const int zb = z - w.grp * (int)p->d_batch.d;
+    w.zo = (int)fast_div(zb, p->d_zdiv), w.zi = zb - w.zo * (int)p->d_zdiv.d;
+    w.a = DA::slab_base(reinterpret_cast<const T*>(p->a) + w.grp * p->a_sg + w.zo * p->a_so + w.zi * p->a_si, p->lda, w.m0);
+    w.b = DB::slab_base(reinterpret_cast<const T*>(p->b) + w.grp * p->b_sg + w.zo * p->b_so + w.zi * p->b_si, p->ldb, w.n0);
+    return w;
+  };
+  const int kdim = args->k, rows_a = args->m, rows_b = args->n;
+  const long lda = args->lda, ldb = args->ldb;
+  const int nk_seg = (kdim + BK - 1) / BK;
+  const int nk = nk_seg * args->ksegs;
+
+  f32x16 acc[MT][NT];
+  float rsum[MT];
+  auto clear = [&] {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      rsum[i] = 0.0f;
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    }
+  };
+
+  // ---- this wave's share of the loads, which run ahead of the products and into the next tile ----
+  Tile here = tile_at(slot), next = here;
+  DA da[2];
+  DB db[2];
+  auto init_a = [&](const Tile& w) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) da[h].init(lda, w.m0, rows_a, wave, lane_now(), [=](int r) { return half_row<BLKA>(r, h); });
+  };
+  auto init_b = [&](const Tile& w) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) db[h].init(ldb, w.n0, rows_b, wave, lane_now(), [=](int r) { return half_row<BLKB>(r, h); });
+  };
+  init_a(here);
+  init_b(here);
+  const char *ca = here.a, *cb = here.b;
+  constexpr long SZ = (long)sizeof(T);
+  const long step_a = (AKC ? (long)BK : (long)BK * lda) * SZ, step_b = (BKC ? (long)BK : (long)BK * ldb) * SZ;
+  const int k0_last = (nk_seg - 1) * BK;
+  const int tail = kdim % BK != 0;
+  const unsigned lds0 = (unsigned)(uintptr_t)(lptr_t)lds;
+  // Slabs behind the one at ca / cb in its K segment; segments behind that one; the lanes whose vectors lie inside the contraction.
+  int left = nk_seg, segs = args->ksegs - 1;
+  unsigned long long in_a[NI], in_b[NI];
+  int ragged = 0;  // not all of them do
+  auto inside = [&](auto KC, unsigned long long(&m)[NI]) {
+    const int l = lane_now();
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int j = wave * NI + i, k = decltype(KC)::value ? ((l & 7) ^ kc_swizzle<SB>(j * 8 + (l >> 3))) * 8 : j * 4 + (l >> 4);
+      m[i] = __ballot(k0_last + k < kdim);
+    }
+    ragged = 1;
+  };
+  auto all_inside = [&] {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) in_a[i] = in_b[i] = ~0ull;
+    ragged = 0;
+  };
+  // To the next slab of the tile or the first of the next tile.  The loop around the products is one piece of code, whose rare
+  // events are short branches that are not taken: a second copy of its MFMAs (for slabs without events, say) joins the
+  // first in 128 accumulators, and the compiler then moves those about.
+  auto step = [&] {
+    if (__builtin_expect(left <= 1, 0)) {
+      if (left == 0) {
+        const KernArgs p = kernel_args();
+        if (segs != 0) {
+          ca += p->a_sk * SZ - nk_seg * step_a, cb += p->b_sk * SZ - nk_seg * step_b;
+          --segs;
+        } else {
+          if (rows_a % BM != 0) init_a(next);
+          if (rows_b % BN != 0) init_b(next);
+          ca = next.a - step_a, cb = next.b - step_b, segs = p->ksegs - 1;
+        }
+        left = nk_seg;
+        all_inside();
+      }
+      if (tail && left == 1) inside(std::bool_constant<AKC>{}, in_a), inside(std::bool_constant<BKC>{}, in_b);
+    }
+    ca += step_a, cb += step_b, --left;
+  };
+  // Half tile h of an operand into the slab at byte `at` of the LDS; vectors beyond the contraction become zeros.
+  auto issue = [&](const auto& d, const unsigned long long(&m)[NI], unsigned at, const char* base) {
+    const unsigned to = lds0 + at + wave * (NI * 1024);
+    static_assert(NI == 2, "two loads");
+    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %2\n\tglobal_load_lds_dwordx4 %4, %6\n\t"
+                 "s_mov_b32 m0, %1\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %5, %6\n\ts_mov_b64 exec, -1"
+                 :
+                 : "s"(to), "s"(to + 1024), "s"(m[0]), "s"(m[1]), "v"(d.ofs[0]), "v"(d.ofs[1]), "s"(base)
+                 : "memory");
+    if (__builtin_expect(ragged, 0)) {
+      const int l = lane_now();
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+        if (!(m[i] >> l & 1)) lds_store<u32x4>(to + i * 1024 + l * 16, u32x4{0u, 0u, 0u, 0u});
+    }
+  };
+  auto issue_a = [&](unsigned at, auto H) { issue(da[decltype(H)::value], in_a, at + decltype(H)::value * HALF, ca); };
+  auto issue_b = [&](unsigned at, auto H) { issue(db[decltype(H)::value], in_b, at + (2 + decltype(H)::value) * HALF, cb); };
+
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  Frag<T> fa[2][KS], fb0[KS], fb0n[KS], fb1[KS];  // B half 0 of the next slab is read while this slab's is multiplied
+  FragPlace<AKC, 2> pa;
+  FragPlace<BKC, 1> pb;
+  pa.init(lds0, wm * BLKA, lane);
+  pb.init(lds0 + 2 * HALF, wn * BLKB, lane);
+  bool rowsum = false;
+  auto read_a = [&](auto H) {
+#pragma unroll
+    for (int q = 0; q < KS; ++q)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) fa[i][q] = pa.read(decltype(H)::value * HALF, i, q);
+  };
+  auto read_b = [&](auto H, Frag<T>(&fb)[KS]) {
+#pragma unroll
+    for (int q = 0; q < KS; ++q) fb[q] = pb.read(decltype(H)::value * HALF, 0, q);
+  };
+  auto barrier = [] {
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // the barrier that ends a read half, the MFMA half and its end, where this wave's reads have returned (the first MFMAs
+  // wait only for their own fragments)
+  auto multiply = [&](auto H, auto J, const Frag<T>(&fb)[KS], bool sums) {
+    constexpr int h = decltype(H)::value, j = decltype(J)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    barrier();
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int q = 0; q < KS; ++q)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) mma(fb[q], fa[i][q], acc[h * 2 + i][j]);  // transposed: a lane holds columns of one row
+    __builtin_amdgcn_s_setprio(0);
+    if (!AKC && sums && rowsum) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int q = 0; q < KS; ++q) rsum[h * 2 + i] = frag_sum(fa[i][q], rsum[h * 2 + i]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    barrier();
+  };
+  int behind = 0;    // phases whose loads are older than the last epilogue's stores
+  unsigned cur = 0;  // byte of the LDS where the slab being multiplied is
+  // the loads of five phases ago have landed
+  auto landed = [&] {
+    RTP_WAIT_VM(5 * NI + NSTORE);
+    if (__builtin_expect(behind == 0, 1)) RTP_WAIT_VM(5 * NI);
+    behind = behind != 0 ? behind - 1 : 0;
+  };
+  // A slab.  REST: slabs of this and the following tile behind it (2: two or more).
+  auto slab = [&](auto REST) {
+    constexpr int rest = decltype(REST)::value;
+    const unsigned other = cur ^ SLAB;
+    read_a(I0{});
+    if constexpr (rest >= 1) issue_a(other, I1{});
+    if constexpr (rest >= 1) landed();
+    else RTP_WAIT_VM(NI);
+    multiply(I0{}, I0{}, fb0, true);
+
+    read_b(I1{}, fb1);
+    if constexpr (rest >= 2) step();
+    if constexpr (rest >= 2) issue_b(cur, I0{});
+    pb.other_slab(SLAB);
+    if constexpr (rest >= 2) landed();
+    else if constexpr (rest == 1) RTP_WAIT_VM(4 * NI);
+    else RTP_WAIT_VM(0);
+    multiply(I0{}, I1{}, fb1, false);
+
+    read_a(I1{});
+    if constexpr (rest >= 2) issue_a(cur, I0{});
+    if constexpr (rest >= 2) landed();
+    else if constexpr (rest == 1) RTP_WAIT_VM(3 * NI);
+    multiply(I1{}, I1{}, fb1, true);
+
+    if constexpr (rest >= 1) read_b(I0{}, fb0n);
+    if constexpr (rest >= 2) issue_b(cur, I1{});
+    pa.other_slab(SLAB);
+    if constexpr (rest >= 2) landed();
+    else if constexpr (rest == 1) RTP_WAIT_VM(2 * NI);
+    multiply(I1{}, I0{}, fb0, false);
+    if constexpr (rest >= 1) {
+#pragma unroll
+      for (int q = 0; q < KS; ++q) fb0[q] = fb0n[q];
+    }
+    cur = other;
+  };
+
+  const unsigned page = lds0 + 2 * SLAB + wave * PAGE;
+  // Eight neighbouring columns of a row per lane: columns 16 h + 8 g of block (i, j), after the two halves of the wave have
+  // exchanged four of them.
+  auto columns = [&](const f32x16& c, auto H, float(&v)[8]) {
+    constexpr int h = decltype(H)::value;
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const u32x2 r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, (float)c[8 * h + e]),
+                                                       __builtin_bit_cast(unsigned, (float)c[8 * h + 4 + e]), false, false);
+      const unsigned lo = r.x, hi = r.y;  // (the cast of a vector's element itself would be one of element 0)
+      v[e] = __builtin_bit_cast(float, lo), v[4 + e] = __builtin_bit_cast(float, hi);
+    }
+  };
+  // the bias of columns col0 + 8 g .. + 7: by scalar loads, which no vector load or store has to be waited for
+  auto bias8 = [&](KernArgs p, const Tile& w, int col, int g, float(&v)[8]) {
+    typedef const __attribute__((address_space(4))) u32x4* scalar_t;
+    const T* bias = reinterpret_cast<const T*>(p->bias) + w.grp * p->bias_sg + w.zo * p->bias_so + w.zi * p->bias_si;
+    const T *lo = bias + (col < rows_b ? col : 0), *hi = bias + (col + 8 < rows_b ? col + 8 : 0);
+    const int nb_seg = p->bias_sk ? p->ksegs : 1;  // a bias per K segment is summed in segment order
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = 0.0f;
+#pragma unroll 1
+    for (int sgm = 0; sgm < nb_seg; ++sgm) {
+      const u32x4 s0 = *(scalar_t)(uintptr_t)(lo + sgm * p->bias_sk), s1 = *(scalar_t)(uintptr_t)(hi + sgm * p->bias_sk);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const unsigned two = g ? s1[e] : s0[e];
+        v[2 * e] += __builtin_bit_cast(float, two << 16);
+        v[2 * e + 1] += __builtin_bit_cast(float, two & 0xffff0000u);
+      }
+    }
+  };
+  // Whole tiles, results in bf16, addend (ADD) or mask (MASK) or bias or none: 32 rows at a time go through the wave's page, so that
+  // loads and stores are whole lines (8 lanes a row, 16 bytes a lane).  An addend passes it in the other direction first.
+  auto finish = [&](const Tile& w, auto ADD, auto MASK, auto BIAS, auto RELU) {
+    constexpr bool add = decltype(ADD)::value, mask = decltype(MASK)::value, bias = decltype(BIAS)::value, relu = decltype(RELU)::value;
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    const KernArgs p = kernel_args();
+    const int lane = lane_now(), li = lane & 31, g = lane >> 5;
+    const bool stream_out = p->flags & RTP_GEMM_STREAM_OUT;
+    const int row0 = w.m0 + wm * WM, col0 = w.n0 + wn * WN;
+    const int lr = lane >> 3, lc = (lane & 7) * 8;  // row (and + 8, 16, 24) and column of this lane's lines
+    const long ldc = p->ldc, ld_in = mask ? p->ld_gate : p->ld_cin;
+    T* dst = reinterpret_cast<T*>(p->c_out) + w.grp * p->c_sg + w.zo * p->c_so + w.zi * p->c_si + (row0 + lr) * ldc + col0 + lc;
+    u32x4 in[MT][4];
+    if constexpr (add || mask) {
+      const T* src = mask ? reinterpret_cast<const T*>(p->gate) + w.grp * p->gate_sg + w.zo * p->gate_so + w.zi * p->gate_si
+                          : reinterpret_cast<const T*>(p->c_in) + w.grp * p->cin_sg + w.zo * p->cin_so + w.zi * p->cin_si;
+      src += (row0 + lr) * ld_in + col0 + lc;
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) in[i][s] = *reinterpret_cast<const u32x4*>(src + (i * 32 + s * 8) * ld_in);
+    }
+    float b[NT][4][4];  // of columns 32 j + 8 t + 4 g ..
+    if constexpr (bias) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) b[j][t][e] = 0.0f;
+      const int nb_seg = p->bias_sk ? p->ksegs : 1;  // a bias per K segment is summed in segment order
+#pragma unroll 1
+      for (int sgm = 0; sgm < nb_seg; ++sgm)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const bf16x4 x = __builtin_bit_cast(bf16x4, lds_load<u32x2>(page + sgm * (WN * 2) + (j * 32 + t * 8 + 4 * g) * 2));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) b[j][t][e] += (float)x[e];
+          }
+    }
+    const unsigned wr = page + li * 128 + 8 * g, rd = page + lr * 128;  // 16-byte chunk c of row r is at chunk c ^ (r >> 1 & 7)
+    const unsigned swz = (li >> 1) & 7;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      if constexpr (add) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+          lds_store<u32x4>(rd + s * 1024 + (((lane & 7) ^ (((lr + s * 8) >> 1) & 7)) << 4), in[i][s]);
+      }
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const unsigned at = wr + ((unsigned)((j * 4 + t) ^ swz) << 4);
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = acc[i][j][4 * t + e];
+          if constexpr (add) {
+            const bf16x4 x = __builtin_bit_cast(bf16x4, lds_load<u32x2>(at));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += (float)x[e];
+          }
+          if constexpr (bias) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += b[j][t][e];
+          }
+          if constexpr (relu) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = fmaxf(v[e], 0.0f);
+          }
+          bf16x4 o;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = from_f32<T>(v[e]);
+          lds_store<u32x2>(at, __builtin_bit_cast(u32x2, o));
+        }
+      u32x4 o[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        o[s] = lds_load<u32x4>(rd + s * 1024 + (((lane & 7) ^ (((lr + s * 8) >> 1) & 7)) << 4));
+        if constexpr (mask) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const unsigned two = in[i][s][e], lo = two << 16, hi = two & 0xffff0000u;
+            o[s][e] = (__builtin_bit_cast(float, lo) > 0.0f ? o[s][e] & 0xffffu : 0u) |
+                      (__builtin_bit_cast(float, hi) > 0.0f ? o[s][e] & 0xffff0000u : 0u);
+          }
+        }
+      }
+      if (stream_out) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) __builtin_nontemporal_store(o[s], reinterpret_cast<u32x4*>(dst + s * 8 * ldc));
+      } else {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) *reinterpret_cast<u32x4*>(dst + s * 8 * ldc) = o[s];
+      }
+      dst += 32 * ldc;
+    }
+  };
+  // everything else, block after block in a loop
+  auto finish_any = [&](const Tile& w, bool whole) {
+    const KernArgs p = kernel_args();
+    const int lane = lane_now(), li = lane & 31, g = lane >> 5;
+    const int flags = p->flags;
+    const bool stream_out = flags & RTP_GEMM_STREAM_OUT, relu = flags & RTP_GEMM_RELU;
+    const bool out_f32 = flags & RTP_GEMM_OUT_F32, cin_f32 = flags & RTP_GEMM_CIN_F32;
+    char* cbase = p->c_out + (w.grp * p->c_sg + w.zo * p->c_so + w.zi * p->c_si) * (out_f32 ? 4 : SZ);
+    const char* cin = p->c_in ? p->c_in + (w.grp * p->cin_sg + w.zo * p->cin_so + w.zi * p->cin_si) * (cin_f32 ? 4 : SZ) : nullptr;
+    const T* gate =
+        p->gate ? reinterpret_cast<const T*>(p->gate) + w.grp * p->gate_sg + w.zo * p->gate_so + w.zi * p->gate_si : nullptr;
+#pragma unroll 1
+    for (int blk = 0; blk < MT * NT; ++blk) {
+      f32x16 part;
+      // (an empty instruction per copy: merged into one copy from a computed place, the accumulators would have to be in memory)
+      auto take = [&](const f32x16& from) {
+        part = from;
+        asm volatile("" : "+v"(part));
+      };
+      switch (blk) {
+        case 0: take(acc[0][0]); break;
+        case 1: take(acc[0][1]); break;
+        case 2: take(acc[1][0]); break;
+        case 3: take(acc[1][1]); break;
+        case 4: take(acc[2][0]); break;
+        case 5: take(acc[2][1]); break;
+        case 6: take(acc[3][0]); break;
+        default: take(acc[3][1]);
+      }
+      const int row = w.m0 + wm * WM + (blk >> 1) * 32 + li, col0 = w.n0 + wn * WN + (blk & 1) * 32;
+      const long rowc = row < rows_a ? row : rows_a - 1;
+      Raw8<T> rg[2], rc16[2];
+      Raw8<float> rc32[2];
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int col = col0 + 16 * c + 8 * g, colc = col < rows_b ? col : 0;
+        if (cin) {
+          if (cin_f32)
+            rc32[c].load(reinterpret_cast<const float*>(cin) + rowc * p->ld_cin + colc);
+          else
+            rc16[c].load(reinterpret_cast<const T*>(cin) + rowc * p->ld_cin + colc);
+        }
+        if (gate) rg[c].load(gate + rowc * p->ld_gate + colc);
+      }
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int col = col0 + 16 * c + 8 * g;
+        float v[8], t[8];
+        if (c & 1)
+          columns(part, I1{}, v);
+        else
+          columns(part, I0{}, v);
+        if (cin) {
+          if (cin_f32)
+            rc32[c].get(t);
+          else
+            rc16[c].get(t);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] += t[e];
+        }
+        if (p->bias) {
+          bias8(p, w, col0 + 16 * c, g, t);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] += t[e];
+        }
+        if (relu) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = fmaxf(v[e], 0.0f);
+        }
+        if (gate) {
+          rg[c].get(t);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = t[e] > 0.0f ? v[e] : 0.0f;
+        }
+        if (whole || (row < rows_a && col < rows_b)) {
+          if (p->xent_mode == 2) xent_gradient8<T>(*p, v, row, col, w.grp);
+          const long off = (long)row * p->ldc + col;
+          if (out_f32)
+            store8(reinterpret_cast<float*>(cbase) + off, v, stream_out);
+          else
+            store8(reinterpret_cast<T*>(cbase) + off, v, stream_out);
+        }
+      }
+    }
+  };
+  // how a tile is finished: 0 by the loop above, 1 plainly, 2 with a bias, 3 with a bias and a ReLU, 4 an addend, 5 a mask
+  auto finish_form = [&](const Tile& w) {
+    const KernArgs p = kernel_args();
+    const bool add = p->c_in != nullptr, mask = p->gate != nullptr, bias = p->bias != nullptr, relu = p->flags & RTP_GEMM_RELU;
+    if (w.m0 + BM > rows_a || w.n0 + BN > rows_b || (int)add + (int)mask + (int)bias > 1 || (relu && !bias) || (p->flags & RTP_GEMM_OUT_F32) ||
+        (add && (p->flags & RTP_GEMM_CIN_F32)) || p->xent_mode != 0 || (bias && p->bias_sk && p->ksegs > kBiasSegs))
+      return 0;
+    return add ? 4 : mask ? 5 : relu ? 3 : bias ? 2 : 1;
+  };
+  // the biases of the wave's columns on their way to its page: 128 bytes a K segment, two of them a load; they have landed when
+  // the loads of the tile's second slab have
+  auto request_bias = [&](const Tile& w) {
+    const KernArgs p = kernel_args();
+    const int lane = lane_now(), li = lane & 31, g = lane >> 5;
+    const T* bias = reinterpret_cast<const T*>(p->bias) + w.grp * p->bias_sg + w.zo * p->bias_so + w.zi * p->bias_si + w.n0 + wn * WN;
+    const int nb_seg = p->bias_sk ? p->ksegs : 1;
+    for (int s0 = 0; s0 < nb_seg; s0 += 2) {
+      const int s = s0 + g < nb_seg ? s0 + g : s0;
+      const T* src = bias + s * p->bias_sk + 2 * li;
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(page + s0 * (WN * 2)), "v"(src) : "memory");
+    }
+  };
+  auto epilogue = [&](const Tile& w, int form) {
+    const KernArgs p = kernel_args();
+    using Yes = std::true_type;
+    using No = std::false_type;
+    if (!AKC && rowsum) {
+      const int lane = lane_now(), li = lane & 31, g = lane >> 5;
+      T* dst = reinterpret_cast<T*>(p->a_rowsum) + w.grp * p->rowsum_sg;
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        const float v = rsum[i] + __shfl_xor(rsum[i], 32, 64);
+        const int row = w.m0 + wm * WM + i * 32 + li;
+        if (g == 0 && row < rows_a) dst[row] = from_f32<T>((p->flags & RTP_GEMM_ROWSUM_ACCUM) ? to_f32(dst[row]) + v : v);
+      }
+    }
+    if (p->alpha != 1.0f) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[i][j][r] *= p->alpha;
+    }
+    if (form == 0)
+      finish_any(w, w.m0 + BM <= rows_a && w.n0 + BN <= rows_b);
+    else if (form == 1)
+      finish(w, No{}, No{}, No{}, No{});
+    else if (form == 2)
+      finish(w, No{}, No{}, Yes{}, No{});
+    else if (form == 3)
+      finish(w, No{}, No{}, Yes{}, Yes{});
+    else if (form == 4)
+      finish(w, Yes{}, No{}, No{}, No{});
+    else
+      finish(w, No{}, Yes{}, No{}, No{});
+  };
+
+  // what phases before the first would have issued, in their order; the host sends no problem of a single slab here
+  all_inside();
+  if (left == 1 && tail) inside(std::bool_constant<AKC>{}, in_a), inside(std::bool_constant<BKC>{}, in_b);
+  --left;
+  issue_b(0, I0{});
+  issue_a(0, I0{});
+  issue_b(0, I1{});
+  issue_a(0, I1{});
+  step();
+  issue_b(SLAB, I0{});
+  issue_a(SLAB, I0{});
+  issue_b(SLAB, I1{});
+  clear();
+  RTP_WAIT_VM(5 * NI);  // halves 0 of slab 0 have landed
+  barrier();
+  read_b(I0{}, fb0);
+  __builtin_amdgcn_sched_barrier(0);
+  for (;;) {
+    const bool more = slot + stride < mine;
+    slot += stride;
+    if (more) next = tile_at(slot);
+    const int form = finish_form(here);
+    if (form == 2 || form == 3) request_bias(here);
+    rowsum = !AKC && kernel_args()->a_rowsum != nullptr && here.n0 == 0 && wn == 0;
+    if (wm == 1) __builtin_amdgcn_s_barrier();
+    for (int todo = more ? nk : nk - 2; todo > 0; --todo) slab(std::integral_constant<int, 2>{});
+    if (!more) {
+      slab(I1{});
+      slab(I0{});
+    }
+    if (wm == 0) __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    epilogue(here, form);
+    if (!more) break;
+    asm volatile("" ::: "memory");
+    behind = here.m0 + BM <= rows_a && here.n0 + BN <= rows_b ? 5 : 0;
+    clear();
+    here = next;
+  }
+  if (kernel_args()->trace != nullptr && tid == 0) atomicMax(kernel_args()->trace + 1, (unsigned long long)wall_clock64());
+}
+
+int launch_large(hipStream_t s, const GemmArgs& a, bool akc, bool bkc) {
+  const dim3 block(512), grid(8 * (a.per_xcd < 32 ? a.per_xcd : 32));
+  if (akc && bkc)
+    hipLaunchKernelGGL((gemm_large_kernel<true, true>), grid, block, 0, s, a);
+  else if (akc && !bkc)
+    hipLaunchKernelGGL((gemm_large_kernel<true, false>), grid, block, 0, s, a);
+  else if (!akc && bkc)
+    hipLaunchKernelGGL((gemm_large_kernel<false, true>), grid, block, 0, s, a);
+  else
+    hipLaunchKernelGGL((gemm_large_kernel<false, false>), grid, block, 0, s, a);
+  RTP_LAUNCH_CHECK();
+  return RTP_OK;
+}
+
+}  // namespace rtp

@@ -38,6 +38,7 @@ struct GemmArgs {
   FastDiv d_batch, d_zdiv, d_tiles_n, d_brick, d_panel, d_prow, d_pm;  // divisors mbk*nbk, prow*pcol, prow, mbk/prow
   int mbk, nbk, prow, pcol;
   int xn_shift, xm_shift, zbk;  // log2 of xn and xm, batch*groups entries per brick
+  unsigned tiles, per_xcd;      // all tiles of the launch, an XCD's share of them (rounded up)
   unsigned long long* trace;    // null, or two words: earliest start / latest end of the launch on the wall clock
   float* sgd_master;            // null, or the fp32 parameters the product updates (indexed like c_out)
   char* sgd_w;                  // null, or the compute-dtype copy of the parameters
@@ -217,8 +218,8 @@ struct Raw8 {
 
 // Eight logits -> their cross-entropy gradient: (softmax - onehot(target)) * dloss (* scale); rows whose target is the
 // ignore index or outside the classes get zeros.
-template <typename T>
-__device__ __forceinline__ void xent_gradient8(const GemmArgs& p, float (&v)[8], long row, int col, int grp) {
+template <typename T, typename Args>  // (the arguments in either address space)
+__device__ __forceinline__ void xent_gradient8(Args& p, float (&v)[8], long row, int col, int grp) {
   const long tg = p.xent_target[row];
   const bool live = tg != p.xent_ignore && tg >= 0 && tg < (long)p.xent_blocks * 64;
   const float2 st = p.xent_stats[row];
@@ -872,6 +873,9 @@ struct RegOperand {
 
 // The fp32 products of gemm_split.hip, in tiles of bm (128 or 64) x 64; ragged: an operand is not vector-aligned.
 int launch_split(hipStream_t s, const GemmArgs& a, bool akc, bool bkc, int bm, bool ragged, dim3 grid);
+
+// bf16 products in tiles of 256 x 256 by workgroups that stay (gemm_large.hip); two K slabs or more, no update, no statistics.
+int launch_large(hipStream_t s, const GemmArgs& a, bool akc, bool bkc);
 
 // Many tiles of 128 x 128 over a K slab or two (gemm_shortk.hip).
 int launch_shortk(hipStream_t s, const GemmArgs& a, bool bf16, bool akc, bool bkc, dim3 grid);

@@ -1,0 +1,112 @@
+"""The 256 x 256 product kernel where a workgroup goes through several tiles: its loads run on into the next tile while the epilogue of
+the last one is written, so every form of the epilogue, K segment ends, ragged last slabs and ragged tiles are met between two tiles.
+Against torch's fp32 product of the same values on the device; bf16 results within their rounding (TOL), fp32 ones within 1e-5, which
+covers some hundred fp32 additions an element."""
+import pytest
+import torch
+
+from test_gpu_gemm import DEV, TOL, _rand, rel_err
+from test_gpu_gemm_256 import _pair, _run
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+
+# 17 x 17 and 33 x 17 tiles, ragged in both directions: no split over the XCDs; 16 x 24: bricks
+SHAPES = [(4344, 4264), (8200, 4344), (4096, 6144)]
+
+
+@pytest.mark.parametrize("akc,bkc", [(True, True), (True, False), (False, False), (False, True)])
+@pytest.mark.parametrize("m,n", SHAPES)
+@pytest.mark.parametrize("k", [136, 192, 264])
+def test_plain(akc, bkc, m, n, k):
+    """Three slabs with a ragged last one, three whole ones, five with a ragged one."""
+    gen = torch.Generator().manual_seed(m + k)
+    a, b, ref = _pair(gen, m, n, k, akc, bkc)
+    out = torch.full((m, n), float("nan"), dtype=BF, device=DEV)
+    _run(a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=a.stride(0), ldb=b.stride(0), ldc=n,
+         a_kcontig=akc, b_kcontig=bkc)
+    assert rel_err(out, ref) <= TOL[BF]
+
+
+@pytest.mark.parametrize("m,n", SHAPES)
+@pytest.mark.parametrize("form", ["bias", "bias+relu", "relu", "addend", "mask", "mask+addend", "bias+addend", "alpha", "stream",
+                                  "fp32", "fp32 addend", "row sums"])
+def test_epilogues(m, n, form):
+    gen = torch.Generator().manual_seed(n)
+    k = 200
+    akc = form != "row sums"
+    a, b, ref = _pair(gen, m, n, k, akc, akc)
+    kw, dt = {}, BF
+    if form == "alpha":
+        kw["alpha"], ref = 0.125, ref * 0.125
+    if "addend" in form:
+        c = _rand((m, n), torch.float32 if "fp32" in form else BF, gen).to(DEV)
+        kw.update(c_in=c.data_ptr(), ld_cin=n, cin_f32="fp32" in form)
+        ref = ref + c.float()
+    if "bias" in form:
+        bias = _rand((n,), BF, gen).to(DEV)
+        kw["bias"], ref = bias.data_ptr(), ref + bias.float()
+    if "relu" in form:
+        kw["relu"], ref = True, ref.clamp(min=0)
+    if "mask" in form:
+        gate = _rand((m, n), BF, gen).to(DEV)
+        gate[::3, ::5] = 0.0
+        gate[1::7, 3::11] = float("nan")
+        kw.update(gate=gate.data_ptr(), ld_gate=n)
+        ref = torch.where(gate.float() > 0, ref, torch.zeros_like(ref))
+    if form == "stream":
+        kw["stream_out"] = True
+    if form == "fp32":
+        kw["out_f32"], dt = True, torch.float32
+    sums = torch.full((m,), float("nan"), dtype=BF, device=DEV)
+    if form == "row sums":
+        kw["rowsum"] = sums.data_ptr()
+    out = torch.full((m, n), float("nan"), dtype=dt, device=DEV)
+    done = _run(a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=a.stride(0), ldb=b.stride(0), ldc=n,
+                a_kcontig=akc, b_kcontig=akc, **kw)
+    assert rel_err(out, ref) <= (TOL[BF] if dt == BF else 1e-5)
+    if form == "row sums":
+        assert done and rel_err(sums, a.float().sum(0)) <= TOL[BF]
+
+
+@pytest.mark.parametrize("segs,k", [(2, 72), (3, 64), (17, 64)])
+def test_segments_and_their_biases(segs, k):
+    """K segments that end inside a tile, of one slab and of two with a ragged one; a bias a segment (17: more than a wave's page holds)."""
+    gen = torch.Generator().manual_seed(segs)
+    m, n = 4096, 6144
+    a = _rand((segs, m, k), BF, gen).to(DEV)
+    b = _rand((segs, n, k), BF, gen).to(DEV)
+    bias = _rand((segs, n), BF, gen).to(DEV)
+    ref = bias.float().sum(0) + sum(a[s].float() @ b[s].float().t() for s in range(segs))
+    out = torch.full((m, n), float("nan"), dtype=BF, device=DEV)
+    _run(a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=k, ldb=k, ldc=n, a_kcontig=True,
+         b_kcontig=True, ksegs=segs, a_sk=m * k, b_sk=n * k, bias=bias.data_ptr(), bias_sk=n)
+    assert rel_err(out, ref) <= TOL[BF]
+
+
+@pytest.mark.parametrize("groups", [3, 8])
+def test_groups(groups):
+    """Tiles of several groups, with and without a split over the XCDs, a bias a group."""
+    gen = torch.Generator().manual_seed(groups)
+    m, n, k = 2056, 4104, 264
+    a = _rand((groups, m, k), BF, gen).to(DEV)
+    b = _rand((groups, k, n), BF, gen).to(DEV)
+    bias = _rand((groups, n), BF, gen).to(DEV)
+    out = torch.full((groups, m, n), float("nan"), dtype=BF, device=DEV)
+    _run(a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=k, ldb=n, ldc=n, a_kcontig=True, b_kcontig=False,
+         groups=groups, a_sg=m * k, b_sg=k * n, c_sg=m * n, bias=bias.data_ptr(), bias_sg=n)
+    for g in range(groups):
+        assert rel_err(out[g], a[g].float() @ b[g].float() + bias[g].float()) <= TOL[BF], g
+
+
+def test_values_beyond_the_contraction_do_not_count():
+    """What lies behind a row's last k in memory, and in the LDS from slabs before, may be anything."""
+    gen = torch.Generator().manual_seed(9)
+    m, n, k, ld = 4344, 4264, 136, 192
+    a = torch.full((m, ld), float("nan"), dtype=BF, device=DEV)
+    b = torch.full((n, ld), float("inf"), dtype=BF, device=DEV)
+    a[:, :k] = _rand((m, k), BF, gen).to(DEV)
+    b[:, :k] = _rand((n, k), BF, gen).to(DEV)
+    out = torch.full((m, n), float("nan"), dtype=BF, device=DEV)
+    _run(a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=ld, ldb=ld, ldc=n, a_kcontig=True, b_kcontig=True)
+    assert rel_err(out, a[:, :k].float() @ b[:, :k].float().t()) <= TOL[BF]

@@ -33,7 +33,7 @@ def test_plain(akc, bkc, m, n, k):
                                   "fp32", "fp32 addend", "row sums"])
 def test_epilogues(m, n, form):
     gen = torch.Generator().manual_seed(n)
-    k = 200
+    k = 520
     akc = form != "row sums"
     a, b, ref = _pair(gen, m, n, k, akc, akc)
     kw, dt = {}, BF

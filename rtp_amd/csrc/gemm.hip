@@ -16,6 +16,7 @@
 // ring of register buffers, which is what hides HBM/L2 latency when only one workgroup fits a CU.
 #include "gemm_tile.h"
 
+#include <algorithm>
 #include <atomic>
 #include <cstdlib>
 #include <type_traits>
@@ -1115,9 +1116,11 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   int shape = 3;  // 64 x 64 unless the model finds something cheaper
   double best = 0.0;
   for (int i = 0; fast && i < kNumShapes; ++i) {
-    // the 256 x 256 kernel is built for 16-bit operands and the plain epilogue (the update and the statistics epilogue
-    // are never routed to it, forced or not)
-    if (i == 5 && (sizeof(T) != 2 || d->sgd_master || d->xent_mode == 1)) continue;
+    // the 256 x 256 kernel is built for 16-bit operands and has no statistics epilogue (never routed to it, forced or not)
+    if (i == 5 && (sizeof(T) != 2 || d->xent_mode == 1)) continue;
+    // ... and an update only where it is a weight gradient's and the parameters' rows are whole 128-byte lines: its waves write 64
+    // columns each, and on rows that are not (3000 x 3000 x 512) it takes 49 us where 128 x 128 takes 38
+    if (i == 5 && d->sgd_master && (akc || bkc || d->ldc % 32 != 0)) continue;
     if (i == 6 && d->xent_mode == 1) continue;  // 160 columns are no whole number of 64-column statistics blocks
     if (!vec && i != 1 && i != 3) continue;  // the kernels for unaligned operands: 128 x 128 and 64 x 64
     // 128 x 160 is priced at the rate measured where it is meant for -- products of at most two rounds of tiles, such
@@ -1138,8 +1141,17 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
     const bool rare = (d->bias != nullptr) + (d->c_in != nullptr) + (d->gate != nullptr) > 1 || (relu && !d->bias) ||
                       (d->flags & (RTP_GEMM_OUT_F32 | RTP_GEMM_CIN_F32)) || d->xent_mode;
     const double outside = fixed_ns[i] + (i == 5 && rare ? 3000.0 : 0.0);
-    const double cost = (double)ceil_div(tiles, 256) *
-                        (vec ? nslabs * slab_ns[i] + outside : nslabs * odd_slab_ns[sizeof(T) == 4][i == 1] + odd_fixed_ns[i == 1]);
+    const double rounds = (double)ceil_div(tiles, 256);
+    // An update moves 10 bytes a parameter (12 with the gradient) behind the K loop, a round's tiles together at the memory's 4.9 TB/s, a CU at no
+    // more than 32 bytes a ns.  So few large tiles are behind where they leave CUs idle: us with 128 x 128 / 256 x 256, K = 1024, 2048 x 2048
+    // 19.2 / 39, 8 of 1280 x 2048 97 / 101, 6144 x 2048 59.7 / 49.9, 4096 x 4096 75 / 61; 8192 x 2048 x 4096 174 / 145.
+    double update = 0.0;
+    if (d->sgd_master && vec) {
+      const double tile_bytes = (double)kShapes[i].bm * kShapes[i].bn * (8.0 + (d->sgd_weights ? 2.0 : 0.0) + (d->flags & RTP_GEMM_SGD_SKIP_OUT ? 0.0 : 2.0));
+      const auto round_ns = [&](double n) { return std::max(n * tile_bytes / 4900.0, tile_bytes / 32.0); };
+      update = (rounds - 1.0) * round_ns(256.0) + round_ns((double)tiles - 256.0 * (rounds - 1.0));
+    }
+    const double cost = rounds * (vec ? nslabs * slab_ns[i] + outside : nslabs * odd_slab_ns[sizeof(T) == 4][i == 1] + odd_fixed_ns[i == 1]) + update;
     if (best == 0.0 || cost < best || i == forced) {
       best = i == forced ? -1.0 : cost;
       shape = i;

@@ -140,6 +140,7 @@ __global__ __launch_bounds__(512) void gemm_large_kernel(GemmArgs) {
   constexpr int NI = DA::NI;           // load instructions per wave and half tile
   constexpr int NSTORE = MT * NT * 2;  // stores of a wave in a whole tile's epilogue, at least
   constexpr int PAGE = 4096;           // a wave's own LDS: 32 rows of its 64 columns in bf16, or the bias of its columns
+  constexpr bool kUpdates = !AKC && !BKC;  // weight gradients may come with an update
   constexpr int kBiasSegs = 16;        // K segments whose biases are brought there
   static_assert(DB::BYTES == HALF && DB::NI == NI && 5 * NI + NSTORE < 64, "half tiles of one size; vmcnt is a 6-bit counter");
   static_assert(2 * SLAB + NL * PAGE <= 160 * 1024 && kBiasSegs * WN * 2 <= PAGE, "160 KiB of LDS");
@@ -274,9 +275,11 @@ __global__ __launch_bounds__(512) void gemm_large_kernel(GemmArgs) {
                  : "memory");
     if (__builtin_expect(ragged, 0)) {
       const int l = lane_now();
+      unsigned zero;
+      asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
 #pragma unroll
       for (int i = 0; i < NI; ++i)
-        if (!(m[i] >> l & 1)) lds_store<u32x4>(to + i * 1024 + l * 16, u32x4{0u, 0u, 0u, 0u});
+        if (!(m[i] >> l & 1)) lds_store<u32x4>(to + i * 1024 + l * 16, u32x4{zero, zero, zero, zero});
     }
   };
   auto issue_a = [&](unsigned at, auto H) { issue(da[decltype(H)::value], in_a, at + decltype(H)::value * HALF, ca); };
@@ -507,6 +510,82 @@ __global__ __launch_bounds__(512) void gemm_large_kernel(GemmArgs) {
       dst += 32 * ldc;
     }
   };
+  // Clip + SGD on the tile's parameters (the arithmetic of finish_tile_sgd): the gradients pass the wave's page in bf16, which is what the
+  // update takes them as, the fp32 parameters of 32 rows are requested while the 32 before them are finished.
+  auto finish_update = [&](const Tile& w, bool whole) {
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    const KernArgs p = kernel_args();
+    const int lane = lane_now(), li = lane & 31, g = lane >> 5;
+    const bool stream_out = p->flags & RTP_GEMM_STREAM_OUT, skip_out = p->flags & RTP_GEMM_SGD_SKIP_OUT, copy = p->sgd_w != nullptr;
+    const float lr_ = p->sgd_lr, clip = p->sgd_clip;
+    // this lane's row (and + 8, 16, 24) and columns (4 of the first 32, 4 of the others): eight lanes cover a line of fp32 parameters
+    const int lr = lane >> 3, l8 = lane & 7;
+    const int row0 = w.m0 + wm * WM + lr, col0 = w.n0 + wn * WN + 4 * l8;
+    const long ldc = p->ldc, zoff = w.grp * p->c_sg + w.zo * p->c_so + w.zi * p->c_si;
+    float* const master = p->sgd_master + zoff;
+    T* const wcopy = reinterpret_cast<T*>(p->sgd_w) + zoff;
+    T* const out = reinterpret_cast<T*>(p->c_out) + zoff;
+    const unsigned wr = page + li * 128 + 8 * g, swz = (li >> 1) & 7;
+    auto inside = [&](int row, int h) { return whole || (row < rows_a && col0 + 32 * h < rows_b); };
+    f32x4 par[2][2][2];  // of 16 rows
+    auto request = [&](int u) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int row = row0 + (u >> 1) * 32 + (2 * (u & 1) + s) * 8;
+          par[u & 1][s][h] =
+              __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(master + (inside(row, h) ? (long)row * ldc + col0 + 32 * h : 0)));
+        }
+      asm volatile("" ::: "memory");
+    };
+    request(0);
+#pragma unroll
+    for (int u = 0; u < 2 * MT; ++u) {
+      const int i = u >> 1;
+      if (u + 1 < 2 * MT) request(u + 1);
+      if (u % 2 == 0) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            bf16x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = from_f32<T>(acc[i][j][4 * t + e]);
+            lds_store<u32x2>(wr + ((unsigned)((j * 4 + t) ^ swz) << 4), __builtin_bit_cast(u32x2, o));
+          }
+      }
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int r = lr + (2 * (u & 1) + s) * 8, row = row0 + (u >> 1) * 32 + (2 * (u & 1) + s) * 8;
+          const u32x2 grad = lds_load<u32x2>(page + r * 128 + (((l8 >> 1) + 4 * h) ^ ((r >> 1) & 7)) * 16 + (l8 & 1) * 8);
+          const bf16x4 gr = __builtin_bit_cast(bf16x4, grad);
+          f32x4 x;
+          bf16x4 c;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            x[e] = sgd_update<T>(par[u & 1][s][h][e], (float)gr[e], lr_, clip);
+            c[e] = from_f32<T>(x[e]);
+          }
+          if (inside(row, h)) {
+            const long off = (long)row * ldc + col0 + 32 * h;
+            __builtin_nontemporal_store(x, reinterpret_cast<f32x4*>(master + off));
+            if (copy) __builtin_nontemporal_store(__builtin_bit_cast(u32x2, c), reinterpret_cast<u32x2*>(wcopy + off));
+            if (!skip_out) {
+              u32x2* to = reinterpret_cast<u32x2*>(out + off);
+              if (stream_out)
+                __builtin_nontemporal_store(grad, to);
+              else
+                *to = grad;
+            }
+          }
+        }
+    }
+  };
   // everything else, block after block in a loop
   auto finish_any = [&](const Tile& w, bool whole) {
     const KernArgs p = kernel_args();
@@ -592,10 +671,11 @@ __global__ __launch_bounds__(512) void gemm_large_kernel(GemmArgs) {
       }
     }
   };
-  // how a tile is finished: 0 by the loop above, 1 plainly, 2 with a bias, 3 with a bias and a ReLU, 4 an addend, 5 a mask
+  // how a tile is finished: 0 by the loop above, 1 plainly, 2 with a bias, 3 with a bias and a ReLU, 4 an addend, 5 a mask, 6 by an update
   auto finish_form = [&](const Tile& w) {
     const KernArgs p = kernel_args();
     const bool add = p->c_in != nullptr, mask = p->gate != nullptr, bias = p->bias != nullptr, relu = p->flags & RTP_GEMM_RELU;
+    if (kUpdates && p->sgd_master != nullptr) return 6;
     if (w.m0 + BM > rows_a || w.n0 + BN > rows_b || (int)add + (int)mask + (int)bias > 1 || (relu && !bias) || (p->flags & RTP_GEMM_OUT_F32) ||
         (add && (p->flags & RTP_GEMM_CIN_F32)) || p->xent_mode != 0 || (bias && p->bias_sk && p->ksegs > kBiasSegs))
       return 0;
@@ -636,8 +716,11 @@ __global__ __launch_bounds__(512) void gemm_large_kernel(GemmArgs) {
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[i][j][r] *= p->alpha;
     }
+    const bool whole = w.m0 + BM <= rows_a && w.n0 + BN <= rows_b;
     if (form == 0)
-      finish_any(w, w.m0 + BM <= rows_a && w.n0 + BN <= rows_b);
+      finish_any(w, whole);
+    else if (kUpdates && form == 6)
+      finish_update(w, whole);
     else if (form == 1)
       finish(w, No{}, No{}, No{}, No{});
     else if (form == 2)

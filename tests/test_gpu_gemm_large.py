@@ -110,3 +110,33 @@ def test_values_beyond_the_contraction_do_not_count():
     out = torch.full((m, n), float("nan"), dtype=BF, device=DEV)
     _run(a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=ld, ldb=ld, ldc=n, a_kcontig=True, b_kcontig=True)
     assert rel_err(out, a[:, :k].float() @ b[:, :k].float().t()) <= TOL[BF]
+
+
+@pytest.mark.parametrize("m,n,k", [(6144, 2048, 200), (4096, 4096, 136), (4104, 3808, 264)])
+@pytest.mark.parametrize("keep,clip", [(False, 0.05), (True, 0.0)])
+def test_update(m, n, k, keep, clip):
+    """Clip + SGD on a tile's parameters, several tiles a workgroup, ragged ones too: bit for bit the separate update of the gradients that the
+    same product leaves (which the kernel writes where they are kept)."""
+    class Sgd:
+        lr, keep_grads, missed = 1e-3, keep, False
+    Sgd.clip = clip
+    gen = torch.Generator().manual_seed(m + n)
+    a, b, ref = _pair(gen, m, n, k, False, False)
+    master = _rand((m, n), torch.float32, gen).to(DEV)
+    old, copy = master.clone(), torch.full((m, n), float("nan"), dtype=BF, device=DEV)
+    out = torch.full((m, n), float("nan"), dtype=BF, device=DEV)
+    kw = dict(a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=m, ldb=n, ldc=n, a_kcontig=False, b_kcontig=False)
+    _run(sgd=Sgd(), sgd_master=master.data_ptr(), sgd_weights=copy.data_ptr(), stream_out=True, **kw)
+    if keep:
+        assert rel_err(out, ref) <= TOL[BF]
+        grad = out.clone()
+    else:
+        assert out.isnan().all()
+        _run(**kw)
+        grad = out
+    g32 = grad.float()
+    if clip:
+        g32 = g32.clamp(-clip, clip)
+    step = Sgd.lr * g32
+    assert torch.equal(master, old - step)
+    assert torch.equal(copy, (old - step).to(BF))

@@ -23,7 +23,7 @@ from .. import ops
 from ..ring import rotation, run_wgrad
 from . import shard_ops as S
 from .collectives import RotatedLayer
-from .utils import (affine_weight, affine_weight_attention, as_rows, attention_block_index,
+from .utils import (affine_weight, affine_weight_attention, apply_function, as_rows, attention_block_index,
                     divide_and_check_no_remainder)
 
 
@@ -639,11 +639,11 @@ class ParallelMultiheadAttention(RotatedLayer):
                 if key_bias is not None:
                     key_bias = F.pad(key_bias, (0, extra))
             hides_only = all(m is None or m.dtype == torch.bool for m in (attn_mask, key_padding_mask))
-            out, weights = _GeneralAttentionFn.apply(x, k_in, v_in, self._anchor, self, mask, key_bias,
-                                                     bool(need_weights), drop_p, hides_only)
+            out, weights = apply_function(_GeneralAttentionFn, x, k_in, v_in, self._anchor, self, mask, key_bias,
+                                          bool(need_weights), drop_p, hides_only)
         else:
-            out, weights = _AttentionFn.apply(x, self._anchor, self, mask, causal, bool(need_weights),
-                                              bool(residual_grad), key_bias, drop_p)
+            out, weights = apply_function(_AttentionFn, x, self._anchor, self, mask, causal, bool(need_weights),
+                                          bool(residual_grad), key_bias, drop_p)
         if need_weights and weights is not None and average_attn_weights:
             weights = weights.float().mean(dim=1).to(out.dtype)
         if self.batch_first:

@@ -22,7 +22,7 @@ import torch.nn as nn
 from .. import ops
 from ..ring import rotation, run_wgrad
 from .collectives import RotatedLayer, resolve_world
-from .utils import affine_weight, divide_and_check_no_remainder
+from .utils import affine_weight, apply_function, divide_and_check_no_remainder
 
 
 class ModelParallelConv2d(nn.Conv2d):
@@ -142,7 +142,7 @@ class ColumnParallelConv2d(RotatedLayer):
         if input_.dim() != 4 or input_.shape[1] != self.in_channels:
             raise ValueError(f"ColumnParallelConv2d: expected an [N, {self.in_channels}, H, W] input, got "
                              f"{tuple(input_.shape)}")
-        return _ColumnConvFn.apply(input_, self._anchor, self)
+        return apply_function(_ColumnConvFn, input_, self._anchor, self)
 
     def extra_repr(self) -> str:
         return (f"{self.in_channels}, {self.out_channels}, kernel_size={self.kernel_size}, stride={self.stride}, "

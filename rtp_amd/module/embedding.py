@@ -18,7 +18,7 @@ from .. import ops
 from ..ring import rotation
 from .collectives import RotatedLayer
 from .shard_ops import _fused, _fused_done
-from .utils import affine_weight, divide_and_check_no_remainder
+from .utils import affine_weight, apply_function, divide_and_check_no_remainder
 
 
 class ModelParallelEmbedding(nn.Embedding):
@@ -144,7 +144,7 @@ class ParallelEmbedding(RotatedLayer):
     def forward(self, input_: torch.Tensor) -> torch.Tensor:
         if input_.dtype != torch.int64:
             input_ = input_.long()
-        return _EmbeddingFn.apply(input_, self._anchor, self)
+        return apply_function(_EmbeddingFn, input_, self._anchor, self)
 
     def forward_scaled_positional(self, input_: torch.Tensor, scale: float, pos: torch.Tensor) -> torch.Tensor:
         """(self(input_) * scale) + pos[:input_.size(0), None, :] in one gather per shard group, with the rounding
@@ -156,4 +156,4 @@ class ParallelEmbedding(RotatedLayer):
             raise ValueError("forward_scaled_positional: sequence longer than the positional table")
         if input_.dtype != torch.int64:
             input_ = input_.long()
-        return _EmbeddingFn.apply(input_, self._anchor, self, float(scale), pos)
+        return apply_function(_EmbeddingFn, input_, self._anchor, self, float(scale), pos)

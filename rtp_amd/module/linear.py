@@ -20,7 +20,7 @@ from .. import ops
 from ..ring import rotation, run_wgrad
 from . import shard_ops as S
 from .collectives import RotatedLayer, resolve_world
-from .utils import affine_weight, as_rows, divide_and_check_no_remainder
+from .utils import affine_weight, apply_function, as_rows, divide_and_check_no_remainder
 
 
 class ModelParallelLinear(nn.Linear):
@@ -200,7 +200,7 @@ def column_relu_mlp(x: torch.Tensor, lin1: "ColumnParallelLinear", lin2: "Column
         rows = x.numel() // x.shape[-1]
         keep = torch.empty(rows, lin1.out_features, dtype=x.dtype, device=x.device).bernoulli_(1.0 - dropout_p)
         keep.mul_(1.0 / (1.0 - dropout_p))
-    return _ColumnReluMlpFn.apply(x, lin1._anchor, lin2._anchor, lin1, lin2, bool(residual_grad), keep)
+    return apply_function(_ColumnReluMlpFn, x, lin1._anchor, lin2._anchor, lin1, lin2, bool(residual_grad), keep)
 
 
 class _RowLinearFn(torch.autograd.Function):
@@ -289,7 +289,7 @@ class _ParallelLinearBase(RotatedLayer):
         self.linear = self.linears[self.rank]
 
     def forward(self, input_: torch.Tensor) -> torch.Tensor:
-        return type(self)._fn.apply(input_, self._anchor, self)
+        return apply_function(type(self)._fn, input_, self._anchor, self)
 
     def extra_repr(self) -> str:
         return (f"in_features={self.in_features}, out_features={self.out_features}, bias={self.has_bias}, "

@@ -10,6 +10,7 @@ import torch.nn as nn
 
 from .. import ops
 from .. import ring as _ring
+from .utils import apply_function
 
 
 class _DeferredParamGrads:
@@ -142,4 +143,4 @@ def add_layer_norm(x: torch.Tensor, r: torch.Tensor, norm: nn.LayerNorm, x_grad_
         raise RtpError(f"add_layer_norm: x {tuple(x.shape)} {x.dtype} on {x.device}, branch {tuple(r.shape)} {r.dtype}, "
                        f"LayerNorm{tuple(norm.normalized_shape)}: needs device tensors of one dtype, a LayerNorm over "
                        "the last dimension with elementwise affine, rows of whole 16-byte vectors (at most 1024)")
-    return _AddLayerNormFn.apply(x, r, norm.weight, norm.bias, norm.eps, bool(x_grad_via_branch))
+    return apply_function(_AddLayerNormFn, x, r, norm.weight, norm.bias, norm.eps, bool(x_grad_via_branch))

@@ -1105,12 +1105,12 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   // 5000 ns, the price of the kernel before this one, 0.8 %), the most 12 % (4096 x 2048 x 6144, 128 tiles: 119 us with 256 x 128 against 111); it is
   // the same for 975 - 1100 and 4000 - 5000 ns.  Where 256 x 256 is close and not taken: 4096 x 2048 x 2048, 128 tiles, 39 - 43 us against 37 - 38.
   static const double fixed_ns[kNumShapes] = {3000.0, 3000.0, 3000.0, 3000.0, 3000.0, 4500.0, 3000.0};
-  // The two tiles for operands or outputs of any alignment, 64 x 64 and 128 x 128: the element-wise epilogue makes the larger one's
-  // share outside the loop 14.5 us, the register loaders make a slab take twice as long.  Measured on 16 odd shapes x 3 layouts
-  // with either tile forced; with the prices above, 128 x 128 was taken where 64 x 64 is ahead: us, bf16 3864 x 321 x 201 17.4 -> 11.9,
-  // 500 x 3001 x 1000 23.2 -> 19.8, 4001 x 1025 x 33 29.4 -> 20.2, 8 of 1001 x 256 x 992 (weight gradient) 24.5 -> 21.3; fp32 3222 x
-  // 4321 x 137 94 -> 80.  Where it is behind, 2001 x 2003 x 2005 39 against 54, it is not taken.
-  static const double odd_slab_ns[2][2] = {{330.0, 750.0}, {480.0, 2100.0}}, odd_fixed_ns[2] = {3600.0, 14500.0};
+  // The two tiles for operands or outputs of any alignment, 64 x 64 and 128 x 128: the register loaders make a slab take nearly twice as
+  // long, the epilogue's unaligned accesses the larger tile's share outside the loop 10 us.  Either tile forced on 20 odd shapes x 3 layouts:
+  // with these prices the one taken costs 0.1 % over the better one in the mean (with 14.5 us, the price of the element-wise epilogue, 0.3 %).
+  // us, 64 x 64 / 128 x 128, bf16: 3864 x 321 x 201 10.5 / 12.6, 1024 x 3001 x 4096 55 / 43, 2001 x 2003 x 2005 50 / 33, 3000 x 3001 x 150 30 / 28, 1000
+  // x 501 x 512 with 4 shards (weight gradient) 13.3 / 26.3; fp32 3222 x 4321 x 137 70 / 75.
+  static const double odd_slab_ns[2][2] = {{330.0, 750.0}, {480.0, 2100.0}}, odd_fixed_ns[2] = {3600.0, 10000.0};
   static const int slab_bytes[kNumShapes] = {128, 128, 128, 128, 128, 128, 128};
   const bool vec = direct && a.vec_c;  // else the kernels for operands of any alignment
   int shape = 3;  // 64 x 64 unless the model finds something cheaper

@@ -383,14 +383,52 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& p, const float* ct, 
   }
 }
 
-// The epilogue where an operand of it is not vector-aligned (an odd width, a shard of odd size): the same operations
-// element by element, the lanes of a wave on consecutive columns of a row (with 8 columns per lane each store would touch every
-// line of the row), the addends and masks of EB elements requested together.
+// Up to eight consecutive values at any alignment, as fp32; those from `n` on, which may lie outside the operand, are left out.
+template <typename S>
+__device__ __forceinline__ void load8_any(const S* src, int n, float (&v)[8]) {
+  constexpr int VEC = 16 / (int)sizeof(S);
+  typedef S vec_t __attribute__((ext_vector_type(VEC), aligned(sizeof(S))));
+  if (n >= 8) {
+#pragma unroll
+    for (int h = 0; h < 8 / VEC; ++h) {
+      const vec_t q = *reinterpret_cast<const vec_t*>(src + h * VEC);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) v[h * VEC + e] = to_f32((S)q[e]);
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = e < n ? to_f32(src[e]) : 0.0f;
+  }
+}
+template <typename S>
+__device__ __forceinline__ void store8_any(S* dst, int n, const float (&v)[8]) {
+  constexpr int VEC = 16 / (int)sizeof(S);
+  typedef S vec_t __attribute__((ext_vector_type(VEC), aligned(sizeof(S))));
+  if (n >= 8) {
+#pragma unroll
+    for (int h = 0; h < 8 / VEC; ++h) {
+      vec_t q;
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) q[e] = from_f32<S>(v[h * VEC + e]);
+      *reinterpret_cast<vec_t*>(dst + h * VEC) = q;
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (e < n) dst[e] = from_f32<S>(v[e]);
+  }
+}
+
+// The epilogue where an operand of it is not vector-aligned (an odd width, a shard of odd size): the operations of finish_tile on
+// 16-byte accesses of any alignment, element by element only in the eight columns that the product's last ones lie in.
+// (Its predecessor went element by element throughout: 14.5 us outside the K loop of a 128 x 128 tile in bf16, now 6 - 10.  us, before ->
+// now, forward / weight gradient: 1250 x 9090 x 1792, 2 shards, 164 / 206 -> 136 / 160; 2001 x 2003 x 2005 36.9 / 47.9 -> 32.7 /
+// 44.1; 992 x 126 x 2048, 8 shards, 18.8 / 20.1 -> 17.8 / 18.1; 255 x 1023 x 3333 16.9 / 18.4 -> 16.4 / 13.3; fp32 3222 x 4321 x 137 79 / 77 -> 70 / 75.)
 template <typename T, int BM, int BN, int NTHR>
 __device__ __forceinline__ void finish_tile_ragged(const GemmArgs& p, const float* ct, int m0, int n0, int tid, int grp,
                                                    long zo, long zi) {
-  constexpr int CP = BN + 4, TOTAL = BM * BN, EB = 4;
-  static_assert(TOTAL % (NTHR * EB) == 0, "whole batches");
+  constexpr int CP = BN + 4, CPR = BN / 8, NCH = BM * CPR / NTHR;
+  static_assert(BM * CPR % NTHR == 0 && NTHR % CPR == 0, "whole chunks, all of a thread's in the same columns");
   const bool out_f32 = p.flags & RTP_GEMM_OUT_F32;
   const bool cin_f32 = p.flags & RTP_GEMM_CIN_F32;
   const bool relu = p.flags & RTP_GEMM_RELU;
@@ -406,53 +444,63 @@ __device__ __forceinline__ void finish_tile_ragged(const GemmArgs& p, const floa
   float* master = p.sgd_master ? p.sgd_master + zoff : nullptr;
   T* wcopy = p.sgd_w ? reinterpret_cast<T*>(p.sgd_w) + zoff : nullptr;
   const bool skip_out = p.flags & RTP_GEMM_SGD_SKIP_OUT;
-  // a thread's elements all lie in one column where the thread count is a multiple of the tile's width
-  constexpr bool SAMECOL = NTHR % BN == 0;
-  auto bias_of = [&](int col) {
-    float bv = 0.0f;
-    if (bias)
-      for (int sgm = 0; sgm < nb_seg; ++sgm) bv += to_f32(bias[sgm * p.bias_sk + col]);
-    return bv;
-  };
-  float bcol = SAMECOL ? bias_of(min(n0 + tid % BN, p.n - 1)) : 0.0f;
-  for (int e0 = tid; e0 < TOTAL; e0 += NTHR * EB) {
-    float v[EB], add[EB], msk[EB];
-    long row[EB];
-    int col[EB];
+  const int lc = (tid % CPR) * 8, col = n0 + lc, live = p.n - col;
+  if (live <= 0) return;
+  // what the thread's chunks need from memory, requested before the first is finished
+  float add[NCH][8], msk[NCH][8], bv[8];
 #pragma unroll
-    for (int i = 0; i < EB; ++i) {
-      const int e = e0 + i * NTHR;
-      row[i] = m0 + e / BN, col[i] = n0 + e % BN;
-      const long rc = row[i] < p.m ? row[i] : p.m - 1;
-      const int cc = col[i] < p.n ? col[i] : p.n - 1;
-      add[i] = 0.0f, msk[i] = 1.0f;
-      if (cin) {
-        const long off = rc * p.ld_cin + cc;
-        add[i] = cin_f32 ? reinterpret_cast<const float*>(cin)[off] : to_f32(reinterpret_cast<const T*>(cin)[off]);
-      }
-      if (gate) msk[i] = to_f32(gate[rc * p.ld_gate + cc]);
-      v[i] = p.alpha * ct[(e / BN) * CP + e % BN];
-    }
-#pragma unroll
-    for (int i = 0; i < EB; ++i) {
-      if (row[i] >= p.m || col[i] >= p.n) continue;
-      float x = v[i];
-      if (cin) x += add[i];
-      if (bias) x += SAMECOL ? bcol : bias_of(col[i]);
-      if (relu) x = fmaxf(x, 0.0f);
-      if (gate) x = msk[i] > 0.0f ? x : 0.0f;
-      const long off = row[i] * p.ldc + col[i];
-      if (master) {
-        const float w = sgd_update<T>(master[off], x, p.sgd_lr, p.sgd_clip);
-        master[off] = w;
-        if (wcopy) wcopy[off] = from_f32<T>(w);
-      }
-      if (skip_out) continue;
-      if (out_f32)
-        reinterpret_cast<float*>(cbase)[off] = x;
+  for (int i = 0; i < NCH; ++i) {
+    const long row = min(m0 + (tid + i * NTHR) / CPR, p.m - 1);
+    if (cin) {
+      const long off = row * p.ld_cin + col;
+      if (cin_f32)
+        load8_any(reinterpret_cast<const float*>(cin) + off, live, add[i]);
       else
-        reinterpret_cast<T*>(cbase)[off] = from_f32<T>(x);
+        load8_any(reinterpret_cast<const T*>(cin) + off, live, add[i]);
     }
+    if (gate) load8_any(gate + row * p.ld_gate + col, live, msk[i]);
+    if (master) load8_any(master + row * p.ldc + col, live, add[i]);  // (an update excludes an addend)
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) bv[e] = 0.0f;
+  if (bias)
+    for (int s0 = 0; s0 < nb_seg; s0 += 4) {  // four segments' at a time, added in their order
+      float bt[4][8];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) load8_any(bias + (s0 + j < nb_seg ? s0 + j : 0) * p.bias_sk + col, live, bt[j]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (s0 + j < nb_seg) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) bv[e] += bt[j][e];
+        }
+    }
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    const int lr = (tid + i * NTHR) / CPR;
+    if (m0 + lr >= p.m) break;  // the rows behind this one as well
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      v[e] = p.alpha * ct[lr * CP + lc + e];
+      if (cin) v[e] += add[i][e];
+      if (bias) v[e] += bv[e];
+      if (relu) v[e] = fmaxf(v[e], 0.0f);
+      if (gate) v[e] = msk[i][e] > 0.0f ? v[e] : 0.0f;
+    }
+    const long off = (long)(m0 + lr) * p.ldc + col;
+    if (master) {
+      float w[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) w[e] = sgd_update<T>(add[i][e], v[e], p.sgd_lr, p.sgd_clip);
+      store8_any(master + off, live, w);
+      if (wcopy) store8_any(wcopy + off, live, w);
+    }
+    if (skip_out) continue;
+    if (out_f32)
+      store8_any(reinterpret_cast<float*>(cbase) + off, live, v);
+    else
+      store8_any(reinterpret_cast<T*>(cbase) + off, live, v);
   }
 }
 

@@ -232,6 +232,14 @@ int rtp_gemm(void* stream, int dtype, const rtp_gemm_desc* d);
 int rtp_gemm_warm_next(const void* src, size_t bytes);
 int rtp_gemm_warm_pending(void);
 
+/* Scratch memory for the products of the calling thread (no counterpart in the reference).  A large bf16 product on operands that are
+ * not vector-aligned is faster on aligned copies of them: while `alloc` is set, rtp_gemm and rtp_rotated_linear_* ask it for
+ * that memory (256-byte aligned, on the current device; `context` is handed through) and use it on the product's stream
+ * until the product has run.  NULL from it, or no `alloc` (the state a thread starts in): the product reads its operands where they
+ * are.  No result depends on it.  At most 1 GiB a product. */
+typedef void* (*rtp_alloc_fn)(void* context, size_t bytes);
+int rtp_gemm_workspace(rtp_alloc_fn alloc, void* context);
+
 /* Measurement aid (no counterpart in the reference; bench.py reports it beside the published peak): TFLOP/s of a
  * register-only loop of v_mfma_f32_32x32x16_bf16 on every SIMD of the device, `iters` iterations of 32 MFMAs per
  * wavefront, with constant operands (random_operands == 0) or normally distributed ones (1).  Synchronises on

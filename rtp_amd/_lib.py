@@ -101,6 +101,7 @@ PROTOTYPES = {
     "rtp_gemm": (_i, [_vp, _i, C.POINTER(GemmDesc)]),
     "rtp_gemm_warm_next": (_i, [_vp, _sz]),
     "rtp_gemm_warm_pending": (_i, []),
+    "rtp_gemm_workspace": (_i, [_vp, _vp]),
     "rtp_probe_mfma_rate": (_i, [_vp, _i, _i, C.POINTER(C.c_double)]),
     "rtp_gemm_rowsum_fused": (_i, [_i, C.POINTER(GemmDesc)]),
     "rtp_gemm_sgd_fused": (_i, [_i, C.POINTER(GemmDesc)]),

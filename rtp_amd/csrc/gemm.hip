@@ -413,8 +413,8 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
     } else {
     DA da;
     DB db;
-    da.init(p.lda, m0, p.m, lw, lane);
-    db.init(p.ldb, n0, p.n, lw, lane);
+    da.init(p.lda, m0, p.rows_a, lw, lane);
+    db.init(p.ldb, n0, p.rows_b, lw, lane);
     const char* ca = DA::slab_base(A, p.lda, m0);  // base of the next slab, uniform: scalar registers
     const char* cb = DB::slab_base(B, p.ldb, n0);
     constexpr long SZ = (long)sizeof(T);
@@ -918,6 +918,52 @@ static const void* warm_source() {
   return t_warm_src && t_warm_call == g_warm_call.load(std::memory_order_relaxed) ? t_warm_src : nullptr;
 }
 
+// rtp_gemm_workspace: the calling thread's source of scratch memory.
+static thread_local rtp_alloc_fn t_alloc = nullptr;
+static thread_local void* t_alloc_context = nullptr;
+
+// Which operands of a bf16 product are copied to whole vectors first.
+struct Packing {
+  bool a = false, b = false;
+  PackShape sa, sb;
+};
+static Packing pack_plan(const rtp_gemm_desc* d, bool vec_c) {
+  Packing p;
+  const bool akc = d->a_kcontig, bkc = d->b_kcontig;
+  if (t_alloc == nullptr || d->batch != 1 || d->xent_mode || d->sgd_master || d->m < 128 || d->n < 128 || d->k < 8 || takes_dma_kernel<bf16_t>(d))
+    return p;
+  const int64_t ld_max = ((int64_t)1 << 23) - 64;
+  const auto shape = [&](const void* x, int64_t ld, int64_t sg, int64_t sk, bool kc, int64_t rows) {
+    PackShape q;
+    q.src = (const char*)x, q.ld = ld, q.copy = sg, q.seg = sk;
+    q.copies = sg != 0 ? d->groups : 1, q.segs = sk != 0 ? d->ksegs : 1;
+    q.lines = kc ? rows : d->k, q.len = kc ? d->k : rows;
+    return q;
+  };
+  const auto fits = [&](const PackShape& q) {
+    return mult((int64_t)(uintptr_t)q.src, 16) && mult(q.ld, 8) && mult(q.copy, 8) && mult(q.seg, 8) && mult(q.len, 8);
+  };
+  p.sa = shape(d->a, d->lda, d->a_sg, d->a_sk, akc, d->m), p.sb = shape(d->b, d->ldb, d->b_sg, d->b_sk, bkc, d->n);
+  const bool a = !fits(p.sa), b = !fits(p.sb);
+  const int64_t vectors = (a ? p.sa.vectors() : 0) + (b ? p.sb.vectors() : 0);
+  if (vectors > (1 << 26) || p.sa.len > ld_max || p.sb.len > ld_max || (!a && d->lda > ld_max) || (!b && d->ldb > ld_max)) return p;
+  // It pays where the copies (their bytes in and out at 4.5 TB/s, 8 us each between their neighbours on the stream) take less than what
+  // the register loaders add.  ns a slab of 128 x 128, every CU busy: register loaders 600 / 700 / 800 (both operands k-contiguous /
+  // one / none), direct-to-LDS 480; outside the slabs 6 and 5 us; 256 x 256, which only aligned results can take, 1650 a slab and
+  // 6 us.  us without -> with the copies, forward / input gradient / weight gradient (=: not taken): 6546 x 482 x 6400, 8 shards, 460 / 540 /
+  // 628 -> 367 / 353 / 407; 4096 x 1023 x 4096 = / 76 / 80 -> = / 47 / 46; 8192 x 33 x 7000, 8 shards, = / 185 / = -> = / 111 / =;
+  // 1024 x 3001 x 4096 = / 45.8 (taken: 47.6) / 64 -> = / = / 50; 1250 x 9090 x 1792, 2 shards, = / 187 (taken: 199) / 160 -> = / = / 145; 2001 x 2003 x
+  // 2005 = (taken: 35.9 / 42.1 / 47.1 against 32.7 / 38.5 / 44.0).
+  const int64_t slabs = ceil_div(d->k, 64) * d->ksegs;
+  const auto rounds = [&](int t) { return (double)ceil_div(ceil_div(d->m, t) * ceil_div(d->n, t) * d->groups, 256); };
+  const double slow = rounds(128) * ((double)slabs * (akc && bkc ? 600.0 : akc || bkc ? 700.0 : 800.0) + 6000.0);
+  double fast = rounds(128) * ((double)slabs * 480.0 + 5000.0);
+  if (vec_c && slabs >= 2) fast = std::min(fast, rounds(256) * ((double)slabs * 1650.0 + 6000.0));
+  const double copies = 32.0 * (double)vectors / 4500.0 + (a ? 8000.0 : 0.0) + (b ? 8000.0 : 0.0);
+  if (slow - fast > 1.2 * copies) p.a = a, p.b = b;
+  return p;
+}
+
 template <typename T>
 static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   // the hint of rtp_gemm_warm_next rides in this launch or ends with it
@@ -925,6 +971,38 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   t_warm_src = nullptr;
   constexpr int VEC = 16 / sizeof(T);
   GemmArgs a;
+  {
+    auto ok = [](const void* ptr, int64_t ld, int64_t so, int64_t si, int64_t sg) {
+      return mult((int64_t)(uintptr_t)ptr, 16) && mult(ld, 8) && mult(so, 8) && mult(si, 8) && mult(sg, 8);
+    };
+    a.vec_c = mult(d->n, 8) && ok(d->c_out, d->ldc, d->c_so, d->c_si, d->c_sg) &&
+              (!d->c_in || ok(d->c_in, d->ld_cin, d->cin_so, d->cin_si, d->cin_sg)) &&
+              (!d->gate || ok(d->gate, d->ld_gate, d->gate_so, d->gate_si, d->gate_sg)) &&
+              (!d->bias || (ok(d->bias, 8, d->bias_so, d->bias_si, d->bias_sg) && mult(d->bias_sk, 8)));
+  }
+  a.rows_a = (int)d->m, a.rows_b = (int)d->n;
+  bool packed = false;
+  rtp_gemm_desc aligned;
+  if constexpr (sizeof(T) == 2) {
+    if (const Packing p = pack_plan(d, a.vec_c); p.a || p.b) {
+      const int64_t bytes_a = p.a ? p.sa.vectors() * 16 : 0, bytes_b = p.b ? p.sb.vectors() * 16 : 0;
+      if (char* at = (char*)t_alloc(t_alloc_context, (size_t)(bytes_a + bytes_b)); at != nullptr && (uintptr_t)at % 16 == 0) {
+        aligned = *d, packed = true;
+        const auto move = [&](const PackShape& q, char* to, const void*& x, int64_t& ld, int64_t& sg, int64_t& sk, bool kc, int& rows) {
+          x = to, ld = ceil_div(q.len, 8) * 8;
+          if (sk != 0) sk = q.lines * ld;
+          if (sg != 0) sg = q.segs * q.lines * ld;
+          if (!kc) rows = (int)ld;
+          return launch_pack(s, q, to);
+        };
+        int rc = RTP_OK;
+        if (p.a) rc = move(p.sa, at, aligned.a, aligned.lda, aligned.a_sg, aligned.a_sk, d->a_kcontig, a.rows_a);
+        if (p.b && rc == RTP_OK) rc = move(p.sb, at + bytes_a, aligned.b, aligned.ldb, aligned.b_sg, aligned.b_sk, d->b_kcontig, a.rows_b);
+        if (rc != RTP_OK) return rc;
+        d = &aligned;
+      }
+    }
+  }
   a.a = (const char*)d->a;
   a.b = (const char*)d->b;
   a.c_out = (char*)d->c_out;
@@ -955,18 +1033,8 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   a.vec_b = mult((int64_t)(uintptr_t)d->b, 16) && mult(d->ldb, VEC) && mult(d->b_so, VEC) && mult(d->b_si, VEC) &&
             mult(d->b_sg, VEC) && mult(d->b_sk, VEC);
 
-  {
-    auto ok = [](const void* ptr, int64_t ld, int64_t so, int64_t si, int64_t sg) {
-      return mult((int64_t)(uintptr_t)ptr, 16) && mult(ld, 8) && mult(so, 8) && mult(si, 8) && mult(sg, 8);
-    };
-    a.vec_c = mult(d->n, 8) && ok(d->c_out, d->ldc, d->c_so, d->c_si, d->c_sg) &&
-              (!d->c_in || ok(d->c_in, d->ld_cin, d->cin_so, d->cin_si, d->cin_sg)) &&
-              (!d->gate || ok(d->gate, d->ld_gate, d->gate_so, d->gate_si, d->gate_sg)) &&
-              (!d->bias || (ok(d->bias, 8, d->bias_so, d->bias_si, d->bias_sg) && mult(d->bias_sk, 8)));
-  }
-
   const bool akc = d->a_kcontig, bkc = d->b_kcontig;
-  const bool direct = takes_dma_kernel<T>(d), fast = direct || takes_reg_kernel<T>(d);
+  const bool direct = packed || takes_dma_kernel<T>(d), fast = direct || takes_reg_kernel<T>(d);
   const int64_t nz = d->batch * d->groups;
   a.a_rowsum = (char*)d->a_rowsum;
   a.rowsum_sg = d->rowsum_sg;
@@ -1048,7 +1116,7 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
                     : tiles64 <= 256 && (sizeof(T) == 4 || (k_all >= 2048 && akc == bkc))          ? 64
                     : sizeof(T) == 4 && k_all >= 768 && tiles32 <= 512                             ? 32
                                                                                                    : 0;
-  if (fast && !relu && !d->xent_mode && nz < 65536 && k_all >= 256 && !(sizeof(T) == 4 && !direct && !akc && !bkc) && kw_bm != 0) {
+  if (fast && !packed && !relu && !d->xent_mode && nz < 65536 && k_all >= 256 && !(sizeof(T) == 4 && !direct && !akc && !bkc) && kw_bm != 0) {
     a.tiles_m = (int)ceil_div(d->m, kw_bm);
     a.tiles_n = (int)ceil_div(d->n, 32);
     static const char* const names[2][2][2] = {{{"gemm_f32_kwaves_rc_rc", "gemm_f32_kwaves_rc_kc"}, {"gemm_f32_kwaves_kc_rc", "gemm_f32_kwaves_kc_kc"}},
@@ -1061,7 +1129,7 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   // Many outputs, at most two K slabs: see gemm_shortk.hip.  From 384 of its tiles on it is ahead, in every layout; with 256, one
   // workgroup a CU, it is behind (us, before -> this, bf16: 2048 x 2048 x 64 7.0 -> 7.0, 1024 x 4096 x 96 7.6 -> 8.1, 4096 x 1536 x 32
   // 9.0 -> 8.0, 2048 x 8192 x 96 16.7 -> 13.3; three slabs: 8192 x 1536 x 256 18.8 -> 17.0 in bf16, but 66 -> 70 in fp32).
-  if (direct && a.vec_c && !d->xent_mode && nz < 65536 && k_all * (int64_t)sizeof(T) <= 256 &&
+  if (direct && !packed && a.vec_c && !d->xent_mode && nz < 65536 && k_all * (int64_t)sizeof(T) <= 256 &&
       ceil_div(d->m, 128) * ceil_div(d->n, 128) * nz >= 384) {
     a.tiles_m = (int)ceil_div(d->m, 128);
     a.tiles_n = (int)ceil_div(d->n, 128);
@@ -1106,11 +1174,11 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   // the same for 975 - 1100 and 4000 - 5000 ns.  Where 256 x 256 is close and not taken: 4096 x 2048 x 2048, 128 tiles, 39 - 43 us against 37 - 38.
   static const double fixed_ns[kNumShapes] = {3000.0, 3000.0, 3000.0, 3000.0, 3000.0, 4500.0, 3000.0};
   // The two tiles for operands or outputs of any alignment, 64 x 64 and 128 x 128: the register loaders make a slab take nearly twice as
-  // long, the epilogue's unaligned accesses the larger tile's share outside the loop 10 us.  Either tile forced on 20 odd shapes x 3 layouts:
-  // with these prices the one taken costs 0.1 % over the better one in the mean (with 14.5 us, the price of the element-wise epilogue, 0.3 %).
-  // us, 64 x 64 / 128 x 128, bf16: 3864 x 321 x 201 10.5 / 12.6, 1024 x 3001 x 4096 55 / 43, 2001 x 2003 x 2005 50 / 33, 3000 x 3001 x 150 30 / 28, 1000
-  // x 501 x 512 with 4 shards (weight gradient) 13.3 / 26.3; fp32 3222 x 4321 x 137 70 / 75.
-  static const double odd_slab_ns[2][2] = {{330.0, 750.0}, {480.0, 2100.0}}, odd_fixed_ns[2] = {3600.0, 10000.0};
+  // long and the larger tile's share outside the loop 10 us; where only the results are unaligned that is 4.  Either tile forced on 20 odd
+  // shapes x 3 layouts: with these prices the one taken costs 0.1 % over the better one in the mean (with 14.5 us, the price of an
+  // element-wise epilogue, 0.3 %).  us, 64 x 64 / 128 x 128, bf16: 3864 x 321 x 201 10.5 / 12.6, 1024 x 3001 x 4096 55 / 43, 2001 x 2003 x 2005
+  // 50 / 33, 1000 x 501 x 512 with 4 shards (weight gradient) 13.3 / 26.3, 4096 x 1023 x 512 15.3 / 11.8 (1024 wide 15.0 / 10.8); fp32 3222 x 4321 x 137 70 / 75.
+  static const double odd_slab_ns[2][2] = {{330.0, 750.0}, {480.0, 2100.0}}, odd_fixed_ns[2][2] = {{3600.0, 10000.0}, {3500.0, 4000.0}};
   static const int slab_bytes[kNumShapes] = {128, 128, 128, 128, 128, 128, 128};
   const bool vec = direct && a.vec_c;  // else the kernels for operands of any alignment
   int shape = 3;  // 64 x 64 unless the model finds something cheaper
@@ -1151,7 +1219,8 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
       const auto round_ns = [&](double n) { return std::max(n * tile_bytes / 4900.0, tile_bytes / 32.0); };
       update = (rounds - 1.0) * round_ns(256.0) + round_ns((double)tiles - 256.0 * (rounds - 1.0));
     }
-    const double cost = rounds * (vec ? nslabs * slab_ns[i] + outside : nslabs * odd_slab_ns[sizeof(T) == 4][i == 1] + odd_fixed_ns[i == 1]) + update;
+    const double slab = vec || direct ? slab_ns[i] : odd_slab_ns[sizeof(T) == 4][i == 1];
+    const double cost = rounds * (nslabs * slab + (vec ? outside : odd_fixed_ns[direct][i == 1])) + update;
     if (best == 0.0 || cost < best || i == forced) {
       best = i == forced ? -1.0 : cost;
       shape = i;
@@ -1457,6 +1526,11 @@ extern "C" int rtp_gemm_warm_next(const void* src, size_t bytes) {
   rtp::t_warm_src = bytes ? src : nullptr;
   rtp::t_warm_bytes = bytes;
   rtp::t_warm_call = ++rtp::g_warm_call;
+  return RTP_OK;
+}
+
+extern "C" int rtp_gemm_workspace(rtp_alloc_fn alloc, void* context) {
+  rtp::t_alloc = alloc, rtp::t_alloc_context = context;
   return RTP_OK;
 }
 

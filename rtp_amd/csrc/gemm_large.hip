@@ -210,11 +210,11 @@ __global__ __launch_bounds__(512) void gemm_large_kernel(GemmArgs) {
   DB db[2];
   auto init_a = [&](const Tile& w) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) da[h].init(lda, w.m0, rows_a, wave, lane_now(), [=](int r) { return half_row<BLKA>(r, h); });
+    for (int h = 0; h < 2; ++h) da[h].init(lda, w.m0, kernel_args()->rows_a, wave, lane_now(), [=](int r) { return half_row<BLKA>(r, h); });
   };
   auto init_b = [&](const Tile& w) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) db[h].init(ldb, w.n0, rows_b, wave, lane_now(), [=](int r) { return half_row<BLKB>(r, h); });
+    for (int h = 0; h < 2; ++h) db[h].init(ldb, w.n0, kernel_args()->rows_b, wave, lane_now(), [=](int r) { return half_row<BLKB>(r, h); });
   };
   init_a(here);
   init_b(here);

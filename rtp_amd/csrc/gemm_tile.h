@@ -57,6 +57,7 @@ struct GemmArgs {
   // bytes that some later launch will read from HBM (the next layer's shards): requested here, see warm_ahead()
   const char* warm;
   long warm_bytes;
+  int rows_a, rows_b;  // m and n as the direct-to-LDS loaders see them: to whole vectors where an operand's lines are padded to those
 };
 
 // The per-lane MFMA operand: VEC consecutive k values of one tile row.
@@ -924,6 +925,16 @@ int launch_split(hipStream_t s, const GemmArgs& a, bool akc, bool bkc, int bm, b
 
 // bf16 products in tiles of 256 x 256 by workgroups that stay (gemm_large.hip); two K slabs or more, no update, no statistics.
 int launch_large(hipStream_t s, const GemmArgs& a, bool akc, bool bkc);
+
+// `copies` x `segs` matrices of `lines` lines of `len` bf16 elements -> lines of whole 16-byte vectors, zeros behind their ends, all
+// contiguous (gemm_pack.hip).
+struct PackShape {
+  const char* src;
+  long ld, seg, copy;  // strides in elements
+  int64_t copies, segs, lines, len;
+  int64_t vectors() const { return copies * segs * lines * ((len + 7) / 8); }
+};
+int launch_pack(hipStream_t s, const PackShape& p, char* dst);
 
 // Many tiles of 128 x 128 over a K slab or two (gemm_shortk.hip).
 int launch_shortk(hipStream_t s, const GemmArgs& a, bool bf16, bool akc, bool bkc, dim3 grid);

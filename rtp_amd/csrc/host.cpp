@@ -139,6 +139,7 @@ RTP_ENTRY_POINTS(WRAP_X, WRAP_P)
 #undef WRAP
 
 decltype(&rtp_gemm) f_gemm = nullptr;
+decltype(&rtp_gemm_workspace) f_gemm_workspace = nullptr;
 decltype(&rtp_gemm_rowsum_fused) f_rowsum_fused = nullptr;
 decltype(&rtp_gemm_sgd_fused) f_sgd_fused = nullptr;
 decltype(&rtp_rotated_linear_fwd) f_linear_fwd = nullptr;
@@ -157,7 +158,7 @@ PyObject* py_bind(PyObject*, PyObject* args) {
     if (!f) PyErr_Format(PyExc_OSError, "librtp_hip.so has no %s", name);
     return f != nullptr;
   };
-  bool ok = get("rtp_last_error", f_last_error) && get("rtp_gemm", f_gemm) &&
+  bool ok = get("rtp_last_error", f_last_error) && get("rtp_gemm", f_gemm) && get("rtp_gemm_workspace", f_gemm_workspace) &&
             get("rtp_gemm_rowsum_fused", f_rowsum_fused) && get("rtp_gemm_sgd_fused", f_sgd_fused) &&
             get("rtp_rotated_linear_fwd", f_linear_fwd) && get("rtp_rotated_linear_bwd", f_linear_bwd);
 #define RESOLVE(name) ok = ok && get(#name, f_##name);
@@ -166,6 +167,23 @@ PyObject* py_bind(PyObject*, PyObject* args) {
   if (!ok) return nullptr;
   Py_RETURN_NONE;
 }
+
+// Scratch memory for the products launched while it lives, from torch's allocator on the current stream: given back with it, for what
+// that stream runs afterwards.  (The allocator itself, not at::empty: no dispatch, and no Python under a mode of it.)
+struct Workspace {
+  std::vector<c10::DataPtr> held;
+  Workspace() { f_gemm_workspace(&get, this); }
+  ~Workspace() { f_gemm_workspace(nullptr, nullptr); }
+  static void* get(void* self, size_t bytes) noexcept {
+    try {
+      auto& held = static_cast<Workspace*>(self)->held;
+      held.push_back(c10::GetAllocator(c10::kCUDA)->allocate(bytes));
+      return held.back().get();
+    } catch (...) {  // no memory: the product does without
+      return nullptr;
+    }
+  }
+};
 
 int dtype_code(at::ScalarType t) {
   return t == at::kFloat ? (int)RTP_F32 : t == at::kBFloat16 ? (int)RTP_BF16 : -1;
@@ -229,7 +247,7 @@ bool launch_product(int dt, rtp_gemm_desc& d, uint32_t flags, int& done) {
       d.a_rowsum = nullptr, d.rowsum_sg = 0;
   }
   void* st = current_stream();
-  const int rc = (WithoutGil(), f_gemm(st, dt, &d));
+  const int rc = (WithoutGil(), Workspace(), f_gemm(st, dt, &d));
   if (rc < 0) raise_status(rc);
   return rc >= 0;
 }
@@ -335,7 +353,7 @@ PyObject* py_linear_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
   // one row: any leading dimension that holds it
   const int64_t ldo = o.rows > 1 ? o.ld : std::max<int64_t>(o.cols, 1);
   char* out = o.p + col0 * (int64_t)y.element_size();
-  const int rc = (WithoutGil(), f_linear_fwd(st, dt, &L, x.p, x.ld, x.rows, out, ldo, flags));
+  const int rc = (WithoutGil(), Workspace(), f_linear_fwd(st, dt, &L, x.p, x.ld, x.rows, out, ldo, flags));
   if (rc < 0) return raise_status(rc);
   Py_RETURN_NONE;
 }
@@ -401,7 +419,7 @@ PyObject* py_linear_bwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* st = current_stream();
   const int64_t ldy = dy.rows > 1 ? dy.ld : std::max<int64_t>(dy.cols, 1);
   const char* in = dy.p + col0 * (int64_t)dy2.element_size();
-  const int rc = (WithoutGil(), f_linear_bwd(st, dt, &L, in, ldy, x.p, x.ld, dy.rows, &o));
+  const int rc = (WithoutGil(), Workspace(), f_linear_bwd(st, dt, &L, in, ldy, x.p, x.ld, dy.rows, &o));
   if (rc < 0) return raise_status(rc);
   return PyLong_FromLong(done);
 }

@@ -99,6 +99,7 @@ PROTOTYPES = {
                                          _i64]),
     "rtp_softmax_xent_combine": (_i, [_vp, _vp, _i64, _vp, _vp, _i64, _i64, _vp, _vp]),
     "rtp_gemm": (_i, [_vp, _i, C.POINTER(GemmDesc)]),
+    "rtp_gemm_pair": (_i, [_vp, _i, C.POINTER(GemmDesc), C.POINTER(GemmDesc)]),
     "rtp_gemm_warm_next": (_i, [_vp, _sz]),
     "rtp_gemm_warm_pending": (_i, []),
     "rtp_gemm_workspace": (_i, [_vp, _vp]),

@@ -142,13 +142,14 @@ inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // Reads one word of every 64-byte line of a kernel's BYTES bytes of arguments (and of the launch dimensions that
 // follow them) in one batch, first thing in the kernel.  The scalar cache is cold at kernel start and the compiler
 // fetches arguments where they are first used: a kernel that needs them at three places pays three trips to
-// memory in a row, a microsecond in a ten-microsecond kernel.  After this every later fetch hits the cache.
+// memory in a row, a microsecond in a ten-microsecond kernel.  After this every later fetch hits the cache.  from: the byte
+// that those arguments start at.
 template <size_t BYTES>
-__device__ __forceinline__ void touch_kernel_arguments() {
+__device__ __forceinline__ void touch_kernel_arguments(unsigned from = 0) {
   constexpr int LINES = (int)(BYTES / 64) + 1;
   static_assert(LINES <= 10, "at most 640 bytes of kernel arguments");
   typedef const __attribute__((address_space(4))) int* kernarg_t;
-  kernarg_t ka = (kernarg_t)__builtin_amdgcn_kernarg_segment_ptr();
+  kernarg_t ka = (kernarg_t)__builtin_amdgcn_kernarg_segment_ptr() + from / 4;
   const int w0 = ka[0], w1 = ka[LINES > 1 ? 16 : 0], w2 = ka[LINES > 2 ? 32 : 0], w3 = ka[LINES > 3 ? 48 : 0];
   const int w4 = ka[LINES > 4 ? 64 : 0], w5 = ka[LINES > 5 ? 80 : 0], w6 = ka[LINES > 6 ? 96 : 0];
   const int w7 = ka[LINES > 7 ? 112 : 0], w8 = ka[LINES > 8 ? 128 : 0], w9 = ka[LINES > 9 ? 144 : 0];

@@ -964,11 +964,21 @@ static Packing pack_plan(const rtp_gemm_desc* d, bool vec_c) {
   return p;
 }
 
+// What one of two products would take by itself, and its arguments as a launch of 256 x 256 tiles (none: it cannot be one).
+struct PairPlan {
+  GemmArgs args;
+  bool large = false;
+  double alone = 0.0;  // ns
+  double slabs = 0.0, update_bytes = 0.0, flops = 0.0, bytes = 0.0;
+};
+
+// plan: nothing is launched, it is filled instead.
 template <typename T>
-static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
+static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d, PairPlan* plan = nullptr) {
+  if (plan && (sizeof(T) != 2 || d->a_kcontig || d->b_kcontig || d->xent_mode || is_tiny(d) || !takes_dma_kernel<T>(d))) return RTP_OK;
   // the hint of rtp_gemm_warm_next rides in this launch or ends with it
   const void* warm_src = warm_source();
-  t_warm_src = nullptr;
+  if (!plan) t_warm_src = nullptr;
   constexpr int VEC = 16 / sizeof(T);
   GemmArgs a;
   {
@@ -1116,6 +1126,7 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
                     : tiles64 <= 256 && (sizeof(T) == 4 || (k_all >= 2048 && akc == bkc))          ? 64
                     : sizeof(T) == 4 && k_all >= 768 && tiles32 <= 512                             ? 32
                                                                                                    : 0;
+  if (plan && (!a.vec_c || kw_bm != 0 || k_all <= 128)) return RTP_OK;
   if (fast && !packed && !relu && !d->xent_mode && nz < 65536 && k_all >= 256 && !(sizeof(T) == 4 && !direct && !akc && !bkc) && kw_bm != 0) {
     a.tiles_m = (int)ceil_div(d->m, kw_bm);
     a.tiles_n = (int)ceil_div(d->n, 32);
@@ -1221,10 +1232,20 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
     }
     const double slab = vec || direct ? slab_ns[i] : odd_slab_ns[sizeof(T) == 4][i == 1];
     const double cost = rounds * (nslabs * slab + (vec ? outside : odd_fixed_ns[direct][i == 1])) + update;
+    if (plan && i == 5) {
+      plan->large = true;
+      plan->slabs = nslabs;
+      if (d->sgd_master)
+        plan->update_bytes = (double)tiles * 65536.0 * (8.0 + (d->sgd_weights ? 2.0 : 0.0) + (d->flags & RTP_GEMM_SGD_SKIP_OUT ? 0.0 : 2.0));
+    }
     if (best == 0.0 || cost < best || i == forced) {
       best = i == forced ? -1.0 : cost;
       shape = i;
     }
+  }
+  if (plan) {
+    if (!plan->large) return RTP_OK;
+    plan->alone = best, shape = 5;
   }
   // fp32 contractions of 384 and more go to gemm_split.hip, whose K loop is 1.2 - 1.9 times as fast and whose prologue and epilogue
   // are 1 - 2 us longer (a workgroup fills a CU there): us, fp32 MFMA -> this, forward layout: 64 matrices of 420 x 420 with
@@ -1332,10 +1353,15 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d) {
   const double bytes = ((double)d->m * copies(d->a_so, d->a_si, d->a_sg, d->a_sk) +
                         (double)d->n * copies(d->b_so, d->b_si, d->b_sg, d->b_sk)) * (double)d->k * sizeof(T) +
                        mn * (out_sz + cin_sz + upd_sz);
-  ProfileScope prof(s, name, 2.0 * mn * kk, bytes);
-  a.trace = fast ? prof.trace_slot() : nullptr;
   a.warm = nullptr;
   a.warm_bytes = 0;
+  if (plan) {
+    a.trace = nullptr;
+    plan->args = a, plan->flops = 2.0 * mn * kk, plan->bytes = bytes;
+    return RTP_OK;
+  }
+  ProfileScope prof(s, name, 2.0 * mn * kk, bytes);
+  a.trace = fast ? prof.trace_slot() : nullptr;
   if (!fast) return launch_layout<T, 64, 64, 1, false>(s, a, akc, bkc, grid);
   // Carried by the kernels whose MFMA waves wait for loader waves at their start.  In the others every wave's own loads would queue
   // behind the hint's.  fp32 products lose nothing by it, their slabs take longer than HBM does: us, weights in the memory-side
@@ -1492,7 +1518,7 @@ __global__ __launch_bounds__(kThreads) void colsum_final_kernel(const float* par
 
 }  // namespace rtp
 
-extern "C" int rtp_gemm(void* stream, int dtype, const rtp_gemm_desc* d) {
+static int check_gemm(const rtp_gemm_desc* d) {
   using namespace rtp;
   RTP_REQUIRE(d != nullptr, "rtp_gemm: null descriptor");
   RTP_REQUIRE(d->a && d->b && d->c_out, "rtp_gemm: null operand pointer");
@@ -1506,11 +1532,46 @@ extern "C" int rtp_gemm(void* stream, int dtype, const rtp_gemm_desc* d) {
   RTP_REQUIRE(d->lda >= 1 && d->ldb >= 1 && d->ldc >= 1, "rtp_gemm: leading dimensions must be >= 1");
   RTP_REQUIRE(!d->c_in || d->ld_cin >= 1, "rtp_gemm: ld_cin must be >= 1 when c_in is given");
   RTP_REQUIRE(!d->gate || d->ld_gate >= 1, "rtp_gemm: ld_gate must be >= 1 when gate is given");
+  return RTP_OK;
+}
+
+extern "C" int rtp_gemm(void* stream, int dtype, const rtp_gemm_desc* d) {
+  using namespace rtp;
+  if (int rc = check_gemm(d)) return rc;
   if (d->m == 0 || d->n == 0) return RTP_OK;
   hipStream_t s = (hipStream_t)stream;
   if (dtype == RTP_F32) return launch_gemm<float>(s, d);
   if (dtype == RTP_BF16) return launch_gemm<bf16_t>(s, d);
   return fail(RTP_ERR_ARG, "rtp_gemm: unknown dtype %d", dtype);
+}
+
+extern "C" int rtp_gemm_pair(void* stream, int dtype, const rtp_gemm_desc* first, const rtp_gemm_desc* second) {
+  using namespace rtp;
+  RTP_REQUIRE(first && second, "rtp_gemm_pair: null descriptor");
+  // A round of 256 x 256 tiles that leaves CUs idle takes a second product's tiles along.  It pays by the prices of the products alone: the
+  // longer contraction, one epilogue, both updates at the memory's rate.  us, one after the other -> together, attention layers of width 2048
+  // (64 + 192 tiles): causal over 4096 rows, forward + backward, 512 -> 496; padded over 6000 rows 1024 -> 997; LM step of 10 blocks over 992
+  // rows, Adam, 4842 -> 4679, over 1024 with the update in the epilogues 3863 -> 3729.
+  if (dtype == RTP_BF16 && first->m > 0 && second->m > 0 && first->n > 0 && second->n > 0 && first->k > 0 && second->k > 0) {
+    hipStream_t s = (hipStream_t)stream;
+    PairPlan p[2];
+    for (int i = 0; i < 2; ++i)
+      if (int rc = check_gemm(i ? second : first)) return rc;
+    for (int i = 0; i < 2; ++i) {
+      if (int rc = launch_gemm<bf16_t>(s, i ? second : first, &p[i])) return rc;
+      if (!p[i].large) break;
+    }
+    if (p[0].large && p[1].large && p[0].args.per_xcd + p[1].args.per_xcd <= 32) {
+      const double together = std::max(p[0].slabs, p[1].slabs) * 1050.0 + 4500.0 + (p[0].update_bytes + p[1].update_bytes) / 4900.0;
+      if (together < p[0].alone + p[1].alone) {
+        t_warm_src = nullptr;  // 256 x 256 tiles carry no hint; it ends here
+        ProfileScope prof(s, "gemm_bf16_256x256_pair_rc_rc", p[0].flops + p[1].flops, p[0].bytes + p[1].bytes);
+        return launch_large_pair(s, p[0].args, p[1].args);
+      }
+    }
+  }
+  if (int rc = rtp_gemm(stream, dtype, first)) return rc;
+  return rtp_gemm(stream, dtype, second);
 }
 
 extern "C" int rtp_gemm_rowsum_fused(int dtype, const rtp_gemm_desc* d) {

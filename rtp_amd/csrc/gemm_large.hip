@@ -56,8 +56,8 @@ __device__ __forceinline__ constexpr int half_row(int r, int h) {
 // The kernel's arguments where they stand, in the kernel-argument segment, through a pointer that the compiler knows nothing
 // about: what is fetched through it is not kept in scalar registers over the K loops (all of them together do not fit).
 typedef const __attribute__((address_space(4))) GemmArgs* KernArgs;
-__device__ __forceinline__ KernArgs kernel_args() {
-  KernArgs q = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
+__device__ __forceinline__ KernArgs kernel_args_at(unsigned bytes) {
+  KernArgs q = (KernArgs)((const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr() + bytes);
   asm volatile("" : "+s"(q));
   return q;
 }
@@ -126,8 +126,15 @@ struct FragPlace {
   }
 };
 
-template <bool AKC, bool BKC>
-__global__ __launch_bounds__(512) void gemm_large_kernel(GemmArgs) {
+// Two products in one launch: workgroups 0 .. split - 1 have the first one's tiles, the others the second one's (split: a multiple of 8, so
+// that a workgroup's XCD is its number's in either).
+struct GemmPair {
+  GemmArgs product[2];
+  unsigned split;
+};
+
+template <bool AKC, bool BKC, bool PAIR>
+__device__ __forceinline__ void large_body() {
   using T = bf16_t;
   constexpr int BM = 256, BN = 256, NL = 8, SB = 128;
   constexpr int WM = 128, WN = 64, MT = 4, NT = 2;
@@ -146,7 +153,12 @@ __global__ __launch_bounds__(512) void gemm_large_kernel(GemmArgs) {
   static_assert(2 * SLAB + NL * PAGE <= 160 * 1024 && kBiasSegs * WN * 2 <= PAGE, "160 KiB of LDS");
   __shared__ __attribute__((aligned(1024))) char lds[2 * SLAB + NL * PAGE];  // [slab & 1][A0, A1, B0, B1], pages
 
-  touch_kernel_arguments<sizeof(GemmArgs)>();
+  const unsigned split = PAIR ? ((const __attribute__((address_space(4))) GemmPair*)kernel_args_at(0))->split : 0;
+  const bool second = PAIR && blockIdx.x >= split;
+  const unsigned block = second ? blockIdx.x - split : blockIdx.x, blocks = PAIR && !second ? split : gridDim.x - split;
+  const unsigned at = second ? (unsigned)sizeof(GemmArgs) : 0;
+  touch_kernel_arguments<sizeof(GemmArgs)>(at);
+  auto kernel_args = [=] { return kernel_args_at(at); };
   const KernArgs args = kernel_args();
   const int tid = threadIdx.x;
   if (args->trace != nullptr && tid == 0) atomicMin(args->trace, (unsigned long long)wall_clock64());
@@ -155,10 +167,10 @@ __global__ __launch_bounds__(512) void gemm_large_kernel(GemmArgs) {
   const int wm = wave >> 2, wn = wave & 3;
 
   // ---- the tiles of this workgroup ----
-  const unsigned xcd = blockIdx.x & 7, stride = gridDim.x >> 3;
+  const unsigned xcd = block & 7, stride = blocks >> 3;
   const unsigned chunk = args->xg != 0 ? 0 : xcd * args->per_xcd;  // where no split into bricks fits: an eighth of the tiles
   const unsigned mine = args->xg != 0 ? args->per_xcd : chunk >= args->tiles ? 0 : min(args->per_xcd, args->tiles - chunk);
-  unsigned slot = blockIdx.x >> 3;
+  unsigned slot = block >> 3;
   if (slot >= mine) return;
   struct Tile {
     int m0, n0, grp, zo, zi;
@@ -773,6 +785,20 @@ __global__ __launch_bounds__(512) void gemm_large_kernel(GemmArgs) {
     here = next;
   }
   if (kernel_args()->trace != nullptr && tid == 0) atomicMax(kernel_args()->trace + 1, (unsigned long long)wall_clock64());
+}
+
+template <bool AKC, bool BKC>
+__global__ __launch_bounds__(512) void gemm_large_kernel(GemmArgs) {
+  large_body<AKC, BKC, false>();
+}
+__global__ __launch_bounds__(512) void gemm_large_pair_kernel(GemmPair) { large_body<false, false, true>(); }
+
+int launch_large_pair(hipStream_t s, const GemmArgs& a, const GemmArgs& b) {
+  GemmPair pair;
+  pair.product[0] = a, pair.product[1] = b, pair.split = 8 * a.per_xcd;
+  hipLaunchKernelGGL(gemm_large_pair_kernel, dim3(8 * (a.per_xcd + b.per_xcd)), dim3(512), 0, s, pair);
+  RTP_LAUNCH_CHECK();
+  return RTP_OK;
 }
 
 int launch_large(hipStream_t s, const GemmArgs& a, bool akc, bool bkc) {

@@ -925,6 +925,8 @@ int launch_split(hipStream_t s, const GemmArgs& a, bool akc, bool bkc, int bm, b
 
 // bf16 products in tiles of 256 x 256 by workgroups that stay (gemm_large.hip); two K slabs or more, no update, no statistics.
 int launch_large(hipStream_t s, const GemmArgs& a, bool akc, bool bkc);
+// Two weight gradients at once, a tile a workgroup: per_xcd of both together at most 32.
+int launch_large_pair(hipStream_t s, const GemmArgs& a, const GemmArgs& b);
 
 // `copies` x `segs` matrices of `lines` lines of `len` bf16 elements -> lines of whole 16-byte vectors, zeros behind their ends, all
 // contiguous (gemm_pack.hip).

@@ -140,6 +140,7 @@ RTP_ENTRY_POINTS(WRAP_X, WRAP_P)
 
 decltype(&rtp_gemm) f_gemm = nullptr;
 decltype(&rtp_gemm_workspace) f_gemm_workspace = nullptr;
+decltype(&rtp_gemm_pair) f_gemm_pair = nullptr;
 decltype(&rtp_gemm_rowsum_fused) f_rowsum_fused = nullptr;
 decltype(&rtp_gemm_sgd_fused) f_sgd_fused = nullptr;
 decltype(&rtp_rotated_linear_fwd) f_linear_fwd = nullptr;
@@ -159,6 +160,7 @@ PyObject* py_bind(PyObject*, PyObject* args) {
     return f != nullptr;
   };
   bool ok = get("rtp_last_error", f_last_error) && get("rtp_gemm", f_gemm) && get("rtp_gemm_workspace", f_gemm_workspace) &&
+            get("rtp_gemm_pair", f_gemm_pair) &&
             get("rtp_gemm_rowsum_fused", f_rowsum_fused) && get("rtp_gemm_sgd_fused", f_sgd_fused) &&
             get("rtp_rotated_linear_fwd", f_linear_fwd) && get("rtp_rotated_linear_bwd", f_linear_bwd);
 #define RESOLVE(name) ok = ok && get(#name, f_##name);
@@ -223,9 +225,9 @@ Field g_fields[] = {
 #undef AT
 PyObject* g_field_index = nullptr;  // name -> index into g_fields
 
-// Runs the product on the current stream and adds to `done` ROWSUM (1) if the row sums asked for were produced, SGD (2) if the
-// update was applied: what the operands do not allow is left out of the launch and reported by its missing bit.
-bool launch_product(int dt, rtp_gemm_desc& d, uint32_t flags, int& done) {
+// Adds to `done` ROWSUM (1) if the row sums asked for will be produced, SGD (2) if the update will be applied: what the operands do not
+// allow is left out of the launch and reported by its missing bit.
+void settle_product(int dt, rtp_gemm_desc& d, uint32_t flags, int& done) {
   if (d.sgd_master) {
     void *const master = d.sgd_master, *const weights = d.sgd_weights;
     d.sgd_master = d.sgd_weights = nullptr;
@@ -246,6 +248,10 @@ bool launch_product(int dt, rtp_gemm_desc& d, uint32_t flags, int& done) {
     else
       d.a_rowsum = nullptr, d.rowsum_sg = 0;
   }
+}
+// Runs the product on the current stream.
+bool launch_product(int dt, rtp_gemm_desc& d, uint32_t flags, int& done) {
+  settle_product(dt, d, flags, done);
   void* st = current_stream();
   const int rc = (WithoutGil(), Workspace(), f_gemm(st, dt, &d));
   if (rc < 0) raise_status(rc);
@@ -530,6 +536,71 @@ PyObject* py_row_wgrad(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
   return run_product(dt, d, flags);
 }
 
+// attention_wgrad(dout, o, dqkv, x, grads, first, cnt, accumulate, w_o, b_o, width, part, b_in, masters, weights, lr, clip, skip_store, apart) ->
+// done flags, the in-projection's two bits up: the weight gradients of an attention layer whose shards hold W_in [3 part, width] at
+// 0 and W_o [width, part] at w_o (biases at b_in, b_o or None) for the runs of `cnt` shards from `first` on, in one launch where that is
+// faster and not `apart`: grads[first+g] (+)= dout^T o[:, block g] and dqkv[:, block g]^T x.  masters / weights: None, or the addresses of the
+// fp32 parameters and their copies (W_o's, W_in's) as pairs.
+PyObject* py_attention_wgrad(PyObject*, PyObject* const* a, Py_ssize_t nargs) {
+  if (nargs != 19) return PyErr_Format(PyExc_TypeError, "attention_wgrad: 19 arguments, got %zd", nargs);
+  if (!tensors_at("attention_wgrad", a, {0, 1, 2, 3, 4})) return nullptr;
+  const at::Tensor &dout = THPVariable_Unpack(a[0]), &o = THPVariable_Unpack(a[1]), &dqkv = THPVariable_Unpack(a[2]),
+                   &x = THPVariable_Unpack(a[3]), &grads = THPVariable_Unpack(a[4]);
+  int64_t first, cnt, w_o, width, part;
+  if (!from_py(a[5], first) || !from_py(a[6], cnt) || !from_py(a[8], w_o) || !from_py(a[10], width) || !from_py(a[11], part)) return nullptr;
+  rtp_rotated_linear lo, li;
+  int dt;
+  Mat mdo, mo, mdq, mx;
+  if (!layer_of(grads, w_o, a[9], width, part, lo, dt) || !layer_of(grads, 0, a[12], 3 * part, width, li, dt) || !as_mat(dout, "operand", mdo) ||
+      !as_mat(o, "operand", mo) || !as_mat(dqkv, "operand", mdq) || !as_mat(x, "operand", mx))
+    return nullptr;
+  for (const at::Tensor* t : {&dout, &o, &dqkv, &x})
+    if (t->scalar_type() != grads.scalar_type() || t->size(0) != dout.size(0) || !t->is_cuda())
+      return bad("attention_wgrad: operands are matrices of as many rows in the gradients' dtype on the GPU");
+  if (first < 0 || cnt < 1 || first + cnt > lo.shards || mdo.cols < width || mx.cols < width || mo.cols < (first + cnt) * part ||
+      mdq.cols < (first + cnt) * 3 * part || w_o + width * part > lo.numel || 3 * part * width > lo.numel)
+    return bad("attention_wgrad: operands do not fit the layer");
+  const bool accumulate = PyObject_IsTrue(a[7]);
+  const uint32_t flags = RTP_GEMM_STREAM_OUT | (accumulate ? (uint32_t)RTP_GEMM_ROWSUM_ACCUM : 0u) | (PyObject_IsTrue(a[17]) ? (uint32_t)RTP_GEMM_SGD_SKIP_OUT : 0u);
+  void *masters[2] = {nullptr, nullptr}, *weights[2] = {nullptr, nullptr};
+  float lr = 0.0f, clip = 0.0f;
+  for (int side = 0; side < 2; ++side)
+    if (PyObject* v = a[13 + side]; v != Py_None) {
+      void** to = side ? weights : masters;
+      if (!PyTuple_Check(v) || PyTuple_GET_SIZE(v) != 2 || !from_py(PyTuple_GET_ITEM(v, 0), to[0]) || !from_py(PyTuple_GET_ITEM(v, 1), to[1]))
+        return PyErr_Occurred() ? nullptr : bad("attention_wgrad: a pair of addresses");
+    }
+  if (!from_py(a[15], lr) || !from_py(a[16], clip)) return nullptr;
+  auto gradient = [&](const rtp_rotated_linear& L, const Mat& g, int64_t g_col, int64_t g_step, const Mat& in, int64_t in_col, int64_t in_step, int which) {
+    const int64_t es = grads.element_size();
+    rtp_gemm_desc d = product(L.n_s, L.k, g.rows, false, false);
+    d.a = g.p + g_col * es, d.lda = g.ld, d.a_sg = g_step;
+    d.b = in.p + in_col * es, d.ldb = in.ld, d.b_sg = in_step;
+    d.c_out = at_element(grads, first * L.numel + L.w_off), d.ldc = L.k, d.c_sg = L.numel;
+    d.c_in = accumulate ? d.c_out : nullptr, d.ld_cin = L.k, d.cin_sg = L.numel;
+    if (L.bias_off >= 0) d.a_rowsum = at_element(grads, first * L.numel + L.bias_off);
+    d.rowsum_sg = L.numel;
+    d.groups = cnt;
+    d.sgd_master = masters[which], d.sgd_weights = weights[which], d.sgd_lr = lr, d.sgd_clip = clip;
+    return d;
+  };
+  rtp_gemm_desc d_o = gradient(lo, mdo, 0, 0, mo, first * part, part, 0);
+  rtp_gemm_desc d_in = gradient(li, mdq, first * 3 * part, 3 * part, mx, 0, 0, 1);
+  int done_o = 0, done_in = 0;
+  settle_product(dt, d_o, flags, done_o);
+  settle_product(dt, d_in, flags, done_in);
+  void* st = current_stream();
+  const bool apart = PyObject_IsTrue(a[18]);
+  auto launch = [&] {
+    if (!apart) return f_gemm_pair(st, dt, &d_o, &d_in);
+    const int rc = f_gemm(st, dt, &d_o);
+    return rc < 0 ? rc : f_gemm(st, dt, &d_in);
+  };
+  const int rc = (WithoutGil(), Workspace(), launch());
+  if (rc < 0) return raise_status(rc);
+  return PyLong_FromLong(done_o | done_in << 2);
+}
+
 // bmm(a, a_off, lda, a_kcontig, a_s, a_sg,  b, ... (as a),  c, c_off, ldc, c_s, c_sg,  m, n, k, batch, zdiv, groups):
 // C = A B for every (group, outer, inner) problem, offsets and strides in elements, (outer, inner) strides as pairs; C in the
 // operands' dtype or fp32
@@ -763,7 +834,8 @@ PyTypeObject g_book_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 PyMethodDef g_methods[] = {{"bind", Entry<py_bind>::call, METH_VARARGS, nullptr},
                            {"gemm", (PyCFunction)(void*)Entry<py_gemm>::call, METH_FASTCALL | METH_KEYWORDS, nullptr},
                            METHOD(linear_fwd) METHOD(linear_bwd) METHOD(row_fwd) METHOD(row_dgrad)
-                           METHOD(row_wgrad) METHOD(bmm) METHOD(experts_fwd) METHOD(experts_dgrad) METHOD(experts_wgrad)
+                           METHOD(row_wgrad) METHOD(attention_wgrad) METHOD(bmm) METHOD(experts_fwd)
+                           METHOD(experts_dgrad) METHOD(experts_wgrad)
                            RTP_ENTRY_POINTS(METHOD, METHOD){nullptr, nullptr, 0, nullptr}};
 #undef METHOD
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_rtp_native", "librtp_hip.so for the calls of a training step", -1, g_methods};

@@ -298,10 +298,7 @@ class _AttentionFn(torch.autograd.Function):
 
         def param_grads():
             for first, cnt, accumulate in runs:
-                S.row_wgrad(dout2, o, store.grads, first, w_o_off, E, e_s, first * e_s, cnt, accumulate,
-                            b_off=b_o_off if layer.has_bias else None, store=store)
-                S.col_wgrad(dqkv, x2, store.grads, first, 0, 3 * e_s, E, first * 3 * e_s, cnt, accumulate,
-                            b_off=b_in_off if layer.has_bias else None, store=store)
+                S.attention_wgrad(dout2, o, dqkv, x2, store, first, cnt, accumulate, w_o_off, b_o_off, E, e_s, b_in_off)
             store.grads_ready()
 
         run_wgrad(dev, param_grads, (dout2, o, dqkv, x2))

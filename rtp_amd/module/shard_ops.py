@@ -12,7 +12,10 @@ from typing import Optional
 
 import torch
 
-from .. import _lib, ops
+from .. import _lib, ops, ring
+
+
+_ROWSUM_DONE, _SGD_DONE = 1, 2  # of native().gemm and its relatives
 
 
 def _rows(t: torch.Tensor):
@@ -125,6 +128,32 @@ def row_wgrad(dy2, x2, grads, first, w_off, n, k_s, col0, cnt, accumulate, b_off
                                       False)
     if b_off is not None and not done & _lib.ROTATED_BIAS_DONE:
         row_bgrad(dy2, grads, first, b_off, n, cnt, accumulate)
+
+
+def attention_wgrad(dout2, o, dqkv, x2, store, first, cnt, accumulate, w_o_off, b_o_off, E, e_s, b_in_off):
+    """row_wgrad of an attention layer's out-projection and col_wgrad of its in-projection (rows q, k, v at offset 0 of a shard),
+    in one launch where that is faster."""
+    grads, parts = store.grads, ((w_o_off, E * e_s), (0, 3 * e_s * E))
+    kws = [_fused(store, accumulate, first, cnt, *p) for p in parts]
+    # Beside the input gradients on another stream the CUs that a round leaves idle are in use, and two updates at once hold that stream up:
+    # replayed LM step 3690 us apart, 3716 together (without updates 4882 / 4870; on one stream 3863 / 3729).
+    apart = bool(kws[0]) and ring.wgrad_overlap()
+    if kws[0]:
+        sgd = kws[0]["sgd"]
+        weights = tuple(kw["sgd_weights"] for kw in kws)
+        update = (tuple(kw["sgd_master"] for kw in kws), weights if weights[0] else None, sgd.lr, sgd.clip, not sgd.keep_grads)
+    else:
+        update = (None, None, 0.0, 0.0, False)
+    done = ops.native().attention_wgrad(dout2, o, dqkv, x2, grads, first, cnt, accumulate, w_o_off, b_o_off, E, e_s, b_in_off, *update, apart)
+    for i, p in enumerate(parts):
+        if kws[0]:
+            kw = _fused(store, accumulate, first, cnt, *p)
+            kw["sgd"].missed = not done >> 2 * i & _SGD_DONE
+            _fused_done(store, kw)
+    if b_o_off is not None and not done & _ROWSUM_DONE:
+        row_bgrad(dout2, grads, first, b_o_off, E, cnt, accumulate)
+    if b_in_off is not None and not done >> 2 & _ROWSUM_DONE:
+        col_bgrad(dqkv, grads, first, b_in_off, 3 * e_s, first * 3 * e_s, cnt, accumulate)
 
 
 def row_bgrad(dy2, grads, first, b_off, n, cnt, accumulate):

@@ -1192,28 +1192,28 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d, PairPlan* plan = n
   static const double odd_slab_ns[2][2] = {{330.0, 750.0}, {480.0, 2100.0}}, odd_fixed_ns[2][2] = {{3600.0, 10000.0}, {3500.0, 4000.0}};
   static const int slab_bytes[kNumShapes] = {128, 128, 128, 128, 128, 128, 128};
   const bool vec = direct && a.vec_c;  // else the kernels for operands of any alignment
-  int shape = 3;  // 64 x 64 unless the model finds something cheaper
-  double best = 0.0;
-  for (int i = 0; fast && i < kNumShapes; ++i) {
+  constexpr double kNever = 1e300;
+  // ns of the first `m` rows in tiles of shape i
+  const auto price = [&](int i, int64_t m) {
     // the 256 x 256 kernel is built for 16-bit operands and has no statistics epilogue (never routed to it, forced or not)
-    if (i == 5 && (sizeof(T) != 2 || d->xent_mode == 1)) continue;
+    if (i == 5 && (sizeof(T) != 2 || d->xent_mode == 1)) return kNever;
     // ... and an update only where it is a weight gradient's and the parameters' rows are whole 128-byte lines: its waves write 64
     // columns each, and on rows that are not (3000 x 3000 x 512) it takes 49 us where 128 x 128 takes 38
-    if (i == 5 && d->sgd_master && (akc || bkc || d->ldc % 32 != 0)) continue;
-    if (i == 6 && d->xent_mode == 1) continue;  // 160 columns are no whole number of 64-column statistics blocks
-    if (!vec && i != 1 && i != 3) continue;  // the kernels for unaligned operands: 128 x 128 and 64 x 64
+    if (i == 5 && d->sgd_master && (akc || bkc || d->ldc % 32 != 0)) return kNever;
+    if (i == 6 && d->xent_mode == 1) return kNever;  // 160 columns are no whole number of 64-column statistics blocks
+    if (!vec && i != 1 && i != 3) return kNever;  // the kernels for unaligned operands: 128 x 128 and 64 x 64
     // 128 x 160 is priced at the rate measured where it is meant for -- products of at most two rounds of tiles, such
     // as the LM's logits layer (shards of 1280 columns); larger products keep the shapes measured on large products
-    if (i == 6 && ceil_div(d->m, 128) * ceil_div(d->n, 160) * nz > 512 && i != forced) continue;
+    if (i == 6 && ceil_div(m, 128) * ceil_div(d->n, 160) * nz > 512 && i != forced) return kNever;
     // It needs neither a full round nor a long contraction to pay: on 144 - 255 tiles it is one round where the others take
     // two or more (6000 x 2048 x 2048, 192 tiles: 51 us against 57 with 128 x 128 and 65 with 256 x 128), and at K = 512 it is
     // 89 us against 123 (8192^2).
-    if (i == 5 && ceil_div(d->k, 64) * d->ksegs < 2) continue;  // its pipeline is primed with two slabs
+    if (i == 5 && ceil_div(d->k, 64) * d->ksegs < 2) return kNever;  // its pipeline is primed with two slabs
     // never a tile that is mostly padding: a 32 x 32 problem (one attention head at seq 32) stays at 64 x 64
-    if ((!akc && (kShapes[i].bm & (kShapes[i].bm - 1))) || (!bkc && (kShapes[i].bn & (kShapes[i].bn - 1)))) continue;
-    if (kShapes[i].bm > 64 && kShapes[i].bm > ceil_div(d->m, 64) * 64) continue;
-    if (kShapes[i].bn > 64 && kShapes[i].bn > ceil_div(d->n, 64) * 64) continue;
-    const int64_t tiles = ceil_div(d->m, kShapes[i].bm) * ceil_div(d->n, kShapes[i].bn) * nz;
+    if ((!akc && (kShapes[i].bm & (kShapes[i].bm - 1))) || (!bkc && (kShapes[i].bn & (kShapes[i].bn - 1)))) return kNever;
+    if (kShapes[i].bm > 64 && kShapes[i].bm > ceil_div(m, 64) * 64) return kNever;
+    if (kShapes[i].bn > 64 && kShapes[i].bn > ceil_div(d->n, 64) * 64) return kNever;
+    const int64_t tiles = ceil_div(m, kShapes[i].bm) * ceil_div(d->n, kShapes[i].bn) * nz;
     const double nslabs = (double)ceil_div(d->k * (int64_t)sizeof(T), slab_bytes[i]) * (double)d->ksegs;
     // The 256 x 256 kernel finishes the rarer combinations block after block, a trip to memory each: with bias, addend and ReLU 8 of 1024 x
     // 1280 x 520 is 41.3 us (19.2 plain) against 41.1 (25.2) with 128 x 160 tiles, x 2048 61.5 (46.3) against 67.2 (58.3).
@@ -1231,17 +1231,60 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d, PairPlan* plan = n
       update = (rounds - 1.0) * round_ns(256.0) + round_ns((double)tiles - 256.0 * (rounds - 1.0));
     }
     const double slab = vec || direct ? slab_ns[i] : odd_slab_ns[sizeof(T) == 4][i == 1];
-    const double cost = rounds * (nslabs * slab + (vec ? outside : odd_fixed_ns[direct][i == 1])) + update;
-    if (plan && i == 5) {
-      plan->large = true;
-      plan->slabs = nslabs;
-      if (d->sgd_master)
-        plan->update_bytes = (double)tiles * 65536.0 * (8.0 + (d->sgd_weights ? 2.0 : 0.0) + (d->flags & RTP_GEMM_SGD_SKIP_OUT ? 0.0 : 2.0));
+    return rounds * (nslabs * slab + (vec ? outside : odd_fixed_ns[direct][i == 1])) + update;
+  };
+  const auto cheapest = [&](int64_t m, int& shape) {
+    double best = kNever;
+    shape = 3;  // 64 x 64 unless the model finds something cheaper
+    for (int i = 0; fast && i < kNumShapes; ++i) {
+      const double cost = price(i, m);
+      if (cost != kNever && i == forced) return shape = i, -1.0;
+      if (cost < best) best = cost, shape = i;
     }
-    if (best == 0.0 || cost < best || i == forced) {
-      best = i == forced ? -1.0 : cost;
-      shape = i;
+    return best;
+  };
+  int shape;
+  const double best = cheapest(d->m, shape);
+  // A last round of few 256 x 256 tiles takes as long as a full one, and a last row of tiles that is mostly padding as long as the others:
+  // whole rounds' rows (or whole tiles' rows) go in those, the others in the tiles that suit them, where the two launches are priced 5 %
+  // below the one.  us, one launch -> two, forward / input gradient / weight gradient layouts: 4352 x 4096 x 4096 159 / 165 / 178 -> 120 / 125 / 129, 6144
+  // x 3072 x 4096 159 / 165 / 178 -> 127 / 133 / 136, 4608 x 4096 x 2048 84 / 87 / 95 -> 71 / 74 / 76, 6000 x 6144 x 2048 161 / 150 / 157 -> 147 / 139 /
+  // 141, 2300 x 8192 x 2048 89 / 92 -> 68 / 71, 3000 x 6144 x 3000 131 / 131 / 143 -> 109 / 105 / 105; level, so not taken: 5632 x 4096 x 1024 47,
+  // 4096 x 6144 x 2048 87, 9000 x 5120 x 1536 112.
+  if (shape == 5 && best > 0.0 && !plan && !packed && !d->xent_mode) {
+    const int64_t row_tiles = ceil_div(d->n, 256) * nz, rounds = ceil_div(ceil_div(d->m, 256) * row_tiles, 256);
+    double least = 0.95 * best;
+    int64_t cut = 0;
+    const auto consider = [&](int64_t m) {
+      int other;
+      if (m <= 0 || m >= d->m) return;
+      const double cost = price(5, m) + cheapest(d->m - m, other) + 4000.0;
+      if (cost < least) least = cost, cut = m;
+    };
+    for (int64_t r = std::max<int64_t>(1, rounds - 2); r < rounds; ++r) consider(256 * r / row_tiles * 256);
+    consider(d->m / 256 * 256);
+    if (cut != 0) {
+      rtp_gemm_desc part = *d;
+      const int64_t es = (int64_t)sizeof(T);
+      part.m = cut;
+      if (int rc = launch_gemm<T>(s, &part)) return rc;
+      const auto down = [&](const void* x, int64_t ld, int64_t size) { return x ? (char*)x + cut * ld * size : nullptr; };
+      part.m = d->m - cut;
+      part.a = down(d->a, akc ? d->lda : 1, es);
+      part.c_out = down(d->c_out, d->ldc, d->flags & RTP_GEMM_OUT_F32 ? 4 : es);
+      part.c_in = down(d->c_in, d->ld_cin, d->flags & RTP_GEMM_CIN_F32 ? 4 : es);
+      part.gate = down(d->gate, d->ld_gate, es);
+      part.a_rowsum = down(d->a_rowsum, 1, es);
+      part.sgd_master = down(d->sgd_master, d->ldc, 4), part.sgd_weights = down(d->sgd_weights, d->ldc, es);
+      return launch_gemm<T>(s, &part);
     }
+  }
+  if (plan && price(5, d->m) != kNever) {
+    plan->large = true;
+    plan->slabs = (double)ceil_div(d->k, 64) * (double)d->ksegs;
+    if (d->sgd_master)
+      plan->update_bytes = (double)(ceil_div(d->m, 256) * ceil_div(d->n, 256) * nz) * 65536.0 *
+                           (8.0 + (d->sgd_weights ? 2.0 : 0.0) + (d->flags & RTP_GEMM_SGD_SKIP_OUT ? 0.0 : 2.0));
   }
   if (plan) {
     if (!plan->large) return RTP_OK;

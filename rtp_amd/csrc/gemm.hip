@@ -907,6 +907,36 @@ static bool rowsum_fused(const rtp_gemm_desc* d) {
   return !d->a_kcontig && d->batch == 1 && !is_tiny(d) && (takes_dma_kernel<T>(d) || takes_reg_kernel<T>(d));
 }
 
+// Few tiles, whatever the layout: see gemm_kwaves.hip.  256 tiles of 32 x 32 are one workgroup a CU, and up to there it is ahead at
+// every contraction from 256 on (measured in a replayed graph on 70 shapes x 3 layouts x 2 types; bf16 1.1 - 2.5 times, fp32 1.5 - 2.3).
+// From 257 on some CU has two and only fp32 with K of 768 and more gains, up to 512 (where 64 x 32, below, does not fit).  us, before -> this:
+// 256 tiles bf16 64 x 4096, K = 512 5.7 -> 4.6, 4096 19.2 -> 10.3; 288 tiles 384 x 768, K = 256 5.2 -> 6.7, 1024 7.6 -> 8.7, 2048
+// 12.1 -> 11.7; 512 tiles fp32 512 x 1024, K = 384 10.8 -> 12.6, 1024 19.6 -> 18.1; 768 tiles 512 x 1536, K = 2048 36 -> 44.
+// Operands that are not vector-aligned, 12 shapes: bf16 255 x 1023 x 3333 24.0 -> 17.6, 31 x 2049 x 515 8.6 -> 8.2, one of 25 behind
+// (7 x 8101 x 1027, input gradient, 13.4 -> 14.2); fp32 65.6 -> 28.5 and 15.8 -> 11.1.  (Row-contiguous fp32 has gemm_ksplit_kernel.)
+// With tiles of 64 x 32 twice as many outputs are one workgroup a CU: in fp32 ahead at any contraction (1.05 - 1.46 times on 24 shapes,
+// two of 72 behind by 1 and 3 %), in bf16 only at long ones, with operands that lie alike (K >= 2048: 1.0 - 1.2, unaligned weight gradients
+// 1.4 - 1.8; K = 512 0.83 - 0.98; the input gradient's layout 0.95 - 1.09).
+// 0: not few, otherwise the tile's rows.
+template <typename T>
+static int few_tiles(const rtp_gemm_desc* d) {
+  const int64_t nz = d->batch * d->groups, k_all = d->k * d->ksegs;
+  const int64_t tiles32 = ceil_div(d->m, 32) * ceil_div(d->n, 32) * nz, tiles64 = ceil_div(d->m, 64) * ceil_div(d->n, 32) * nz;
+  return tiles32 <= 256                                                                          ? 32
+         : tiles64 <= 256 && (sizeof(T) == 4 || (k_all >= 2048 && d->a_kcontig == d->b_kcontig)) ? 64
+         : sizeof(T) == 4 && k_all >= 768 && tiles32 <= 512                                      ? 32
+                                                                                                 : 0;
+}
+// Whether gemm_kwaves.hip takes the product, which splits its contraction over the waves of a workgroup.
+// A product under a ReLU stays in the order of its sums, here and below: a sum within its rounding of zero decides whether the
+// backward pass sees the unit at all, and of 16 M such sums (1000 tokens, 8 experts of 768 x 8064) some ten are that near.
+template <typename T>
+static bool takes_kwaves(const rtp_gemm_desc* d) {
+  const bool direct = takes_dma_kernel<T>(d);
+  return (direct || takes_reg_kernel<T>(d)) && !is_tiny(d) && !(d->flags & RTP_GEMM_RELU) && !d->xent_mode && d->batch * d->groups < 65536 &&
+         d->k * d->ksegs >= 256 && !(sizeof(T) == 4 && !direct && !d->a_kcontig && !d->b_kcontig) && few_tiles<T>(d) != 0;
+}
+
 // rtp_gemm_warm_next: bytes the next product launched by this host thread requests at its start.  A later call, from any
 // thread, ends an earlier hint: a caller holds the memory of the last one only, and a forward pass and its backward pass
 // run on two threads.
@@ -930,7 +960,8 @@ struct Packing {
 static Packing pack_plan(const rtp_gemm_desc* d, bool vec_c) {
   Packing p;
   const bool akc = d->a_kcontig, bkc = d->b_kcontig;
-  if (t_alloc == nullptr || d->batch != 1 || d->xent_mode || d->sgd_master || d->m < 128 || d->n < 128 || d->k < 8 || takes_dma_kernel<bf16_t>(d))
+  if (t_alloc == nullptr || d->batch != 1 || d->xent_mode || d->sgd_master || d->m < 128 || d->n < 128 || d->k < 8 || takes_dma_kernel<bf16_t>(d) ||
+      takes_kwaves<bf16_t>(d))  // (few tiles: that kernel loads at any alignment, and on its own the product keeps the order of its sums)
     return p;
   const int64_t ld_max = ((int64_t)1 << 23) - 64;
   const auto shape = [&](const void* x, int64_t ld, int64_t sg, int64_t sk, bool kc, int64_t rows) {
@@ -1107,27 +1138,11 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d, PairPlan* plan = n
     RTP_LAUNCH_CHECK();
     return RTP_OK;
   }
-  // Few tiles, whatever the layout: see gemm_kwaves.hip.  256 tiles of 32 x 32 are one workgroup a CU, and up to there it is ahead at
-  // every contraction from 256 on (measured in a replayed graph on 70 shapes x 3 layouts x 2 types; bf16 1.1 - 2.5 times, fp32 1.5 - 2.3).
-  // From 257 on some CU has two and only fp32 with K of 768 and more gains, up to 512 (where 64 x 32, below, does not fit).  us, before -> this:
-  // 256 tiles bf16 64 x 4096, K = 512 5.7 -> 4.6, 4096 19.2 -> 10.3; 288 tiles 384 x 768, K = 256 5.2 -> 6.7, 1024 7.6 -> 8.7, 2048
-  // 12.1 -> 11.7; 512 tiles fp32 512 x 1024, K = 384 10.8 -> 12.6, 1024 19.6 -> 18.1; 768 tiles 512 x 1536, K = 2048 36 -> 44.
-  // Operands that are not vector-aligned, 12 shapes: bf16 255 x 1023 x 3333 24.0 -> 17.6, 31 x 2049 x 515 8.6 -> 8.2, one of 25 behind
-  // (7 x 8101 x 1027, input gradient, 13.4 -> 14.2); fp32 65.6 -> 28.5 and 15.8 -> 11.1.  (Row-contiguous fp32 has gemm_ksplit_kernel.)
-  // A product under a ReLU stays in the order of its sums, here and below: a sum within its rounding of zero decides whether the
-  // backward pass sees the unit at all, and of 16 M such sums (1000 tokens, 8 experts of 768 x 8064) some ten are that near.
   const bool relu = d->flags & RTP_GEMM_RELU;
-  const int64_t tiles32 = ceil_div(d->m, 32) * ceil_div(d->n, 32) * nz, k_all = d->k * d->ksegs;
-  // With tiles of 64 x 32 twice as many outputs are one workgroup a CU: in fp32 ahead at any contraction (1.05 - 1.46 times on 24 shapes,
-  // two of 72 behind by 1 and 3 %), in bf16 only at long ones, with operands that lie alike (K >= 2048: 1.0 - 1.2, unaligned weight gradients
-  // 1.4 - 1.8; K = 512 0.83 - 0.98; the input gradient's layout 0.95 - 1.09).
-  const int64_t tiles64 = ceil_div(d->m, 64) * ceil_div(d->n, 32) * nz;
-  const int kw_bm = tiles32 <= 256                                                                 ? 32
-                    : tiles64 <= 256 && (sizeof(T) == 4 || (k_all >= 2048 && akc == bkc))          ? 64
-                    : sizeof(T) == 4 && k_all >= 768 && tiles32 <= 512                             ? 32
-                                                                                                   : 0;
-  if (plan && (!a.vec_c || kw_bm != 0 || k_all <= 128)) return RTP_OK;
-  if (fast && !packed && !relu && !d->xent_mode && nz < 65536 && k_all >= 256 && !(sizeof(T) == 4 && !direct && !akc && !bkc) && kw_bm != 0) {
+  const int64_t k_all = d->k * d->ksegs;
+  if (plan && (!a.vec_c || few_tiles<T>(d) != 0 || k_all <= 128)) return RTP_OK;
+  if (!packed && takes_kwaves<T>(d)) {
+    const int kw_bm = few_tiles<T>(d);
     a.tiles_m = (int)ceil_div(d->m, kw_bm);
     a.tiles_n = (int)ceil_div(d->n, 32);
     static const char* const names[2][2][2] = {{{"gemm_f32_kwaves_rc_rc", "gemm_f32_kwaves_rc_kc"}, {"gemm_f32_kwaves_kc_rc", "gemm_f32_kwaves_kc_kc"}},

@@ -186,3 +186,21 @@ def test_captured_layer_and_two_streams():
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(held, want[i]))
         assert all(torch.equal(a, b) for a, b in zip(eager, want[(i + 1) % 3]))
+
+
+# weight gradients of 100, 256 (64 x 32), 160 and 232 tiles, an input gradient of 88; the last one's 512 x 600 are 304 tiles of 32 x 32
+@pytest.mark.parametrize("akc,bkc,m,n,k,few", [(False, False, 300, 300, 8192, True), (False, False, 500, 1000, 8000, True),
+                                               (False, False, 130, 1000, 8190, True), (False, False, 500, 900, 8000, True),
+                                               (True, False, 250, 333, 9001, True), (True, False, 512, 600, 12001, False)])
+def test_few_tiles_stay_with_their_kernel(akc, bkc, m, n, k, few):
+    """What gemm_kwaves.hip takes it takes at any alignment, scratch memory or not: its order of the sums is another one."""
+    gen = torch.Generator().manual_seed(m + n + k)
+    _, a, af = _operand(gen, m, k, akc, 1, 1, 1)
+    _, b, bf = _operand(gen, n, k, bkc, 1, 1, 1)
+    outs = [torch.full((m, n), float("nan"), dtype=BF, device=DEV) for _ in range(2)]
+    kw = dict(a=a.data_ptr(), b=b.data_ptr(), m=m, n=n, k=k, lda=a.stride(1), ldb=b.stride(1), ldc=n, a_kcontig=akc, b_kcontig=bkc)
+    names = _packed(dict(kw, c_out=outs[0].data_ptr()), not few)
+    assert not few or (len(names) == 1 and "kwaves" in names[0]), names
+    _direct(dict(kw, c_out=outs[1].data_ptr()))
+    assert torch.equal(*outs)
+    assert rel_err(outs[0], af[0].float() @ bf[0].float().t()) <= TOL[BF]

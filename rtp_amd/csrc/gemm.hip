@@ -1003,9 +1003,10 @@ struct PairPlan {
   double slabs = 0.0, update_bytes = 0.0, flops = 0.0, bytes = 0.0;
 };
 
-// plan: nothing is launched, it is filled instead.
+// plan: nothing is launched, it is filled instead.  in_order: rows of a product whose others go in another launch, so that the contraction is
+// summed in one sequence, as there: equal rows have equal results wherever they are.
 template <typename T>
-static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d, PairPlan* plan = nullptr) {
+static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d, PairPlan* plan = nullptr, bool in_order = false) {
   if (plan && (sizeof(T) != 2 || d->a_kcontig || d->b_kcontig || d->xent_mode || is_tiny(d) || !takes_dma_kernel<T>(d))) return RTP_OK;
   // the hint of rtp_gemm_warm_next rides in this launch or ends with it
   const void* warm_src = warm_source();
@@ -1141,7 +1142,7 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d, PairPlan* plan = n
   const bool relu = d->flags & RTP_GEMM_RELU;
   const int64_t k_all = d->k * d->ksegs;
   if (plan && (!a.vec_c || few_tiles<T>(d) != 0 || k_all <= 128)) return RTP_OK;
-  if (!packed && takes_kwaves<T>(d)) {
+  if (!packed && !in_order && takes_kwaves<T>(d)) {
     const int kw_bm = few_tiles<T>(d);
     a.tiles_m = (int)ceil_div(d->m, kw_bm);
     a.tiles_n = (int)ceil_div(d->n, 32);
@@ -1266,6 +1267,8 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d, PairPlan* plan = n
   // x 3072 x 4096 159 / 165 / 178 -> 127 / 133 / 136, 4608 x 4096 x 2048 84 / 87 / 95 -> 71 / 74 / 76, 6000 x 6144 x 2048 161 / 150 / 157 -> 147 / 139 /
   // 141, 2300 x 8192 x 2048 89 / 92 -> 68 / 71, 3000 x 6144 x 3000 131 / 131 / 143 -> 109 / 105 / 105; level, so not taken: 5632 x 4096 x 1024 47,
   // 4096 x 6144 x 2048 87, 9000 x 5120 x 1536 112.
+  // Few rows behind the cut stay with these tiles too, in the order of the sums before it: gemm_kwaves.hip would be faster, us, this / that, 4128 x
+  // 4096 x 2048 70 / 73 / 76 against 66 / 70 / 75, 4104 x 4096 x 8192 234 / 245 / 262 against 217 / 236 / 256, but equal rows would differ.
   if (shape == 5 && best > 0.0 && !plan && !packed && !d->xent_mode) {
     const int64_t row_tiles = ceil_div(d->n, 256) * nz, rounds = ceil_div(ceil_div(d->m, 256) * row_tiles, 256);
     double least = 0.95 * best;
@@ -1282,7 +1285,7 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d, PairPlan* plan = n
       rtp_gemm_desc part = *d;
       const int64_t es = (int64_t)sizeof(T);
       part.m = cut;
-      if (int rc = launch_gemm<T>(s, &part)) return rc;
+      if (int rc = launch_gemm<T>(s, &part, nullptr, true)) return rc;
       const auto down = [&](const void* x, int64_t ld, int64_t size) { return x ? (char*)x + cut * ld * size : nullptr; };
       part.m = d->m - cut;
       part.a = down(d->a, akc ? d->lda : 1, es);
@@ -1291,7 +1294,7 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d, PairPlan* plan = n
       part.gate = down(d->gate, d->ld_gate, es);
       part.a_rowsum = down(d->a_rowsum, 1, es);
       part.sgd_master = down(d->sgd_master, d->ldc, 4), part.sgd_weights = down(d->sgd_weights, d->ldc, es);
-      return launch_gemm<T>(s, &part);
+      return launch_gemm<T>(s, &part, nullptr, true);
     }
   }
   if (plan && price(5, d->m) != kNever) {

@@ -76,3 +76,38 @@ def test_route_and_groups(m, n, groups, two):
     assert (len(names) == 2) == two, names
     for g in range(groups):
         assert rel_err(out[g], a[g].float() @ b[g].float().t()) <= TOL[BF]
+
+
+@pytest.mark.parametrize("akc,bkc,update", [(True, True, False), (True, False, False), (False, False, False), (False, False, True)])
+@pytest.mark.parametrize("m,extra", [(4128, 32), (8200, 8)])
+def test_equal_rows_are_equal_on_either_side_of_the_cut(akc, bkc, update, m, extra):
+    """The few rows behind the cut are by themselves a product that gemm_kwaves.hip would take, whose sums have another order.  Equal bits, row sums
+    and updated parameters too; an update of 4128 rows is not cut, so it goes over 8200 alone."""
+    from rtp_amd import ops
+    if update and m != 8200:
+        m, extra = 8224, 32
+    n, k = 4096, 2048
+    gen = torch.Generator().manual_seed(m)
+    a, b, ref = _pair(gen, m, n, k, akc, bkc)
+    rows = a if akc else a.t()
+    rows[m - extra:] = rows[:extra]
+    ref[m - extra:] = ref[:extra]
+    out, sums = torch.full((m, n), float("nan"), dtype=BF, device=DEV), torch.full((m,), float("nan"), dtype=BF, device=DEV)
+    kw, compared = {}, [out]
+    if not akc:
+        kw["rowsum"] = sums.data_ptr()
+        compared.append(sums)
+    if update:
+        class Sgd:
+            lr, clip, keep_grads, missed = 1e-3, 0.05, True, False
+        master = torch.randn(m, n, generator=gen).to(DEV)
+        master[m - extra:] = master[:extra]
+        copy = torch.full((m, n), float("nan"), dtype=BF, device=DEV)
+        kw.update(sgd=Sgd(), sgd_master=master.data_ptr(), sgd_weights=copy.data_ptr())
+        compared += [master, copy]
+    names = _names(lambda: ops.gemm_raw(BF, a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=a.stride(0),
+                                        ldb=b.stride(0), ldc=n, a_kcontig=akc, b_kcontig=bkc, **kw))
+    assert len(names) == 2, names
+    assert rel_err(out, ref) <= TOL[BF] and not out.isnan().any()
+    for t in compared:
+        assert torch.equal(t[m - extra:], t[:extra])

@@ -21,6 +21,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cstring>
 #include <exception>
 #include <string>
@@ -172,20 +173,33 @@ PyObject* py_bind(PyObject*, PyObject* args) {
 
 // Scratch memory for the products launched while it lives, from torch's allocator on the current stream: given back with it, for what
 // that stream runs afterwards.  (The allocator itself, not at::empty: no dispatch, and no Python under a mode of it.)
+// Before the allocator refuses it waits for the device and gives all that it holds in reserve back, which costs a program near its memory's
+// end more than the copies gain.  So a thread that was refused asks for as much on that device again only after a second.
 struct Workspace {
+  struct Refusal {
+    std::chrono::steady_clock::time_point until;
+    size_t bytes = 0;
+    int device = -1;
+  };
+  static thread_local Refusal refused;
   std::vector<c10::DataPtr> held;
   Workspace() { f_gemm_workspace(&get, this); }
   ~Workspace() { f_gemm_workspace(nullptr, nullptr); }
   static void* get(void* self, size_t bytes) noexcept {
+    int device = -1;
     try {
+      device = c10::hip::getCurrentHIPStream().device_index();
+      if (device == refused.device && bytes >= refused.bytes && std::chrono::steady_clock::now() < refused.until) return nullptr;
       auto& held = static_cast<Workspace*>(self)->held;
       held.push_back(c10::GetAllocator(c10::kCUDA)->allocate(bytes));
       return held.back().get();
     } catch (...) {  // no memory: the product does without
+      refused = {std::chrono::steady_clock::now() + std::chrono::seconds(1), bytes, device};
       return nullptr;
     }
   }
 };
+thread_local Workspace::Refusal Workspace::refused;
 
 int dtype_code(at::ScalarType t) {
   return t == at::kFloat ? (int)RTP_F32 : t == at::kBFloat16 ? (int)RTP_BF16 : -1;

@@ -204,3 +204,36 @@ def test_few_tiles_stay_with_their_kernel(akc, bkc, m, n, k, few):
     _direct(dict(kw, c_out=outs[1].data_ptr()))
     assert torch.equal(*outs)
     assert rel_err(outs[0], af[0].float() @ bf[0].float().t()) <= TOL[BF]
+
+
+def test_a_refusal_of_memory_is_remembered():
+    """Where torch's allocator has no memory left it is asked once and not by every product; a second later it is asked again."""
+    import time
+
+    from rtp_amd import ops
+    gen = torch.Generator().manual_seed(3)
+    m, n, k = 4098, 4096, 2050
+    _, a, _ = _operand(gen, m, k, False, 1, 1, 1)
+    _, b, _ = _operand(gen, n, k, False, 1, 1, 1)
+    outs = [torch.zeros(m, n, dtype=BF, device=DEV) for _ in range(7)]
+    kw = dict(a=a.data_ptr(), b=b.data_ptr(), m=m, n=n, k=k, lda=a.stride(1), ldb=b.stride(1), ldc=n, a_kcontig=False, b_kcontig=False)
+    refusals = lambda: torch.cuda.memory_stats()["num_ooms"]  # noqa: E731
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total, fill = torch.cuda.get_device_properties(DEV).total_memory, []
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (4 << 20)) / total)
+    try:
+        with pytest.raises(torch.cuda.OutOfMemoryError):  # what the allocator still holds in pieces
+            while True:
+                fill.append(torch.empty(8 << 20, dtype=torch.uint8, device=DEV))
+        before = refusals()
+        for out in outs[:5]:
+            ops.gemm_raw(BF, c_out=out.data_ptr(), **kw)
+        assert refusals() == before + 1
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+        fill.clear()
+        time.sleep(1.1)
+    _packed(dict(kw, c_out=outs[5].data_ptr()))
+    _direct(dict(kw, c_out=outs[6].data_ptr()))
+    assert all(torch.equal(out, outs[6]) for out in outs[:6])

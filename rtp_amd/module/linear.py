@@ -289,7 +289,10 @@ class _ParallelLinearBase(RotatedLayer):
         self.linear = self.linears[self.rank]
 
     def forward(self, input_: torch.Tensor) -> torch.Tensor:
-        return apply_function(type(self)._fn, input_, self._anchor, self)
+        fn = type(self)._fn
+        if fn is _ColumnLinearFn or fn is _RowLinearFn:
+            return apply_function(fn, input_, self._anchor, self)
+        return fn.apply(input_, self._anchor, self)  # a subclass's own, which may use all that apply gives a function
 
     def extra_repr(self) -> str:
         return (f"in_features={self.in_features}, out_features={self.out_features}, bias={self.has_bias}, "

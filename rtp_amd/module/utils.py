@@ -86,7 +86,8 @@ def apply_function(fn, *args):
     """fn.apply(*args), or fn.forward alone where nothing can come of the rest: gradients are off, and no transform (vmap, grad,
     jvp), forward-mode level, tracer or compiler is looking, all of which take hold of a function in apply.  apply enters the
     autograd machinery without gradients too and is then a part of a small layer's forward that is felt (32 x 256 x 256: 12.2 -> 10.5 us a call).
-    For functions that return new tensors: apply gives a view where a function returns one of its arguments."""
+    For the layers' own functions, which return new tensors and use nothing of the context but what _NoGradContext has: apply gives a view
+    where a function returns one of its arguments."""
     if (torch.is_grad_enabled() or torch.compiler.is_compiling() or torch._C._are_functorch_transforms_active()
             or forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None):
         return fn.apply(*args)

@@ -79,6 +79,31 @@ def test_results_of_either_refuse_a_later_in_place_use_alike():
     _Twice.calls.clear()
 
 
+def test_a_subclass_with_a_function_of_its_own():
+    """It may use all of apply's context, and hand an argument back."""
+    from rtp_amd import emulate_shards
+    from rtp_amd.module.linear import ColumnParallelLinear
+
+    class Own(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x, anchor, layer):
+            ctx.set_materialize_grads(False)
+            assert ctx.needs_input_grad[0] == x.requires_grad
+            ctx.mark_dirty(x)
+            return x.add_(1)
+
+    class Layer(ColumnParallelLinear):
+        _fn = Own
+
+    with emulate_shards(2):
+        layer = Layer(8, 4)
+    x = torch.zeros(3, 8)
+    for off in (torch.no_grad, torch.inference_mode):
+        with off():
+            assert layer(x) is x
+    assert torch.equal(x, torch.full((3, 8), 2.0))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_layers_give_the_same_with_and_without_gradients(dtype):

@@ -4,8 +4,14 @@ from __future__ import annotations
 from typing import List, Sequence
 
 import torch
-from torch._C._functorch import unwrap_if_dead
-from torch.autograd import forward_ad
+
+try:  # what takes hold of an autograd function, besides gradients; not public: in a torch without one of them functions go through apply
+    from torch._C import _are_functorch_transforms_active as _in_transform, _get_tracing_state as _tracing
+    from torch._C._functorch import unwrap_if_dead
+    from torch.autograd import forward_ad
+    _may_run_alone = isinstance(forward_ad._current_level, int)  # (-1: outside all levels)
+except (ImportError, AttributeError):
+    _may_run_alone = False
 
 
 def ensure_divisibility(numerator: int, denominator: int) -> None:
@@ -88,7 +94,7 @@ def apply_function(fn, *args):
     autograd machinery without gradients too and is then a part of a small layer's forward that is felt (32 x 256 x 256: 12.2 -> 10.5 us a call).
     For the layers' own functions, which return new tensors and use nothing of the context but what _NoGradContext has: apply gives a view
     where a function returns one of its arguments."""
-    if (torch.is_grad_enabled() or torch.compiler.is_compiling() or torch._C._are_functorch_transforms_active()
-            or forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None):
+    if (torch.is_grad_enabled() or not _may_run_alone or torch.compiler.is_compiling() or _in_transform()
+            or forward_ad._current_level >= 0 or _tracing() is not None):
         return fn.apply(*args)
     return fn.forward(_NoGradContext(), *[unwrap_if_dead(a) if isinstance(a, torch.Tensor) else a for a in args])

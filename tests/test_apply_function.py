@@ -79,6 +79,22 @@ def test_results_of_either_refuse_a_later_in_place_use_alike():
     _Twice.calls.clear()
 
 
+@pytest.mark.parametrize("where,name", [(torch._C, "_are_functorch_transforms_active"), (torch._C, "_get_tracing_state"),
+                                        (torch._C._functorch, "unwrap_if_dead"), (forward_ad, "_current_level")])
+def test_in_a_torch_without_one_of_the_names_it_is_apply(where, name, monkeypatch):
+    import importlib.util
+
+    import rtp_amd.module.utils as utils
+    with monkeypatch.context() as m:
+        m.delattr(where, name)
+        spec = importlib.util.spec_from_file_location("utils_of_another_torch", utils.__file__)
+        other = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(other)
+    with torch.no_grad():
+        other.apply_function(_Twice, torch.randn(2, 3))
+    assert not _plain()
+
+
 def test_a_subclass_with_a_function_of_its_own():
     """It may use all of apply's context, and hand an argument back."""
     from rtp_amd import emulate_shards

@@ -952,6 +952,33 @@ static const void* warm_source() {
 static thread_local rtp_alloc_fn t_alloc = nullptr;
 static thread_local void* t_alloc_context = nullptr;
 
+// The price of 256 x 256 tiles and of an update, for every rule that weighs them: ns in the units of launch_gemm's table, where only ratios matter.
+// 256 x 256 is priced by its ratio to the others with every CU busy.  Every tile forced on 59 products x 3 layouts, operands from memory: with
+// these two numbers the shape taken costs 0.1 % over the best one in the mean (with 1350 and 5000 ns, the price of the kernel before this
+// one, 0.8 %), the most 12 % (4096 x 2048 x 6144, 128 tiles: 119 us with 256 x 128 against 111); it is the same for 975 - 1100 and 4000 -
+// 5000 ns.  Where 256 x 256 is close and not taken: 4096 x 2048 x 2048, 128 tiles, 39 - 43 us against 37 - 38.
+constexpr double kLargeSlabNs = 1050.0, kLargeTileNs = 4500.0;
+// The kernel finishes the rarer combinations block after block, a trip to memory each: with bias, addend and ReLU 8 of 1024 x 1280 x 520 is 41.3 us
+// (19.2 plain) against 41.1 (25.2) with 128 x 160 tiles, x 2048 61.5 (46.3) against 67.2 (58.3).
+static bool rare_epilogue(const rtp_gemm_desc* d) {
+  return (d->bias != nullptr) + (d->c_in != nullptr) + (d->gate != nullptr) > 1 || ((d->flags & RTP_GEMM_RELU) && !d->bias) ||
+         (d->flags & (RTP_GEMM_OUT_F32 | RTP_GEMM_CIN_F32)) || d->xent_mode;
+}
+static double large_ns(double rounds, double slabs, bool rare) {
+  return rounds * (slabs * kLargeSlabNs + kLargeTileNs + (rare ? 3000.0 : 0.0));
+}
+// An update moves 10 bytes a parameter (12 with the gradient) behind the K loop, a round's tiles together at the memory's 4.9 TB/s, a CU at no
+// more than 32 bytes a ns.  So few large tiles are behind where they leave CUs idle: us with 128 x 128 / 256 x 256, K = 1024, 2048 x 2048
+// 19.2 / 39, 8 of 1280 x 2048 97 / 101, 6144 x 2048 59.7 / 49.9, 4096 x 4096 75 / 61; 8192 x 2048 x 4096 174 / 145.
+static double update_bytes(const rtp_gemm_desc* d) {  // a parameter
+  return !d->sgd_master ? 0.0 : 8.0 + (d->sgd_weights ? 2.0 : 0.0) + (d->flags & RTP_GEMM_SGD_SKIP_OUT ? 0.0 : 2.0);
+}
+static double update_ns(double tiles, double tile_bytes) {
+  const auto round_ns = [&](double n) { return std::max(n * tile_bytes / 4900.0, tile_bytes / 32.0); };
+  const double rounds = (double)ceil_div((int64_t)tiles, 256);
+  return (rounds - 1.0) * round_ns(256.0) + round_ns(tiles - 256.0 * (rounds - 1.0));
+}
+
 // Which operands of a bf16 product are copied to whole vectors first.
 struct Packing {
   bool a = false, b = false;
@@ -980,8 +1007,8 @@ static Packing pack_plan(const rtp_gemm_desc* d, bool vec_c) {
   if (vectors > (1 << 26) || p.sa.len > ld_max || p.sb.len > ld_max || (!a && d->lda > ld_max) || (!b && d->ldb > ld_max)) return p;
   // It pays where the copies (their bytes in and out at 4.5 TB/s, 8 us each between their neighbours on the stream) take less than what
   // the register loaders add.  ns a slab of 128 x 128, every CU busy: register loaders 600 / 700 / 800 (both operands k-contiguous /
-  // one / none), direct-to-LDS 480; outside the slabs 6 and 5 us; 256 x 256, which only aligned results can take, 1650 a slab and
-  // 6 us.  us without -> with the copies, forward / input gradient / weight gradient (=: not taken): 6546 x 482 x 6400, 8 shards, 460 / 540 /
+  // one / none), direct-to-LDS 480; outside the slabs 6 and 5 us; 256 x 256, which only aligned results can take, 1.5 times its price (1650 a
+  // slab and 6 us were seen).  us without -> with the copies, forward / input gradient / weight gradient (=: not taken): 6546 x 482 x 6400, 8 shards, 460 / 540 /
   // 628 -> 367 / 353 / 407; 4096 x 1023 x 4096 = / 76 / 80 -> = / 47 / 46; 8192 x 33 x 7000, 8 shards, = / 185 / = -> = / 111 / =;
   // 1024 x 3001 x 4096 = / 45.8 (taken: 47.6) / 64 -> = / = / 50; 1250 x 9090 x 1792, 2 shards, = / 187 (taken: 199) / 160 -> = / = / 145; 2001 x 2003 x
   // 2005 = (taken: 35.9 / 42.1 / 47.1 against 32.7 / 38.5 / 44.0).
@@ -989,7 +1016,7 @@ static Packing pack_plan(const rtp_gemm_desc* d, bool vec_c) {
   const auto rounds = [&](int t) { return (double)ceil_div(ceil_div(d->m, t) * ceil_div(d->n, t) * d->groups, 256); };
   const double slow = rounds(128) * ((double)slabs * (akc && bkc ? 600.0 : akc || bkc ? 700.0 : 800.0) + 6000.0);
   double fast = rounds(128) * ((double)slabs * 480.0 + 5000.0);
-  if (vec_c && slabs >= 2) fast = std::min(fast, rounds(256) * ((double)slabs * 1650.0 + 6000.0));
+  if (vec_c && slabs >= 2) fast = std::min(fast, 1.5 * large_ns(rounds(256), (double)slabs, rare_epilogue(d)));
   const double copies = 32.0 * (double)vectors / 4500.0 + (a ? 8000.0 : 0.0) + (b ? 8000.0 : 0.0);
   if (slow - fast > 1.2 * copies) p.a = a, p.b = b;
   return p;
@@ -998,7 +1025,7 @@ static Packing pack_plan(const rtp_gemm_desc* d, bool vec_c) {
 // What one of two products would take by itself, and its arguments as a launch of 256 x 256 tiles (none: it cannot be one).
 struct PairPlan {
   GemmArgs args;
-  bool large = false;
+  bool large = false, rare = false;
   double alone = 0.0;  // ns
   double slabs = 0.0, update_bytes = 0.0, flops = 0.0, bytes = 0.0;
 };
@@ -1194,12 +1221,8 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d, PairPlan* plan = n
     const char* e = getenv("RTP_GEMM_TILE");  // debugging aid: index into kShapes
     return e ? atoi(e) : -1;
   }();
-  static const double slab_ns[kNumShapes] = {966.0, 470.0, 283.0, 167.0, 800.0, 1050.0, 545.0};
-  // Per tile outside the K loop.  256 x 256 is priced by its ratio to the others with every CU busy.  Every tile forced on 59 products
-  // x 3 layouts, operands from memory: with these two numbers the shape taken costs 0.1 % over the best one in the mean (with 1350 and
-  // 5000 ns, the price of the kernel before this one, 0.8 %), the most 12 % (4096 x 2048 x 6144, 128 tiles: 119 us with 256 x 128 against 111); it is
-  // the same for 975 - 1100 and 4000 - 5000 ns.  Where 256 x 256 is close and not taken: 4096 x 2048 x 2048, 128 tiles, 39 - 43 us against 37 - 38.
-  static const double fixed_ns[kNumShapes] = {3000.0, 3000.0, 3000.0, 3000.0, 3000.0, 4500.0, 3000.0};
+  static const double slab_ns[kNumShapes] = {966.0, 470.0, 283.0, 167.0, 800.0, kLargeSlabNs, 545.0};
+  static const double fixed_ns[kNumShapes] = {3000.0, 3000.0, 3000.0, 3000.0, 3000.0, kLargeTileNs, 3000.0};  // per tile outside the K loop
   // The two tiles for operands or outputs of any alignment, 64 x 64 and 128 x 128: the register loaders make a slab take nearly twice as
   // long and the larger tile's share outside the loop 10 us; where only the results are unaligned that is 4.  Either tile forced on 20 odd
   // shapes x 3 layouts: with these prices the one taken costs 0.1 % over the better one in the mean (with 14.5 us, the price of an
@@ -1231,23 +1254,11 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d, PairPlan* plan = n
     if (kShapes[i].bn > 64 && kShapes[i].bn > ceil_div(d->n, 64) * 64) return kNever;
     const int64_t tiles = ceil_div(m, kShapes[i].bm) * ceil_div(d->n, kShapes[i].bn) * nz;
     const double nslabs = (double)ceil_div(d->k * (int64_t)sizeof(T), slab_bytes[i]) * (double)d->ksegs;
-    // The 256 x 256 kernel finishes the rarer combinations block after block, a trip to memory each: with bias, addend and ReLU 8 of 1024 x
-    // 1280 x 520 is 41.3 us (19.2 plain) against 41.1 (25.2) with 128 x 160 tiles, x 2048 61.5 (46.3) against 67.2 (58.3).
-    const bool rare = (d->bias != nullptr) + (d->c_in != nullptr) + (d->gate != nullptr) > 1 || (relu && !d->bias) ||
-                      (d->flags & (RTP_GEMM_OUT_F32 | RTP_GEMM_CIN_F32)) || d->xent_mode;
-    const double outside = fixed_ns[i] + (i == 5 && rare ? 3000.0 : 0.0);
     const double rounds = (double)ceil_div(tiles, 256);
-    // An update moves 10 bytes a parameter (12 with the gradient) behind the K loop, a round's tiles together at the memory's 4.9 TB/s, a CU at no
-    // more than 32 bytes a ns.  So few large tiles are behind where they leave CUs idle: us with 128 x 128 / 256 x 256, K = 1024, 2048 x 2048
-    // 19.2 / 39, 8 of 1280 x 2048 97 / 101, 6144 x 2048 59.7 / 49.9, 4096 x 4096 75 / 61; 8192 x 2048 x 4096 174 / 145.
-    double update = 0.0;
-    if (d->sgd_master && vec) {
-      const double tile_bytes = (double)kShapes[i].bm * kShapes[i].bn * (8.0 + (d->sgd_weights ? 2.0 : 0.0) + (d->flags & RTP_GEMM_SGD_SKIP_OUT ? 0.0 : 2.0));
-      const auto round_ns = [&](double n) { return std::max(n * tile_bytes / 4900.0, tile_bytes / 32.0); };
-      update = (rounds - 1.0) * round_ns(256.0) + round_ns((double)tiles - 256.0 * (rounds - 1.0));
-    }
+    const double update = d->sgd_master && vec ? update_ns((double)tiles, (double)kShapes[i].bm * kShapes[i].bn * update_bytes(d)) : 0.0;
+    if (i == 5) return large_ns(rounds, nslabs, rare_epilogue(d)) + update;
     const double slab = vec || direct ? slab_ns[i] : odd_slab_ns[sizeof(T) == 4][i == 1];
-    return rounds * (nslabs * slab + (vec ? outside : odd_fixed_ns[direct][i == 1])) + update;
+    return rounds * (nslabs * slab + (vec ? fixed_ns[i] : odd_fixed_ns[direct][i == 1])) + update;
   };
   const auto cheapest = [&](int64_t m, int& shape) {
     double best = kNever;
@@ -1297,16 +1308,12 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d, PairPlan* plan = n
       return launch_gemm<T>(s, &part, nullptr, true);
     }
   }
-  if (plan && price(5, d->m) != kNever) {
-    plan->large = true;
-    plan->slabs = (double)ceil_div(d->k, 64) * (double)d->ksegs;
-    if (d->sgd_master)
-      plan->update_bytes = (double)(ceil_div(d->m, 256) * ceil_div(d->n, 256) * nz) * 65536.0 *
-                           (8.0 + (d->sgd_weights ? 2.0 : 0.0) + (d->flags & RTP_GEMM_SGD_SKIP_OUT ? 0.0 : 2.0));
-  }
   if (plan) {
-    if (!plan->large) return RTP_OK;
-    plan->alone = best, shape = 5;
+    if (price(5, d->m) == kNever) return RTP_OK;
+    plan->large = true, plan->rare = rare_epilogue(d), plan->alone = best;  // (what fits a round is not cut)
+    plan->slabs = (double)ceil_div(d->k, 64) * (double)d->ksegs;
+    plan->update_bytes = (double)(ceil_div(d->m, 256) * ceil_div(d->n, 256) * nz) * 65536.0 * update_bytes(d);
+    shape = 5;
   }
   // fp32 contractions of 384 and more go to gemm_split.hip, whose K loop is 1.2 - 1.9 times as fast and whose prologue and epilogue
   // are 1 - 2 us longer (a workgroup fills a CU there): us, fp32 MFMA -> this, forward layout: 64 matrices of 420 x 420 with
@@ -1613,6 +1620,8 @@ extern "C" int rtp_gemm_pair(void* stream, int dtype, const rtp_gemm_desc* first
   // longer contraction, one epilogue, both updates at the memory's rate.  us, one after the other -> together, attention layers of width 2048
   // (64 + 192 tiles): causal over 4096 rows, forward + backward, 512 -> 496; padded over 6000 rows 1024 -> 997; LM step of 10 blocks over 992
   // rows, Adam, 4842 -> 4679, over 1024 with the update in the epilogues 3863 -> 3729.
+  // Updates of parameters in memory, us, apart / together, tiles: 64 + 192, K = 1024 72.8 / 64.7; 49 + 147 67.3 / 58.3; 64 + 64, K = 640 38.9 / 37.2; 36 +
+  // 108, K = 640 44.1 / 41.8, 2048 67.8 / 70.0; the floor of a CU's rate that update_ns has would keep all but the first two apart.
   if (dtype == RTP_BF16 && first->m > 0 && second->m > 0 && first->n > 0 && second->n > 0 && first->k > 0 && second->k > 0) {
     hipStream_t s = (hipStream_t)stream;
     PairPlan p[2];
@@ -1623,7 +1632,8 @@ extern "C" int rtp_gemm_pair(void* stream, int dtype, const rtp_gemm_desc* first
       if (!p[i].large) break;
     }
     if (p[0].large && p[1].large && p[0].args.per_xcd + p[1].args.per_xcd <= 32) {
-      const double together = std::max(p[0].slabs, p[1].slabs) * 1050.0 + 4500.0 + (p[0].update_bytes + p[1].update_bytes) / 4900.0;
+      const double together = large_ns(1.0, std::max(p[0].slabs, p[1].slabs), p[0].rare || p[1].rare) +
+                              (p[0].update_bytes + p[1].update_bytes) / 4900.0;
       if (together < p[0].alone + p[1].alone) {
         t_warm_src = nullptr;  // 256 x 256 tiles carry no hint; it ends here
         ProfileScope prof(s, "gemm_bf16_256x256_pair_rc_rc", p[0].flops + p[1].flops, p[0].bytes + p[1].bytes);

@@ -5,14 +5,31 @@ covers some hundred fp32 additions an element."""
 import pytest
 import torch
 
-from test_gpu_gemm import DEV, TOL, _rand, rel_err
+from test_gpu_gemm import DEV, TOL, _ops, _rand, rel_err
 from test_gpu_gemm_256 import _pair, _run
 
 pytestmark = pytest.mark.gpu
 BF = torch.bfloat16
 
-# 17 x 17 and 33 x 17 tiles, ragged in both directions: no split over the XCDs; 16 x 24: bricks
-SHAPES = [(4344, 4264), (8200, 4344), (4096, 6144)]
+# 17 x 17 and 33 x 17 tiles, ragged in both directions: no split over the XCDs; 16 x 24: bricks.  The first two are cut at most contractions, and
+# their last rows go to other tiles (test_gpu_gemm_rounds.py); ONE_LAUNCH are not: 27 x 16 ragged in both directions, 33 x 15 in rows.
+ONE_LAUNCH = [(4096, 6144), (6664, 3872), (8200, 3840)]
+SHAPES = [(4344, 4264), (8200, 4344)] + ONE_LAUNCH
+
+
+def _run_alone(shape, **kw):
+    """The product; of the shapes of ONE_LAUNCH it is one kernel's, more tiles than CUs."""
+    from rtp_amd import _lib
+    _lib.profile_enable(1)
+    try:
+        got = _ops().gemm_raw(BF, **kw)
+        torch.cuda.synchronize()
+        launches = {name: s["launches"] for name, s in _lib.profile_collect().items()}
+    finally:
+        _lib.profile_enable(0)
+    if shape in ONE_LAUNCH:
+        assert list(launches.values()) == [1] and "256x256" in next(iter(launches)), launches
+    return got
 
 
 @pytest.mark.parametrize("akc,bkc", [(True, True), (True, False), (False, False), (False, True)])
@@ -23,8 +40,8 @@ def test_plain(akc, bkc, m, n, k):
     gen = torch.Generator().manual_seed(m + k)
     a, b, ref = _pair(gen, m, n, k, akc, bkc)
     out = torch.full((m, n), float("nan"), dtype=BF, device=DEV)
-    _run(a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=a.stride(0), ldb=b.stride(0), ldc=n,
-         a_kcontig=akc, b_kcontig=bkc)
+    _run_alone((m, n), a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=a.stride(0), ldb=b.stride(0), ldc=n,
+               a_kcontig=akc, b_kcontig=bkc)
     assert rel_err(out, ref) <= TOL[BF]
 
 
@@ -62,8 +79,8 @@ def test_epilogues(m, n, form):
     if form == "row sums":
         kw["rowsum"] = sums.data_ptr()
     out = torch.full((m, n), float("nan"), dtype=dt, device=DEV)
-    done = _run(a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=a.stride(0), ldb=b.stride(0), ldc=n,
-                a_kcontig=akc, b_kcontig=akc, **kw)
+    done = _run_alone((m, n), a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=a.stride(0), ldb=b.stride(0), ldc=n,
+                      a_kcontig=akc, b_kcontig=akc, **kw)
     assert rel_err(out, ref) <= (TOL[BF] if dt == BF else 1e-5)
     if form == "row sums":
         assert done and rel_err(sums, a.float().sum(0)) <= TOL[BF]
@@ -102,17 +119,18 @@ def test_groups(groups):
 def test_values_beyond_the_contraction_do_not_count():
     """What lies behind a row's last k in memory, and in the LDS from slabs before, may be anything."""
     gen = torch.Generator().manual_seed(9)
-    m, n, k, ld = 4344, 4264, 136, 192
+    m, n, k, ld = 6664, 3872, 136, 192
     a = torch.full((m, ld), float("nan"), dtype=BF, device=DEV)
     b = torch.full((n, ld), float("inf"), dtype=BF, device=DEV)
     a[:, :k] = _rand((m, k), BF, gen).to(DEV)
     b[:, :k] = _rand((n, k), BF, gen).to(DEV)
     out = torch.full((m, n), float("nan"), dtype=BF, device=DEV)
-    _run(a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=ld, ldb=ld, ldc=n, a_kcontig=True, b_kcontig=True)
+    _run_alone((m, n), a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=ld, ldb=ld, ldc=n, a_kcontig=True, b_kcontig=True)
     assert rel_err(out, a[:, :k].float() @ b[:, :k].float().t()) <= TOL[BF]
 
 
-@pytest.mark.parametrize("m,n,k", [(6144, 2048, 200), (4096, 4096, 136), (4104, 3808, 264)])
+@pytest.mark.parametrize("m,n,k", [(6144, 2048, 200), (4096, 4096, 136), (4104, 3808, 264),    # 192, 256 and 255 tiles
+                                   (4096, 6144, 520), (6664, 3872, 136), (6664, 3872, 520), (8200, 3840, 264)])  # 384, 432, 495
 @pytest.mark.parametrize("keep,clip", [(False, 0.05), (True, 0.0)])
 def test_update(m, n, k, keep, clip):
     """Clip + SGD on a tile's parameters, several tiles a workgroup, ragged ones too: bit for bit the separate update of the gradients that the
@@ -126,13 +144,13 @@ def test_update(m, n, k, keep, clip):
     old, copy = master.clone(), torch.full((m, n), float("nan"), dtype=BF, device=DEV)
     out = torch.full((m, n), float("nan"), dtype=BF, device=DEV)
     kw = dict(a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=m, ldb=n, ldc=n, a_kcontig=False, b_kcontig=False)
-    _run(sgd=Sgd(), sgd_master=master.data_ptr(), sgd_weights=copy.data_ptr(), stream_out=True, **kw)
+    _run_alone((m, n), sgd=Sgd(), sgd_master=master.data_ptr(), sgd_weights=copy.data_ptr(), stream_out=True, **kw)
     if keep:
         assert rel_err(out, ref) <= TOL[BF]
         grad = out.clone()
     else:
         assert out.isnan().all()
-        _run(**kw)
+        _run_alone((m, n), **kw)
         grad = out
     g32 = grad.float()
     if clip:

@@ -21,20 +21,31 @@ def _names(fn):
         _lib.profile_enable(0)
 
 
-@pytest.mark.parametrize("akc,bkc", [(True, True), (True, False), (False, False)])
-@pytest.mark.parametrize("m,n,k", [(4352, 4096, 520), (4360, 4104, 1032), (2312, 8192, 264), (1064, 20000, 520)])
-@pytest.mark.parametrize("form", ["plain", "bias", "addend", "fp32 addend", "mask", "fp32", "row sums", "update"])
+SHAPES = [(4352, 4096, 1544), (4360, 4104, 1032), (2312, 8192, 1032), (1032, 16384, 520)]  # 256, 520, 264 and 8 rows behind the cut
+UPDATED = [(4352, 4096, 4096), (8200, 4096, 2048), (6144, 3072, 4096)]  # an update is cut where the K loop is long enough
+FORMS = ["plain", "bias", "addend", "fp32 addend", "mask", "fp32"]
+
+
+@pytest.mark.parametrize("akc,bkc,form,m,n,k",
+                         [(True, bkc, form, *shape) for bkc in (True, False) for form in FORMS for shape in SHAPES] +
+                         [(False, False, form, *shape) for form in ("plain", "addend", "row sums", "accumulated") for shape in SHAPES] +
+                         [(False, False, "update", *shape) for shape in UPDATED])
 def test_forms(akc, bkc, m, n, k, form):
+    """Weight gradients (the last layout) with row sums, added to earlier ones and both, and with an update."""
     from rtp_amd import ops
-    if (form in ("row sums", "update")) != (not akc):
-        pytest.skip("the weight gradient's forms, and only those in its layout")
     gen = torch.Generator().manual_seed(m + k)
     a, b, ref = _pair(gen, m, n, k, akc, bkc)
     kw, dt = {}, BF
     sums = torch.full((m,), float("nan"), dtype=BF, device=DEV)
+    out = torch.full((m, n), float("nan"), dtype=torch.float32 if form == "fp32" else BF, device=DEV)
     if "addend" in form:
         c = torch.randn(m, n, generator=gen).to(torch.float32 if "fp32" in form else BF).to(DEV)
         kw, ref = dict(c_in=c.data_ptr(), ld_cin=n, cin_f32="fp32" in form), ref + c.float()
+    elif form == "accumulated":  # gradients on top of what is there, the bias's too
+        out.copy_(torch.randn(m, n, generator=gen))
+        sums.copy_(torch.randn(m, generator=gen))
+        ref, old_sums = ref + out.float(), sums.float()
+        kw = dict(c_in=out.data_ptr(), ld_cin=n, rowsum=sums.data_ptr(), rowsum_accum=True)
     elif form == "bias":
         bias = torch.randn(n, generator=gen).to(BF).to(DEV)
         kw, ref = dict(bias=bias.data_ptr()), ref + bias.float()
@@ -51,13 +62,15 @@ def test_forms(akc, bkc, m, n, k, form):
         master = torch.randn(m, n, generator=gen).to(DEV)
         old, copy = master.clone(), torch.full((m, n), float("nan"), dtype=BF, device=DEV)
         kw = dict(sgd=Sgd(), sgd_master=master.data_ptr(), sgd_weights=copy.data_ptr())
-    out = torch.full((m, n), float("nan"), dtype=dt, device=DEV)
-    ops.gemm_raw(BF, a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=a.stride(0), ldb=b.stride(0), ldc=n,
-                 a_kcontig=akc, b_kcontig=bkc, **kw)
+    names = _names(lambda: ops.gemm_raw(BF, a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=a.stride(0),
+                                        ldb=b.stride(0), ldc=n, a_kcontig=akc, b_kcontig=bkc, **kw))
+    assert len(names) == 2 and any("256x256" in name for name in names), names
     assert rel_err(out, ref) <= (TOL[BF] if dt == BF else 1e-5)
     assert not out.isnan().any()
     if form == "row sums":
         assert rel_err(sums, a.float().sum(0)) <= TOL[BF]
+    if form == "accumulated":
+        assert rel_err(sums, a.float().sum(0) + old_sums) <= TOL[BF]
     if form == "update":
         step = Sgd.lr * out.float().clamp(-Sgd.clip, Sgd.clip)
         assert torch.equal(master, old - step) and torch.equal(copy, (old - step).to(BF))

@@ -233,14 +233,14 @@ int rtp_gemm_warm_next(const void* src, size_t bytes);
 int rtp_gemm_warm_pending(void);
 
 /* Two products that do not depend on each other (the weight gradients of an attention layer): as rtp_gemm(first), rtp_gemm(second), with the
- * same results, in one launch where that is faster. */
+ * same results bit for bit, in one launch where that is faster. */
 int rtp_gemm_pair(void* stream, int dtype, const rtp_gemm_desc* first, const rtp_gemm_desc* second);
 
 /* Scratch memory for the products of the calling thread (no counterpart in the reference).  A large bf16 product on operands that are
- * not vector-aligned is faster on aligned copies of them: while `alloc` is set, rtp_gemm and rtp_rotated_linear_* ask it for
+ * not vector-aligned is faster on aligned copies of them: while `alloc` is set, rtp_gemm, rtp_gemm_pair and rtp_rotated_linear_* ask it for
  * that memory (256-byte aligned, on the current device; `context` is handed through) and use it on the product's stream
  * until the product has run.  NULL from it, or no `alloc` (the state a thread starts in): the product reads its operands where they
- * are.  No result depends on it.  At most 1 GiB a product. */
+ * are, and has the same bits.  At most 1 GiB a product. */
 typedef void* (*rtp_alloc_fn)(void* context, size_t bytes);
 int rtp_gemm_workspace(rtp_alloc_fn alloc, void* context);
 

@@ -274,7 +274,7 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs p) {
 // The body of the product kernel: workgroup `id` of the `nwg` that work on the problem `p` (`bx`, `by`: its
 // coordinates in a launch that does not use XCD bricks).  `p` lives in the kernel-argument segment.
 // REG: the loader waves go through registers (RegOperand) instead of loading straight into LDS.  RAG: the epilogue's operands
-// may be unaligned; kernels of their own, since the element-wise epilogue inside every kernel cost the others registers
+// may be unaligned; kernels of their own, since a second epilogue inside every kernel cost the others registers
 // and code (1 % of the LM attention's time).
 template <typename T, int BM, int BN, bool AKC, bool BKC, int NSTAGE, int SB, int PD, bool REG, bool RAG>
 __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned id, const unsigned bx, const unsigned by,

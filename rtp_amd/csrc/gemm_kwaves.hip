@@ -17,8 +17,8 @@ namespace rtp {
 // MT = 2: tiles of 64 x 32, slabs of 64 bytes a row and three stages, where 32 x 32 would be two workgroups a CU (fp32 256 x 2048 x 512
 // 13.1 -> 11.0 us, 100 x 3072 x 384 10.5 -> 8.2; bf16 100 x 3072 x 8192 32.6 -> 27.3, weight gradient 250 x 2048 x 4096 37.6 -> 24.5).
 // REG: operands of any alignment, through registers into the wave's LDS, three slabs ahead (bf16 255 x 1023 x 3333 24.0 -> 17.6 us,
-// 64 x 1001 x 2048 10.7 -> 7.8, its weight gradient 22.5 -> 14.4; fp32 255 x 1023 x 3333 65.6 -> 28.5, 1 x 1303 x 1364 29.4 -> 11.7); RAG: the element-wise epilogue (an output,
-// addend or mask that is not vector-aligned).
+// 64 x 1001 x 2048 10.7 -> 7.8, its weight gradient 22.5 -> 14.4; fp32 255 x 1023 x 3333 65.6 -> 28.5, 1 x 1303 x 1364 29.4 -> 11.7); RAG: the epilogue for any alignment
+// (an output, addend or mask that is not vector-aligned).
 template <typename T, int MT, bool AKC, bool BKC, bool REG, bool RAG>
 __global__ __launch_bounds__(512) void gemm_kwaves_kernel(GemmArgs p) {
   constexpr int BM = 32 * MT, SB = MT == 1 ? 128 : 64, NST = MT == 1 ? 2 : 3;  // bytes of a slab's row, stages per wave

@@ -265,7 +265,7 @@ struct SlabAt {
   }
 };
 
-// RAG: an operand is not vector-aligned (A by register loads, the element-wise epilogue).
+// RAG: an operand is not vector-aligned (A by register loads, the epilogue for any alignment).
 template <int BM, bool AKC, bool BKC, bool RAG>
 __global__ __launch_bounds__(512) void gemm_split_kernel(GemmArgs p) {
   constexpr int BN = 64, NT = BN / 32, NW = 4;              // MFMA waves

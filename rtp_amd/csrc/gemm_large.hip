@@ -421,8 +421,12 @@ __device__ __forceinline__ void large_body() {
       }
     }
   };
-  // Whole tiles, results in bf16, addend (ADD) or mask (MASK) or bias or none: 32 rows at a time go through the wave's page, so that
-  // loads and stores are whole lines (8 lanes a row, 16 bytes a lane).  An addend passes it in the other direction first.
+  // Results in bf16, addend (ADD) or mask (MASK) or bias or none: 32 rows at a time go through the wave's page, so that
+  // loads and stores are whole lines (8 lanes a row, 16 bytes a lane).  An addend passes it in the other direction first.  Lanes outside the
+  // product load its first vector and store nothing.
+  // Tiles across the product's edge too: through the general loop below, where a bias comes by scalar loads, they set the time of a launch of one
+  // round.  us, before that loop / with it / this, forward with a bias: 2766 rows, 8 groups of 384, K = 1024 34.7 / 36.6 / 28.2, 5000 x 2504 x 1000
+  // 39.2 / 40.4 / 32.7, 4104 x 3808 x 264 24.2 / 27.5 / 19.3; input gradient with an addend, 4104 x 3808 x 1024 47.5 / 44.1 / 39.3.
   auto finish = [&](const Tile& w, auto ADD, auto MASK, auto BIAS, auto RELU) {
     constexpr bool add = decltype(ADD)::value, mask = decltype(MASK)::value, bias = decltype(BIAS)::value, relu = decltype(RELU)::value;
     typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
@@ -431,18 +435,21 @@ __device__ __forceinline__ void large_body() {
     const int lane = lane_now(), li = lane & 31, g = lane >> 5;
     const bool stream_out = p->flags & RTP_GEMM_STREAM_OUT;
     const int row0 = w.m0 + wm * WM, col0 = w.n0 + wn * WN;
+    if (row0 >= rows_a || col0 >= rows_b) return;
     const int lr = lane >> 3, lc = (lane & 7) * 8;  // row (and + 8, 16, 24) and column of this lane's lines
+    const int rows = col0 + lc < rows_b ? rows_a - (row0 + lr) : 0;  // of the product from this lane's first on
     const long ldc = p->ldc, ld_in = mask ? p->ld_gate : p->ld_cin;
     T* dst = reinterpret_cast<T*>(p->c_out) + w.grp * p->c_sg + w.zo * p->c_so + w.zi * p->c_si + (row0 + lr) * ldc + col0 + lc;
     u32x4 in[MT][4];
     if constexpr (add || mask) {
-      const T* src = mask ? reinterpret_cast<const T*>(p->gate) + w.grp * p->gate_sg + w.zo * p->gate_so + w.zi * p->gate_si
-                          : reinterpret_cast<const T*>(p->c_in) + w.grp * p->cin_sg + w.zo * p->cin_so + w.zi * p->cin_si;
-      src += (row0 + lr) * ld_in + col0 + lc;
+      const T* first = mask ? reinterpret_cast<const T*>(p->gate) + w.grp * p->gate_sg + w.zo * p->gate_so + w.zi * p->gate_si
+                            : reinterpret_cast<const T*>(p->c_in) + w.grp * p->cin_sg + w.zo * p->cin_so + w.zi * p->cin_si;
+      const T* src = first + (row0 + lr) * ld_in + col0 + lc;
 #pragma unroll
       for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) in[i][s] = *reinterpret_cast<const u32x4*>(src + (i * 32 + s * 8) * ld_in);
+        for (int s = 0; s < 4; ++s)
+          in[i][s] = *reinterpret_cast<const u32x4*>(i * 32 + s * 8 < rows ? src + (i * 32 + s * 8) * ld_in : first);
     }
     float b[NT][4][4];  // of columns 32 j + 8 t + 4 g ..
     if constexpr (bias) {
@@ -514,10 +521,12 @@ __device__ __forceinline__ void large_body() {
       }
       if (stream_out) {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) __builtin_nontemporal_store(o[s], reinterpret_cast<u32x4*>(dst + s * 8 * ldc));
+        for (int s = 0; s < 4; ++s)
+          if (i * 32 + s * 8 < rows) __builtin_nontemporal_store(o[s], reinterpret_cast<u32x4*>(dst + s * 8 * ldc));
       } else {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) *reinterpret_cast<u32x4*>(dst + s * 8 * ldc) = o[s];
+        for (int s = 0; s < 4; ++s)
+          if (i * 32 + s * 8 < rows) *reinterpret_cast<u32x4*>(dst + s * 8 * ldc) = o[s];
       }
       dst += 32 * ldc;
     }
@@ -688,8 +697,8 @@ __device__ __forceinline__ void large_body() {
     const KernArgs p = kernel_args();
     const bool add = p->c_in != nullptr, mask = p->gate != nullptr, bias = p->bias != nullptr, relu = p->flags & RTP_GEMM_RELU;
     if (kUpdates && p->sgd_master != nullptr) return 6;
-    if (w.m0 + BM > rows_a || w.n0 + BN > rows_b || (int)add + (int)mask + (int)bias > 1 || (relu && !bias) || (p->flags & RTP_GEMM_OUT_F32) ||
-        (add && (p->flags & RTP_GEMM_CIN_F32)) || p->xent_mode != 0 || (bias && p->bias_sk && p->ksegs > kBiasSegs))
+    if ((int)add + (int)mask + (int)bias > 1 || (relu && !bias) || (p->flags & RTP_GEMM_OUT_F32) || (add && (p->flags & RTP_GEMM_CIN_F32)) ||
+        p->xent_mode != 0 || (bias && p->bias_sk && p->ksegs > kBiasSegs))
       return 0;
     return add ? 4 : mask ? 5 : relu ? 3 : bias ? 2 : 1;
   };
@@ -698,11 +707,11 @@ __device__ __forceinline__ void large_body() {
   auto request_bias = [&](const Tile& w) {
     const KernArgs p = kernel_args();
     const int lane = lane_now(), li = lane & 31, g = lane >> 5;
-    const T* bias = reinterpret_cast<const T*>(p->bias) + w.grp * p->bias_sg + w.zo * p->bias_so + w.zi * p->bias_si + w.n0 + wn * WN;
-    const int nb_seg = p->bias_sk ? p->ksegs : 1;
+    const T* bias = reinterpret_cast<const T*>(p->bias) + w.grp * p->bias_sg + w.zo * p->bias_so + w.zi * p->bias_si;
+    const int nb_seg = p->bias_sk ? p->ksegs : 1, col = w.n0 + wn * WN + 2 * li;
     for (int s0 = 0; s0 < nb_seg; s0 += 2) {
       const int s = s0 + g < nb_seg ? s0 + g : s0;
-      const T* src = bias + s * p->bias_sk + 2 * li;
+      const T* src = bias + s * p->bias_sk + (col < rows_b ? col : 0);
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(page + s0 * (WN * 2)), "v"(src) : "memory");
     }
   };

@@ -86,6 +86,48 @@ def test_epilogues(m, n, form):
         assert done and rel_err(sums, a.float().sum(0)) <= TOL[BF]
 
 
+@pytest.mark.parametrize("form", ["plain", "bias", "bias+relu", "addend", "mask", "stream", "in place"])
+@pytest.mark.parametrize("m,n,groups", [(6664, 3872, 1), (2766, 384, 8), (4100, 264, 6), (3000, 1000, 3)])
+def test_ragged_tiles_touch_their_own_alone(m, n, groups, form):
+    """Waves of a ragged tile that lie inside, across an edge and outside: results in the midst of NaN, addends, masks and biases too, whose
+    surroundings stay as they are and out of the sums."""
+    gen = torch.Generator().manual_seed(m + n)
+    k, gap = 200, 24
+    a = _rand((m, k), BF, gen).to(DEV)
+    b = _rand((groups, n, k), BF, gen).to(DEV)
+    ref = torch.stack([a.float() @ w.float().t() for w in b])
+
+    def field(rows, value=None):  # [groups, rows, n] whose rows, and groups, lie `gap` elements or more apart
+        whole = torch.full((groups, rows + 2, n + gap), float("nan"), dtype=BF, device=DEV)
+        if value is not None:
+            whole[:, 1:rows + 1, :n] = value
+        return whole, whole[:, 1:rows + 1, :n]
+
+    whole, out = field(m)
+    kw = {}
+    if form.startswith("bias"):
+        _, bias = field(1, _rand((groups, 1, n), BF, gen).to(DEV))
+        kw, ref = dict(bias=bias.data_ptr(), bias_sg=bias.stride(0), relu="relu" in form), ref + bias.float()
+        ref = ref.clamp(min=0) if "relu" in form else ref
+    elif form == "addend":
+        _, c = field(m, _rand((groups, m, n), BF, gen).to(DEV))
+        kw, ref = dict(c_in=c.data_ptr(), ld_cin=c.stride(1), cin_sg=c.stride(0)), ref + c.float()
+    elif form == "in place":
+        out.copy_(_rand((groups, m, n), BF, gen))
+        kw, ref = dict(c_in=out.data_ptr(), ld_cin=out.stride(1), cin_sg=out.stride(0)), ref + out.float()
+    elif form == "mask":
+        _, gate = field(m, _rand((groups, m, n), BF, gen).to(DEV))
+        kw = dict(gate=gate.data_ptr(), ld_gate=gate.stride(1), gate_sg=gate.stride(0))
+        ref = torch.where(gate.float() > 0, ref, torch.zeros_like(ref))
+    elif form == "stream":
+        kw = dict(stream_out=True)
+    _run(a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=k, ldb=k, ldc=out.stride(1), a_kcontig=True,
+         b_kcontig=True, groups=groups, b_sg=n * k, c_sg=out.stride(0), **kw)
+    assert rel_err(out, ref) <= TOL[BF] and not out.isnan().any()
+    out.fill_(float("nan"))
+    assert whole.isnan().all()
+
+
 @pytest.mark.parametrize("segs,k", [(2, 72), (3, 64), (17, 64)])
 def test_segments_and_their_biases(segs, k):
     """K segments that end inside a tile, of one slab and of two with a ragged one; a bias a segment (17: more than a wave's page holds)."""

@@ -413,8 +413,8 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
     } else {
     DA da;
     DB db;
-    da.init(p.lda, m0, p.rows_a, lw, lane);
-    db.init(p.ldb, n0, p.rows_b, lw, lane);
+    da.init(p.lda, m0, p.m, lw, lane);
+    db.init(p.ldb, n0, p.n, lw, lane);
     const char* ca = DA::slab_base(A, p.lda, m0);  // base of the next slab, uniform: scalar registers
     const char* cb = DB::slab_base(B, p.ldb, n0);
     constexpr long SZ = (long)sizeof(T);
@@ -1049,7 +1049,6 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d, PairPlan* plan = n
               (!d->gate || ok(d->gate, d->ld_gate, d->gate_so, d->gate_si, d->gate_sg)) &&
               (!d->bias || (ok(d->bias, 8, d->bias_so, d->bias_si, d->bias_sg) && mult(d->bias_sk, 8)));
   }
-  a.rows_a = (int)d->m, a.rows_b = (int)d->n;
   bool packed = false;
   rtp_gemm_desc aligned;
   if constexpr (sizeof(T) == 2) {
@@ -1057,16 +1056,15 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d, PairPlan* plan = n
       const int64_t bytes_a = p.a ? p.sa.vectors() * 16 : 0, bytes_b = p.b ? p.sb.vectors() * 16 : 0;
       if (char* at = (char*)t_alloc(t_alloc_context, (size_t)(bytes_a + bytes_b)); at != nullptr && (uintptr_t)at % 16 == 0) {
         aligned = *d, packed = true;
-        const auto move = [&](const PackShape& q, char* to, const void*& x, int64_t& ld, int64_t& sg, int64_t& sk, bool kc, int& rows) {
+        const auto move = [&](const PackShape& q, char* to, const void*& x, int64_t& ld, int64_t& sg, int64_t& sk) {
           x = to, ld = ceil_div(q.len, 8) * 8;
           if (sk != 0) sk = q.lines * ld;
           if (sg != 0) sg = q.segs * q.lines * ld;
-          if (!kc) rows = (int)ld;
           return launch_pack(s, q, to);
         };
         int rc = RTP_OK;
-        if (p.a) rc = move(p.sa, at, aligned.a, aligned.lda, aligned.a_sg, aligned.a_sk, d->a_kcontig, a.rows_a);
-        if (p.b && rc == RTP_OK) rc = move(p.sb, at + bytes_a, aligned.b, aligned.ldb, aligned.b_sg, aligned.b_sk, d->b_kcontig, a.rows_b);
+        if (p.a) rc = move(p.sa, at, aligned.a, aligned.lda, aligned.a_sg, aligned.a_sk);
+        if (p.b && rc == RTP_OK) rc = move(p.sb, at + bytes_a, aligned.b, aligned.ldb, aligned.b_sg, aligned.b_sk);
         if (rc != RTP_OK) return rc;
         d = &aligned;
       }

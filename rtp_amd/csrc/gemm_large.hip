@@ -222,11 +222,11 @@ __device__ __forceinline__ void large_body() {
   DB db[2];
   auto init_a = [&](const Tile& w) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) da[h].init(lda, w.m0, kernel_args()->rows_a, wave, lane_now(), [=](int r) { return half_row<BLKA>(r, h); });
+    for (int h = 0; h < 2; ++h) da[h].init(lda, w.m0, kernel_args()->m, wave, lane_now(), [=](int r) { return half_row<BLKA>(r, h); });
   };
   auto init_b = [&](const Tile& w) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) db[h].init(ldb, w.n0, kernel_args()->rows_b, wave, lane_now(), [=](int r) { return half_row<BLKB>(r, h); });
+    for (int h = 0; h < 2; ++h) db[h].init(ldb, w.n0, kernel_args()->n, wave, lane_now(), [=](int r) { return half_row<BLKB>(r, h); });
   };
   init_a(here);
   init_b(here);

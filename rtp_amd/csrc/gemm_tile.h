@@ -38,7 +38,6 @@ struct GemmArgs {
   FastDiv d_batch, d_zdiv, d_tiles_n, d_brick, d_panel, d_prow, d_pm;  // divisors mbk*nbk, prow*pcol, prow, mbk/prow
   int mbk, nbk, prow, pcol;
   int xn_shift, xm_shift, zbk;  // log2 of xn and xm, batch*groups entries per brick
-  unsigned tiles, per_xcd;      // all tiles of the launch, an XCD's share of them (rounded up)
   unsigned long long* trace;    // null, or two words: earliest start / latest end of the launch on the wall clock
   float* sgd_master;            // null, or the fp32 parameters the product updates (indexed like c_out)
   char* sgd_w;                  // null, or the compute-dtype copy of the parameters
@@ -57,7 +56,7 @@ struct GemmArgs {
   // bytes that some later launch will read from HBM (the next layer's shards): requested here, see warm_ahead()
   const char* warm;
   long warm_bytes;
-  int rows_a, rows_b;  // m and n as the direct-to-LDS loaders see them: to whole vectors where an operand's lines are padded to those
+  unsigned tiles, per_xcd;  // gemm_large.hip: all tiles of the launch, an XCD's share of them (rounded up)
 };
 
 // The per-lane MFMA operand: VEC consecutive k values of one tile row.
@@ -690,7 +689,7 @@ struct DmaOperand {
         const int kl = j * (1024 / LINE) + byte / LINE;
         const int chunk = ((byte % LINE) >> 4) ^ rc_swizzle<T, R>(kl);  // which 16 bytes of the k line land here
         int src = row_of(chunk * VEC);
-        if (row0 + src + VEC > rows) src = 0;  // past the end: re-read the tile's first rows
+        if (row0 + src >= rows) src = 0;  // past the end: re-read the tile's first rows (a k line that is no whole number of vectors is padded)
         ofs[i] = (unsigned)((long)kl * ld * (long)sizeof(T)) + (unsigned)(src * (int)sizeof(T));
         koff[i] = kl;
       }

@@ -383,7 +383,8 @@ __device__ __forceinline__ void finish_tile(const GemmArgs& p, const float* ct, 
   }
 }
 
-// Up to eight consecutive values at any alignment, as fp32; those from `n` on, which may lie outside the operand, are left out.
+// Up to eight consecutive values at any alignment, as fp32; those from `n` (at least 1) on, which may lie outside the operand, are left out:
+// the last one is read in their place, so that the loads are without branches and wait together.
 template <typename S>
 __device__ __forceinline__ void load8_any(const S* src, int n, float (&v)[8]) {
   constexpr int VEC = 16 / (int)sizeof(S);
@@ -397,7 +398,7 @@ __device__ __forceinline__ void load8_any(const S* src, int n, float (&v)[8]) {
     }
   } else {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = e < n ? to_f32(src[e]) : 0.0f;
+    for (int e = 0; e < 8; ++e) v[e] = to_f32(src[min(e, n - 1)]);
   }
 }
 template <typename S>
@@ -463,7 +464,9 @@ __device__ __forceinline__ void finish_tile_ragged(const GemmArgs& p, const floa
   }
 #pragma unroll
   for (int e = 0; e < 8; ++e) bv[e] = 0.0f;
-  if (bias)
+  if (bias && nb_seg == 1)
+    load8_any(bias + col, live, bv);
+  else if (bias)
     for (int s0 = 0; s0 < nb_seg; s0 += 4) {  // four segments' at a time, added in their order
       float bt[4][8];
 #pragma unroll

@@ -1230,13 +1230,16 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d, PairPlan* plan = n
   static const int slab_bytes[kNumShapes] = {128, 128, 128, 128, 128, 128, 128};
   const bool vec = direct && a.vec_c;  // else the kernels for operands of any alignment
   constexpr double kNever = 1e300;
+  const bool whole_lines = mult((int64_t)(uintptr_t)d->sgd_master, 128) && mult(d->ldc, 32) && (d->groups == 1 || mult(d->c_sg, 32)) &&
+                           (d->batch == 1 || (mult(d->c_so, 32) && mult(d->c_si, 32)));
   // ns of the first `m` rows in tiles of shape i
   const auto price = [&](int i, int64_t m) {
     // the 256 x 256 kernel is built for 16-bit operands and has no statistics epilogue (never routed to it, forced or not)
     if (i == 5 && (sizeof(T) != 2 || d->xent_mode == 1)) return kNever;
-    // ... and an update only where it is a weight gradient's and the parameters' rows are whole 128-byte lines: its waves write 64
-    // columns each, and on rows that are not (3000 x 3000 x 512) it takes 49 us where 128 x 128 takes 38
-    if (i == 5 && d->sgd_master && (akc || bkc || d->ldc % 32 != 0)) return kNever;
+    // ... and an update only where it is a weight gradient's and the parameters' rows are whole 128-byte lines in every group: its waves write
+    // 64 columns each.  us, 128 x 128 or 256 x 128 tiles / these, parameters from memory: rows that are not, 3000 x 3000 x 512, 38 / 49; 8 groups of 1024 x
+    // 2048 x 1024 that lie 32, 64 and 128 bytes beyond a line apart 69.9 / 95.8, 69.3 / 78.0 and 68.9 / 64.9; 2 of 6144 x 2048 118.9 / 133.9, 108.9 / 115.7, 105.0 / 102.6
+    if (i == 5 && d->sgd_master && (akc || bkc || !whole_lines)) return kNever;
     if (i == 6 && d->xent_mode == 1) return kNever;  // 160 columns are no whole number of 64-column statistics blocks
     if (!vec && i != 1 && i != 3) return kNever;  // the kernels for unaligned operands: 128 x 128 and 64 x 64
     // 128 x 160 is priced at the rate measured where it is meant for -- products of at most two rounds of tiles, such

@@ -926,7 +926,7 @@ struct RegOperand {
 int launch_split(hipStream_t s, const GemmArgs& a, bool akc, bool bkc, int bm, bool ragged, dim3 grid);
 
 // bf16 products in tiles of 256 x 256 by workgroups that stay (gemm_large.hip): vector-aligned operands and results, two K slabs or more, no
-// statistics epilogue; an update only with both operands row-contiguous and ldc a multiple of 32.
+// statistics epilogue; an update with both operands row-contiguous alone, and worth it only on parameters whose rows are whole 128-byte lines.
 int launch_large(hipStream_t s, const GemmArgs& a, bool akc, bool bkc);
 // Two weight gradients at once, a tile a workgroup: per_xcd of both together at most 32.
 int launch_large_pair(hipStream_t s, const GemmArgs& a, const GemmArgs& b);

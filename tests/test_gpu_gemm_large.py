@@ -200,3 +200,33 @@ def test_update(m, n, k, keep, clip):
     step = Sgd.lr * g32
     assert torch.equal(master, old - step)
     assert torch.equal(copy, (old - step).to(BF))
+
+
+@pytest.mark.parametrize("shift,gap,large", [(0, 32, True), (0, 8, False), (8, 32, False)])
+def test_updates_of_parameters_that_are_no_whole_lines_go_elsewhere(shift, gap, large):
+    """Groups of parameters at a multiple of 128 bytes or not: the tiles differ, the results do not."""
+    from rtp_amd import _lib
+
+    class Sgd:
+        lr, clip, keep_grads, missed = 1e-3, 0.05, True, False
+
+    gen = torch.Generator().manual_seed(shift + gap)
+    m, n, k, groups = 1024, 2048, 264, 8
+    a, b = _rand((k, groups * m), BF, gen).to(DEV), _rand((k, n), BF, gen).to(DEV)
+    step = m * n + gap
+    master = _rand((shift + groups * step,), torch.float32, gen).to(DEV)[shift:].view(groups, step)
+    old, copy, out = master.clone(), *(torch.full((shift + groups * step,), float("nan"), dtype=BF, device=DEV)[shift:].view(groups, step) for _ in range(2))
+    _lib.profile_enable(1)
+    try:
+        _ops().gemm_raw(BF, a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=groups * m, ldb=n, ldc=n, a_kcontig=False,
+                        b_kcontig=False, groups=groups, a_sg=m, c_sg=step, sgd=Sgd(), sgd_master=master.data_ptr(), sgd_weights=copy.data_ptr())
+        torch.cuda.synchronize()
+        names = list(_lib.profile_collect())
+    finally:
+        _lib.profile_enable(0)
+    assert any("256x256" in name for name in names) == large, names
+    grad, rest = out[:, :m * n], slice(m * n, None)
+    assert rel_err(grad.reshape(groups, m, n), torch.stack([a[:, g * m:g * m + m].float().t() @ b.float() for g in range(groups)])) <= TOL[BF]
+    new = old[:, :m * n] - Sgd.lr * grad.float().clamp(-Sgd.clip, Sgd.clip)
+    assert torch.equal(master[:, :m * n], new) and torch.equal(copy[:, :m * n], new.to(BF))
+    assert torch.equal(master[:, rest], old[:, rest]) and copy[:, rest].isnan().all() and out[:, rest].isnan().all()

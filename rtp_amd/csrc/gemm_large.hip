@@ -204,16 +204,15 @@ __device__ __forceinline__ void large_body() {
   const int nk = nk_seg * args->ksegs;
 
   f32x16 acc[MT][NT];
-  float rsum[MT];
+  float rsum = 0.0f;
   auto clear = [&] {
+    rsum = 0.0f;
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      rsum[i] = 0.0f;
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
       for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-    }
   };
 
   // ---- this wave's share of the loads, which run ahead of the products and into the next tile ----
@@ -304,7 +303,12 @@ __device__ __forceinline__ void large_body() {
   FragPlace<BKC, 1> pb;
   pa.init(lds0, wm * BLKA, lane);
   pb.init(lds0 + 2 * HALF, wn * BLKB, lane);
-  bool rowsum = false;
+  // The block of 32 rows whose sums of A this wave adds up beside the products, or -1.  The additions are one chain behind the MFMAs of a phase, and
+  // the waves go in step: a phase with sums is 250 clocks longer for the tile.  So the four blocks of a wave tile's rows go to the first four tile
+  // columns, a wave each (with two or three columns two in the same phase), instead of all to the first.  us without sums / all in the first /
+  // so: 8 of 8192 x 2048 x 1024 242 / 257 / 245, 2 of 3888 x 3112 x 5139 245 / 264 / 247, 6144 x 2048 x 4096 92 / 98 / 92, 4096^3 108 / 116 / 110.
+  // (In the read halves of the phases behind: 239 / - / 262, 246 / - / 263, 92 / - / 98, 108 / - / 114.)
+  int sum_block = -1;
   auto read_a = [&](auto H) {
 #pragma unroll
     for (int q = 0; q < KS; ++q)
@@ -315,6 +319,17 @@ __device__ __forceinline__ void large_body() {
 #pragma unroll
     for (int q = 0; q < KS; ++q) fb[q] = pb.read(decltype(H)::value * HALF, 0, q);
   };
+  auto row_sums = [&](auto H) {
+    if (!AKC && sum_block >> 1 == decltype(H)::value) {
+      if (sum_block & 1) {
+#pragma unroll
+        for (int q = 0; q < KS; ++q) rsum = frag_sum(fa[1][q], rsum);
+      } else {
+#pragma unroll
+        for (int q = 0; q < KS; ++q) rsum = frag_sum(fa[0][q], rsum);
+      }
+    }
+  };
   auto barrier = [] {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -322,7 +337,7 @@ __device__ __forceinline__ void large_body() {
   };
   // the barrier that ends a read half, the MFMA half and its end, where this wave's reads have returned (the first MFMAs
   // wait only for their own fragments)
-  auto multiply = [&](auto H, auto J, const Frag<T>(&fb)[KS], bool sums) {
+  auto multiply = [&](auto H, auto J, const Frag<T>(&fb)[KS], auto SUMS) {
     constexpr int h = decltype(H)::value, j = decltype(J)::value;
     __builtin_amdgcn_sched_barrier(0);
     barrier();
@@ -332,12 +347,7 @@ __device__ __forceinline__ void large_body() {
 #pragma unroll
       for (int i = 0; i < 2; ++i) mma(fb[q], fa[i][q], acc[h * 2 + i][j]);  // transposed: a lane holds columns of one row
     __builtin_amdgcn_s_setprio(0);
-    if (!AKC && sums && rowsum) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int q = 0; q < KS; ++q) rsum[h * 2 + i] = frag_sum(fa[i][q], rsum[h * 2 + i]);
-    }
+    if constexpr (decltype(SUMS)::value) row_sums(H);
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     barrier();
@@ -358,7 +368,7 @@ __device__ __forceinline__ void large_body() {
     if constexpr (rest >= 1) issue_a(other, I1{});
     if constexpr (rest >= 1) landed();
     else RTP_WAIT_VM(NI);
-    multiply(I0{}, I0{}, fb0, true);
+    multiply(I0{}, I0{}, fb0, std::true_type{});
 
     read_b(I1{}, fb1);
     if constexpr (rest >= 2) step();
@@ -367,20 +377,20 @@ __device__ __forceinline__ void large_body() {
     if constexpr (rest >= 2) landed();
     else if constexpr (rest == 1) RTP_WAIT_VM(4 * NI);
     else RTP_WAIT_VM(0);
-    multiply(I0{}, I1{}, fb1, false);
+    multiply(I0{}, I1{}, fb1, std::false_type{});
 
     read_a(I1{});
     if constexpr (rest >= 2) issue_a(cur, I0{});
     if constexpr (rest >= 2) landed();
     else if constexpr (rest == 1) RTP_WAIT_VM(3 * NI);
-    multiply(I1{}, I1{}, fb1, true);
+    multiply(I1{}, I1{}, fb1, std::true_type{});
 
     if constexpr (rest >= 1) read_b(I0{}, fb0n);
     if constexpr (rest >= 2) issue_b(cur, I1{});
     pa.other_slab(SLAB);
     if constexpr (rest >= 2) landed();
     else if constexpr (rest == 1) RTP_WAIT_VM(2 * NI);
-    multiply(I1{}, I0{}, fb0, false);
+    multiply(I1{}, I0{}, fb0, std::false_type{});
     if constexpr (rest >= 1) {
 #pragma unroll
       for (int q = 0; q < KS; ++q) fb0[q] = fb0n[q];
@@ -719,15 +729,12 @@ __device__ __forceinline__ void large_body() {
     const KernArgs p = kernel_args();
     using Yes = std::true_type;
     using No = std::false_type;
-    if (!AKC && rowsum) {
+    if (!AKC && sum_block >= 0) {
       const int lane = lane_now(), li = lane & 31, g = lane >> 5;
       T* dst = reinterpret_cast<T*>(p->a_rowsum) + w.grp * p->rowsum_sg;
-#pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const float v = rsum[i] + __shfl_xor(rsum[i], 32, 64);
-        const int row = w.m0 + wm * WM + i * 32 + li;
-        if (g == 0 && row < rows_a) dst[row] = from_f32<T>((p->flags & RTP_GEMM_ROWSUM_ACCUM) ? to_f32(dst[row]) + v : v);
-      }
+      const float v = rsum + __shfl_xor(rsum, 32, 64);
+      const int row = w.m0 + wm * WM + sum_block * 32 + li;
+      if (g == 0 && row < rows_a) dst[row] = from_f32<T>((p->flags & RTP_GEMM_ROWSUM_ACCUM) ? to_f32(dst[row]) + v : v);
     }
     if (p->alpha != 1.0f) {
 #pragma unroll
@@ -777,7 +784,10 @@ __device__ __forceinline__ void large_body() {
     if (more) next = tile_at(slot);
     const int form = finish_form(here);
     if (form == 2 || form == 3) request_bias(here);
-    rowsum = !AKC && kernel_args()->a_rowsum != nullptr && here.n0 == 0 && wn == 0;
+    if (!AKC) {
+      const int part = rows_b > 3 * BN ? wn : rows_b > BN ? wn >> 1 : 0;  // the tile column that has block wn's sums
+      sum_block = kernel_args()->a_rowsum != nullptr && here.n0 == part * BN ? wn : -1;
+    }
     if (wm == 1) __builtin_amdgcn_s_barrier();
     for (int todo = more ? nk : nk - 2; todo > 0; --todo) slab(std::integral_constant<int, 2>{});
     if (!more) {

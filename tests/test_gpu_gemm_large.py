@@ -171,6 +171,26 @@ def test_values_beyond_the_contraction_do_not_count():
     assert rel_err(out, a[:, :k].float() @ b[:, :k].float().t()) <= TOL[BF]
 
 
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("n,groups", [(248, 8), (256, 12), (456, 8), (512, 8), (520, 8), (768, 6), (776, 6), (1032, 4), (4104, 1)])
+def test_row_sums_over_the_tile_columns(n, groups, accumulate):
+    """One to four tile columns and more, which share the sums of a tile's rows among them: the bits of the smaller tiles, each row once."""
+    gen = torch.Generator().manual_seed(n)
+    m, k = 4104, 264
+    a, b = _rand((k, groups * m), BF, gen).to(DEV), _rand((k, n), BF, gen).to(DEV)
+    old = _rand((groups, m), BF, gen).to(DEV) if accumulate else torch.full((groups, m), float("nan"), dtype=BF, device=DEV)
+    results = []
+    for cols, run in ((n, _run), (64, _ops().gemm_raw)):
+        sums = old.clone()
+        out = torch.full((groups, m, cols), float("nan"), dtype=BF, device=DEV)
+        kw = dict(a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=cols, k=k, lda=groups * m, ldb=n, ldc=cols, a_kcontig=False,
+                  b_kcontig=False, groups=groups, a_sg=m, c_sg=m * cols, rowsum=sums.data_ptr(), rowsum_sg=m, rowsum_accum=accumulate)
+        assert run(**kw) if run is _run else run(BF, **kw)
+        results.append(sums)
+    ref = a.float().sum(0).view(groups, m) + (old.float() if accumulate else 0)
+    assert rel_err(results[0], ref) <= TOL[BF] and torch.equal(*results)
+
+
 @pytest.mark.parametrize("m,n,k", [(6144, 2048, 200), (4096, 4096, 136), (4104, 3808, 264),    # 192, 256 and 255 tiles
                                    (4096, 6144, 520), (6664, 3872, 136), (6664, 3872, 520), (8200, 3840, 264)])  # 384, 432, 495
 @pytest.mark.parametrize("keep,clip", [(False, 0.05), (True, 0.0)])

@@ -437,17 +437,20 @@ __device__ __forceinline__ void large_body() {
   // Tiles across the product's edge too: through the general loop below, where a bias comes by scalar loads, they set the time of a launch of one
   // round.  us, before that loop / with it / this, forward with a bias: 2766 rows, 8 groups of 384, K = 1024 34.7 / 36.6 / 28.2, 5000 x 2504 x 1000
   // 39.2 / 40.4 / 32.7, 4104 x 3808 x 264 24.2 / 27.5 / 19.3; input gradient with an addend, 4104 x 3808 x 1024 47.5 / 44.1 / 39.3.
-  auto finish = [&](const Tile& w, auto ADD, auto MASK, auto BIAS, auto RELU) {
+  // (EDGE: the product's edge crosses the tile.  A code of its own: the choice of a place for each load costs whole tiles 4096 x 6144 x 512 with an
+  // addend 38.4 -> 40.5 us, the conditions on the stores 8192 x 4096 x 1024 62.9 -> 63.8.)
+  auto finish = [&](const Tile& w, auto ADD, auto MASK, auto BIAS, auto RELU, auto EDGE) {
     constexpr bool add = decltype(ADD)::value, mask = decltype(MASK)::value, bias = decltype(BIAS)::value, relu = decltype(RELU)::value;
+    constexpr bool edge = decltype(EDGE)::value;
     typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
     typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
     const KernArgs p = kernel_args();
     const int lane = lane_now(), li = lane & 31, g = lane >> 5;
     const bool stream_out = p->flags & RTP_GEMM_STREAM_OUT;
     const int row0 = w.m0 + wm * WM, col0 = w.n0 + wn * WN;
-    if (row0 >= rows_a || col0 >= rows_b) return;
+    if (edge && (row0 >= rows_a || col0 >= rows_b)) return;
     const int lr = lane >> 3, lc = (lane & 7) * 8;  // row (and + 8, 16, 24) and column of this lane's lines
-    const int rows = col0 + lc < rows_b ? rows_a - (row0 + lr) : 0;  // of the product from this lane's first on
+    const int rows = !edge ? WM : col0 + lc < rows_b ? rows_a - (row0 + lr) : 0;  // of the product from this lane's first on
     const long ldc = p->ldc, ld_in = mask ? p->ld_gate : p->ld_cin;
     T* dst = reinterpret_cast<T*>(p->c_out) + w.grp * p->c_sg + w.zo * p->c_so + w.zi * p->c_si + (row0 + lr) * ldc + col0 + lc;
     u32x4 in[MT][4];
@@ -459,7 +462,7 @@ __device__ __forceinline__ void large_body() {
       for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int s = 0; s < 4; ++s)
-          in[i][s] = *reinterpret_cast<const u32x4*>(i * 32 + s * 8 < rows ? src + (i * 32 + s * 8) * ld_in : first);
+          in[i][s] = *reinterpret_cast<const u32x4*>(!edge || i * 32 + s * 8 < rows ? src + (i * 32 + s * 8) * ld_in : first);
     }
     float b[NT][4][4];  // of columns 32 j + 8 t + 4 g ..
     if constexpr (bias) {
@@ -725,6 +728,20 @@ __device__ __forceinline__ void large_body() {
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(page + s0 * (WN * 2)), "v"(src) : "memory");
     }
   };
+  auto finish_lines = [&](const Tile& w, int form, auto EDGE) {
+    using Yes = std::true_type;
+    using No = std::false_type;
+    if (form == 1)
+      finish(w, No{}, No{}, No{}, No{}, EDGE);
+    else if (form == 2)
+      finish(w, No{}, No{}, Yes{}, No{}, EDGE);
+    else if (form == 3)
+      finish(w, No{}, No{}, Yes{}, Yes{}, EDGE);
+    else if (form == 4)
+      finish(w, Yes{}, No{}, No{}, No{}, EDGE);
+    else
+      finish(w, No{}, Yes{}, No{}, No{}, EDGE);
+  };
   auto epilogue = [&](const Tile& w, int form) {
     const KernArgs p = kernel_args();
     using Yes = std::true_type;
@@ -749,16 +766,10 @@ __device__ __forceinline__ void large_body() {
       finish_any(w, whole);
     else if (kUpdates && form == 6)
       finish_update(w, whole);
-    else if (form == 1)
-      finish(w, No{}, No{}, No{}, No{});
-    else if (form == 2)
-      finish(w, No{}, No{}, Yes{}, No{});
-    else if (form == 3)
-      finish(w, No{}, No{}, Yes{}, Yes{});
-    else if (form == 4)
-      finish(w, Yes{}, No{}, No{}, No{});
+    else if (whole)
+      finish_lines(w, form, No{});
     else
-      finish(w, No{}, Yes{}, No{}, No{});
+      finish_lines(w, form, Yes{});
   };
 
   // what phases before the first would have issued, in their order; the host sends no problem of a single slab here

@@ -437,8 +437,10 @@ __device__ __forceinline__ void large_body() {
   // Tiles across the product's edge too: through the general loop below, where a bias comes by scalar loads, they set the time of a launch of one
   // round.  us, before that loop / with it / this, forward with a bias: 2766 rows, 8 groups of 384, K = 1024 34.7 / 36.6 / 28.2, 5000 x 2504 x 1000
   // 39.2 / 40.4 / 32.7, 4104 x 3808 x 264 24.2 / 27.5 / 19.3; input gradient with an addend, 4104 x 3808 x 1024 47.5 / 44.1 / 39.3.
-  // (EDGE: the product's edge crosses the tile.  A code of its own: the choice of a place for each load costs whole tiles 4096 x 6144 x 512 with an
-  // addend 38.4 -> 40.5 us, the conditions on the stores 8192 x 4096 x 1024 62.9 -> 63.8.)
+  // EDGE: the product's edge may cross the tile.  Whole tiles have code of their own: the choice of a place for each load costs 4096 x 6144 x 512 with
+  // an addend 38.4 -> 40.5 us, the conditions on the stores cost forward products 1 - 2 % (8192 x 4096 x 1024 57.8 -> 58.9).  Weight
+  // gradients without an addend keep the conditions, and with them the stores where they stand: 8 of 8192 x 2048 x 1024 with row sums, eight tiles a
+  // workgroup, 287 us without and 278 with them.
   auto finish = [&](const Tile& w, auto ADD, auto MASK, auto BIAS, auto RELU, auto EDGE) {
     constexpr bool add = decltype(ADD)::value, mask = decltype(MASK)::value, bias = decltype(BIAS)::value, relu = decltype(RELU)::value;
     constexpr bool edge = decltype(EDGE)::value;
@@ -731,11 +733,12 @@ __device__ __forceinline__ void large_body() {
   auto finish_lines = [&](const Tile& w, int form, auto EDGE) {
     using Yes = std::true_type;
     using No = std::false_type;
-    if (form == 1)
+    constexpr bool all = AKC || decltype(EDGE)::value;  // (see finish: a weight gradient's whole tiles come here without EDGE for forms 4 and 5 alone)
+    if (all && form == 1)
       finish(w, No{}, No{}, No{}, No{}, EDGE);
-    else if (form == 2)
+    else if (all && form == 2)
       finish(w, No{}, No{}, Yes{}, No{}, EDGE);
-    else if (form == 3)
+    else if (all && form == 3)
       finish(w, No{}, No{}, Yes{}, Yes{}, EDGE);
     else if (form == 4)
       finish(w, Yes{}, No{}, No{}, No{}, EDGE);
@@ -766,7 +769,7 @@ __device__ __forceinline__ void large_body() {
       finish_any(w, whole);
     else if (kUpdates && form == 6)
       finish_update(w, whole);
-    else if (whole)
+    else if (whole && (AKC || form >= 4))
       finish_lines(w, form, No{});
     else
       finish_lines(w, form, Yes{});

@@ -612,16 +612,16 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
 }
 
 template <typename T, int BM, int BN, bool AKC, bool BKC, int NSTAGE, int SB, int PD>
-__global__ __launch_bounds__(512) void gemm_dma_kernel(GemmArgs p) {
-  touch_kernel_arguments<sizeof(GemmArgs)>();
+__global__ __launch_bounds__(512) void gemm_dma_kernel(GemmArgs) {
+  const GemmArgs& p = fetched_arguments<GemmArgs>();
   gemm_dma_body<T, BM, BN, AKC, BKC, NSTAGE, SB, PD, false, false>(p, blockIdx.x + blockIdx.y * gridDim.x, blockIdx.x,
                                                             blockIdx.y, gridDim.x * gridDim.y);
 }
 
 // Operands of any alignment; REG where that includes A or B.
 template <typename T, int BM, int BN, bool AKC, bool BKC, int NSTAGE, int SB, int PD, bool REG>
-__global__ __launch_bounds__(512) void gemm_unaligned_kernel(GemmArgs p) {
-  touch_kernel_arguments<sizeof(GemmArgs)>();
+__global__ __launch_bounds__(512) void gemm_unaligned_kernel(GemmArgs) {
+  const GemmArgs& p = fetched_arguments<GemmArgs>();
   gemm_dma_body<T, BM, BN, AKC, BKC, NSTAGE, SB, PD, REG, true>(p, blockIdx.x + blockIdx.y * gridDim.x, blockIdx.x, blockIdx.y,
                                                           gridDim.x * gridDim.y);
 }

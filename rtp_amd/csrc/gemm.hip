@@ -348,9 +348,13 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-  float rsum[MT];
+  // (bf16: even and odd k-steps apart, which is the order in which the 256 x 256 kernel's fragments add up)
+  constexpr int NSUM = sizeof(T) == 2 && !AKC ? 2 : 1;
+  float rsum[MT][NSUM];
 #pragma unroll
-  for (int i = 0; i < MT; ++i) rsum[i] = 0.0f;
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int c = 0; c < NSUM; ++c) rsum[i][c] = 0.0f;
 
   // Barrier protocol: both paths meet the same nk barriers.  Barrier k is passed when slab k is visible to
   // every wave: a loader reaches it only after its own loads of slab k have landed.  A compute wave reaches
@@ -488,15 +492,15 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
 #pragma unroll
       for (int j = 0; j < NT; ++j) fb[set][j] = read_frag_dma<T, BN, BKC, SB>(sb, wn * WN + j * 32, lane, q);
     };
-    auto mma_step = [&](auto SET) {
-      constexpr int set = decltype(SET)::value;
+    auto mma_step = [&](auto SET, auto Q) {
+      constexpr int set = decltype(SET)::value, c = decltype(Q)::value % NSUM;
 #pragma unroll
       for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) mma(fa[set][i], fb[set][j], acc[i][j]);
       if (rowsum) {
 #pragma unroll
-        for (int i = 0; i < MT; ++i) rsum[i] = frag_sum(fa[set][i], rsum[i]);
+        for (int i = 0; i < MT; ++i) rsum[i][c] = frag_sum(fa[set][i], rsum[i][c]);
       }
     };
     // k-step Q of slab k (stage S).  The scheduling fences keep the order written here: left alone, the compiler
@@ -515,7 +519,7 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
         read_step(std::integral_constant<int, (s + ds) % NSTAGE>{}, std::integral_constant<int, tq>{},
                   std::integral_constant<int, (t + PD) % NSET>{});
       }
-      mma_step(std::integral_constant<int, t % NSET>{});
+      mma_step(std::integral_constant<int, t % NSET>{}, Q);
       // Issue order inside the step: one MFMA, then its share of the step's LDS reads, and so on.  A wave issues in
       // order and an MFMA holds the issue port until the matrix pipe takes it, so only what sits between two
       // MFMAs is issued in an MFMA's shadow; reads bunched up before the first MFMA would leave the pipe idle.
@@ -563,7 +567,8 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
     T* dst = reinterpret_cast<T*>(p.a_rowsum) + grp * p.rowsum_sg;
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
-      const float v = rsum[i] + __shfl_xor(rsum[i], 32, 64);
+      float v = rsum[i][0] + __shfl_xor(rsum[i][0], 32, 64);
+      if constexpr (NSUM == 2) v += rsum[i][1] + __shfl_xor(rsum[i][1], 32, 64);
       const int row = m0 + wm * WM + i * 32 + li;
       if (g == 0 && row < p.m) dst[row] = from_f32<T>((p.flags & RTP_GEMM_ROWSUM_ACCUM) ? to_f32(dst[row]) + v : v);
     }

@@ -9,11 +9,11 @@ namespace rtp {
 // the direct-to-LDS loads themselves.
 //
 // A SIMD holds two of the waves, and their work alternates: a K slab (128 bytes of k per row) is four phases, a phase is a
-// read half -- fragments of half an operand into registers, two load instructions -- and an MFMA half of eight MFMAs,
+// read half -- fragments of half an operand into registers, two load instructions -- and an MFMA half of sixteen MFMAs,
 // each closed by a workgroup barrier.  The waves of the lower tile half (wm = 1, the second wave of every SIMD) pass one
 // barrier more at the start of a tile, so they read while the others multiply and the other way round: LDS reads, loads and scalar
 // work of one wave lie under the MFMAs of the other, and neither waits for its own.  That holds as long as a read half takes no
-// longer than eight MFMAs (256 clocks): it is some 25 instructions, addresses in registers and offsets in the instructions, and its
+// longer than sixteen MFMAs (256 clocks): it is some 25 instructions, addresses in registers and offsets in the instructions, and its
 // rare events are branches that are not taken.
 //
 // An operand's slab is two half tiles of 128 rows (16 KiB each, stored like a 128-row operand), and a wave tile takes half of
@@ -29,6 +29,13 @@ namespace rtp {
 // landed (the ten youngest may be on their way); the next phase's reads lie two barriers behind, so that holds for every
 // wave's share.
 //
+// On random operands the matrix pipes' power sets the clock, and 16 x 16 x 32 is the cheaper MFMA: for the same flops it reads and writes its
+// accumulators half as often as 32 x 32 x 16, and least where the second k-step of an output follows its first directly (a loop of MFMAs
+// in registers, two waves a SIMD, random operands, TF/s: 32 x 32 x 16 1600 in any order; 16 x 16 x 32 with the k-steps apart 1800, back to back
+// 1850; zeros 2210 / 2150 / 2195).  The results have the same bits.  us, 32 x 32 x 16 -> this, forward / input gradient / weight gradient layout:
+// 8 of 1024 x 8192 x 2048 228 / 233 / 246 -> 214 / 220 / 235, 4096^3 103.5 / 108.5 / 112.5 -> 97.5 / 102 / 109.5, 4096 x 6144 x 2048 93 / - / - -> 87,
+// 8192^3 773 / - / - -> 729; half a round of tiles, where the clock is free, 4096 x 2048 x 2048 39.1 / 38.8 / - -> 40.0 / 39.0.
+//
 // A workgroup stays on its CU and goes through its tiles (the tile number advances by the number of workgroups), and the loads run on
 // into the next tile: when a tile's last MFMAs are done, the first slab and a half of the next are in the LDS or on their way, and the
 // epilogue touches neither.  It brings 32 rows of a wave tile at a time through 4 KiB of the wave's own, without a barrier.  The
@@ -37,7 +44,7 @@ namespace rtp {
 // of a line each, take 9 - 20 us a tile: the L2 takes a request, not a byte, per clock.)  vmcnt counts loads and stores in the
 // order of their issue, so the first phases behind an epilogue let its 16 stores be on their way too.
 //
-// Time stamps in the kernel, 8192 x 8192 x 1024 on zeros (at the full clock), us a tile: before (a workgroup a tile, the epilogue
+// Time stamps in the kernel with 32 x 32 x 16 MFMAs, 8192 x 8192 x 1024 on zeros (at the full clock), us a tile: before (a workgroup a tile, the epilogue
 // through 64 KiB of slab memory in four passes between barriers) prologue 2.8, 16 slabs 21 - 22, epilogue 7.9, gap 1.2; now 0.8, 21 -
 // 24 (the stores of the tile before drain beside its loads), 1.7 - 2.5.  On one tile a CU (4096 x 4096 x 2048) 49.9 -> 40.7.  Random
 // operands cost power, and the clock follows (1.5 - 1.9 us a slab instead of 1.1), so they gain less.  us, forward / input gradient /
@@ -87,39 +94,39 @@ __device__ __forceinline__ void lds_store(unsigned at, V v) {
   *(__attribute__((address_space(3))) V*)(uintptr_t)at = v;
 }
 
-// Where a lane's fragments of a half tile (128 rows, as DmaOperand leaves them) are: of BLOCKS blocks of 32 rows from `row0` on, in
+// Where a lane's fragments of a half tile (128 rows, as DmaOperand leaves them) are: of BLOCKS blocks of 16 rows from `row0` on, in
 // the slab at `at`.  k-contiguous: an address for every k-step, the blocks at constant distances; row-contiguous the other way round.
 template <bool KC, int BLOCKS>
 struct FragPlace {
-  unsigned v[KC ? 4 : BLOCKS];
+  unsigned v[KC ? 2 : BLOCKS];
   __device__ __forceinline__ void init(unsigned at, int row0, int lane) {
-    const int li = lane & 31, g = lane >> 5;
+    const int li = lane & 15, g = lane >> 4;
     if (KC) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] = at + (row0 + li) * 128 + (((2 * q + g) ^ kc_swizzle<128>(li)) << 4);
+      for (int q = 0; q < 2; ++q) v[q] = at + (row0 + li) * 128 + (((4 * q + g) ^ kc_swizzle<128>(li)) << 4);
     } else {
-      const int s16 = lane & 15, kl = g * 8 + (s16 >> 2);
+      const int kl = g * 8 + (li >> 2);
 #pragma unroll
       for (int i = 0; i < BLOCKS; ++i) {
-        const int rb = (row0 + i * 32 + 16 * ((lane >> 4) & 1) + 4 * (s16 & 3)) * 2;
-        v[i] = at + kl * 256 + (((rb >> 4) ^ rc_swizzle<bf16_t, 128>(kl)) << 4) + (rb & 15);
+        const int rb = (row0 + i * 16 + 4 * (li & 3)) * 2;
+        v[i] = at + kl * 256 + (((rb >> 4) ^ rc_swizzle<bf16_t, 128, 16>(kl)) << 4) + (rb & 15);
       }
     }
   }
   __device__ __forceinline__ void other_slab(unsigned bytes) {
 #pragma unroll
-    for (int i = 0; i < (KC ? 4 : BLOCKS); ++i) v[i] ^= bytes;
+    for (int i = 0; i < (KC ? 2 : BLOCKS); ++i) v[i] ^= bytes;
   }
   // block i, k-step q of the half tile `half` bytes into the slab
   __device__ __forceinline__ Frag<bf16_t> read(int half, int i, int q) const {
     Frag<bf16_t> f;
     if (KC) {
-      f.v = __builtin_bit_cast(bf16x8, lds_load<u32x4>(v[q] + half + i * 4096));
+      f.v = __builtin_bit_cast(bf16x8, lds_load<u32x4>(v[q] + half + i * 2048));
     } else {
       typedef short short8_t __attribute__((ext_vector_type(8)));
       typedef __attribute__((address_space(3))) short4_t* tr_t;
-      const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_t)(uintptr_t)(v[i] + half + q * 4096));
-      const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_t)(uintptr_t)(v[i] + half + q * 4096 + 1024));
+      const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_t)(uintptr_t)(v[i] + half + q * 8192));
+      const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_t)(uintptr_t)(v[i] + half + q * 8192 + 1024));
       f.v = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     }
     return f;
@@ -137,15 +144,15 @@ template <bool AKC, bool BKC, bool PAIR>
 __device__ __forceinline__ void large_body() {
   using T = bf16_t;
   constexpr int BM = 256, BN = 256, NL = 8, SB = 128;
-  constexpr int WM = 128, WN = 64, MT = 4, NT = 2;
+  constexpr int WM = 128, WN = 64, MT = 8, NT = 4;  // wave tile, blocks of 16 x 16
   constexpr int BLKA = WM / 2, BLKB = WN / 2;
-  using DA = DmaOperand<T, BM / 2, AKC, NL, SB>;
-  using DB = DmaOperand<T, BN / 2, BKC, NL, SB>;
+  using DA = DmaOperand<T, BM / 2, AKC, NL, SB, 16>;
+  using DB = DmaOperand<T, BN / 2, BKC, NL, SB, 16>;
   constexpr int BK = SB / sizeof(T);
-  constexpr int KS = SB / 32;
+  constexpr int KS = SB / 64;          // k-steps of a slab
   constexpr int HALF = DA::BYTES, SLAB = 4 * HALF;
   constexpr int NI = DA::NI;           // load instructions per wave and half tile
-  constexpr int NSTORE = MT * NT * 2;  // stores of a wave in a whole tile's epilogue, at least
+  constexpr int NSTORE = MT * NT / 2;  // stores of a wave in a whole tile's epilogue, at least
   constexpr int PAGE = 4096;           // a wave's own LDS: 32 rows of its 64 columns in bf16, or the bias of its columns
   constexpr bool kUpdates = !AKC && !BKC;  // weight gradients may come with an update
   constexpr int kBiasSegs = 16;        // K segments whose biases are brought there
@@ -162,7 +169,6 @@ __device__ __forceinline__ void large_body() {
   const KernArgs args = kernel_args();
   const int tid = threadIdx.x;
   if (args->trace != nullptr && tid == 0) atomicMin(args->trace, (unsigned long long)wall_clock64());
-  const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 2, wn = wave & 3;
 
@@ -203,16 +209,16 @@ __device__ __forceinline__ void large_body() {
   const int nk_seg = (kdim + BK - 1) / BK;
   const int nk = nk_seg * args->ksegs;
 
-  f32x16 acc[MT][NT];
-  float rsum = 0.0f;
+  f32x4 acc[MT][NT];
+  float rsum[2] = {0.0f, 0.0f};
   auto clear = [&] {
-    rsum = 0.0f;
+    rsum[0] = rsum[1] = 0.0f;
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
       for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+        for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.0f;
   };
 
   // ---- this wave's share of the loads, which run ahead of the products and into the next tile ----
@@ -298,11 +304,13 @@ __device__ __forceinline__ void large_body() {
 
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
-  Frag<T> fa[2][KS], fb0[KS], fb0n[KS], fb1[KS];  // B half 0 of the next slab is read while this slab's is multiplied
-  FragPlace<AKC, 2> pa;
-  FragPlace<BKC, 1> pb;
-  pa.init(lds0, wm * BLKA, lane);
-  pb.init(lds0 + 2 * HALF, wn * BLKB, lane);
+  Frag<T> fa[4][KS], fb0[2][KS], fb0n[2][KS], fb1[2][KS];  // B half 0 of the next slab is read while this slab's is multiplied
+  FragPlace<AKC, 4> pa;
+  FragPlace<BKC, 2> pb;
+  auto place = [&](unsigned slab_at) {
+    pa.init(lds0 + slab_at, wm * BLKA, lane_now());
+    pb.init(lds0 + slab_at + 2 * HALF, wn * BLKB, lane_now());
+  };
   // The block of 32 rows whose sums of A this wave adds up beside the products, or -1.  The additions are one chain behind the MFMAs of a phase, and
   // the waves go in step: a phase with sums is 250 clocks longer for the tile.  So the four blocks of a wave tile's rows go to the first four tile
   // columns, a wave each (with two or three columns two in the same phase), instead of all to the first.  us without sums / all in the first /
@@ -311,22 +319,24 @@ __device__ __forceinline__ void large_body() {
   int sum_block = -1;
   auto read_a = [&](auto H) {
 #pragma unroll
-    for (int q = 0; q < KS; ++q)
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int i = 0; i < 2; ++i) fa[i][q] = pa.read(decltype(H)::value * HALF, i, q);
+      for (int q = 0; q < KS; ++q) fa[i][q] = pa.read(decltype(H)::value * HALF, i, q);
   };
-  auto read_b = [&](auto H, Frag<T>(&fb)[KS]) {
+  auto read_b = [&](auto H, Frag<T>(&fb)[2][KS]) {
 #pragma unroll
-    for (int q = 0; q < KS; ++q) fb[q] = pb.read(decltype(H)::value * HALF, 0, q);
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int q = 0; q < KS; ++q) fb[j][q] = pb.read(decltype(H)::value * HALF, j, q);
   };
   auto row_sums = [&](auto H) {
     if (!AKC && sum_block >> 1 == decltype(H)::value) {
       if (sum_block & 1) {
 #pragma unroll
-        for (int q = 0; q < KS; ++q) rsum = frag_sum(fa[1][q], rsum);
+        for (int q = 0; q < KS; ++q) rsum[0] = frag_sum(fa[2][q], rsum[0]), rsum[1] = frag_sum(fa[3][q], rsum[1]);
       } else {
 #pragma unroll
-        for (int q = 0; q < KS; ++q) rsum = frag_sum(fa[0][q], rsum);
+        for (int q = 0; q < KS; ++q) rsum[0] = frag_sum(fa[0][q], rsum[0]), rsum[1] = frag_sum(fa[1][q], rsum[1]);
       }
     }
   };
@@ -337,15 +347,20 @@ __device__ __forceinline__ void large_body() {
   };
   // the barrier that ends a read half, the MFMA half and its end, where this wave's reads have returned (the first MFMAs
   // wait only for their own fragments)
-  auto multiply = [&](auto H, auto J, const Frag<T>(&fb)[KS], auto SUMS) {
+  auto multiply = [&](auto H, auto J, const Frag<T>(&fb)[2][KS], auto SUMS) {
     constexpr int h = decltype(H)::value, j = decltype(J)::value;
     __builtin_amdgcn_sched_barrier(0);
     barrier();
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int q = 0; q < KS; ++q)
+    for (int n = 0; n < 8; ++n) {
+      const int i = n >> 1, jj = (n ^ i) & 1;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) mma(fb[q], fa[i][q], acc[h * 2 + i][j]);  // transposed: a lane holds columns of one row
+      for (int q = 0; q < KS; ++q) {
+        mma(fb[jj][q], fa[i][q], acc[h * 4 + i][j * 2 + jj]);  // transposed: a lane holds columns of one row
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
     __builtin_amdgcn_s_setprio(0);
     if constexpr (decltype(SUMS)::value) row_sums(H);
     __builtin_amdgcn_sched_barrier(0);
@@ -393,39 +408,41 @@ __device__ __forceinline__ void large_body() {
     multiply(I1{}, I0{}, fb0, std::false_type{});
     if constexpr (rest >= 1) {
 #pragma unroll
-      for (int q = 0; q < KS; ++q) fb0[q] = fb0n[q];
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int q = 0; q < KS; ++q) fb0[j][q] = fb0n[j][q];
     }
     cur = other;
   };
 
   const unsigned page = lds0 + 2 * SLAB + wave * PAGE;
-  // Eight neighbouring columns of a row per lane: columns 16 h + 8 g of block (i, j), after the two halves of the wave have
-  // exchanged four of them.
-  auto columns = [&](const f32x16& c, auto H, float(&v)[8]) {
-    constexpr int h = decltype(H)::value;
+  // Eight neighbouring columns of a row per lane: of two blocks side by side, columns 16 (g & 1) + 8 (g >> 1) of the 32, after
+  // neighbouring groups of 16 lanes have exchanged four of them.
+  auto columns = [&](const f32x4& left, const f32x4& right, float(&v)[8]) {
     typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const u32x2 r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, (float)c[8 * h + e]),
-                                                       __builtin_bit_cast(unsigned, (float)c[8 * h + 4 + e]), false, false);
+      const u32x2 r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, (float)left[e]),
+                                                       __builtin_bit_cast(unsigned, (float)right[e]), false, false);
       const unsigned lo = r.x, hi = r.y;  // (the cast of a vector's element itself would be one of element 0)
       v[e] = __builtin_bit_cast(float, lo), v[4 + e] = __builtin_bit_cast(float, hi);
     }
   };
-  // the bias of columns col0 + 8 g .. + 7: by scalar loads, which no vector load or store has to be waited for
+  // the bias of a lane's eight of the 32 columns from col on: by scalar loads, which no vector load or store has to be waited for
   auto bias8 = [&](KernArgs p, const Tile& w, int col, int g, float(&v)[8]) {
     typedef const __attribute__((address_space(4))) u32x4* scalar_t;
     const T* bias = reinterpret_cast<const T*>(p->bias) + w.grp * p->bias_sg + w.zo * p->bias_so + w.zi * p->bias_si;
-    const T *lo = bias + (col < rows_b ? col : 0), *hi = bias + (col + 8 < rows_b ? col + 8 : 0);
     const int nb_seg = p->bias_sk ? p->ksegs : 1;  // a bias per K segment is summed in segment order
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = 0.0f;
 #pragma unroll 1
     for (int sgm = 0; sgm < nb_seg; ++sgm) {
-      const u32x4 s0 = *(scalar_t)(uintptr_t)(lo + sgm * p->bias_sk), s1 = *(scalar_t)(uintptr_t)(hi + sgm * p->bias_sk);
+      u32x4 s[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) s[c] = *(scalar_t)(uintptr_t)(bias + (col + 8 * c < rows_b ? col + 8 * c : 0) + sgm * p->bias_sk);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const unsigned two = g ? s1[e] : s0[e];
+        const unsigned two = g & 1 ? g & 2 ? s[3][e] : s[2][e] : g & 2 ? s[1][e] : s[0][e];
         v[2 * e] += __builtin_bit_cast(float, two << 16);
         v[2 * e + 1] += __builtin_bit_cast(float, two & 0xffff0000u);
       }
@@ -447,7 +464,7 @@ __device__ __forceinline__ void large_body() {
     typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
     typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
     const KernArgs p = kernel_args();
-    const int lane = lane_now(), li = lane & 31, g = lane >> 5;
+    const int lane = lane_now(), li = lane & 15, g = lane >> 4;
     const bool stream_out = p->flags & RTP_GEMM_STREAM_OUT;
     const int row0 = w.m0 + wm * WM, col0 = w.n0 + wn * WN;
     if (edge && (row0 >= rows_a || col0 >= rows_b)) return;
@@ -455,54 +472,50 @@ __device__ __forceinline__ void large_body() {
     const int rows = !edge ? WM : col0 + lc < rows_b ? rows_a - (row0 + lr) : 0;  // of the product from this lane's first on
     const long ldc = p->ldc, ld_in = mask ? p->ld_gate : p->ld_cin;
     T* dst = reinterpret_cast<T*>(p->c_out) + w.grp * p->c_sg + w.zo * p->c_so + w.zi * p->c_si + (row0 + lr) * ldc + col0 + lc;
-    u32x4 in[MT][4];
+    u32x4 in[MT / 2][4];
     if constexpr (add || mask) {
       const T* first = mask ? reinterpret_cast<const T*>(p->gate) + w.grp * p->gate_sg + w.zo * p->gate_so + w.zi * p->gate_si
                             : reinterpret_cast<const T*>(p->c_in) + w.grp * p->cin_sg + w.zo * p->cin_so + w.zi * p->cin_si;
       const T* src = first + (row0 + lr) * ld_in + col0 + lc;
 #pragma unroll
-      for (int i = 0; i < MT; ++i)
+      for (int i = 0; i < MT / 2; ++i)
 #pragma unroll
         for (int s = 0; s < 4; ++s)
           in[i][s] = *reinterpret_cast<const u32x4*>(!edge || i * 32 + s * 8 < rows ? src + (i * 32 + s * 8) * ld_in : first);
     }
-    float b[NT][4][4];  // of columns 32 j + 8 t + 4 g ..
+    float b[NT][4];  // of columns 16 j + 4 g ..
     if constexpr (bias) {
 #pragma unroll
       for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) b[j][t][e] = 0.0f;
+        for (int e = 0; e < 4; ++e) b[j][e] = 0.0f;
       const int nb_seg = p->bias_sk ? p->ksegs : 1;  // a bias per K segment is summed in segment order
 #pragma unroll 1
       for (int sgm = 0; sgm < nb_seg; ++sgm)
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
+        for (int j = 0; j < NT; ++j) {
+          const bf16x4 x = __builtin_bit_cast(bf16x4, lds_load<u32x2>(page + sgm * (WN * 2) + (j * 16 + 4 * g) * 2));
 #pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            const bf16x4 x = __builtin_bit_cast(bf16x4, lds_load<u32x2>(page + sgm * (WN * 2) + (j * 32 + t * 8 + 4 * g) * 2));
-#pragma unroll
-            for (int e = 0; e < 4; ++e) b[j][t][e] += (float)x[e];
-          }
+          for (int e = 0; e < 4; ++e) b[j][e] += (float)x[e];
+        }
     }
-    const unsigned wr = page + li * 128 + 8 * g, rd = page + lr * 128;  // 16-byte chunk c of row r is at chunk c ^ (r >> 1 & 7)
-    const unsigned swz = (li >> 1) & 7;
+    const unsigned wr = page + li * 128 + 8 * (g & 1), rd = page + lr * 128;  // 16-byte chunk c of row r is at chunk c ^ (r >> 1 & 7)
+    const unsigned swz = ((li >> 1) & 7) ^ (g >> 1);
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
+    for (int i = 0; i < MT / 2; ++i) {
       if constexpr (add) {
 #pragma unroll
         for (int s = 0; s < 4; ++s)
           lds_store<u32x4>(rd + s * 1024 + (((lane & 7) ^ (((lr + s * 8) >> 1) & 7)) << 4), in[i][s]);
       }
 #pragma unroll
-      for (int j = 0; j < NT; ++j)
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const unsigned at = wr + ((unsigned)((j * 4 + t) ^ swz) << 4);
+        for (int j = 0; j < NT; ++j) {
+          const unsigned at = wr + t * 2048 + ((unsigned)((j * 2) ^ swz) << 4);
           float v[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = acc[i][j][4 * t + e];
+          for (int e = 0; e < 4; ++e) v[e] = acc[2 * i + t][j][e];
           if constexpr (add) {
             const bf16x4 x = __builtin_bit_cast(bf16x4, lds_load<u32x2>(at));
 #pragma unroll
@@ -510,7 +523,7 @@ __device__ __forceinline__ void large_body() {
           }
           if constexpr (bias) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] += b[j][t][e];
+            for (int e = 0; e < 4; ++e) v[e] += b[j][e];
           }
           if constexpr (relu) {
 #pragma unroll
@@ -550,10 +563,9 @@ __device__ __forceinline__ void large_body() {
   // update takes them as, the fp32 parameters of 32 rows are requested while the 32 before them are finished.
   auto finish_update = [&](const Tile& w, bool whole) {
     typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
     typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
     const KernArgs p = kernel_args();
-    const int lane = lane_now(), li = lane & 31, g = lane >> 5;
+    const int lane = lane_now(), li = lane & 15, g = lane >> 4;
     const bool stream_out = p->flags & RTP_GEMM_STREAM_OUT, skip_out = p->flags & RTP_GEMM_SGD_SKIP_OUT, copy = p->sgd_w != nullptr;
     const float lr_ = p->sgd_lr, clip = p->sgd_clip;
     // this lane's row (and + 8, 16, 24) and columns (4 of the first 32, 4 of the others): eight lanes cover a line of fp32 parameters
@@ -563,7 +575,7 @@ __device__ __forceinline__ void large_body() {
     float* const master = p->sgd_master + zoff;
     T* const wcopy = reinterpret_cast<T*>(p->sgd_w) + zoff;
     T* const out = reinterpret_cast<T*>(p->c_out) + zoff;
-    const unsigned wr = page + li * 128 + 8 * g, swz = (li >> 1) & 7;
+    const unsigned wr = page + li * 128 + 8 * (g & 1), swz = ((li >> 1) & 7) ^ (g >> 1);
     auto inside = [&](int row, int h) { return whole || (row < rows_a && col0 + 32 * h < rows_b); };
     f32x4 par[2][2][2];  // of 16 rows
     auto request = [&](int u) {
@@ -579,18 +591,17 @@ __device__ __forceinline__ void large_body() {
     };
     request(0);
 #pragma unroll
-    for (int u = 0; u < 2 * MT; ++u) {
-      const int i = u >> 1;
-      if (u + 1 < 2 * MT) request(u + 1);
+    for (int u = 0; u < MT; ++u) {
+      if (u + 1 < MT) request(u + 1);
       if (u % 2 == 0) {
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int t = 0; t < 4; ++t) {
+          for (int j = 0; j < NT; ++j) {
             bf16x4 o;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = from_f32<T>(acc[i][j][4 * t + e]);
-            lds_store<u32x2>(wr + ((unsigned)((j * 4 + t) ^ swz) << 4), __builtin_bit_cast(u32x2, o));
+            for (int e = 0; e < 4; ++e) o[e] = from_f32<T>(acc[u + t][j][e]);
+            lds_store<u32x2>(wr + t * 2048 + ((unsigned)((j * 2) ^ swz) << 4), __builtin_bit_cast(u32x2, o));
           }
       }
 #pragma unroll
@@ -622,10 +633,10 @@ __device__ __forceinline__ void large_body() {
         }
     }
   };
-  // everything else, block after block in a loop
+  // everything else, 16 rows after 16 rows in a loop
   auto finish_any = [&](const Tile& w, bool whole) {
     const KernArgs p = kernel_args();
-    const int lane = lane_now(), li = lane & 31, g = lane >> 5;
+    const int lane = lane_now(), li = lane & 15, g = lane >> 4;
     const int flags = p->flags;
     const bool stream_out = flags & RTP_GEMM_STREAM_OUT, relu = flags & RTP_GEMM_RELU;
     const bool out_f32 = flags & RTP_GEMM_OUT_F32, cin_f32 = flags & RTP_GEMM_CIN_F32;
@@ -634,56 +645,56 @@ __device__ __forceinline__ void large_body() {
     const T* gate =
         p->gate ? reinterpret_cast<const T*>(p->gate) + w.grp * p->gate_sg + w.zo * p->gate_so + w.zi * p->gate_si : nullptr;
 #pragma unroll 1
-    for (int blk = 0; blk < MT * NT; ++blk) {
-      f32x16 part;
+    for (int blk = 0; blk < MT; ++blk) {
+      f32x4 part[NT];
       // (an empty instruction per copy: merged into one copy from a computed place, the accumulators would have to be in memory)
-      auto take = [&](const f32x16& from) {
-        part = from;
-        asm volatile("" : "+v"(part));
+      auto take = [&](const f32x4(&from)[NT]) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          part[j] = from[j];
+          asm volatile("" : "+v"(part[j]));
+        }
       };
       switch (blk) {
-        case 0: take(acc[0][0]); break;
-        case 1: take(acc[0][1]); break;
-        case 2: take(acc[1][0]); break;
-        case 3: take(acc[1][1]); break;
-        case 4: take(acc[2][0]); break;
-        case 5: take(acc[2][1]); break;
-        case 6: take(acc[3][0]); break;
-        default: take(acc[3][1]);
+        case 0: take(acc[0]); break;
+        case 1: take(acc[1]); break;
+        case 2: take(acc[2]); break;
+        case 3: take(acc[3]); break;
+        case 4: take(acc[4]); break;
+        case 5: take(acc[5]); break;
+        case 6: take(acc[6]); break;
+        default: take(acc[7]);
       }
-      const int row = w.m0 + wm * WM + (blk >> 1) * 32 + li, col0 = w.n0 + wn * WN + (blk & 1) * 32;
+      const int row = w.m0 + wm * WM + blk * 16 + li, col0 = w.n0 + wn * WN, mine8 = 16 * (g & 1) + 8 * (g >> 1);
       const long rowc = row < rows_a ? row : rows_a - 1;
-      Raw8<T> rg[2], rc16[2];
-      Raw8<float> rc32[2];
+      Raw8<T> rg[2];
+      Raw8<float> rc[2];  // (an addend in bf16 in its first vector)
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
-        const int col = col0 + 16 * c + 8 * g, colc = col < rows_b ? col : 0;
+        const int col = col0 + 32 * c + mine8, colc = col < rows_b ? col : 0;
         if (cin) {
           if (cin_f32)
-            rc32[c].load(reinterpret_cast<const float*>(cin) + rowc * p->ld_cin + colc);
+            rc[c].load(reinterpret_cast<const float*>(cin) + rowc * p->ld_cin + colc);
           else
-            rc16[c].load(reinterpret_cast<const T*>(cin) + rowc * p->ld_cin + colc);
+            rc[c].q[0] = *reinterpret_cast<const uint4*>(reinterpret_cast<const T*>(cin) + rowc * p->ld_cin + colc);
         }
         if (gate) rg[c].load(gate + rowc * p->ld_gate + colc);
       }
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
-        const int col = col0 + 16 * c + 8 * g;
+        const int col = col0 + 32 * c + mine8;
         float v[8], t[8];
-        if (c & 1)
-          columns(part, I1{}, v);
-        else
-          columns(part, I0{}, v);
+        columns(part[2 * c], part[2 * c + 1], v);
         if (cin) {
           if (cin_f32)
-            rc32[c].get(t);
+            rc[c].get(t);
           else
-            rc16[c].get(t);
+            Raw8<T>{{rc[c].q[0]}}.get(t);
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] += t[e];
         }
         if (p->bias) {
-          bias8(p, w, col0 + 16 * c, g, t);
+          bias8(p, w, col0 + 32 * c, g, t);
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[e] += t[e];
         }
@@ -750,11 +761,17 @@ __device__ __forceinline__ void large_body() {
     using Yes = std::true_type;
     using No = std::false_type;
     if (!AKC && sum_block >= 0) {
-      const int lane = lane_now(), li = lane & 31, g = lane >> 5;
+      const int lane = lane_now(), li = lane & 31;
       T* dst = reinterpret_cast<T*>(p->a_rowsum) + w.grp * p->rowsum_sg;
-      const float v = rsum + __shfl_xor(rsum, 32, 64);
+      float v = 0.0f;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const float h = rsum[t] + __shfl_xor(rsum[t], 16, 64);
+        const float f = h + __shfl_xor(h, 32, 64);
+        v = li >> 4 == t ? f : v;
+      }
       const int row = w.m0 + wm * WM + sum_block * 32 + li;
-      if (g == 0 && row < rows_a) dst[row] = from_f32<T>((p->flags & RTP_GEMM_ROWSUM_ACCUM) ? to_f32(dst[row]) + v : v);
+      if (lane < 32 && row < rows_a) dst[row] = from_f32<T>((p->flags & RTP_GEMM_ROWSUM_ACCUM) ? to_f32(dst[row]) + v : v);
     }
     if (p->alpha != 1.0f) {
 #pragma unroll
@@ -762,7 +779,7 @@ __device__ __forceinline__ void large_body() {
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) acc[i][j][r] *= p->alpha;
+          for (int r = 0; r < 4; ++r) acc[i][j][r] *= p->alpha;
     }
     const bool whole = w.m0 + BM <= rows_a && w.n0 + BN <= rows_b;
     if (form == 0)
@@ -790,6 +807,7 @@ __device__ __forceinline__ void large_body() {
   clear();
   RTP_WAIT_VM(5 * NI);  // halves 0 of slab 0 have landed
   barrier();
+  place(0);
   read_b(I0{}, fb0);
   __builtin_amdgcn_sched_barrier(0);
   for (;;) {
@@ -817,6 +835,7 @@ __device__ __forceinline__ void large_body() {
     asm volatile("" ::: "memory");
     behind = here.m0 + BM <= rows_a && here.n0 + BN <= rows_b ? 5 : 0;
     clear();
+    place(cur);  // (anew: held over the epilogue the addresses spill)
     here = next;
   }
   if (kernel_args()->trace != nullptr && tid == 0) atomicMax(kernel_args()->trace + 1, (unsigned long long)wall_clock64());

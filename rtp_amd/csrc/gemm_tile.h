@@ -9,6 +9,7 @@ namespace rtp {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 struct GemmArgs {
   const char* a;
@@ -73,6 +74,10 @@ struct Frag<float> {
 
 __device__ __forceinline__ void mma(const Frag<bf16_t>& a, const Frag<bf16_t>& b, f32x16& c) {
   c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.v, b.v, c, 0, 0, 0);
+}
+// 16 x 16 outputs over 32 k: lane group g = lane / 16 holds k = 8g + e in element e and rows 4g + r of the results in register r.
+__device__ __forceinline__ void mma(const Frag<bf16_t>& a, const Frag<bf16_t>& b, f32x4& c) {
+  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, b.v, c, 0, 0, 0);
 }
 __device__ __forceinline__ void mma(const Frag<float>& a, const Frag<float>& b, f32x16& c) {
   // Lane group g holds k = 4g+e in element e, so MFMA number e contracts k in {e, 4+e}.
@@ -633,10 +638,13 @@ typedef __attribute__((address_space(3))) void* lptr_t;
 //    chunk position c ^ ((r >> 1) & 7), which together with the row's parity (rows alternate between the two
 //    128-byte halves of the bank space) gives 16 different 16-byte bank slots.
 //  * row-contiguous 16-bit operand, [k][rows]: a transposing read touches 4 consecutive k lines x 64 bytes; the
-//    chunk index inside k line kl is XORed with rc_swizzle(kl) so that the 4 lines fall on different slots.
-template <typename T, int R>
+//    chunk index inside k line kl is XORed with rc_swizzle(kl) so that the 4 lines fall on different slots.  Fragments of FR = 16
+//    rows take 32 bytes of eight lines at a time, four neighbouring ones from each of two of the fragment's four octets of k.
+template <typename T, int R, int FR = 32>
 __device__ __forceinline__ constexpr int rc_swizzle(int kl) {
   if (sizeof(T) != 2 || R < 64) return 0;  // (the 64-byte lines of 32 rows fall on different slots as they stand)
+  static_assert(FR == 32 || R >= 128, "fragments of 16 rows: lines of 256 bytes");
+  if (FR == 16) return (kl & 3) << 2 | ((kl >> 3 ^ kl >> 4) & 1) << 1;
   return R >= 128 ? (kl & 3) << 2 : ((kl >> 1) & 1) << 2;
 }
 
@@ -647,7 +655,7 @@ __device__ __forceinline__ constexpr int kc_swizzle(int row) {
   return SB == 128 ? (row >> 1) & 7 : (row >> 2) & 3;
 }
 
-template <typename T, int R, bool KC, int NL, int SB>
+template <typename T, int R, bool KC, int NL, int SB, int FR = 32>
 struct DmaOperand {
   static constexpr int VEC = 16 / sizeof(T);
   static_assert(SB == 128 || SB == 64, "slab rows of 128 or 64 bytes");
@@ -690,7 +698,7 @@ struct DmaOperand {
       } else {
         const int byte = lane * 16;
         const int kl = j * (1024 / LINE) + byte / LINE;
-        const int chunk = ((byte % LINE) >> 4) ^ rc_swizzle<T, R>(kl);  // which 16 bytes of the k line land here
+        const int chunk = ((byte % LINE) >> 4) ^ rc_swizzle<T, R, FR>(kl);  // which 16 bytes of the k line land here
         int src = row_of(chunk * VEC);
         if (row0 + src >= rows) src = 0;  // past the end: re-read the tile's first rows (a k line that is no whole number of vectors is padded)
         ofs[i] = (unsigned)((long)kl * ld * (long)sizeof(T)) + (unsigned)(src * (int)sizeof(T));

@@ -18,9 +18,8 @@
 // wait for.  Shared blocks need a quarter of that and their latency is hidden; the loop is then bound by LDS
 // reads, MFMA and the softmax's vector instructions in equal parts (about 1000 clocks each for a wave's 32 x 64 scores at
 // D = 128, bf16), which two or more waves per SIMD overlap.
-// Measured (one wave per tile -> this; forward, backward): 64 heads of 1500 x 128 in bf16 261 -> 113 us (650 TFLOP/s), with a key
-// bias 117, 636 -> 340 us; 256 causal heads of 512 x 64 28 -> 21 us, 78 -> 70 us; with a [512, 512] mask, D = 32, 44 us both
-// ways, 116 -> 93 us.
+// Measured (one wave per tile -> shared blocks -> this; forward, backward): 64 heads of 1500 x 128 in bf16 261 -> 113 -> 106 us (690 TFLOP/s),
+// 636 -> 309 -> 269 us; 256 causal heads of 512 x 64 28 -> 22 -> 21 us, 78 -> 72 -> 65 us.
 #include "common.h"
 
 #include <type_traits>
@@ -169,16 +168,28 @@ __device__ __forceinline__ void pack(const float* v, typename Op<T>::Frag (&f)[N
     for (int e = 0; e < Op<T>::MR; ++e) f[m][e] = from_f32<T>(v[Op<T>::MR * m + e]);
 }
 
-// Accumulator (registers = features, lanes = rows) -> 4 consecutive features of a row per store.
-template <typename T>
-__device__ __forceinline__ void store_acc(char* row, int db, int g, const f32x16& acc, float scale) {
+// Accumulators (registers = features, lanes = rows) of a wave's 32 rows -> memory, through LDS of the wave's own (32 rows of D elements;
+// the 16-byte chunks of a row permuted by XOR), whole lines at a time.  With a lane's own 4 features a store (16 bytes of each of 32 rows)
+// the stores of a workgroup took 3.8 - 5.2 us, a quarter of a workgroup's time at 512 keys.  us, such stores -> these: 256 causal heads of
+// 512 x 64 22.1 -> 21.4 forward, 72 -> 66 backward; of 512 x 128 45.8 -> 42.3, 154 -> 128.
+template <typename T, int D>
+__device__ __forceinline__ void store_rows(char* own, const f32x16 (&acc)[D / 32], float scale, char* first, long stride, int rows, int lane) {
+  constexpr int PITCH = D * (int)sizeof(T), CPR = PITCH / 16;
+  const int li = lane & 31, g = lane >> 5;
 #pragma unroll
-  for (int a4 = 0; a4 < 4; ++a4) {
-    T e[4];
+  for (int db = 0; db < D / 32; ++db)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) e[i] = from_f32<T>(acc[4 * a4 + i] * scale);
-    char* dst = row + (32 * db + 8 * a4 + 4 * g) * (int)sizeof(T);
-    *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<const uint2*>(e);
+    for (int a4 = 0; a4 < 4; ++a4) {
+      T e[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) e[i] = from_f32<T>(acc[db][4 * a4 + i] * scale);
+      *reinterpret_cast<uint2*>(own + li * PITCH + (((4 * db + a4) ^ (li % CPR)) << 4) + 8 * g) = *reinterpret_cast<const uint2*>(e);
+    }
+#pragma unroll
+  for (int i = 0; i < CPR / 2; ++i) {
+    const int row = (i * 64 + lane) / CPR, chunk = lane % CPR;
+    const uint4 v = *reinterpret_cast<const uint4*>(own + row * PITCH + ((chunk ^ (row % CPR)) << 4));
+    if (row < rows) *reinterpret_cast<uint4*>(first + row * stride + chunk * 16) = v;
   }
 }
 
@@ -253,12 +264,21 @@ constexpr int fwd_waves() {
 }
 template <typename T, int D>
 constexpr int dq_waves() {
-  return D == 128 ? 2 : D == 64 ? 3 : 4;
+  return D == 32 ? 4 : 2;
 }
 template <typename T, int D>
 constexpr int dkv_waves() {
   return D == 128 ? 1 : D == 64 ? 2 : 3;
 }
+// Whether blocks without edges or masks go through loops of their own that put the vector work between the MFMAs of the other half of the
+// block.  An MFMA leaves 28 of its 32 clocks to other instructions of its wave, but instructions that depend on each other take 8.5
+// clocks each, a read of an accumulation register 8 and an LDS read 14, so such a wave gains where no other one fills the gaps: one or two
+// a SIMD.  dQ at D = 128 needs 290 registers that way, one wave a SIMD instead of two: 139 -> 144 us for 64 heads of 1500.  At D = 32 the four
+// waves a SIMD that it costs are worth more (256 causal heads of 512 50.5 -> 51.4).  dK / dV of 64 heads of 1500 x 128 208 -> 180 us.
+template <int D>
+constexpr bool kInterleaveDq = D == 64;
+template <int D>
+constexpr bool kInterleaveDkv = D >= 64;
 
 // ADD: something joins the scaled scores (a mask, a key bias), or the scale is not positive and their order turns round: scores
 // are brought to the log2 domain first and their maximum is subtracted there, exactly: a mask may lower all keys of a query by
@@ -414,11 +434,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(fwd_wav
   float lo, hi;
   halves(l_run, lo, hi);
   const float l = lo + hi;
+  block_barrier();  // every wave has left the last block
+  store_rows<T, D>(lds + wave * 32 * B::PITCH, acc, l > 0.0f ? 1.0f / l : a.empty, a.out + it.o + q0 * a.o_l, a.o_l, a.L - q0, lane);
   if (query < a.L) {
-    const float inv = l > 0.0f ? 1.0f / l : a.empty;
-    char* row = a.out + it.o + (long)query * a.o_l;
-#pragma unroll
-    for (int db = 0; db < DB; ++db) store_acc<T>(row, db, g, acc[db], inv);
     if (g == 0) a.lse[(long)it.z * a.L + query] = l > 0.0f ? (m_run + __builtin_amdgcn_logf(l)) * kLn2 : a.empty;
   }
 }
@@ -442,6 +460,47 @@ __device__ __forceinline__ void p_and_ds(const FlashArgs& a, const f32x16& s, co
   }
 #pragma unroll
   for (int r = 0; r < 16; ++r) ds[r] = p[r] * (dp[r] - delta[KEYS_IN_REGS ? 0 : r]);
+}
+
+// N MFMAs in a row, one slot each: read(n) is MFMA n's operand from LDS, AHEAD slots before its use, between(n) a share of the vector
+// work, which a wave issues in the MFMA's shadow.
+template <typename Frag, int N, int AHEAD, typename Read, typename Mul, typename Between>
+__device__ __forceinline__ void mfma_stream(Read read, Mul mul, Between between) {
+  constexpr int R = AHEAD + 1;
+  Frag f[R];
+  [&]<int... I>(std::integer_sequence<int, I...>) __attribute__((always_inline)) {
+    ((f[I] = read(std::integral_constant<int, I>{})), ...);
+  }(std::make_integer_sequence<int, AHEAD>{});
+  __builtin_amdgcn_sched_barrier(0);
+  [&]<int... I>(std::integer_sequence<int, I...>) __attribute__((always_inline)) {
+    ([&] __attribute__((always_inline)) {
+      if constexpr (I + AHEAD < N) f[(I + AHEAD) % R] = read(std::integral_constant<int, I + AHEAD>{});
+      mul(std::integral_constant<int, I>{}, f[I % R]);
+      between(std::integral_constant<int, I>{});
+      __builtin_amdgcn_sched_barrier(0);
+    }(),
+     ...);
+  }(std::make_integer_sequence<int, N>{});
+}
+template <int D>
+constexpr int kAhead = D == 128 ? 6 : 3;
+
+// Scores that vector instructions take next, in vector registers.  A kernel of one wave per SIMD has its MFMA results in accumulation
+// registers otherwise, each of which costs a vector instruction of 8 clocks to read.  The compiler does not know what is inside: a
+// reader comes behind scores_settle().
+template <bool ONE_WAVE, bool FIRST>
+__device__ __forceinline__ void mma_scores(bf16x8 a, bf16x8 b, f32x16& c) {
+  if constexpr (ONE_WAVE && FIRST)
+    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b));
+  else if constexpr (ONE_WAVE)
+    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+  else
+    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, FIRST ? f32x16{} : c, 0, 0, 0);
+}
+// (a 32 x 32 x 16 MFMA's results are there 11 instructions behind it; two MFMAs more lie between as well)
+template <bool ONE_WAVE>
+__device__ __forceinline__ void scores_settle() {
+  if constexpr (ONE_WAVE) asm volatile("s_nop 10" ::: "memory");
 }
 
 template <typename T, int D, int NW>
@@ -491,6 +550,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dq_wave
   landed(qf);
   landed(gf);
   asm volatile("" : "+v"(lse));
+  if (!kbias && wave == 0) {  // both stages of the bias are read all the same
+    reinterpret_cast<float*>(lds + 4 * B::BYTES)[lane] = 0.0f;
+    reinterpret_cast<float*>(lds + 4 * B::BYTES)[64 + lane] = 0.0f;
+  }
   int lrow = B::lane_rows(lane), lcol = B::lane_cols(lane);
   f32x16 acc[DB];
 #pragma unroll
@@ -498,11 +561,73 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dq_wave
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[db][r] = 0.0f;
 
-  for (int kb = 0; kb < nkb; ++kb) {
+  // Both groups of a block, all of whose keys the wave's queries see (as in flash_dkv_kernel).
+  auto both = [&](const char* ks, const char* vs, const float* bias) __attribute__((always_inline)) {
+    constexpr int NA = 2 * NK, NC = NM * DB, EA = 16 / NA, EC = 16 / NC;
+    constexpr bool ONE_WAVE = dq_waves<T, D>() == 1;
+    f32x16 s[2], dp[2];
+    Frag df[2][NM];
+    f32x4 off[2];
+    auto offsets = [&](int quarter) __attribute__((always_inline)) {
+      off[quarter & 1] = *reinterpret_cast<const f32x4*>(bias + 8 * quarter + 4 * g);
+    };
+    auto element = [&](auto Hc, auto R) __attribute__((always_inline)) {
+      constexpr int h = decltype(Hc)::value, r = decltype(R)::value;
+      const float p = __builtin_amdgcn_exp2f(fmaf(s[h][r], a.scale, -lse + off[r / 4 & 1][r % 4]) * kLog2e);
+      df[h][r / Op<T>::MR][r % Op<T>::MR] = from_f32<T>(p * (dp[h][r] - delta[0]));
+      if constexpr (r % 4 == 3 && 4 * h + r / 4 + 2 < 8) offsets(4 * h + r / 4 + 2);
+    };
+    mfma_stream<Frag, 2 * NA + 2 * NC, kAhead<D>>(
+        [&](auto N) __attribute__((always_inline)) {
+          constexpr int n = decltype(N)::value, c = n - 2 * NA;
+          if constexpr (n < 2 * NA)
+            return B::rows(n & 1 ? vs : ks, lrow, n / NA, n % NA / 2);
+          else
+            return B::cols(ks, lcol, c / NC, c % NC / DB, c % DB);
+        },
+        [&](auto N, const Frag& f) __attribute__((always_inline)) {
+          constexpr int n = decltype(N)::value, c = n - 2 * NA;
+          if constexpr (n < 2 * NA) {
+            constexpr int h = n / NA, i = n % NA / 2;
+            if constexpr (n & 1)
+              mma_scores<ONE_WAVE, i == 0>(f, gf[i], dp[h]);
+            else
+              mma_scores<ONE_WAVE, i == 0>(f, qf[i], s[h]);
+          } else {
+            constexpr int h = c / NC, m = c % NC / DB, db = c % DB;
+            acc[db] = Op<T>::mma(f, df[h][m], acc[db]);
+          }
+        },
+        [&](auto N) __attribute__((always_inline)) {
+          constexpr int n = decltype(N)::value;
+          if constexpr (n == NA - 4) offsets(0), offsets(1);
+          if constexpr (n == NA || n == 2 * NA) scores_settle<ONE_WAVE>();
+          if constexpr (n >= NA && n < 2 * NA)
+            [&]<int... E>(std::integer_sequence<int, E...>) __attribute__((always_inline)) {
+              (element(std::integral_constant<int, 0>{}, std::integral_constant<int, (n - NA) * EA + E>{}), ...);
+            }(std::make_integer_sequence<int, EA>{});
+          if constexpr (n >= 2 * NA && n < 2 * NA + NC)
+            [&]<int... E>(std::integer_sequence<int, E...>) __attribute__((always_inline)) {
+              (element(std::integral_constant<int, 1>{}, std::integral_constant<int, (n - 2 * NA) * EC + E>{}), ...);
+            }(std::make_integer_sequence<int, EC>{});
+        });
+  };
+  auto next = [&](int kb) __attribute__((always_inline)) {
     block_barrier();
     keep_in_loop(lrow, lcol);
     if (kb + 1 < nkb) issue(kb + 1);
-    const char* ks = lds + (kb & 1) * 2 * B::BYTES;
+    return lds + (kb & 1) * 2 * B::BYTES;
+  };
+  // blocks whose keys all of the wave's queries see (a loop of its own: two ways through one loop would move the accumulators about)
+  int kb = 0;
+  const int whole = !kInterleaveDq<D> || a.mask || q0 >= a.L ? 0 : min(a.causal ? (q0 + 1) / ROWS : nkb, a.S / ROWS);
+  if constexpr (kInterleaveDq<D>)
+    for (; kb < whole; ++kb) {
+      const char* ks = next(kb);
+      both(ks, ks + B::BYTES, reinterpret_cast<const float*>(lds + 4 * B::BYTES) + (kb & 1) * 64);
+    }
+  for (; kb < nkb; ++kb) {
+    const char* ks = next(kb);
     const char* vs = ks + B::BYTES;
 #pragma unroll
     for (int h = 0; h < NH; ++h) {
@@ -538,10 +663,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dq_wave
         for (int db = 0; db < DB; ++db) acc[db] = Op<T>::mma(B::cols(ks, lcol, h, m, db), df[m], acc[db]);
     }
   }
-  if (query < a.L) {
-#pragma unroll
-    for (int db = 0; db < DB; ++db) store_acc<T>(a.dq + it.q + (long)query * a.q_l, db, g, acc[db], a.scale);
-  }
+  block_barrier();  // every wave has left the last block
+  store_rows<T, D>(lds + wave * 32 * B::PITCH, acc, a.scale, a.dq + it.q + q0 * a.q_l, a.q_l, a.L - q0, lane);
 }
 
 // Key pass.  Scores are formed as S[query][key] (A = Q rows, B = K rows), so a lane is a KEY and its 16 accumulator
@@ -591,11 +714,73 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dkv_wav
 #pragma unroll
     for (int r = 0; r < 16; ++r) dk[db][r] = dv[db][r] = 0.0f;
 
-  for (int qb = first; qb < nqb; ++qb) {
+  // Both groups of a block, all of whose queries see all of the wave's keys: the vector work on the first group's scores lies under the
+  // products that form the second's, and that on the second's under the products that use the first's.
+  auto both = [&](const char* qs, const char* gs, const float* stat) __attribute__((always_inline)) {
+    constexpr int NA = 2 * NK, NC = 2 * NM * DB, EA = 16 / NA, EC = 16 / NC;
+    constexpr bool ONE_WAVE = dkv_waves<T, D>() == 1;
+    f32x16 s[2], dp[2];
+    Frag pf[2][NM], df[2][NM];
+    f32x4 off[2], delta[2];
+    auto stats = [&](int quarter) __attribute__((always_inline)) {  // of the block's queries: eight, four of them this lane's
+      off[quarter & 1] = *reinterpret_cast<const f32x4*>(stat + 8 * quarter + 4 * g);
+      delta[quarter & 1] = *reinterpret_cast<const f32x4*>(stat + 64 + 8 * quarter + 4 * g);
+    };
+    auto element = [&](auto Hc, auto R) __attribute__((always_inline)) {
+      constexpr int h = decltype(Hc)::value, r = decltype(R)::value;
+      const float p = __builtin_amdgcn_exp2f(fmaf(s[h][r], a.scale, kb - off[r / 4 & 1][r % 4]) * kLog2e);
+      const float ds = p * (dp[h][r] - delta[r / 4 & 1][r % 4]);
+      constexpr int MR = Op<T>::MR;
+      pf[h][r / MR][r % MR] = from_f32<T>(p);
+      df[h][r / MR][r % MR] = from_f32<T>(ds);
+      if constexpr (r % 4 == 3 && 4 * h + r / 4 + 2 < 8) stats(4 * h + r / 4 + 2);
+    };
+    mfma_stream<Frag, 2 * NA + 2 * NC, kAhead<D>>(
+        [&](auto N) __attribute__((always_inline)) {
+          constexpr int n = decltype(N)::value, c = n - 2 * NA, w = n & 1;
+          if constexpr (n < 2 * NA)
+            return B::rows(w ? gs : qs, lrow, n / NA, n % NA / 2);
+          else
+            return B::cols(w ? qs : gs, lcol, c / NC, c % NC / (2 * DB), c % (2 * DB) / 2);
+        },
+        [&](auto N, const Frag& f) __attribute__((always_inline)) {
+          constexpr int n = decltype(N)::value, c = n - 2 * NA, w = n & 1;
+          if constexpr (n < 2 * NA) {
+            constexpr int h = n / NA, i = n % NA / 2;
+            if constexpr (w)
+              mma_scores<ONE_WAVE, i == 0>(f, vf[i], dp[h]);
+            else
+              mma_scores<ONE_WAVE, i == 0>(f, kf[i], s[h]);
+          } else {
+            constexpr int h = c / NC, m = c % NC / (2 * DB), db = c % (2 * DB) / 2;
+            if constexpr (w)
+              dk[db] = Op<T>::mma(f, df[h][m], dk[db]);
+            else
+              dv[db] = Op<T>::mma(f, pf[h][m], dv[db]);
+          }
+        },
+        [&](auto N) __attribute__((always_inline)) {
+          constexpr int n = decltype(N)::value;
+          if constexpr (n == NA - 4) stats(0), stats(1);
+          if constexpr (n == NA || n == 2 * NA) scores_settle<ONE_WAVE>();
+          if constexpr (n >= NA && n < 2 * NA)
+            [&]<int... E>(std::integer_sequence<int, E...>) __attribute__((always_inline)) {
+              (element(std::integral_constant<int, 0>{}, std::integral_constant<int, (n - NA) * EA + E>{}), ...);
+            }(std::make_integer_sequence<int, EA>{});
+          if constexpr (n >= 2 * NA && n < 2 * NA + NC)
+            [&]<int... E>(std::integer_sequence<int, E...>) __attribute__((always_inline)) {
+              (element(std::integral_constant<int, 1>{}, std::integral_constant<int, (n - 2 * NA) * EC + E>{}), ...);
+            }(std::make_integer_sequence<int, EC>{});
+        });
+  };
+  auto next = [&](int qb) __attribute__((always_inline)) {
     block_barrier();
     keep_in_loop(lrow, lcol);
     if (qb + 1 < nqb) issue(qb + 1);
-    const char* qs = lds + (qb & 1) * 2 * B::BYTES;
+    return lds + (qb & 1) * 2 * B::BYTES;
+  };
+  auto any = [&](int qb) __attribute__((always_inline)) {
+    const char* qs = next(qb);
     const char* gs = qs + B::BYTES;
     const float* stat = reinterpret_cast<const float*>(lds + 4 * B::BYTES) + (qb & 1) * 128;
 #pragma unroll
@@ -630,14 +815,21 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dkv_wav
           dk[db] = Op<T>::mma(B::cols(qs, lcol, h, m, db), df[m], dk[db]);
         }
     }
-  }
-  if (key < a.S) {
-#pragma unroll
-    for (int db = 0; db < DB; ++db) {
-      store_acc<T>(a.dk + it.k + (long)key * a.k_l, db, g, dk[db], a.scale);
-      store_acc<T>(a.dv + it.k + (long)key * a.k_l, db, g, dv[db], 1.0f);
+  };
+  // blocks whose queries all see all of the wave's keys (loops of their own: two ways through one loop would move the accumulators about)
+  const int whole0 = !kInterleaveDkv<D> || a.mask || k0 >= a.S ? nqb : a.causal ? (k0 + 31 + ROWS - 1) / ROWS : first, whole1 = a.L / ROWS;
+  int qb = first;
+  if constexpr (kInterleaveDkv<D>)
+    for (; qb < min(whole0, nqb); ++qb) any(qb);
+  if constexpr (kInterleaveDkv<D>)
+    for (; qb < whole1; ++qb) {
+      const char* qs = next(qb);
+      both(qs, qs + B::BYTES, reinterpret_cast<const float*>(lds + 4 * B::BYTES) + (qb & 1) * 128);
     }
-  }
+  for (; qb < nqb; ++qb) any(qb);
+  block_barrier();  // every wave has left the last block
+  store_rows<T, D>(lds + wave * 64 * B::PITCH, dk, a.scale, a.dk + it.k + k0 * a.k_l, a.k_l, a.S - k0, lane);
+  store_rows<T, D>(lds + (wave * 64 + 32) * B::PITCH, dv, 1.0f, a.dv + it.k + k0 * a.k_l, a.k_l, a.S - k0, lane);
 }
 
 static constexpr int64_t kFlashMaxLen = 1 << 20;

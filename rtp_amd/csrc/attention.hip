@@ -99,9 +99,9 @@ __device__ __forceinline__ bf16x8 gather_natural(const bf16_t* tile, int pitch, 
   return join(lds_transposed4(tile, pitch, 16 * m + 8 * g, c, t), lds_transposed4(tile, pitch, 16 * m + 8 * g + 4, c, t));
 }
 
-// Accumulator (rows = feature dd, columns = sequence position li) -> dst[li][32*db + dd], 4 consecutive dd
-// (8 bytes) per store.
-__device__ __forceinline__ void store_transposed(bf16_t* dst_row, int db, int g, const f32x16& acc) {
+// Accumulator (rows = feature dd, columns = sequence position li) -> columns 32*db .. of a tile's row li, 4 consecutive dd (8 bytes) per
+// store.  The tile is the operand whose columns 32*db .. the product has just read: its results take their place.
+__device__ __forceinline__ void put_transposed(bf16_t* tile, int pitch, int db, int li, int g, const f32x16& acc) {
 #pragma unroll
   for (int a4 = 0; a4 < 4; ++a4) {
     union {
@@ -110,7 +110,20 @@ __device__ __forceinline__ void store_transposed(bf16_t* dst_row, int db, int g,
     } pk;
 #pragma unroll
     for (int e = 0; e < 4; ++e) pk.e[e] = from_f32<bf16_t>(acc[4 * a4 + e]);
-    *reinterpret_cast<uint2*>(dst_row + 32 * db + 8 * a4 + 4 * g) = pk.u;
+    *reinterpret_cast<uint2*>(tile + li * pitch + 32 * db + 8 * a4 + 4 * g) = pk.u;
+  }
+}
+// The tile's `rows` rows of D elements -> memory, 16 bytes a lane, whole lines.  (Straight from the accumulators, 16 bytes of each of 32 rows
+// an instruction, the L2 takes four times as many requests.)
+template <int D>
+__device__ __forceinline__ void store_tile_rows(const bf16_t* tile, bf16_t* dst, long stride, int rows, int lane) {
+  constexpr int P = D + 8, CPR = D / 8;
+  wave_lds_fence();
+#pragma unroll
+  for (int i = 0; i < CPR / 2; ++i) {
+    const int row = (i * 64 + lane) / CPR, c = lane % CPR;
+    const uint4 v = *reinterpret_cast<const uint4*>(tile + row * P + c * 8);
+    if (row < rows) *reinterpret_cast<uint4*>(dst + row * stride + c * 8) = v;
   }
 }
 
@@ -259,8 +272,9 @@ __global__ __launch_bounds__(NWV * 64) void attn_fwd_small_kernel(AttnArgs a) {
 #pragma unroll
     for (int m = 0; m < 2; ++m)
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gather_acc_order(Vs, P, 32 * db, m, lane), pb[m], acc, 0, 0, 0);
-    if (pr.live && qlive) store_transposed(a.o + pr.o_off + li * a.o_l, db, g, acc);
+    put_transposed(Vs, P, db, li, g, acc);
   }
+  store_tile_rows<D>(Vs, a.o + pr.o_off, a.o_l, pr.live ? a.L : 0, lane);
 }
 
 template <int DB, int NWV>
@@ -350,7 +364,6 @@ __global__ __launch_bounds__(NWV * 64) void attn_bwd_small_kernel(AttnArgs a) {
   }
   __syncthreads();
 
-  const bool store = pr.live && qlive;  // li is the query for dQ and the key for dK / dV; both run to L
 #pragma unroll
   for (int db = 0; db < DB; ++db) {
     f32x16 acc;
@@ -360,7 +373,7 @@ __global__ __launch_bounds__(NWV * 64) void attn_bwd_small_kernel(AttnArgs a) {
 #pragma unroll
     for (int m = 0; m < 2; ++m)
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gather_acc_order(Ks, P, 32 * db, m, lane), dsb[m], acc, 0, 0, 0);
-    if (store) store_transposed(a.dq + pr.qkv_off + li * a.s_l, db, g, acc);
+    put_transposed(Ks, P, db, li, g, acc);
     // dK^T[dd][key] = sum_query Q[query][dd] dS[query][key]
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
@@ -368,7 +381,7 @@ __global__ __launch_bounds__(NWV * 64) void attn_bwd_small_kernel(AttnArgs a) {
     for (int m = 0; m < 2; ++m)
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gather_natural(Qs, P, 32 * db, m, lane),
                                                     gather_natural(DSs, kPPitch, 0, m, lane), acc, 0, 0, 0);
-    if (store) store_transposed(a.dk + pr.qkv_off + li * a.s_l, db, g, acc);
+    put_transposed(Qs, P, db, li, g, acc);
     // dV^T[dd][key] = sum_query dO[query][dd] P[query][key]
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
@@ -376,9 +389,20 @@ __global__ __launch_bounds__(NWV * 64) void attn_bwd_small_kernel(AttnArgs a) {
     for (int m = 0; m < 2; ++m)
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gather_natural(Gs, P, 32 * db, m, lane),
                                                     gather_natural(Ps, kPPitch, 0, m, lane), acc, 0, 0, 0);
-    if (store) store_transposed(a.dv + pr.qkv_off + li * a.s_l, db, g, acc);
+    put_transposed(Gs, P, db, li, g, acc);
   }
+  const int rows = pr.live ? a.L : 0;  // li was the query for dQ and the key for dK / dV; both run to L
+  store_tile_rows<D>(Ks, a.dq + pr.qkv_off, a.s_l, rows, lane);
+  store_tile_rows<D>(Qs, a.dk + pr.qkv_off, a.s_l, rows, lane);
+  store_tile_rows<D>(Gs, a.dv + pr.qkv_off, a.s_l, rows, lane);
 }
+
+// Problems (waves) per workgroup.  One wave's 14 - 24 KiB of LDS at D = 64 fit beside the 121 - 129 KiB that a product's workgroup on another
+// stream holds, where four waves' 55 - 94 KiB wait for it to leave the CU, and a problem's loads do not wait for its neighbours'.  Many small
+// problems are set up faster in groups.  us forward / backward with 1, 2 and 4 a workgroup (before: 4, results by 8-byte stores): 1024 problems of 32 x
+// 64 6.2 / 11.1, 6.9 / 10.9, 6.4 / 11.3 (7.2 / 13.1), 3072 of them 16.9 / 26.5, 16.2 / 24.9, 15.6 / 29.7 (17.9 / 35.1); 2048 of 32 x 128 19.4 /
+// 33.5, 19.2 / 34.1, 21.5 / 34.1 (26.4 / 41.2); of 32 x 32 1024 5.4 / 7.8, 5.1 / 6.9, 5.1 / 6.8, 4096 16.9 / 26.7, 13.5 / 25.5, 12.6 / 21.7 (14.7 / 25.2).
+static int small_waves(int64_t nprob, int64_t D) { return D == 32 ? 4 : D == 64 && nprob > 2048 ? 2 : 1; }
 
 static bool aligned8(int64_t v) { return v % 8 == 0; }
 
@@ -421,13 +445,16 @@ extern "C" int rtp_attn_fwd(void* stream, int dtype, const void* q, const void* 
   hipStream_t st = (hipStream_t)stream;
   const double np = (double)a.nprob;
   ProfileScope prof(st, "attn_fwd_small", 4.0 * np * L * L * D, np * (4.0 * L * D + (double)L * L) * 2.0);
-  const unsigned grid = (unsigned)ceil_div(a.nprob, 4);
+  const int waves = small_waves(a.nprob, D);
+  const dim3 grid((unsigned)ceil_div(a.nprob, waves)), block(64 * waves);
   if (D == 32)
-    hipLaunchKernelGGL((attn_fwd_small_kernel<1, 4>), dim3(grid), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((attn_fwd_small_kernel<1, 4>), grid, block, 0, st, a);
+  else if (D == 64 && waves == 2)
+    hipLaunchKernelGGL((attn_fwd_small_kernel<2, 2>), grid, block, 0, st, a);
   else if (D == 64)
-    hipLaunchKernelGGL((attn_fwd_small_kernel<2, 4>), dim3(grid), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((attn_fwd_small_kernel<2, 1>), grid, block, 0, st, a);
   else
-    hipLaunchKernelGGL((attn_fwd_small_kernel<4, 4>), dim3(grid), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((attn_fwd_small_kernel<4, 1>), grid, block, 0, st, a);
   RTP_LAUNCH_CHECK();
   return RTP_OK;
 }
@@ -451,12 +478,16 @@ extern "C" int rtp_attn_bwd(void* stream, int dtype, const void* q, const void* 
   hipStream_t st = (hipStream_t)stream;
   const double np = (double)a.nprob;
   ProfileScope prof(st, "attn_bwd_small", 8.0 * np * L * L * D, np * (7.0 * L * D + (double)L * L) * 2.0);
+  const int waves = small_waves(a.nprob, D);
+  const dim3 grid((unsigned)ceil_div(a.nprob, waves)), block(64 * waves);
   if (D == 32)
-    hipLaunchKernelGGL((attn_bwd_small_kernel<1, 4>), dim3((unsigned)ceil_div(a.nprob, 4)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((attn_bwd_small_kernel<1, 4>), grid, block, 0, st, a);
+  else if (D == 64 && waves == 2)
+    hipLaunchKernelGGL((attn_bwd_small_kernel<2, 2>), grid, block, 0, st, a);
   else if (D == 64)
-    hipLaunchKernelGGL((attn_bwd_small_kernel<2, 4>), dim3((unsigned)ceil_div(a.nprob, 4)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((attn_bwd_small_kernel<2, 1>), grid, block, 0, st, a);
   else
-    hipLaunchKernelGGL((attn_bwd_small_kernel<4, 2>), dim3((unsigned)ceil_div(a.nprob, 2)), dim3(128), 0, st, a);
+    hipLaunchKernelGGL((attn_bwd_small_kernel<4, 1>), grid, block, 0, st, a);
   RTP_LAUNCH_CHECK();
   return RTP_OK;
 }

@@ -137,6 +137,13 @@ __device__ __forceinline__ unsigned fast_div(unsigned n, const FastDiv& f) {
   return (t + ((n - t) >> f.s1)) >> f.s2;
 }
 
+// What lanes of this wave have written to LDS is read by its other lanes behind it (no instruction: a wave's LDS accesses happen in order).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // A kernel's arguments, its only ones, after every 64-byte line of them has been requested in one batch.  The scalar cache is cold at kernel

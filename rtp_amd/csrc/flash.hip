@@ -185,6 +185,7 @@ __device__ __forceinline__ void store_rows(char* own, const f32x16 (&acc)[D / 32
       for (int i = 0; i < 4; ++i) e[i] = from_f32<T>(acc[db][4 * a4 + i] * scale);
       *reinterpret_cast<uint2*>(own + li * PITCH + (((4 * db + a4) ^ (li % CPR)) << 4) + 8 * g) = *reinterpret_cast<const uint2*>(e);
     }
+  wave_lds_fence();
 #pragma unroll
   for (int i = 0; i < CPR / 2; ++i) {
     const int row = (i * 64 + lane) / CPR, chunk = lane % CPR;

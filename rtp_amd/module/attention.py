@@ -344,9 +344,15 @@ def _shard_inputs_grad(sums, flat, e_s, c0, i) -> None:
     """The run's part of the three projections' input gradients; an entry of `sums` is None where nobody asks for it."""
     for item in sums:
         if item is not None:
-            _, acc, src, width, w_off = item
+            _, acc, src, width, w_off, blocks = item
             c_out, c_in = acc.target(i)
-            S.col_dgrad(src, flat, w_off, e_s, width, c_out, c0, c_in=c_in)
+            S.col_dgrad(src, flat, w_off, blocks * e_s, width, c_out, blocks * c0, c_in=c_in)
+
+
+def _columns_from(k: int, v: int, width: int):
+    """Equally many columns of k's and v's rows from the given ones on (the core's entry points take one offset into all operands)."""
+    n = width - max(k, v)
+    return slice(k, k + n), slice(v, v + n)
 
 
 class _GeneralAttentionFn(torch.autograd.Function):
@@ -354,7 +360,10 @@ class _GeneralAttentionFn(torch.autograd.Function):
     [S, N, vdim]; functional.py:575-609 projects them with three row blocks of the shard), optionally with the
     learned key / value bias_k / bias_v (add_bias_kv, functional.py:711-716) and then one all-zero key / value
     (add_zero_attn, functional.py:746-753) appended per batch entry.  Three projections per shard run into
-    q [L*N, E], k and v [(S+z)*N, E] (group g at column block g; z appended positions); the core is the running-softmax
+    q [L*N, E], k and v [(S+z)*N, E] (group g at column block g; z appended positions).  Where keys and values are the same tensor
+    (value None: a decoder's attention over the encoder's states) its two projections are one of 2 e_s rows a shard into [S*N, 2E], group g's k and v
+    side by side, and so are their input and weight gradients: three launches and autograd's sum less (16 sequences of 100 / 180, 8
+    heads of 64, fp32, forward and backward: 280 -> 255 us).  The core is the running-softmax
     launch, or, in fp32, with dropout, per-head masks, masks given as floats or the weights wanted back, batched products and
     the softmax kernel with p [ws*N*h_s, L, S+z] in memory.
 
@@ -372,14 +381,17 @@ class _GeneralAttentionFn(torch.autograd.Function):
         sk = s_in + bkv + zero
         ws, h_s, d, e_s = layer.world_size, layer.num_heads_per_partition, layer.head_dim, layer.embed_dim_per_partition
         dt, dev = query.dtype, query.device
-        q2, k2, v2 = as_rows(query, E), as_rows(key, layer.kdim), as_rows(value, layer.vdim)
+        shared = value is None
+        q2, k2 = as_rows(query, E), as_rows(key, layer.kdim)
+        v2 = k2 if shared else as_rows(value, layer.vdim)
         wq, wk, wv, b_in, w_o, b_o = _shard_layout(layer)
         bq, bk, bv = (b_in, b_in + e_s, b_in + 2 * e_s) if b_in is not None else (None, None, None)
         Z = N * h_s
         scale = 1.0 / math.sqrt(d)
         qb = torch.empty(L * N, E, dtype=dt, device=dev)
-        kb = torch.empty(sk * N, E, dtype=dt, device=dev)
-        vb = torch.empty(sk * N, E, dtype=dt, device=dev)
+        width = 2 * E if shared else E  # of a row of k and v
+        kb = torch.empty(sk * N, width, dtype=dt, device=dev)
+        vb = kb if shared else torch.empty(sk * N, E, dtype=dt, device=dev)
         if zero:
             kb[(s_in + bkv) * N:].zero_()
             vb[(s_in + bkv) * N:].zero_()
@@ -394,7 +406,8 @@ class _GeneralAttentionFn(torch.autograd.Function):
             p = torch.empty(ws * Z, L, sk, dtype=dt, device=dev)
         drop = torch.empty(ws * Z, L, sk, dtype=torch.float32, device=dev) if drop_p > 0.0 else None
         pv = torch.empty_like(p) if drop_p > 0.0 else p
-        ld = N * E  # one step along the sequence in q, k, v and o
+        ld = N * E  # one step along the sequence in q and o
+        kv_ld, kv_s, kv_g = N * width, (width, d), 2 * e_s if shared else e_s  # ... in k and v; batch and head, group
         bmm = ops.native().bmm
         rot = rotation(store, layer.rank)
         acc = ops.ShardSum(out, sum(len(w) for w in rot.windows))
@@ -403,20 +416,24 @@ class _GeneralAttentionFn(torch.autograd.Function):
             for flat, first, cnt in rot.acquire(j):
                 c0 = first * e_s
                 S.col_fwd(q2, flat, wq, e_s, E, bq, qb, c0)
-                S.col_fwd(k2, flat, wk, e_s, layer.kdim, bk, kb[:s_in * N], c0)
-                S.col_fwd(v2, flat, wv, e_s, layer.vdim, bv, vb[:s_in * N], c0)
+                k0, v0 = (2 * c0, 2 * c0 + e_s) if shared else (c0, c0)  # the first group's columns of k and v
+                S.col_fwd(k2, flat, wk, kv_g, layer.kdim, bk, kb[:s_in * N], k0)
+                if not shared:
+                    S.col_fwd(v2, flat, wv, e_s, layer.vdim, bv, vb[:s_in * N], c0)
                 if bkv:  # position s_in of every batch entry: the head groups' slices of bias_k / bias_v
                     kb[s_in * N:(s_in + 1) * N, c0:c0 + cnt * e_s] = flat[:, bk_off:bk_off + e_s].reshape(1, cnt * e_s)
                     vb[s_in * N:(s_in + 1) * N, c0:c0 + cnt * e_s] = flat[:, bv_off:bv_off + e_s].reshape(1, cnt * e_s)
                 if flash:
-                    ops.attn_flash_kv_fwd(qb, kb, vb, o, c0, (ld, E, d, e_s), (ld, E, d, e_s), p[first * Z:(first + cnt) * Z],
+                    k_at, v_at = _columns_from(k0 - c0, v0 - c0, width)
+                    ops.attn_flash_kv_fwd(qb, kb[:, k_at], vb[:, v_at], o, c0, (ld, E, d, e_s),
+                                          (kv_ld, width, d, kv_g), p[first * Z:(first + cnt) * Z],
                                           mask, scale, L, sk, N, h_s, d, cnt, key_bias=key_bias)
                     c_out, c_in = acc.target(i)
                     S.row_fwd(o, flat, w_o, E, e_s, b_o, c_out, c0, c_in=c_in)
                     i += 1
                     continue
                 scores = torch.empty(cnt * Z, L, sk, dtype=torch.float32, device=dev)
-                bmm(qb, c0, ld, True, (E, d), e_s, kb, c0, ld, True, (E, d), e_s,
+                bmm(qb, c0, ld, True, (E, d), e_s, kb, k0, kv_ld, True, kv_s, kv_g,
                     scores, 0, sk, (h_s * L * sk, L * sk), Z * L * sk, L, sk, d, Z, h_s, cnt)
                 if drop is not None:
                     ops.softmax_fwd(scores, p[first * Z:(first + cnt) * Z], mask=mask, causal=False, scale=scale,
@@ -428,7 +445,7 @@ class _GeneralAttentionFn(torch.autograd.Function):
                                     key_bias=key_bias, heads=h_s)
                 del scores
                 bmm(pv, first * Z * L * sk, sk, True, (h_s * L * sk, L * sk), Z * L * sk,
-                    vb, c0, ld, False, (E, d), e_s, o, c0, ld, (E, d), e_s, L, d, sk, Z, h_s, cnt)
+                    vb, v0, kv_ld, False, kv_s, kv_g, o, c0, ld, (E, d), e_s, L, d, sk, Z, h_s, cnt)
                 c_out, c_in = acc.target(i)
                 S.row_fwd(o, flat, w_o, E, e_s, b_o, c_out, c0, c_in=c_in)
                 i += 1
@@ -439,6 +456,7 @@ class _GeneralAttentionFn(torch.autograd.Function):
             weights = pv[last * Z:(last + 1) * Z].view(N, h_s, L, sk)
         ctx.layer = layer
         ctx.dims = (L, N, E, s_in, sk)
+        ctx.shared = shared
         ctx.flash = (mask, key_bias) if flash else None
         ctx.dropped = drop is not None
         ctx.save_for_backward(q2, k2, v2, qb, kb, vb, p, o, *((drop, pv) if drop is not None else ()))
@@ -462,8 +480,11 @@ class _GeneralAttentionFn(torch.autograd.Function):
         dout2 = as_rows(dout, E)
         do = torch.empty(L * N, E, dtype=dt, device=dev)
         dqb = torch.empty(L * N, E, dtype=dt, device=dev)
-        dkb = torch.empty(sk * N, E, dtype=dt, device=dev)
-        dvb = torch.empty(sk * N, E, dtype=dt, device=dev)
+        shared = ctx.shared
+        width = 2 * E if shared else E
+        kv_ld, kv_s, kv_g = N * width, (width, d), 2 * e_s if shared else e_s
+        dkb = torch.empty(sk * N, width, dtype=dt, device=dev)
+        dvb = dkb if shared else torch.empty(sk * N, E, dtype=dt, device=dev)
         delta = torch.empty_like(p) if ctx.flash is not None else None
         bmm = ops.native().bmm
         rot = rotation(store, layer.rank, reverse=True)
@@ -471,44 +492,47 @@ class _GeneralAttentionFn(torch.autograd.Function):
         # input gradients of the three projections, each summed over the shards; the rows of an appended zero key
         # belong to no input
         sums = []
-        for need, src, rows, width, w_off in ((ctx.needs_input_grad[0], dqb, L * N, E, wq),
-                                              (ctx.needs_input_grad[1], dkb, s_in * N, layer.kdim, wk),
-                                              (ctx.needs_input_grad[2], dvb, s_in * N, layer.vdim, wv)):
+        for need, src, rows, n_in, w_off, blocks in ((ctx.needs_input_grad[0], dqb, L * N, E, wq, 1),
+                                                     (ctx.needs_input_grad[1], dkb, s_in * N, layer.kdim, wk, 2 if shared else 1),
+                                                     (ctx.needs_input_grad[2], dvb, s_in * N, layer.vdim, wv, 1)):
             if need:
-                dx = torch.empty(rows, width, dtype=dt, device=dev)
-                sums.append((dx, ops.ShardSum(dx, parts), src[:rows], width, w_off))
+                dx = torch.empty(rows, n_in, dtype=dt, device=dev)
+                sums.append((dx, ops.ShardSum(dx, parts), src[:rows], n_in, w_off, blocks))
             else:
                 sums.append(None)
         i = 0
         for j in range(rot.steps):
             for flat, first, cnt in rot.acquire(j):
                 c0 = first * e_s
+                k0, v0 = (2 * c0, 2 * c0 + e_s) if shared else (c0, c0)
                 p_off = first * Z * L * sk
                 p_s, p_sg = (h_s * L * sk, L * sk), Z * L * sk
                 S.row_dgrad(dout2, flat, w_o, E, e_s, do, c0)
                 if ctx.flash is not None:
-                    ops.attn_flash_kv_bwd(qb, kb, vb, o, do, c0, (ld, E, d, e_s), (ld, E, d, e_s),
-                                          p[first * Z:(first + cnt) * Z], delta[first * Z:(first + cnt) * Z], dqb, dkb, dvb,
+                    k_at, v_at = _columns_from(k0 - c0, v0 - c0, width)
+                    ops.attn_flash_kv_bwd(qb, kb[:, k_at], vb[:, v_at], o, do, c0, (ld, E, d, e_s),
+                                          (kv_ld, width, d, kv_g), p[first * Z:(first + cnt) * Z],
+                                          delta[first * Z:(first + cnt) * Z], dqb, dkb[:, k_at], dvb[:, v_at],
                                           ctx.flash[0], scale, L, sk, N, h_s, d, cnt, key_bias=ctx.flash[1])
                     _shard_inputs_grad(sums, flat, e_s, c0, i)
                     i += 1
                     continue
                 # dP = dO V^T
                 dp = torch.empty(cnt * Z, L, sk, dtype=torch.float32, device=dev)
-                bmm(do, c0, ld, True, (E, d), e_s, vb, c0, ld, True, (E, d), e_s, dp, 0, sk, p_s, p_sg,
+                bmm(do, c0, ld, True, (E, d), e_s, vb, v0, kv_ld, True, kv_s, kv_g, dp, 0, sk, p_s, p_sg,
                     L, sk, d, Z, h_s, cnt)
                 # dV = P^T dO
-                bmm(pv, p_off, sk, False, p_s, p_sg, do, c0, ld, False, (E, d), e_s, dvb, c0, ld, (E, d), e_s,
+                bmm(pv, p_off, sk, False, p_s, p_sg, do, c0, ld, False, (E, d), e_s, dvb, v0, kv_ld, kv_s, kv_g,
                     sk, d, L, Z, h_s, cnt)
                 ds = torch.empty(cnt * Z, L, sk, dtype=dt, device=dev)
                 ops.softmax_bwd(p[first * Z:(first + cnt) * Z], dp, ds, scale,
                                 keep=None if drop is None else drop[first * Z:(first + cnt) * Z])
                 del dp
                 # dQ = dS K
-                bmm(ds, 0, sk, True, p_s, p_sg, kb, c0, ld, False, (E, d), e_s, dqb, c0, ld, (E, d), e_s,
+                bmm(ds, 0, sk, True, p_s, p_sg, kb, k0, kv_ld, False, kv_s, kv_g, dqb, c0, ld, (E, d), e_s,
                     L, d, sk, Z, h_s, cnt)
                 # dK = dS^T Q
-                bmm(ds, 0, sk, False, p_s, p_sg, qb, c0, ld, False, (E, d), e_s, dkb, c0, ld, (E, d), e_s,
+                bmm(ds, 0, sk, False, p_s, p_sg, qb, c0, ld, False, (E, d), e_s, dkb, k0, kv_ld, kv_s, kv_g,
                     sk, d, L, Z, h_s, cnt)
                 _shard_inputs_grad(sums, flat, e_s, c0, i)
                 i += 1
@@ -521,8 +545,11 @@ class _GeneralAttentionFn(torch.autograd.Function):
                 c0 = first * e_s
                 S.row_wgrad(dout2, o, store.grads, first, w_o, E, e_s, c0, cnt, accumulate, b_off=b_o, store=store)
                 S.col_wgrad(dqb, q2, store.grads, first, wq, e_s, E, c0, cnt, accumulate, b_off=bq, store=store)
-                S.col_wgrad(dk_in, k2, store.grads, first, wk, e_s, layer.kdim, c0, cnt, accumulate, b_off=bk, store=store)
-                S.col_wgrad(dv_in, v2, store.grads, first, wv, e_s, layer.vdim, c0, cnt, accumulate, b_off=bv, store=store)
+                S.col_wgrad(dk_in, k2, store.grads, first, wk, kv_g, layer.kdim, 2 * c0 if shared else c0, cnt, accumulate,
+                            b_off=bk, store=store)
+                if not shared:
+                    S.col_wgrad(dv_in, v2, store.grads, first, wv, e_s, layer.vdim, c0, cnt, accumulate, b_off=bv,
+                                store=store)
                 if layer.add_bias_kv:
                     # the appended position's key / value gradient, summed over the batch entries it was copied to
                     bk_off, bv_off = _bias_kv_layout(layer)
@@ -621,6 +648,8 @@ class ParallelMultiheadAttention(RotatedLayer):
         if general:
             if residual_grad:
                 raise ValueError("residual_grad is for self-attention (the residual is the attention's own input)")
+            # one tensor's two projections side by side, unless they are weights of their own or positions are appended
+            shared = key is value and not (self.separate_proj or self.add_zero_attn or self.add_bias_kv)
             k_in, v_in = (key.transpose(0, 1), value.transpose(0, 1)) if self.batch_first else (key, value)
             if k_in.shape[0] != v_in.shape[0] or k_in.shape[1] != x.shape[1] or v_in.shape[1] != x.shape[1] or \
                     x.shape[2] != self.embed_dim or k_in.shape[2] != self.kdim or v_in.shape[2] != self.vdim:
@@ -636,7 +665,7 @@ class ParallelMultiheadAttention(RotatedLayer):
                 if key_bias is not None:
                     key_bias = F.pad(key_bias, (0, extra))
             hides_only = all(m is None or m.dtype == torch.bool for m in (attn_mask, key_padding_mask))
-            out, weights = apply_function(_GeneralAttentionFn, x, k_in, v_in, self._anchor, self, mask, key_bias,
+            out, weights = apply_function(_GeneralAttentionFn, x, k_in, None if shared else v_in, self._anchor, self, mask, key_bias,
                                           bool(need_weights), drop_p, hides_only)
         else:
             out, weights = apply_function(_AttentionFn, x, self._anchor, self, mask, causal, bool(need_weights),

@@ -242,29 +242,39 @@ struct AdamChunk {
   float *exp_avg, *exp_avg_sq;
   long n;  // parameters in the chunk
 };
+// A chunk is dealt over kAdamParts workgroups, 1024 parameters each of a full one (16384), four a lane.  Bound by memory, which is faster
+// where the workgroups in flight walk a few MB of each array in order than with streams 64 KiB apart.  294 M parameters in bf16, 8.2 GB,
+// us: a workgroup a chunk, eight accesses in flight a lane, 1566; 2 and 4 workgroups with sixteen in flight 1517 and 1475 - 1497, 8 with eight 1505, 16 with
+// four 1417 (5.8 TB/s); 32 of 128 threads 1460, and 1462 where beta^t is worked out by squaring, so that stores follow the loads at once.
+constexpr int kAdamParts = 16;
 template <typename T>
-__global__ __launch_bounds__(256) void adam_multi_kernel(const AdamChunk* chunks, AdamScalars c) {
+__global__ __launch_bounds__(256) void adam_multi_kernel(const AdamChunk* chunks, int parts, AdamScalars c) {
   using P = typename Sgd4<T>::Pack;
-  adam_bias_corrections(c);
-  const AdamChunk ch = chunks[blockIdx.x];
+  const unsigned chunk = parts == 1 ? blockIdx.x : blockIdx.x / kAdamParts, part = parts == 1 ? 0 : blockIdx.x % kAdamParts;
+  const AdamChunk ch = chunks[chunk];
   const T* grad = reinterpret_cast<const T*>(ch.grad);
   T* shadow = reinterpret_cast<T*>(ch.shadow);
   // the moments are checked as two more arrays of the master's type
   const long head = max(chunk_head(ch.master, grad, shadow, ch.n),
                         chunk_head<float>(ch.master, ch.exp_avg, ch.exp_avg_sq, ch.n));
   const long n4 = (ch.n - head) >> 2;
-  for (long i = threadIdx.x; i < ch.n - 4 * n4; i += 256) {
-    const long k = i < head ? i : i + 4 * n4;
-    float w = ch.master[k], m = ch.exp_avg[k], v = ch.exp_avg_sq[k];
-    adam_update(w, m, v, to_f32(grad[k]), c);
-    ch.master[k] = w, ch.exp_avg[k] = m, ch.exp_avg_sq[k] = v;
-    if (shadow) shadow[k] = from_f32<T>(w);
-  }
+  const long per = ((n4 + parts - 1) / parts + 255) & ~255l, first = part * per, last = min(first + per, n4);
+  // the bias corrections of a step count in device memory are powers in fp64: one wave's work, beside the first loads
+  __shared__ float corrections[2];
+  const auto corrected = [&] {
+    if (!c.step_dev) return;
+    if (threadIdx.x < 64) {
+      adam_bias_corrections(c);
+      if (threadIdx.x == 0) corrections[0] = c.bc2_sqrt, corrections[1] = c.neg_step_size;
+    }
+    __syncthreads();
+    c.bc2_sqrt = corrections[0], c.neg_step_size = corrections[1];
+  };
   float4* master = reinterpret_cast<float4*>(ch.master + head);
   float4* m4 = reinterpret_cast<float4*>(ch.exp_avg + head);
   float4* v4 = reinterpret_cast<float4*>(ch.exp_avg_sq + head);
-  grad += head;
-  if (shadow) shadow += head;
+  const T* g4 = grad + head;
+  T* s4 = shadow ? shadow + head : nullptr;
   auto one = [&](long i, const P& g, float4 w, float4 m, float4 v) {
     float *wf = reinterpret_cast<float*>(&w), *mf = reinterpret_cast<float*>(&m), *vf = reinterpret_cast<float*>(&v);
     P sh;
@@ -274,19 +284,28 @@ __global__ __launch_bounds__(256) void adam_multi_kernel(const AdamChunk* chunks
       sh.e[e] = from_f32<T>(wf[e]);
     }
     nt_store(w, master + i), nt_store(m, m4 + i), nt_store(v, v4 + i);
-    if (shadow) Sgd4<T>::store(shadow, i, sh);
+    if (shadow) Sgd4<T>::store(s4, i, sh);
   };
-  long i = threadIdx.x;
-  for (; i + 256 < n4; i += 512) {
-    const long k = i + 256;
-    const P g0 = Sgd4<T>::load(grad, i), g1 = Sgd4<T>::load(grad, k);
-    const float4 w0 = nt_load(master + i), w1 = nt_load(master + k);
-    const float4 a0 = nt_load(m4 + i), a1 = nt_load(m4 + k);
-    const float4 b0 = nt_load(v4 + i), b1 = nt_load(v4 + k);
-    one(i, g0, w0, a0, b0);
-    one(k, g1, w1, a1, b1);
+  // the lane's four, and what they need, on their way before anything else
+  long i = first + threadIdx.x;
+  P g;
+  float4 w, m, v;
+  const auto request = [&] { g = Sgd4<T>::load(g4, i), w = nt_load(master + i), m = nt_load(m4 + i), v = nt_load(v4 + i); };
+  if (i < last) request();
+  corrected();
+  if (part == 0)
+    for (long j = threadIdx.x; j < ch.n - 4 * n4; j += 256) {
+      const long k = j < head ? j : j + 4 * n4;
+      float w1 = ch.master[k], m1 = ch.exp_avg[k], v1 = ch.exp_avg_sq[k];
+      adam_update(w1, m1, v1, to_f32(grad[k]), c);
+      ch.master[k] = w1, ch.exp_avg[k] = m1, ch.exp_avg_sq[k] = v1;
+      if (shadow) shadow[k] = from_f32<T>(w1);
+    }
+  while (i < last) {
+    one(i, g, w, m, v);
+    i += 256;
+    if (i < last) request();  // (chunks longer than the optimisers')
   }
-  for (; i < n4; i += 256) one(i, Sgd4<T>::load(grad, i), nt_load(master + i), nt_load(m4 + i), nt_load(v4 + i));
 }
 
 template <typename S, typename D>
@@ -413,10 +432,11 @@ extern "C" int rtp_adam_step_multi(void* stream, int dtype, const rtp_adam_chunk
   c.weight_decay = (float)weight_decay, c.clip = (float)clip;
   ProfileScope prof(s, "adam_step", 12.0 * total_params, total_params * (dtype == RTP_F32 ? 32.0 : 28.0));
   const AdamChunk* table = reinterpret_cast<const AdamChunk*>(chunks);
+  const int parts = n_chunks < (1ll << 31) / kAdamParts ? kAdamParts : 1;
   if (dtype == RTP_F32)
-    hipLaunchKernelGGL(adam_multi_kernel<float>, dim3((unsigned)n_chunks), dim3(256), 0, s, table, c);
+    hipLaunchKernelGGL(adam_multi_kernel<float>, dim3((unsigned)n_chunks * parts), dim3(256), 0, s, table, parts, c);
   else
-    hipLaunchKernelGGL(adam_multi_kernel<bf16_t>, dim3((unsigned)n_chunks), dim3(256), 0, s, table, c);
+    hipLaunchKernelGGL(adam_multi_kernel<bf16_t>, dim3((unsigned)n_chunks * parts), dim3(256), 0, s, table, parts, c);
   RTP_LAUNCH_CHECK();
   return RTP_OK;
 }

@@ -1,0 +1,43 @@
+"""The Adam update of many buffers: chunks of every length around the parts they are dealt over, at any alignment, with the step count
+from the host or from device memory, against adam_step on each buffer alone (the same arithmetic: the same bits)."""
+import pytest
+import torch
+
+from gpu_util import DEV
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = [1, 3, 4, 1020, 1023, 1024, 1028, 4099, 16383, 16384, 16385, 40000]
+
+
+@pytest.mark.parametrize("device_step", [False, True])
+@pytest.mark.parametrize("offset", [0, 1, 4])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_chunks_of_any_length(dtype, offset, device_step):
+    from rtp_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(offset)
+
+    def buffer(n, dt, scale=1.0):
+        return (torch.randn(n + 8, generator=gen, device=DEV) * scale).to(dt)[offset:offset + n]
+
+    step = torch.tensor([7], dtype=torch.int64, device=DEV) if device_step else 7
+    sets = []
+    for n in LENGTHS:
+        master, grad, m = buffer(n, torch.float32), buffer(n, dtype, 0.1), buffer(n, torch.float32, 0.01)
+        v = buffer(n, torch.float32, 0.01).abs()
+        shadow = master.to(dtype) if dtype != torch.float32 else None
+        sets.append((master, grad, shadow, m, v))
+    alone = [tuple(None if t is None else t.clone() for t in s) for s in sets]
+    table = ops.adam_chunk_table(sets, DEV)
+    # and one chunk longer than the optimisers make them
+    long = [buffer(100003, torch.float32), buffer(100003, dtype, 0.1), None, buffer(100003, torch.float32, 0.01),
+            buffer(100003, torch.float32, 0.01).abs()]
+    alone.append(tuple(None if t is None else t.clone() for t in long))
+    row = [0 if t is None else t.data_ptr() for t in long] + [100003]
+    table = torch.cat([table, torch.tensor([row], dtype=torch.int64, device=DEV)])
+    ops.adam_step_multi(table, dtype, step, 1e-3, (0.9, 0.999), 1e-8, 0.01, 0.05, sum(LENGTHS) + 100003)
+    for got, want in zip(sets + [tuple(long)], alone):
+        master, grad, shadow, m, v = want
+        ops.adam_step(master, grad.contiguous(), shadow, m, v, step, 1e-3, (0.9, 0.999), 1e-8, 0.01, 0.05)
+        for a, b in zip(got, want):
+            assert a is None or torch.equal(a, b)

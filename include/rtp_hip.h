@@ -220,7 +220,7 @@ int rtp_gemm(void* stream, int dtype, const rtp_gemm_desc* d);
  * step's product, rtp/module/linear.py:211-220, rtp/module/collectives.py:240-317) for shards that are read from
  * their home rows: hands `bytes` at `src` (16-byte aligned; the shards of the layer that runs next) to the next
  * product that this host thread launches through rtp_gemm or rtp_rotated_linear_* on the wave-specialised kernel.
- * That launch requests them at its start, so they sit in the GPU's memory-side cache when their own products run
+ * That launch requests them as it goes, so they sit in the GPU's memory-side cache when their own products run
  * (weights are read once per pass and would otherwise come from HBM at their turn).  Up to 192 KiB per workgroup
  * of the carrying launch.  A hint: no result depends on it; it ends with that next product launch whether or not
  * the launch could carry it: the wave-specialised kernels of tiles below 256 x 256 can, those for few tiles, for

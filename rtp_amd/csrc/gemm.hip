@@ -296,7 +296,7 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
   static_assert(NSTAGE * STAGE + 1024 <= 160 * 1024, "160 KiB of LDS per workgroup");
   static_assert(BM * (BN + 4) * 4 <= NSTAGE * STAGE, "the epilogue stages the fp32 tile in the slab memory");
   // Stage addresses are compile-time offsets into one array, so LDS reads carry immediate offsets.  The last KiB
-  // is where the loads of warm_ahead() land.
+  // is where the loads of WarmAhead land.
   __shared__ __attribute__((aligned(1024))) char lds[NSTAGE * STAGE + 1024];
 
   const int tid = threadIdx.x;
@@ -534,8 +534,10 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
       }(std::make_integer_sequence<int, NM>{});
       __builtin_amdgcn_sched_barrier(0);
     };
+    WarmAhead warm(p, (unsigned)(uintptr_t)(lptr_t)lds + NSTAGE * STAGE, id, nwg, wave, lane, nk);
     auto phase = [&](auto S, int k, auto STEADY) {
       if (!decltype(STEADY)::value && k >= nk) return;
+      warm.slab();
       [&]<int... Q>(std::integer_sequence<int, Q...>) {
         (step(S, std::integral_constant<int, Q>{}, k, STEADY), ...);
       }(std::make_integer_sequence<int, KS>{});
@@ -546,7 +548,6 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
         (phase(std::integral_constant<int, S>{}, kt + S, STEADY), ...);
       }(std::make_integer_sequence<int, NSTAGE>{});
     };
-    warm_ahead(p, (unsigned)(uintptr_t)(lptr_t)lds + NSTAGE * STAGE, id, nwg, wave, lane);
     if (!RAG || p.vec_c)
       request_epilogue<T, BM, BN>(p, (unsigned)(uintptr_t)(lptr_t)lds + NSTAGE * STAGE, m0, n0, grp, zo, zi, wave, lane);
     __builtin_amdgcn_s_barrier();  // barrier 0
@@ -942,7 +943,7 @@ static bool takes_kwaves(const rtp_gemm_desc* d) {
          d->k * d->ksegs >= 256 && !(sizeof(T) == 4 && !direct && !d->a_kcontig && !d->b_kcontig) && few_tiles<T>(d) != 0;
 }
 
-// rtp_gemm_warm_next: bytes the next product launched by this host thread requests at its start.  A later call, from any
+// rtp_gemm_warm_next: bytes the next product launched by this host thread requests beside its own.  A later call, from any
 // thread, ends an earlier hint: a caller holds the memory of the last one only, and a forward pass and its backward pass
 // run on two threads.
 static std::atomic<unsigned long long> g_warm_call{0};

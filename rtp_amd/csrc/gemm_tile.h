@@ -54,7 +54,7 @@ struct GemmArgs {
   const float2* xent_stats;     // mode 2: [m] {max, sum exp} of the whole row
   const float* xent_dloss;      // mode 2: upstream gradient, one scalar
   const float* xent_scale;      // mode 2: second scalar factor (1 / rows counted), or null
-  // bytes that some later launch will read from HBM (the next layer's shards): requested here, see warm_ahead()
+  // bytes that some later launch will read from HBM (the next layer's shards): requested here, see WarmAhead
   const char* warm;
   long warm_bytes;
   unsigned tiles, per_xcd;  // gemm_large.hip: all tiles of the launch, an XCD's share of them (rounded up)
@@ -736,26 +736,44 @@ struct DmaOperand {
 // The next layer's shards arrive while this product computes.  Weights are read once per pass, so at their turn
 // they come from HBM, whose latency the NSTAGE - 1 slabs in flight do not cover: measured on the LM's shapes, a
 // product takes 15 - 30 % longer on weights from HBM than on weights that sit in the 256 MiB memory-side cache.
-// So a product can be handed the bytes that the *next* products will need: its MFMA waves, idle until the first
-// slab has landed, request them right at kernel start, 1 KiB per instruction, straight into 1 KiB of LDS that
-// nothing reads (no registers, and nobody ever waits for these loads: an MFMA wave next waits for vector memory
-// in the epilogue).  Pieces are dealt round-robin over (workgroup, wave), so the launch as a whole reads the region
-// front to back; a wave asks for at most kWarmMax pieces (the counter of outstanding loads has 6 bits), the rest
-// of a larger region stays unread.
+// So a product can be handed the bytes that the *next* products will need: its MFMA waves request them, 1 KiB per
+// instruction, straight into 1 KiB of LDS that nothing reads (no registers, and nobody ever waits for these loads: an
+// MFMA wave next waits for vector memory in the epilogue).  Pieces are dealt round-robin over (workgroup, wave), so
+// the launch as a whole reads the region front to back; a wave asks for at most kWarmMax pieces (the counter of
+// outstanding loads has 6 bits), the rest of a larger region stays unread.  They are asked for a few a slab, over the
+// first three quarters of the K loop: all of them at the start of the kernel stood in front of its own first slabs and
+// residual or mask (the language model's step 3544 us against 3509; over a quarter of the loop 3520, half 3510, all of it
+// 3522, where the last ones are still on their way when the epilogue waits for its operands).
 constexpr int kWarmMax = 48;
-__device__ __forceinline__ void warm_ahead(const GemmArgs& p, unsigned lds_dst, unsigned wg, unsigned nwg, int wave,
-                                           int lane) {
-  if (p.warm == nullptr) return;
-  const long pieces = p.warm_bytes >> 10;
-  long piece = (long)wg * 4 + wave;
-  for (int j = 0; j < kWarmMax && piece < pieces; ++j, piece += (long)nwg * 4) {
-    const char* src = p.warm + (piece << 10) + lane * 16;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_dst), "v"(src) : "memory");
+struct WarmAhead {
+  const char* src;  // the wave's next piece
+  long step;        // bytes from one of its pieces to the next
+  unsigned off, lds_dst;
+  int left, per_slab;
+  __device__ __forceinline__ WarmAhead(const GemmArgs& p, unsigned dst, unsigned wg, unsigned nwg, int wave, int lane, int nk) {
+    const long piece = (long)wg * 4 + wave, step_pieces = (long)nwg * 4;
+    const long total = p.warm == nullptr ? 0 : p.warm_bytes >> 10;
+    const long mine = total > piece ? (total - piece + step_pieces - 1) / step_pieces : 0;
+    left = mine < kWarmMax ? (int)mine : kWarmMax;
+    const int slabs = nk > 0 ? nk - nk / 4 : 1;
+    per_slab = (left + slabs - 1) / slabs;
+    src = p.warm + (piece << 10);
+    step = step_pieces << 10;
+    off = (unsigned)lane * 16u;
+    lds_dst = dst;
   }
-}
+  __device__ __forceinline__ void slab() {
+    if (left <= 0) return;
+    for (int j = 0; j < per_slab && left > 0; ++j, --left, src += step)
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                   :
+                   : "s"(lds_dst), "v"(off), "s"(src)
+                   : "memory");
+  }
+};
 
 // Epilogue operands with vector alignment, requested by the MFMA waves before the K loop (into LDS that nothing reads, like the
-// loads of warm_ahead).
+// loads of WarmAhead).
 template <typename T, int BM, int BN>
 __device__ __forceinline__ void request_epilogue(const GemmArgs& p, unsigned lds_dst, int m0, int n0, int grp, long zo, long zi,
                                                  int wave, int lane) {

@@ -64,7 +64,7 @@ def rotation_mode() -> str:
 # product takes 15 - 30 % longer on weights from HBM than on weights that sit in the 256 MiB memory-side cache (an fp32
 # one does not, and neither it nor the kernel for few rows carries the hint that is set here).  With
 # the switch on, a rotation that starts hands the home rows of the layer that followed this one the last time round
-# to its own first product (rtp_gemm_warm_next), whose workgroups request them at their start: the one-GPU form of
+# to its own first product (rtp_gemm_warm_next), whose workgroups request them along the way: the one-GPU form of
 # the reference's irecv of the next shard during the current step (rtp/module/linear.py:211-220).  Which layer
 # follows is learned from the order of the rotations (keyed by the last two layers, so the forward and the backward
 # order are told apart); nothing depends on the guess being right.  No second stream is involved: a read pass on a

@@ -13,7 +13,7 @@
 // its rows) for the whole contraction, and everything that depends on k alone -- offset inside an image, kernel position --
 // is worked out once per slab by one thread per k and handed round through LDS.  The first version called an index function
 // with five integer divisions per element and gave every shard tiles of its own: MNIST's second convolution (64 x 32 x 26 x
-// 26 -> 64, four shards, fp32) took 127 + 162 + 196 us forward / input / weight gradient; this one takes 29 + 43 + 34.
+// 26 -> 64, four shards, fp32) took 127 + 162 + 196 us forward / input / weight gradient; this one takes 29 + 37 + 34.
 #include <algorithm>
 
 #include "common.h"
@@ -67,6 +67,7 @@ struct ConvArgs {
   FastDiv d_khkw, d_kw, d_ns, d_sh, d_sw;
   int M, N, K, splits, kchunk;
   int n_s, kp, khkw;             // channels per shard, weights per channel, kernel positions
+  int co;                        // APART: contracted channels
   long numel;                    // elements per shard row
   const T* act;                  // x (forward, weight gradient) or dy (input gradient), at the run's first channel
   Strides s;
@@ -126,7 +127,11 @@ constexpr int kOutside = 1 << 30;
 // their MFMAs: the grids are small (MNIST's second convolution: two waves per SIMD), so the trip to memory has to
 // be covered by the wave itself.  SIMPLE: forward and weight gradient without padding (every gathered element exists),
 // input gradient with unit strides.
-template <typename T, ConvPass PASS, int BM, int BN, bool SIMPLE, bool WIDE>
+// APART (input gradient): a slab is 32 channels at one kernel position, so a pixel's neighbour is tested and, with strides, divided
+// for once a slab, the rest is scalar and there is no table; a slab's weights lie khkw elements apart, and a wave's lanes run along the input
+// channels, where 64 of them share ten lines.  us, forward and both gradients, before -> after (the input gradient's share): MNIST's second
+// convolution 102.8 -> 96.9, 128 x 64 x 32 x 32 -> 128 padded in bf16 368 -> 333, 37 x 24 x 31 x 31 -> 80 with strides of 2 128 -> 98.
+template <typename T, ConvPass PASS, int BM, int BN, bool SIMPLE, bool WIDE, bool APART = false>
 __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
   typedef typename Gather<T, WIDE>::off_t Off;
   constexpr int PITCH = kConvSlab + 16 / (int)sizeof(T);  // elements; rows stay 16-byte aligned
@@ -161,7 +166,7 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
     return e;
   };
   auto build_table = [&](int slab) {  // of the slab `slab` steps behind kb
-    if (PASS != kConvWgrad && tid < kConvSlab) {
+    if (PASS != kConvWgrad && !APART && tid < kConvSlab) {
       const int k = kb + slab * kConvSlab + tid;
       Off a = 0;
       tab[PASS == kConvWgrad ? 0 : slab & 3][tid] = entry_of(min(k, p.K - 1), k < ke, &a);
@@ -171,7 +176,22 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
 
   // ---- operand A: k = tid % 32, rows tid / 32 + 8 q ----
   const int ak = tid & 31, ar = tid >> 5;
+  // (APART: the thread's row m = tid % BM, k = tid / BM * NA + q, whose neighbours in a wave lie khkw elements apart)
   Off aoff[NA];
+  const int am = tid & (BM - 1), akq = tid / BM;
+  const unsigned a_row = (unsigned)(min(m0 + am, p.M - 1) * p.khkw);
+  int c0 = 0, pi = 0, pj = 0;  // APART: first channel and kernel position of the slab that is requested next
+  auto channel_rows = [&] {
+#pragma unroll
+    for (int q = 0; q < NA; ++q) {
+      const int co = min(c0 + akq * NA + q, p.co - 1);
+      const unsigned sft = fast_div((unsigned)co, p.d_ns);
+      aoff[q] = (Off)((sft * p.numel + (long)(co - sft * p.n_s) * p.kp + a_row) * ES);
+    }
+  };
+  if constexpr (APART)
+    channel_rows();
+  else
 #pragma unroll
   for (int q = 0; q < NA; ++q) {
     const int m = min(m0 + ar + 8 * q, p.M - 1);
@@ -205,8 +225,10 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
   };
   if (PASS != kConvWgrad) {
     bpix = locate(min(n0 + bn, p.N - 1), bh, bw);
-    build_table(0), build_table(1), build_table(2);
-    __syncthreads();
+    if constexpr (!APART) {
+      build_table(0), build_table(1), build_table(2);
+      __syncthreads();
+    }
   } else {
     Off unused;
     if (tid < BN) tab[0][tid] = entry_of(min(n0 + tid, p.N - 1), n0 + tid < p.N, &unused);
@@ -221,6 +243,35 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
   // requests a slab (one behind the contraction: nothing but zeros)
   auto fetch = [&](int slab, Regs& v) {
     const int k0 = kb + slab * kConvSlab;
+    if constexpr (APART) {  // slabs are requested in sequence
+      const int ij = (pi * g.kw + pj) * ES;
+#pragma unroll
+      for (int q = 0; q < NA; ++q) v.a[q] = wts.get(aoff[q] + ij, c0 + akq * NA + q < p.co);
+      const int di = pi * g.dh, dj = pj * g.dw;
+      Off at;
+      bool in;
+      if (SIMPLE) {
+        in = ((unsigned)(bh - di) < (unsigned)g.ho) & ((unsigned)(bw - dj) < (unsigned)g.wo);
+        at = bpix - (Off)((di * p.s.h + dj * p.s.w) * ES);
+      } else {
+        const int hn = bh - di, wn_ = bw - dj;
+        const int ho = (int)fast_div((unsigned)max(hn, 0), p.d_sh), wo = (int)fast_div((unsigned)max(wn_, 0), p.d_sw);
+        in = (hn >= 0) & (wn_ >= 0) & (ho * g.sh == hn) & (wo * g.sw == wn_) & (ho < g.ho) & (wo < g.wo);
+        at = bpix + (Off)((ho * p.s.h + wo * p.s.w) * ES);
+      }
+      const int c = c0 + __builtin_amdgcn_readfirstlane(kq) * NB;
+      const unsigned sc = (unsigned)(p.s.c * ES);
+#pragma unroll
+      for (int q = 0; q < NB; ++q) v.b[q] = act.get(at + (unsigned)(c + q) * sc, in & (c + q < p.co));
+      if (++pj == g.kw) {
+        pj = 0;
+        if (++pi == g.kh) {
+          pi = 0, c0 += kConvSlab;
+          channel_rows();
+        }
+      }
+      return;
+    }
     if (PASS == kConvWgrad) {
       const bool live = k0 + ak < ke;
       const int pix = live ? k0 + ak : p.K - 1;
@@ -274,8 +325,16 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
   auto stash = [&](int buf, const Regs& v) {
 #pragma unroll
     for (int q = 0; q < NA; ++q) {
-      As[buf][(ar + 8 * q) * PITCH + ak] = v.a[q];
+      if (!APART) As[buf][(ar + 8 * q) * PITCH + ak] = v.a[q];
       if (PASS == kConvWgrad) rsum[q] += to_f32(v.a[q]);
+    }
+    if constexpr (APART) {
+      struct alignas(NA * ES < 16 ? NA * ES : 16) Run {
+        T e[NA];
+      } u;
+#pragma unroll
+      for (int q = 0; q < NA; ++q) u.e[q] = v.a[q];
+      *reinterpret_cast<Run*>(&As[buf][am * PITCH + akq * NA]) = u;
     }
     if (PASS == kConvWgrad) {
 #pragma unroll
@@ -453,6 +512,16 @@ static int check_run(const char* who, int dtype, int64_t numel, int64_t shards, 
   return RTP_OK;
 }
 
+// Whether the input gradient contracts slabs of 32 channels at one kernel position each (APART) rather than channels with all
+// their positions: such slabs are filled up to whole ones, which costs MFMAs and saves the tests of every element.  us for
+// both gradients and the forward of 64 x 32 x 28 x 28, fp32 / bf16, mixed slabs -> slabs of a position: 3 x 3, 24 channels 88.8
+// / 65.9 -> 88.3 / 63.8, 20 of 32 84.8 / 62.9 -> 87.5 / 62.7, 40 of 64 109 / 70.3 -> 114 / 70.0; with strides of 2, where an element's test
+// has two divisions, 5 x 5, 20 channels 131 / 97.4 -> 123 / 88.1, 40 170 / 124 -> 161 / 113, 33 of 64 152 / 111 -> 160 / 109.
+static bool channels_apart(long co, bool unit_strides) {
+  const long padded = ceil_div(co, kConvSlab) * kConvSlab;
+  return unit_strides ? 3 * padded <= 4 * co : 5 * padded <= 8 * co;
+}
+
 template <typename T, ConvPass PASS, int BM, int BN>
 static void launch_tile(hipStream_t st, const ConvArgs<T>& a, dim3 grid) {
   const ConvGeom& g = a.g;
@@ -467,6 +536,16 @@ static void launch_tile(hipStream_t st, const ConvArgs<T>& a, dim3 grid) {
   if (PASS == kConvWgrad) far = std::max(far, reach(a.sd, g.n, co, g.ho, g.wo));
   const bool wide = (far + 1.0) * sizeof(T) >= (double)kBeyond;
 #define RTP_CONV(SIMPLE, WIDE) hipLaunchKernelGGL((conv_igemm_kernel<T, PASS, BM, BN, SIMPLE, WIDE>), grid, dim3(256), 0, st, a)
+  if constexpr (PASS == kConvDgrad)
+    if (!wide && channels_apart(co, simple)) {
+      ConvArgs<T> b = a;
+      b.co = (int)co, b.K = b.kchunk = (int)(ceil_div(co, kConvSlab) * kConvSlab) * a.khkw;
+      if (simple)
+        hipLaunchKernelGGL((conv_igemm_kernel<T, PASS, BM, BN, true, false, true>), grid, dim3(256), 0, st, b);
+      else
+        hipLaunchKernelGGL((conv_igemm_kernel<T, PASS, BM, BN, false, false, true>), grid, dim3(256), 0, st, b);
+      return;
+    }
   if (wide)
     RTP_CONV(false, true);
   else if (simple)

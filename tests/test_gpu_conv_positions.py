@@ -1,0 +1,37 @@
+"""The convolution's input gradient where a slab is one kernel position of 32 channels: channel counts that fill whole slabs,
+all but a quarter of them and just too little, shards whose channels end inside a slab, strides that skip pixels, dilation, 32- and 64-row
+tiles, channels-last gradients and a run in the middle of a wider one, against torch's input gradient in fp64 on the CPU."""
+import pytest
+import torch
+
+from gpu_util import DEV
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,ci,h,w,co,shards,k,s,p,d", [
+    (2, 3, 9, 11, 32, 1, (3, 3), (1, 1), (0, 0), (1, 1)), (1, 33, 7, 8, 24, 3, (3, 2), (1, 1), (1, 2), (1, 2)),
+    (3, 70, 6, 6, 48, 4, (1, 1), (1, 1), (0, 0), (1, 1)), (2, 32, 13, 12, 20, 2, (5, 3), (2, 1), (2, 1), (1, 1)),
+    (1, 65, 17, 16, 40, 8, (3, 3), (3, 2), (1, 0), (2, 1)), (2, 8, 10, 10, 66, 3, (3, 3), (1, 1), (1, 1), (1, 1)),
+    (1, 1, 5, 5, 160, 5, (5, 5), (1, 1), (2, 2), (1, 1))])
+def test_input_gradient_against_torch(n, ci, h, w, co, shards, k, s, p, d, dtype):
+    from rtp_amd import ops
+    gen = torch.Generator().manual_seed(co + h)
+    g = ops.conv_geom((n, ci, h, w), k, s, p, d)
+    kp, n_s, extra = ci * k[0] * k[1], co // shards, 5
+    flat = torch.randn(shards, extra + n_s * kp + n_s, generator=gen).to(dtype)
+    flat[:, :extra], flat[:, extra + n_s * kp:] = float("nan"), float("nan")  # around the weights: nothing of it comes through
+    dy = torch.randn(n, co + 2, g.ho, g.wo, generator=gen).to(dtype)
+    dy[:, 0], dy[:, -1] = float("nan"), float("nan")
+    weight = torch.cat([r[extra:extra + n_s * kp].view(n_s, ci, *k) for r in flat]).double()
+    grad = dy[:, 1:-1].double()
+    want = torch.nn.grad.conv2d_input((n, ci, h, w), weight, grad, s, p, d)
+    terms = torch.nn.grad.conv2d_input((n, ci, h, w), weight.abs(), grad.abs(), s, p, d)
+    # products of bf16 are exact in fp32: a sum of K terms in any order is within K units of 2^-24 of their magnitudes, and the
+    # result rounds once more (bf16 has 8 significant bits: half a unit of the last one is at most 2^-8 of the value)
+    bound = terms * (co * k[0] * k[1] + 1) * 2.0 ** -24 + want.abs() * (2.0 ** -8 if dtype == torch.bfloat16 else 0)
+    for fmt in (torch.contiguous_format, torch.channels_last):
+        dx = torch.empty(n, ci, h, w, dtype=dtype, device=DEV)
+        ops.conv2d_dgrad(dy.to(DEV).contiguous(memory_format=fmt), g, flat.to(DEV), extra, n_s, 1, dx)
+        assert bool(((dx.cpu().double() - want).abs() <= bound).all())

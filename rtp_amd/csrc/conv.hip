@@ -13,7 +13,7 @@
 // its rows) for the whole contraction, and everything that depends on k alone -- offset inside an image, kernel position --
 // is worked out once per slab by one thread per k and handed round through LDS.  The first version called an index function
 // with five integer divisions per element and gave every shard tiles of its own: MNIST's second convolution (64 x 32 x 26 x
-// 26 -> 64, four shards, fp32) took 127 + 162 + 196 us forward / input / weight gradient; this one takes 29 + 37 + 34.
+// 26 -> 64, four shards, fp32) took 127 + 162 + 196 us forward / input / weight gradient; this one takes 27 + 37 + 34.
 #include <algorithm>
 
 #include "common.h"
@@ -127,6 +127,8 @@ constexpr int kOutside = 1 << 30;
 // their MFMAs: the grids are small (MNIST's second convolution: two waves per SIMD), so the trip to memory has to
 // be covered by the wave itself.  SIMPLE: forward and weight gradient without padding (every gathered element exists),
 // input gradient with unit strides.
+// Forward: a thread takes NA consecutive weights of a row by one load or two at any alignment instead of NA loads (128 x 64 x 32 x 32 -> 128
+// padded in bf16, forward and both gradients 332 -> 317 us, MNIST's second convolution in fp32 96.6 -> 94.9).
 // APART (input gradient): a slab is 32 channels at one kernel position, so a pixel's neighbour is tested and, with strides, divided
 // for once a slab, the rest is scalar and there is no table; a slab's weights lie khkw elements apart, and a wave's lanes run along the input
 // channels, where 64 of them share ten lines.  us, forward and both gradients, before -> after (the input gradient's share): MNIST's second
@@ -174,7 +176,7 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
     }
   };
 
-  // ---- operand A: k = tid % 32, rows tid / 32 + 8 q ----
+  // ---- operand A: k = tid % 32, rows tid / 32 + 8 q (forward: the thread's row, NA consecutive k) ----
   const int ak = tid & 31, ar = tid >> 5;
   // (APART: the thread's row m = tid % BM, k = tid / BM * NA + q, whose neighbours in a wave lie khkw elements apart)
   Off aoff[NA];
@@ -189,16 +191,29 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
       aoff[q] = (Off)((sft * p.numel + (long)(co - sft * p.n_s) * p.kp + a_row) * ES);
     }
   };
-  if constexpr (APART)
+  constexpr bool RUNS = PASS == kConvFwd;
+  constexpr int RUNW = NA * ES / 4;
+  struct __attribute__((packed, aligned(ES))) AnyRun {  // at the elements' alignment
+    unsigned w[RUNW];
+  };
+  union PackedRun {
+    T e[NA];
+    unsigned w[RUNW];
+  };
+  const int rr = tid / (kConvSlab / NA), rk = tid % (kConvSlab / NA) * NA;
+  const T* run_row = nullptr;
+  if constexpr (RUNS) {
+    const unsigned m = (unsigned)min(m0 + rr, p.M - 1), sft = fast_div(m, p.d_ns);
+    run_row = p.w + (sft * p.numel + (long)(m - sft * p.n_s) * p.kp);
+  }
+  if constexpr (RUNS) {
+  } else if constexpr (APART)
     channel_rows();
   else
 #pragma unroll
   for (int q = 0; q < NA; ++q) {
     const int m = min(m0 + ar + 8 * q, p.M - 1);
-    if (PASS == kConvFwd) {
-      const unsigned sft = fast_div((unsigned)m, p.d_ns);
-      aoff[q] = (Off)((sft * p.numel + (long)(m - sft * p.n_s) * p.kp) * ES);
-    } else if (PASS == kConvDgrad) {
+    if (PASS == kConvDgrad) {
       aoff[q] = (Off)((long)m * p.khkw * ES);
     } else {
       aoff[q] = (Off)(m * p.sd.c * ES);
@@ -239,6 +254,7 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
 
   struct Regs {
     T a[NA], b[NB];
+    unsigned run[RUNW];  // RUNS, in place of a: kept as it was loaded, so that nothing waits for it before it is stored
   } reg[2];
   // requests a slab (one behind the contraction: nothing but zeros)
   auto fetch = [&](int slab, Regs& v) {
@@ -293,9 +309,29 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
       return;
     }
     const int slot = PASS == kConvWgrad ? 0 : slab & 3;
-    {
+    if constexpr (RUNS) {
+      if (k0 + kConvSlab <= p.K) {
+        const AnyRun run = *reinterpret_cast<const AnyRun*>(run_row + k0 + rk);
+#pragma unroll
+        for (int q = 0; q < RUNW; ++q) v.run[q] = run.w[q];
+      } else {  // the slab that the contraction ends in, or one behind it
+        PackedRun u;
+#pragma unroll
+        for (int q = 0; q < RUNW; ++q) u.w[q] = 0;
+        if (k0 < p.K) {
+#pragma unroll
+          for (int q = 0; q < NA; ++q) {
+            const int k = k0 + rk + q;
+            const T t = run_row[min(k, p.K - 1)];
+            u.e[q] = k < p.K ? t : from_f32<T>(0.0f);
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < RUNW; ++q) v.run[q] = u.w[q];
+      }
+    } else {
       const bool live = k0 + ak < ke;
-      const Off off = PASS == kConvDgrad ? tab_a[slot][ak] : (Off)(k0 + ak) * ES;
+      const Off off = tab_a[slot][ak];
 #pragma unroll
       for (int q = 0; q < NA; ++q) v.a[q] = wts.get(aoff[q] + off, live);
     }
@@ -325,16 +361,24 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
   auto stash = [&](int buf, const Regs& v) {
 #pragma unroll
     for (int q = 0; q < NA; ++q) {
-      if (!APART) As[buf][(ar + 8 * q) * PITCH + ak] = v.a[q];
+      if (!APART && !RUNS) As[buf][(ar + 8 * q) * PITCH + ak] = v.a[q];
       if (PASS == kConvWgrad) rsum[q] += to_f32(v.a[q]);
     }
-    if constexpr (APART) {
+    if constexpr (APART || RUNS) {
       struct alignas(NA * ES < 16 ? NA * ES : 16) Run {
-        T e[NA];
-      } u;
+        unsigned w[RUNW];
+      } out;
+      if constexpr (RUNS) {
 #pragma unroll
-      for (int q = 0; q < NA; ++q) u.e[q] = v.a[q];
-      *reinterpret_cast<Run*>(&As[buf][am * PITCH + akq * NA]) = u;
+        for (int q = 0; q < RUNW; ++q) out.w[q] = v.run[q];
+      } else {
+        PackedRun u;
+#pragma unroll
+        for (int q = 0; q < NA; ++q) u.e[q] = v.a[q];
+#pragma unroll
+        for (int q = 0; q < RUNW; ++q) out.w[q] = u.w[q];
+      }
+      *reinterpret_cast<Run*>(&As[buf][RUNS ? rr * PITCH + rk : am * PITCH + akq * NA]) = out;
     }
     if (PASS == kConvWgrad) {
 #pragma unroll

@@ -13,7 +13,7 @@
 // its rows) for the whole contraction, and everything that depends on k alone -- offset inside an image, kernel position --
 // is worked out once per slab by one thread per k and handed round through LDS.  The first version called an index function
 // with five integer divisions per element and gave every shard tiles of its own: MNIST's second convolution (64 x 32 x 26 x
-// 26 -> 64, four shards, fp32) took 127 + 162 + 196 us forward / input / weight gradient; this one takes 27 + 37 + 34.
+// 26 -> 64, four shards, fp32) took 127 + 162 + 196 us forward / input / weight gradient; this one takes 27 + 37 + 32.
 #include <algorithm>
 
 #include "common.h"
@@ -67,7 +67,7 @@ struct ConvArgs {
   FastDiv d_khkw, d_kw, d_ns, d_sh, d_sw;
   int M, N, K, splits, kchunk;
   int n_s, kp, khkw;             // channels per shard, weights per channel, kernel positions
-  int co;                        // APART: contracted channels
+  int co;                        // WHOLE: contracted channels
   long numel;                    // elements per shard row
   const T* act;                  // x (forward, weight gradient) or dy (input gradient), at the run's first channel
   Strides s;
@@ -104,6 +104,21 @@ struct Gather {
     else
       return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b16(r, (int)off, 0, 0));
   }
+  // N words at an offset that 16 bytes divide (two words: 8)
+  template <int N>
+  __device__ __forceinline__ void run(unsigned (&w)[N], unsigned off) const {
+    typedef __attribute__((ext_vector_type(N < 4 ? N : 4))) unsigned vec;
+#pragma unroll
+    for (int i = 0; i < N; i += 4) {
+      vec t;
+      if constexpr (N == 2)
+        t = __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0));
+      else  // (an offset beyond the buffer stays one: the next 16 bytes' own is not added to it)
+        t = __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(off == kBeyond ? off : off + 4 * i), 0, 0));
+#pragma unroll
+      for (int e = 0; e < (N < 4 ? N : 4); ++e) w[i + e] = t[e];
+    }
+  }
 };
 template <typename T>
 struct Gather<T, true> {
@@ -129,11 +144,14 @@ constexpr int kOutside = 1 << 30;
 // input gradient with unit strides.
 // Forward: a thread takes NA consecutive weights of a row by one load or two at any alignment instead of NA loads (128 x 64 x 32 x 32 -> 128
 // padded in bf16, forward and both gradients 332 -> 317 us, MNIST's second convolution in fp32 96.6 -> 94.9).
-// APART (input gradient): a slab is 32 channels at one kernel position, so a pixel's neighbour is tested and, with strides, divided
+// WHOLE (weight gradient): runs of NA output pixels of a plane are whole and aligned in dy and come by one load or two, as the forward's weights
+// do (launch_tile has the rule; the same case 317 -> 291 us, in 64-row tiles 1 - 9 %, in those of 32 rows no difference).  The bias gradient's 32
+// chains of additions a row are the same ones on either way.
+// WHOLE (input gradient): a slab is 32 channels at one kernel position, so a pixel's neighbour is tested and, with strides, divided
 // for once a slab, the rest is scalar and there is no table; a slab's weights lie khkw elements apart, and a wave's lanes run along the input
 // channels, where 64 of them share ten lines.  us, forward and both gradients, before -> after (the input gradient's share): MNIST's second
 // convolution 102.8 -> 96.9, 128 x 64 x 32 x 32 -> 128 padded in bf16 368 -> 333, 37 x 24 x 31 x 31 -> 80 with strides of 2 128 -> 98.
-template <typename T, ConvPass PASS, int BM, int BN, bool SIMPLE, bool WIDE, bool APART = false>
+template <typename T, ConvPass PASS, int BM, int BN, bool SIMPLE, bool WIDE, bool WHOLE = false>
 __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
   typedef typename Gather<T, WIDE>::off_t Off;
   constexpr int PITCH = kConvSlab + 16 / (int)sizeof(T);  // elements; rows stay 16-byte aligned
@@ -168,7 +186,7 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
     return e;
   };
   auto build_table = [&](int slab) {  // of the slab `slab` steps behind kb
-    if (PASS != kConvWgrad && !APART && tid < kConvSlab) {
+    if (PASS != kConvWgrad && !WHOLE && tid < kConvSlab) {
       const int k = kb + slab * kConvSlab + tid;
       Off a = 0;
       tab[PASS == kConvWgrad ? 0 : slab & 3][tid] = entry_of(min(k, p.K - 1), k < ke, &a);
@@ -176,13 +194,13 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
     }
   };
 
-  // ---- operand A: k = tid % 32, rows tid / 32 + 8 q (forward: the thread's row, NA consecutive k) ----
+  // ---- operand A: k = tid % 32, rows tid / 32 + 8 q (RUNS: the thread's row, NA consecutive k) ----
   const int ak = tid & 31, ar = tid >> 5;
-  // (APART: the thread's row m = tid % BM, k = tid / BM * NA + q, whose neighbours in a wave lie khkw elements apart)
+  // (WHOLE: the thread's row m = tid % BM, k = tid / BM * NA + q, whose neighbours in a wave lie khkw elements apart)
   Off aoff[NA];
   const int am = tid & (BM - 1), akq = tid / BM;
   const unsigned a_row = (unsigned)(min(m0 + am, p.M - 1) * p.khkw);
-  int c0 = 0, pi = 0, pj = 0;  // APART: first channel and kernel position of the slab that is requested next
+  int c0 = 0, pi = 0, pj = 0;  // WHOLE: first channel and kernel position of the slab that is requested next
   auto channel_rows = [&] {
 #pragma unroll
     for (int q = 0; q < NA; ++q) {
@@ -191,7 +209,7 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
       aoff[q] = (Off)((sft * p.numel + (long)(co - sft * p.n_s) * p.kp + a_row) * ES);
     }
   };
-  constexpr bool RUNS = PASS == kConvFwd;
+  constexpr bool RUNS = PASS == kConvFwd || (PASS == kConvWgrad && WHOLE);
   constexpr int RUNW = NA * ES / 4;
   struct __attribute__((packed, aligned(ES))) AnyRun {  // at the elements' alignment
     unsigned w[RUNW];
@@ -202,12 +220,13 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
   };
   const int rr = tid / (kConvSlab / NA), rk = tid % (kConvSlab / NA) * NA;
   const T* run_row = nullptr;
-  if constexpr (RUNS) {
+  if constexpr (PASS == kConvFwd) {
     const unsigned m = (unsigned)min(m0 + rr, p.M - 1), sft = fast_div(m, p.d_ns);
     run_row = p.w + (sft * p.numel + (long)(m - sft * p.n_s) * p.kp);
   }
   if constexpr (RUNS) {
-  } else if constexpr (APART)
+    aoff[0] = (Off)(min(m0 + rr, p.M - 1) * p.sd.c * ES);
+  } else if constexpr (PASS == kConvDgrad && WHOLE)
     channel_rows();
   else
 #pragma unroll
@@ -240,7 +259,7 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
   };
   if (PASS != kConvWgrad) {
     bpix = locate(min(n0 + bn, p.N - 1), bh, bw);
-    if constexpr (!APART) {
+    if constexpr (!(PASS == kConvDgrad && WHOLE)) {
       build_table(0), build_table(1), build_table(2);
       __syncthreads();
     }
@@ -259,7 +278,7 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
   // requests a slab (one behind the contraction: nothing but zeros)
   auto fetch = [&](int slab, Regs& v) {
     const int k0 = kb + slab * kConvSlab;
-    if constexpr (APART) {  // slabs are requested in sequence
+    if constexpr (PASS == kConvDgrad && WHOLE) {  // slabs are requested in sequence
       const int ij = (pi * g.kw + pj) * ES;
 #pragma unroll
       for (int q = 0; q < NA; ++q) v.a[q] = wts.get(aoff[q] + ij, c0 + akq * NA + q < p.co);
@@ -297,8 +316,14 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
       const int r = pix - img * p.d_pix_img.d;
       const unsigned yo = fast_div((unsigned)r, p.d_pix_row);
       const Off d = (Off)(((long)img * p.sd.n + (long)yo * p.sd.h + (long)(r - yo * p.d_pix_row.d) * p.sd.w) * ES);
+      if constexpr (PASS == kConvWgrad && RUNS) {  // (a run is inside one image and inside or beyond the contraction)
+        const unsigned at = (unsigned)(k0 + rk), rimg = fast_div(at, p.d_pix_img);
+        const unsigned off = (unsigned)(((long)rimg * p.sd.n + (at - rimg * p.d_pix_img.d)) * ES) + (unsigned)aoff[0];
+        wts.run(v.run, (int)at < ke ? off : kBeyond);
+      } else {
 #pragma unroll
-      for (int q = 0; q < NA; ++q) v.a[q] = wts.get(d + aoff[q], live);
+        for (int q = 0; q < NA; ++q) v.a[q] = wts.get(d + aoff[q], live);
+      }
 #pragma unroll
       for (int q = 0; q < NB; ++q) {
         const KEntry<Off>& e = brow[PASS == kConvWgrad ? q : 0];
@@ -361,10 +386,17 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
   auto stash = [&](int buf, const Regs& v) {
 #pragma unroll
     for (int q = 0; q < NA; ++q) {
-      if (!APART && !RUNS) As[buf][(ar + 8 * q) * PITCH + ak] = v.a[q];
-      if (PASS == kConvWgrad) rsum[q] += to_f32(v.a[q]);
+      if (!WHOLE && !RUNS) As[buf][(ar + 8 * q) * PITCH + ak] = v.a[q];
+      if (PASS == kConvWgrad && !RUNS) rsum[q] += to_f32(v.a[q]);
     }
-    if constexpr (APART || RUNS) {
+    if constexpr (PASS == kConvWgrad && RUNS) {
+      PackedRun u;
+#pragma unroll
+      for (int q = 0; q < RUNW; ++q) u.w[q] = v.run[q];
+#pragma unroll
+      for (int q = 0; q < NA; ++q) rsum[q] += to_f32(u.e[q]);
+    }
+    if constexpr (WHOLE || RUNS) {
       struct alignas(NA * ES < 16 ? NA * ES : 16) Run {
         unsigned w[RUNW];
       } out;
@@ -478,14 +510,26 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
       }
     }
   }
-  if (want_rows) {  // bias gradient: the rows' sums over this workgroup's pixels, 32 lanes each in a fixed order
+  if (want_rows) {  // bias gradient: the rows' sums over this workgroup's pixels, 32 chains (pixel % 32) each in a fixed order
+    if constexpr (RUNS) {
 #pragma unroll
-    for (int q = 0; q < NA; ++q) {
+      for (int o = 16; o >= NA; o >>= 1)
+#pragma unroll
+        for (int q = 0; q < NA; ++q) rsum[q] += __shfl_xor(rsum[q], o / NA, 64);
+#pragma unroll
+      for (int o = NA / 2; o > 0; o >>= 1)
+#pragma unroll
+        for (int q = 0; q < o; ++q) rsum[q] += rsum[q + o];
+    }
+#pragma unroll
+    for (int q = 0; q < (RUNS ? 1 : NA); ++q) {
       float v = rsum[q];
+      if constexpr (!RUNS) {
 #pragma unroll
-      for (int o = 16; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-      const int m = m0 + ar + 8 * q;
-      if (ak != 0 || m >= p.M) continue;
+        for (int o = 16; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+      }
+      const int m = RUNS ? m0 + rr : m0 + ar + 8 * q;
+      if ((RUNS ? rk : ak) != 0 || m >= p.M) continue;
       if (p.part != nullptr) {
         p.part[((long)split * p.M + m) * (p.kp + 1) + p.kp] = v;
       } else if (p.b_off >= 0) {
@@ -556,12 +600,12 @@ static int check_run(const char* who, int dtype, int64_t numel, int64_t shards, 
   return RTP_OK;
 }
 
-// Whether the input gradient contracts slabs of 32 channels at one kernel position each (APART) rather than channels with all
+// Whether the input gradient contracts slabs of 32 channels at one kernel position each (WHOLE) rather than channels with all
 // their positions: such slabs are filled up to whole ones, which costs MFMAs and saves the tests of every element.  us for
 // both gradients and the forward of 64 x 32 x 28 x 28, fp32 / bf16, mixed slabs -> slabs of a position: 3 x 3, 24 channels 88.8
 // / 65.9 -> 88.3 / 63.8, 20 of 32 84.8 / 62.9 -> 87.5 / 62.7, 40 of 64 109 / 70.3 -> 114 / 70.0; with strides of 2, where an element's test
 // has two divisions, 5 x 5, 20 channels 131 / 97.4 -> 123 / 88.1, 40 170 / 124 -> 161 / 113, 33 of 64 152 / 111 -> 160 / 109.
-static bool channels_apart(long co, bool unit_strides) {
+static bool whole_positions(long co, bool unit_strides) {
   const long padded = ceil_div(co, kConvSlab) * kConvSlab;
   return unit_strides ? 3 * padded <= 4 * co : 5 * padded <= 8 * co;
 }
@@ -581,7 +625,7 @@ static void launch_tile(hipStream_t st, const ConvArgs<T>& a, dim3 grid) {
   const bool wide = (far + 1.0) * sizeof(T) >= (double)kBeyond;
 #define RTP_CONV(SIMPLE, WIDE) hipLaunchKernelGGL((conv_igemm_kernel<T, PASS, BM, BN, SIMPLE, WIDE>), grid, dim3(256), 0, st, a)
   if constexpr (PASS == kConvDgrad)
-    if (!wide && channels_apart(co, simple)) {
+    if (!wide && whole_positions(co, simple)) {
       ConvArgs<T> b = a;
       b.co = (int)co, b.K = b.kchunk = (int)(ceil_div(co, kConvSlab) * kConvSlab) * a.khkw;
       if (simple)
@@ -590,6 +634,17 @@ static void launch_tile(hipStream_t st, const ConvArgs<T>& a, dim3 grid) {
         hipLaunchKernelGGL((conv_igemm_kernel<T, PASS, BM, BN, false, false, true>), grid, dim3(256), 0, st, b);
       return;
     }
+  if constexpr (PASS == kConvWgrad) {  // dy contiguous, and planes and images whole aligned runs
+    constexpr int NA = BM * kConvSlab / 256;
+    if (!wide && a.sd.w == 1 && a.sd.h == g.wo && (long)g.ho * g.wo % NA == 0 && a.sd.n % NA == 0 && a.sd.c % NA == 0 &&
+        reinterpret_cast<uintptr_t>(a.dy) % std::min<size_t>(16, NA * sizeof(T)) == 0) {
+      if (simple)
+        hipLaunchKernelGGL((conv_igemm_kernel<T, PASS, BM, BN, true, false, true>), grid, dim3(256), 0, st, a);
+      else
+        hipLaunchKernelGGL((conv_igemm_kernel<T, PASS, BM, BN, false, false, true>), grid, dim3(256), 0, st, a);
+      return;
+    }
+  }
   if (wide)
     RTP_CONV(false, true);
   else if (simple)

@@ -35,3 +35,32 @@ def test_input_gradient_against_torch(n, ci, h, w, co, shards, k, s, p, d, dtype
         dx = torch.empty(n, ci, h, w, dtype=dtype, device=DEV)
         ops.conv2d_dgrad(dy.to(DEV).contiguous(memory_format=fmt), g, flat.to(DEV), extra, n_s, 1, dx)
         assert bool(((dx.cpu().double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,ci,h,co,shards,k,s,p", [
+    (1, 3, 6, 32, 1, 3, 1, 0), (7, 5, 10, 40, 2, 3, 1, 0), (3, 33, 8, 64, 4, 1, 1, 0), (5, 4, 17, 30, 3, 3, 2, 1),
+    (2, 16, 6, 130, 5, 3, 1, 1), (9, 2, 4, 72, 1, 1, 1, 0)])
+def test_weight_gradient_of_whole_runs(n, ci, h, co, shards, k, s, p, dtype):
+    """Planes of output pixels that runs of four or eight divide are read by runs, others and channels-last gradients by elements: the
+    same sums in the same order, so the same bits; images of 16 - 100 pixels end inside slabs of 32."""
+    from rtp_amd import ops
+    gen = torch.Generator().manual_seed(co + h)
+    g = ops.conv_geom((n, ci, h, h), (k, k), (s, s), (p, p), (1, 1))
+    kp, n_s = ci * k * k, co // shards
+    x = torch.randn(n, ci, h, h, generator=gen).to(dtype)
+    dy = torch.randn(n, co + 2, g.ho, g.wo, generator=gen).to(dtype)
+    dy[:, 0], dy[:, -1] = float("nan"), float("nan")
+    got = []
+    for fmt in (torch.contiguous_format, torch.channels_last):
+        grads = torch.zeros(shards, n_s * (kp + 1), dtype=dtype, device=DEV)
+        ops.conv2d_wgrad(dy.to(DEV).contiguous(memory_format=fmt), x.to(DEV), g, grads, 0, n_s * kp, n_s, 1, False)
+        got.append(grads.cpu())
+    assert torch.equal(got[0], got[1])
+    shape, d64, x64 = (co, ci, k, k), dy[:, 1:-1].double(), x.double()
+    weight, bias = torch.nn.grad.conv2d_weight(x64, shape, d64, s, p), d64.sum((0, 2, 3))
+    w_abs, b_abs = torch.nn.grad.conv2d_weight(x64.abs(), shape, d64.abs(), s, p), d64.abs().sum((0, 2, 3))
+    rows = got[0].double()
+    for have, want, terms in ((rows[:, :n_s * kp].reshape(shape), weight, w_abs), (rows[:, n_s * kp:].reshape(co), bias, b_abs)):
+        bound = terms * (n * g.ho * g.wo + 1) * 2.0 ** -24 + want.abs() * (2.0 ** -8 if dtype == torch.bfloat16 else 0)
+        assert bool(((have - want).abs() <= bound).all())

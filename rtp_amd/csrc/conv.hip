@@ -185,12 +185,13 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
     }
     return e;
   };
-  auto build_table = [&](int slab) {  // of the slab `slab` steps behind kb
-    if (PASS != kConvWgrad && !WHOLE && tid < kConvSlab) {
-      const int k = kb + slab * kConvSlab + tid;
+  // of two slabs, by one wave: the slabs `slab` and `slab` + 1 steps behind kb
+  auto build_table = [&](int slab) {
+    if (PASS != kConvWgrad && !WHOLE && tid < 2 * kConvSlab) {
+      const int k = kb + slab * kConvSlab + tid, slot = (slab + tid / kConvSlab) & 3, at = tid & (kConvSlab - 1);
       Off a = 0;
-      tab[PASS == kConvWgrad ? 0 : slab & 3][tid] = entry_of(min(k, p.K - 1), k < ke, &a);
-      if (PASS == kConvDgrad) tab_a[slab & 3][tid] = a;
+      tab[PASS == kConvWgrad ? 0 : slot][at] = entry_of(min(k, p.K - 1), k < ke, &a);
+      if (PASS == kConvDgrad) tab_a[slot][at] = a;
     }
   };
 
@@ -260,7 +261,7 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
   if (PASS != kConvWgrad) {
     bpix = locate(min(n0 + bn, p.N - 1), bh, bw);
     if constexpr (!(PASS == kConvDgrad && WHOLE)) {
-      build_table(0), build_table(1), build_table(2);
+      build_table(0), build_table(2);
       __syncthreads();
     }
   } else {
@@ -438,8 +439,9 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
   fetch(1, reg[1]);
   stash(0, reg[0]);
   __syncthreads();
-  // step s: requests slab s + 2 into the registers that slab s left, multiplies slab s, stores slab s + 1.  The table of slab
-  // s + 3 is built meanwhile: it is read behind the next barrier, and its slot (s + 3) % 4 by nobody now.
+  // step s: requests slab s + 2 into the registers that slab s left, multiplies slab s, stores slab s + 1.  The tables of slabs
+  // s + 3 and s + 4 are built meanwhile by odd s: they are read behind the next barrier, and their slots (s + 3) % 4 and s % 4 by
+  // nobody now.
   auto step = [&](int sl, Regs& mine, Regs& next, int buf) {
     fetch(sl + 2, mine);  // unconditionally: the wait for slab s + 1 below counts the loads in flight
     constexpr int STEP = ConvFrag<T>::kStep, VEC = 16 / (int)sizeof(T);
@@ -453,7 +455,7 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
       b.q = *reinterpret_cast<const uint4*>(&Bs[buf][(wn * 32 + li) * PITCH + ks * STEP + lg * VEC]);
       conv_mma(a.f, b.f, acc);
     }
-    build_table(sl + 3);
+    if (buf == 1) build_table(sl + 3);
     stash(buf ^ 1, next);
     __syncthreads();
   };

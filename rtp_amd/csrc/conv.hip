@@ -13,7 +13,7 @@
 // its rows) for the whole contraction, and everything that depends on k alone -- offset inside an image, kernel position --
 // is worked out once per slab by one thread per k and handed round through LDS.  The first version called an index function
 // with five integer divisions per element and gave every shard tiles of its own: MNIST's second convolution (64 x 32 x 26 x
-// 26 -> 64, four shards, fp32) took 127 + 162 + 196 us forward / input / weight gradient; this one takes 27 + 37 + 32.
+// 26 -> 64, four shards, fp32) took 127 + 162 + 196 us forward / input / weight gradient; this one takes 25 + 36 + 30.
 #include <algorithm>
 
 #include "common.h"
@@ -137,8 +137,8 @@ struct alignas(16) KEntry {
 };
 constexpr int kOutside = 1 << 30;
 
-// BM x BN outputs per workgroup (BM * BN = 4096), four waves, each one row of MFMA blocks wide: 64 x 64 as 2 x 2 waves, or
-// 32 x 128 as 1 x 4 for products of at most 32 rows.  LDS is double buffered and elements are requested two slabs ahead of
+// BM x BN outputs per workgroup, four waves: 64 x 64 or 64 x 128 as 2 x 2 waves of one or two MFMA blocks, or 32 x 128 as 1 x 4 for
+// products of at most 32 rows.  LDS is double buffered and elements are requested two slabs ahead of
 // their MFMAs: the grids are small (MNIST's second convolution: two waves per SIMD), so the trip to memory has to
 // be covered by the wave itself.  SIMPLE: forward and weight gradient without padding (every gathered element exists),
 // input gradient with unit strides.
@@ -163,7 +163,8 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
   __shared__ Off tab_a[4][kConvSlab];  // input gradient: offset of the weight
   const ConvGeom& g = p.g;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = BM == 64 ? wave >> 1 : 0, wn = BM == 64 ? wave & 1 : wave, li = lane & 31, lg = lane >> 5;
+  constexpr int NT = BM * BN / 4096;  // MFMA blocks of a wave
+  const int wm = BM == 64 ? wave >> 1 : 0, wn = (BM == 64 ? wave & 1 : wave) * NT, li = lane & 31, lg = lane >> 5;
   const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
   const int split = blockIdx.z, kb = split * p.kchunk, ke = min(kb + p.kchunk, p.K);
   const Gather<T, WIDE> act(p.act), wts(PASS == kConvWgrad ? p.dy : p.w);  // wts: operand A
@@ -431,9 +432,11 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
     }
   };
 
-  conv_f32x16 acc;
+  conv_f32x16 accs[NT];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) accs[t][r] = 0.0f;
   const int slabs = (ke - kb + kConvSlab - 1) / kConvSlab;
   fetch(0, reg[0]);
   fetch(1, reg[1]);
@@ -450,10 +453,13 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
       union {
         uint4 q;
         ConvFrag<T> f;
-      } a, b;
+      } a, b[NT];
       a.q = *reinterpret_cast<const uint4*>(&As[buf][(wm * 32 + li) * PITCH + ks * STEP + lg * VEC]);
-      b.q = *reinterpret_cast<const uint4*>(&Bs[buf][(wn * 32 + li) * PITCH + ks * STEP + lg * VEC]);
-      conv_mma(a.f, b.f, acc);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        b[t].q = *reinterpret_cast<const uint4*>(&Bs[buf][((wn + t) * 32 + li) * PITCH + ks * STEP + lg * VEC]);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) conv_mma(a.f, b[t].f, accs[t]);
     }
     if (buf == 1) build_table(sl + 3);
     stash(buf ^ 1, next);
@@ -465,8 +471,11 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
   }
 
   // ---- results: accumulator register r of lane (li, lg) is row 8*(r/4) + 4*lg + r%4 of the wave's block, column li ----
-  const int col = n0 + wn * 32 + li;
-  if (col < p.N) {
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int col = n0 + (wn + t) * 32 + li;
+    if (col >= p.N) continue;
+    const conv_f32x16& acc = accs[t];
     long at = 0;
     if (PASS != kConvWgrad) {
       const unsigned img = fast_div((unsigned)col, p.d_pix_img);
@@ -659,9 +668,17 @@ static void launch_tile(hipStream_t st, const ConvArgs<T>& a, dim3 grid) {
 // Products of at most 32 rows (few channels) take the 32-row tile.
 static int tile_rows(long M) { return M <= 32 ? 32 : 64; }
 
+// The input gradient in bf16, whose weights are its dearest loads, takes 64 x 128 tiles, which read them half as often, wherever there are
+// more tiles of 64 x 64 than CUs.  us, forward and both gradients, 64 x 64 -> 64 x 128: 128 x 64 x 32 x 32 -> 128 290 -> 256 (2048 tiles of 64 x 64),
+// 32 x 48 x 40 x 40 -> 128 129 -> 118 (800), 32 x 64 x 32 x 32 -> 64 65.9 -> 63.8 (512), 24 x 64 x 28 x 28 -> 64 5 x 5 152 -> 123 (294); 16 x 64 x 32 x 32
+// -> 64 52.7 -> 56.9 (256).  In fp32, which waits for its MFMAs, 0.94 - 1.02 times as fast with most counts; the forward, whose weights come by
+// runs, loses (the second of these 118 -> 126).
 template <typename T, ConvPass PASS>
 static int launch_igemm(hipStream_t st, const char* name, ConvArgs<T>& a, double bytes) {
-  const int bm = tile_rows(a.M), bn = 4096 / bm;
+  constexpr bool WIDER = PASS == kConvDgrad && sizeof(T) == 2;
+  const int bm = tile_rows(a.M);
+  const bool wider = WIDER && bm == 64 && ceil_div(a.M, 64) * ceil_div(a.N, 64) > 256;
+  const int bn = wider ? 128 : 4096 / bm;
   const long tm = ceil_div(a.M, bm), tn = ceil_div(a.N, bn);
   RTP_REQUIRE(tn < (1l << 31) && tm < 65536 && a.splits < 65536, "%s: grid %ld x %ld x %d too large", name, tn, tm, a.splits);
   if (a.splits == 1) a.kchunk = (int)(ceil_div(a.K, kConvSlab) * kConvSlab);
@@ -669,6 +686,8 @@ static int launch_igemm(hipStream_t st, const char* name, ConvArgs<T>& a, double
   const dim3 grid((unsigned)tn, (unsigned)tm, (unsigned)a.splits);
   if (bm == 32)
     launch_tile<T, PASS, 32, 128>(st, a, grid);
+  else if (wider)
+    launch_tile<T, PASS, 64, WIDER ? 128 : 64>(st, a, grid);
   else
     launch_tile<T, PASS, 64, 64>(st, a, grid);
   RTP_LAUNCH_CHECK();

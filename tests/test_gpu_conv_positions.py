@@ -64,3 +64,18 @@ def test_weight_gradient_of_whole_runs(n, ci, h, co, shards, k, s, p, dtype):
     for have, want, terms in ((rows[:, :n_s * kp].reshape(shape), weight, w_abs), (rows[:, n_s * kp:].reshape(co), bias, b_abs)):
         bound = terms * (n * g.ho * g.wo + 1) * 2.0 ** -24 + want.abs() * (2.0 ** -8 if dtype == torch.bfloat16 else 0)
         assert bool(((have - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("n,h,ci,co,p", [(1, 129, 40, 70, 1), (9, 61, 100, 32, 0), (3, 75, 64, 24, 1)])
+def test_input_gradient_of_many_bf16_pixels(n, h, ci, co, p):
+    """More tiles of 64 x 64 than CUs, taken as 64 x 128: ragged last ones, 40 to 100 rows, contractions of whole positions and of mixed slabs,
+    against fp64 on the CPU; inputs of few bits make every sum exact in fp32, so that only the rounding to bf16 is left."""
+    from rtp_amd import ops
+    gen = torch.Generator().manual_seed(co)
+    g = ops.conv_geom((n, ci, h, h), (3, 3), (1, 1), (p, p), (1, 1))
+    dy = torch.randint(-3, 4, (n, co, g.ho, g.wo), generator=gen).to(torch.bfloat16)
+    flat = torch.randint(-3, 4, (2, co // 2 * ci * 9), generator=gen).to(torch.bfloat16)
+    dx = torch.empty(n, ci, h, h, dtype=torch.bfloat16, device=DEV)
+    ops.conv2d_dgrad(dy.to(DEV), g, flat.to(DEV), 0, co // 2, 0, dx)
+    want = torch.nn.grad.conv2d_input((n, ci, h, h), flat.view(co, ci, 3, 3).double(), dy.double(), 1, p)
+    assert torch.equal(dx.cpu(), want.to(torch.bfloat16))

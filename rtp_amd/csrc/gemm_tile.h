@@ -751,14 +751,18 @@ struct WarmAhead {
   unsigned off, lds_dst;
   int left, per_slab;
   __device__ __forceinline__ WarmAhead(const GemmArgs& p, unsigned dst, unsigned wg, unsigned nwg, int wave, int lane, int nk) {
-    const long piece = (long)wg * 4 + wave, step_pieces = (long)nwg * 4;
-    const long total = p.warm == nullptr ? 0 : p.warm_bytes >> 10;
-    const long mine = total > piece ? (total - piece + step_pieces - 1) / step_pieces : 0;
-    left = mine < kWarmMax ? (int)mine : kWarmMax;
-    const int slabs = nk > 0 ? nk - nk / 4 : 1;
-    per_slab = (left + slabs - 1) / slabs;
-    src = p.warm + (piece << 10);
-    step = step_pieces << 10;
+    src = nullptr, step = 0, left = 0, per_slab = 0;
+    if (p.warm != nullptr) {  // (launches without a hint are spared the divisions)
+      const unsigned piece = wg * 4 + wave, step_pieces = nwg * 4;
+      const long all = p.warm_bytes >> 10;
+      const unsigned total = all < (1l << 30) ? (unsigned)all : 1u << 30;
+      const unsigned mine = total > piece ? (total - piece - 1) / step_pieces + 1 : 0;
+      left = mine < (unsigned)kWarmMax ? (int)mine : kWarmMax;
+      const int slabs = nk > 0 ? nk - nk / 4 : 1;  // (0: all at once)
+      per_slab = (left + slabs - 1) / slabs;
+      src = p.warm + ((long)piece << 10);
+      step = (long)step_pieces << 10;
+    }
     off = (unsigned)lane * 16u;
     lds_dst = dst;
   }

@@ -487,8 +487,8 @@ template <int D>
 constexpr int kAhead = D == 128 ? 6 : 3;
 
 // Scores that vector instructions take next, in vector registers.  A kernel of one wave per SIMD has its MFMA results in accumulation
-// registers otherwise, each of which costs a vector instruction of 8 clocks to read.  The compiler does not know what is inside: a
-// reader comes behind scores_settle().
+// registers otherwise, each of which costs a vector instruction of 8 clocks to read.  The compiler does not know what is inside, so it
+// does not wait for the results: scores_settle() does, and hands the registers on, so that no reader can be moved in front of it.
 template <bool ONE_WAVE, bool FIRST>
 __device__ __forceinline__ void mma_scores(bf16x8 a, bf16x8 b, f32x16& c) {
   if constexpr (ONE_WAVE && FIRST)
@@ -498,10 +498,10 @@ __device__ __forceinline__ void mma_scores(bf16x8 a, bf16x8 b, f32x16& c) {
   else
     c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, FIRST ? f32x16{} : c, 0, 0, 0);
 }
-// (a 32 x 32 x 16 MFMA's results are there 11 instructions behind it; two MFMAs more lie between as well)
+// (twelve wait states between a 32 x 32 x 16 MFMA and the first vector instruction that takes its results)
 template <bool ONE_WAVE>
-__device__ __forceinline__ void scores_settle() {
-  if constexpr (ONE_WAVE) asm volatile("s_nop 10" ::: "memory");
+__device__ __forceinline__ void scores_settle(f32x16& s, f32x16& dp) {
+  if constexpr (ONE_WAVE) asm volatile("s_nop 11" : "+v"(s), "+v"(dp));
 }
 
 template <typename T, int D, int NW>
@@ -602,7 +602,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dq_wave
         [&](auto N) __attribute__((always_inline)) {
           constexpr int n = decltype(N)::value;
           if constexpr (n == NA - 4) offsets(0), offsets(1);
-          if constexpr (n == NA || n == 2 * NA) scores_settle<ONE_WAVE>();
+          if constexpr (n == NA || n == 2 * NA) scores_settle<ONE_WAVE>(s[n / NA - 1], dp[n / NA - 1]);
           if constexpr (n >= NA && n < 2 * NA)
             [&]<int... E>(std::integer_sequence<int, E...>) __attribute__((always_inline)) {
               (element(std::integral_constant<int, 0>{}, std::integral_constant<int, (n - NA) * EA + E>{}), ...);
@@ -763,7 +763,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dkv_wav
         [&](auto N) __attribute__((always_inline)) {
           constexpr int n = decltype(N)::value;
           if constexpr (n == NA - 4) stats(0), stats(1);
-          if constexpr (n == NA || n == 2 * NA) scores_settle<ONE_WAVE>();
+          if constexpr (n == NA || n == 2 * NA) scores_settle<ONE_WAVE>(s[n / NA - 1], dp[n / NA - 1]);
           if constexpr (n >= NA && n < 2 * NA)
             [&]<int... E>(std::integer_sequence<int, E...>) __attribute__((always_inline)) {
               (element(std::integral_constant<int, 0>{}, std::integral_constant<int, (n - NA) * EA + E>{}), ...);

@@ -726,8 +726,8 @@ typedef struct {
 int rtp_sgd_step_multi(void* stream, int dtype, const rtp_sgd_chunk* chunks, int64_t n_chunks, float lr,
                        float clip, double total_params);
 
-/* Adam for many buffers in one launch, like rtp_sgd_step_multi: `chunks` is a table in DEVICE memory, one entry per
- * workgroup; the other arguments as for rtp_adam_step.  total_params only feeds the profiler. */
+/* Adam for many buffers in one launch, like rtp_sgd_step_multi: `chunks` is a table in DEVICE memory of less than
+ * 2^24 entries; the other arguments as for rtp_adam_step.  total_params only feeds the profiler. */
 typedef struct {
   float* master;
   const void* grad;

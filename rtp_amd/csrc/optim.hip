@@ -415,7 +415,7 @@ extern "C" int rtp_adam_step_multi(void* stream, int dtype, const rtp_adam_chunk
                                    const int64_t* step_dev, double clip, double total_params) {
   static_assert(sizeof(rtp_adam_chunk) == sizeof(AdamChunk), "rtp_adam_chunk layout");
   RTP_REQUIRE(chunks, "rtp_adam_step_multi: null chunk table");
-  RTP_REQUIRE(n_chunks >= 0 && n_chunks < (1ll << 31), "rtp_adam_step_multi: chunk count %lld out of range",
+  RTP_REQUIRE(n_chunks >= 0 && n_chunks < (1ll << 24), "rtp_adam_step_multi: chunk count %lld out of range",
               (long long)n_chunks);
   RTP_REQUIRE(dtype == RTP_F32 || dtype == RTP_BF16, "rtp_adam_step_multi: unknown dtype %d", dtype);
   RTP_REQUIRE(step_dev || step >= 1, "rtp_adam_step_multi: step counts from 1 (got %lld)", (long long)step);
@@ -432,7 +432,8 @@ extern "C" int rtp_adam_step_multi(void* stream, int dtype, const rtp_adam_chunk
   c.weight_decay = (float)weight_decay, c.clip = (float)clip;
   ProfileScope prof(s, "adam_step", 12.0 * total_params, total_params * (dtype == RTP_F32 ? 32.0 : 28.0));
   const AdamChunk* table = reinterpret_cast<const AdamChunk*>(chunks);
-  const int parts = n_chunks < (1ll << 31) / kAdamParts ? kAdamParts : 1;
+  // a launch has less than 2^32 threads: a table of 2^20 chunks or more (short ones, then) is a workgroup a chunk
+  const int parts = n_chunks * kAdamParts * 256 < (1ll << 32) ? kAdamParts : 1;
   if (dtype == RTP_F32)
     hipLaunchKernelGGL(adam_multi_kernel<float>, dim3((unsigned)n_chunks * parts), dim3(256), 0, s, table, parts, c);
   else

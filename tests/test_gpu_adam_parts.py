@@ -41,3 +41,21 @@ def test_chunks_of_any_length(dtype, offset, device_step):
         ops.adam_step(master, grad.contiguous(), shadow, m, v, step, 1e-3, (0.9, 0.999), 1e-8, 0.01, 0.05)
         for a, b in zip(got, want):
             assert a is None or torch.equal(a, b)
+
+
+def test_more_chunks_than_one_launch_deals_over_parts():
+    """2^20 chunks: sixteen workgroups each would be a launch of 2^32 threads, which is one too many."""
+    from rtp_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    chunks, n = 1 << 20, 3
+    total = chunks * n
+    bufs = [torch.randn(total, generator=gen, device=DEV) * s for s in (1.0, 0.1, 0.01, 0.01)]
+    bufs[3].abs_()
+    want = [b.clone() for b in bufs]
+    first = torch.arange(chunks, dtype=torch.int64, device=DEV) * (4 * n)
+    master, grad, m, v = (b.data_ptr() + first for b in bufs)
+    table = torch.stack([master, grad, torch.zeros_like(first), m, v, torch.full_like(first, n)], dim=1).contiguous()
+    ops.adam_step_multi(table, torch.float32, 7, 1e-3, (0.9, 0.999), 1e-8, 0.01, 0.05, total)
+    ops.adam_step(want[0], want[1], None, want[2], want[3], 7, 1e-3, (0.9, 0.999), 1e-8, 0.01, 0.05)
+    for a, b in zip(bufs, want):
+        assert torch.equal(a, b)

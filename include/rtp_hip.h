@@ -727,7 +727,8 @@ int rtp_sgd_step_multi(void* stream, int dtype, const rtp_sgd_chunk* chunks, int
                        float clip, double total_params);
 
 /* Adam for many buffers in one launch, like rtp_sgd_step_multi: `chunks` is a table in DEVICE memory of less than
- * 2^24 entries; the other arguments as for rtp_adam_step.  total_params only feeds the profiler. */
+ * 2^24 entries; the other arguments as for rtp_adam_step.  total_params, the sum of their n, sizes the launch and feeds the
+ * profiler: no result depends on it. */
 typedef struct {
   float* master;
   const void* grad;

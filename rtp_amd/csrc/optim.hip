@@ -242,15 +242,18 @@ struct AdamChunk {
   float *exp_avg, *exp_avg_sq;
   long n;  // parameters in the chunk
 };
-// A chunk is dealt over kAdamParts workgroups, 1024 parameters each of a full one (16384), four a lane.  Bound by memory, which is faster
-// where the workgroups in flight walk a few MB of each array in order than with streams 64 KiB apart.  294 M parameters in bf16, 8.2 GB,
-// us: a workgroup a chunk, eight accesses in flight a lane, 1566; 2 and 4 workgroups with sixteen in flight 1517 and 1475 - 1497, 8 with eight 1505, 16 with
-// four 1417 (5.8 TB/s); 32 of 128 threads 1460, and 1462 where beta^t is worked out by squaring, so that stores follow the loads at once.
-constexpr int kAdamParts = 16;
+// A chunk is dealt over 1, 2, 4, 8 or 16 workgroups (1 << parts_log2), 1024 parameters each of a full one (16384), four a lane.  Bound by
+// memory, which is faster where the workgroups in flight walk a few MB of each array in order than with streams 64 KiB apart.  294 M
+// parameters in bf16, 8.2 GB, us: a workgroup a chunk, eight accesses in flight a lane, 1566; 2 and 4 workgroups with sixteen in flight 1517
+// and 1475 - 1497, 8 with eight 1505, 16 with four 1417 (5.8 TB/s); 32 of 128 threads 1460, and 1462 where beta^t is worked out by squaring,
+// so that stores follow the loads at once.  Short chunks pay for every workgroup, busy or not: us, a workgroup a chunk (of the kernel before) / always
+// sixteen / as many as their lengths fill: 4096 chunks of 64 with the step count on the device 16.9 / 105 / 10.0, of 1000 24.2 / 171 / 21.7, of 4096
+// 86 / 175 / 77; 16384 of 2100 201 / 689 / 225, of 3000 291 / 699 / 262, of 9000 935 / 863 / 867
+// (at most 1280 a part 924); 256 of 16384 25.6 / 21.0 / 20.9.
 template <typename T>
-__global__ __launch_bounds__(256) void adam_multi_kernel(const AdamChunk* chunks, int parts, AdamScalars c) {
+__global__ __launch_bounds__(256) void adam_multi_kernel(const AdamChunk* chunks, int parts_log2, AdamScalars c) {
   using P = typename Sgd4<T>::Pack;
-  const unsigned chunk = parts == 1 ? blockIdx.x : blockIdx.x / kAdamParts, part = parts == 1 ? 0 : blockIdx.x % kAdamParts;
+  const unsigned chunk = blockIdx.x >> parts_log2, part = blockIdx.x & ((1u << parts_log2) - 1);
   const AdamChunk ch = chunks[chunk];
   const T* grad = reinterpret_cast<const T*>(ch.grad);
   T* shadow = reinterpret_cast<T*>(ch.shadow);
@@ -258,7 +261,8 @@ __global__ __launch_bounds__(256) void adam_multi_kernel(const AdamChunk* chunks
   const long head = max(chunk_head(ch.master, grad, shadow, ch.n),
                         chunk_head<float>(ch.master, ch.exp_avg, ch.exp_avg_sq, ch.n));
   const long n4 = (ch.n - head) >> 2;
-  const long per = ((n4 + parts - 1) / parts + 255) & ~255l, first = part * per, last = min(first + per, n4);
+  const long per = (((n4 - 1) >> parts_log2) + 256) & ~255l, first = part * per, last = min(first + per, n4);
+  if (part != 0 && first >= n4) return;  // a short chunk
   // the bias corrections of a step count in device memory are powers in fp64: one wave's work, beside the first loads
   __shared__ float corrections[2];
   const auto corrected = [&] {
@@ -432,12 +436,15 @@ extern "C" int rtp_adam_step_multi(void* stream, int dtype, const rtp_adam_chunk
   c.weight_decay = (float)weight_decay, c.clip = (float)clip;
   ProfileScope prof(s, "adam_step", 12.0 * total_params, total_params * (dtype == RTP_F32 ? 32.0 : 28.0));
   const AdamChunk* table = reinterpret_cast<const AdamChunk*>(chunks);
-  // a launch has less than 2^32 threads: a table of 2^20 chunks or more (short ones, then) is a workgroup a chunk
-  const int parts = n_chunks * kAdamParts * 256 < (1ll << 32) ? kAdamParts : 1;
+  // parts of at most 1024 parameters of an average chunk, as far as the launch stays below 2^32 threads
+  int parts_log2 = 0;
+  while (parts_log2 < 4 && (double)(1024ll << parts_log2) * (double)n_chunks < total_params && (n_chunks << (parts_log2 + 1)) < (1ll << 24))
+    ++parts_log2;
+  const dim3 grid((unsigned)(n_chunks << parts_log2));
   if (dtype == RTP_F32)
-    hipLaunchKernelGGL(adam_multi_kernel<float>, dim3((unsigned)n_chunks * parts), dim3(256), 0, s, table, parts, c);
+    hipLaunchKernelGGL(adam_multi_kernel<float>, grid, dim3(256), 0, s, table, parts_log2, c);
   else
-    hipLaunchKernelGGL(adam_multi_kernel<bf16_t>, dim3((unsigned)n_chunks * parts), dim3(256), 0, s, table, parts, c);
+    hipLaunchKernelGGL(adam_multi_kernel<bf16_t>, grid, dim3(256), 0, s, table, parts_log2, c);
   RTP_LAUNCH_CHECK();
   return RTP_OK;
 }

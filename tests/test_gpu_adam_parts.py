@@ -14,6 +14,17 @@ LENGTHS = [1, 3, 4, 1020, 1023, 1024, 1028, 4099, 16383, 16384, 16385, 40000]
 @pytest.mark.parametrize("offset", [0, 1, 4])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_chunks_of_any_length(dtype, offset, device_step):
+    _check(dtype, offset, device_step, sum(LENGTHS) + 100003)
+
+
+@pytest.mark.parametrize("average", [0, 1500, 3000, 6000])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_parts_by_the_average_chunk(dtype, average):
+    """1, 2, 4 and 8 parts a chunk (16 above): what the launch is sized by changes no result."""
+    _check(dtype, 1, True, average * (len(LENGTHS) + 1))
+
+
+def _check(dtype, offset, device_step, total):
     from rtp_amd import ops
     gen = torch.Generator(device=DEV).manual_seed(offset)
 
@@ -35,7 +46,7 @@ def test_chunks_of_any_length(dtype, offset, device_step):
     alone.append(tuple(None if t is None else t.clone() for t in long))
     row = [0 if t is None else t.data_ptr() for t in long] + [100003]
     table = torch.cat([table, torch.tensor([row], dtype=torch.int64, device=DEV)])
-    ops.adam_step_multi(table, dtype, step, 1e-3, (0.9, 0.999), 1e-8, 0.01, 0.05, sum(LENGTHS) + 100003)
+    ops.adam_step_multi(table, dtype, step, 1e-3, (0.9, 0.999), 1e-8, 0.01, 0.05, total)
     for got, want in zip(sets + [tuple(long)], alone):
         master, grad, shadow, m, v = want
         ops.adam_step(master, grad.contiguous(), shadow, m, v, step, 1e-3, (0.9, 0.999), 1e-8, 0.01, 0.05)

@@ -611,18 +611,52 @@ static int check_run(const char* who, int dtype, int64_t numel, int64_t shards, 
   return RTP_OK;
 }
 
-// Whether the input gradient contracts slabs of 32 channels at one kernel position each (WHOLE) rather than channels with all
-// their positions: such slabs are filled up to whole ones, which costs MFMAs and saves the tests of every element.  us for
-// both gradients and the forward of 64 x 32 x 28 x 28, fp32 / bf16, mixed slabs -> slabs of a position: 3 x 3, 24 channels 88.8
-// / 65.9 -> 88.3 / 63.8, 20 of 32 84.8 / 62.9 -> 87.5 / 62.7, 40 of 64 109 / 70.3 -> 114 / 70.0; with strides of 2, where an element's test
-// has two divisions, 5 x 5, 20 channels 131 / 97.4 -> 123 / 88.1, 40 170 / 124 -> 161 / 113, 33 of 64 152 / 111 -> 160 / 109.
-static bool whole_positions(long co, bool unit_strides) {
-  const long padded = ceil_div(co, kConvSlab) * kConvSlab;
-  return unit_strides ? 3 * padded <= 4 * co : 5 * padded <= 8 * co;
+// How the input gradient runs.  whole: slabs of 32 channels at one kernel position each (WHOLE) instead of channels with all their positions.
+// They save the tests of every element, are filled up to whole ones, which costs MFMAs, and read a slab's weights khkw elements apart: every
+// position touches the same `lines` lines of each of the 32 channels again, and once those no longer stay in the L1 the weights come from the L2
+// khkw times.  wider: tiles of 64 x 128 (bf16), which read the weights half as often and are half as many.
+// us for the input gradient of 128 x 32 x 32 pixels, channels in -> out (lines of a channel): mixed slabs -> whole ones.
+//   fp32, strides of 1: 3 x 3, 32 -> 64 (9) 70 -> 63, 64 -> 64 (18) 110 -> 124, 64 -> 48 88 -> 110; 5 x 5, 16 -> 64 (13) 173 -> 153, 32 -> 64 (25) 175 ->
+//   210, 64 -> 64 (50) 272 -> 652; 1 x 1, 64 -> 32 24 -> 25, 64 -> 64 27 -> 25.  Strides of 2: 3 x 3, 64 -> 64 150 -> 125; 5 x 5, 32 -> 64 (25) 293 -> 210,
+//   40 -> 64 (32) 379 -> 418.  With a workgroup a CU at most, 16 x 14 x 14: 5 x 5, 32 -> 64 (25) 71 -> 60.
+//   bf16, strides of 1: 3 x 3, 32 -> 64 (5) 40 -> 34, 64 -> 64 (9) 82 -> 66; 5 x 5, 32 -> 64 (13) 93 -> 111, 64 -> 64 (25) 135 -> 327; 4 x 4, 32 -> 64 (8)
+//   60 -> 85, 2 x 2, 64 -> 64 (4) 28 -> 31 (rows of 8, 16 or 32 bytes fall on fewer of the L1's sets).  Strides of 2: 3 x 3, 64 -> 64 95 -> 72; 5 x 5, 32 ->
+//   64 (13) 189 -> 118, 64 -> 64 (25) 204 -> 331.
+// The same in bf16 by 64 x 128, mixed and whole: 3 x 3, 64 -> 64 60 and 49, 64 -> 16 30 -> 29 (whole 31 -> 29); 5 x 5, 64 -> 64 126 and 186, strides of 2 210 and
+// 192; 1 x 1, 64 -> 32 18.8 -> 19.4 (whole 18.6 -> 17.1), 64 -> 8 15.8 -> 18.5.  Fewer pixels, 32 x 32 x 32 (512 tiles of 64 x 64), whole: 1 x 1, 64 -> 64
+// 7.4 -> 8.2, 3 x 3, 64 -> 64 21.6 -> 20; 20 x 30 x 30 (282): 7.4 -> 8.2 and 20.6 -> 19.6.
+struct DgradForm {
+  bool whole, wider;
+};
+template <typename T>
+static DgradForm dgrad_form(const ConvArgs<T>& a) {
+  constexpr bool kBf16 = sizeof(T) == 2;
+  const bool unit = a.g.sh == 1 && a.g.sw == 1, shallow = a.M <= 32;
+  const long co = a.K / a.khkw, padded = ceil_div(co, kConvSlab) * kConvSlab;
+  const bool full = 8 * padded <= 9 * co, most = 3 * padded <= 4 * co, half = 5 * padded <= 8 * co;  // slabs that are filled
+  const long rows = std::min(a.M, 64), lines = std::min<long>(rows, ceil_div(rows * a.khkw * (long)sizeof(T), 128));
+  const long tiles = ceil_div(a.M, 64) * ceil_div(a.N, 64);  // of 64 x 64
+  const int share = (shallow ? ceil_div(a.N, 128) : tiles) <= 256 ? 2 : 1;
+  const bool many = kBf16 && !shallow && tiles > 512, some = kBf16 && !shallow && tiles > 256 && a.khkw >= 9 && co >= 64;
+  DgradForm f;
+  if (a.khkw == 1)
+    f.whole = !unit || shallow || co >= (many ? 32 : 64);
+  else if (unit && shallow)
+    f.whole = (full || (kBf16 && a.khkw <= 9 && most)) && lines <= (kBf16 ? a.khkw % 4 == 0 ? 3 : 9 : 13) * share;
+  else if (unit && a.khkw % 2 == 0)
+    f.whole = full && many && co >= 64 && lines <= 4;
+  else if (unit)
+    f.whole = (full || (kBf16 && most)) && lines <= (kBf16 ? 9 : 12 * share);
+  else if (shallow)
+    f.whole = half && lines <= (kBf16 ? 25 : 32);
+  else
+    f.whole = (most && lines <= (many || some ? 25 : kBf16 ? 10 * share : 20 * share)) || (kBf16 && half && lines <= 9);
+  f.wider = f.whole ? many || some : many && unit && (a.khkw == 1 ? co >= 96 : a.khkw % 2 != 0 && a.khkw >= 9 && a.khkw <= 25 && co >= 16);
+  return f;
 }
 
 template <typename T, ConvPass PASS, int BM, int BN>
-static void launch_tile(hipStream_t st, const ConvArgs<T>& a, dim3 grid) {
+static void launch_tile(hipStream_t st, const ConvArgs<T>& a, dim3 grid, bool whole) {
   const ConvGeom& g = a.g;
   const bool simple = PASS == kConvDgrad ? g.sh == 1 && g.sw == 1 : g.ph == 0 && g.pw == 0;
   // the furthest element of each operand, in bytes from its base
@@ -636,7 +670,7 @@ static void launch_tile(hipStream_t st, const ConvArgs<T>& a, dim3 grid) {
   const bool wide = (far + 1.0) * sizeof(T) >= (double)kBeyond;
 #define RTP_CONV(SIMPLE, WIDE) hipLaunchKernelGGL((conv_igemm_kernel<T, PASS, BM, BN, SIMPLE, WIDE>), grid, dim3(256), 0, st, a)
   if constexpr (PASS == kConvDgrad)
-    if (!wide && whole_positions(co, simple)) {
+    if (!wide && whole) {
       ConvArgs<T> b = a;
       b.co = (int)co, b.K = b.kchunk = (int)(ceil_div(co, kConvSlab) * kConvSlab) * a.khkw;
       if (simple)
@@ -668,28 +702,22 @@ static void launch_tile(hipStream_t st, const ConvArgs<T>& a, dim3 grid) {
 // Products of at most 32 rows (few channels) take the 32-row tile.
 static int tile_rows(long M) { return M <= 32 ? 32 : 64; }
 
-// The input gradient in bf16, whose weights are its dearest loads, takes 64 x 128 tiles, which read them half as often, wherever there are
-// more tiles of 64 x 64 than CUs.  us, forward and both gradients, 64 x 64 -> 64 x 128: 128 x 64 x 32 x 32 -> 128 290 -> 256 (2048 tiles of 64 x 64),
-// 32 x 48 x 40 x 40 -> 128 129 -> 118 (800), 32 x 64 x 32 x 32 -> 64 65.9 -> 63.8 (512), 24 x 64 x 28 x 28 -> 64 5 x 5 152 -> 123 (294); 16 x 64 x 32 x 32
-// -> 64 52.7 -> 56.9 (256).  In fp32, which waits for its MFMAs, 0.94 - 1.02 times as fast with most counts; the forward, whose weights come by
-// runs, loses (the second of these 118 -> 126).
 template <typename T, ConvPass PASS>
 static int launch_igemm(hipStream_t st, const char* name, ConvArgs<T>& a, double bytes) {
   constexpr bool WIDER = PASS == kConvDgrad && sizeof(T) == 2;
-  const int bm = tile_rows(a.M);
-  const bool wider = WIDER && bm == 64 && ceil_div(a.M, 64) * ceil_div(a.N, 64) > 256;
-  const int bn = wider ? 128 : 4096 / bm;
+  const DgradForm form = PASS == kConvDgrad ? dgrad_form(a) : DgradForm{};
+  const int bm = tile_rows(a.M), bn = form.wider ? 128 : 4096 / bm;
   const long tm = ceil_div(a.M, bm), tn = ceil_div(a.N, bn);
   RTP_REQUIRE(tn < (1l << 31) && tm < 65536 && a.splits < 65536, "%s: grid %ld x %ld x %d too large", name, tn, tm, a.splits);
   if (a.splits == 1) a.kchunk = (int)(ceil_div(a.K, kConvSlab) * kConvSlab);
   ProfileScope prof(st, name, 2.0 * (double)a.M * (double)a.N * (double)a.K, bytes);
   const dim3 grid((unsigned)tn, (unsigned)tm, (unsigned)a.splits);
   if (bm == 32)
-    launch_tile<T, PASS, 32, 128>(st, a, grid);
-  else if (wider)
-    launch_tile<T, PASS, 64, WIDER ? 128 : 64>(st, a, grid);
+    launch_tile<T, PASS, 32, 128>(st, a, grid, form.whole);
+  else if (form.wider)
+    launch_tile<T, PASS, 64, WIDER ? 128 : 64>(st, a, grid, form.whole);
   else
-    launch_tile<T, PASS, 64, 64>(st, a, grid);
+    launch_tile<T, PASS, 64, 64>(st, a, grid, form.whole);
   RTP_LAUNCH_CHECK();
   return RTP_OK;
 }

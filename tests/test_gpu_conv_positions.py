@@ -14,7 +14,11 @@ pytestmark = pytest.mark.gpu
     (2, 3, 9, 11, 32, 1, (3, 3), (1, 1), (0, 0), (1, 1)), (1, 33, 7, 8, 24, 3, (3, 2), (1, 1), (1, 2), (1, 2)),
     (3, 70, 6, 6, 48, 4, (1, 1), (1, 1), (0, 0), (1, 1)), (2, 32, 13, 12, 20, 2, (5, 3), (2, 1), (2, 1), (1, 1)),
     (1, 65, 17, 16, 40, 8, (3, 3), (3, 2), (1, 0), (2, 1)), (2, 8, 10, 10, 66, 3, (3, 3), (1, 1), (1, 1), (1, 1)),
-    (1, 1, 5, 5, 160, 5, (5, 5), (1, 1), (2, 2), (1, 1))])
+    (1, 1, 5, 5, 160, 5, (5, 5), (1, 1), (2, 2), (1, 1)),
+    # 33 to 64 rows by positions in both types, the last slab not full; 5 x 5 weights that are read as they lie, and a few tiles of them
+    (3, 70, 6, 6, 72, 4, (1, 1), (1, 1), (0, 0), (1, 1)), (2, 40, 9, 9, 29, 1, (3, 3), (1, 1), (1, 1), (1, 1)),
+    (1, 65, 17, 16, 48, 8, (3, 3), (3, 2), (1, 0), (2, 1)), (1, 64, 9, 9, 32, 2, (5, 5), (1, 1), (2, 2), (1, 1)),
+    (2, 16, 8, 8, 30, 3, (5, 5), (1, 1), (2, 2), (1, 1)), (1, 40, 12, 12, 64, 4, (2, 2), (1, 1), (0, 0), (1, 1))])
 def test_input_gradient_against_torch(n, ci, h, w, co, shards, k, s, p, d, dtype):
     from rtp_amd import ops
     gen = torch.Generator().manual_seed(co + h)
@@ -66,9 +70,10 @@ def test_weight_gradient_of_whole_runs(n, ci, h, co, shards, k, s, p, dtype):
         assert bool(((have - want).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("n,h,ci,co,p", [(1, 129, 40, 70, 1), (9, 61, 100, 32, 0), (3, 75, 64, 24, 1)])
+@pytest.mark.parametrize("n,h,ci,co,p", [(1, 129, 40, 70, 1), (9, 61, 100, 32, 0), (3, 75, 64, 24, 1), (2, 129, 40, 70, 1), (6, 75, 64, 24, 1),
+                                         (6, 75, 33, 22, 0)])
 def test_input_gradient_of_many_bf16_pixels(n, h, ci, co, p):
-    """More tiles of 64 x 64 than CUs, taken as 64 x 128: ragged last ones, 40 to 100 rows, contractions of whole positions and of mixed slabs,
+    """More tiles of 64 x 64 than CUs or twice as many, some taken as 64 x 128: ragged last ones, 40 to 100 rows, contractions of whole positions and of mixed slabs,
     against fp64 on the CPU; inputs of few bits make every sum exact in fp32, so that only the rounding to bf16 is left."""
     from rtp_amd import ops
     gen = torch.Generator().manual_seed(co)

@@ -145,8 +145,9 @@ constexpr int kOutside = 1 << 30;
 // Forward: a thread takes NA consecutive weights of a row by one load or two at any alignment instead of NA loads (128 x 64 x 32 x 32 -> 128
 // padded in bf16, forward and both gradients 332 -> 317 us, MNIST's second convolution in fp32 96.6 -> 94.9).
 // WHOLE (weight gradient): runs of NA output pixels of a plane are whole and aligned in dy and come by one load or two, as the forward's weights
-// do (launch_tile has the rule; the same case 317 -> 291 us, in 64-row tiles 1 - 9 %, in those of 32 rows no difference).  The bias gradient's 32
-// chains of additions a row are the same ones on either way.
+// do (launch_tile has the rule; the same case 317 -> 291 us, in 64-row tiles 1 - 9 %).  In tiles of 32 rows they are read one by one: runs took 2 - 4 %
+// longer there in bf16 with kernels of 3 x 3 and 5 x 5 (128 x 40 x 56 x 56 -> 16, 5 x 5, 163 -> 169 us), and in fp32 no less.  The bias gradient's 32 chains
+// of additions a row are the same ones on either way.
 // WHOLE (input gradient): a slab is 32 channels at one kernel position, so a pixel's neighbour is tested and, with strides, divided
 // for once a slab, the rest is scalar and there is no table; a slab's weights lie khkw elements apart, and a wave's lanes run along the input
 // channels, where 64 of them share ten lines.  us, forward and both gradients, before -> after (the input gradient's share): MNIST's second
@@ -679,7 +680,7 @@ static void launch_tile(hipStream_t st, const ConvArgs<T>& a, dim3 grid, bool wh
         hipLaunchKernelGGL((conv_igemm_kernel<T, PASS, BM, BN, false, false, true>), grid, dim3(256), 0, st, b);
       return;
     }
-  if constexpr (PASS == kConvWgrad) {  // dy contiguous, and planes and images whole aligned runs
+  if constexpr (PASS == kConvWgrad && BM == 64) {  // dy contiguous, and planes and images whole aligned runs
     constexpr int NA = BM * kConvSlab / 256;
     if (!wide && a.sd.w == 1 && a.sd.h == g.wo && (long)g.ho * g.wo % NA == 0 && a.sd.n % NA == 0 && a.sd.c % NA == 0 &&
         reinterpret_cast<uintptr_t>(a.dy) % std::min<size_t>(16, NA * sizeof(T)) == 0) {

@@ -338,24 +338,29 @@ __global__ __launch_bounds__(256) void conv_igemm_kernel(ConvArgs<T> p) {
     }
     const int slot = PASS == kConvWgrad ? 0 : slab & 3;
     if constexpr (RUNS) {
-      if (k0 + kConvSlab <= p.K) {
+      const int left = p.K - (k0 + rk);  // weights of the row from this run on
+      auto whole = [&] {
         const AnyRun run = *reinterpret_cast<const AnyRun*>(run_row + k0 + rk);
 #pragma unroll
         for (int q = 0; q < RUNW; ++q) v.run[q] = run.w[q];
+      };
+      if (k0 + kConvSlab <= p.K) {
+        whole();
       } else {  // the slab that the contraction ends in, or one behind it
-        PackedRun u;
 #pragma unroll
-        for (int q = 0; q < RUNW; ++q) u.w[q] = 0;
-        if (k0 < p.K) {
+        for (int q = 0; q < RUNW; ++q) v.run[q] = 0;
+        if (left >= NA) {
+          whole();
+        } else if (left > 0) {  // the run that it ends in: the only one that is waited for here
+          PackedRun u;
 #pragma unroll
           for (int q = 0; q < NA; ++q) {
-            const int k = k0 + rk + q;
-            const T t = run_row[min(k, p.K - 1)];
-            u.e[q] = k < p.K ? t : from_f32<T>(0.0f);
+            const T t = run_row[k0 + rk + min(q, left - 1)];
+            u.e[q] = q < left ? t : from_f32<T>(0.0f);
           }
-        }
 #pragma unroll
-        for (int q = 0; q < RUNW; ++q) v.run[q] = u.w[q];
+          for (int q = 0; q < RUNW; ++q) v.run[q] = u.w[q];
+        }
       }
     } else {
       const bool live = k0 + ak < ke;

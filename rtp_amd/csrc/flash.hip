@@ -485,6 +485,28 @@ __device__ __forceinline__ void mfma_stream(Read read, Mul mul, Between between)
 }
 template <int D>
 constexpr int kAhead = D == 128 ? 6 : 3;
+// Both groups of a block in one stream: 2 * NA products that form their scores, 2 * NC that use them.  The vector work on the first group's
+// 16 scores a lane lies under the products that form the second's, that on the second's under the products that use the first's.
+// begin(): what the elements need besides the scores; settle(h): group h's scores are read from here on.
+template <typename Frag, int NA, int NC, int AHEAD, typename Read, typename Mul, typename Begin, typename Settle, typename Element>
+__device__ __forceinline__ void block_stream(Read read, Mul mul, Begin begin, Settle settle, Element element) {
+  mfma_stream<Frag, 2 * NA + 2 * NC, AHEAD>(read, mul, [&](auto N) __attribute__((always_inline)) {
+    constexpr int n = decltype(N)::value, EA = 16 / NA, EC = 16 / NC;
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    if constexpr (n == NA - 4) begin();
+    if constexpr (n == NA) settle(I0{});
+    if constexpr (n == 2 * NA) settle(I1{});
+    if constexpr (n >= NA && n < 2 * NA)
+      [&]<int... E>(std::integer_sequence<int, E...>) __attribute__((always_inline)) {
+        (element(I0{}, std::integral_constant<int, (n - NA) * EA + E>{}), ...);
+      }(std::make_integer_sequence<int, EA>{});
+    if constexpr (n >= 2 * NA && n < 2 * NA + NC)
+      [&]<int... E>(std::integer_sequence<int, E...>) __attribute__((always_inline)) {
+        (element(I1{}, std::integral_constant<int, (n - 2 * NA) * EC + E>{}), ...);
+      }(std::make_integer_sequence<int, EC>{});
+  });
+}
 
 // Scores that vector instructions take next, in vector registers.  A kernel of one wave per SIMD has its MFMA results in accumulation
 // registers otherwise, each of which costs a vector instruction of 8 clocks to read.  The compiler does not know what is inside, so it
@@ -551,7 +573,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dq_wave
   landed(qf);
   landed(gf);
   asm volatile("" : "+v"(lse));
-  if (!kbias && wave == 0) {  // both stages of the bias are read all the same
+  if (kInterleaveDq<D> && !kbias && wave == 0) {  // both stages of the bias are read all the same
     reinterpret_cast<float*>(lds + 4 * B::BYTES)[lane] = 0.0f;
     reinterpret_cast<float*>(lds + 4 * B::BYTES)[64 + lane] = 0.0f;
   }
@@ -562,71 +584,58 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dq_wave
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[db][r] = 0.0f;
 
-  // Both groups of a block, all of whose keys the wave's queries see (as in flash_dkv_kernel).
-  auto both = [&](const char* ks, const char* vs, const float* bias) __attribute__((always_inline)) {
-    constexpr int NA = 2 * NK, NC = NM * DB, EA = 16 / NA, EC = 16 / NC;
-    constexpr bool ONE_WAVE = dq_waves<T, D>() == 1;
-    f32x16 s[2], dp[2];
-    Frag df[2][NM];
-    f32x4 off[2];
-    auto offsets = [&](int quarter) __attribute__((always_inline)) {
-      off[quarter & 1] = *reinterpret_cast<const f32x4*>(bias + 8 * quarter + 4 * g);
-    };
-    auto element = [&](auto Hc, auto R) __attribute__((always_inline)) {
-      constexpr int h = decltype(Hc)::value, r = decltype(R)::value;
-      const float p = __builtin_amdgcn_exp2f(fmaf(s[h][r], a.scale, -lse + off[r / 4 & 1][r % 4]) * kLog2e);
-      df[h][r / Op<T>::MR][r % Op<T>::MR] = from_f32<T>(p * (dp[h][r] - delta[0]));
-      if constexpr (r % 4 == 3 && 4 * h + r / 4 + 2 < 8) offsets(4 * h + r / 4 + 2);
-    };
-    mfma_stream<Frag, 2 * NA + 2 * NC, kAhead<D>>(
-        [&](auto N) __attribute__((always_inline)) {
-          constexpr int n = decltype(N)::value, c = n - 2 * NA;
-          if constexpr (n < 2 * NA)
-            return B::rows(n & 1 ? vs : ks, lrow, n / NA, n % NA / 2);
-          else
-            return B::cols(ks, lcol, c / NC, c % NC / DB, c % DB);
-        },
-        [&](auto N, const Frag& f) __attribute__((always_inline)) {
-          constexpr int n = decltype(N)::value, c = n - 2 * NA;
-          if constexpr (n < 2 * NA) {
-            constexpr int h = n / NA, i = n % NA / 2;
-            if constexpr (n & 1)
-              mma_scores<ONE_WAVE, i == 0>(f, gf[i], dp[h]);
-            else
-              mma_scores<ONE_WAVE, i == 0>(f, qf[i], s[h]);
-          } else {
-            constexpr int h = c / NC, m = c % NC / DB, db = c % DB;
-            acc[db] = Op<T>::mma(f, df[h][m], acc[db]);
-          }
-        },
-        [&](auto N) __attribute__((always_inline)) {
-          constexpr int n = decltype(N)::value;
-          if constexpr (n == NA - 4) offsets(0), offsets(1);
-          if constexpr (n == NA || n == 2 * NA) scores_settle<ONE_WAVE>(s[n / NA - 1], dp[n / NA - 1]);
-          if constexpr (n >= NA && n < 2 * NA)
-            [&]<int... E>(std::integer_sequence<int, E...>) __attribute__((always_inline)) {
-              (element(std::integral_constant<int, 0>{}, std::integral_constant<int, (n - NA) * EA + E>{}), ...);
-            }(std::make_integer_sequence<int, EA>{});
-          if constexpr (n >= 2 * NA && n < 2 * NA + NC)
-            [&]<int... E>(std::integer_sequence<int, E...>) __attribute__((always_inline)) {
-              (element(std::integral_constant<int, 1>{}, std::integral_constant<int, (n - 2 * NA) * EC + E>{}), ...);
-            }(std::make_integer_sequence<int, EC>{});
-        });
-  };
   auto next = [&](int kb) __attribute__((always_inline)) {
     block_barrier();
     keep_in_loop(lrow, lcol);
     if (kb + 1 < nkb) issue(kb + 1);
     return lds + (kb & 1) * 2 * B::BYTES;
   };
-  // blocks whose keys all of the wave's queries see (a loop of its own: two ways through one loop would move the accumulators about)
   int kb = 0;
-  const int whole = !kInterleaveDq<D> || a.mask || q0 >= a.L ? 0 : min(a.causal ? (q0 + 1) / ROWS : nkb, a.S / ROWS);
-  if constexpr (kInterleaveDq<D>)
+  // blocks whose keys all of the wave's queries see (a loop of its own: two ways through one loop would move the accumulators about)
+  if constexpr (kInterleaveDq<D>) {
+    auto both = [&](const char* ks, const char* vs, const float* bias) __attribute__((always_inline)) {
+      constexpr int NA = 2 * NK, NC = NM * DB;
+      f32x16 s[2], dp[2];
+      Frag df[2][NM];
+      f32x4 off[2];
+      auto offsets = [&](int quarter) __attribute__((always_inline)) {
+        off[quarter & 1] = *reinterpret_cast<const f32x4*>(bias + 8 * quarter + 4 * g);
+      };
+      auto element = [&](auto Hc, auto R) __attribute__((always_inline)) {
+        constexpr int h = decltype(Hc)::value, r = decltype(R)::value;
+        const float p = __builtin_amdgcn_exp2f(fmaf(s[h][r], a.scale, -lse + off[r / 4 & 1][r % 4]) * kLog2e);
+        df[h][r / Op<T>::MR][r % Op<T>::MR] = from_f32<T>(p * (dp[h][r] - delta[0]));
+        if constexpr (r % 4 == 3 && 4 * h + r / 4 + 2 < 8) offsets(4 * h + r / 4 + 2);
+      };
+      block_stream<Frag, NA, NC, kAhead<D>>(
+          [&](auto N) __attribute__((always_inline)) {
+            constexpr int n = decltype(N)::value, c = n - 2 * NA;
+            if constexpr (n < 2 * NA)
+              return B::rows(n & 1 ? vs : ks, lrow, n / NA, n % NA / 2);
+            else
+              return B::cols(ks, lcol, c / NC, c % NC / DB, c % DB);
+          },
+          [&](auto N, const Frag& f) __attribute__((always_inline)) {
+            constexpr int n = decltype(N)::value, c = n - 2 * NA;
+            if constexpr (n < 2 * NA) {
+              constexpr int h = n / NA, i = n % NA / 2;
+              if constexpr (n & 1)
+                dp[h] = Op<T>::mma(f, gf[i], i == 0 ? f32x16{} : dp[h]);
+              else
+                s[h] = Op<T>::mma(f, qf[i], i == 0 ? f32x16{} : s[h]);
+            } else {
+              constexpr int h = c / NC, m = c % NC / DB, db = c % DB;
+              acc[db] = Op<T>::mma(f, df[h][m], acc[db]);
+            }
+          },
+          [&]() __attribute__((always_inline)) { offsets(0), offsets(1); }, [](auto) {}, element);
+    };
+    const int whole = a.mask || q0 >= a.L ? 0 : min(a.causal ? (q0 + 1) / ROWS : nkb, a.S / ROWS);
     for (; kb < whole; ++kb) {
       const char* ks = next(kb);
       both(ks, ks + B::BYTES, reinterpret_cast<const float*>(lds + 4 * B::BYTES) + (kb & 1) * 64);
     }
+  }
   for (; kb < nkb; ++kb) {
     const char* ks = next(kb);
     const char* vs = ks + B::BYTES;
@@ -715,65 +724,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dkv_wav
 #pragma unroll
     for (int r = 0; r < 16; ++r) dk[db][r] = dv[db][r] = 0.0f;
 
-  // Both groups of a block, all of whose queries see all of the wave's keys: the vector work on the first group's scores lies under the
-  // products that form the second's, and that on the second's under the products that use the first's.
-  auto both = [&](const char* qs, const char* gs, const float* stat) __attribute__((always_inline)) {
-    constexpr int NA = 2 * NK, NC = 2 * NM * DB, EA = 16 / NA, EC = 16 / NC;
-    constexpr bool ONE_WAVE = dkv_waves<T, D>() == 1;
-    f32x16 s[2], dp[2];
-    Frag pf[2][NM], df[2][NM];
-    f32x4 off[2], delta[2];
-    auto stats = [&](int quarter) __attribute__((always_inline)) {  // of the block's queries: eight, four of them this lane's
-      off[quarter & 1] = *reinterpret_cast<const f32x4*>(stat + 8 * quarter + 4 * g);
-      delta[quarter & 1] = *reinterpret_cast<const f32x4*>(stat + 64 + 8 * quarter + 4 * g);
-    };
-    auto element = [&](auto Hc, auto R) __attribute__((always_inline)) {
-      constexpr int h = decltype(Hc)::value, r = decltype(R)::value;
-      const float p = __builtin_amdgcn_exp2f(fmaf(s[h][r], a.scale, kb - off[r / 4 & 1][r % 4]) * kLog2e);
-      const float ds = p * (dp[h][r] - delta[r / 4 & 1][r % 4]);
-      constexpr int MR = Op<T>::MR;
-      pf[h][r / MR][r % MR] = from_f32<T>(p);
-      df[h][r / MR][r % MR] = from_f32<T>(ds);
-      if constexpr (r % 4 == 3 && 4 * h + r / 4 + 2 < 8) stats(4 * h + r / 4 + 2);
-    };
-    mfma_stream<Frag, 2 * NA + 2 * NC, kAhead<D>>(
-        [&](auto N) __attribute__((always_inline)) {
-          constexpr int n = decltype(N)::value, c = n - 2 * NA, w = n & 1;
-          if constexpr (n < 2 * NA)
-            return B::rows(w ? gs : qs, lrow, n / NA, n % NA / 2);
-          else
-            return B::cols(w ? qs : gs, lcol, c / NC, c % NC / (2 * DB), c % (2 * DB) / 2);
-        },
-        [&](auto N, const Frag& f) __attribute__((always_inline)) {
-          constexpr int n = decltype(N)::value, c = n - 2 * NA, w = n & 1;
-          if constexpr (n < 2 * NA) {
-            constexpr int h = n / NA, i = n % NA / 2;
-            if constexpr (w)
-              mma_scores<ONE_WAVE, i == 0>(f, vf[i], dp[h]);
-            else
-              mma_scores<ONE_WAVE, i == 0>(f, kf[i], s[h]);
-          } else {
-            constexpr int h = c / NC, m = c % NC / (2 * DB), db = c % (2 * DB) / 2;
-            if constexpr (w)
-              dk[db] = Op<T>::mma(f, df[h][m], dk[db]);
-            else
-              dv[db] = Op<T>::mma(f, pf[h][m], dv[db]);
-          }
-        },
-        [&](auto N) __attribute__((always_inline)) {
-          constexpr int n = decltype(N)::value;
-          if constexpr (n == NA - 4) stats(0), stats(1);
-          if constexpr (n == NA || n == 2 * NA) scores_settle<ONE_WAVE>(s[n / NA - 1], dp[n / NA - 1]);
-          if constexpr (n >= NA && n < 2 * NA)
-            [&]<int... E>(std::integer_sequence<int, E...>) __attribute__((always_inline)) {
-              (element(std::integral_constant<int, 0>{}, std::integral_constant<int, (n - NA) * EA + E>{}), ...);
-            }(std::make_integer_sequence<int, EA>{});
-          if constexpr (n >= 2 * NA && n < 2 * NA + NC)
-            [&]<int... E>(std::integer_sequence<int, E...>) __attribute__((always_inline)) {
-              (element(std::integral_constant<int, 1>{}, std::integral_constant<int, (n - 2 * NA) * EC + E>{}), ...);
-            }(std::make_integer_sequence<int, EC>{});
-        });
-  };
   auto next = [&](int qb) __attribute__((always_inline)) {
     block_barrier();
     keep_in_loop(lrow, lcol);
@@ -817,16 +767,62 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dkv_wav
         }
     }
   };
-  // blocks whose queries all see all of the wave's keys (loops of their own: two ways through one loop would move the accumulators about)
-  const int whole0 = !kInterleaveDkv<D> || a.mask || k0 >= a.S ? nqb : a.causal ? (k0 + 31 + ROWS - 1) / ROWS : first, whole1 = a.L / ROWS;
   int qb = first;
-  if constexpr (kInterleaveDkv<D>)
+  // blocks whose queries all see all of the wave's keys (loops of their own: two ways through one loop would move the accumulators about)
+  if constexpr (kInterleaveDkv<D>) {
+    auto both = [&](const char* qs, const char* gs, const float* stat) __attribute__((always_inline)) {
+      constexpr int NA = 2 * NK, NC = 2 * NM * DB;
+      constexpr bool ONE_WAVE = dkv_waves<T, D>() == 1;
+      f32x16 s[2], dp[2];
+      Frag pf[2][NM], df[2][NM];
+      f32x4 off[2], delta[2];
+      auto stats = [&](int quarter) __attribute__((always_inline)) {  // of the block's queries: eight, four of them this lane's
+        off[quarter & 1] = *reinterpret_cast<const f32x4*>(stat + 8 * quarter + 4 * g);
+        delta[quarter & 1] = *reinterpret_cast<const f32x4*>(stat + 64 + 8 * quarter + 4 * g);
+      };
+      auto element = [&](auto Hc, auto R) __attribute__((always_inline)) {
+        constexpr int h = decltype(Hc)::value, r = decltype(R)::value;
+        const float p = __builtin_amdgcn_exp2f(fmaf(s[h][r], a.scale, kb - off[r / 4 & 1][r % 4]) * kLog2e);
+        const float ds = p * (dp[h][r] - delta[r / 4 & 1][r % 4]);
+        constexpr int MR = Op<T>::MR;
+        pf[h][r / MR][r % MR] = from_f32<T>(p);
+        df[h][r / MR][r % MR] = from_f32<T>(ds);
+        if constexpr (r % 4 == 3 && 4 * h + r / 4 + 2 < 8) stats(4 * h + r / 4 + 2);
+      };
+      block_stream<Frag, NA, NC, kAhead<D>>(
+          [&](auto N) __attribute__((always_inline)) {
+            constexpr int n = decltype(N)::value, c = n - 2 * NA, w = n & 1;
+            if constexpr (n < 2 * NA)
+              return B::rows(w ? gs : qs, lrow, n / NA, n % NA / 2);
+            else
+              return B::cols(w ? qs : gs, lcol, c / NC, c % NC / (2 * DB), c % (2 * DB) / 2);
+          },
+          [&](auto N, const Frag& f) __attribute__((always_inline)) {
+            constexpr int n = decltype(N)::value, c = n - 2 * NA, w = n & 1;
+            if constexpr (n < 2 * NA) {
+              constexpr int h = n / NA, i = n % NA / 2;
+              if constexpr (w)
+                mma_scores<ONE_WAVE, i == 0>(f, vf[i], dp[h]);
+              else
+                mma_scores<ONE_WAVE, i == 0>(f, kf[i], s[h]);
+            } else {
+              constexpr int h = c / NC, m = c % NC / (2 * DB), db = c % (2 * DB) / 2;
+              if constexpr (w)
+                dk[db] = Op<T>::mma(f, df[h][m], dk[db]);
+              else
+                dv[db] = Op<T>::mma(f, pf[h][m], dv[db]);
+            }
+          },
+          [&]() __attribute__((always_inline)) { stats(0), stats(1); },
+          [&](auto Hc) __attribute__((always_inline)) { scores_settle<ONE_WAVE>(s[decltype(Hc)::value], dp[decltype(Hc)::value]); }, element);
+    };
+    const int whole0 = a.mask || k0 >= a.S ? nqb : a.causal ? (k0 + 31 + ROWS - 1) / ROWS : first, whole1 = a.L / ROWS;
     for (; qb < min(whole0, nqb); ++qb) any(qb);
-  if constexpr (kInterleaveDkv<D>)
     for (; qb < whole1; ++qb) {
       const char* qs = next(qb);
       both(qs, qs + B::BYTES, reinterpret_cast<const float*>(lds + 4 * B::BYTES) + (qb & 1) * 128);
     }
+  }
   for (; qb < nqb; ++qb) any(qb);
   block_barrier();  // every wave has left the last block
   store_rows<T, D>(lds + wave * 64 * B::PITCH, dk, a.scale, a.dk + it.k + k0 * a.k_l, a.k_l, a.S - k0, lane);

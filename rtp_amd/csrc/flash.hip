@@ -263,9 +263,9 @@ template <typename T, int D, bool ADD>
 constexpr int fwd_waves() {
   return D == 128 ? 2 : D == 64 && ADD ? 3 : 4;
 }
-template <typename T, int D>
+template <int D, bool INTERLEAVE>
 constexpr int dq_waves() {
-  return D == 32 ? 4 : 2;
+  return D == 128 || INTERLEAVE ? 2 : D == 64 ? 3 : 4;
 }
 template <typename T, int D>
 constexpr int dkv_waves() {
@@ -526,8 +526,9 @@ __device__ __forceinline__ void scores_settle(f32x16& s, f32x16& dp) {
   if constexpr (ONE_WAVE) asm volatile("s_nop 11" : "+v"(s), "+v"(dp));
 }
 
-template <typename T, int D, int NW>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dq_waves<T, D>()))) void flash_dq_kernel(
+// INTERLEAVE: blocks all of whose keys the wave's queries see go through a loop of their own, see kInterleaveDq.
+template <typename T, int D, int NW, bool INTERLEAVE>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dq_waves<D, INTERLEAVE>()))) void flash_dq_kernel(
     FlashArgs a) {
   touch_kernel_arguments<sizeof(FlashArgs)>();
   typedef Block<T, D, NW> B;
@@ -573,7 +574,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dq_wave
   landed(qf);
   landed(gf);
   asm volatile("" : "+v"(lse));
-  if (kInterleaveDq<D> && !kbias && wave == 0) {  // both stages of the bias are read all the same
+  if (INTERLEAVE && !kbias && wave == 0) {  // both stages of the bias are read all the same
     reinterpret_cast<float*>(lds + 4 * B::BYTES)[lane] = 0.0f;
     reinterpret_cast<float*>(lds + 4 * B::BYTES)[64 + lane] = 0.0f;
   }
@@ -592,7 +593,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dq_wave
   };
   int kb = 0;
   // blocks whose keys all of the wave's queries see (a loop of its own: two ways through one loop would move the accumulators about)
-  if constexpr (kInterleaveDq<D>) {
+  if constexpr (INTERLEAVE) {
     auto both = [&](const char* ks, const char* vs, const float* bias) __attribute__((always_inline)) {
       constexpr int NA = 2 * NK, NC = NM * DB;
       f32x16 s[2], dp[2];
@@ -630,7 +631,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dq_wave
           },
           [&]() __attribute__((always_inline)) { offsets(0), offsets(1); }, [](auto) {}, element);
     };
-    const int whole = a.mask || q0 >= a.L ? 0 : min(a.causal ? (q0 + 1) / ROWS : nkb, a.S / ROWS);
+    const int whole = q0 >= a.L ? 0 : min(a.causal ? (q0 + 1) / ROWS : nkb, a.S / ROWS);
     for (; kb < whole; ++kb) {
       const char* ks = next(kb);
       both(ks, ks + B::BYTES, reinterpret_cast<const float*>(lds + 4 * B::BYTES) + (kb & 1) * 64);
@@ -652,7 +653,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dq_wave
 #pragma unroll
         for (int r = 0; r < 16; ++r) off[r] += kb16[r];
       }
-      add_mask<true>(a, query, k0, g, 1.0f, off);
+      if constexpr (!INTERLEAVE) add_mask<true>(a, query, k0, g, 1.0f, off);
       f32x16 s, dp;
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.0f;
@@ -680,7 +681,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dq_wave
 // Key pass.  Scores are formed as S[query][key] (A = Q rows, B = K rows), so a lane is a KEY and its 16 accumulator
 // registers run over queries: P and dS are then, as they stand, the B operands "lane = key, slots = queries" of
 // dV^T = dO^T P and dK^T = Q^T dS, and the per-query statistics come in from LDS, 16 values per lane.
-template <typename T, int D, int NW>
+// INTERLEAVE: blocks whose queries all see all of the wave's keys go through a loop of their own, see kInterleaveDkv.
+template <typename T, int D, int NW, bool INTERLEAVE>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dkv_waves<T, D>()))) void flash_dkv_kernel(
     FlashArgs a) {
   touch_kernel_arguments<sizeof(FlashArgs)>();
@@ -751,7 +753,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dkv_wav
       lds_values(stat + 64 + 32 * h, g, delta);
 #pragma unroll
       for (int r = 0; r < 16; ++r) off[r] = kb - off[r];
-      add_mask<false>(a, key, q0, g, 1.0f, off);
+      if constexpr (!INTERLEAVE) add_mask<false>(a, key, q0, g, 1.0f, off);
       const bool edge = q0 + 32 > a.L || (a.causal && k0 + 31 > q0);
       p_and_ds<false>(a, s, dp, off, delta, key, q0, g, edge, p, ds);
       Frag pf[NM], df[NM];
@@ -769,7 +771,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dkv_wav
   };
   int qb = first;
   // blocks whose queries all see all of the wave's keys (loops of their own: two ways through one loop would move the accumulators about)
-  if constexpr (kInterleaveDkv<D>) {
+  if constexpr (INTERLEAVE) {
     auto both = [&](const char* qs, const char* gs, const float* stat) __attribute__((always_inline)) {
       constexpr int NA = 2 * NK, NC = 2 * NM * DB;
       constexpr bool ONE_WAVE = dkv_waves<T, D>() == 1;
@@ -816,7 +818,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(dkv_wav
           [&]() __attribute__((always_inline)) { stats(0), stats(1); },
           [&](auto Hc) __attribute__((always_inline)) { scores_settle<ONE_WAVE>(s[decltype(Hc)::value], dp[decltype(Hc)::value]); }, element);
     };
-    const int whole0 = a.mask || k0 >= a.S ? nqb : a.causal ? (k0 + 31 + ROWS - 1) / ROWS : first, whole1 = a.L / ROWS;
+    const int whole0 = k0 >= a.S ? nqb : a.causal ? (k0 + 31 + ROWS - 1) / ROWS : first, whole1 = a.L / ROWS;
     for (; qb < min(whole0, nqb); ++qb) any(qb);
     for (; qb < whole1; ++qb) {
       const char* qs = next(qb);
@@ -844,18 +846,27 @@ struct FlashFwd {
       hipLaunchKernelGGL((flash_fwd_kernel<T, D, NW, false>), grid, dim3(64 * NW), 0, st, a);
   }
 };
+// Calls none of whose blocks are whole for any wave, those with a mask and short ones, have kernels without the second loop, of the registers
+// and waves that they had before there was one.  us, backward with a mask, one kernel before the second loop / with it / a kernel without: 256 heads of
+// 320 x 64 62.6 / 67.4 / 58.9, of 1024 x 64 406 / 408 / 382.
 template <typename T, int D>
 struct FlashDq {
   template <int NW>
   static void run(hipStream_t st, const FlashArgs& a, dim3 grid) {
-    hipLaunchKernelGGL((flash_dq_kernel<T, D, NW>), grid, dim3(64 * NW), 0, st, a);
+    if (kInterleaveDq<D> && !a.mask && a.S >= Op<T>::ROWS && (!a.causal || a.L > Op<T>::ROWS))
+      hipLaunchKernelGGL((flash_dq_kernel<T, D, NW, kInterleaveDq<D>>), grid, dim3(64 * NW), 0, st, a);
+    else
+      hipLaunchKernelGGL((flash_dq_kernel<T, D, NW, false>), grid, dim3(64 * NW), 0, st, a);
   }
 };
 template <typename T, int D>
 struct FlashDkv {
   template <int NW>
   static void run(hipStream_t st, const FlashArgs& a, dim3 grid) {
-    hipLaunchKernelGGL((flash_dkv_kernel<T, D, NW>), grid, dim3(64 * NW), 0, st, a);
+    if (kInterleaveDkv<D> && !a.mask && a.L >= (a.causal ? 2 : 1) * Op<T>::ROWS)
+      hipLaunchKernelGGL((flash_dkv_kernel<T, D, NW, kInterleaveDkv<D>>), grid, dim3(64 * NW), 0, st, a);
+    else
+      hipLaunchKernelGGL((flash_dkv_kernel<T, D, NW, false>), grid, dim3(64 * NW), 0, st, a);
   }
 };
 template <class Pass>

@@ -19,7 +19,8 @@
 // reads, MFMA and the softmax's vector instructions in equal parts (about 1000 clocks each for a wave's 32 x 64 scores at
 // D = 128, bf16), which two or more waves per SIMD overlap.
 // Measured (one wave per tile -> shared blocks -> this; forward, backward): 64 heads of 1500 x 128 in bf16 261 -> 113 -> 106 us (690 TFLOP/s),
-// 636 -> 309 -> 269 us; 256 causal heads of 512 x 64 28 -> 22 -> 21 us, 78 -> 72 -> 65 us.
+// 636 -> 309 -> 269 us; 256 causal heads of 512 x 64 28 -> 22 -> 21 us, 78 -> 72 -> 65 us; with a [512, 512] mask, D = 32, 42 us and 116 ->
+// 90 -> 87 us.
 #include "common.h"
 
 #include <type_traits>
@@ -240,11 +241,22 @@ __device__ __forceinline__ void add_mask(const FlashArgs& a, int mine, int base,
       for (int e = 0; e < 4; ++e) v[4 * a4 + e] = fmaf(m[e], factor, v[4 * a4 + e]);
     }
   } else {
+    float m[16];
+    // A whole block in a column: one offset for all sixteen rows.  With sixteen clamped ones the key pass at D = 32 had no registers left for the
+    // values, and took them one by one: backward of 256 heads of 512 with a mask 149 us, 86.7 so.
+    if (!KEYS_IN_REGS && base + 32 <= last + 1) {
+      const unsigned at = (unsigned)(4 * g * a.S + own);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int other = min(base + 8 * (r >> 2) + 4 * g + (r & 3), last);
-      v[r] = fmaf(a.mask[KEYS_IN_REGS ? (long)own * a.S + other : (long)other * a.S + own], factor, v[r]);
+      for (int r = 0; r < 16; ++r) m[r] = (a.mask + (long)(base + 8 * (r >> 2) + (r & 3)) * a.S)[at];
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int other = min(base + 8 * (r >> 2) + 4 * g + (r & 3), last);
+        m[r] = a.mask[KEYS_IN_REGS ? (long)own * a.S + other : (long)other * a.S + own];
+      }
     }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = fmaf(m[r], factor, v[r]);
   }
 }
 

@@ -1,6 +1,7 @@
 """The running-softmax attention core's backward over blocks of 64 rows without edges (whose vector work runs between the MFMAs) beside
-blocks with edges, and its results' stores by whole lines, against float64 on the CPU: one block, ragged ends, the causal diagonal at every
-wave of a workgroup, hidden keys, results inside wider rows."""
+blocks with edges, and its results' stores by whole lines, against float64 on the CPU: one block, ragged ends, hidden keys, results inside wider
+rows in workgroups of two waves; the causal diagonal at every wave of a workgroup of four, with and without a key bias, and masks, which have
+kernels without the interleaved loop, element by element."""
 import pytest
 import torch
 
@@ -44,6 +45,55 @@ def test_packed_self_attention(L, causal, pad, d):
     for i, r in enumerate(ref):
         assert rel_err(dx[:, :, i * E:(i + 1) * E], r.grad) <= TOL[torch.bfloat16]
     assert torch.equal(dx[:, :, 3 * E:], torch.full_like(dx[:, :, 3 * E:], 7.0))
+
+
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("L,N,H,form", [(193, 16, 8, "causal"), (193, 16, 8, "causal, key bias"), (193, 16, 8, "key bias"), (256, 16, 8, "causal"),
+                                        (193, 16, 8, "mask"), (130, 1, 3, "mask"), (64, 2, 2, "mask"), (33, 5, 3, "causal")])
+def test_every_element(L, N, H, form, d):
+    """Workgroups of four waves from 256 of them on (128 heads of 129 rows or more), of two below."""
+    from rtp_amd import ops
+    gen = torch.Generator().manual_seed(L + d)
+    E = H * d
+    qkv, do = (torch.randn(L, N, n * E, generator=gen).to(torch.bfloat16) for n in (3, 1))
+    add, kb, mask = torch.zeros(N, 1, L, L, dtype=torch.float64), None, None
+    if "causal" in form:
+        add = add.masked_fill(torch.ones(L, L).triu(1).bool(), float("-inf"))
+    if "key bias" in form:  # hidden keys at the end, but never all of a query's
+        kb = torch.randn(N, L, generator=gen)
+        kb[1::2, L - 70:] = float("-inf")
+        add = add + kb.double()[:, None, None, :]
+    if form == "mask":
+        mask = torch.randn(L, L, generator=gen)
+        mask[torch.rand(L, L, generator=gen) < 0.3] = float("-inf")
+        mask[:, 0] = 0.0
+        add = add + mask.double()
+    heads = lambda t: t.double().view(L, N, H, d).permute(1, 2, 0, 3)
+    back = lambda t: t.permute(2, 0, 1, 3).reshape(L, N, E)
+    (q, k, v), g, c = (heads(t) for t in qkv.chunk(3, -1)), heads(do), d ** -0.5
+    p = torch.softmax(q @ k.transpose(2, 3) * c + add, -1)
+    out = p @ v
+    delta = (g * out).sum(-1, keepdim=True)
+    ds = p * (g @ v.transpose(2, 3) - delta)
+    # bf16 keeps 8 significant bits: half a unit of the last one is at most u = 2^-8 of the value.  P and dS are rounded once, as factors; O once, and
+    # delta is formed from it; results once.  The fp32 sums of up to 256 terms and the exponentials of scores below 16 are within 2^-16 of their
+    # terms: a sixteenth of u covers them.
+    u = 2.0 ** -8
+    near = u + u / 16
+    ds_err = near * (ds.abs() + p * (g.abs() * out.abs()).sum(-1, keepdim=True)) + u / 16 * p * (g.abs() @ v.abs().transpose(2, 3))
+    wants = [(ds @ k * c, ds_err @ k.abs() * c), (ds.transpose(2, 3) @ q * c, ds_err.transpose(2, 3) @ q.abs() * c),
+             (p.transpose(2, 3) @ g, near * (p.transpose(2, 3) @ g.abs()))]
+    xd, dd = qkv.to(DEV), do.to(DEV)
+    kd, md = (None if t is None else t.to(DEV) for t in (kb, mask))
+    o, dx = torch.empty_like(dd), torch.empty_like(xd)
+    lse, delta_d = (torch.empty(N * H, L, device=DEV) for _ in range(2))
+    st, os_ = (3 * N * E, 3 * E, d, 3 * E), (N * E, E, d, E)
+    ops.attn_flash_fwd(xd, 0, E, 2 * E, st, o, 0, os_, lse, md, "causal" in form, c, L, N, H, d, 1, key_bias=kd)
+    ops.attn_flash_bwd(xd, 0, E, 2 * E, st, o, dd, 0, os_, lse, delta_d, dx, md, "causal" in form, c, L, N, H, d, 1, key_bias=kd)
+    wants.append((out, near * (p @ v.abs())))
+    for got, (want, err) in zip(list(dx.cpu().chunk(3, -1)) + [o.cpu()], wants):
+        bound = err + u * (want.abs() + err)
+        assert bool(((got.double() - back(want)).abs() <= back(bound)).all())
 
 
 @pytest.mark.parametrize("L,N,H,d", [(32, 1, 1, 64), (5, 3, 3, 64), (32, 257, 8, 64), (31, 2049, 1, 64), (32, 5, 1, 32), (9, 7, 1, 128)])

@@ -348,11 +348,15 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-  // (bf16: even and odd k-steps apart, which is the order in which the 256 x 256 kernel's fragments add up)
+  // Row sums of A: bf16 even and odd k-steps apart, which is the order in which the 256 x 256 kernel's fragments add up.  Both wave columns hold the same
+  // rows; in the 256 x 128 tile, whose registers don't hold twice the sums of four blocks, each takes two of them (5085 x 1280 x 5120 as a weight
+  // gradient, with or without sums, 108 us where one took all and the loop spilled, 88 so; smaller tiles lose by a second branch).
   constexpr int NSUM = sizeof(T) == 2 && !AKC ? 2 : 1;
-  float rsum[MT][NSUM];
+  constexpr bool SHARED_SUMS = NSUM == 2 && WGN == 2 && MT == 4;
+  constexpr int MS = SHARED_SUMS ? MT / 2 : MT;  // blocks whose rows a wave sums
+  float rsum[MS][NSUM];
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
+  for (int i = 0; i < MS; ++i)
 #pragma unroll
     for (int c = 0; c < NSUM; ++c) rsum[i][c] = 0.0f;
 
@@ -482,7 +486,7 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
     Frag<T> fa[NSET][MT], fb[NSET][NT];
     // Row sums of A (a bias gradient) ride along in the waves of the tile row's first tile that own column
     // block 0: each lane adds up the k values of its own row as the fragments pass by.
-    const bool rowsum = p.a_rowsum != nullptr && tile_n == 0 && wn == 0;
+    const bool rowsum = p.a_rowsum != nullptr && tile_n == 0 && (SHARED_SUMS || wn == 0);
     auto read_step = [&](auto S, auto Q, auto SET) {
       const char* sa = lds + (decltype(S)::value % NSTAGE) * STAGE;
       const char* sb = sa + DA::BYTES;
@@ -499,8 +503,13 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
 #pragma unroll
         for (int j = 0; j < NT; ++j) mma(fa[set][i], fb[set][j], acc[i][j]);
       if (rowsum) {
+        if (SHARED_SUMS && wn != 0) {
 #pragma unroll
-        for (int i = 0; i < MT; ++i) rsum[i][c] = frag_sum(fa[set][i], rsum[i][c]);
+          for (int i = 0; i < MS; ++i) rsum[i][c] = frag_sum(fa[set][MT - MS + i], rsum[i][c]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < MS; ++i) rsum[i][c] = frag_sum(fa[set][i], rsum[i][c]);
+        }
       }
     };
     // k-step Q of slab k (stage S).  The scheduling fences keep the order written here: left alone, the compiler
@@ -535,8 +544,9 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
       __builtin_amdgcn_sched_barrier(0);
     };
     // A condition a slab holds up loops that issue more for an MFMA than the aligned bf16 ones: 180 x 1024 x 1024 in fp32 26.1 -> 27.5 us,
-    // the fp32 cores' batched products 9.5 -> 10.3.  Those ask for everything at their start.
-    constexpr bool PACED = sizeof(T) == 2 && !REG && !RAG;
+    // the fp32 cores' batched products 9.5 -> 10.3.  Those ask for everything at their start, and so does the 256 x 128 tile, which has no
+    // registers left.
+    constexpr bool PACED = sizeof(T) == 2 && !REG && !RAG && BM * BN < 256 * 128;
     WarmAhead warm(p, (unsigned)(uintptr_t)(lptr_t)lds + NSTAGE * STAGE, id, nwg, wave, lane, PACED ? nk : 0);
     auto phase = [&](auto S, int k, auto STEADY) {
       if (!decltype(STEADY)::value && k >= nk) return;
@@ -567,14 +577,14 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
     if (p.trace != nullptr && tid == 0) t_loop = (unsigned long long)wall_clock64();
   }
   const bool computes = wave < 4;
-  if (computes && p.a_rowsum != nullptr && tile_n == 0 && wn == 0) {
+  if (computes && p.a_rowsum != nullptr && tile_n == 0 && (SHARED_SUMS || wn == 0)) {
     // lanes 0..31 and 32..63 hold the two k halves of the same 32 rows
     T* dst = reinterpret_cast<T*>(p.a_rowsum) + grp * p.rowsum_sg;
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
+    for (int i = 0; i < MS; ++i) {
       float v = rsum[i][0] + __shfl_xor(rsum[i][0], 32, 64);
       if constexpr (NSUM == 2) v += rsum[i][1] + __shfl_xor(rsum[i][1], 32, 64);
-      const int row = m0 + wm * WM + i * 32 + li;
+      const int row = m0 + wm * WM + (SHARED_SUMS ? wn * MS + i : i) * 32 + li;
       if (g == 0 && row < p.m) dst[row] = from_f32<T>((p.flags & RTP_GEMM_ROWSUM_ACCUM) ? to_f32(dst[row]) + v : v);
     }
   }

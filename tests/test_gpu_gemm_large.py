@@ -250,3 +250,21 @@ def test_updates_of_parameters_that_are_no_whole_lines_go_elsewhere(shift, gap, 
     new = old[:, :m * n] - Sgd.lr * grad.float().clamp(-Sgd.clip, Sgd.clip)
     assert torch.equal(master[:, :m * n], new) and torch.equal(copy[:, :m * n], new.to(BF))
     assert torch.equal(master[:, rest], old[:, rest]) and copy[:, rest].isnan().all() and out[:, rest].isnan().all()
+
+
+@pytest.mark.parametrize("m,n,k", [(2048, 4096, 1024), (2040, 4096, 1000), (1288, 4608, 1032)])
+def test_row_sums_shared_by_two_wave_columns(m, n, k):
+    """The 256 x 128 tile, whose wave columns sum two of a wave tile's four row blocks each: every row once, whole and ragged tiles, on top of what is
+    there and alone.  A sum of k terms in fp32 is within k units of 2^-24 of their magnitudes, and rounds to bf16's 8 bits (half a unit: 2^-8)."""
+    gen = torch.Generator().manual_seed(k)
+    a, b = _rand((k, m), BF, gen).to(DEV), _rand((k, n), BF, gen).to(DEV)
+    old = _rand((m,), BF, gen).to(DEV)
+    out = torch.empty(m, n, dtype=BF, device=DEV)
+    for accumulate in (False, True):
+        sums = old.clone()
+        fused = _run("256x128", a=a.data_ptr(), b=b.data_ptr(), c_out=out.data_ptr(), m=m, n=n, k=k, lda=m, ldb=n, ldc=n, a_kcontig=False,
+                     b_kcontig=False, rowsum=sums.data_ptr(), rowsum_accum=accumulate)
+        want = a.double().sum(0) + (old.double() if accumulate else 0)
+        bound = (k + 2) * 2.0 ** -24 * (a.double().abs().sum(0) + old.double().abs()) + 2.0 ** -8 * want.abs()
+        assert fused and bool(((sums.double() - want).abs() <= bound).all())
+    assert rel_err(out, a.float().t() @ b.float()) <= TOL[BF]

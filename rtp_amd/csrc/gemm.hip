@@ -544,10 +544,10 @@ __device__ __forceinline__ void gemm_dma_body(const GemmArgs& p, const unsigned 
       __builtin_amdgcn_sched_barrier(0);
     };
     // A condition a slab holds up loops that issue more for an MFMA than the aligned bf16 ones: 180 x 1024 x 1024 in fp32 26.1 -> 27.5 us,
-    // the fp32 cores' batched products 9.5 -> 10.3.  Those ask for everything at their start, and so does the 256 x 128 tile, which has no
-    // registers left.
-    constexpr bool PACED = sizeof(T) == 2 && !REG && !RAG && BM * BN < 256 * 128;
-    WarmAhead warm(p, (unsigned)(uintptr_t)(lptr_t)lds + NSTAGE * STAGE, id, nwg, wave, lane, PACED ? nk : 0);
+    // the fp32 cores' batched products 9.5 -> 10.3.  Those ask for everything at their start, and so do the 256 x 128 tile, which has no
+    // registers left, and 64 x 64, whose loops are short.
+    constexpr bool PACED = sizeof(T) == 2 && !REG && !RAG && BM >= 128 && BM * BN < 256 * 128;
+    WarmAhead warm(p, (unsigned)(uintptr_t)(lptr_t)lds + NSTAGE * STAGE, id, nwg, wave, lane, PACED);
     auto phase = [&](auto S, int k, auto STEADY) {
       if (!decltype(STEADY)::value && k >= nk) return;
       if constexpr (PACED) warm.slab();
@@ -1443,7 +1443,6 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d, PairPlan* plan = n
                         (double)d->n * copies(d->b_so, d->b_si, d->b_sg, d->b_sk)) * (double)d->k * sizeof(T) +
                        mn * (out_sz + cin_sz + upd_sz);
   a.warm = nullptr;
-  a.warm_bytes = 0;
   if (plan) {
     a.trace = nullptr;
     plan->args = a, plan->flops = 2.0 * mn * kk, plan->bytes = bytes;
@@ -1457,10 +1456,8 @@ static int launch_gemm(hipStream_t s, const rtp_gemm_desc* d, PairPlan* plan = n
   // cache / in HBM, 1024 x 2048 x 2048 split 56 - 61 / 58 - 60, with fp32 MFMAs 77 / 71, 1024 x 6144 x 2048 164 / 164 and 196 / 184.
   // Few rows do (bf16 64 x 2048 x 2048 6.3 / 8.5, input gradient 7.0 / 11.9; fp32 13.5 / 15.3), and are ahead of the tiles that
   // carry hints all the same (gemm_kwaves.hip).
-  if (shape != 5 && !split && warm_src != nullptr) {
-    a.warm = (const char*)warm_src;
-    a.warm_bytes = (long)t_warm_bytes;
-  }
+  if (shape != 5 && !split && warm_src != nullptr)
+    warm_launch(a, warm_src, t_warm_bytes, (int64_t)grid.x * grid.y, ceil_div(d->k, (int64_t)(128 / sizeof(T))) * d->ksegs);
   if (split) return launch_split(s, a, akc, bkc, ts.bm, !vec, grid);
   if (!vec) {
     if (direct)

@@ -56,7 +56,8 @@ struct GemmArgs {
   const float* xent_scale;      // mode 2: second scalar factor (1 / rows counted), or null
   // bytes that some later launch will read from HBM (the next layer's shards): requested here, see WarmAhead
   const char* warm;
-  long warm_bytes;
+  unsigned warm_pieces;         // KiB
+  int warm_each, warm_slab;     // pieces of a wave at most, and those that it asks for in a slab
   unsigned tiles, per_xcd;  // gemm_large.hip: all tiles of the launch, an XCD's share of them (rounded up)
 };
 
@@ -745,21 +746,24 @@ struct DmaOperand {
 // residual or mask (the language model's step 3544 us against 3509; over a quarter of the loop 3520, half 3510, all of it
 // 3522, where the last ones are still on their way when the epilogue waits for its operands).
 constexpr int kWarmMax = 48;
+inline void warm_launch(GemmArgs& a, const void* src, size_t bytes, int64_t workgroups, int64_t slabs) {
+  const int64_t pieces = bytes >> 10 < 1u << 30 ? (int64_t)(bytes >> 10) : 1 << 30, each = ceil_div(pieces, 4 * workgroups), over = slabs - slabs / 4;
+  if (pieces == 0) return;
+  a.warm = (const char*)src, a.warm_pieces = (unsigned)pieces;
+  a.warm_each = each < kWarmMax ? (int)each : kWarmMax;
+  a.warm_slab = (int)ceil_div(a.warm_each, over > 0 ? over : 1);
+}
 struct WarmAhead {
   const char* src;  // the wave's next piece
   long step;        // bytes from one of its pieces to the next
   unsigned off, lds_dst;
   int left, per_slab;
-  __device__ __forceinline__ WarmAhead(const GemmArgs& p, unsigned dst, unsigned wg, unsigned nwg, int wave, int lane, int nk) {
+  __device__ __forceinline__ WarmAhead(const GemmArgs& p, unsigned dst, unsigned wg, unsigned nwg, int wave, int lane, bool paced) {
     src = nullptr, step = 0, left = 0, per_slab = 0;
-    if (p.warm != nullptr) {  // (launches without a hint are spared the divisions)
+    if (p.warm != nullptr) {  // (the launch has divided: in front of the first MFMA two divisions took 0.2 us of products of four slabs)
       const unsigned piece = wg * 4 + wave, step_pieces = nwg * 4;
-      const long all = p.warm_bytes >> 10;
-      const unsigned total = all < (1l << 30) ? (unsigned)all : 1u << 30;
-      const unsigned mine = total > piece ? (total - piece - 1) / step_pieces + 1 : 0;
-      left = mine < (unsigned)kWarmMax ? (int)mine : kWarmMax;
-      const int slabs = nk > 0 ? nk - nk / 4 : 1;  // (0: all at once)
-      per_slab = (left + slabs - 1) / slabs;
+      left = piece + (p.warm_each - 1) * step_pieces < p.warm_pieces ? p.warm_each : p.warm_each - 1;
+      per_slab = paced ? p.warm_slab : left;
       src = p.warm + ((long)piece << 10);
       step = (long)step_pieces << 10;
     }

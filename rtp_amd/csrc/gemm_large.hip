@@ -34,7 +34,9 @@ namespace rtp {
 // in registers, two waves a SIMD, random operands, TF/s: 32 x 32 x 16 1600 in any order; 16 x 16 x 32 with the k-steps apart 1800, back to back
 // 1850; zeros 2210 / 2150 / 2195).  The results have the same bits.  us, 32 x 32 x 16 -> this, forward / input gradient / weight gradient layout:
 // 8 of 1024 x 8192 x 2048 228 / 233 / 246 -> 214 / 220 / 235, 4096^3 103.5 / 108.5 / 112.5 -> 97.5 / 102 / 109.5, 4096 x 6144 x 2048 93 / - / - -> 87,
-// 8192^3 773 / - / - -> 729; half a round of tiles, where the clock is free, 4096 x 2048 x 2048 39.1 / 38.8 / - -> 40.0 / 39.0.
+// 8192^3 773 / - / - -> 729 (cards differ: on a slower one 4096^3 112 -> 104 as a weight gradient).  It takes 11 % more clocks (the same LDS accesses and
+// conflicts, longer waits for them), which costs where the clock is free: half a round of tiles, 4096 x 2048 x 2048 39.1 / 38.8 / - -> 40.0 / 39.0,
+// 135 tiles, 1280 x 6912 x 8192, 132.5 / 137 / 150 -> 139.5 / 147 / 165, 155 tiles of four slabs 12.0 / 12.1 / 12.7 -> 12.3 / 12.7 / 13.4; from 192 tiles on it gains.
 //
 // A workgroup stays on its CU and goes through its tiles (the tile number advances by the number of workgroups), and the loads run on
 // into the next tile: when a tile's last MFMAs are done, the first slab and a half of the next are in the LDS or on their way, and the
